@@ -215,6 +215,7 @@ struct bpsx_sim {
   std::vector<Group> groups;
   GeoSlot* d_slots = nullptr;
   uint32_t geo_blocks = 0, snap_blocks = 0;
+  uint32_t max_geo_blocks = 0, compute_units = 0;   // what the device holds of k_geodesic at once, whatever the number of envs
   uint32_t* d_error = nullptr;
   uint64_t* d_counters = nullptr;
   float turn_left[4], turn_right[4];
@@ -225,6 +226,8 @@ struct bpsx_sim {
   // scratch for the batched query entry points
   void* d_batch = nullptr;
   size_t batch_bytes = 0;
+  GeoSlot* d_batch_slots = nullptr;   // node pools of a batch of path queries that needs more wavefronts than the steps have
+  uint32_t batch_slot_blocks = 0;
   uint32_t* d_batch_counts = nullptr;
 
   template <class T>
@@ -603,6 +606,8 @@ int bpsx_finalize(bpsx_sim* sim) {
   HIP_TRY(hipGetDeviceProperties(&prop, sim->cfg.gpu_id));
   uint32_t per_cu = geodesic_blocks_per_cu();   // blocks of two wavefronts
   uint32_t blocks = (uint32_t)prop.multiProcessorCount * per_cu;
+  sim->max_geo_blocks = blocks;
+  sim->compute_units = (uint32_t)prop.multiProcessorCount;
   if (blocks > sim->envs_per_group) blocks = sim->envs_per_group;
   sim->geo_blocks = std::max(1u, blocks);
   sim->snap_blocks = std::max(1u, std::min((uint32_t)prop.multiProcessorCount * 16u, sim->envs_per_group));
@@ -666,6 +671,7 @@ void bpsx_destroy(bpsx_sim* sim) {
   }
   for (void* p : sim->owned) (void)hipFree(p);
   if (sim->d_batch) (void)hipFree(sim->d_batch);
+  if (sim->d_batch_slots) (void)hipFree(sim->d_batch_slots);
   delete sim;
 }
 
@@ -862,6 +868,25 @@ static int batch_reserve(bpsx_sim* sim, size_t bytes) {
   sim->batch_bytes = bytes;
   return BPSX_OK;
 }
+// Node pools for a batch of n path queries: as many blocks of k_geodesic as the device holds at
+// once, or one per query where that is less.  The steps' own pools serve if they are enough (a
+// simulator has no more of them than envs in a group); otherwise the batch has pools of its own,
+// kept until a larger batch or bpsx_destroy replaces them (at most 0.7 GB).
+// (1000 pairs over a maze, simulator of 4 envs, so far served by 4 blocks: 131 -> 2.3 ms a call.)
+static int batch_reserve_slots(bpsx_sim* sim, uint32_t n, GeoSlot** slots, uint32_t* blocks) {
+  const uint32_t want = std::min(sim->max_geo_blocks, n);
+  if (want <= sim->geo_blocks) { *slots = sim->d_slots; *blocks = sim->geo_blocks; return BPSX_OK; }
+  if (want > sim->batch_slot_blocks) {
+    if (sim->d_batch_slots) HIP_TRY(hipFree(sim->d_batch_slots));
+    sim->d_batch_slots = nullptr;
+    sim->batch_slot_blocks = 0;
+    HIP_TRY(hipMalloc((void**)&sim->d_batch_slots, (size_t)want * 2 * sizeof(GeoSlot)));
+    sim->batch_slot_blocks = want;
+  }
+  *slots = sim->d_batch_slots;
+  *blocks = want;
+  return BPSX_OK;
+}
 // Brings the host's view of a slot up to date: a swap whose envs have all moved is complete.
 static int settle_slot(bpsx_sim* sim, uint32_t slot, uint32_t* remaining_out) {
   SceneSlot& sl = sim->slots[slot];
@@ -1015,7 +1040,10 @@ int bpsx_snap_points(bpsx_sim* sim, uint32_t scene, const float* pts, uint32_t n
   char* b = (char*)sim->d_batch;
   float* d_in = (float*)b; float* d_xyz = (float*)(b + f3); uint32_t* d_ref = (uint32_t*)(b + 2 * f3);
   HIP_TRY(hipMemcpy(d_in, pts, f3, hipMemcpyHostToDevice));
-  launch_snap_batch(sim->nav, scene_entry(sim, scene), d_in, n, d_xyz, d_ref, sim->snap_blocks * 4, nullptr);
+  // a wavefront per point, as many as the device holds at once (32 per CU), not as a group has
+  // envs: 50000 samples, moves and snaps over a cluttered plan by a
+  // simulator of two envs took 316 ms, nearly all of it the snaps on 8 wavefronts, now 2.2 ms
+  launch_snap_batch(sim->nav, scene_entry(sim, scene), d_in, n, d_xyz, d_ref, sim->compute_units * 32u, nullptr);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpy(out_xyz, d_xyz, f3, hipMemcpyDeviceToHost));
   HIP_TRY(hipMemcpy(out_ref, d_ref, (size_t)n * 4, hipMemcpyDeviceToHost));
@@ -1056,12 +1084,15 @@ int bpsx_geodesic(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const u
   float* d_s = (float*)(b + qb); float* d_e = (float*)(b + qb + f3);
   uint32_t* d_sr = (uint32_t*)(b + qb + 2 * f3); uint32_t* d_er = (uint32_t*)(b + qb + 2 * f3 + u1);
   float* d_o = (float*)(b + qb + 2 * f3 + 2 * u1);
+  GeoSlot* slots = nullptr;
+  uint32_t blocks = 0;
+  if ((rc = batch_reserve_slots(sim, n, &slots, &blocks))) return rc;
   HIP_TRY(hipMemcpy(d_s, start_xyz, f3, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_e, end_xyz, f3, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_sr, start_ref, u1, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_er, end_ref, u1, hipMemcpyHostToDevice));
-  launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, d_q, sim->d_batch_counts, d_o, sim->d_slots,
-                        sim->geo_blocks, sim->d_counters, nullptr);
+  launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, d_q, sim->d_batch_counts, d_o, slots, blocks,
+                        sim->d_counters, nullptr);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpy(out_dist, d_o, u1, hipMemcpyDeviceToHost));
   return BPSX_OK;

@@ -689,9 +689,9 @@ __global__ void k_random_points(NavData nav, uint32_t scene, const float* u, uin
   oxyz[(size_t)i * 3] = p[0]; oxyz[(size_t)i * 3 + 1] = p[1]; oxyz[(size_t)i * 3 + 2] = p[2];
   oref[i] = ok ? (s.ref_base | ip) : 0;
 }
-// counts and both ticket counters of a batch of n queries, all in the class of the shortest
-__global__ void k_set_counts(uint32_t* p, uint32_t n) {
-  if (threadIdx.x <= (uint32_t)kGeoClasses) p[threadIdx.x] = threadIdx.x == (uint32_t)kGeoClasses - 1u ? n : 0u;
+// counts and ticket counter of a batch of n queries, all in class cls
+__global__ void k_set_counts(uint32_t* p, uint32_t n, uint32_t cls) {
+  if (threadIdx.x <= (uint32_t)kGeoClasses) p[threadIdx.x] = threadIdx.x == cls ? n : 0u;
 }
 
 }  // namespace
@@ -771,8 +771,11 @@ void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz
                            const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */, float* out,
                            GeoSlot* slots, uint32_t geo_blocks, uint64_t* counters, hipStream_t st) {
   hipLaunchKernelGGL(k_make_queries, grid_for(n, 256), dim3(256), 0, st, scene, sxyz, sref, exyz, eref, n, qbuf);
-  hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n);
-  // one class only: stride 0 puts its queries at the start of the buffer
+  // One class only.  With a block for every query they count as the longest: each then runs on
+  // its block's whole LDS.  Otherwise as the shortest: two to a block.
+  const uint32_t cls = n <= geo_blocks ? 0u : (uint32_t)kGeoClasses - 1u;
+  hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n, cls);
+  // stride 0 puts the class's queries at the start of the buffer
   launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, slots,
                   geo_blocks, counters, st);
 }
