@@ -6,19 +6,17 @@
 // a shared queue when done.  The search touches almost only nodes it created recently (the
 // frontier of A* is narrow), so LDS holds what is hot and small and HBM holds the rest:
 //   - the open list in registers: sorted by total, up to 256 entries (OpenList), which lets a
-//     pass expand up to kRows nodes at once (astar_fast); the reference's binary heap, also in
-//     registers while it has fewer than 128 entries (RegHeap, entry q in lane q mod 64), is
-//     what a search falls back to when totals tie or the list outgrows its registers; a heap
-//     longer than that (rare) keeps its top kHeapLds entries in LDS,
+//     pass expand up to kRows nodes at once (astar_fast); when totals tie, the reference's binary
+//     heap is rebuilt from a log of the list's operations (RefHeap, replay_log), and a search whose
+//     list outgrows the registers goes on with that heap,
 //   - the hash heads of the node pool,
 //   - for the first kLinksLds nodes one word with the polygon id, the open/closed flags and the
 //     hash chain link (the parent index is read once per expansion and lives in HBM only),
 //   - the position, cost and total of the kWindow most recently created nodes (slot = index
 //     modulo kWindow) and their parent index; every write of those also goes to the
 //     wavefront's slot in HBM, so an older node is simply read from there.
-// Heap entries beyond kHeapLds and links beyond kLinksLds spill to the same slot.  A query
-// runs the instantiation of the loop without spill code until one more expansion could
-// outgrow the links in LDS or the register heap, then carries on in a spilling instantiation.
+// Links beyond kLinksLds spill to the same slot.  A query runs the instantiation of the loop without
+// spill code until one more pass could outgrow the links in LDS, then carries on in a spilling one.
 // Per expanded node the regular HBM traffic is the polygon's six 16-byte edge records (lane j
 // of the wavefront handles edge j: node lookup, cost, heuristic) plus the write-through of
 // updated nodes; heap updates are applied in edge order, which is what makes the result
@@ -31,7 +29,7 @@
 // :1661-1696, 1765-1994 (appendVertex, findStraightPath), :2279-2381 (getPortalPoints,
 // getEdgeMidPoint); DetourNode.cpp:50-200 (node pool, heap order); PathFinder.cpp:473-541.
 //
-// The sizes of the LDS structures are build parameters (BPSX_LINKS_LDS, BPSX_HEAP_LDS,
+// The sizes of the LDS structures are build parameters (BPSX_LINKS_LDS,
 // BPSX_WINDOW, BPSX_HASH, BPSX_TAG_SLOTS), and everything that depends on them lives in namespace
 // bpsx::BPSX_GEO_NS (default geo): the file can be included again with other values and
 // another namespace name to get a second instantiation of the same search.
@@ -100,7 +98,6 @@ BPSX_DEV void wlane2(uint32_t& a, uint32_t va, uint32_t& b, uint32_t vb, int lan
   asm("s_mov_b32 m0, %4\n\tv_writelane_b32 %0, %2, m0\n\tv_writelane_b32 %1, %3, m0" : "+v"(a), "+v"(b) : "s"(sa), "s"(sb), "s"(sl) : "m0");
 }
 
-// lanes 8..15 of each row of 16 take src of the lane 8 below them, lanes 0..7 keep low
 // min(v, v of the lane that the DPP control names); lanes without such a lane, or outside the
 // row mask (one bit per 16 lanes), keep v.  (The other lane's value defaults to the identity of
 // the minimum, which lets the compiler fold the lane move into the v_min itself.)
@@ -108,30 +105,6 @@ template <int Ctrl, int RowMask> BPSX_DEV uint32_t umin_dpp(uint32_t v) {
   const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, Ctrl, RowMask, 0xf, false);
   return o < v ? o : v;
 }
-BPSX_DEV float lanes_up8(float low, float src) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(low), __float_as_int(src), 0x118 /* row_shr:8 */, 0xf, 0xf, false));
-}
-// lanes 0..7 of each row take v of the lane 8 above them
-BPSX_DEV float lanes_down8(float v) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x108 /* row_shl:8 */, 0xf, 0xf, false));
-}
-// Correctly rounded square root, the value sqrtf returns on the host: the hardware estimate is
-// within one unit in the last place, and the residuals of its two neighbours say which of the
-// three is the rounded root.  Same scheme as the compiler's own expansion of sqrtf, minus its
-// rescaling of arguments below 2^-96 (needed there for the residuals not to underflow): the
-// arguments here are squared distances, zero or far above that; a wavefront that meets one in
-// between takes the library routine.
-BPSX_DEV float sqrt_exact(float x) {
-  const uint32_t xb = __float_as_uint(x);
-  if (__builtin_expect(lanes_where(xb - 1u < 0x0f800000u - 1u) != 0, 0)) return sqrtf(x);   // 0 < x < 2^-96 in some lane: never in practice
-  const float s = __builtin_amdgcn_sqrtf(x);
-  const float down = __uint_as_float(__float_as_uint(s) - 1u), up = __uint_as_float(__float_as_uint(s) + 1u);
-  const float rdown = fmaf(-down, s, x), rup = fmaf(-up, s, x);
-  float r = rdown <= 0.0f ? down : s;
-  r = rup > 0.0f ? up : r;
-  return r;
-}
-
 // One word per node holds what the search loop reads of it besides the window: the parent
 // index is needed once per expansion and for the final path, and lives in HBM only.
 constexpr uint32_t kChainEnd = 0xfffu;
@@ -142,144 +115,12 @@ BPSX_DEV uint32_t link_next(uint32_t l) { return l >> 20; }
 BPSX_DEV uint32_t make_link(uint32_t id, uint32_t flags, uint32_t next) { return id | (flags << 15) | (next << 20); }
 BPSX_DEV uint32_t with_flags(uint32_t l, uint32_t flags) { return (l & ~(3u << 15)) | (flags << 15); }
 
-// The open list in registers.  Heap position q (1-based, root = 1; the reference's index + 1)
-// lives in lane q & 63 of the first register pair (q < 64) or of the second (64 <= q < 128).
-// Totals are kept as bit patterns and compared as unsigned integers: they are sums of
-// distances, never negative and never NaN, and for such floats the integer order of the bits
-// is the float order.  Same algorithm as dtNodeQueue (DetourNode.cpp:150-200).
-constexpr int kRegHeap = 127;
-static_assert(kMaxNodes <= 2048, "heap entries keep the node index in 11 bits");
-struct RegHeap {
-  uint32_t t0, t1;   // total bits
-  uint32_t n0, n1;   // node index (bits 0-10) | the node's polygon index << 11, so that popping
-                     // the root names the edge records to fetch without a detour through LDS
-  int size;
-  // constants of the lane: the positions that must each be the smaller of their sibling pair
-  // for the hole of a pop to pass through position `lane` (itself and its ancestors below the
-  // root), as a bit set, and the same for the parent of position 64 + lane
-  uint32_t anc0, anc1, panc0, panc1;
-  static constexpr uint32_t kEmpty = 0x7fffffffu;   // above +inf; every key stays below 2^31
-  static BPSX_DEV unsigned long long route_set(int q) {
-    unsigned long long m = 0;
-    for (; q >= 2; q >>= 1) m |= 1ull << q;
-    return m;
-  }
-  BPSX_DEV void init(int lane) {
-    t0 = t1 = kEmpty; n0 = n1 = 0; size = 0;
-    const unsigned long long a = route_set(lane), pa = route_set(32 + (lane >> 1));
-    anc0 = (uint32_t)a; anc1 = (uint32_t)(a >> 32);
-    panc0 = (uint32_t)pa; panc1 = (uint32_t)(pa >> 32);
-  }
-  // v of the neighbouring lane (lane ^ 1)
-  static BPSX_DEV uint32_t quad_swap(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xb1 /* quad_perm:[1,0,3,2] */, 0xf, 0xf, false);
-  }
-  static BPSX_DEV uint32_t xlane(int src_lane, uint32_t v) {   // v of another lane; all lanes must be active
-    return (uint32_t)__builtin_amdgcn_ds_bpermute(src_lane * 4, (int)v);
-  }
-
-  // dtNodeQueue::bubbleUp of entry (t, n) from position q, by all lanes at once.  The lanes on
-  // the way from q to the root read their parent's entry; ancestors with a greater key move
-  // one step down that way (they form a run from q upwards: keys never increase towards the
-  // root) and the entry lands on top of the run.  Positions 64..127 have all their ancestors
-  // in the first pair, so only q itself can be in the second.
-  template <bool W = true> BPSX_DEV void bubble_up(int q, uint32_t t, uint32_t n, int lane) {
-    const int up = (31 - __clz(q)) - (31 - __clz(lane));   // lane 0 (clz 32) is no heap position
-    const bool on = lane >= 1 && up >= 0 && (q >> (up & 31)) == lane;
-    const uint32_t pk = xlane(lane >> 1, t0), pn = xlane(lane >> 1, n0);
-    const bool parentMoves = on && lane > 1 && pk > t;
-    const bool vacant = lane == q || t0 > t;
-    const bool land = on && vacant && !parentMoves;
-    if (W && q >= 64) {
-      const uint32_t qk = rlane(t0, q >> 1), qn = rlane(n0, q >> 1);
-      const bool here = lane == (q & 63);
-      t1 = here ? (qk > t ? qk : t) : t1;
-      n1 = here ? (qk > t ? qn : n) : n1;
-    }
-    t0 = parentMoves ? pk : (land ? t : t0);
-    n0 = parentMoves ? pn : (land ? n : n0);
-  }
-  BPSX_DEV void push(uint32_t t, uint32_t n, int lane) {
-    size++;
-    bubble_up(size, t, n, lane);
-  }
-  // heap position of node n's entry, 0 if it has none
-  template <bool W = true> BPSX_DEV int position(uint32_t n, int lane) const {
-    const unsigned long long m0 = lanes_where(lane >= 1 && lane <= size && n0 == n);
-    if (m0) return __ffsll((long long)m0) - 1;
-    if (!W || size < 64) return 0;
-    const unsigned long long m1 = lanes_where(64 + lane <= size && n1 == n);
-    return m1 ? 64 + __ffsll((long long)m1) - 1 : 0;
-  }
-  // push (open false) or modify (open true) through one copy of the walk; an open node without
-  // an entry (there is none) would be a walk from position 0, which changes nothing
-  // Most entries stay where they start (a new total is rarely below its parent's): that case is
-  // two lane writes on the scalar unit's word, without the lane-parallel walk.
-  template <bool W = true> BPSX_DEV void update(bool open, uint32_t n, uint32_t t, int lane) {
-    int q;
-    if (open) q = position<W>(n, lane);
-    else q = ++size;
-    const uint32_t pk = rlane(t0, q >> 1);   // position 0 holds kEmpty: no entry (q = 0) and the root take the walk
-    if (pk <= t) {
-      if (!W || q < 64) { t0 = wlane(t0, t, q); n0 = wlane(n0, n, q); }
-      else { t1 = wlane(t1, t, q & 63); n1 = wlane(n1, n, q & 63); }
-      return;
-    }
-    bubble_up<W>(q, t, n, lane);
-  }
-  // dtNodeQueue::pop after the caller has taken the root.  The reference moves the hole left
-  // by the root down to a leaf along the smaller children and then bubbles the former last
-  // entry up from there; along that route keys never decrease, so the entry ends up above the
-  // first route element greater than it and nothing below moves.  Which child the hole moves to
-  // depends only on the children's keys, which the moves above them do not change, so the
-  // route is known at once: siblings sit in neighbouring lanes, one comparison with the
-  // neighbour says for every position whether it is the smaller of its pair (the left one when
-  // equal), and a position is on the route when that holds for itself and all its ancestors,
-  // a test of the ballot against a per-lane constant.  Then every route position whose
-  // smaller child is not greater than the entry takes that child, and the first one whose
-  // child is greater takes the entry.  Positions past the end hold kEmpty and never move.
-  // W false: the caller knows that the list has fewer than 64 entries.
-  template <bool W = true> BPSX_DEV void pop(int lane) {
-    const int last = size;
-    size--;
-    uint32_t lt, ln;
-    if (!W || last < 64) { lt = rlane(t0, last); ln = rlane(n0, last); t0 = wlane(t0, kEmpty, last); }
-    else { lt = rlane(t1, last & 63); ln = rlane(n1, last & 63); t1 = wlane(t1, kEmpty, last & 63); }
-    if (size == 0) return;
-    const bool wide = W && size >= 64;      // entries in the second pair
-    const bool lo = lane < 32;              // children of positions 32..63 are in the second pair
-    constexpr unsigned long long kOdd = 0xaaaaaaaaaaaaaaaaull;
-    // less0: the position's key is below its sibling's.  A right child is the smaller one when
-    // that holds, a left child unless it holds for its right neighbour.
-    const unsigned long long less0 = lanes_where(t0 < quad_swap(t0));
-    const unsigned long long lose0 = ~((less0 & kOdd) | (~(less0 >> 1) & ~kOdd));
-    unsigned long long less1 = 0;
-    if (wide) less1 = lanes_where(t1 < quad_swap(t1));
-    const bool on = lane >= 1 && ((anc0 & (uint32_t)lose0) | (anc1 & (uint32_t)(lose0 >> 32))) == 0;
-    // the smaller child of this lane's position: the right one if its key is below the left one's
-    const int c0 = (2 * lane) & 63;
-    const unsigned long long lessc = lo ? less0 : less1;
-    const int c = c0 + (int)((uint32_t)(lessc >> (c0 + 1)) & 1u);
-    uint32_t ck = xlane(c, t0), cn = xlane(c, n0);
-    if (wide) {
-      const uint32_t hk = xlane(c, t1), hn = xlane(c, n1);
-      ck = lo ? ck : hk; cn = lo ? cn : hn;
-    } else {
-      ck = lo ? ck : kEmpty;
-    }
-    const bool take = on && ck <= lt;
-    const bool land = on && !take && (lane == 1 || t0 <= lt);
-    if (wide) {
-      // positions 64..127 have no children: the one on the route takes the entry if its parent took it
-      const unsigned long long lose1 = ~((less1 & kOdd) | (~(less1 >> 1) & ~kOdd));
-      const bool here = ((lose1 >> lane) & 1ull) == 0 && ((panc0 & (uint32_t)lose0) | (panc1 & (uint32_t)(lose0 >> 32))) == 0 && t1 <= lt;
-      t1 = here ? lt : t1;
-      n1 = here ? ln : n1;
-    }
-    t0 = take ? ck : (land ? lt : t0);
-    n0 = take ? cn : (land ? ln : n0);
-  }
-};
+// Open-list entries: the total as a bit pattern, compared as an unsigned integer (totals are sums of
+// distances, never negative and never NaN, and for such floats the integer order of the bits is the
+// float order), and the node's index (bits 0-10) with its polygon index above it, so that the entry
+// at the front names the edge records to fetch without a detour through LDS.
+static_assert(kMaxNodes <= 2048, "open-list entries keep the node index in 11 bits");
+constexpr uint32_t kEmptyKey = 0x7fffffffu;   // above +inf; every key stays below 2^31
 
 // The open list as a sorted array in registers.  dtNodeQueue::pop returns the entry with the
 // smallest total; while that smallest total is held by one entry only, which entry that is
@@ -292,9 +133,9 @@ struct RegHeap {
 // keys and kNone nodes.  Entries with equal totals sit next to each other in no defined order.
 struct OpenList {
   static constexpr int kPairs = 4;
-  uint32_t t[kPairs], n[kPairs];   // totals as bit patterns (see RegHeap), nodes packed like RegHeap's
+  uint32_t t[kPairs], n[kPairs];
   int size;
-  static constexpr uint32_t kEmpty = 0x7fffffffu;
+  static constexpr uint32_t kEmpty = kEmptyKey;
   static constexpr uint32_t kNone = 0xffffffffu;    // no packed node looks like this (26 bits)
   BPSX_DEV void init() { t[0] = kEmpty; n[0] = kNone; size = 0; }   // further pairs are cleared when the list grows into them
   BPSX_DEV void clear_pair(int k) { t[k] = kEmpty; n[k] = kNone; }
@@ -386,62 +227,21 @@ struct OpenList {
 struct AstarState {
   int lastBest;      // the goal's node once it has been popped
   bool outOfNodes;
-  RegHeap rh;        // the reference's heap: always (exact loops), or as of log record `synced` (sorted-list loop)
   OpenList ol;
   int logEnd;        // records in the slot's operation log
-  int synced;        // records already applied to rh
+  int synced;        // records already applied to the replay's heap
+  int replaySize;    // entries of that heap, which the slot keeps between replays
+  uint32_t replayRoot;   // packed node of the entry at its root after a replay
 };
 
-// Applies log records [st.synced, st.logEnd) to the reference's heap, pass by pass.  Records are
-// fetched 64 at a time, one per lane, and again when the next pass is not among them in full
-// (a pass has at most 1 + 8 * 6 records).  False when the heap
-// outgrows the registers.
-BPSX_DEV bool replay_log(const OpRec* log, AstarState& st, int lane) {
-  RegHeap& rh = st.rh;
-  int base = -64;              // record held by lane 0
-  uint32_t rk = 0, rw = 0;
-  auto fetch = [&](int from) {
-    base = from;
-    rk = 0; rw = 0;
-    if (base + lane < st.logEnd) { const OpRec r = log[base + lane]; rk = r.key; rw = r.word; }
-  };
-  for (int pos = st.synced; pos < st.logEnd;) {
-    // a fetch is a round trip to HBM: one only when the pass at hand is not all there
-    if (pos >= base + 64) fetch(pos);
-    if (pos - base + 1 + (int)(rlane(rk, pos - base) >> 8) > 64) fetch(pos);
-    const int h = pos - base;
-    const uint32_t hk = rlane(rk, h), hw = rlane(rw, h);
-    const int c = (int)(hk & 0xffu), nrec = (int)(hk >> 8);
-    // rows in the reference's order: the first two swap when the heap has row 1's node on top
-    const bool swap = (hw & kOpUnordered) && rlane(rh.n0, 1) != (hw & 0x3ffffffu);
-    const bool mine = lane > h && lane <= h + nrec;
-    const int myRow = (int)((rw >> 26) & 7u);
-    for (int i = 0; i < c; ++i) {
-      const int row = (swap && i < 2) ? 1 - i : i;
-      rh.pop(lane);
-      unsigned long long m = lanes_where(mine && myRow == row);
-      while (m) {
-        const int j = __ffsll((long long)m) - 1;
-        m &= m - 1;
-        const uint32_t key = rlane(rk, j), word = rlane(rw, j);
-        const uint32_t node = word & 0x3ffffffu;
-        // a node seen as open whose entry has left (its row came earlier in the pass) is pushed
-        int q = ((word >> 29) & 1u) ? rh.position(node, lane) : 0;
-        if (!q) {
-          if (rh.size >= kRegHeap) return false;
-          q = ++rh.size;
-        }
-        rh.bubble_up(q, key, node, lane);
-      }
-    }
-    pos += 1 + nrec;
-  }
-  st.synced = st.logEnd;
-  return true;
-}
 enum AstarExit { kAstarEmpty = 0, kAstarGoal = 1, kAstarGrowLinks = 2, kAstarGrowHeap = 3, kAstarTie = 4, kAstarLogFull = 5 };
 
-// Two roots at once: one test of the arguments' range for both.
+// Two correctly rounded square roots, the values sqrtf returns on the host: the hardware estimate is
+// within one unit in the last place, and the residuals of its two neighbours say which of the
+// three is the rounded root.  Same scheme as the compiler's own expansion of sqrtf, minus its
+// rescaling of arguments below 2^-96 (needed there for the residuals not to underflow): the
+// arguments here are squared distances, zero or far above that; a wavefront that meets one in
+// between takes the library routine.  One test of the arguments' range for both.
 BPSX_DEV void sqrt_exact2(float x, float y, float* rx, float* ry) {
   const uint32_t xb = __float_as_uint(x), yb = __float_as_uint(y);
   if (__builtin_expect(lanes_where(xb - 1u < 0x0f800000u - 1u || yb - 1u < 0x0f800000u - 1u) != 0, 0)) {
@@ -481,14 +281,10 @@ namespace BPSX_GEO_NS {
 #ifndef BPSX_LINKS_LDS
 #define BPSX_LINKS_LDS 1016
 #endif
-#ifndef BPSX_HEAP_LDS
-#define BPSX_HEAP_LDS 32
-#endif
 #ifndef BPSX_WINDOW
 #define BPSX_WINDOW 128
 #endif
 constexpr int kLinksLds = BPSX_LINKS_LDS;   // nodes whose link word is kept in LDS
-constexpr int kHeapLds = BPSX_HEAP_LDS;     // entries of an open list that has left the registers kept in LDS (its top levels)
 constexpr int kWindow = BPSX_WINDOW;        // most recent nodes whose position/cost/total are kept in LDS
 #ifndef BPSX_HASH
 #define BPSX_HASH 512
@@ -509,10 +305,7 @@ static_assert((kWindow & (kWindow - 1)) == 0 && kWindow >= 2 * kNvp, "window mus
 // LDS of one wavefront.
 struct GeoLds {
   uint16_t first[kHashSize];
-  union {
-    HeapEntry heap[kHeapLds];      // open list once it has left the registers
-    uint16_t w_parent[kWindow];    // until then: 1-based parent index of the window's nodes
-  };
+  uint16_t w_parent[kWindow];      // 1-based parent index of the window's nodes
   uint32_t n_link[kLinksLds];      // polygon index (bits 0-14) | flags (bits 15-16: 1 open, 2 closed) | next node of the hash chain << 20
   float w_total[kWindow];
   float w_cost[kWindow];
@@ -527,39 +320,38 @@ struct FunnelLds {
   uint16_t pad[kHashSize - kMaxPath];
   float portals[kMaxPath][6];
 };
-static_assert(offsetof(FunnelLds, portals) == offsetof(GeoLds, heap), "corridor must overlay the hash heads only");
+static_assert(offsetof(FunnelLds, portals) == offsetof(GeoLds, w_parent), "corridor must overlay the hash heads only");
 union GeoShared {
   GeoLds a;
   FunnelLds f;
 };
 
-// Accessors take the instantiation's spill switch S: with S false every node index is below
-// kLinksLds and every heap index below kHeapLds, and no address-space branch is generated.
+// Accessors take the instantiation's spill switch S: with S false, or with room in LDS for the links
+// of all nodes, every node index is below kLinksLds and no address-space branch is generated.
 struct GeoWave {
   GeoLds* L;
   GeoSlot* ws;
   int lane;
-  int heapSize;
   int nodeCount;
-  uint32_t linkSpills, heapSpills;   // queries that left the LDS links / the register heap
+  uint32_t linkSpills, heapSpills;   // queries that left the LDS links / whose open list left the registers
   uint32_t tagNow;                   // mark of the current pass in L->tag, counting down
 #ifdef BPSX_PHASE_TIMING
   unsigned long long phase[8], phase_t0;
 #endif
-  uint32_t exactRuns;                // queries run again with the exact heap
+  uint32_t exactRuns;                // queries that went on with the reference's heap
   uint32_t tieReplays;               // ties resolved by replaying the operation log through the exact heap
   uint32_t pairTies;                 // passes that took two nodes of equal total in one go
 
   // ---------------------------------------------------------------- node pool
   template <bool S> BPSX_DEV uint32_t link(int i) const {
-    if (!S || i < kLinksLds) return L->n_link[i];
+    if (!S || kLinksLds >= kMaxNodes || i < kLinksLds) return L->n_link[i];
     BPSX_KEEP_APART();
     const uint32_t v = ws->nodes[i].link;
     BPSX_KEEP_APART();
     return v;
   }
   template <bool S> BPSX_DEV void set_link(int i, uint32_t v) const {
-    if (!S || i < kLinksLds) L->n_link[i] = v;
+    if (!S || kLinksLds >= kMaxNodes || i < kLinksLds) L->n_link[i] = v;
     else { BPSX_KEEP_APART(); ws->nodes[i].link = v; BPSX_KEEP_APART(); }
   }
   // node i still has its position/cost/total in LDS
@@ -570,11 +362,13 @@ struct GeoWave {
     asm("v_mul_u32_u24 %0, %1, %2" : "=v"(m) : "v"(ip), "s"(0x9e3779u));
     return (m >> 9) & (kHashSize - 1);
   }
-  BPSX_DEV void clear() {
-    for (int i = lane; i < kHashSize; i += 64) L->first[i] = (uint16_t)kChainEnd;
+  BPSX_DEV void clear_marks() {
     for (int i = lane; i < kTagSlots; i += 64) L->tag[i] = 0xffffffffu;
     tagNow = 0x1fffffffu;
-    heapSize = 0;
+  }
+  BPSX_DEV void clear() {
+    for (int i = lane; i < kHashSize; i += 64) L->first[i] = (uint16_t)kChainEnd;
+    clear_marks();
     nodeCount = 0;
     wave_sync();
   }
@@ -599,407 +393,239 @@ struct GeoWave {
     *hlink = fl;
     return found;
   }
+};
 
-  // ---------------------------------------------------------------- open list, once it has
-  // left the registers (more than kRegHeap entries: rare)
-  // The heap is walked with wave-uniform indices: every lane issues the same LDS access and the
-  // values are moved to scalar registers, so the loops below branch on the scalar unit and cost
-  // a handful of vector instructions per level.
-  template <bool S> BPSX_DEV HeapEntry hget(int i) const {
-    if (!S || i < kHeapLds) return L->heap[i];
-    BPSX_KEEP_APART();
-    const HeapEntry e = ws->heap_spill[i];
-    BPSX_KEEP_APART();
-    return e;
+// The reference's heap (dtNodeQueue, DetourNode.cpp:150-200), needed when the sorted list cannot say
+// what comes first (a tie) or cannot hold what is open: position q (root = 1) in entry q of an array
+// in LDS, over the window's arrays and the conflict marks, or in the wavefront's slot.  All lanes
+// work on one operation: a pop takes one round of accesses per five levels, a push one.
+// (A heap in registers, entry q in lane q mod 64, held 127 entries; one search in seven hundred over
+// a cluttered plan of 20k polygons ties with a longer list or outgrows the sorted list, and ran
+// again from its start with a heap walked level by level in HBM: 6.6 ms, against 1.5 ms for the
+// longest of the others.)
+constexpr int kHeapLds = (int)((sizeof(GeoLds) - offsetof(GeoLds, w_total)) / sizeof(uint2)) - 1;
+static_assert(offsetof(GeoLds, w_total) % sizeof(uint2) == 0, "the heap's entries are accessed as 8 bytes");
+static_assert(kHeapLds >= 64 * OpenList::kPairs + 2 * kRows * kNvp, "a heap with as many entries as the sorted list must fit");
+struct RefHeap {
+  uint2* h;    // total bits, packed node
+  int size, lane;
+  uint32_t anc0, anc1;   // as bits, the lane and its ancestors below the root of a subtree with node l in lane l
+  BPSX_DEV RefHeap(uint2* entries, int n, int lane_) : h(entries), size(n), lane(lane_) {
+    unsigned long long a = 0;
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+      if ((lane >> k) >= 2) a |= 1ull << (lane >> k);
+    anc0 = (uint32_t)a; anc1 = (uint32_t)(a >> 32);
   }
-  template <bool S> BPSX_DEV void hset(int i, float t, int n) const {
-    const HeapEntry e{t, (uint32_t)n};
-    if (!S || i < kHeapLds) L->heap[i] = e;   // all lanes store the same value to the same address
-    else if (lane == 0) { BPSX_KEEP_APART(); ws->heap_spill[i] = e; BPSX_KEEP_APART(); }
-  }
-  // dtNodeQueue::bubbleUp from index i with entry (t, n)
-  template <bool S> BPSX_DEV void bubble_up(int i, float t, int n) const {
-    while (i > 0) {
-      const int parent = (i - 1) >> 1;
-      const HeapEntry pe = hget<S>(parent);
-      const float pt = uniform_f(pe.total);
-      if (!(pt > t)) break;
-      hset<S>(i, pt, uniform_i((int)pe.node));
-      i = parent;
-    }
-    hset<S>(i, t, n);
+  // the entry (t, n), on its way up from position q: lane k looks at the ancestor k levels up; those
+  // with a greater total, a run from q upwards, move down one level each
+  BPSX_DEV void bubble_up(int q, uint32_t t, uint32_t n) {
+    const int up = q >> (lane & 31);
+    const bool on = lane >= 1 && lane < 31 && up >= 1;
+    const uint2 e = h[on ? up : 1];
+    wave_sync();
+    const unsigned long long greater = lanes_where(on && e.x > t) >> 1;
+    const int m = __builtin_ctzll(~greater);
+    if (on && lane <= m) h[q >> (lane - 1)] = e;
+    if (lane == 0) h[q >> m] = make_uint2(t, n);
     wave_sync();
   }
-  template <bool S> BPSX_DEV void push(float t, int n) {
-    heapSize++;
-    bubble_up<S>(heapSize - 1, t, n);
-  }
-  template <bool S> BPSX_DEV void modify(int n, float t) const {
-    int found = -1;
-    for (int base = 0; base < heapSize; base += 64) {
+  // where node n's entry is, 0 if it has none
+  BPSX_DEV int position(uint32_t n) const {
+    for (int base = 1; base <= size; base += 64) {
       const int i = base + lane;
-      const unsigned long long m = lanes_where(i < heapSize && (int)hget<S>(i).node == n);
-      if (m) { found = base + (__ffsll((long long)m) - 1); break; }
+      const unsigned long long m = lanes_where(h[i <= size ? i : size].y == n);
+      if (m) { const int q = base + first_lane(m); return q <= size ? q : size; }
     }
-    if (found >= 0) bubble_up<S>(found, t, n);
+    return 0;
   }
-  // dtNodeQueue::pop (the caller has read the root). The reference moves the hole left by the
-  // root down to a leaf along the smaller children and then bubbles the former last entry up
-  // from there; along that route keys never decrease, so the entry ends up above the first
-  // route element that is greater than it: the walk can stop there, nothing below moves.
-  template <bool S> BPSX_DEV void pop() {
-    heapSize--;
-    const int size = heapSize;
-    if (size == 0) return;
-    const HeapEntry lastE = hget<S>(size);
-    const float lt = uniform_f(lastE.total);
-    const int ln = uniform_i((int)lastE.node);
-    int i = 0;
+  // a node that has an entry takes a smaller total (dtNodeQueue::modify), one without gets one (push)
+  BPSX_DEV void update(bool mayHaveEntry, uint32_t t, uint32_t n) {
+    int q = mayHaveEntry ? position(n) : 0;
+    if (!q) q = ++size;
+    bubble_up(q, t, n);
+  }
+  // The root leaves: the hole moves to a leaf along the smaller children (the left one of two
+  // equal), then the former last entry rises from there.  Totals never decrease along that route,
+  // so the entry lands above the first route element greater than it and nothing below moves.
+  BPSX_DEV void pop() {
+    const int depth = 31 - __clz(lane | (lane == 0));
+    uint32_t lt = 0, ln = 0;
+    int root = 1, at = 1;
     for (;;) {
-      const int c = 2 * i + 1;
-      if (c >= size) break;
-      const bool two = c + 1 < size;
-      // odd lanes fetch the right child, even lanes the left one: one LDS instruction
-      const HeapEntry e = hget<S>(c + ((two && (lane & 1)) ? 1 : 0));
-      const float t0 = lane_f(e.total, 0), t1 = lane_f(e.total, 1);
-      const bool right = two && t0 > t1;
-      const float tc = right ? t1 : t0;
-      if (!(tc <= lt)) break;
-      const int nc = right ? lane_i((int)e.node, 1) : lane_i((int)e.node, 0);
-      hset<S>(i, tc, nc);
-      i = c + (right ? 1 : 0);
+      // lane l >= 1: node l of the subtree under `root`, six levels of it; lane 0: the last entry
+      const int pos = lane == 0 ? size : (root << depth) | (lane & ((1 << depth) - 1));
+      const bool there = pos < size;
+      uint2 e = h[pos <= size ? pos : 1];
+      if (root == 1) { lt = rlane(e.x, 0); ln = rlane(e.y, 0); }
+      if (!there) e.x = kEmptyKey;
+      // one comparison with the neighbouring lane says which of two siblings the hole moves to
+      const uint32_t sibling = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)e.x, 0xb1 /* quad_perm:[1,0,3,2] */, 0xf, 0xf, false);
+      constexpr unsigned long long kOdd = 0xaaaaaaaaaaaaaaaaull;
+      const unsigned long long less = lanes_where(e.x < sibling);
+      const unsigned long long greater = ~((less & kOdd) | (~(less >> 1) & ~kOdd));
+      // the hole comes by where neither the node nor one of its ancestors is the greater of its pair
+      const bool take = there && e.x <= lt && ((anc0 & (uint32_t)greater) | (anc1 & (uint32_t)(greater >> 32))) == 0;
+      const int q = 63 - __builtin_clzll(lanes_where(take && lane > 1) | 2ull);   // the deepest that moves up
+      wave_sync();
+      if (take && lane > 1) h[pos >> 1] = e;
+      wave_sync();
+      const int m = 31 - __builtin_clz((uint32_t)q);
+      at = (root << m) | (q & ((1 << m) - 1));
+      if (m < 5 || 2 * at >= size) break;
+      root = at;
     }
-    hset<S>(i, lt, ln);
+    if (lane == 0) h[at] = make_uint2(lt, ln);   // of a heap of one entry: that entry once more, beyond the end
+    size--;
     wave_sync();
   }
 };
 
-// The expansion loop of findPath for an open list that has left the registers (more than
-// kRegHeap entries: an obstacle-free hall does it, the benchmark's mazes and rooms do not): the
-// reference's heap in LDS/HBM, one node per pass, links wherever they are.
-BPSX_DEV AstarExit astar_loop(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops) {
+// Applies log records [st.synced, st.logEnd) to the reference's heap, pass by pass.  Records are
+// fetched 64 at a time, one per lane, and again when the next pass is not among them in full (a
+// pass has at most 1 + 8 * 6 records).  Between replays the slot keeps the heap; during one it lies
+// over the window, which the caller has restored if it goes on with the sorted list.
+BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
+  const int lane = g.lane;
+  const OpRec* log = g.ws->oplog;
+  uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
+  RefHeap rh(reinterpret_cast<uint2*>(g.L->w_total), st.replaySize, lane);
+  wave_sync();
+  for (int i = lane + 1; i <= rh.size; i += 64) rh.h[i] = kept[i];
+  wave_sync();
+  int base = -64;              // record held by lane 0
+  uint32_t rk = 0, rw = 0;
+  auto fetch = [&](int from) {
+    base = from;
+    rk = 0; rw = 0;
+    if (base + lane < st.logEnd) { const OpRec r = log[base + lane]; rk = r.key; rw = r.word; }
+  };
+  for (int pos = st.synced; pos < st.logEnd;) {
+    // a fetch is a round trip to HBM: one only when the pass at hand is not all there
+    if (pos >= base + 64) fetch(pos);
+    if (pos - base + 1 + (int)(rlane(rk, pos - base) >> 8) > 64) fetch(pos);
+    const int h = pos - base;
+    const uint32_t hk = rlane(rk, h), hw = rlane(rw, h);
+    const int c = (int)(hk & 0xffu), nrec = (int)(hk >> 8);
+    // rows in the reference's order: the first two swap when the heap has row 1's node on top
+    const bool swap = (hw & kOpUnordered) && (uint32_t)uniform_i((int)rh.h[1].y) != (hw & 0x3ffffffu);
+    const bool mine = lane > h && lane <= h + nrec;
+    const int myRow = (int)((rw >> 26) & 7u);
+    for (int i = 0; i < c; ++i) {
+      const int row = (swap && i < 2) ? 1 - i : i;
+      rh.pop();
+      unsigned long long m = lanes_where(mine && myRow == row);
+      while (m) {
+        const int j = first_lane(m);
+        m = without_lane(m, j);
+        const uint32_t word = rlane(rw, j);
+        // a node seen as open whose entry has left (its row came earlier in the pass) is pushed
+        rh.update(((word >> 29) & 1u) != 0, rlane(rk, j), word & 0x3ffffffu);
+      }
+    }
+    pos += 1 + nrec;
+  }
+  st.synced = st.logEnd;
+  st.replaySize = rh.size;
+  st.replayRoot = (uint32_t)uniform_i((int)rh.h[1].y);
+  for (int i = lane + 1; i <= rh.size; i += 64) kept[i] = rh.h[i];
+  wave_sync();
+}
+// The window and the marks after something else has used their LDS.
+BPSX_DEV void restore_window(GeoWave& g) {
+  const int from = g.nodeCount > kWindow ? g.nodeCount - kWindow : 0;
+  for (int i = from + g.lane; i < g.nodeCount; i += 64) {
+    const ANode& hn = g.ws->nodes[i];
+    const int w = i & (kWindow - 1);
+    BPSX_KEEP_APART();
+    const float4 pc = *reinterpret_cast<const float4*>(hn.pos);   // pos, cost
+    const float total = hn.total;
+    BPSX_KEEP_APART();
+    g.L->w_pos[0][w] = pc.x; g.L->w_pos[1][w] = pc.y; g.L->w_pos[2][w] = pc.z;
+    g.L->w_cost[w] = pc.w; g.L->w_total[w] = total;
+  }
+  g.clear_marks();
+  wave_sync();
+}
+
+// One node per round with the reference's heap as it is: what a search goes on with when its open
+// list outgrows the sorted form's registers or its log is full.  The nodes' bodies are read from
+// the slot (the heap lies over the window).  Lds: the heap is in LDS, and the loop ends with
+// kAstarGrowHeap before it outgrows it; otherwise it is in the slot, which holds any heap.
+template <bool Lds>
+BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops) {
   const int lane = g.lane;
   GeoLds* L = g.L;
+  ANode* nodes = g.ws->nodes;
   const float H_SCALE = 0.999f;
-  const float e0 = endPos[0], e1 = endPos[1], e2 = endPos[2];
-  endIp = (uint32_t)uniform_i((int)endIp);   // the same in all lanes: the goal test stays on the scalar unit
-  constexpr bool S = true;    // links and states may be in HBM
-  while (g.heapSize > 0) {
-    // the node about to be popped is the root: fetch its edges while the heap is repaired
-    const int bi = uniform_i((int)L->heap[0].node);
-    const uint32_t blink = g.link<S>(bi);   // the node's link word: closing the node rewrites its flags
-    const uint32_t bestIp = link_id((uint32_t)uniform_i((int)blink));
+  RefHeap rh(Lds ? reinterpret_cast<uint2*>(L->w_total) : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
+  for (;;) {
+    st.replaySize = rh.size;
+    if (rh.size <= 0) return kAstarEmpty;
+    if (Lds && rh.size > kHeapLds - kNvp) return kAstarGrowHeap;
+    const uint32_t front = (uint32_t)uniform_i((int)rh.h[1].y);
+    const int bi = (int)(front & 0x7ffu);
+    const uint32_t bestIp = front >> 11;
+    rh.pop();
+    if (bestIp == endIp) { st.lastBest = bi; return kAstarGoal; }
+    (*pops)++;
     uint32_t nb = kNoNb;
     float m0 = 0, m1 = 0, m2 = 0;
     if (lane < kNvp) {
-      const AEdge e = edges[bestIp * kEdgeStride + lane];
+      const AEdge e = edges[bestIp * kEdgeStride + (uint32_t)lane];
       nb = e.nb; m0 = e.mid[0]; m1 = e.mid[1]; m2 = e.mid[2];
     }
-    float b0, b1, b2, bcost;
-    uint32_t bparent;   // read now, moved to a scalar register only after the pop
-    if (g.in_window(bi)) {
-      const int w = bi & (kWindow - 1);
-      b0 = L->w_pos[0][w]; b1 = L->w_pos[1][w]; b2 = L->w_pos[2][w]; bcost = L->w_cost[w];
-      BPSX_KEEP_APART(); bparent = g.ws->nodes[bi].parent; BPSX_KEEP_APART();   // the heap lies over the window's parent indices
-    } else {
-      BPSX_KEEP_APART();
-      const float4 pc = *reinterpret_cast<const float4*>(g.ws->nodes[bi].pos);   // pos, cost
-      b0 = pc.x; b1 = pc.y; b2 = pc.z; bcost = pc.w;
-      bparent = g.ws->nodes[bi].parent;
-      BPSX_KEEP_APART();
-    }
-    g.pop<S>();
-    const uint32_t pidx = (uint32_t)uniform_i((int)bparent);
-    g.set_link<S>(bi, with_flags(blink, 2u));   // open -> closed
-    if (bestIp == endIp) { st.lastBest = bi; return kAstarGoal; }
-    (*pops)++;
+    const float4 b = *reinterpret_cast<const float4*>(nodes[bi].pos);   // pos, cost
+    const uint32_t bparent = nodes[bi].parent;
     const uint32_t bucket = GeoWave::hash(nb);
     uint32_t chainHead, hitLink;
-    int ni = g.find<S>(nb != kNoNb, nb, bucket, &chainHead, &hitLink);
-    // the polygon the expanded node was reached from is not entered again
-    if (pidx && ni + 1 == (int)pidx) nb = kNoNb;
-    // new nodes take consecutive indices in edge order
-    const bool isNew = nb != kNoNb && ni < 0;
-    const unsigned long long need = lanes_where(isNew);
-    if (need) {
-      const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0u));
-      const int count = __popcll(need);
-      const int want = g.nodeCount + count;
-      // the reference carries on without the nodes that do not fit, but reports anything found
-      // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): the search can stop
-      if (want > kMaxNodes) { st.outOfNodes = true; return kAstarEmpty; }
-      if (isNew) ni = g.nodeCount + rank;
-      g.nodeCount = want;
-      bool pending = isNew;
-      // All insert at once in front of the chain head their lookup saw.  Of several that share a
-      // bucket one store wins; the others see that when they read the head back and go round
-      // again behind the winner.  One new node needs no check.  A new node is open from the
-      // start: the cost computation below always takes it.
-      uint32_t head = chainHead;
-      for (;;) {
-        if (pending) {
-          g.set_link<S>(ni, make_link(nb, 1u, head));
-          L->first[bucket] = (uint16_t)ni;
-        }
-        wave_sync();
-        if (count == 1) break;
-        if (pending) {
-          head = L->first[bucket];
-          pending = head != (uint32_t)ni;
-        }
-        wave_sync();
-        if (!lanes_where(pending)) break;
-      }
-    }
-    // Costs of the step to each neighbour (lane-wise).  Written with few branches: all lanes
-    // issue the one round of LDS reads a revisited node needs (idle lanes read slot 0; its flags
-    // came with the lookup), the rare node that has left the window is fetched under a
-    // wave-uniform test, new nodes take the portal midpoint instead, and everything is stored
-    // in one predicated block.
+    int ni = g.find<true>(nb != kNoNb, nb, bucket, &chainHead, &hitLink);
+    if (bparent && ni + 1 == (int)bparent) nb = kNoNb;   // the polygon the node was reached from is not entered again
     const bool valid = nb != kNoNb;
-    const int nis = valid ? ni : 0;
-    const int w = nis & (kWindow - 1);
-    const bool inw = g.in_window(nis);   // new nodes always are
-    ANode& hn = g.ws->nodes[nis];
-    uint32_t fl = link_flags(hitLink);
-    float p0 = L->w_pos[0][w], p1 = L->w_pos[1][w], p2 = L->w_pos[2][w], oldTotal = L->w_total[w];
-    const bool miss = valid && !isNew && !inw;
-    if (lanes_where(miss)) {
-      if (miss) {
-        BPSX_KEEP_APART();
-        const float4 pc = *reinterpret_cast<const float4*>(hn.pos);     // pos, cost
-        p0 = pc.x; p1 = pc.y; p2 = pc.z; oldTotal = hn.total;
-        BPSX_KEEP_APART();
-      }
+    const bool known = valid && ni >= 0;
+    float oldTotal = 0;
+    if (known) {
+      const float4 pc = *reinterpret_cast<const float4*>(nodes[ni].pos);
+      m0 = pc.x; m1 = pc.y; m2 = pc.z; oldTotal = nodes[ni].total;
     }
-    if (isNew) { p0 = m0; p1 = m1; p2 = m2; fl = 0; }
-    // both square roots in one pass: lanes 8..13 take the second operand of lanes 0..5
-    const float cx = p0 - b0, cy = p1 - b1, cz = p2 - b2;
-    const float ex = e0 - p0, ey = e1 - p1, ez = e2 - p2;
-    const float cc = cx * cx + cy * cy + cz * cz, ee = ex * ex + ey * ey + ez * ez;
-    const float roots = sqrt_exact(lanes_up8(cc, ee));
-    const float curCost = roots * 1.0f;
-    const float toEnd = lanes_down8(roots);
+    const float cx = m0 - b.x, cy = m1 - b.y, cz = m2 - b.z;
+    const float ex = endPos[0] - m0, ey = endPos[1] - m1, ez = endPos[2] - m2;
+    float curCost, toEnd;
+    sqrt_exact2(cx * cx + cy * cy + cz * cz, ex * ex + ey * ey + ez * ez, &curCost, &toEnd);
     const bool last = nb == endIp;
-    const float cost = last ? bcost + curCost + toEnd * 1.0f : bcost + curCost;
-    const float heuristic = last ? 0.0f : toEnd * H_SCALE;
-    const float total = cost + heuristic;
-    const bool update = valid && !(fl && total >= oldTotal);
-    const bool wasOpen = update && (fl & 1u) != 0;
-    if (update) {
-      if (!isNew) g.set_link<S>(ni, with_flags(hitLink, 1u));   // open (again)
-      if (inw) {
-        L->w_pos[0][w] = p0; L->w_pos[1][w] = p1; L->w_pos[2][w] = p2;   // unchanged for a revisited node
-        L->w_cost[w] = cost; L->w_total[w] = total;
+    const float cost = last ? b.w + curCost * 1.0f + toEnd * 1.0f : b.w + curCost * 1.0f;
+    const float total = cost + (last ? 0.0f : toEnd * H_SCALE);
+    const bool update = valid && !(known && total >= oldTotal);
+    // new nodes take consecutive indices in edge order; those that share a bucket are chained one after the other
+    unsigned long long fresh = lanes_where(update && !known);
+    const int want = g.nodeCount + __popcll(fresh);
+    if (want > kMaxNodes) { st.outOfNodes = true; return kAstarEmpty; }   // reported as failure whatever follows
+    if (update && !known) ni = g.nodeCount + (int)__builtin_amdgcn_mbcnt_lo((uint32_t)fresh, 0u);
+    g.nodeCount = want;
+    while (fresh) {
+      const int src = first_lane(fresh);
+      fresh = without_lane(fresh, src);
+      if (lane == src) {
+        g.set_link<true>(ni, make_link(nb, 1u, L->first[bucket]));
+        L->first[bucket] = (uint16_t)ni;
       }
-      *reinterpret_cast<float4*>(hn.pos) = make_float4(p0, p1, p2, cost);
-      *reinterpret_cast<uint2*>(&hn.total) = make_uint2(__float_as_uint(total), (uint32_t)(bi + 1));   // total, parent = expanded node
+      wave_sync();
+    }
+    if (update) {
+      ANode& hn = nodes[ni];
+      *reinterpret_cast<float4*>(hn.pos) = make_float4(m0, m1, m2, cost);
+      *reinterpret_cast<uint2*>(&hn.total) = make_uint2(__float_as_uint(total), (uint32_t)bi + 1u);
       g.ws->parents[ni] = (uint16_t)(bi + 1);
     }
     wave_sync();
-    // ---- ordered phase, in edge order: the open list.  (findPath's "nearest so far" record,
-    // lastBestNode, is not kept: it only matters to a search that ends without reaching the
-    // goal, and the caller reports DT_PARTIAL_RESULT as failure, PathFinder.cpp:506.)
-    unsigned long long upd = lanes_where(update);
-    const unsigned long long openMask = lanes_where(wasOpen);
-    while (upd) {
-      const int src = __ffsll((long long)upd) - 1;
-      upd &= upd - 1;
-      const int node = (int)rlane((uint32_t)ni, src);
-      const float t = lane_f(total, src);
-      if ((openMask >> src) & 1ull) g.modify<S>(node, t);
-      else g.push<S>(t, node);
-    }
-  }
-  return kAstarEmpty;
-}
-
-// The same loop for an open list in registers (S as above), two nodes per pass.  Besides the
-// node at the root (A, lanes 0..5) the pass works on the smaller child of the root (B, lanes
-// 16..21), which is what the reference pops next unless A's expansion puts something smaller
-// on the list: the edge records of both arrive in one load, and node lookup, costs, node
-// creation and stores of both are done by the same instructions.  B's results are computed
-// from the state before A's expansion; they are what the reference computes after it when
-//   - every total A puts on the open list is at least B's (B stays at the root: an entry
-//     moves past its parent only when its key is smaller),
-//   - A created or updated no node that B read (a neighbour of both) and not B's own node
-//     (A's own node is closed before either looks anything up, as it is when B's turn comes),
-// and B is not the goal.  Then the pass applies A's and B's updates in the reference's order:
-// new nodes take consecutive indices, A's first; the "nearest so far" record and the open
-// list see A's updates in edge order, then B's pop, then B's updates.  Otherwise B's lanes
-// are dropped and B becomes A of the next pass.
-template <bool S, bool W>
-BPSX_DEV AstarExit astar_loop2(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops) {
-  const int lane = g.lane;
-  GeoLds* L = g.L;
-  const float H_SCALE = 0.999f;
-  const float e0 = endPos[0], e1 = endPos[1], e2 = endPos[2];
-  endIp = (uint32_t)uniform_i((int)endIp);
-  RegHeap& rh = st.rh;
-  const bool rowB = lane >= 16;
-  const int el = lane & 15;                      // edge handled by this lane
-  const bool edgeLane = el < kNvp && lane < 32;
-  while (rh.size > 0) {
-    if (!S && g.nodeCount > kLinksLds - 2 * kNvp) return kAstarGrowLinks;
-    if (rh.size > (W ? kRegHeap : 63) - 2 * kNvp) return kAstarGrowHeap;   // W false: all entries in the first register pair
-    const uint32_t rootA = rlane(rh.n0, 1);
-    const int biA = (int)(rootA & 0x7ffu);
-    const uint32_t ipA = rootA >> 11;
-    const uint32_t kl = rlane(rh.t0, 2), kr = rlane(rh.t0, 3);   // kEmpty past the end
-    const uint32_t nl = rlane(rh.n0, 2), nr = rlane(rh.n0, 3);
-    const uint32_t rootB = kr < kl ? nr : nl;
-    const uint32_t keyB = kr < kl ? kr : kl;
-    const int biB = (int)(rootB & 0x7ffu);
-    const uint32_t ipB = rootB >> 11;
-    const bool spec = rh.size >= 2 && ipA != endIp && ipB != endIp;
-    const uint32_t blinkA = g.link<S>(biA);
-    const uint32_t blinkB = g.link<S>(spec ? biB : biA);   // unchanged by A whenever B is committed
-    const bool act = edgeLane && (!rowB || spec);
-    const int bi = (rowB && spec) ? biB : biA;   // the node this lane expands
-    uint32_t nb = kNoNb;
-    float m0 = 0, m1 = 0, m2 = 0;
-    if (act) {
-      const AEdge e = edges[(rowB ? ipB : ipA) * kEdgeStride + (uint32_t)el];
-      nb = e.nb; m0 = e.mid[0]; m1 = e.mid[1]; m2 = e.mid[2];
-    }
-    float b0, b1, b2, bcost;
-    uint32_t bparent;
-    {
-      const int w = bi & (kWindow - 1);
-      const bool binw = g.in_window(bi);
-      b0 = L->w_pos[0][w]; b1 = L->w_pos[1][w]; b2 = L->w_pos[2][w]; bcost = L->w_cost[w];
-      bparent = L->w_parent[w];
-      if (lanes_where(!binw)) {
-        if (!binw) {
-          BPSX_KEEP_APART();
-          const float4 pc = *reinterpret_cast<const float4*>(g.ws->nodes[bi].pos);   // pos, cost
-          b0 = pc.x; b1 = pc.y; b2 = pc.z; bcost = pc.w;
-          bparent = g.ws->nodes[bi].parent;
-          BPSX_KEEP_APART();
-        }
-      }
-    }
-    rh.template pop<W>(lane);
-    g.set_link<S>(biA, with_flags(blinkA, 2u));   // open -> closed
-    if (ipA == endIp) { st.lastBest = biA; return kAstarGoal; }
-    (*pops)++;
-    const uint32_t bucket = GeoWave::hash(nb);
-    uint32_t chainHead, hitLink;
-    int ni = g.find<S>(nb != kNoNb, nb, bucket, &chainHead, &hitLink);
-    // the polygon the expanded node was reached from is not entered again
-    if (bparent && ni + 1 == (int)bparent) nb = kNoNb;
-    // ---- costs of both nodes' steps (new nodes have no index yet and read slot 0)
-    const bool isNew = nb != kNoNb && ni < 0;
-    const bool valid = nb != kNoNb;
-    const int nis = (valid && !isNew) ? ni : 0;
-    const int rw = nis & (kWindow - 1);
-    uint32_t fl = link_flags(hitLink);
-    float p0 = L->w_pos[0][rw], p1 = L->w_pos[1][rw], p2 = L->w_pos[2][rw], oldTotal = L->w_total[rw];
-    const bool miss = valid && !isNew && !g.in_window(nis);
-    if (lanes_where(miss)) {
-      if (miss) {
-        const ANode& hn = g.ws->nodes[nis];
-        BPSX_KEEP_APART();
-        const float4 pc = *reinterpret_cast<const float4*>(hn.pos);     // pos, cost
-        p0 = pc.x; p1 = pc.y; p2 = pc.z; oldTotal = hn.total;
-        BPSX_KEEP_APART();
-      }
-    }
-    if (isNew) { p0 = m0; p1 = m1; p2 = m2; fl = 0; }
-    const float cx = p0 - b0, cy = p1 - b1, cz = p2 - b2;
-    const float ex = e0 - p0, ey = e1 - p1, ez = e2 - p2;
-    const float cc = cx * cx + cy * cy + cz * cz, ee = ex * ex + ey * ey + ez * ez;
-    const float roots = sqrt_exact(lanes_up8(cc, ee));
-    const float curCost = roots * 1.0f;
-    const float toEnd = lanes_down8(roots);
-    const bool last = nb == endIp;
-    const float cost = last ? bcost + curCost + toEnd * 1.0f : bcost + curCost;
-    const float heuristic = last ? 0.0f : toEnd * H_SCALE;
-    const float total = cost + heuristic;
-    bool update = valid && !(fl && total >= oldTotal);
-    // ---- does B stand?
-    bool two = false;
-    if (spec) {
-      const uint32_t anb = (update && !rowB) ? nb : kNoNb;   // a lane of A that updates nothing leaves its node as B saw it
-      const uint32_t bnb = (valid && rowB) ? nb : kNoNb - 1u;   // never equal to anb of an idle lane
-      uint32_t clash = (uint32_t)(!rowB && update) & ((uint32_t)(__float_as_uint(total) < keyB) | (uint32_t)(nb == ipB));
-#pragma unroll
-      for (int j = 0; j < kNvp; ++j) clash |= (uint32_t)(bnb == rlane(anb, j));
-      two = !lanes_where(clash != 0);
-    }
-    update = update & (!rowB | two);   // B's lanes are dropped unless B stands
-    const bool wasOpen = update && (fl & 1u) != 0;
-    // ---- new nodes take consecutive indices in edge order, A's before B's
-    {
-      const bool mine = isNew && update;   // a new node is always taken
-      const unsigned long long need = lanes_where(mine);
-      if (need) {
-        const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0u));
-        const int count = __popcll(need);
-        const int want = g.nodeCount + count;
-        // the reference carries on without the nodes that do not fit, but reports anything found
-        // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): stop
-        if (S && want > kMaxNodes) { st.outOfNodes = true; return kAstarEmpty; }
-        if (mine) ni = g.nodeCount + rank;
-        g.nodeCount = want;
-        // All insert at once in front of the chain head their lookup saw.  Of several that share a
-        // bucket one store wins; the others see that when they read the head back and go round
-        // again behind the winner.  One new node needs no check.
-        bool pending = mine;
-        uint32_t head = chainHead;
-        for (;;) {
-          if (pending) {
-            g.set_link<S>(ni, make_link(nb, 1u, head));
-            L->first[bucket] = (uint16_t)ni;
-          }
-          wave_sync();
-          if (count == 1) break;
-          if (pending) {
-            head = L->first[bucket];
-            pending = head != (uint32_t)ni;
-          }
-          wave_sync();
-          if (!lanes_where(pending)) break;
-        }
-      }
-    }
-    if (update) {
-      ANode& hn = g.ws->nodes[ni];
-      const int w = ni & (kWindow - 1);
-      const uint32_t parent = (uint32_t)bi + 1u;
-      if (!isNew) g.set_link<S>(ni, with_flags(hitLink, 1u));   // open (again)
-      if (g.in_window(ni)) {
-        L->w_pos[0][w] = p0; L->w_pos[1][w] = p1; L->w_pos[2][w] = p2;
-        L->w_cost[w] = cost; L->w_total[w] = total;
-        L->w_parent[w] = (uint16_t)parent;
-      }
-      *reinterpret_cast<float4*>(hn.pos) = make_float4(p0, p1, p2, cost);
-      *reinterpret_cast<uint2*>(&hn.total) = make_uint2(__float_as_uint(total), parent);
-      g.ws->parents[ni] = (uint16_t)parent;
-    }
-    wave_sync();
-    // ---- ordered phase, in the reference's order: A's lanes come before B's.  (findPath's
-    // "nearest so far" record, lastBestNode, is not kept: it only matters to a search that ends
-    // without reaching the goal, which the caller reports as failure, PathFinder.cpp:506.)
     const uint32_t packed = (uint32_t)ni | (nb << 11);
-    const unsigned long long upd = lanes_where(update);
-    const unsigned long long openMask = lanes_where(wasOpen);
-    auto apply = [&](unsigned long long m) {
-      while (m) {
-        const int src = __ffsll((long long)m) - 1;
-        m &= m - 1;
-        rh.template update<W>((openMask >> src) & 1ull, rlane(packed, src), __float_as_uint(lane_f(total, src)), lane);
-      }
-    };
-    apply(upd & 0xffffull);
-    if (two) {   // A's updates are in: B leaves the open list
-      rh.template pop<W>(lane);
-      g.set_link<S>(biB, with_flags(blinkB, 2u));
-      (*pops)++;
-      apply(upd & ~0xffffull);
+    const unsigned long long was = lanes_where(known);
+    for (unsigned long long upd = lanes_where(update); upd;) {
+      const int src = first_lane(upd);
+      upd = without_lane(upd, src);
+      rh.update(((was >> src) & 1ull) != 0, __float_as_uint(lane_f(total, src)), rlane(packed, src));
     }
   }
-  return kAstarEmpty;
 }
 
 // The expansion loop with the open list as a sorted array (OpenList), up to kRows nodes per
@@ -1229,7 +855,11 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
         const int want = g.nodeCount + count;
         // the reference carries on without the nodes that do not fit, but reports anything found
         // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): stop
-        if (S && want > kMaxNodes) { st.outOfNodes = true; return kAstarEmpty; }
+        if (S && want > kMaxNodes) {
+          if (kLinksLds >= kMaxNodes) g.linkSpills++;   // where the LDS holds the links of a full pool: a search that needs more than those
+          st.outOfNodes = true;
+          return kAstarEmpty;
+        }
         if (isNew) ni = g.nodeCount + rank;
         g.nodeCount = want;
         bool pending = isNew;
@@ -1309,113 +939,83 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   }
   AstarState st;
   const AEdge* edges = nav.aedges + (size_t)(uint32_t)uniform_i((int)s.poly_base) * kEdgeStride;
-#define ASTAR_ARGS g, st, edges, endIp, endPos, pops
-  const uint32_t pops0 = *pops;
-  AstarExit ex;
-  bool exact = false;   // first with the sorted open list; with the exact loops when that cannot go on
-  for (;;) {
-    g.clear();
-    const float dx = endPos[0] - startPos[0], dy = endPos[1] - startPos[1], dz = endPos[2] - startPos[2];
-    const float total = sqrtf(dx * dx + dy * dy + dz * dz) * 0.999f;
-    g.nodeCount = 1;
-    if (lane == 0) {
-      GeoLds* L = g.L;
-      ANode& hn = g.ws->nodes[0];
-      for (int k = 0; k < 3; ++k) { L->w_pos[k][0] = startPos[k]; hn.pos[k] = startPos[k]; }
-      L->w_cost[0] = 0; L->w_total[0] = total;
-      hn.cost = 0; hn.total = total;
-      hn.parent = 0;
-      g.ws->parents[0] = 0;
-      L->w_parent[0] = 0;
-      L->n_link[0] = make_link(startIp, 1u, kChainEnd);   // open
-      L->first[GeoWave::hash(startIp)] = 0;
-    }
-    wave_sync();
-    st.lastBest = 0;
-    st.outOfNodes = false;
-    st.rh.init(lane);
-    st.rh.push(__float_as_uint(total), startIp << 11, lane);
-    bool spill = false, wide = false;
-    if (!exact) {
+  g.clear();
+  const float dx = endPos[0] - startPos[0], dy = endPos[1] - startPos[1], dz = endPos[2] - startPos[2];
+  const float total = sqrtf(dx * dx + dy * dy + dz * dz) * 0.999f;
+  g.nodeCount = 1;
+  if (lane == 0) {
+    GeoLds* L = g.L;
+    ANode& hn = g.ws->nodes[0];
+    for (int k = 0; k < 3; ++k) { L->w_pos[k][0] = startPos[k]; hn.pos[k] = startPos[k]; }
+    L->w_cost[0] = 0; L->w_total[0] = total;
+    hn.cost = 0; hn.total = total;
+    hn.parent = 0;
+    g.ws->parents[0] = 0;
+    L->w_parent[0] = 0;
+    L->n_link[0] = make_link(startIp, 1u, kChainEnd);   // open
+    L->first[GeoWave::hash(startIp)] = 0;
+    reinterpret_cast<uint2*>(g.ws->heap_spill)[1] = make_uint2(__float_as_uint(total), startIp << 11);
+  }
+  wave_sync();
+  st.lastBest = 0;
+  st.outOfNodes = false;
+  st.logEnd = st.synced = 0;
+  st.replaySize = 1;
 #ifdef BPSX_PHASE_TIMING
-      g.phase_t0 = __builtin_readcyclecounter();
+  g.phase_t0 = __builtin_readcyclecounter();
 #endif
-      st.ol.init();
-      st.ol.template update<1>(startIp << 11, __float_as_uint(total), lane);
-      st.ol.template count<1>();
-      st.logEnd = st.synced = 0;
-      // the loop is instantiated for links in LDS only or spilling, and for a list within one
-      // register pair or two; a search moves on when one more pass could outgrow what it runs in
-      bool resolved = false, restart = false;
-      int pairs = 1;   // register pairs of the list in use
-      for (;;) {
+  st.ol.init();
+  st.ol.template update<1>(startIp << 11, __float_as_uint(total), lane);
+  st.ol.template count<1>();
+  // the loop is instantiated for links in LDS only or spilling (one instantiation where the LDS
+  // holds all links), and for a list within one register pair, two or four; a search moves on when
+  // one more pass could outgrow what it runs in
+  AstarExit ex;
+  bool resolved = false;
+  bool spill = kLinksLds >= kMaxNodes;
+  int pairs = 1;   // register pairs of the list in use
+  for (;;) {
 #define BPSX_FAST_RUN(SP) (pairs == 1 ? astar_fast<SP, 1>(g, st, edges, endIp, endPos, pops, resolved) : \
                            pairs == 2 ? astar_fast<SP, 2>(g, st, edges, endIp, endPos, pops, resolved) : \
                                         astar_fast<SP, 4>(g, st, edges, endIp, endPos, pops, resolved))
-        ex = spill ? BPSX_FAST_RUN(true) : BPSX_FAST_RUN(false);
+    if constexpr (kLinksLds >= kMaxNodes) ex = BPSX_FAST_RUN(true);
+    else ex = spill ? BPSX_FAST_RUN(true) : BPSX_FAST_RUN(false);
 #undef BPSX_FAST_RUN
-        resolved = false;
-        if (ex == kAstarGrowLinks) { g.linkSpills++; spill = true; continue; }
-        if (ex == kAstarGrowHeap && pairs < OpenList::kPairs) {
-          // the list grows into further registers, empty so far
-          if (pairs == 1) { st.ol.clear_pair(1); pairs = 2; }
-          else { st.ol.clear_pair(2); st.ol.clear_pair(3); pairs = 4; }
-          continue;
-        }
-        // a list beyond the registers or a full log (neither met in the benchmark configurations'
-        // mazes and rooms, both in a hall without obstacles): the search runs again with the exact loops
-        if (ex == kAstarGrowHeap || ex == kAstarLogFull) { restart = true; break; }
-        if (ex != kAstarTie) break;
-        __builtin_amdgcn_s_setprio(3);   // a search that pays for a replay is late from here on
-        // a tie: the reference pops what its heap has at the root, so the heap is brought up to
-        // date from the log, and that entry goes first
-        if (!replay_log(g.ws->oplog, st, lane) || st.rh.size != st.ol.size) { restart = true; break; }
-        g.tieReplays++;
-        const uint32_t root = rlane(st.rh.n0, 1);
-        const unsigned long long at = lanes_where(st.ol.n[0] == root);
-        const int p = at ? __ffsll((long long)at) - 1 : -1;
-        if (p < 0 || rlane(st.ol.t[0], p) != rlane(st.ol.t[0], 0)) { restart = true; break; }
-        const uint32_t front = rlane(st.ol.n[0], 0);
-        st.ol.n[0] = wlane(st.ol.n[0], root, 0);
-        st.ol.n[0] = wlane(st.ol.n[0], front, p);
-        resolved = true;
-      }
-      if (restart) {
-        g.exactRuns++;
-        *pops = pops0;
-        exact = true;
-        continue;
-      }
-      break;
+    resolved = false;
+    if (ex == kAstarGrowLinks) { g.linkSpills++; spill = true; continue; }
+    if (ex == kAstarGrowHeap && pairs < OpenList::kPairs) {
+      // the list grows into further registers, empty so far
+      if (pairs == 1) { st.ol.clear_pair(1); pairs = 2; }
+      else { st.ol.clear_pair(2); st.ol.clear_pair(3); pairs = 4; }
+      continue;
     }
-    {
-      wide = false;
-      for (;;) {
-        if (!spill) ex = wide ? astar_loop2<false, true>(ASTAR_ARGS) : astar_loop2<false, false>(ASTAR_ARGS);
-        else ex = wide ? astar_loop2<true, true>(ASTAR_ARGS) : astar_loop2<true, false>(ASTAR_ARGS);
-        if (ex == kAstarGrowLinks) { g.linkSpills++; spill = true; }
-        else if (ex == kAstarGrowHeap && !wide) wide = true;
-        else break;
-      }
+    if (ex == kAstarEmpty || ex == kAstarGoal) break;
+    __builtin_amdgcn_s_setprio(3);   // a search that pays for a replay is late from here on
+    replay_log(g, st);
+    if (ex == kAstarTie) {
+      // the reference pops what its heap has at the root: that entry goes first
+      restore_window(g);
+      g.tieReplays++;
+      const int p = first_lane(lanes_where(st.ol.n[0] == st.replayRoot));   // among the front's equal totals
+      const uint32_t front = rlane(st.ol.n[0], 0);
+      st.ol.n[0] = wlane(st.ol.n[0], st.replayRoot, 0);
+      st.ol.n[0] = wlane(st.ol.n[0], front, p);
+      resolved = true;
+      continue;
     }
+    // a list beyond the registers or a full log: on with the reference's heap
+    g.exactRuns++;
+    if (ex == kAstarGrowHeap) g.heapSpills++;
+    ex = astar_exact<true>(g, st, edges, endIp, endPos, pops);
     if (ex == kAstarGrowHeap) {
-      g.heapSpills++;
-      // the open list leaves the registers: entry q goes to index q - 1 of the LDS heap
-      const RegHeap& rh = st.rh;
-      auto put = [&](int i, uint32_t t, uint32_t n) {
-        const HeapEntry e{__uint_as_float(t), n & 0x7ffu};
-        if (i < kHeapLds) g.L->heap[i] = e;
-        else { BPSX_KEEP_APART(); g.ws->heap_spill[i] = e; BPSX_KEEP_APART(); }
-      };
-      if (lane >= 1 && lane <= rh.size) put(lane - 1, rh.t0, rh.n0);
-      if (64 + lane <= rh.size) put(63 + lane, rh.t1, rh.n1);
-      g.heapSize = rh.size;
+      uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
+      const uint2* h = reinterpret_cast<const uint2*>(g.L->w_total);
+      for (int i = lane + 1; i <= st.replaySize; i += 64) kept[i] = h[i];
       wave_sync();
-      ex = astar_loop(ASTAR_ARGS);
+      ex = astar_exact<false>(g, st, edges, endIp, endPos, pops);
     }
     break;
   }
-#undef ASTAR_ARGS
   // an open list that ran empty, or a pool that ran out, is DT_PARTIAL_RESULT or
   // DT_OUT_OF_NODES in the reference: no path to build, the result is a failure
   if (ex != kAstarGoal || st.outOfNodes) return 0;

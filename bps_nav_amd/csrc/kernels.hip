@@ -33,12 +33,10 @@
 // whole two-wavefront block (see k_geodesic).
 #undef BPSX_GEO_NS
 #undef BPSX_LINKS_LDS
-#undef BPSX_HEAP_LDS
 #undef BPSX_WINDOW
 #undef BPSX_HASH
 #define BPSX_GEO_NS geo_long
 #define BPSX_LINKS_LDS 2048
-#define BPSX_HEAP_LDS 32
 #define BPSX_WINDOW 256
 #define BPSX_HASH 1024
 #include "geodesic_device.h"
@@ -586,7 +584,6 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
     gl.lane = lane;
     gl.L = &reinterpret_cast<geo_long::GeoShared*>(lds)->a;
     gl.ws = slot;
-    gl.heapSize = 0;
     gl.nodeCount = 0;
     gl.linkSpills = gl.heapSpills = gl.exactRuns = gl.tieReplays = gl.pairTies = 0;
 #ifdef BPSX_PHASE_TIMING
@@ -605,7 +602,6 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
   g.lane = lane;
   g.L = &reinterpret_cast<geo::GeoShared*>(lds + (size_t)half * kHalf)->a;
   g.ws = slot;
-  g.heapSize = 0;
   g.nodeCount = 0;
   g.linkSpills = g.heapSpills = g.exactRuns = g.tieReplays = g.pairTies = 0;
 #ifdef BPSX_PHASE_TIMING
