@@ -128,9 +128,8 @@ struct alignas(16) ANode {
   float pos[3];
   float cost;
   float total;
-  uint32_t parent;  // 1-based index of the node this one was reached from, 0 for the start node
-  uint32_t link;    // polygon index within the scene (bits 0-14) | flags (bits 15-16: 1 open, 2 closed) | next node of the hash chain << 20
-  uint32_t pad;
+  uint32_t link;    // polygon index within the scene | next node of the hash chain << 16
+  uint32_t pad[2];
 };
 static_assert(sizeof(ANode) == 32, "ANode");
 
@@ -145,7 +144,7 @@ struct HeapEntry {
 // geodesic_device.h): per pass one header (key = number of entries popped | number of records
 // that follow << 8, word = kOpHeader) followed by the pass's pushes and modifies in row and
 // edge order (key = total as bits, word = packed node | row of the pass << 26 | 1 << 29 if the
-// node was open).  A header with kOpUnordered says that the pass's first two rows had the same
+// node was known before).  A header with kOpUnordered says that the pass's first two rows had the same
 // total: the reference expanded them in the order its heap had them in, which the replay finds
 // out; the header's low 26 bits then name row 0's node.
 struct OpRec {
@@ -159,7 +158,7 @@ struct alignas(128) GeoSlot {
   ANode nodes[kMaxNodes];
   HeapEntry heap_spill[kMaxNodes];
   OpRec oplog[kOpLogCap];
-  uint16_t parents[kMaxNodes];   // the nodes' parent indices once more, side by side: what the final walk up the path reads
+  uint16_t parents[kMaxNodes];   // per node, 1-based index of the node it was reached from, 0 for the start node: what the final walk up the path reads
 };
 
 struct GeoQuery {
