@@ -141,12 +141,8 @@ struct OpenList {
   int size;
   static constexpr uint32_t kEmpty = kEmptyKey;
   static constexpr uint32_t kNone = 0xffffffffu;    // no packed node looks like this (26 bits)
-  BPSX_DEV void init() { t[0] = kEmpty; n[0] = kNone; size = 0; }   // further pairs are cleared when the list grows into them
+  BPSX_DEV void init(int lane, uint32_t total, uint32_t node) { t[0] = lane ? kEmpty : total; n[0] = lane ? kNone : node; size = 1; }   // further pairs are cleared when the list grows into them
   BPSX_DEV void clear_pair(int k) { t[k] = kEmpty; n[k] = kNone; }
-  // lane L takes v of lane L - 1, lane 0 keeps `first`
-  static BPSX_DEV uint32_t up1(uint32_t first, uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)first, (int)v, 0x138 /* wave_shr:1 */, 0xf, 0xf, false);
-  }
   // lane L takes v of lane L + 1, lane 63 keeps `last`
   static BPSX_DEV uint32_t down1(uint32_t last, uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp((int)last, (int)v, 0x130 /* wave_shl:1 */, 0xf, 0xf, false);
@@ -157,74 +153,87 @@ struct OpenList {
     asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(no), "v"(yes), "s"(mask));
     return r;
   }
-  // The first c entries leave.  P: register pairs in use (64 entries each).
-  template <int P> BPSX_DEV void drop_front(int c, int lane) {
-    if (P == 1) {
-      for (int i = 0; i < c; ++i) { t[0] = down1(kEmpty, t[0]); n[0] = down1(kNone, n[0]); }
-    } else {
-      const int src = ((lane + c) & 63) * 4;
-      uint32_t a[P], b[P];
+  // A pass's changes at once: the first c entries leave, and so does the entry of every node in lanes
+  // `known` that has one (a modify; a node without an entry is pushed); the nodes in lanes `upd`,
+  // packed and with total bits tb, enter behind the entries with totals up to theirs.  P: register
+  // pairs in use (64 entries each).  buf: 128 entries in LDS.
+  // Every entry's new place is counted, then all of them move through LDS: an old entry's place is
+  // the number of entries before it that stay plus that of new totals below its own, a new one's
+  // the number of old entries up to it plus that of new ones before it.  Per new entry that is one
+  // comparison with the old ones and one with the other new ones, and no comparison waits for the one
+  // before.  (One insertion after the other, each a shift of the list behind the place that a
+  // comparison found, is a chain of some ten dependent steps per entry and register pair.)
+  template <int P> BPSX_DEV void merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
+                                       uint32_t packed, int lane) {
+    unsigned long long dead[P];
 #pragma unroll
-      for (int k = 0; k < P; ++k) { a[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)t[k]); b[k] = (uint32_t)__builtin_amdgcn_ds_bpermute(src, (int)n[k]); }
-      const bool same = lane + c < 64;
+    for (int k = 0; k < P; ++k) dead[k] = 0;
+    dead[0] = (1ull << c) - 1ull;
+    while (known) {
+      const int src = first_lane(known);
+      known = without_lane(known, src);
+      const uint32_t node = rlane(packed, src);
+#pragma unroll
+      for (int k = 0; k < P; ++k) dead[k] |= lanes_where(n[k] == node);
+    }
+    uint32_t pos[P];
+    int live = 0;
+#pragma unroll
+    for (int k = 0; k < P; ++k) {
+      pos[k] = (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(~dead[k] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)~dead[k], (uint32_t)live));
+      live += __popcll(~dead[k]);
+    }
+    size += __popcll(upd) - (64 * P - live);
+    uint32_t upTo = 0, before = 0;
+    const unsigned long long key = ((unsigned long long)tb << 32) | (uint32_t)lane;   // equal totals in lane order
+    const bool enters = tb != 0xffffffffu;
+    while (upd) {
+      const int src = first_lane(upd);
+      upd = without_lane(upd, src);
+      const uint32_t ti = rlane(tb, src);
+      int le = 0;
 #pragma unroll
       for (int k = 0; k < P; ++k) {
-        t[k] = same ? a[k] : (k + 1 < P ? a[k + 1 < P ? k + 1 : k] : kEmpty);
-        n[k] = same ? b[k] : (k + 1 < P ? b[k + 1 < P ? k + 1 : k] : kNone);
+        const bool above = t[k] > ti;
+        le += __popcll(~(lanes_where(above) | dead[k]));
+        pos[k] += above;
       }
+      upTo = wlane(upTo, (uint32_t)le, src);
+      before += key > (((unsigned long long)ti << 32) | (uint32_t)src);
     }
-  }
-  // the number of entries, after drops and updates (which do not keep it)
-  template <int P> BPSX_DEV void count() {
-    size = 0;
-#pragma unroll
-    for (int k = 0; k < P; ++k) size += __popcll(lanes_where(t[k] != kEmpty));
-  }
-  // lane L takes v of lane L - 1 (lane 0: anything)
-  static BPSX_DEV uint32_t from_below(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x138 /* wave_shr:1 */, 0xf, 0xf, true);
-  }
-  // Node n_ gets total t_: its entry, if it has one, leaves, and the new entry goes behind those
-  // with totals up to t_.  (A node has an entry exactly when it is open and has not just been
-  // taken off the front, so whether this is the reference's push or its modify need not be told.)
-  template <int P> BPSX_DEV void update(uint32_t n_, uint32_t t_, int lane) {
+    const uint32_t place = upTo + before;
     if (P == 1) {
-      // No branches: without an old entry its place is -1, as an unsigned bound that keeps every lane
-      const unsigned long long g0 = lanes_where(t[0] > t_), h0 = lanes_where(n[0] == n_);
-      const unsigned long long m0 = g0 & (h0 | (h0 - 1ull));   // the lanes up to the old entry's; without one, all
-      const int p = first_lane(m0);   // never empty: the unused places compare greater
-      t[0] = pick(m0, from_below(t[0]), t[0]);
-      n[0] = pick(m0, from_below(n[0]), n[0]);
-      wlane2(t[0], t_, n[0], n_, p);
-      return;
-    }
-    unsigned long long m[P];
-    int rp = -1, rl = 0;   // pair and lane of the old entry
+      // places up to 63 + 48 fit the buffer: no lane needs to be left out, those that leave go to its end
+      buf[pick(dead[0], 127u, pos[0])] = make_uint2(t[0], n[0]);
+      if (enters) buf[place] = make_uint2(tb, packed);
+      wave_sync();
+      const uint2 e = buf[lane];
+      t[0] = lane < size ? e.x : kEmpty;
+      n[0] = lane < size ? e.y : kNone;
+    } else {
+      uint32_t a[P];
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
-      m[k] = lanes_where(t[k] > t_);
-      const unsigned long long h = lanes_where(n[k] == n_);
-      if (h && rp < 0) { rp = k; rl = __ffsll((long long)h) - 1; }
-    }
-    // only the entries from the new place up to the old one move
-    int pp = -1, pl = 0;   // pair and lane of the new place
+      for (int k = 0; k < P; ++k) a[k] = pick(dead[k], kEmpty, t[k]);
+      uint32_t nt[P], nn[P];
 #pragma unroll
-    for (int k = 0; k < P; ++k) {
-      if (rp >= 0 && k > rp) m[k] = 0;
-      if (k == rp) m[k] &= (2ull << rl) - 1ull;
-      if (m[k] && pp < 0) { pp = k; pl = __ffsll((long long)m[k]) - 1; }
-    }
+      for (int half = 0; half < P / 2; ++half) {
 #pragma unroll
-    for (int k = P - 1; k >= 1; --k) {
-      const uint32_t ct = rlane(t[k - 1], 63), cn = rlane(n[k - 1], 63);   // what moves up into pair k
-      t[k] = pick(m[k], up1(ct, t[k]), t[k]);
-      n[k] = pick(m[k], up1(cn, n[k]), n[k]);
-    }
-    t[0] = pick(m[0], from_below(t[0]), t[0]);
-    n[0] = pick(m[0], from_below(n[0]), n[0]);
+        for (int k = 0; k < P; ++k)
+          if (a[k] != kEmpty && (pos[k] >> 7) == (uint32_t)half) buf[pos[k] & 127u] = make_uint2(t[k], n[k]);
+        if (enters && (place >> 7) == (uint32_t)half) buf[place & 127u] = make_uint2(tb, packed);
+        wave_sync();
 #pragma unroll
-    for (int k = 0; k < P; ++k)
-      if (pp == k) wlane2(t[k], t_, n[k], n_, pl);
+        for (int k = 2 * half; k < 2 * half + 2; ++k) {
+          const uint2 e = buf[(k & 1) * 64 + lane];
+          nt[k] = 64 * k + lane < size ? e.x : kEmpty;
+          nn[k] = 64 * k + lane < size ? e.y : kNone;
+        }
+        wave_sync();
+      }
+#pragma unroll
+      for (int k = 0; k < P; ++k) { t[k] = nt[k]; n[k] = nn[k]; }
+    }
+    wave_sync();
   }
 };
 
@@ -313,7 +322,10 @@ struct GeoLds {
   float w_total[kWindow];
   float w_cost[kWindow];
   float w_pos[3][kWindow];
-  uint32_t tag[kTagSlots];         // which nodes of a pass touch a polygon (see astar_fast)
+  union {
+    alignas(16) uint32_t tag[kTagSlots];   // which row of a pass updates a polygon first (see astar_fast)
+    uint2 merge[128];                      // the open list on its way to its new order
+  };
 };
 // After A* its LDS is dead; the funnel reuses it for the corridor and its portals.  The
 // corridor is written while the nodes' links are still being read: it lies over the hash
@@ -337,7 +349,6 @@ struct GeoWave {
   int lane;
   int nodeCount;
   uint32_t linkSpills, heapSpills;   // queries that left the LDS links / whose open list left the registers
-  uint32_t tagNow;                   // mark of the current pass in L->tag, counting down
 #ifdef BPSX_PHASE_TIMING
   unsigned long long phase[8], phase_t0;
 #endif
@@ -366,8 +377,8 @@ struct GeoWave {
     return (m >> 9) & (kHashSize - 1);
   }
   BPSX_DEV void clear_marks() {
-    for (int i = lane; i < kTagSlots; i += 64) L->tag[i] = 0xffffffffu;
-    tagNow = 0x1fffffffu;
+    static_assert(kTagSlots == 256, "one 16-byte store per lane");
+    reinterpret_cast<uint4*>(L->tag)[lane] = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
   }
   BPSX_DEV void clear() {
     for (int i = lane; i < kHashSize; i += 64) L->first[i] = (uint16_t)kChainEnd;
@@ -786,14 +797,12 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       const unsigned long long reached = lanes_where(before <= ol.t[0]) & (rows_below(1) & ~1ull);
       const int jv = reached ? __builtin_ctzll(reached) : kRows;
       c = jv < c ? jv : c;
-      // conflicts: the earliest row that updates a polygon leaves its mark (pass, row) at the
-      // polygon's hash, later rows look for it: a mark of this pass is base + row
-      g.tagNow--;
-      const uint32_t base = g.tagNow << 3;
+      // conflicts: the earliest row that updates a polygon leaves its mark at the
+      // polygon's hash, later rows look for it (no marks stand when a pass begins)
       const uint32_t slot = bucket & (uint32_t)(kTagSlots - 1);
-      if (tb != 0xffffffffu) atomicMin(&L->tag[slot], base | (uint32_t)row);
+      if (tb != 0xffffffffu) atomicMin(&L->tag[slot], (uint32_t)row);
       wave_sync();
-      const uint32_t seen = L->tag[slot] - base;   // the marking row, or something above 7
+      const uint32_t seen = L->tag[slot];   // the marking row, or all ones
       // an earlier row's update matters to a row only at its own node and at the polygons it
       // updates itself: where it reads and leaves alone (a total no better than the node's), a
       // total lowered further changes nothing
@@ -880,8 +889,6 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     }
     wave_sync();
     FM(8);
-    // ---- the open list: the committed entries leave, the updates enter
-    ol.template drop_front<P>(c, lane);
     const uint32_t packed = (uint32_t)ni | (nb << 11);
     {
       // the pass in the operation log: the header from an idle lane, the updates in lane order
@@ -898,12 +905,9 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       st.logEnd += 1 + nrec;
     }
     FM(9);
-    while (upd) {
-      const int src = first_lane(upd);
-      upd = without_lane(upd, src);
-      ol.template update<P>(rlane(packed, src), rlane(tb, src), lane);
-    }
-    ol.template count<P>();
+    // ---- the open list: the committed entries leave, the updates enter
+    ol.template merge<P>(L->merge, c, upd, lanes_where(update && known), tb, packed, lane);
+    g.clear_marks();
     FM(10);
   }
 }
@@ -943,9 +947,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
 #ifdef BPSX_PHASE_TIMING
   g.phase_t0 = __builtin_readcyclecounter();
 #endif
-  st.ol.init();
-  st.ol.template update<1>(startIp << 11, __float_as_uint(total), lane);
-  st.ol.template count<1>();
+  st.ol.init(lane, __float_as_uint(total), startIp << 11);
   // the loop is instantiated for links in LDS only or spilling (one instantiation where the LDS
   // holds all links), and for a list within one register pair, two or four; a search moves on when
   // one more pass could outgrow what it runs in
@@ -963,6 +965,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     resolved = false;
     if (ex == kAstarGrowLinks) { g.linkSpills++; spill = true; continue; }
     if (ex == kAstarGrowHeap && pairs < OpenList::kPairs) {
+      g.clear_marks();   // the pass that did not fit has left its own
       // the list grows into further registers, empty so far
       if (pairs == 1) { st.ol.clear_pair(1); pairs = 2; }
       else { st.ol.clear_pair(2); st.ol.clear_pair(3); pairs = 4; }
