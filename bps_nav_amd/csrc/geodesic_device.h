@@ -68,6 +68,9 @@ BPSX_DEV void set_wave_priority(int p) {
 }
 // mask of the lanes where b holds (takes the condition as such, not widened to an integer and compared again)
 BPSX_DEV unsigned long long lanes_where(bool b) { return __builtin_amdgcn_ballot_w64(b); }
+// a lane mask held in scalar registers as a condition: sets algebra of conditions on the scalar unit,
+// instead of conditions that are widened to integers and compared again for the next mask
+BPSX_DEV bool in_mask(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 BPSX_DEV int uniform_i(int v) { return __builtin_amdgcn_readfirstlane(v); }
 BPSX_DEV float uniform_f(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
 BPSX_DEV float lane_f(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
@@ -161,8 +164,9 @@ struct OpenList {
   // then took 1.229 ms instead of 1.207 at 16384 agents over mazes, 3.11 instead of 2.59 at 4096
   // over cluttered plans, whose lists fill two to four pairs, 1.16 instead of 0.99 at 1024 over room
   // plans, where a launch lasts as long as its longest search alone.)
-  template <int P> BPSX_DEV void merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
-                                       uint32_t packed, int lane) {
+  // Returns entry `row` of the new list (anything where there is none).
+  template <int P> BPSX_DEV uint32_t merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
+                                           uint32_t packed, int lane, int row) {
     unsigned long long dead[P];
 #pragma unroll
     for (int k = 0; k < P; ++k) dead[k] = 0;
@@ -184,7 +188,8 @@ struct OpenList {
     size += __popcll(upd) - (64 * P - live);
     uint32_t upTo = 0, before = 0;
     const unsigned long long key = ((unsigned long long)tb << 32) | (uint32_t)lane;   // equal totals in lane order
-    const bool enters = tb != 0xffffffffu;
+    const bool enters = in_mask(upd);
+    uint32_t front;
     while (upd) {
       const int src = first_lane(upd);
       upd = without_lane(upd, src);
@@ -206,6 +211,7 @@ struct OpenList {
       if (enters) buf[place] = make_uint2(tb, packed);
       wave_sync();
       const uint2 e = buf[lane];
+      front = buf[row].y;
       t[0] = lane < size ? e.x : kEmpty;
       n[0] = lane < size ? e.y : kNone;
     } else {
@@ -220,6 +226,7 @@ struct OpenList {
           if (a[k] != kEmpty && (pos[k] >> 7) == (uint32_t)half) buf[pos[k] & 127u] = make_uint2(t[k], n[k]);
         if (enters && (place >> 7) == (uint32_t)half) buf[place & 127u] = make_uint2(tb, packed);
         wave_sync();
+        if (half == 0) front = buf[row].y;
 #pragma unroll
         for (int k = 2 * half; k < 2 * half + 2; ++k) {
           const uint2 e = buf[(k & 1) * 64 + lane];
@@ -232,6 +239,7 @@ struct OpenList {
       for (int k = 0; k < P; ++k) { t[k] = nt[k]; n[k] = nn[k]; }
     }
     wave_sync();
+    return front;
   }
 };
 
@@ -242,6 +250,7 @@ struct AstarState {
   int logEnd;        // records in the slot's operation log
   int synced;        // records already applied to the replay's heap
   int replaySize;    // entries of that heap, which the slot keeps between replays
+  int replayNodes;       // nodes created by the records already applied
   uint32_t replayRoot;   // packed node of the entry at its root after a replay
 };
 
@@ -289,8 +298,11 @@ BPSX_DEV bool vequal(const float* a, const float* b) {
 namespace bpsx {
 namespace BPSX_GEO_NS {
 
+// As many links as let nine blocks of two wavefronts share a CU's 160 KB, which are given out in units
+// of 1280 bytes: 14 units a block.  (With 1119 links a block takes 15 and only eight fit: 1.384 instead
+// of 1.144 ms at 16384 agents over mazes.)
 #ifndef BPSX_LINKS_LDS
-#define BPSX_LINKS_LDS 1016
+#define BPSX_LINKS_LDS 1087
 #endif
 #ifndef BPSX_WINDOW
 #define BPSX_WINDOW 128
@@ -316,8 +328,8 @@ static_assert((kWindow & (kWindow - 1)) == 0 && kWindow >= 2 * kNvp, "window mus
 // LDS of one wavefront.
 struct GeoLds {
   uint16_t first[kHashSize];
-  uint32_t n_link[kLinksLds];      // polygon index | next node of the hash chain << 16
-  float w_total[kWindow];
+  uint32_t n_link[kLinksLds + 1];  // polygon index | next node of the hash chain << 16; the last one ends every chain
+  alignas(16) float w_total[kWindow];
   float w_cost[kWindow];
   float w_pos[3][kWindow];
   union {
@@ -381,23 +393,32 @@ struct GeoWave {
   BPSX_DEV void clear() {
     for (int i = lane; i < kHashSize; i += 64) L->first[i] = (uint16_t)kChainEnd;
     clear_marks();
+    if (lane == 0) L->n_link[kLinksLds] = make_link(0xfffeu, kChainEnd);   // no polygon has this index
     nodeCount = 0;
     wave_sync();
   }
   // Node index of polygon ip, or -1; *head receives the bucket's first node (what a new node of
-  // this bucket links to).  Called by all lanes (idle ones with valid = false): the chains are
-  // walked in step, one LDS access per lane and round, until every lane has hit or run out.
+  // this bucket links to).  Called by all lanes (idle ones with an ip that no polygon has): the
+  // chains are walked in step, one LDS access per lane and round, until every lane has hit or run
+  // out.  Where all links are in LDS a lane that is done goes on reading the word behind them.
   template <bool S> BPSX_DEV int find(bool valid, uint32_t ip, uint32_t bucket, uint32_t* head) const {
     uint32_t cur = L->first[bucket];
-    if (!valid) cur = kChainEnd;
+    cur = valid ? cur : kChainEnd;
     *head = cur;
     int found = -1;
     while (lanes_where(cur != kChainEnd)) {
-      const bool live = cur != kChainEnd;
-      const uint32_t l = link<S>(live ? (int)cur : 0);
-      const bool hit = live && link_id(l) == ip;
-      found = hit ? (int)cur : found;
-      cur = (live && !hit) ? link_next(l) : kChainEnd;
+      if (!S || kLinksLds >= kMaxNodes) {
+        const uint32_t l = L->n_link[cur < (uint32_t)kLinksLds ? cur : (uint32_t)kLinksLds];
+        const bool hit = link_id(l) == ip;
+        found = hit ? (int)cur : found;
+        cur = hit ? kChainEnd : link_next(l);
+      } else {
+        const bool live = cur != kChainEnd;
+        const uint32_t l = link<S>(live ? (int)cur : 0);
+        const bool hit = live && link_id(l) == ip;
+        found = hit ? (int)cur : found;
+        cur = (live && !hit) ? link_next(l) : kChainEnd;
+      }
     }
     return found;
   }
@@ -502,6 +523,7 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
   for (int i = lane + 1; i <= rh.size; i += 64) rh.h[i] = kept[i];
   wave_sync();
   int base = -64;              // record held by lane 0
+  int seen = st.replayNodes;   // nodes created so far
   uint32_t rk = 0, rw = 0;
   auto fetch = [&](int from) {
     base = from;
@@ -519,6 +541,8 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
     const bool swap = (hw & kOpUnordered) && (uint32_t)uniform_i((int)rh.h[1].y) != (hw & 0x3ffffffu);
     const bool mine = lane > h && lane <= h + nrec;
     const int myRow = (int)((rw >> 26) & 7u);
+    // the pass's new nodes are those whose index had not been given out before it
+    const unsigned long long fresh = lanes_where(mine && (int)(rw & 0x7ffu) >= seen);
     for (int i = 0; i < c; ++i) {
       const int row = (swap && i < 2) ? 1 - i : i;
       rh.pop();
@@ -528,12 +552,14 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
         m = without_lane(m, j);
         const uint32_t word = rlane(rw, j);
         // a known node without an entry (closed, or its row came earlier in the pass) is pushed
-        rh.update(((word >> 29) & 1u) != 0, rlane(rk, j), word & 0x3ffffffu);
+        rh.update(((fresh >> j) & 1ull) == 0, rlane(rk, j), word & 0x3ffffffu);
       }
     }
     pos += 1 + nrec;
+    seen += __popcll(fresh);
   }
   st.synced = st.logEnd;
+  st.replayNodes = seen;
   st.replaySize = rh.size;
   st.replayRoot = (uint32_t)uniform_i((int)rh.h[1].y);
   for (int i = lane + 1; i <= rh.size; i += 64) kept[i] = rh.h[i];
@@ -666,14 +692,18 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
   endIp = (uint32_t)uniform_i((int)endIp);
   OpenList& ol = st.ol;
   const int row = lane >> kRowShift, el = lane & (kRowLanes - 1);
-  const bool edgeLane = el < kNvp;
-  const bool ownLane = el == kNvp;   // looks after the row's own node in the conflict test
-  constexpr unsigned long long kRowStart = 0x0101010101010101ull;   // the first lane of every row
+  // of every row: the first lane, the edges' lanes, the lane that looks after the row's own node in the conflict test
+  constexpr unsigned long long kRowStart = 0x0101010101010101ull, kEdgeLanes = 0x3f3f3f3f3f3f3f3full, kOwnLanes = 0x4040404040404040ull;
+  static_assert(kNvp == 6 && kRowLanes == 8, "the lane masks of a row");
   constexpr unsigned long long kRows1 = rows_below(1), kRows2 = rows_below(2);   // lanes of the first rows
   unsigned long long resolved = frontResolved ? 1ull : 0ull;
-  // Written for few instructions on the common path: what is rare sits behind one branch each,
-  // and conditions that feed a ballot are folded into the compared value first, so that the
-  // ballot is the comparison's own result.
+  uint32_t cand = (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4, (int)ol.n[0]);   // entry `row` of the list
+  // Written for few instructions and few waits on the common path: what is rare sits behind one branch
+  // each; conditions are lane masks on the scalar unit; LDS reads whose results are needed later go out
+  // early (the marks' before the scan over the rows, the chain heads' before the stores); the next
+  // pass's nodes come back with the merged list instead of through a lane permute; stores take 32-bit
+  // offsets from uniform bases.  Together: 1.207 -> 1.144 ms at 16384 agents over mazes, 0.99 -> 0.92
+  // at 1024 over room plans.
   for (;;) {
     if (ol.size <= 0) return kAstarEmpty;
     if (!S && g.nodeCount > kLinksLds - kRows * kNvp) return kAstarGrowLinks;
@@ -682,7 +712,6 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     // ---- how many entries at the front are each the only one with their total
     const unsigned long long uniq = lanes_where(ol.t[0] < OpenList::down1(OpenList::kEmpty, ol.t[0]));
     int lim = __builtin_ctzll(~uniq | (1ull << kRows));
-    const uint32_t cand = (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4, (int)ol.n[0]);   // entry `row`
     const int bi = (int)(cand & 0x7ffu);
     const uint32_t ip = cand >> 11;
     const unsigned long long goal = lanes_where(ip == endIp) & kRowStart;
@@ -709,47 +738,51 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       else if (goal) { const int jg = __builtin_ctzll(goal) >> kRowShift; lim = jg < lim ? jg : lim; }
     }
     FM(1);
-    const bool rowOn = row < lim;
-    const bool act = edgeLane && rowOn;
+    const unsigned long long rowOn = lanes_where(row < lim);
     uint32_t nb = kNoNb;
     float m0 = 0, m1 = 0, m2 = 0;
-    if (act) {
+    if (in_mask(rowOn & kEdgeLanes)) {
       const AEdge e = edges[ip * kEdgeStride + (uint32_t)el];
       nb = e.nb; m0 = e.mid[0]; m1 = e.mid[1]; m2 = e.mid[2];
     }
     if (__builtin_expect(goalInPair, 0)) nb = ip == endIp ? kNoNb : nb;
-    const int bis = rowOn ? bi : 0;
-    float b0, b1, b2, bcost;
+    const int bw = bi & (kWindow - 1);
+    float b0 = L->w_pos[0][bw], b1 = L->w_pos[1][bw], b2 = L->w_pos[2][bw], bcost = L->w_cost[bw];
     {
-      const int w = bis & (kWindow - 1);
-      b0 = L->w_pos[0][w]; b1 = L->w_pos[1][w]; b2 = L->w_pos[2][w]; bcost = L->w_cost[w];
-      if (bis < g.nodeCount - kWindow) {   // the node has left the window: rare
-        BPSX_KEEP_APART();
-        const float4 pc = *reinterpret_cast<const float4*>(g.ws->nodes[bis].pos);   // pos, cost
-        b0 = pc.x; b1 = pc.y; b2 = pc.z; bcost = pc.w;
-        BPSX_KEEP_APART();
+      const unsigned long long left = lanes_where(bi < g.nodeCount - kWindow) & rowOn;
+      if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
+        if (in_mask(left)) {
+          BPSX_KEEP_APART();
+          const float4 pc = *reinterpret_cast<const float4*>(g.ws->nodes[bi].pos);   // pos, cost
+          b0 = pc.x; b1 = pc.y; b2 = pc.z; bcost = pc.w;
+          BPSX_KEEP_APART();
+        }
       }
     }
     FM(2);
     // ---- node lookup; the row's own lane hashes its own polygon for the conflict test
-    const uint32_t bucket = GeoWave::hash(ownLane ? ip : nb);
+    const uint32_t bucket = GeoWave::hash(in_mask(kOwnLanes) ? ip : nb);
     uint32_t chainHead;
-    int ni = g.find<S>(nb != kNoNb, nb, bucket, &chainHead);
+    const unsigned long long valid = lanes_where(nb != kNoNb);
+    int ni = g.find<S>(in_mask(valid), nb, bucket, &chainHead);
     FM(3);
-    // ---- costs.  A lane without a node to read (idle, or its node is new) reads window slot 127.
-    const bool valid = nb != kNoNb;
-    const int nis = (valid && ni >= 0) ? ni : 0x7fffffff;
-    const int rw = nis & (kWindow - 1);
+    // ---- costs.  A lane without a node to read (idle, or its node is new) reads the window's last slot.
+    const unsigned long long known = lanes_where(ni >= 0);
+    const int rw = ni & (kWindow - 1);
     float p0 = L->w_pos[0][rw], p1 = L->w_pos[1][rw], p2 = L->w_pos[2][rw], oldTotal = L->w_total[rw];
-    if (nis < g.nodeCount - kWindow) {   // the node has left the window: rare
-      const ANode& hn = g.ws->nodes[nis];
-      BPSX_KEEP_APART();
-      const float4 pc = *reinterpret_cast<const float4*>(hn.pos);     // pos, cost
-      p0 = pc.x; p1 = pc.y; p2 = pc.z; oldTotal = hn.total;
-      BPSX_KEEP_APART();
+    {
+      const unsigned long long left = lanes_where(ni < g.nodeCount - kWindow) & known;
+      if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
+        if (in_mask(left)) {
+          const ANode& hn = g.ws->nodes[ni];
+          BPSX_KEEP_APART();
+          const float4 pc = *reinterpret_cast<const float4*>(hn.pos);     // pos, cost
+          p0 = pc.x; p1 = pc.y; p2 = pc.z; oldTotal = hn.total;
+          BPSX_KEEP_APART();
+        }
+      }
     }
-    const bool known = ni >= 0;
-    if (!known) { p0 = m0; p1 = m1; p2 = m2; }   // a new node lies on the portal's midpoint
+    p0 = in_mask(known) ? p0 : m0; p1 = in_mask(known) ? p1 : m1; p2 = in_mask(known) ? p2 : m2;   // a new node lies on the portal's midpoint
     const float cx = p0 - b0, cy = p1 - b1, cz = p2 - b2;
     const float ex = e0 - p0, ey = e1 - p1, ez = e2 - p2;
     const float cc = cx * cx + cy * cy + cz * cz, ee = ex * ex + ey * ey + ez * ez;
@@ -760,8 +793,9 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const float cost = last ? bcost + curCost + toEnd * 1.0f : bcost + curCost;
     const float heuristic = last ? 0.0f : toEnd * H_SCALE;
     const float total = cost + heuristic;
-    // the total as bits where the lane updates its node, all ones where it does not
-    uint32_t tb = (valid && !(known && total >= oldTotal)) ? __float_as_uint(total) : 0xffffffffu;
+    // the lanes that update their node, and the total as bits there, all ones elsewhere
+    unsigned long long upd = valid & ~(known & lanes_where(total >= oldTotal));
+    uint32_t tb = in_mask(upd) ? __float_as_uint(total) : 0xffffffffu;
     FM(4);
     if (__builtin_expect(goalInPair, 0)) {
       // The goal shares the smallest total with one other node.  If the reference takes the goal
@@ -769,9 +803,8 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       // then.  The path is the goal's node and its ancestors: it is the same both ways when
       // that expansion only creates nodes (none of them can be on the path) and the node pool
       // holds them (an exhausted pool is reported as failure).  Otherwise the heap must say.
-      const unsigned long long touches = lanes_where(tb != 0xffffffffu && ni >= 0);
-      const int fresh = __popcll(lanes_where(tb != 0xffffffffu));
-      if (touches || g.nodeCount + fresh > kMaxNodes) return kAstarTie;
+      const int fresh = __popcll(upd);
+      if ((upd & known) || g.nodeCount + fresh > kMaxNodes) return kAstarTie;
       st.lastBest = (int)rlane((uint32_t)bi, first_lane(goal & kRows2));
       return kAstarGoal;
     }
@@ -779,6 +812,12 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     int c = lim;
     bool pairFails = false;
     if (lim > 1) {
+      // conflicts: the earliest row that updates a polygon leaves its mark at the
+      // polygon's hash, later rows look for it (no marks stand when a pass begins)
+      const uint32_t slot = bucket & (uint32_t)(kTagSlots - 1);
+      if (in_mask(upd)) atomicMin(&L->tag[slot], (uint32_t)row);
+      wave_sync();
+      const uint32_t seen = L->tag[slot];   // the marking row, or all ones
       // the first entry j that an update of a row before it reaches or undercuts: the smallest
       // updated total of every row, then of all rows up to it (a scan over the rows), and entry j's
       // lane compares its total with that of the rows before j
@@ -795,27 +834,21 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       const unsigned long long reached = lanes_where(before <= ol.t[0]) & (rows_below(1) & ~1ull);
       const int jv = reached ? __builtin_ctzll(reached) : kRows;
       c = jv < c ? jv : c;
-      // conflicts: the earliest row that updates a polygon leaves its mark at the
-      // polygon's hash, later rows look for it (no marks stand when a pass begins)
-      const uint32_t slot = bucket & (uint32_t)(kTagSlots - 1);
-      if (tb != 0xffffffffu) atomicMin(&L->tag[slot], (uint32_t)row);
-      wave_sync();
-      const uint32_t seen = L->tag[slot];   // the marking row, or all ones
       // an earlier row's update matters to a row only at its own node and at the polygons it
       // updates itself: where it reads and leaves alone (a total no better than the node's), a
       // total lowered further changes nothing
-      const uint32_t seenr = (tb != 0xffffffffu || (ownLane && rowOn)) ? seen : 0xffffffffu;
-      const uint32_t jc = (uint32_t)first_lane(lanes_where(seenr < (uint32_t)row)) >> kRowShift;   // none: far above kRows
+      const unsigned long long cares = upd | (rowOn & kOwnLanes);
+      const uint32_t jc = (uint32_t)first_lane(lanes_where(seen < (uint32_t)row) & cares) >> kRowShift;   // none: far above kRows
       c = jc < (uint32_t)c ? (int)jc : c;
       // rows 0 and 1 of a tied pair in either order: row 0 must not read what row 1 updates either
       if (__builtin_expect(pairTie, 0)) {
-        pairFails = c < 2 || (lanes_where(seenr == 1u) & kRows1) != 0;
+        pairFails = c < 2 || (lanes_where(seen == 1u) & cares & kRows1) != 0;
         if (pairFails && jv >= 2) {
           // The marks are kept per polygon hash, and a pair that fails costs a replay of the log:
           // the polygons that either row updates are compared with those the other row reads,
           // and a clash that was two polygons with one hash lets the pair (and only it) stand.
-          const uint32_t readPoly = ownLane ? (rowOn ? ip : 0xffffffffu) : (tb != 0xffffffffu ? nb : 0xffffffffu);
-          unsigned long long w = lanes_where(tb != 0xffffffffu) & kRows2;
+          const uint32_t readPoly = in_mask(cares & kOwnLanes) ? ip : (in_mask(upd) ? nb : 0xffffffffu);
+          unsigned long long w = upd & kRows2;
           bool real = false;
           while (w) {
             const int src = first_lane(w);
@@ -829,82 +862,81 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     }
     if (__builtin_expect(pairFails, 0)) return kAstarTie;
     FM(5);
-    const bool rowIn = row < c;
-    tb = rowIn ? tb : 0xffffffffu;
-    const bool update = tb != 0xffffffffu;
-    const bool isNew = update && ni < 0;   // a new node is always taken
-    unsigned long long upd = lanes_where(tb != 0xffffffffu);
+    upd &= lanes_where(row < c);
+    tb = in_mask(upd) ? tb : 0xffffffffu;
+    const int nrec = __popcll(upd);
     // nothing has changed yet: a list that would outgrow its registers goes on in the wider instantiation
-    if (__builtin_expect(ol.size - c + __popcll(upd) > 64 * P, 0)) return kAstarGrowHeap;
+    if (__builtin_expect(ol.size - c + nrec > 64 * P, 0)) return kAstarGrowHeap;
     (*pops) += (uint32_t)c;
     FM(6);
-    // ---- new nodes take consecutive indices in row and edge order
-    {
-      const unsigned long long need = lanes_where((update ? ni : 0) < 0);
-      if (need) {
-        const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(need >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)need, 0u));
-        const int count = __popcll(need);
-        const int want = g.nodeCount + count;
-        // the reference carries on without the nodes that do not fit, but reports anything found
-        // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): stop
-        if (S && want > kMaxNodes) {
-          if (kLinksLds >= kMaxNodes) g.linkSpills++;   // where the LDS holds the links of a full pool: a search that needs more than those
-          st.outOfNodes = true;
-          return kAstarEmpty;
-        }
-        if (isNew) ni = g.nodeCount + rank;
-        g.nodeCount = want;
-        bool pending = isNew;
-        uint32_t head = chainHead;
-        for (;;) {
-          if (pending) {
-            g.set_link<S>(ni, make_link(nb, head));
-            L->first[bucket] = (uint16_t)ni;
-          }
-          wave_sync();
-          if (count == 1) break;
-          if (pending) {
-            head = L->first[bucket];
-            pending = head != (uint32_t)ni;
-          }
-          wave_sync();
-          if (!lanes_where(pending)) break;
-        }
+    // ---- new nodes (always taken) get consecutive indices in row and edge order
+    const unsigned long long fresh = upd & ~known;
+    uint32_t head = (uint32_t)ni;
+    if (fresh) {
+      const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(fresh >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)fresh, 0u));
+      const int want = g.nodeCount + __popcll(fresh);
+      // the reference carries on without the nodes that do not fit, but reports anything found
+      // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): stop
+      if (S && want > kMaxNodes) {
+        if (kLinksLds >= kMaxNodes) g.linkSpills++;   // where the LDS holds the links of a full pool: a search that needs more than those
+        st.outOfNodes = true;
+        return kAstarEmpty;
       }
+      // All insert at once in front of the chain head their lookup saw.  Of several that share a
+      // bucket one store wins; the others see that when the head that is read back here has come
+      // (looked at below, after the stores that need not wait for it).
+      if (in_mask(fresh)) {
+        ni = g.nodeCount + rank;
+        g.set_link<S>(ni, make_link(nb, chainHead));
+        L->first[bucket] = (uint16_t)ni;
+      }
+      g.nodeCount = want;
+      wave_sync();
+      head = L->first[bucket];
     }
     FM(7);
-    if (update) {
-      ANode& hn = g.ws->nodes[ni];
+    if (in_mask(upd)) {
+      char* const nodes = reinterpret_cast<char*>(g.ws->nodes);
+      const uint32_t at = (uint32_t)ni * (uint32_t)sizeof(ANode);
       const int w = ni & (kWindow - 1);
-      const uint32_t parent = (uint32_t)bi + 1u;
       if (g.in_window(ni)) {
         L->w_pos[0][w] = p0; L->w_pos[1][w] = p1; L->w_pos[2][w] = p2;
         L->w_cost[w] = cost; L->w_total[w] = total;
       }
-      *reinterpret_cast<float4*>(hn.pos) = make_float4(p0, p1, p2, cost);
-      hn.total = total;
-      g.ws->parents[ni] = (uint16_t)parent;
+      *reinterpret_cast<float4*>(nodes + at) = make_float4(p0, p1, p2, cost);
+      *reinterpret_cast<float*>(nodes + (at + (uint32_t)offsetof(ANode, total))) = total;
+      *reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(g.ws->parents) + (uint32_t)ni * 2u) = (uint16_t)(bi + 1);
     }
-    wave_sync();
     FM(8);
     const uint32_t packed = (uint32_t)ni | (nb << 11);
     {
       // the pass in the operation log: the header from an idle lane, the updates in lane order
-      const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(upd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)upd, 0u));
-      const bool header = lane == kRowLanes - 1;   // idle: neither an edge's lane nor the node's own
-      const int nrec = __popcll(upd);
-      if (update || header) {
+      constexpr unsigned long long kHeader = 1ull << (kRowLanes - 1);   // neither an edge's lane nor the node's own
+      uint32_t headerWord = kOpHeader;
+      if (__builtin_expect(pairTie, 0)) headerWord = kOpHeader | kOpUnordered | rlane(cand, 0);
+      const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(upd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)upd, 1u));
+      if (in_mask(upd | kHeader)) {
         OpRec r;
-        r.key = header ? ((uint32_t)c | ((uint32_t)nrec << 8)) : tb;
-        r.word = header ? (pairTie ? (kOpHeader | kOpUnordered | rlane(cand, 0)) : kOpHeader)
-                        : (packed | ((uint32_t)row << 26) | ((uint32_t)known << 29));
-        g.ws->oplog[st.logEnd + (header ? 0 : 1 + rank)] = r;
+        r.key = OpenList::pick(kHeader, (uint32_t)c | ((uint32_t)nrec << 8), tb);
+        r.word = OpenList::pick(kHeader, headerWord, packed | ((uint32_t)row << 26));
+        *reinterpret_cast<OpRec*>(reinterpret_cast<char*>(g.ws->oplog) + ((uint32_t)st.logEnd + OpenList::pick(kHeader, 0u, (uint32_t)rank)) * (uint32_t)sizeof(OpRec)) = r;
       }
       st.logEnd += 1 + nrec;
     }
+    // new nodes that another of their bucket has overwritten at the chain's head go in behind it
+    for (unsigned long long lost = fresh & lanes_where(head != (uint32_t)ni); __builtin_expect(lost != 0, 0);) {
+      if (in_mask(lost)) {
+        g.set_link<S>(ni, make_link(nb, head));
+        L->first[bucket] = (uint16_t)ni;
+      }
+      wave_sync();
+      head = L->first[bucket];
+      lost &= lanes_where(head != (uint32_t)ni);
+      wave_sync();
+    }
     FM(9);
     // ---- the open list: the committed entries leave, the updates enter
-    ol.template merge<P>(L->merge, c, upd, lanes_where(update && known), tb, packed, lane);
+    cand = ol.template merge<P>(L->merge, c, upd, upd & known, tb, packed, lane, row);
     g.clear_marks();
     FM(10);
   }
@@ -941,7 +973,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   st.lastBest = 0;
   st.outOfNodes = false;
   st.logEnd = st.synced = 0;
-  st.replaySize = 1;
+  st.replaySize = st.replayNodes = 1;
 #ifdef BPSX_PHASE_TIMING
   g.phase_t0 = __builtin_readcyclecounter();
 #endif
