@@ -6,6 +6,9 @@
 // gathers per step is indexed by (scene polygon base + polygon index).
 #pragma once
 #include <cstdint>
+#ifdef __HIPCC__
+#include <hip/hip_runtime.h>
+#endif
 
 namespace bpsx {
 
@@ -123,21 +126,6 @@ struct NavData {
   const float* episodes;   // [.][10]
 };
 
-// A* node of the per-slot pool (dtNode, DetourNode.h:36-45) as kept in HBM: 32 bytes.
-struct alignas(16) ANode {
-  float pos[3];
-  float cost;
-  float total;
-  uint32_t link;    // polygon index within the scene | next node of the hash chain << 16
-  uint32_t pad[2];
-};
-static_assert(sizeof(ANode) == 32, "ANode");
-
-struct HeapEntry {
-  float total;
-  uint32_t node;
-};
-
 // HBM slot of one A* wavefront: the node pool (LDS caches its hot part) and the open-list
 // entries beyond what LDS holds.
 // Record of the open-list operations of a search that keeps its open list sorted (see
@@ -153,12 +141,15 @@ struct OpRec {
 constexpr uint32_t kOpHeader = 0x80000000u, kOpUnordered = 0x40000000u;
 constexpr int kOpLogCap = 8192;
 
+#ifdef __HIPCC__
 struct alignas(128) GeoSlot {
-  ANode nodes[kMaxNodes];
-  HeapEntry heap_spill[kMaxNodes];
+  float4 nodes[kMaxNodes];       // position and cost (dtNode, DetourNode.h:36-45; the total is their sum with the heuristic)
+  uint32_t links[kMaxNodes];     // polygon index within the scene | next node of the hash chain << 16, of nodes beyond what LDS holds
+  uint2 heap_spill[kMaxNodes];   // the reference's heap between replays (total as bits, packed node)
   OpRec oplog[kOpLogCap];
   uint16_t parents[kMaxNodes];   // per node, 1-based index of the node it was reached from, 0 for the start node: what the final walk up the path reads
 };
+#endif
 
 struct GeoQuery {
   float a[3];

@@ -11,7 +11,7 @@
 //     list outgrows the registers goes on with that heap,
 //   - the hash heads of the node pool,
 //   - for the first kLinksLds nodes one word with the polygon id and the hash chain link,
-//   - the position, cost and total of the kWindow most recently created nodes (slot = index
+//   - the position and cost of the kWindow most recently created nodes (slot = index
 //     modulo kWindow); every write of those also goes to the wavefront's slot in HBM, so an older
 //     node is simply read from there.
 // Links beyond kLinksLds spill to the same slot.  A query runs the instantiation of the loop without
@@ -190,19 +190,28 @@ struct OpenList {
     const unsigned long long key = ((unsigned long long)tb << 32) | (uint32_t)lane;   // equal totals in lane order
     const bool enters = in_mask(upd);
     uint32_t front;
+    // Two at a time, so that one's lane moves fill the other's waits.  With an odd number the last
+    // round's second is lane 63 (first_lane of an empty mask, taken modulo 64): no edge's lane, its
+    // total is above all keys and counts nowhere.
     while (upd) {
-      const int src = first_lane(upd);
-      upd = without_lane(upd, src);
-      const uint32_t ti = rlane(tb, src);
-      int le = 0;
+      const int sa = first_lane(upd);
+      upd = without_lane(upd, sa);
+      const int sb = first_lane(upd);
+      upd = without_lane(upd, sb);
+      const uint32_t ta = rlane(tb, sa), tc = rlane(tb, sb);
+      int la = 0, lb = 0;
 #pragma unroll
       for (int k = 0; k < P; ++k) {
-        const bool above = t[k] > ti;
-        le += __popcll(~(lanes_where(above) | dead[k]));
+        const bool above = t[k] > ta, above2 = t[k] > tc;
+        la += __popcll(~(lanes_where(above) | dead[k]));
+        lb += __popcll(~(lanes_where(above2) | dead[k]));
         pos[k] += above;
+        pos[k] += above2;
       }
-      upTo = wlane(upTo, (uint32_t)le, src);
-      before += key > (((unsigned long long)ti << 32) | (uint32_t)src);
+      before += key > (((unsigned long long)ta << 32) | (uint32_t)sa);
+      before += key > (((unsigned long long)tc << 32) | (uint32_t)sb);
+      upTo = wlane(upTo, (uint32_t)la, sa);
+      upTo = wlane(upTo, (uint32_t)lb, sb);
     }
     const uint32_t place = upTo + before;
     if (P == 1) {
@@ -302,7 +311,7 @@ namespace BPSX_GEO_NS {
 // of 1280 bytes: 14 units a block.  (With 1119 links a block takes 15 and only eight fit: 1.384 instead
 // of 1.144 ms at 16384 agents over mazes.)
 #ifndef BPSX_LINKS_LDS
-#define BPSX_LINKS_LDS 1087
+#define BPSX_LINKS_LDS 1215
 #endif
 #ifndef BPSX_WINDOW
 #define BPSX_WINDOW 128
@@ -329,9 +338,7 @@ static_assert((kWindow & (kWindow - 1)) == 0 && kWindow >= 2 * kNvp, "window mus
 struct GeoLds {
   uint16_t first[kHashSize];
   uint32_t n_link[kLinksLds + 1];  // polygon index | next node of the hash chain << 16; the last one ends every chain
-  alignas(16) float w_total[kWindow];
-  float w_cost[kWindow];
-  float w_pos[3][kWindow];
+  alignas(16) float4 w_node[kWindow];   // position, cost
   union {
     alignas(16) uint32_t tag[kTagSlots];   // which row of a pass updates a polygon first (see astar_fast)
     uint2 merge[128];                      // the open list on its way to its new order
@@ -370,13 +377,13 @@ struct GeoWave {
   template <bool S> BPSX_DEV uint32_t link(int i) const {
     if (!S || kLinksLds >= kMaxNodes || i < kLinksLds) return L->n_link[i];
     BPSX_KEEP_APART();
-    const uint32_t v = ws->nodes[i].link;
+    const uint32_t v = ws->links[i];
     BPSX_KEEP_APART();
     return v;
   }
   template <bool S> BPSX_DEV void set_link(int i, uint32_t v) const {
     if (!S || kLinksLds >= kMaxNodes || i < kLinksLds) L->n_link[i] = v;
-    else { BPSX_KEEP_APART(); ws->nodes[i].link = v; BPSX_KEEP_APART(); }
+    else { BPSX_KEEP_APART(); ws->links[i] = v; BPSX_KEEP_APART(); }
   }
   // node i still has its position/cost/total in LDS
   BPSX_DEV bool in_window(int i) const { return i >= nodeCount - kWindow; }
@@ -432,8 +439,8 @@ struct GeoWave {
 // a cluttered plan of 20k polygons ties with a longer list or outgrows the sorted list, and ran
 // again from its start with a heap walked level by level in HBM: 6.6 ms, against 1.5 ms for the
 // longest of the others.)
-constexpr int kHeapLds = (int)((sizeof(GeoLds) - offsetof(GeoLds, w_total)) / sizeof(uint2)) - 1;
-static_assert(offsetof(GeoLds, w_total) % sizeof(uint2) == 0, "the heap's entries are accessed as 8 bytes");
+constexpr int kHeapLds = (int)((sizeof(GeoLds) - offsetof(GeoLds, w_node)) / sizeof(uint2)) - 1;
+static_assert(offsetof(GeoLds, w_node) % sizeof(uint2) == 0, "the heap's entries are accessed as 8 bytes");
 static_assert(kHeapLds >= 64 * OpenList::kPairs + 2 * kRows * kNvp, "a heap with as many entries as the sorted list must fit");
 struct RefHeap {
   uint2* h;    // total bits, packed node
@@ -518,7 +525,7 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
   const int lane = g.lane;
   const OpRec* log = g.ws->oplog;
   uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
-  RefHeap rh(reinterpret_cast<uint2*>(g.L->w_total), st.replaySize, lane);
+  RefHeap rh(reinterpret_cast<uint2*>(g.L->w_node), st.replaySize, lane);
   wave_sync();
   for (int i = lane + 1; i <= rh.size; i += 64) rh.h[i] = kept[i];
   wave_sync();
@@ -569,14 +576,10 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
 BPSX_DEV void restore_window(GeoWave& g) {
   const int from = g.nodeCount > kWindow ? g.nodeCount - kWindow : 0;
   for (int i = from + g.lane; i < g.nodeCount; i += 64) {
-    const ANode& hn = g.ws->nodes[i];
-    const int w = i & (kWindow - 1);
     BPSX_KEEP_APART();
-    const float4 pc = *reinterpret_cast<const float4*>(hn.pos);   // pos, cost
-    const float total = hn.total;
+    const float4 node = g.ws->nodes[i];
     BPSX_KEEP_APART();
-    g.L->w_pos[0][w] = pc.x; g.L->w_pos[1][w] = pc.y; g.L->w_pos[2][w] = pc.z;
-    g.L->w_cost[w] = pc.w; g.L->w_total[w] = total;
+    g.L->w_node[i & (kWindow - 1)] = node;
   }
   g.clear_marks();
   wave_sync();
@@ -590,9 +593,9 @@ template <bool Lds>
 BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops) {
   const int lane = g.lane;
   GeoLds* L = g.L;
-  ANode* nodes = g.ws->nodes;
+  float4* nodes = g.ws->nodes;
   const float H_SCALE = 0.999f;
-  RefHeap rh(Lds ? reinterpret_cast<uint2*>(L->w_total) : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
+  RefHeap rh(Lds ? reinterpret_cast<uint2*>(L->w_node) : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
   for (;;) {
     st.replaySize = rh.size;
     if (rh.size <= 0) return kAstarEmpty;
@@ -609,16 +612,16 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
       const AEdge e = edges[bestIp * kEdgeStride + (uint32_t)lane];
       nb = e.nb; m0 = e.mid[0]; m1 = e.mid[1]; m2 = e.mid[2];
     }
-    const float4 b = *reinterpret_cast<const float4*>(nodes[bi].pos);   // pos, cost
+    const float4 b = nodes[bi];
     const uint32_t bucket = GeoWave::hash(nb);
     uint32_t chainHead;
     int ni = g.find<true>(nb != kNoNb, nb, bucket, &chainHead);
     const bool valid = nb != kNoNb;
     const bool known = valid && ni >= 0;
-    float oldTotal = 0;
+    float oldCost = 0;
     if (known) {
-      const float4 pc = *reinterpret_cast<const float4*>(nodes[ni].pos);
-      m0 = pc.x; m1 = pc.y; m2 = pc.z; oldTotal = nodes[ni].total;
+      const float4 pc = nodes[ni];
+      m0 = pc.x; m1 = pc.y; m2 = pc.z; oldCost = pc.w;
     }
     const float cx = m0 - b.x, cy = m1 - b.y, cz = m2 - b.z;
     const float ex = endPos[0] - m0, ey = endPos[1] - m1, ez = endPos[2] - m2;
@@ -626,8 +629,9 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     sqrt_exact2(cx * cx + cy * cy + cz * cz, ex * ex + ey * ey + ez * ez, &curCost, &toEnd);
     const bool last = nb == endIp;
     const float cost = last ? b.w + curCost * 1.0f + toEnd * 1.0f : b.w + curCost * 1.0f;
-    const float total = cost + (last ? 0.0f : toEnd * H_SCALE);
-    const bool update = valid && !(known && total >= oldTotal);
+    const float heuristic = last ? 0.0f : toEnd * H_SCALE;
+    const float total = cost + heuristic;
+    const bool update = valid && !(known && total >= oldCost + heuristic);
     // new nodes take consecutive indices in edge order; those that share a bucket are chained one after the other
     unsigned long long fresh = lanes_where(update && !known);
     const int want = g.nodeCount + __popcll(fresh);
@@ -644,9 +648,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
       wave_sync();
     }
     if (update) {
-      ANode& hn = nodes[ni];
-      *reinterpret_cast<float4*>(hn.pos) = make_float4(m0, m1, m2, cost);
-      hn.total = total;
+      nodes[ni] = make_float4(m0, m1, m2, cost);
       g.ws->parents[ni] = (uint16_t)(bi + 1);
     }
     wave_sync();
@@ -747,14 +749,13 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     }
     if (__builtin_expect(goalInPair, 0)) nb = ip == endIp ? kNoNb : nb;
     const int bw = bi & (kWindow - 1);
-    float b0 = L->w_pos[0][bw], b1 = L->w_pos[1][bw], b2 = L->w_pos[2][bw], bcost = L->w_cost[bw];
+    float4 b = L->w_node[bw];
     {
       const unsigned long long left = lanes_where(bi < g.nodeCount - kWindow) & rowOn;
       if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
         if (in_mask(left)) {
           BPSX_KEEP_APART();
-          const float4 pc = *reinterpret_cast<const float4*>(g.ws->nodes[bi].pos);   // pos, cost
-          b0 = pc.x; b1 = pc.y; b2 = pc.z; bcost = pc.w;
+          b = g.ws->nodes[bi];
           BPSX_KEEP_APART();
         }
       }
@@ -769,32 +770,31 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     // ---- costs.  A lane without a node to read (idle, or its node is new) reads the window's last slot.
     const unsigned long long known = lanes_where(ni >= 0);
     const int rw = ni & (kWindow - 1);
-    float p0 = L->w_pos[0][rw], p1 = L->w_pos[1][rw], p2 = L->w_pos[2][rw], oldTotal = L->w_total[rw];
+    float4 p = L->w_node[rw];
     {
       const unsigned long long left = lanes_where(ni < g.nodeCount - kWindow) & known;
       if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
         if (in_mask(left)) {
-          const ANode& hn = g.ws->nodes[ni];
           BPSX_KEEP_APART();
-          const float4 pc = *reinterpret_cast<const float4*>(hn.pos);     // pos, cost
-          p0 = pc.x; p1 = pc.y; p2 = pc.z; oldTotal = hn.total;
+          p = g.ws->nodes[ni];
           BPSX_KEEP_APART();
         }
       }
     }
-    p0 = in_mask(known) ? p0 : m0; p1 = in_mask(known) ? p1 : m1; p2 = in_mask(known) ? p2 : m2;   // a new node lies on the portal's midpoint
-    const float cx = p0 - b0, cy = p1 - b1, cz = p2 - b2;
+    const float p0 = in_mask(known) ? p.x : m0, p1 = in_mask(known) ? p.y : m1, p2 = in_mask(known) ? p.z : m2;   // a new node lies on the portal's midpoint
+    const float cx = p0 - b.x, cy = p1 - b.y, cz = p2 - b.z;
     const float ex = e0 - p0, ey = e1 - p1, ez = e2 - p2;
     const float cc = cx * cx + cy * cy + cz * cz, ee = ex * ex + ey * ey + ez * ez;
     float curCost, toEnd;
     sqrt_exact2(cc, ee, &curCost, &toEnd);
     curCost = curCost * 1.0f;
     const bool last = nb == endIp;
-    const float cost = last ? bcost + curCost + toEnd * 1.0f : bcost + curCost;
+    const float cost = last ? b.w + curCost + toEnd * 1.0f : b.w + curCost;
     const float heuristic = last ? 0.0f : toEnd * H_SCALE;
     const float total = cost + heuristic;
-    // the lanes that update their node, and the total as bits there, all ones elsewhere
-    unsigned long long upd = valid & ~(known & lanes_where(total >= oldTotal));
+    // the lanes that update their node, and the total as bits there, all ones elsewhere.  (A node's
+    // total so far is the sum it was computed as, of its cost and the same heuristic.)
+    unsigned long long upd = valid & ~(known & lanes_where(total >= p.w + heuristic));
     uint32_t tb = in_mask(upd) ? __float_as_uint(total) : 0xffffffffu;
     FM(4);
     if (__builtin_expect(goalInPair, 0)) {
@@ -896,15 +896,9 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     }
     FM(7);
     if (in_mask(upd)) {
-      char* const nodes = reinterpret_cast<char*>(g.ws->nodes);
-      const uint32_t at = (uint32_t)ni * (uint32_t)sizeof(ANode);
-      const int w = ni & (kWindow - 1);
-      if (g.in_window(ni)) {
-        L->w_pos[0][w] = p0; L->w_pos[1][w] = p1; L->w_pos[2][w] = p2;
-        L->w_cost[w] = cost; L->w_total[w] = total;
-      }
-      *reinterpret_cast<float4*>(nodes + at) = make_float4(p0, p1, p2, cost);
-      *reinterpret_cast<float*>(nodes + (at + (uint32_t)offsetof(ANode, total))) = total;
+      const float4 node = make_float4(p0, p1, p2, cost);
+      if (g.in_window(ni)) L->w_node[ni & (kWindow - 1)] = node;
+      *reinterpret_cast<float4*>(reinterpret_cast<char*>(g.ws->nodes) + (uint32_t)ni * (uint32_t)sizeof(float4)) = node;
       *reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(g.ws->parents) + (uint32_t)ni * 2u) = (uint16_t)(bi + 1);
     }
     FM(8);
@@ -960,10 +954,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   g.nodeCount = 1;
   if (lane == 0) {
     GeoLds* L = g.L;
-    ANode& hn = g.ws->nodes[0];
-    for (int k = 0; k < 3; ++k) { L->w_pos[k][0] = startPos[k]; hn.pos[k] = startPos[k]; }
-    L->w_cost[0] = 0; L->w_total[0] = total;
-    hn.cost = 0; hn.total = total;
+    L->w_node[0] = g.ws->nodes[0] = make_float4(startPos[0], startPos[1], startPos[2], 0.0f);
     g.ws->parents[0] = 0;
     L->n_link[0] = make_link(startIp, kChainEnd);
     L->first[GeoWave::hash(startIp)] = 0;
@@ -1021,7 +1012,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     ex = astar_exact<true>(g, st, edges, endIp, endPos, pops);
     if (ex == kAstarGrowHeap) {
       uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
-      const uint2* h = reinterpret_cast<const uint2*>(g.L->w_total);
+      const uint2* h = reinterpret_cast<const uint2*>(g.L->w_node);
       for (int i = lane + 1; i <= st.replaySize; i += 64) kept[i] = h[i];
       wave_sync();
       ex = astar_exact<false>(g, st, edges, endIp, endPos, pops);
@@ -1037,11 +1028,9 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   // chain of dependent reads, 70 of them on average: the parent indices, which HBM also holds
   // side by side, are first copied into the window's arrays (no longer needed), so that the
   // chain runs in LDS; a node beyond what fits there is read from HBM.
-  static_assert(offsetof(GeoLds, w_cost) == offsetof(GeoLds, w_total) + sizeof(GeoLds::w_total) &&
-                offsetof(GeoLds, w_pos) == offsetof(GeoLds, w_cost) + sizeof(GeoLds::w_cost), "the window's arrays must be contiguous");
-  constexpr int kParentsLds = (int)((sizeof(GeoLds::w_total) + sizeof(GeoLds::w_cost) + sizeof(GeoLds::w_pos)) / sizeof(uint16_t));
+  constexpr int kParentsLds = kWindow * (int)(sizeof(float4) / sizeof(uint16_t));
   static_assert(sizeof(GeoLds::tag) >= kMaxPath * sizeof(uint16_t), "the walk must fit the array it reuses");
-  uint16_t* lparent = reinterpret_cast<uint16_t*>(g.L->w_total);
+  uint16_t* lparent = reinterpret_cast<uint16_t*>(g.L->w_node);
   uint16_t* walk = reinterpret_cast<uint16_t*>(g.L->tag);
   wave_sync();
   const int inLds = g.nodeCount < kParentsLds ? g.nodeCount : kParentsLds;
