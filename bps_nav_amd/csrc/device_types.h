@@ -51,7 +51,7 @@ struct AEdge {
 };
 static_assert(sizeof(AEdge) == 16, "AEdge");
 constexpr int kEdgeStride = 8;   // records per polygon in HBM: six edges and two unused, one 128-byte line
-constexpr uint32_t kNoNb = 0xffffu;
+constexpr uint32_t kNoNb = 0xfffeu;   // (not all ones: that is what a lane past the end of its hash chain reads)
 
 // dtBVNode repacked at upload: same quantised bounds; a leaf carries its polygon index, an
 // internal node carries Detour's escape offset (for the in-order walk) and the index of its

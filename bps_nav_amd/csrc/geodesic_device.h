@@ -111,7 +111,7 @@ template <int Ctrl, int RowMask> BPSX_DEV uint32_t umin_dpp(uint32_t v) {
 //     length, and rounding is monotonic), so its total is no better and it is left alone anyway.
 // Without both a pass is some 25 of 630 instructions and three LDS accesses shorter: 1.286 -> 1.229 ms
 // of k_geodesic at 16384 agents over mazes, 5 % off the longest of 64 searches alone on the GPU.
-constexpr uint32_t kChainEnd = 0xfffu;
+constexpr uint32_t kChainEnd = 0xffffu;
 static_assert(kMaxNodes <= (int)kChainEnd, "node indices must stay below the chain end marker");
 BPSX_DEV uint32_t link_id(uint32_t l) { return l & 0xffffu; }
 BPSX_DEV uint32_t link_next(uint32_t l) { return l >> 16; }
@@ -307,11 +307,12 @@ BPSX_DEV bool vequal(const float* a, const float* b) {
 namespace bpsx {
 namespace BPSX_GEO_NS {
 
-// As many links as let nine blocks of two wavefronts share a CU's 160 KB, which are given out in units
-// of 1280 bytes: 14 units a block.  (With 1119 links a block takes 15 and only eight fit: 1.384 instead
-// of 1.144 ms at 16384 agents over mazes.)
+// As many links as let ten blocks of two wavefronts share a CU's 160 KB, which are given out in units of
+// 1280 bytes: 12 units a block, 20 wavefronts a CU, which is also what 96 vector registers allow.
+// (With 1215 links, 14 units and nine blocks: 4.43 instead of 3.80 ms at 65536 agents over mixed
+// scenes, within the noise at 16384 over mazes.)
 #ifndef BPSX_LINKS_LDS
-#define BPSX_LINKS_LDS 1215
+#define BPSX_LINKS_LDS 896
 #endif
 #ifndef BPSX_WINDOW
 #define BPSX_WINDOW 128
@@ -337,12 +338,14 @@ static_assert((kWindow & (kWindow - 1)) == 0 && kWindow >= 2 * kNvp, "window mus
 // LDS of one wavefront.
 struct GeoLds {
   uint16_t first[kHashSize];
-  uint32_t n_link[kLinksLds + 1];  // polygon index | next node of the hash chain << 16; the last one ends every chain
+  // Node links: polygon index | next node of the hash chain << 16.  Behind them the marks of which row of
+  // a pass updates a polygon first (see astar_fast), all ones between passes and while chains are
+  // walked: the first of them is the word that ends every chain there.  A pass's open list moves
+  // to its new order over the marks.
+  alignas(16) uint32_t n_link[kLinksLds + kTagSlots];
   alignas(16) float4 w_node[kWindow];   // position, cost
-  union {
-    alignas(16) uint32_t tag[kTagSlots];   // which row of a pass updates a polygon first (see astar_fast)
-    uint2 merge[128];                      // the open list on its way to its new order
-  };
+  BPSX_DEV uint32_t* marks() { return n_link + kLinksLds; }
+  BPSX_DEV uint2* entries() { return reinterpret_cast<uint2*>(n_link + kLinksLds); }   // 128 of them over the marks
 };
 // After A* its LDS is dead; the funnel reuses it for the corridor and its portals.  The
 // corridor is written while the nodes' links are still being read: it lies over the hash
@@ -395,12 +398,11 @@ struct GeoWave {
   }
   BPSX_DEV void clear_marks() {
     static_assert(kTagSlots == 256, "one 16-byte store per lane");
-    reinterpret_cast<uint4*>(L->tag)[lane] = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
+    reinterpret_cast<uint4*>(L->marks())[lane] = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
   }
   BPSX_DEV void clear() {
     for (int i = lane; i < kHashSize; i += 64) L->first[i] = (uint16_t)kChainEnd;
     clear_marks();
-    if (lane == 0) L->n_link[kLinksLds] = make_link(0xfffeu, kChainEnd);   // no polygon has this index
     nodeCount = 0;
     wave_sync();
   }
@@ -433,14 +435,15 @@ struct GeoWave {
 
 // The reference's heap (dtNodeQueue, DetourNode.cpp:150-200), needed when the sorted list cannot say
 // what comes first (a tie) or cannot hold what is open: position q (root = 1) in entry q of an array
-// in LDS, over the window's arrays and the conflict marks, or in the wavefront's slot.  All lanes
+// in LDS, over the conflict marks (but the first two) and the window, or in the wavefront's slot.  All lanes
 // work on one operation: a pop takes one round of accesses per five levels, a push one.
 // (A heap in registers, entry q in lane q mod 64, held 127 entries; one search in seven hundred over
 // a cluttered plan of 20k polygons ties with a longer list or outgrows the sorted list, and ran
 // again from its start with a heap walked level by level in HBM: 6.6 ms, against 1.5 ms for the
 // longest of the others.)
-constexpr int kHeapLds = (int)((sizeof(GeoLds) - offsetof(GeoLds, w_node)) / sizeof(uint2)) - 1;
-static_assert(offsetof(GeoLds, w_node) % sizeof(uint2) == 0, "the heap's entries are accessed as 8 bytes");
+constexpr int kHeapLds = (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
+static_assert(kLinksLds % 4 == 0 && offsetof(GeoLds, w_node) == offsetof(GeoLds, n_link) + 4 * (kLinksLds + kTagSlots),
+              "the marks are accessed as 16 bytes, and the heap lies over the marks and the window");
 static_assert(kHeapLds >= 64 * OpenList::kPairs + 2 * kRows * kNvp, "a heap with as many entries as the sorted list must fit");
 struct RefHeap {
   uint2* h;    // total bits, packed node
@@ -525,7 +528,10 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
   const int lane = g.lane;
   const OpRec* log = g.ws->oplog;
   uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
-  RefHeap rh(reinterpret_cast<uint2*>(g.L->w_node), st.replaySize, lane);
+  RefHeap rh(g.L->entries(), st.replaySize, lane);
+  // the pass that ended here has left its marks: the first of them, which ends the hash chains, lies
+  // under the heap's unused entry 0 and has to stand while a search goes on with the heap
+  g.clear_marks();
   wave_sync();
   for (int i = lane + 1; i <= rh.size; i += 64) rh.h[i] = kept[i];
   wave_sync();
@@ -595,7 +601,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
   GeoLds* L = g.L;
   float4* nodes = g.ws->nodes;
   const float H_SCALE = 0.999f;
-  RefHeap rh(Lds ? reinterpret_cast<uint2*>(L->w_node) : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
+  RefHeap rh(Lds ? L->entries() : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
   for (;;) {
     st.replaySize = rh.size;
     if (rh.size <= 0) return kAstarEmpty;
@@ -815,9 +821,9 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       // conflicts: the earliest row that updates a polygon leaves its mark at the
       // polygon's hash, later rows look for it (no marks stand when a pass begins)
       const uint32_t slot = bucket & (uint32_t)(kTagSlots - 1);
-      if (in_mask(upd)) atomicMin(&L->tag[slot], (uint32_t)row);
+      if (in_mask(upd)) atomicMin(&L->marks()[slot], (uint32_t)row);
       wave_sync();
-      const uint32_t seen = L->tag[slot];   // the marking row, or all ones
+      const uint32_t seen = L->marks()[slot];   // the marking row, or all ones
       // the first entry j that an update of a row before it reaches or undercuts: the smallest
       // updated total of every row, then of all rows up to it (a scan over the rows), and entry j's
       // lane compares its total with that of the rows before j
@@ -930,7 +936,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     }
     FM(9);
     // ---- the open list: the committed entries leave, the updates enter
-    cand = ol.template merge<P>(L->merge, c, upd, upd & known, tb, packed, lane, row);
+    cand = ol.template merge<P>(L->entries(), c, upd, upd & known, tb, packed, lane, row);
     g.clear_marks();
     FM(10);
   }
@@ -1012,7 +1018,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     ex = astar_exact<true>(g, st, edges, endIp, endPos, pops);
     if (ex == kAstarGrowHeap) {
       uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
-      const uint2* h = reinterpret_cast<const uint2*>(g.L->w_node);
+      const uint2* h = g.L->entries();
       for (int i = lane + 1; i <= st.replaySize; i += 64) kept[i] = h[i];
       wave_sync();
       ex = astar_exact<false>(g, st, edges, endIp, endPos, pops);
@@ -1029,9 +1035,9 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   // side by side, are first copied into the window's arrays (no longer needed), so that the
   // chain runs in LDS; a node beyond what fits there is read from HBM.
   constexpr int kParentsLds = kWindow * (int)(sizeof(float4) / sizeof(uint16_t));
-  static_assert(sizeof(GeoLds::tag) >= kMaxPath * sizeof(uint16_t), "the walk must fit the array it reuses");
+  static_assert(kTagSlots * sizeof(uint32_t) >= kMaxPath * sizeof(uint16_t), "the walk must fit the marks it reuses");
   uint16_t* lparent = reinterpret_cast<uint16_t*>(g.L->w_node);
-  uint16_t* walk = reinterpret_cast<uint16_t*>(g.L->tag);
+  uint16_t* walk = reinterpret_cast<uint16_t*>(g.L->marks());
   wave_sync();
   const int inLds = g.nodeCount < kParentsLds ? g.nodeCount : kParentsLds;
   {
