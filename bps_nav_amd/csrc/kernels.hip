@@ -561,6 +561,9 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
     nq += (uint32_t)uniform_i((int)counts[c]);
     if (c + 1 == kLongClasses) nlong = nq;
   }
+  // With a block for every query all of them are run that way (1024 agents over room plans, 560
+  // queries: 0.90 -> 0.87 ms).
+  if (nq <= gridDim.x) nlong = nq;
   int curCls = 0;
   uint32_t curLo = 0, curHi = (uint32_t)uniform_i((int)counts[0]);
   auto class_of = [&](uint32_t ticket) {   // ticket < nq, not below an earlier one
@@ -767,10 +770,8 @@ void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz
                            const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */, float* out,
                            GeoSlot* slots, uint32_t geo_blocks, uint64_t* counters, hipStream_t st) {
   hipLaunchKernelGGL(k_make_queries, grid_for(n, 256), dim3(256), 0, st, scene, sxyz, sref, exyz, eref, n, qbuf);
-  // One class only.  With a block for every query they count as the longest: each then runs on
-  // its block's whole LDS.  Otherwise as the shortest: two to a block.
-  const uint32_t cls = n <= geo_blocks ? 0u : (uint32_t)kGeoClasses - 1u;
-  hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n, cls);
+  // one class only, that of the shortest
+  hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n, (uint32_t)kGeoClasses - 1u);
   // stride 0 puts the class's queries at the start of the buffer
   launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, slots,
                   geo_blocks, counters, st);

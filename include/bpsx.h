@@ -209,8 +209,8 @@ BPSX_API int bpsx_check_errors(bpsx_sim *sim);
  * (cycle counts of the A* loop's phases, a diagnostic build); [16] path searches that needed
  * more node links than the kernel keeps in LDS, [17] path searches whose open list outgrew
  * the kernel's registers (both continue in slower code; results are the same), [18] path
- * searches expected to be among the longest of their step, which the kernel runs with larger
- * LDS structures (same results).  The path search keeps its open list sorted by total instead of
+ * searches that the kernel runs with larger LDS structures: those expected to be among the longest
+ * of their step, or all where there is a block for each (same results).  The path search keeps its open list sorted by total instead of
  * in the reference's heap arrangement, which only matters when two open nodes share the
  * smallest total: [21] counts the passes that found such a pair and tried to expand both at once
  * (possible when neither affects the other), [20] the times the reference's arrangement had to be
