@@ -213,9 +213,9 @@ struct bpsx_sim {
   AgentArrays A{};
   std::vector<void*> owned;  // every device allocation, for destroy
   std::vector<Group> groups;
-  GeoSlot* d_slots = nullptr;
-  uint32_t geo_blocks = 0, snap_blocks = 0;
-  uint32_t max_geo_blocks = 0, compute_units = 0;   // what the device holds of k_geodesic at once, whatever the number of envs
+  GeoPool geo{};                      // of the steps: what their envs can fill
+  uint32_t snap_blocks = 0;
+  uint32_t max_geo_blocks = 0, max_few_blocks = 0, compute_units = 0;   // what the device holds at once, whatever the number of envs
   uint32_t* d_error = nullptr;
   uint64_t* d_counters = nullptr;
   float turn_left[4], turn_right[4];
@@ -227,7 +227,7 @@ struct bpsx_sim {
   void* d_batch = nullptr;
   size_t batch_bytes = 0;
   GeoSlot* d_batch_slots = nullptr;   // node pools of a batch of path queries that needs more wavefronts than the steps have
-  uint32_t batch_slot_blocks = 0;
+  uint32_t batch_slots = 0;
   uint32_t* d_batch_counts = nullptr;
 
   template <class T>
@@ -609,9 +609,11 @@ int bpsx_finalize(bpsx_sim* sim) {
   sim->max_geo_blocks = blocks;
   sim->compute_units = (uint32_t)prop.multiProcessorCount;
   if (blocks > sim->envs_per_group) blocks = sim->envs_per_group;
-  sim->geo_blocks = std::max(1u, blocks);
+  sim->geo.blocks = std::max(1u, blocks);
+  sim->max_few_blocks = (uint32_t)prop.multiProcessorCount * geodesic_few_blocks_per_cu();
+  sim->geo.few_blocks = std::min(sim->max_few_blocks, sim->geo.blocks * 2u);
   sim->snap_blocks = std::max(1u, std::min((uint32_t)prop.multiProcessorCount * 16u, sim->envs_per_group));
-  if ((rc = sim->alloc(&sim->d_slots, (size_t)sim->geo_blocks * 2))) return rc;   // one per wavefront
+  if ((rc = sim->alloc(&sim->geo.slots, (size_t)sim->geo.blocks * 2))) return rc;   // one per wavefront
 
   // ---- per-group queues
   sim->groups.resize(sim->num_groups);
@@ -696,7 +698,7 @@ int bpsx_reset(bpsx_sim* sim, uint32_t group, void* hip_stream) {
   HIP_TRY(hipSetDevice(sim->cfg.gpu_id));
   if ((rc = quiesce(sim))) return rc;
   hipStream_t st = (hipStream_t)hip_stream;
-  launch_reset(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], sim->params(group), sim->d_slots, sim->geo_blocks, sim->snap_blocks, st);
+  launch_reset(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], sim->params(group), sim->geo, sim->snap_blocks, st);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(st));
   return BPSX_OK;
@@ -726,7 +728,7 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   g.profiled = sim->profiling;
   StepParams P = sim->params(group);
   P.defer_first_distance = 1;
-  launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->d_slots, sim->geo_blocks, sim->snap_blocks, st,
+  launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->geo, sim->snap_blocks, st,
               sim->side, g.moved, g.snapped, g.profiled ? g.ev : nullptr);
   g.turn ^= 1;
   HIP_TRY(hipGetLastError());
@@ -868,23 +870,28 @@ static int batch_reserve(bpsx_sim* sim, size_t bytes) {
   sim->batch_bytes = bytes;
   return BPSX_OK;
 }
-// Node pools for a batch of n path queries: as many blocks of k_geodesic as the device holds at
-// once, or one per query where that is less.  The steps' own pools serve if they are enough (a
-// simulator has no more of them than envs in a group); otherwise the batch has pools of its own,
-// kept until a larger batch or bpsx_destroy replaces them (at most 0.7 GB).
+// Node pools for a batch of n path queries: one per query while k_geodesic_few serves it, else as
+// many blocks of k_geodesic as the device holds at once, or one per query where that is less.  The
+// steps' own pools serve if they are enough (a simulator has no more of them than envs in a group);
+// otherwise the batch has pools of its own, kept until a larger batch or bpsx_destroy replaces them
+// (at most 0.7 GB).
 // (1000 pairs over a maze, simulator of 4 envs, so far served by 4 blocks: 131 -> 2.3 ms a call.)
-static int batch_reserve_slots(bpsx_sim* sim, uint32_t n, GeoSlot** slots, uint32_t* blocks) {
-  const uint32_t want = std::min(sim->max_geo_blocks, n);
-  if (want <= sim->geo_blocks) { *slots = sim->d_slots; *blocks = sim->geo_blocks; return BPSX_OK; }
-  if (want > sim->batch_slot_blocks) {
-    if (sim->d_batch_slots) HIP_TRY(hipFree(sim->d_batch_slots));
-    sim->d_batch_slots = nullptr;
-    sim->batch_slot_blocks = 0;
-    HIP_TRY(hipMalloc((void**)&sim->d_batch_slots, (size_t)want * 2 * sizeof(GeoSlot)));
-    sim->batch_slot_blocks = want;
+static int batch_reserve_slots(bpsx_sim* sim, uint32_t n, GeoPool* out) {
+  const bool few = n <= sim->max_few_blocks;
+  const uint32_t want = few ? n : 2u * std::min(sim->max_geo_blocks, n);
+  *out = sim->geo;
+  if (want > sim->geo.blocks * 2u) {
+    if (want > sim->batch_slots) {
+      if (sim->d_batch_slots) HIP_TRY(hipFree(sim->d_batch_slots));
+      sim->d_batch_slots = nullptr;
+      sim->batch_slots = 0;
+      HIP_TRY(hipMalloc((void**)&sim->d_batch_slots, (size_t)want * sizeof(GeoSlot)));
+      sim->batch_slots = want;
+    }
+    out->slots = sim->d_batch_slots;
+    out->blocks = want / 2u;
   }
-  *slots = sim->d_batch_slots;
-  *blocks = want;
+  out->few_blocks = few ? n : 0u;
   return BPSX_OK;
 }
 // Brings the host's view of a slot up to date: a swap whose envs have all moved is complete.
@@ -1084,14 +1091,13 @@ int bpsx_geodesic(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const u
   float* d_s = (float*)(b + qb); float* d_e = (float*)(b + qb + f3);
   uint32_t* d_sr = (uint32_t*)(b + qb + 2 * f3); uint32_t* d_er = (uint32_t*)(b + qb + 2 * f3 + u1);
   float* d_o = (float*)(b + qb + 2 * f3 + 2 * u1);
-  GeoSlot* slots = nullptr;
-  uint32_t blocks = 0;
-  if ((rc = batch_reserve_slots(sim, n, &slots, &blocks))) return rc;
+  GeoPool geo{};
+  if ((rc = batch_reserve_slots(sim, n, &geo))) return rc;
   HIP_TRY(hipMemcpy(d_s, start_xyz, f3, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_e, end_xyz, f3, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_sr, start_ref, u1, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_er, end_ref, u1, hipMemcpyHostToDevice));
-  launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, d_q, sim->d_batch_counts, d_o, slots, blocks,
+  launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, d_q, sim->d_batch_counts, d_o, geo,
                         sim->d_counters, nullptr);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpy(out_dist, d_o, u1, hipMemcpyDeviceToHost));
@@ -1115,7 +1121,8 @@ int bpsx_geodesic_static(bpsx_sim* sim, uint32_t scene, const float* start_xyz, 
   // The counters are rewritten by a kernel at the start of every call; node pools and queries
   // are written before they are read.  Nothing else of the previous call's contents is used.
   launch_geodesic_batch(sim->nav, scene_entry(sim, scene), start_xyz, start_ref, end_xyz, end_ref, n, d_q, d_counts, out_dist,
-                        d_slots, std::min(kStaticBlocks, std::max(1u, (n + 1) / 2)), sim->d_counters, (hipStream_t)hip_stream);
+                        GeoPool{d_slots, std::min(kStaticBlocks, std::max(1u, (n + 1) / 2)), n <= kStaticBlocks * 2u ? n : 0u}, sim->d_counters,
+                        (hipStream_t)hip_stream);
   HIP_TRY(hipGetLastError());
   return BPSX_OK;
 }

@@ -323,6 +323,8 @@ constexpr int kWindow = BPSX_WINDOW;        // most recent nodes whose position/
 #define BPSX_HASH 512
 #endif
 constexpr int kHashSize = BPSX_HASH;        // buckets of the node pool's hash table
+constexpr bool kAllLds = kWindow >= kMaxNodes;   // every node is kept in LDS, and none in HBM
+static_assert(!kAllLds || kLinksLds >= kMaxNodes, "a pool in LDS has its links there too");
 #ifndef BPSX_TAG_SLOTS
 #define BPSX_TAG_SLOTS 256
 #endif
@@ -346,6 +348,14 @@ struct GeoLds {
   alignas(16) float4 w_node[kWindow];   // position, cost
   BPSX_DEV uint32_t* marks() { return n_link + kLinksLds; }
   BPSX_DEV uint2* entries() { return reinterpret_cast<uint2*>(n_link + kLinksLds); }   // 128 of them over the marks
+#if BPSX_WINDOW >= 2048
+  // with every node in LDS: parent indices, and a place of its own for the reference's heap
+  uint2 ref_heap[64 * OpenList::kPairs + 2 * 8 * kNvp + 2];
+  uint16_t parents[kMaxNodes];
+  BPSX_DEV uint2* heap() { return ref_heap; }
+#else
+  BPSX_DEV uint2* heap() { return entries(); }
+#endif
 };
 // After A* its LDS is dead; the funnel reuses it for the corridor and its portals.  The
 // corridor is written while the nodes' links are still being read: it lies over the hash
@@ -389,7 +399,24 @@ struct GeoWave {
     else { BPSX_KEEP_APART(); ws->links[i] = v; BPSX_KEEP_APART(); }
   }
   // node i still has its position/cost/total in LDS
-  BPSX_DEV bool in_window(int i) const { return i >= nodeCount - kWindow; }
+  BPSX_DEV bool in_window(int i) const { return kAllLds || i >= nodeCount - kWindow; }
+  // node i, whose position and cost are not looked for in the window; and a node and its parent index stored outside of it
+  BPSX_DEV float4 node(int i) const {
+#if BPSX_WINDOW >= 2048
+    return L->w_node[i];
+#else
+    return ws->nodes[i];
+#endif
+  }
+  BPSX_DEV void keep_node(int i, float4 n, int parent) const {
+#if BPSX_WINDOW >= 2048
+    L->w_node[i] = n;
+    L->parents[i] = (uint16_t)parent;
+#else
+    *reinterpret_cast<float4*>(reinterpret_cast<char*>(ws->nodes) + (uint32_t)i * (uint32_t)sizeof(float4)) = n;
+    *reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(ws->parents) + (uint32_t)i * 2u) = (uint16_t)parent;
+#endif
+  }
   // the multiply as the full-rate 24-bit instruction (polygon indices have 15 bits)
   static BPSX_DEV uint32_t hash(uint32_t ip) {
     uint32_t m;
@@ -441,7 +468,7 @@ struct GeoWave {
 // a cluttered plan of 20k polygons ties with a longer list or outgrows the sorted list, and ran
 // again from its start with a heap walked level by level in HBM: 6.6 ms, against 1.5 ms for the
 // longest of the others.)
-constexpr int kHeapLds = (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
+constexpr int kHeapLds = kAllLds ? 64 * OpenList::kPairs + 2 * kRows * kNvp + 1 : (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
 static_assert(kLinksLds % 4 == 0 && offsetof(GeoLds, w_node) == offsetof(GeoLds, n_link) + 4 * (kLinksLds + kTagSlots),
               "the marks are accessed as 16 bytes, and the heap lies over the marks and the window");
 static_assert(kHeapLds >= 64 * OpenList::kPairs + 2 * kRows * kNvp, "a heap with as many entries as the sorted list must fit");
@@ -528,7 +555,7 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
   const int lane = g.lane;
   const OpRec* log = g.ws->oplog;
   uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
-  RefHeap rh(g.L->entries(), st.replaySize, lane);
+  RefHeap rh(g.L->heap(), st.replaySize, lane);
   // the pass that ended here has left its marks: the first of them, which ends the hash chains, lies
   // under the heap's unused entry 0 and has to stand while a search goes on with the heap
   g.clear_marks();
@@ -580,6 +607,7 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
 }
 // The window and the marks after something else has used their LDS.
 BPSX_DEV void restore_window(GeoWave& g) {
+  if (kAllLds) return;   // nothing else has
   const int from = g.nodeCount > kWindow ? g.nodeCount - kWindow : 0;
   for (int i = from + g.lane; i < g.nodeCount; i += 64) {
     BPSX_KEEP_APART();
@@ -599,9 +627,8 @@ template <bool Lds>
 BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops) {
   const int lane = g.lane;
   GeoLds* L = g.L;
-  float4* nodes = g.ws->nodes;
   const float H_SCALE = 0.999f;
-  RefHeap rh(Lds ? L->entries() : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
+  RefHeap rh(Lds ? L->heap() : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
   for (;;) {
     st.replaySize = rh.size;
     if (rh.size <= 0) return kAstarEmpty;
@@ -618,7 +645,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
       const AEdge e = edges[bestIp * kEdgeStride + (uint32_t)lane];
       nb = e.nb; m0 = e.mid[0]; m1 = e.mid[1]; m2 = e.mid[2];
     }
-    const float4 b = nodes[bi];
+    const float4 b = g.node(bi);
     const uint32_t bucket = GeoWave::hash(nb);
     uint32_t chainHead;
     int ni = g.find<true>(nb != kNoNb, nb, bucket, &chainHead);
@@ -626,7 +653,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     const bool known = valid && ni >= 0;
     float oldCost = 0;
     if (known) {
-      const float4 pc = nodes[ni];
+      const float4 pc = g.node(ni);
       m0 = pc.x; m1 = pc.y; m2 = pc.z; oldCost = pc.w;
     }
     const float cx = m0 - b.x, cy = m1 - b.y, cz = m2 - b.z;
@@ -654,8 +681,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
       wave_sync();
     }
     if (update) {
-      nodes[ni] = make_float4(m0, m1, m2, cost);
-      g.ws->parents[ni] = (uint16_t)(bi + 1);
+      g.keep_node(ni, make_float4(m0, m1, m2, cost), bi + 1);
     }
     wave_sync();
     const uint32_t packed = (uint32_t)ni | (nb << 11);
@@ -756,7 +782,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     if (__builtin_expect(goalInPair, 0)) nb = ip == endIp ? kNoNb : nb;
     const int bw = bi & (kWindow - 1);
     float4 b = L->w_node[bw];
-    {
+    if (!kAllLds) {
       const unsigned long long left = lanes_where(bi < g.nodeCount - kWindow) & rowOn;
       if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
         if (in_mask(left)) {
@@ -777,7 +803,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const unsigned long long known = lanes_where(ni >= 0);
     const int rw = ni & (kWindow - 1);
     float4 p = L->w_node[rw];
-    {
+    if (!kAllLds) {
       const unsigned long long left = lanes_where(ni < g.nodeCount - kWindow) & known;
       if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
         if (in_mask(left)) {
@@ -903,9 +929,8 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     FM(7);
     if (in_mask(upd)) {
       const float4 node = make_float4(p0, p1, p2, cost);
-      if (g.in_window(ni)) L->w_node[ni & (kWindow - 1)] = node;
-      *reinterpret_cast<float4*>(reinterpret_cast<char*>(g.ws->nodes) + (uint32_t)ni * (uint32_t)sizeof(float4)) = node;
-      *reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(g.ws->parents) + (uint32_t)ni * 2u) = (uint16_t)(bi + 1);
+      if (!kAllLds && g.in_window(ni)) L->w_node[ni & (kWindow - 1)] = node;
+      g.keep_node(ni, node, bi + 1);
     }
     FM(8);
     const uint32_t packed = (uint32_t)ni | (nb << 11);
@@ -960,8 +985,8 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   g.nodeCount = 1;
   if (lane == 0) {
     GeoLds* L = g.L;
-    L->w_node[0] = g.ws->nodes[0] = make_float4(startPos[0], startPos[1], startPos[2], 0.0f);
-    g.ws->parents[0] = 0;
+    L->w_node[0] = make_float4(startPos[0], startPos[1], startPos[2], 0.0f);
+    g.keep_node(0, L->w_node[0], 0);
     L->n_link[0] = make_link(startIp, kChainEnd);
     L->first[GeoWave::hash(startIp)] = 0;
     reinterpret_cast<uint2*>(g.ws->heap_spill)[1] = make_uint2(__float_as_uint(total), startIp << 11);
@@ -1018,7 +1043,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     ex = astar_exact<true>(g, st, edges, endIp, endPos, pops);
     if (ex == kAstarGrowHeap) {
       uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
-      const uint2* h = g.L->entries();
+      const uint2* h = g.L->heap();
       for (int i = lane + 1; i <= st.replaySize; i += 64) kept[i] = h[i];
       wave_sync();
       ex = astar_exact<false>(g, st, edges, endIp, endPos, pops);
@@ -1034,11 +1059,15 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   // chain of dependent reads, 70 of them on average: the parent indices, which HBM also holds
   // side by side, are first copied into the window's arrays (no longer needed), so that the
   // chain runs in LDS; a node beyond what fits there is read from HBM.
-  constexpr int kParentsLds = kWindow * (int)(sizeof(float4) / sizeof(uint16_t));
   static_assert(kTagSlots * sizeof(uint32_t) >= kMaxPath * sizeof(uint16_t), "the walk must fit the marks it reuses");
-  uint16_t* lparent = reinterpret_cast<uint16_t*>(g.L->w_node);
   uint16_t* walk = reinterpret_cast<uint16_t*>(g.L->marks());
   wave_sync();
+#if BPSX_WINDOW >= 2048
+  const uint16_t* lparent = g.L->parents;
+  constexpr int inLds = kMaxNodes;
+#else
+  constexpr int kParentsLds = kWindow * (int)(sizeof(float4) / sizeof(uint16_t));
+  uint16_t* lparent = reinterpret_cast<uint16_t*>(g.L->w_node);
   const int inLds = g.nodeCount < kParentsLds ? g.nodeCount : kParentsLds;
   {
     const uint32_t* src = reinterpret_cast<const uint32_t*>(g.ws->parents);
@@ -1046,6 +1075,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     for (int i = lane; i < (inLds + 1) / 2; i += 64) dst[i] = src[i];
   }
   wave_sync();
+#endif
   int length = 0;
   for (int c = lastBest + 1; c && length <= kMaxNodes;) {
     if (lane == 0 && length < kMaxPath) walk[length] = (uint16_t)(c - 1);

@@ -6,6 +6,13 @@
 
 namespace bpsx {
 
+// Node pools of the path searches and the launches they allow: one pool per wavefront.
+struct GeoPool {
+  GeoSlot* slots;
+  uint32_t blocks;       // blocks of two wavefronts of k_geodesic
+  uint32_t few_blocks;   // blocks of one wavefront of k_geodesic_few; 0: never
+};
+
 enum QueueCounter { kQGeo = 0 /* one per cost class */, kQGeoHead = kGeoClasses, kQReset, kQCounters };
 
 // Work queues of one step, all in HBM, sized for every agent of a group.
@@ -46,26 +53,26 @@ constexpr int kStepEvents = 5;  // timestamps recorded by launch_step when asked
 // while the searches run on `st`, and their first queries go to Qnext, the next step's queues.
 // `moved` and `snapped` are events of the caller's for the fork and the join of the two streams.
 void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
-                 const int64_t* actions_dev, GeoSlot* slots, uint32_t geo_blocks, uint32_t snap_blocks, hipStream_t st,
+                 const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st,
                  hipStream_t side, hipEvent_t moved, hipEvent_t snapped, hipEvent_t* ev);
 // Reset of a whole group, all on st; Qother (the group's other set of queues) is emptied.
 void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
-                  GeoSlot* slots, uint32_t geo_blocks, uint32_t snap_blocks, hipStream_t st);
+                  const GeoPool& G, uint32_t snap_blocks, hipStream_t st);
 void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz, uint32_t* oref,
                        uint32_t snap_blocks, hipStream_t st);
 void launch_try_step_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                            uint32_t n, float* oxyz, uint32_t* oref, hipStream_t st);
 void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                            const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */,
-                           float* out,
-                           GeoSlot* slots, uint32_t geo_blocks, uint64_t* counters, hipStream_t st);
+                           float* out, const GeoPool& G, uint64_t* counters, hipStream_t st);
 void launch_random_points(const NavData& nav, uint32_t scene, const float* u, uint32_t n, float* oxyz, uint32_t* oref,
                           hipStream_t st);
 
 void launch_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint32_t slot, uint32_t target, uint32_t envs,
                      hipStream_t st);
 
-// Wavefronts of the A* kernel that one compute unit holds at once (bounded by their LDS).
+// Blocks of the A* kernels that one compute unit holds at once (bounded by their LDS).
 uint32_t geodesic_blocks_per_cu();
+uint32_t geodesic_few_blocks_per_cu();
 
 }  // namespace bpsx

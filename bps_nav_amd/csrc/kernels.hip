@@ -40,6 +40,15 @@
 #define BPSX_WINDOW 256
 #define BPSX_HASH 1024
 #include "geodesic_device.h"
+// A third, for launches of few queries, where a launch lasts as long as its longest search: the
+// whole node pool and 2048 hash heads in LDS, 52 KB for each wavefront (see k_geodesic_few).
+#undef BPSX_GEO_NS
+#undef BPSX_WINDOW
+#undef BPSX_HASH
+#define BPSX_GEO_NS geo_few
+#define BPSX_WINDOW 2048
+#define BPSX_HASH 2048
+#include "geodesic_device.h"
 #include "kernels.h"
 
 namespace bpsx {
@@ -502,6 +511,24 @@ __global__ __launch_bounds__(128) void k_reset_snap(NavData nav, AgentArrays A, 
 // result and the agent's cost estimate.
 struct GeoTotals {
   uint32_t pops = 0, corridor = 0, done = 0;
+  uint32_t linkSpills = 0, heapSpills = 0, exactRuns = 0, tieReplays = 0, pairTies = 0;
+  template <class Wave> BPSX_DEV void add(const Wave& g, int lane, uint64_t* counters) {
+    linkSpills += g.linkSpills; heapSpills += g.heapSpills; exactRuns += g.exactRuns; tieReplays += g.tieReplays; pairTies += g.pairTies;
+#ifdef BPSX_PHASE_TIMING
+    if (lane == 0) for (int k = 0; k < 8; ++k) atomicAdd((unsigned long long*)&counters[8 + k], g.phase[k]);
+#endif
+  }
+  BPSX_DEV void count(int lane, uint64_t* counters) const {
+    if (lane != 0 || !done) return;
+    atomicAdd((unsigned long long*)&counters[kCntGeoQueries], (unsigned long long)done);
+    atomicAdd((unsigned long long*)&counters[kCntAstarPops], (unsigned long long)pops);
+    atomicAdd((unsigned long long*)&counters[kCntCorridor], (unsigned long long)corridor);
+    if (linkSpills) atomicAdd((unsigned long long*)&counters[kCntLinkSpills], (unsigned long long)linkSpills);
+    if (heapSpills) atomicAdd((unsigned long long*)&counters[kCntHeapSpills], (unsigned long long)heapSpills);
+    if (exactRuns) atomicAdd((unsigned long long*)&counters[kCntExactRuns], (unsigned long long)exactRuns);
+    if (tieReplays) atomicAdd((unsigned long long*)&counters[kCntTieReplays], (unsigned long long)tieReplays);
+    if (pairTies) atomicAdd((unsigned long long*)&counters[kCntPairTies], (unsigned long long)pairTies);
+  }
 };
 template <class Wave>
 BPSX_DEV void serve_query(Wave& g, const NavData& nav, const GeoQuery& q, int cls, float* out, uint32_t* last_cost, GeoTotals& T) {
@@ -575,7 +602,6 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
     return curCls;
   };
   GeoTotals T;
-  uint32_t linkSpills = 0, heapSpills = 0, exactRuns = 0, tieReplays = 0, pairTies = 0;
   // The first query of every wavefront needs no ticket counter: the grid is what the device
   // holds at once, so block b takes long query b if there is one, and the wavefronts of the
   // other blocks take the queries after the long ones in the order of their index.  (Some
@@ -595,11 +621,8 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
     const int cls = class_of(lt);
     const GeoQuery q = queries[(size_t)cls * stride + (lt - curLo)];
     serve_query(gl, nav, q, cls, out, last_cost, T);
-    linkSpills += gl.linkSpills; heapSpills += gl.heapSpills; exactRuns += gl.exactRuns; tieReplays += gl.tieReplays; pairTies += gl.pairTies;
+    T.add(gl, lane, counters);
     if (lane == 0) atomicAdd((unsigned long long*)&counters[kCntLongPath], 1ull);
-#ifdef BPSX_PHASE_TIMING
-    if (lane == 0) for (int k = 0; k < 8; ++k) atomicAdd((unsigned long long*)&counters[8 + k], gl.phase[k]);
-#endif
   }
   geo::GeoWave g;
   g.lane = lane;
@@ -628,20 +651,49 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
     const GeoQuery q = queries[(size_t)cls * stride + (qi - curLo)];
     serve_query(g, nav, q, cls, out, last_cost, T);
   }
-  linkSpills += g.linkSpills; heapSpills += g.heapSpills; exactRuns += g.exactRuns; tieReplays += g.tieReplays; pairTies += g.pairTies;
-  if (lane == 0 && T.done) {
-    atomicAdd((unsigned long long*)&counters[kCntGeoQueries], (unsigned long long)T.done);
-    atomicAdd((unsigned long long*)&counters[kCntAstarPops], (unsigned long long)T.pops);
-    atomicAdd((unsigned long long*)&counters[kCntCorridor], (unsigned long long)T.corridor);
-    if (linkSpills) atomicAdd((unsigned long long*)&counters[kCntLinkSpills], (unsigned long long)linkSpills);
-    if (heapSpills) atomicAdd((unsigned long long*)&counters[kCntHeapSpills], (unsigned long long)heapSpills);
-    if (exactRuns) atomicAdd((unsigned long long*)&counters[kCntExactRuns], (unsigned long long)exactRuns);
-    if (tieReplays) atomicAdd((unsigned long long*)&counters[kCntTieReplays], (unsigned long long)tieReplays);
-    if (pairTies) atomicAdd((unsigned long long*)&counters[kCntPairTies], (unsigned long long)pairTies);
+  T.add(g, lane, counters);
+  T.count(lane, counters);
+}
+
+// The same for launches of few queries: one wavefront per block, three blocks per CU.  Such a launch
+// lasts as long as its longest search, a chain of dependent steps; with every node in LDS no step of it
+// waits for a node that has left a window, hash chains are short, and only the log is written.  (1024
+// agents over room plans, 560 queries: 0.87 ms with a block's 15 KB for each, 0.82 here; 510 agents in two
+// groups: 0.75 and 0.71 each.)
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_geodesic_few(NavData nav, const GeoQuery* __restrict__ queries, uint32_t stride,
+                                                  const uint32_t* __restrict__ counts, uint32_t* head,
+                                                  float* out, uint32_t* last_cost, GeoSlot* slots, uint64_t* counters) {
+  __shared__ __attribute__((aligned(16))) geo_few::GeoShared lds;
+  static_assert(sizeof(geo_few::GeoShared) <= 42 * 1280, "three blocks per CU");
+  geo_few::GeoWave g;
+  g.lane = (int)threadIdx.x;
+  g.L = &lds.a;
+  g.ws = &slots[blockIdx.x];
+  g.nodeCount = 0;
+  g.linkSpills = g.heapSpills = g.exactRuns = g.tieReplays = g.pairTies = 0;
 #ifdef BPSX_PHASE_TIMING
-    for (int k = 0; k < 8; ++k) atomicAdd((unsigned long long*)&counters[8 + k], g.phase[k]);
+  for (int k = 0; k < 8; ++k) g.phase[k] = 0;
 #endif
+  uint32_t nq = 0;
+  for (int c = 0; c < kGeoClasses; ++c) nq += (uint32_t)uniform_i((int)counts[c]);
+  int cls = 0;
+  uint32_t lo = 0, hi = (uint32_t)uniform_i((int)counts[0]);
+  GeoTotals T;
+  // the first query by the block's index, further ones from the counter, the longest classes first
+  for (uint32_t qi = blockIdx.x; qi < nq;) {
+    while (qi >= hi) {
+      cls++;
+      lo = hi;
+      hi += (uint32_t)uniform_i((int)counts[cls]);
+    }
+    const GeoQuery q = queries[(size_t)cls * stride + (qi - lo)];
+    serve_query(g, nav, q, cls, out, last_cost, T);
+    if (g.lane == 0) qi = atomicAdd(head, 1u);
+    qi = gridDim.x + (uint32_t)uniform_i((int)qi);
   }
+  T.add(g, g.lane, counters);
+  T.count(g.lane, counters);
+  if (g.lane == 0 && T.done) atomicAdd((unsigned long long*)&counters[kCntLongPath], (unsigned long long)T.done);
 }
 
 // ---- batched PathFinder-level kernels (one lane per item, or one group per item)
@@ -703,17 +755,27 @@ uint32_t geodesic_blocks_per_cu() {
   if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic, 128, 0) != hipSuccess || n < 1) n = 1;
   return (uint32_t)n;
 }
+uint32_t geodesic_few_blocks_per_cu() {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic_few, 64, 0) != hipSuccess || n < 1) n = 1;
+  return (uint32_t)n;
+}
 
-// num_blocks blocks of two wavefronts; slots holds one GeoSlot per wavefront
+// Where the number of queries to expect is no more than the wavefronts that k_geodesic_few keeps on
+// the device at once it serves them, otherwise k_geodesic.
 void launch_geodesic(const NavData& nav, const GeoQuery* queries, uint32_t stride, const uint32_t* counts, uint32_t* head,
-                     float* out, uint32_t* last_cost, GeoSlot* slots, uint32_t num_blocks,
+                     float* out, uint32_t* last_cost, const GeoPool& G, uint32_t expected,
                      uint64_t* counters, hipStream_t st) {
-  hipLaunchKernelGGL(k_geodesic, dim3(num_blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
-                     last_cost, slots, counters);
+  if (expected <= G.few_blocks)
+    hipLaunchKernelGGL(k_geodesic_few, dim3(G.few_blocks), dim3(64), 0, st, nav, queries, stride, counts, head, out,
+                       last_cost, G.slots, counters);
+  else
+    hipLaunchKernelGGL(k_geodesic, dim3(G.blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
+                       last_cost, G.slots, counters);
 }
 
 void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
-                 const int64_t* actions_dev, GeoSlot* slots, uint32_t geo_blocks, uint32_t snap_blocks, hipStream_t st,
+                 const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st,
                  hipStream_t side, hipEvent_t moved, hipEvent_t snapped, hipEvent_t* ev) {
   int e = 0;
   auto mark = [&]() { if (ev) (void)hipEventRecord(ev[e++], st); };
@@ -738,7 +800,7 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
   if (fork) (void)hipEventRecord(snapped, side);
   mark();
   launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                  A.last_cost, slots, geo_blocks, P.counters, st);
+                  A.last_cost, G, P.n - P.n / 4u, P.counters, st);   // three agents in five ask for a distance in a step
   mark();
   hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, A, P, Q.counts, Qnext.counts);
   if (fork) (void)hipStreamWaitEvent(st, snapped, 0);
@@ -746,13 +808,13 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
 }
 
 void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
-                  GeoSlot* slots, uint32_t geo_blocks, uint32_t snap_blocks, hipStream_t st) {
+                  const GeoPool& G, uint32_t snap_blocks, hipStream_t st) {
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Qother);
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Qother, Qother);
   hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 256), dim3(256), 0, st, nav, A, Q, P);
   hipLaunchKernelGGL(k_reset_snap, dim3(snap_blocks), dim3(128), 0, st, nav, A, Q, Q, P);
   launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                  A.last_cost, slots, geo_blocks, P.counters, st);
+                  A.last_cost, G, P.n, P.counters, st);
   hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, A, P, Q.counts, Qother.counts);
   // the next step finds its lists of queries empty, not with this launch's queries still in them
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Q);
@@ -768,13 +830,13 @@ void launch_try_step_batch(const NavData& nav, uint32_t scene, const float* sxyz
 }
 void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                            const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */, float* out,
-                           GeoSlot* slots, uint32_t geo_blocks, uint64_t* counters, hipStream_t st) {
+                           const GeoPool& G, uint64_t* counters, hipStream_t st) {
   hipLaunchKernelGGL(k_make_queries, grid_for(n, 256), dim3(256), 0, st, scene, sxyz, sref, exyz, eref, n, qbuf);
   // one class only, that of the shortest
   hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n, (uint32_t)kGeoClasses - 1u);
   // stride 0 puts the class's queries at the start of the buffer
-  launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, slots,
-                  geo_blocks, counters, st);
+  launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, G, n,
+                  counters, st);
 }
 void launch_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint32_t slot, uint32_t target, uint32_t envs,
                      hipStream_t st) {
