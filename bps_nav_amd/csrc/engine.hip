@@ -75,7 +75,9 @@ int dev_alloc(T** p, size_t count) {
 // GPU, held until the process ends: the queries built from the caller's arrays, the queue
 // counters, and the node pools of the kStaticBlocks * 2 wavefronts that serve the queue.
 namespace {
-constexpr uint32_t kStaticBlocks = 16;
+// As many pools as k_geodesic_few keeps wavefronts on the device (three on each of 256 CUs): every
+// query of a call of that size has a wavefront of its own, larger calls share them.
+constexpr uint32_t kStaticBlocks = 384;
 constexpr size_t kStaticQueriesBytes = (size_t)BPSX_STATIC_MAX_QUERIES * sizeof(GeoQuery);
 constexpr size_t kStaticCountsBytes = 512;
 static_assert((kGeoClasses + 2) * sizeof(uint32_t) <= kStaticCountsBytes, "queue counters must fit their part");
