@@ -54,15 +54,19 @@ constexpr int kEdgeStride = 8;   // records per polygon in HBM: six edges and tw
 constexpr uint32_t kNoNb = 0xfffeu;   // (not all ones: that is what a lane past the end of its hash chain reads)
 
 // dtBVNode repacked at upload: same quantised bounds; a leaf carries its polygon index, an
-// internal node carries Detour's escape offset (for the in-order walk) and the index of its
-// right child (its left child is the next node), so a wavefront can descend level by level.
+// internal node Detour's escape offset (for the in-order walk).  A scene's nodes are followed by its
+// walkable leaves alone, in the order of the nodes, and those by the bounds of every kSnapGroup of
+// them: what a wavefront snaps points with.
 struct BVNodeDev {
   uint16_t bmin[3], bmax[3];
   uint16_t a;   // leaf: polygon index; internal: escape offset
-  uint16_t b;   // leaf: 0xffff; internal: index of the right child
+  uint16_t b;   // leaf: kBVLeaf; internal: 0
 };
 static_assert(sizeof(BVNodeDev) == 16, "BV node");
 constexpr uint16_t kBVLeaf = 0xffff;
+constexpr uint32_t kSnapGroup = 64;
+constexpr float kSnapCoord = 1024.0f;      // largest coordinate, and how far height samples may lie outside of
+constexpr float kSnapOverhang = 5e-4f;     // their polygon's bounds, in a scene that snap_prune allows
 
 struct SceneDev {
   uint32_t poly_base, poly_count;
@@ -76,8 +80,9 @@ struct SceneDev {
   float qfac;                       // bvQuantFactor
   float climb;                      // walkableClimb
   float area_total;
-  uint32_t bv_tree_ok;              // 1: child links verified, level-by-level descent allowed
-  uint32_t pad[2];
+  uint32_t snap_leaves;             // walkable leaves behind the nodes; 0: the tree does not bound them, it is walked
+  uint32_t snap_prune;              // 1: a polygon is no nearer than its leaf's bounds (verified at load)
+  uint32_t pad;
 };
 
 // ---- per-agent state, structure of arrays over all agents of the simulator

@@ -303,7 +303,8 @@ int bpsx_add_scene(bpsx_sim* sim, const void* navmesh_bytes, size_t navmesh_size
   if (episodes && num_episodes) ps.episodes.assign(episodes, episodes + (size_t)num_episodes * 10);
   ps.parsed->episodes = ps.episodes;
   ps.parsed->dev.ep_count = num_episodes;
-  ps.blob.assign((const uint8_t*)navmesh_bytes, (const uint8_t*)navmesh_bytes + navmesh_size);
+  // the bytes are parsed again when a scene comes back into rotation, and only then
+  if (sim->cfg.rotate_scenes) ps.blob.assign((const uint8_t*)navmesh_bytes, (const uint8_t*)navmesh_bytes + navmesh_size);
   sim->pool.push_back(std::move(ps));
   return BPSX_OK;
 }

@@ -157,15 +157,17 @@ BPSX_DEV float snap_candidate(const NavData& nav, const SceneDev& s, const PolyR
   return dx * dx + dy * dy + dz * dz;
 }
 
+constexpr float kSnapHalf = 2.0f;
 struct SnapBox {
   uint16_t bmin[3], bmax[3];
   bool hit_tile;
 };
 BPSX_DEV float clampf(float v, float lo, float hi) { return v < lo ? lo : (v > hi ? hi : v); }
-BPSX_DEV SnapBox snap_box(const SceneDev& s, float px, float py, float pz) {
+// the query box around a point: the reference's has a half extent of 2 m in x and z
+BPSX_DEV SnapBox snap_box(const SceneDev& s, float px, float py, float pz, float half) {
   SnapBox b;
-  const float qmin[3] = {px - 2.0f, py - 4.0f, pz - 2.0f};
-  const float qmax[3] = {px + 2.0f, py + 4.0f, pz + 2.0f};
+  const float qmin[3] = {px - half, py - 4.0f, pz - half};
+  const float qmax[3] = {px + half, py + 4.0f, pz + half};
   const int minx = (int)floorf((qmin[0] - s.orig[0]) / s.tile_w), miny = (int)floorf((qmin[2] - s.orig[2]) / s.tile_h);
   const int maxx = (int)floorf((qmax[0] - s.orig[0]) / s.tile_w), maxy = (int)floorf((qmax[2] - s.orig[2]) / s.tile_h);
   b.hit_tile = !(s.tx < minx || s.tx > maxx || s.ty < miny || s.ty > maxy);
@@ -177,14 +179,22 @@ BPSX_DEV SnapBox snap_box(const SceneDev& s, float px, float py, float pz) {
   }
   return b;
 }
+BPSX_DEV bool box_overlaps(const SnapBox& box, const BVNodeDev& nd) {
+  bool overlap = true;
+#pragma unroll
+  for (int k = 0; k < 3; ++k)
+    if (box.bmin[k] > nd.bmax[k] || box.bmax[k] < nd.bmin[k]) overlap = false;
+  return overlap;
+}
 
 // snapPoint, one lane per point: BV-tree walk with escape indices, candidates taken in tree
-// order with a strict '<' so the first of equally near polygons wins.
+// order with a strict '<' so the first of equally near polygons wins.  For trees whose inner nodes do
+// not bound what lies below them (see SceneDev::snap_leaves).
 BPSX_DEV NavPt snap_point(const NavData& nav, const SceneDev& s, float px, float py, float pz, uint32_t* ncand) {
   const float qnan = __int_as_float(0x7fc00000);
   NavPt out{qnan, qnan, qnan, 0};
   if (!finite3(px, py, pz)) return out;
-  const SnapBox box = snap_box(s, px, py, pz);
+  const SnapBox box = snap_box(s, px, py, pz, kSnapHalf);
   if (!box.hit_tile) return out;
   float best = 3.402823466e+38f;
   float bp[3] = {0, 0, 0};
@@ -192,10 +202,7 @@ BPSX_DEV NavPt snap_point(const NavData& nav, const SceneDev& s, float px, float
   uint32_t i = 0;
   while (i < s.bv_count) {
     const BVNodeDev nd = nav.bv[s.bv_base + i];
-    bool overlap = true;
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      if (box.bmin[k] > nd.bmax[k] || box.bmax[k] < nd.bmin[k]) overlap = false;
+    const bool overlap = box_overlaps(box, nd);
     const bool leaf = nd.b == kBVLeaf;
     if (leaf && overlap) {
       const PolyRec& r = nav.polys[s.poly_base + (uint32_t)nd.a];
@@ -208,130 +215,6 @@ BPSX_DEV NavPt snap_point(const NavData& nav, const SceneDev& s, float px, float
     }
     if (overlap || leaf) i++;
     else i += (uint32_t)nd.a;
-  }
-  if (bestIp == kInvalidPoly || isnan(bp[0])) return out;
-  out.x = bp[0]; out.y = bp[1]; out.z = bp[2];
-  out.ref = s.ref_base | bestIp;
-  return out;
-}
-
-// snapPoint by a whole wavefront (64 lanes), for callers where few points are snapped at a
-// time.  The BV tree is descended level by level through an LDS frontier (every lane tests
-// one node per round), the leaves that overlap the query box become candidates, each lane
-// evaluates one candidate, and the winner is the smallest (distance, position in the tree's
-// node array): the same polygon the in-order walk with its strict '<' picks.
-constexpr int kSnapFrontier = 1024;
-struct SnapLds {
-  uint16_t frontier[2][kSnapFrontier];
-  uint16_t cand_node[64];   // tree position of the candidates of the current batch
-  uint16_t cand_poly[64];
-};
-BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, float py, float pz, SnapLds& L,
-                               uint32_t* ncand) {
-  const int lane = (int)(threadIdx.x & 63);
-  const float qnan = __int_as_float(0x7fc00000);
-  NavPt out{qnan, qnan, qnan, 0};
-  if (!finite3(px, py, pz)) return out;
-  const SnapBox box = snap_box(s, px, py, pz);
-  if (!box.hit_tile || s.bv_count == 0) return out;
-  if (!s.bv_tree_ok) return snap_point(nav, s, px, py, pz, ncand);  // every lane walks the same tree
-  float best = 3.402823466e+38f;   // per-lane running best
-  uint32_t bestKey = 0xffffffffu;  // tree position of the lane's best candidate
-  uint32_t bestIp = kInvalidPoly;
-  float bp[3] = {0, 0, 0};
-  int ncands = 0;  // candidates waiting in the batch (uniform)
-  auto flush = [&]() {
-    if (lane < ncands) {
-      const uint32_t ip = L.cand_poly[lane];
-      float cp[3];
-      const float d = snap_candidate(nav, s, nav.polys[s.poly_base + ip], px, py, pz, cp);
-      const uint32_t key = L.cand_node[lane];
-      if (d < best || (d == best && d < 3.402823466e+38f && key < bestKey)) {
-        best = d; bestKey = key; bestIp = ip; bp[0] = cp[0]; bp[1] = cp[1]; bp[2] = cp[2];
-      }
-    }
-    *ncand += (uint32_t)ncands;
-    ncands = 0;
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  };
-  // roots: the tree proper and whatever the builder left behind it in the array
-  int nf = 0, cur = 0;
-  {
-    uint32_t k = 0;
-    while (k < s.bv_count && nf < kSnapFrontier) {
-      if (lane == 0) L.frontier[0][nf] = (uint16_t)k;
-      nf++;
-      const BVNodeDev nd = nav.bv[s.bv_base + k];
-      k += nd.b == kBVLeaf ? 1u : (uint32_t)nd.a;
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-  }
-  bool overflow = false;
-  while (nf > 0 && !overflow) {
-    int nnext = 0;
-    for (int basei = 0; basei < nf; basei += 64) {
-      const int fi = basei + lane;
-      bool isCand = false, isInner = false;
-      uint32_t node = 0;
-      BVNodeDev nd{};
-      if (fi < nf) {
-        node = L.frontier[cur][fi];
-        nd = nav.bv[s.bv_base + node];
-        bool overlap = true;
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-          if (box.bmin[k] > nd.bmax[k] || box.bmax[k] < nd.bmin[k]) overlap = false;
-        if (overlap) {
-          if (nd.b == kBVLeaf) isCand = (nav.polys[s.poly_base + nd.a].flags & 1) != 0;
-          else isInner = true;
-        }
-      }
-      // children of overlapping inner nodes go to the next frontier
-      const unsigned long long mi = __ballot(isInner);
-      const int ni = __popcll(mi);
-      if (nnext + 2 * ni > kSnapFrontier) { overflow = true; break; }
-      if (isInner) {
-        const int pos = nnext + 2 * __popcll(mi & ((1ull << lane) - 1ull));
-        L.frontier[cur ^ 1][pos] = (uint16_t)(node + 1);
-        L.frontier[cur ^ 1][pos + 1] = nd.b;
-      }
-      nnext += 2 * ni;
-      // overlapping walkable leaves join the candidate batch; a full batch is evaluated
-      unsigned long long mc = __ballot(isCand);
-      while (mc) {
-        const int room = 64 - ncands;
-        const int take = min(room, (int)__popcll(mc));
-        const int rank = __popcll(mc & ((1ull << lane) - 1ull));
-        if (isCand && rank < take) {
-          L.cand_node[ncands + rank] = (uint16_t)node;
-          L.cand_poly[ncands + rank] = nd.a;
-          isCand = false;
-        }
-        ncands += take;
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        if (ncands == 64) flush();
-        mc = __ballot(isCand);
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    cur ^= 1;
-    nf = nnext;
-  }
-  if (overflow) return snap_point(nav, s, px, py, pz, ncand);
-  if (ncands) flush();
-  // wave-wide minimum of (distance, tree position)
-  for (int o = 32; o > 0; o >>= 1) {
-    const float od = __shfl_xor(best, o);
-    const uint32_t ok = (uint32_t)__shfl_xor((int)bestKey, o);
-    const uint32_t oi = (uint32_t)__shfl_xor((int)bestIp, o);
-    const float o0 = __shfl_xor(bp[0], o), o1 = __shfl_xor(bp[1], o), o2 = __shfl_xor(bp[2], o);
-    const bool mineValid = bestIp != kInvalidPoly, otherValid = oi != kInvalidPoly;
-    const bool takeOther = otherValid && (!mineValid || od < best || (od == best && ok < bestKey));
-    if (takeOther) { best = od; bestKey = ok; bestIp = oi; bp[0] = o0; bp[1] = o1; bp[2] = o2; }
   }
   if (bestIp == kInvalidPoly || isnan(bp[0])) return out;
   out.x = bp[0]; out.y = bp[1]; out.z = bp[2];
@@ -450,6 +333,212 @@ BPSX_DEV bool poly_height(const NavData& nav, const PolyRegs& P, const PolyRec& 
   closest_on_detail_edges<false>(nav, mem, px, py, pz, c);
   h = c[1];
   return true;
+}
+
+// the smallest v of a wavefront, known to be uniform (the totals of a row of 16 lanes through quad
+// permutes and mirrors, then across the rows)
+BPSX_DEV uint32_t wave_umin(uint32_t v) {
+  auto take = [&v](uint32_t o) BPSX_INLINE_LAMBDA { v = o < v ? o : v; };
+  take((uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0xb1 /* quad_perm [1,0,3,2] */, 0xf, 0xf, false));
+  take((uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x4e /* quad_perm [2,3,0,1] */, 0xf, 0xf, false));
+  take((uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x141 /* row_half_mirror */, 0xf, 0xf, false));
+  take((uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x140 /* row_mirror */, 0xf, 0xf, false));
+  take((uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x142 /* row_bcast:15 */, 0xa, 0xf, false));
+  take((uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x143 /* row_bcast:31 */, 0xc, 0xf, false));
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// closest_on_detail_edges<true> on a record in registers.
+BPSX_DEV void closest_on_boundary(const NavData& nav, const PolyRegs& P, float px, float py, float pz, float* out) {
+  float dmin = 3.402823466e+38f, tmin = 0;
+  float lo[3] = {px, py, pz}, hi[3] = {px, py, pz};   // without an edge the point itself
+  const int tc = P.tri_count(), nv = P.nv();
+  const uint32_t* tris = reinterpret_cast<const uint32_t*>(nav.dtris) + P.tri_base();
+  auto corner = [&](uint32_t k, float* o) BPSX_INLINE_LAMBDA {
+    if ((int)k < nv) P.vertex((int)k, o);
+    else {
+      const float* d = &nav.dverts[(size_t)(P.dvert_base() + (k - (uint32_t)nv)) * 3];
+      o[0] = d[0]; o[1] = d[1]; o[2] = d[2];
+    }
+  };
+  uint32_t next = 0 < tc ? tris[0] : 0u;
+  for (int i = 0; i < tc; ++i) {
+    const uint32_t t = next;
+    next = i + 1 < tc ? tris[i + 1] : 0u;
+    if ((t & 0x15000000u) == 0) continue;
+    float v[3][3];
+    corner(t & 0xffu, v[0]); corner((t >> 8) & 0xffu, v[1]); corner((t >> 16) & 0xffu, v[2]);
+    auto edge = [&](uint32_t flag, const float* a, const float* b) BPSX_INLINE_LAMBDA {
+      if (!(t & flag)) return;
+      float u;
+      const float d = dist_pt_seg_sqr2d(px, pz, a, b, u);
+      if (d < dmin) {
+        dmin = d; tmin = u;
+        lo[0] = a[0]; lo[1] = a[1]; lo[2] = a[2];
+        hi[0] = b[0]; hi[1] = b[1]; hi[2] = b[2];
+      }
+    };
+    edge(0x10000000u, v[2], v[0]);
+    edge(0x01000000u, v[0], v[1]);
+    edge(0x04000000u, v[1], v[2]);
+  }
+  if (dmin == 3.402823466e+38f) { out[0] = px; out[1] = py; out[2] = pz; return; }
+  out[0] = lo[0] + (hi[0] - lo[0]) * tmin;
+  out[1] = lo[1] + (hi[1] - lo[1]) * tmin;
+  out[2] = lo[2] + (hi[2] - lo[2]) * tmin;
+}
+
+// snapPoint by a whole wavefront.  The reference takes every walkable polygon whose bounds overlap a
+// box of 4 x 8 x 4 m in the order of the BV tree's array and keeps the first of the nearest ones: the
+// smallest (distance, place in the array).
+//
+// The walkable leaves lie in one array in that order, with the bounds of every 64 of them in another
+// (a run of the tree's in-order array is a compact part of the mesh): all groups' bounds are read at
+// once, then the leaves of the groups that overlap, 64 in one load, then one polygon per lane.  That
+// is four dependent loads where a descent of the binary tree has seventeen.
+//
+// Where the scene allows it (SceneDev::snap_prune) the box begins with a half extent of kSnapFirst and
+// grows: a polygon outside a box of half extent r is at least r - kSnapSlack away, so once the best
+// distance is below that, the reference's box holds no better one and none as good.  In a batch, the
+// polygons that the point is above or below come first, and the boundary of the others is looked at
+// only if their bounds are no farther away than the best so far.
+//
+// Bound by the latency of those loads and by the divide-heavy edge distances of the candidates: most
+// points are on the mesh, and of the 200 polygons of a cluttered plan in the full box five remain.
+// (50000 points over a cluttered plan of 20k polygons: 1730 -> 277 us; 4096 points there, a wavefront
+// each, 64 -> 14 us; snaps of 165 new episodes there next to the searches 135 -> 24 us.  The descent
+// tested one level per load and evaluated the whole box, a field of a record at a time.)
+constexpr float kSnapFirst = 0.25f;
+// above the rounding of interpolated points, distances and boxes at coordinates up to kSnapCoord, and
+// what height samples may lie outside of their polygon's bounds (kSnapOverhang, checked at load)
+constexpr float kSnapSlack = 1e-3f;
+static_assert(kSnapGroup == 64, "a lane per leaf of a group");
+struct SnapLds {
+  uint16_t cand_rank[64];   // place among the leaves of the candidates of the current batch
+  uint16_t cand_poly[64];
+};
+BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, float py, float pz, SnapLds& L,
+                               uint32_t* ncand) {
+  const int lane = (int)(threadIdx.x & 63);
+  const float qnan = __int_as_float(0x7fc00000);
+  constexpr float kNone = 3.402823466e+38f;
+  NavPt out{qnan, qnan, qnan, 0};
+  if (!finite3(px, py, pz)) return out;
+  if (!snap_box(s, px, py, pz, kSnapHalf).hit_tile || s.bv_count == 0) return out;
+  if (!s.snap_leaves) return snap_point(nav, s, px, py, pz, ncand);  // every lane walks the same tree
+  const uint32_t nleaves = s.snap_leaves, ngroups = (nleaves + 63u) / 64u;
+  const BVNodeDev* leaves = nav.bv + s.bv_base + s.bv_count;
+  const BVNodeDev* groups = leaves + nleaves;
+  const bool prune = s.snap_prune && fabsf(px) <= 2.0f * kSnapCoord && fabsf(pz) <= 2.0f * kSnapCoord;
+  float best = kNone;              // per-lane running best
+  uint32_t bestKey = 0xffffffffu;  // place of the lane's best candidate
+  uint32_t bestIp = kInvalidPoly;
+  float bp[3] = {0, 0, 0};
+  int ncands = 0;  // candidates waiting in the batch (uniform)
+  auto flush = [&]() {
+    const bool have = lane < ncands;
+    *ncand += (uint32_t)ncands;
+    ncands = 0;
+    uint32_t ip = 0, key = 0;
+    PolyRegs P;
+    const PolyRec* rec = nullptr;
+    bool inside = false;
+    float h = 0;
+    auto take = [&](float d, float x, float y, float z) BPSX_INLINE_LAMBDA {
+      if (d < best || (d == best && d < kNone && key < bestKey)) {
+        best = d; bestKey = key; bestIp = ip; bp[0] = x; bp[1] = y; bp[2] = z;
+      }
+    };
+    if (have) {
+      ip = L.cand_poly[lane];
+      key = L.cand_rank[lane];
+      rec = &nav.polys[s.poly_base + ip];
+      P.load(rec);
+      inside = poly_height(nav, P, *rec, px, py, pz, h);
+      if (inside) {
+        const float d = fabsf(py - h) - s.climb;
+        take(d > 0 ? d * d : 0, px, h, pz);
+      }
+    }
+    const float reached = __uint_as_float(wave_umin(__float_as_uint(best)));
+    if (have && !inside) {
+      float x0 = P.x<0>(), x1 = x0, z0 = P.z<0>(), z1 = z0;
+      const int nv = P.nv();
+      static_for<1, kNvp>([&](auto I) BPSX_INLINE_LAMBDA {
+        constexpr int i = decltype(I)::value;
+        if (i < nv) {
+          x0 = fminf(x0, P.x<i>()); x1 = fmaxf(x1, P.x<i>());
+          z0 = fminf(z0, P.z<i>()); z1 = fmaxf(z1, P.z<i>());
+        }
+      });
+      const float bx = fmaxf(fmaxf(x0 - px, px - x1) - kSnapSlack, 0.0f), bz = fmaxf(fmaxf(z0 - pz, pz - z1) - kSnapSlack, 0.0f);
+      if (!(prune && bx * bx + bz * bz > reached)) {
+        float cp[3];
+        closest_on_boundary(nav, P, px, py, pz, cp);
+        const float dx = px - cp[0], dy = py - cp[1], dz = pz - cp[2];
+        take(dx * dx + dy * dy + dz * dz, cp[0], cp[1], cp[2]);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  float half = prune ? kSnapFirst : kSnapHalf;
+  SnapBox box = snap_box(s, px, py, pz, half), before = box;
+  bool grown = false;   // what overlaps `before` has been looked at
+  for (;;) {
+    for (uint32_t g0 = 0; g0 < ngroups; g0 += 64) {
+      const uint32_t g = g0 + (uint32_t)lane;
+      const BVNodeDev gr = groups[g < ngroups ? g : ngroups - 1u];
+      unsigned long long mg = __ballot(g < ngroups && box_overlaps(box, gr));
+      while (mg) {
+        const uint32_t at = (g0 + (uint32_t)__builtin_ctzll(mg)) * 64u + (uint32_t)lane;
+        mg &= mg - 1ull;
+        const BVNodeDev nd = leaves[at < nleaves ? at : nleaves - 1u];
+        bool isCand = at < nleaves && box_overlaps(box, nd) && !(grown && box_overlaps(before, nd));
+        // they join the candidate batch; a full batch is evaluated
+        unsigned long long mc = __ballot(isCand);
+        while (mc) {
+          const int room = 64 - ncands, found = (int)__popcll(mc);
+          const int fit = room < found ? room : found;
+          const int rank = __popcll(mc & ((1ull << lane) - 1ull));
+          if (isCand && rank < fit) {
+            L.cand_rank[ncands + rank] = (uint16_t)at;
+            L.cand_poly[ncands + rank] = nd.a;
+            isCand = false;
+          }
+          ncands += fit;
+          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          if (ncands == 64) flush();
+          mc = __ballot(isCand);
+        }
+      }
+    }
+    if (ncands) flush();
+    if (half >= kSnapHalf) break;
+    const float reached = __uint_as_float(wave_umin(__float_as_uint(best)));
+    const float clear = half - kSnapSlack;
+    if (reached < clear * clear) break;
+    // the next box reaches as far as the best so far, or is three times as wide
+    half = fminf(reached < kNone ? sqrtf(reached) * 1.0001f + 2.0f * kSnapSlack : 3.0f * half, kSnapHalf);
+    before = box;
+    grown = true;
+    box = snap_box(s, px, py, pz, half);
+  }
+  // the smallest (distance, place in the array)
+  const uint32_t dist = wave_umin(__float_as_uint(best));
+  const bool nearest = bestIp != kInvalidPoly && __float_as_uint(best) == dist;
+  const uint32_t key = wave_umin(nearest ? bestKey : 0xffffffffu);
+  const unsigned long long won = __ballot(nearest && bestKey == key);
+  if (!won) return out;
+  const int w = __builtin_ctzll(won);
+  const float x = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bp[0]), w));
+  if (isnan(x)) return out;
+  out.x = x;
+  out.y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bp[1]), w));
+  out.z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bp[2]), w));
+  out.ref = s.ref_base | (uint32_t)__builtin_amdgcn_readlane((int)bestIp, w);
+  return out;
 }
 
 // The tiny node pool and the queue of moveAlongSurface, one column per lane of a wavefront, in

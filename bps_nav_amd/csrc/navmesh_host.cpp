@@ -5,6 +5,7 @@
 // instead of Detour's pointer-linked tile.  Only single-tile meshes are accepted.
 #include "navmesh_host.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <initializer_list>
@@ -14,6 +15,96 @@
 #include "errors.h"
 
 namespace bpsx {
+
+namespace {
+
+// The walkable leaves of the BV tree in the order of its array, then the bounds of every kSnapGroup of
+// them, behind the nodes.  Testing each leaf finds what the in-order walk finds when no inner node
+// hides a leaf from a box that the leaf overlaps, i.e. when every node lies within the bounds of the
+// inner nodes around it; the builder's trees do, and where one does not the kernels walk it.  (The
+// builder reserves 2N nodes and uses 2N - 1: the last is a zero leaf outside the tree, which the
+// in-order walk visits, so it is among the leaves here.)
+// snap_prune: a polygon's own extents quantise to within its leaf's bounds, the way the query's box is
+// quantised, and so do its height samples up to kSnapOverhang; it has a boundary edge (without one
+// the reference calls it 0 away from everywhere); and coordinates are small enough for kSnapSlack.
+void append_snap_leaves(HostScene& s) {
+  SceneDev& d = s.dev;
+  d.snap_leaves = d.snap_prune = 0;
+  const size_t n = s.bv.size();
+  // quantised coordinates must neither wrap nor fall where coordinates grow
+  bool prune = d.qfac > 0;
+  for (int k = 0; k < 3; k += 2)
+    prune = prune && std::fabs(d.bmin[k]) <= kSnapCoord && std::fabs(d.bmax[k]) <= kSnapCoord && d.bmin[k] <= d.bmax[k] &&
+            d.qfac * (d.bmax[k] - d.bmin[k]) + 1 < 65535.0f;
+  auto quantised = [&](float v, int k, float add) {
+    const float c = v < d.bmin[k] ? d.bmin[k] : (v > d.bmax[k] ? d.bmax[k] : v);
+    return (uint16_t)(int)(d.qfac * (c - d.bmin[k]) + add);
+  };
+  std::vector<bool> bounded(s.polys.size(), false);
+  auto leaf_bounds = [&](const BVNodeDev& nd, const PolyRec& r) {
+    float lo[3], hi[3];
+    for (int k = 0; k < 3; ++k) lo[k] = hi[k] = r.v[0][k];
+    bool finite = true;
+    for (int i = 0; i < r.nv; ++i)
+      for (int k = 0; k < 3; ++k) {
+        finite &= std::fabs(r.v[i][k]) <= kSnapCoord;
+        lo[k] = std::min(lo[k], r.v[i][k]);
+        hi[k] = std::max(hi[k], r.v[i][k]);
+      }
+    if (!finite) return false;
+    for (int i = 0; i < r.dvert_count; ++i)
+      for (int k = 0; k < 3; ++k) {
+        const float v = s.dverts[(size_t)(r.dvert_base + i) * 3 + k];
+        if (!(std::fabs(v) <= kSnapCoord)) return false;
+        if (k != 1 && !(v >= lo[k] - kSnapOverhang && v <= hi[k] + kSnapOverhang)) return false;
+      }
+    bool boundary = false;
+    for (int j = 0; j < r.tri_count && !boundary; ++j) boundary = (s.dtris[(size_t)(r.tri_base + j) * 4 + 3] & 0x15) != 0;
+    if (!boundary) return false;
+    // (a further leaf of a polygon, like the zero leaf, never wins where the first one is looked at)
+    if (bounded[nd.a]) return true;
+    bounded[nd.a] = true;
+    for (int k = 0; k < 3; k += 2)
+      if (nd.bmax[k] < (quantised(hi[k], k, 0.0f) & 0xfffe) || nd.bmin[k] > (quantised(lo[k], k, 1.0f) | 1)) return false;
+    return true;
+  };
+  auto within = [](const BVNodeDev& in, const BVNodeDev& out) {
+    bool ok = true;
+    for (int k = 0; k < 3; ++k) ok &= in.bmin[k] >= out.bmin[k] && in.bmax[k] <= out.bmax[k];
+    return ok;
+  };
+  auto nodes_of = [&](size_t i) { return s.bv[i].b == kBVLeaf ? (size_t)1 : (size_t)s.bv[i].a; };
+  std::vector<BVNodeDev> groups;
+  size_t count = 0;
+  for (size_t i = 0; i < n; ++i) {
+    const BVNodeDev nd = s.bv[i];
+    if (nd.b != kBVLeaf) {
+      // two children that fill the node's range, each within its bounds
+      const size_t left = i + 1, end = i + nd.a, right = left < n ? left + nodes_of(left) : n;
+      if (right >= end || right >= n || right + nodes_of(right) != end || !within(s.bv[left], nd) || !within(s.bv[right], nd)) {
+        s.bv.resize(n);
+        return;
+      }
+      continue;
+    }
+    const PolyRec& r = s.polys[nd.a];
+    if (!(r.flags & kPolyFlagWalk)) continue;
+    s.bv.push_back(nd);
+    if (count++ % kSnapGroup == 0) groups.push_back(nd);
+    BVNodeDev& g = groups.back();
+    for (int k = 0; k < 3; ++k) {
+      g.bmin[k] = std::min(g.bmin[k], nd.bmin[k]);
+      g.bmax[k] = std::max(g.bmax[k], nd.bmax[k]);
+    }
+    prune = prune && leaf_bounds(nd, r);
+  }
+  if (!count || count > 0xffff) { s.bv.resize(n); return; }
+  s.bv.insert(s.bv.end(), groups.begin(), groups.end());
+  d.snap_leaves = (uint32_t)count;
+  d.snap_prune = prune ? 1u : 0u;
+}
+
+}  // namespace
 
 int parse_navmesh(const uint8_t* b, size_t n, HostScene* out) {
   if (!b || !out) return fail(BPSX_E_INVAL, "navmesh: null argument");
@@ -146,59 +237,29 @@ int parse_navmesh(const uint8_t* b, size_t n, HostScene* out) {
     }
     if ((double)area < 1e-5) r.flags = kPolyFlagDisabled;
   }
-  // neighbours that pass the query filter (include WALK, exclude nothing)
-  for (int i = 0; i < np; ++i) {
-    PolyRec& r = s.polys[i];
-    for (int k = 0; k < r.nv; ++k) {
-      const uint16_t ne = r.nei[k];
-      r.walk[k] = (ne && !(ne & kExtLink) && (s.polys[ne - 1].flags & kPolyFlagWalk)) ? ne : 0;
-    }
-  }
-  // per-edge records of the path search
-  s.aedges.assign((size_t)np * kEdgeStride, AEdge{{0, 0, 0}, kNoNb});
-  for (int i = 0; i < np; ++i) {
-    const PolyRec& r = s.polys[i];
-    for (int k = 0; k < r.nv; ++k) {
-      AEdge& e = s.aedges[(size_t)i * kEdgeStride + k];
-      const float* l = r.v[k];
-      const float* rt = r.v[(k + 1) % r.nv];
-      for (int c = 0; c < 3; ++c) e.mid[c] = (l[c] + rt[c]) * 0.5f;
-      e.nb = r.walk[k] ? (uint32_t)(r.walk[k] - 1) : kNoNb;
-      // a polygon behind two edges: expanding through the second never changes its node (same
-      // position, not a lower cost), so only the first edge leads there
-      for (int j = 0; j < k; ++j)
-        if (r.walk[j] == r.walk[k]) e.nb = kNoNb;
-    }
-  }
-  // connected components: polygons are seeded in index order, the seed is not filter-checked,
-  // neighbours are entered in ascending edge order and popped last-in first-out
-  {
-    std::vector<int> isl((size_t)np, -1), stack;
-    int next = 0;
-    for (int sd = 0; sd < np; ++sd) {
-      if (isl[sd] >= 0) continue;
-      const int id = next++;
-      isl[sd] = id;
-      stack.push_back(sd);
-      while (!stack.empty()) {
-        const int ip = stack.back();
-        stack.pop_back();
-        const PolyRec& r = s.polys[ip];
-        for (int k = 0; k < r.nv; ++k) {
-          if (!r.walk[k]) continue;
-          const int nb = r.walk[k] - 1;
-          if (isl[nb] >= 0) continue;
-          isl[nb] = id;
-          stack.push_back(nb);
-        }
-      }
-    }
-    for (int i = 0; i < np; ++i) s.polys[i].island = (uint32_t)isl[i];
-  }
-  // prefix sums of the fan areas that findRandomPoint weighs polygons by
+  // What depends on which polygons pass the query filter (include WALK, exclude nothing), polygon by
+  // polygon: the neighbours that do; the per-edge records of the path search; the prefix sums of the fan
+  // areas that findRandomPoint weighs polygons by
+  s.aedges.reserve((size_t)np * kEdgeStride);
   float acc = 0.0f;
   for (int i = 0; i < np; ++i) {
     PolyRec& r = s.polys[i];
+    AEdge e[kEdgeStride];
+    for (AEdge& x : e) x = AEdge{{0, 0, 0}, kNoNb};
+    for (int k = 0; k < r.nv; ++k) {
+      const uint16_t ne = r.nei[k];
+      r.walk[k] = (ne && !(ne & kExtLink) && (s.polys[ne - 1].flags & kPolyFlagWalk)) ? ne : 0;
+      const float* l = r.v[k];
+      const float* rt = r.v[k + 1 < r.nv ? k + 1 : 0];
+      for (int c = 0; c < 3; ++c) e[k].mid[c] = (l[c] + rt[c]) * 0.5f;
+      if (!r.walk[k]) continue;
+      // a polygon behind two edges: expanding through the second never changes its node (same
+      // position, not a lower cost), so only the first edge leads there
+      bool first = true;
+      for (int j = 0; j < k; ++j) first &= r.walk[j] != r.walk[k];
+      if (first) e[k].nb = (uint32_t)(r.walk[k] - 1);
+    }
+    s.aedges.insert(s.aedges.end(), e, e + kEdgeStride);
     if (r.type == 0 && (r.flags & kPolyFlagWalk)) {
       float a = 0.0f;
       for (int j = 2; j < r.nv; ++j) {
@@ -210,46 +271,50 @@ int parse_navmesh(const uint8_t* b, size_t n, HostScene* out) {
     }
     r.area_cum = acc;
   }
-
-  // BV tree: repack dtBVNode (bounds + int) into BVNodeDev.  Leaves must name valid polygons;
-  // an internal node at i with escape e owns nodes (i, i+e): its left child is i+1 and its
-  // right child follows the left subtree.  The links are verified so that the kernels'
-  // descent always moves to larger indices inside the array.
-  s.bv.assign((size_t)h.bvNodeCount, BVNodeDev{});
-  bool tree_ok = h.bvNodeCount > 0;
+  // connected components: polygons are seeded in index order, the seed is not filter-checked,
+  // neighbours are entered in ascending edge order and popped last-in first-out
   {
-    std::vector<TileBVNode> raw((size_t)h.bvNodeCount);
-    if (h.bvNodeCount) memcpy(raw.data(), bvp, (size_t)h.bvNodeCount * sizeof(TileBVNode));
-    const int64_t cnt = h.bvNodeCount;
-    auto size_of = [&](int64_t i) -> int64_t { return raw[(size_t)i].i >= 0 ? 1 : -(int64_t)raw[(size_t)i].i; };
-    for (int64_t i = 0; i < cnt; ++i) {
-      const TileBVNode& r = raw[(size_t)i];
-      BVNodeDev& o = s.bv[(size_t)i];
-      memcpy(o.bmin, r.bmin, 6);
-      memcpy(o.bmax, r.bmax, 6);
-      if (r.i >= 0) {
-        if (r.i >= np) return fail(BPSX_E_INVAL, "navmesh: BV leaf out of range");
-        o.a = (uint16_t)r.i;
-        o.b = kBVLeaf;
-      } else {
-        const int64_t e = -(int64_t)r.i;
-        if (e < 1 || e > 0xfffe) return fail(BPSX_E_INVAL, "navmesh: BV escape offset out of range");
-        o.a = (uint16_t)e;
-        const int64_t left = i + 1;
-        const int64_t right = left < cnt ? left + size_of(left) : cnt;
-        if (left >= cnt || right >= cnt || right >= i + e || right + size_of(right) != i + e) {
-          tree_ok = false;
-          o.b = (uint16_t)(left < cnt ? left : 0);
-        } else {
-          o.b = (uint16_t)right;
+    constexpr uint32_t kUnlabelled = 0xffffffffu;
+    for (PolyRec& r : s.polys) r.island = kUnlabelled;
+    std::vector<uint16_t> stack((size_t)np);   // a polygon is entered once
+    uint32_t next = 0;
+    for (int sd = 0; sd < np; ++sd) {
+      if (s.polys[sd].island != kUnlabelled) continue;
+      const uint32_t id = next++;
+      s.polys[sd].island = id;
+      size_t top = 0;
+      stack[top++] = (uint16_t)sd;
+      while (top) {
+        const PolyRec& r = s.polys[stack[--top]];
+        for (int k = 0; k < r.nv; ++k) {
+          if (!r.walk[k]) continue;
+          PolyRec& to = s.polys[r.walk[k] - 1];
+          if (to.island != kUnlabelled) continue;
+          to.island = id;
+          stack[top++] = (uint16_t)(r.walk[k] - 1);
         }
       }
     }
-    // the builder reserves 2N nodes and uses 2N-1: the rest are zero leaves outside the tree;
-    // the in-order walk visits them, so the descent must too (they are appended to its frontier)
-    if (tree_ok) {
-      const int64_t root_size = size_of(0);
-      if (root_size > cnt) tree_ok = false;
+  }
+
+  // BV tree: repack dtBVNode (bounds + int) into BVNodeDev.  Leaves must name valid polygons.
+  s.bv.reserve((size_t)h.bvNodeCount + (size_t)h.bvNodeCount / 2 + (size_t)h.bvNodeCount / (2 * kSnapGroup) + 2);   // and its leaves
+  s.bv.resize((size_t)h.bvNodeCount);
+  for (size_t i = 0; i < s.bv.size(); ++i) {
+    TileBVNode r;
+    memcpy(&r, bvp + i * sizeof(r), sizeof(r));
+    BVNodeDev& o = s.bv[i];
+    memcpy(o.bmin, r.bmin, 6);
+    memcpy(o.bmax, r.bmax, 6);
+    if (r.i >= 0) {
+      if (r.i >= np) return fail(BPSX_E_INVAL, "navmesh: BV leaf out of range");
+      o.a = (uint16_t)r.i;
+      o.b = kBVLeaf;
+    } else {
+      const int64_t e = -(int64_t)r.i;
+      if (e < 1 || e > 0xfffe) return fail(BPSX_E_INVAL, "navmesh: BV escape offset out of range");
+      o.a = (uint16_t)e;
+      o.b = 0;
     }
   }
 
@@ -268,7 +333,7 @@ int parse_navmesh(const uint8_t* b, size_t n, HostScene* out) {
   d.qfac = h.bvQuantFactor;
   d.climb = h.walkableClimb;
   d.area_total = acc;
-  d.bv_tree_ok = tree_ok ? 1u : 0u;
+  append_snap_leaves(s);
   return BPSX_OK;
 }
 
