@@ -1,7 +1,7 @@
 // HIP kernels of the batch environment step (gfx950) and their launch wrappers.
 //
 // One step of a group of n agents is four launches:
-//   step_move      lane per agent: action, turn / forward move with wall sliding, polar
+//   step_move      row of eight lanes per agent: action, turn / forward move with wall sliding, polar
 //                  observation, and a geodesic query (goal -> agent) when the agent moved or
 //                  the episode ended; an agent whose episode ended also picks its next episode
 //                  here and is queued for reset (simulator.cpp:620-632, 651-710, 601-610)
@@ -104,41 +104,38 @@ BPSX_DEV void write_polar(const AgentArrays& A, uint32_t gi, const float* pos, c
   A.polars[(size_t)gi * 2 + 1] = -atan2f(y, x);
 }
 
-// Appends one item per lane with `pred` to a queue: one atomic per wavefront.
-BPSX_DEV uint32_t wave_append(bool pred, uint32_t* counter) {
-  const unsigned long long m = __ballot(pred);
-  if (!m) return 0;
-  const int lane = (int)(threadIdx.x & 63);
-  const int leader = __ffsll((long long)m) - 1;
-  uint32_t base = 0;
-  if (lane == leader) base = atomicAdd(counter, (uint32_t)__popcll(m));
-  base = (uint32_t)__shfl((int)base, leader);
-  return base + (uint32_t)__popcll(m & ((1ull << lane) - 1ull));
-}
-
 BPSX_DEV void load3(const float* p, size_t i, float* o) { o[0] = p[i * 3]; o[1] = p[i * 3 + 1]; o[2] = p[i * 3 + 2]; }
 BPSX_DEV void store3(float* p, size_t i, const float* v) { p[i * 3] = v[0]; p[i * 3 + 1] = v[1]; p[i * 3 + 2] = v[2]; }
 
 // Exploration::InfoFunctor::update (simulator.cpp:897-904): the cell of the agent in the frame
-// of the episode's start pose joins the episode's set.  Returns the set's size.
-BPSX_DEV uint32_t visit_cell(const AgentArrays& A, uint32_t gi, const float* pos) {
-  float ip[3], iq[4];
-  load3(A.exp_init, gi, ip);
-  for (int k = 0; k < 4; ++k) iq[k] = A.exp_inv[(size_t)gi * 4 + k];
+// of the episode's start pose (position ip, inverse rotation iq) ...
+BPSX_DEV void cell_of(const float* ip, const float* iq, const float* pos, int32_t* c) {
   const float d[3] = {pos[0] - ip[0], pos[1] - ip[1], pos[2] - ip[2]};
   float g[3];
   quat_rotate(iq, d, g);
   // int(x) of the reference; for a value no int32 holds (or NaN) the x86 conversion the
   // reference compiles to gives INT32_MIN, the GPU's would saturate: made explicit
-  auto cell = [](float x) { return (x > -2147483648.0f && x < 2147483648.0f) ? (int32_t)x : (int32_t)0x80000000; };
-  const int32_t c0 = cell(g[0] / 1.0f), c1 = cell(g[1] / 1.0f), c2 = cell(g[2] / 1.0f);
+  for (int k = 0; k < 3; ++k) {
+    const float x = g[k] / 1.0f;
+    c[k] = (x > -2147483648.0f && x < 2147483648.0f) ? (int32_t)x : (int32_t)0x80000000;
+  }
+}
+// ... joins the episode's set of n cells.  Returns the set's size.  By a row of eight lanes, eight cells
+// at a time (an agent that wanders for hundreds of steps has entered up to a hundred).
+BPSX_DEV uint32_t visit_cell(const Row& row, const AgentArrays& A, uint32_t gi, uint32_t n, const float* ip, const float* iq, const float* pos) {
+  int32_t c[3];
+  cell_of(ip, iq, pos, c);
   int32_t* cells = A.exp_cells + (size_t)gi * A.cell_cap * 3;
-  const uint32_t n = A.exp_count[gi];
-  for (uint32_t i = 0; i < n; ++i)
-    if (cells[i * 3] == c0 && cells[i * 3 + 1] == c1 && cells[i * 3 + 2] == c2) return n;
+  for (uint32_t i = 0; i < n; i += 8) {
+    const uint32_t k = i + (uint32_t)row.el;
+    const int32_t* o = &cells[(size_t)(k < n ? k : i) * 3];
+    if (row.mask(o[0] == c[0] && o[1] == c[1] && o[2] == c[2])) return n;
+  }
   if (n >= A.cell_cap) return n;   // cannot happen: one update per step and per reset
-  cells[n * 3] = c0; cells[n * 3 + 1] = c1; cells[n * 3 + 2] = c2;
-  A.exp_count[gi] = n + 1;
+  if (row.el == 0) {
+    for (int k = 0; k < 3; ++k) cells[(size_t)n * 3 + k] = c[k];
+    A.exp_count[gi] = n + 1;
+  }
   return n + 1;
 }
 
@@ -160,26 +157,22 @@ __global__ void k_clear_queues(StepQueues Q, StepQueues R) {
   }
 }
 
-// Picks the next episode of agent gi and writes its pose; the snaps follow in reset_snap.
-BPSX_DEV void begin_reset(const NavData& nav, const AgentArrays& A, const StepParams& P, uint32_t gi) {
-  const uint32_t count = A.nresets[gi];
-  A.nresets[gi] = count + 1;
-  A.step[gi] = 1;
-  A.last_cost[gi] = kCostUnknown;
-  const uint32_t sc = A.scene[gi];
+// Picks the next episode of agent gi in scene-table entry sc and writes its pose; the snaps follow in
+// reset_snap.  By a row of eight lanes; count: the agent's resets so far.
+BPSX_DEV void begin_reset(const Row& row, const NavData& nav, const AgentArrays& A, const StepParams& P, uint32_t gi, uint32_t sc,
+                          uint32_t count) {
   const SceneDev& s = nav.scenes[sc];
   const uint64_t key = reset_key(P.seed, gi, count);
   float ep[10];
+  uint32_t e = 0;
   if (P.reset_mode == 0) {
-    const uint32_t e = draw_index(reset_draw(key, 0), s.ep_count);
-    A.episode[gi] = e;
+    e = draw_index(reset_draw(key, 0), s.ep_count);
     for (int k = 0; k < 10; ++k) ep[k] = nav.episodes[(size_t)(s.ep_base + e) * 10 + k];
   } else {
-    A.episode[gi] = 0;
     float a[3] = {0, 0, 0}, b[3] = {0, 0, 0};
     uint32_t ip;
-    sample_point(nav, s, draw_unit(reset_draw(key, 0)), draw_unit(reset_draw(key, 1)), draw_unit(reset_draw(key, 2)), a, &ip);
-    sample_point(nav, s, draw_unit(reset_draw(key, 3)), draw_unit(reset_draw(key, 4)), draw_unit(reset_draw(key, 5)), b, &ip);
+    sample_point_row(row, nav, s, draw_unit(reset_draw(key, 0)), draw_unit(reset_draw(key, 1)), draw_unit(reset_draw(key, 2)), a, &ip);
+    sample_point_row(row, nav, s, draw_unit(reset_draw(key, 3)), draw_unit(reset_draw(key, 4)), draw_unit(reset_draw(key, 5)), b, &ip);
     const uint32_t turns = draw_index(reset_draw(key, 6), 36);
     float q[4] = {0, 0, 0, 1};
     for (uint32_t t = 0; t < turns; ++t) quat_mul(q, P.turn_left, q);
@@ -187,15 +180,38 @@ BPSX_DEV void begin_reset(const NavData& nav, const AgentArrays& A, const StepPa
     ep[3] = q[0]; ep[4] = q[1]; ep[5] = q[2]; ep[6] = q[3];
     ep[7] = b[0]; ep[8] = b[1]; ep[9] = b[2];
   }
+  if (row.el != 0) return;
+  A.nresets[gi] = count + 1;
+  A.step[gi] = 1;
+  A.last_cost[gi] = kCostUnknown;
+  A.episode[gi] = e;
   store3(A.pos, gi, ep);
   for (int k = 0; k < 4; ++k) A.rot[(size_t)gi * 4 + k] = ep[3 + k];
   store3(A.goal, gi, ep + 7);
 }
 
-__global__ __launch_bounds__(64) void k_step_move(NavData nav, AgentArrays A, StepQueues Q, StepParams P,
+// A row of eight lanes per agent, kMoveItems agents per block: all lanes of a row read the agent's state
+// and decide alike, the first one writes it.  Bound by latency, a chain of dependent loads (state,
+// scene, polygon, its neighbours, height mesh), which is why the loads of one link go out together.
+// (With a lane per agent: 33 us for 64 agents in a room, now 12; 1017 agents 41 -> 13; 16384 agents over
+// mazes 35 -> 22; 4096 over cluttered plans with sampled resets, whose two searches for a polygon were
+// thirty dependent reads, 79 -> 30; 65536 over mixed scenes 65, as before.)
+struct MoveQueueLds {
+  uint32_t count[kGeoClasses + 1], base[kGeoClasses + 1];   // of the block's queries per class, and of its resets
+  uint32_t forward, polys;
+};
+__global__ __launch_bounds__(kMoveItems * 8) void k_step_move(NavData nav, AgentArrays A, StepQueues Q, StepParams P,
                                                    const int64_t* __restrict__ actions) {
   __shared__ MoveLds move_lds;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ __attribute__((aligned(16))) uint16_t entered[kMoveItems][kTinyNodes];
+  __shared__ MoveQueueLds queue;
+  static_assert(kGeoClasses + 1 <= kMoveItems * 8, "a thread per class");
+  if (threadIdx.x <= (uint32_t)kGeoClasses) queue.count[threadIdx.x] = 0;
+  if (threadIdx.x == 0) queue.forward = queue.polys = 0;
+  __syncthreads();
+  const Row row;
+  const uint32_t item = threadIdx.x >> 3, i = blockIdx.x * kMoveItems + item;
+  const bool lead = row.el == 0;
   bool want = false, reset = false;
   uint32_t cls = 0;
   GeoQuery q{};
@@ -205,8 +221,10 @@ __global__ __launch_bounds__(64) void k_step_move(NavData nav, AgentArrays A, St
     const int64_t action = actions[i];
     if (action < 0 || action > 3) {
       // the reference aborts here (simulator.cpp:704-708); flag it and leave the agent alone
-      atomicOr(P.error_flag, 1u);
-      A.flags[gi] = kAgentSkip;
+      if (lead) {
+        atomicOr(P.error_flag, 1u);
+        A.flags[gi] = kAgentSkip;
+      }
     } else {
       // Everything the step may need of the agent is read here, before the first store: the
       // loads then go out together instead of one dependent round trip after the other.
@@ -222,7 +240,16 @@ __global__ __launch_bounds__(64) void k_step_move(NavData nav, AgentArrays A, St
       const uint32_t goalRef = A.goal_ref[gi];
       const bool distOk = A.dist_ok[gi] == 1;
       const uint32_t expected = A.last_cost[gi];
-      A.step[gi] = step;
+      const uint32_t resets = A.nresets[gi];
+      const bool explore = P.task == BPSX_TASK_EXPLORATION;
+      uint32_t cnt = 0;
+      float ip[3] = {0, 0, 0}, iq[4] = {0, 0, 0, 0};
+      if (explore) {
+        cnt = A.exp_count[gi];
+        load3(A.exp_init, gi, ip);
+        for (int k = 0; k < 4; ++k) iq[k] = A.exp_inv[(size_t)gi * 4 + k];
+      }
+      if (lead) A.step[gi] = step;
       bool done = (float)step >= P.max_steps;
       bool moved = false;
       // The goal->agent distance is a deterministic function of the two navmesh points. When
@@ -238,32 +265,34 @@ __global__ __launch_bounds__(64) void k_step_move(NavData nav, AgentArrays A, St
           quat_rotate(rot, fwd, delta);
           const SceneDev& s = nav.scenes[scene0];
           const NavPt st{navNow[0], navNow[1], navNow[2], navRefNow};
-          const NavPt r = try_step(nav, s, st, pos[0] + delta[0], pos[1] + delta[1], pos[2] + delta[2], &movePolys, move_lds);
+          const NavPt r = try_step_row(row, nav, s, st, pos[0] + delta[0], pos[1] + delta[1], pos[2] + delta[2], &movePolys,
+                                       entered[item], move_lds, (int)item);
           samePoint = __float_as_uint(r.x) == __float_as_uint(st.x) && __float_as_uint(r.y) == __float_as_uint(st.y) &&
                       __float_as_uint(r.z) == __float_as_uint(st.z) && r.ref == st.ref;
           pos[0] = r.x; pos[1] = r.y; pos[2] = r.z;
           navNow[0] = r.x; navNow[1] = r.y; navNow[2] = r.z;
           navRefNow = r.ref;
-          store3(A.nav_xyz, gi, pos);
-          A.nav_ref[gi] = r.ref;
-          store3(A.pos, gi, pos);
+          if (lead) {
+            store3(A.nav_xyz, gi, pos);
+            A.nav_ref[gi] = r.ref;
+            store3(A.pos, gi, pos);
+          }
           moved = true;
         } else {
           quat_mul(rot, action == 2 ? P.turn_left : P.turn_right, rot);
-          for (int k = 0; k < 4; ++k) A.rot[(size_t)gi * 4 + k] = rot[k];
+          if (lead) for (int k = 0; k < 4; ++k) A.rot[(size_t)gi * 4 + k] = rot[k];
         }
-        write_polar(A, gi, pos, rot, goal);
+        if (lead) write_polar(A, gi, pos, rot, goal);
       }
       // PointNav measures the distance on every move and at the end of the episode, Flee on
       // moves only, Exploration never (simulator.cpp:758-790, 845-856, 918-927)
       const bool measure = P.task == BPSX_TASK_POINTNAV ? (done || moved) : (P.task == BPSX_TASK_FLEE && moved);
       const bool reuse = measure && samePoint && distOk;
-      A.flags[gi] = (done ? kAgentDone : 0u) | (moved ? kAgentMoved : 0u) | (reuse ? kAgentReuse : 0u);
-      if (P.task == BPSX_TASK_EXPLORATION) {
+      if (lead) A.flags[gi] = (done ? kAgentDone : 0u) | (moved ? kAgentMoved : 0u) | (reuse ? kAgentReuse : 0u);
+      if (explore) {
         // the count is taken before the pose arrays move on to the next episode
-        uint32_t cnt = A.exp_count[gi];
-        if (moved) cnt = visit_cell(A, gi, pos);
-        A.geo[gi] = (float)(cnt - 1);
+        if (moved) cnt = visit_cell(row, A, gi, cnt, ip, iq, pos);
+        if (lead) A.geo[gi] = (float)(cnt - 1);
       }
       if (measure && !reuse) {
         want = true;
@@ -280,47 +309,42 @@ __global__ __launch_bounds__(64) void k_step_move(NavData nav, AgentArrays A, St
         // the terminal query above holds copies of the old episode's points: the pose arrays can
         // take the next episode now; distance bookkeeping waits for step_finish.  If a new scene
         // waits for this env's slot, the next episode is drawn there (simulator.cpp:1636-1642).
-        {
-          const uint32_t cur = scene0, tgt = P.swap_target[cur % P.num_slots];
-          if (tgt != kNoSwap && tgt != cur) {
+        uint32_t scene = scene0;
+        const uint32_t tgt = P.swap_target[scene0 % P.num_slots];
+        if (tgt != kNoSwap && tgt != scene0) {
+          scene = tgt;
+          if (lead) {
             A.scene[gi] = tgt;
-            atomicSub(&P.swap_remaining[cur % P.num_slots], 1u);
+            atomicSub(&P.swap_remaining[scene0 % P.num_slots], 1u);
           }
         }
-        begin_reset(nav, A, P, gi);
+        begin_reset(row, nav, A, P, gi, scene, resets);
         reset = true;
       }
     }
   }
-  // queue the queries: one atomic per wavefront and class present in it, all of them in flight
-  // together (per-lane atomics on the sixteen class counters serialise, and so do the round
-  // trips of one atomic per class after the other)
-  {
-    const int lane = (int)(threadIdx.x & 63);
-    unsigned long long mine = 0;   // lanes of this wavefront that queue into the same class as this one
-    for (uint32_t c = 0; c < (uint32_t)kGeoClasses; ++c) {
-      const unsigned long long m = __ballot(want && cls == c);
-      if (want && cls == c) mine = m;
-    }
-    const int leader = want ? __ffsll((long long)mine) - 1 : lane;
-    uint32_t base = 0;
-    if (want && lane == leader) base = atomicAdd(&Q.counts[kQGeo + cls], (uint32_t)__popcll(mine));
-    base = (uint32_t)__shfl((int)base, leader);
-    if (want) Q.queries[(size_t)cls * Q.stride + base + (uint32_t)__popcll(mine & ((1ull << lane) - 1ull))] = q;
+  // Queue the queries and the resets: places within the block from counters in LDS, then one atomic per
+  // block and class present in it, all of them in flight together.
+  want = want && lead;
+  reset = reset && lead;
+  uint32_t place = 0, rplace = 0;
+  if (want) place = atomicAdd(&queue.count[cls], 1u);
+  if (reset) rplace = atomicAdd(&queue.count[kGeoClasses], 1u);
+  if (lead && movePolys) {
+    atomicAdd(&queue.forward, 1u);
+    atomicAdd(&queue.polys, movePolys);
   }
-  const uint32_t rslot = wave_append(reset, &Q.counts[kQReset]);
-  if (reset) Q.reset_list[rslot] = gi;
-  // counters, one atomic per wavefront
-  const unsigned long long mv = __ballot(movePolys != 0);
-  uint32_t mp = movePolys;
-  for (int o = 32; o > 0; o >>= 1) mp += (uint32_t)__shfl_xor((int)mp, o);
-  if ((threadIdx.x & 63) == 0) {
-    if (mv) {
-      atomicAdd((unsigned long long*)&P.counters[kCntForward], (unsigned long long)__popcll(mv));
-      atomicAdd((unsigned long long*)&P.counters[kCntMovePolys], (unsigned long long)mp);
-    }
+  __syncthreads();
+  if (threadIdx.x <= (uint32_t)kGeoClasses && queue.count[threadIdx.x])
+    queue.base[threadIdx.x] = atomicAdd(&Q.counts[threadIdx.x < (uint32_t)kGeoClasses ? kQGeo + threadIdx.x : (uint32_t)kQReset], queue.count[threadIdx.x]);
+  if (threadIdx.x == 0 && queue.forward) {
+    atomicAdd((unsigned long long*)&P.counters[kCntForward], (unsigned long long)queue.forward);
+    atomicAdd((unsigned long long*)&P.counters[kCntMovePolys], (unsigned long long)queue.polys);
   }
-  if (i == 0) atomicAdd((unsigned long long*)&P.counters[kCntSteps], (unsigned long long)P.n);
+  __syncthreads();
+  if (want) Q.queries[(size_t)cls * Q.stride + queue.base[cls] + place] = q;
+  if (reset) Q.reset_list[queue.base[kGeoClasses] + rplace] = gi;
+  if (i == 0 && lead) atomicAdd((unsigned long long*)&P.counters[kCntSteps], (unsigned long long)P.n);
 }
 
 // served: the counters of the lists of queries that this step's searches have just served;
@@ -427,10 +451,12 @@ __global__ __launch_bounds__(256) void k_step_finish(AgentArrays A, StepParams P
 }
 
 __global__ __launch_bounds__(256) void k_reset_all(NavData nav, AgentArrays A, StepQueues Q, StepParams P) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t i = blockIdx.x * 32u + (threadIdx.x >> 3);   // a row of eight lanes per agent
   if (i >= P.n) return;
+  const Row row;
   const uint32_t gi = P.base + i;
-  begin_reset(nav, A, P, gi);
+  begin_reset(row, nav, A, P, gi, A.scene[gi], A.nresets[gi]);
+  if (row.el != 0) return;
   A.flags[gi] = kAgentResetOnly;
   Q.reset_list[i] = gi;
   if (i == 0) Q.counts[kQReset] = P.n;
@@ -476,8 +502,8 @@ __global__ __launch_bounds__(128) void k_reset_snap(NavData nav, AgentArrays A, 
           const float inv[4] = {-rot[0] / d, -rot[1] / d, -rot[2] / d, rot[3] / d};
           for (int k = 0; k < 4; ++k) A.exp_inv[(size_t)gi * 4 + k] = inv[k];
           store3(A.exp_init, gi, pos);
-          A.exp_count[gi] = 0;
-          visit_cell(A, gi, pos);
+          cell_of(pos, inv, pos, A.exp_cells + (size_t)gi * A.cell_cap * 3);   // the set's first
+          A.exp_count[gi] = 1;
         }
       }
     } else if (threadIdx.x == 0) {
@@ -709,14 +735,18 @@ __global__ __launch_bounds__(64) void k_snap_batch(NavData nav, uint32_t scene, 
     }
   }
 }
-__global__ void k_try_step_batch(NavData nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
-                                 uint32_t n, float* oxyz, uint32_t* oref) {
+__global__ __launch_bounds__(kMoveItems * 8) void k_try_step_batch(NavData nav, uint32_t scene, const float* sxyz, const uint32_t* sref,
+                                                                   const float* exyz, uint32_t n, float* oxyz, uint32_t* oref) {
   __shared__ MoveLds move_lds;
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  __shared__ __attribute__((aligned(16))) uint16_t entered[kMoveItems][kTinyNodes];
+  const Row row;
+  const uint32_t item = threadIdx.x >> 3, i = blockIdx.x * kMoveItems + item;
   if (i >= n) return;
   uint32_t c = 0;
   NavPt st{sxyz[(size_t)i * 3], sxyz[(size_t)i * 3 + 1], sxyz[(size_t)i * 3 + 2], sref[i]};
-  const NavPt r = try_step(nav, nav.scenes[scene], st, exyz[(size_t)i * 3], exyz[(size_t)i * 3 + 1], exyz[(size_t)i * 3 + 2], &c, move_lds);
+  const NavPt r = try_step_row(row, nav, nav.scenes[scene], st, exyz[(size_t)i * 3], exyz[(size_t)i * 3 + 1], exyz[(size_t)i * 3 + 2], &c,
+                               entered[item], move_lds, (int)item);
+  if (row.el != 0) return;
   oxyz[(size_t)i * 3] = r.x; oxyz[(size_t)i * 3 + 1] = r.y; oxyz[(size_t)i * 3 + 2] = r.z;
   oref[i] = r.ref;
 }
@@ -730,13 +760,15 @@ __global__ void k_make_queries(uint32_t scene, const float* sxyz, const uint32_t
   o.cost_slot = kNoCostSlot; o.pad = 0;
   q[i] = o;
 }
-__global__ void k_random_points(NavData nav, uint32_t scene, const float* u, uint32_t n, float* oxyz, uint32_t* oref) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(256) void k_random_points(NavData nav, uint32_t scene, const float* u, uint32_t n, float* oxyz, uint32_t* oref) {
+  const uint32_t i = blockIdx.x * 32u + (threadIdx.x >> 3);   // a row of eight lanes per point
   if (i >= n) return;
+  const Row row;
   const SceneDev& s = nav.scenes[scene];
   float p[3] = {0, 0, 0};
   uint32_t ip = 0;
-  const bool ok = sample_point(nav, s, u[(size_t)i * 3], u[(size_t)i * 3 + 1], u[(size_t)i * 3 + 2], p, &ip);
+  const bool ok = sample_point_row(row, nav, s, u[(size_t)i * 3], u[(size_t)i * 3 + 1], u[(size_t)i * 3 + 2], p, &ip);
+  if (row.el != 0) return;
   oxyz[(size_t)i * 3] = p[0]; oxyz[(size_t)i * 3 + 1] = p[1]; oxyz[(size_t)i * 3 + 2] = p[2];
   oref[i] = ok ? (s.ref_base | ip) : 0;
 }
@@ -783,7 +815,7 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
   // Q's lists of queries were emptied two steps ago and have since taken the first queries of
   // the episodes that began in the previous step; its reset list and ticket counter, and the
   // lists of Qnext, were emptied by the previous step's last launch
-  hipLaunchKernelGGL(k_step_move, grid_for(P.n, 64), dim3(64), 0, st, nav, A, Q, P, actions_dev);
+  hipLaunchKernelGGL(k_step_move, grid_for(P.n, kMoveItems), dim3(kMoveItems * 8), 0, st, nav, A, Q, P, actions_dev);
   mark();
   // the new episodes' snaps need nothing of this step's searches and the searches nothing of
   // them: they run side by side
@@ -811,7 +843,7 @@ void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q,
                   const GeoPool& G, uint32_t snap_blocks, hipStream_t st) {
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Qother);
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Qother, Qother);
-  hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 256), dim3(256), 0, st, nav, A, Q, P);
+  hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 32), dim3(256), 0, st, nav, A, Q, P);
   hipLaunchKernelGGL(k_reset_snap, dim3(snap_blocks), dim3(128), 0, st, nav, A, Q, Q, P);
   launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
                   A.last_cost, G, P.n, P.counters, st);
@@ -826,7 +858,7 @@ void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uin
 }
 void launch_try_step_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                            uint32_t n, float* oxyz, uint32_t* oref, hipStream_t st) {
-  hipLaunchKernelGGL(k_try_step_batch, grid_for(n, 64), dim3(64), 0, st, nav, scene, sxyz, sref, exyz, n, oxyz, oref);
+  hipLaunchKernelGGL(k_try_step_batch, grid_for(n, kMoveItems), dim3(kMoveItems * 8), 0, st, nav, scene, sxyz, sref, exyz, n, oxyz, oref);
 }
 void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                            const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */, float* out,
@@ -844,7 +876,7 @@ void launch_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint32_t s
 }
 void launch_random_points(const NavData& nav, uint32_t scene, const float* u, uint32_t n, float* oxyz, uint32_t* oref,
                           hipStream_t st) {
-  hipLaunchKernelGGL(k_random_points, grid_for(n, 64), dim3(64), 0, st, nav, scene, u, n, oxyz, oref);
+  hipLaunchKernelGGL(k_random_points, grid_for(n, 32), dim3(256), 0, st, nav, scene, u, n, oxyz, oref);
 }
 
 #ifdef BPSX_QUERY_TRACE
