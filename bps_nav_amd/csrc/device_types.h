@@ -194,6 +194,11 @@ constexpr uint32_t kGeoClassUnknown = geo_class(1000);
 // neither says how long the first search will be, and it is often among the longest.
 constexpr uint32_t kCostUnknown = 0xffffffffu;
 
+// The counters are kept kCounterShards times, a block adding to the copy of its index, and summed when
+// they are read: additions to one word are served one after the other, 6.5 ns each, and a launch of
+// thousands of wavefronts waits for them (4096 snaps and an addition for each: 68 us, now 30; 16384 agents
+// over mazes: k_geodesic 1083 -> 1032 us, k_step_move 23 -> 18; 65536 over mixed scenes 3787 -> 3726, 66 -> 53).
+constexpr uint32_t kCounterShards = 64, kCounterStride = 32;
 enum Counter {
   kCntSteps = 0, kCntForward, kCntGeoQueries, kCntAstarPops, kCntCorridor, kCntResets, kCntMovePolys, kCntSnapCands,
   kCntLinkSpills = 16, kCntHeapSpills = 17, kCntLongPath = 18, kCntExactRuns = 19, kCntTieReplays = 20, kCntPairTies = 21   // 8..15: phase cycles of the diagnostic build

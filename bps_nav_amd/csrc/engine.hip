@@ -40,7 +40,6 @@ struct Group {
   // of the episodes that begin in it into the other set, which the next step serves.
   StepQueues Q[2] = {};
   int turn = 0;
-  hipEvent_t moved = nullptr, snapped = nullptr;   // fork and join of the side stream within a step
   int64_t* d_actions = nullptr;
   int64_t* h_actions = nullptr;  // pinned staging for host-side action arrays
   hipEvent_t ev[kStepEvents] = {};
@@ -202,7 +201,6 @@ struct bpsx_sim {
   std::string loader_error;              // first failure of the loader thread (guarded by loader_mu)
   bool loader_error_reported = false;    // step_end has returned it once
   hipStream_t upload_stream = nullptr;   // uploads of scenes that come in while the simulation runs
-  hipStream_t side = nullptr;            // a step's snaps of new episodes, next to its searches (default priority)
   uint32_t* h_swap_remaining = nullptr;  // d_swap_remaining as of the newest step whose completion has been seen
   StepRecord ring[kStepRing];
   int ring_head = 0, ring_count = 0;     // oldest outstanding record, number outstanding
@@ -554,7 +552,6 @@ int bpsx_finalize(bpsx_sim* sim) {
     HIP_TRY(hipMemcpy(sim->d_swap_target, none.data(), (size_t)S * 4, hipMemcpyHostToDevice));
   }
   HIP_TRY(hipStreamCreateWithFlags(&sim->upload_stream, hipStreamNonBlocking));
-  HIP_TRY(hipStreamCreateWithFlags(&sim->side, hipStreamNonBlocking));
   HIP_TRY(hipHostMalloc((void**)&sim->h_swap_remaining, (size_t)S * 4, hipHostMallocDefault));
   memset(sim->h_swap_remaining, 0, (size_t)S * 4);
   for (StepRecord& rec : sim->ring) {
@@ -601,7 +598,7 @@ int bpsx_finalize(bpsx_sim* sim) {
     for (size_t i = 0; i < N; ++i) rot[i * 4 + 3] = 1.f;
     HIP_TRY(hipMemcpy(A.rot, rot.data(), N * 16, hipMemcpyHostToDevice));
   }
-  if ((rc = sim->alloc(&sim->d_error, 1)) || (rc = sim->alloc(&sim->d_counters, BPSX_NUM_COUNTERS))) return rc;
+  if ((rc = sim->alloc(&sim->d_error, 1)) || (rc = sim->alloc(&sim->d_counters, (size_t)kCounterShards * kCounterStride))) return rc;
   if ((rc = sim->alloc(&sim->d_batch_counts, kGeoClasses + 2))) return rc;
 
   // ---- A* wavefronts: as many as the LDS of the device holds at once, not one per agent
@@ -615,7 +612,7 @@ int bpsx_finalize(bpsx_sim* sim) {
   sim->geo.blocks = std::max(1u, blocks);
   sim->max_few_blocks = (uint32_t)prop.multiProcessorCount * geodesic_few_blocks_per_cu();
   sim->geo.few_blocks = std::min(sim->max_few_blocks, sim->geo.blocks * 2u);
-  sim->snap_blocks = std::max(1u, std::min((uint32_t)prop.multiProcessorCount * 16u, sim->envs_per_group));
+  sim->snap_blocks = (uint32_t)prop.multiProcessorCount * 8u;   // of four wavefronts: what the device holds at once
   if ((rc = sim->alloc(&sim->geo.slots, (size_t)sim->geo.blocks * 2))) return rc;   // one per wavefront
 
   // ---- per-group queues
@@ -629,8 +626,6 @@ int bpsx_finalize(bpsx_sim* sim) {
       Q.stride = (uint32_t)(2 * n);
     }
     if ((rc = sim->alloc(&g.d_actions, n))) return rc;
-    HIP_TRY(hipEventCreateWithFlags(&g.moved, hipEventDisableTiming));
-    HIP_TRY(hipEventCreateWithFlags(&g.snapped, hipEventDisableTiming));
     HIP_TRY(hipHostMalloc((void**)&g.h_actions, n * sizeof(int64_t), hipHostMallocDefault));
     for (auto& e : g.ev) HIP_TRY(hipEventCreate(&e));
   }
@@ -661,7 +656,6 @@ void bpsx_destroy(bpsx_sim* sim) {
     sim->loader.join();
   }
   if (sim->upload_stream) (void)hipStreamDestroy(sim->upload_stream);
-  if (sim->side) (void)hipStreamDestroy(sim->side);
   if (sim->h_swap_remaining) (void)hipHostFree(sim->h_swap_remaining);
   for (StepRecord& rec : sim->ring) {
     if (rec.done) (void)hipEventDestroy(rec.done);
@@ -669,8 +663,6 @@ void bpsx_destroy(bpsx_sim* sim) {
   }
   for (auto& g : sim->groups) {
     if (g.h_actions) (void)hipHostFree(g.h_actions);
-    if (g.moved) (void)hipEventDestroy(g.moved);
-    if (g.snapped) (void)hipEventDestroy(g.snapped);
     for (auto& e : g.ev)
       if (e) (void)hipEventDestroy(e);
   }
@@ -732,7 +724,7 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   StepParams P = sim->params(group);
   P.defer_first_distance = 1;
   launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->geo, sim->snap_blocks, st,
-              sim->side, g.moved, g.snapped, g.profiled ? g.ev : nullptr);
+              g.profiled ? g.ev : nullptr);
   g.turn ^= 1;
   HIP_TRY(hipGetLastError());
   g.record = (sim->ring_head + sim->ring_count) % kStepRing;
@@ -840,7 +832,13 @@ int bpsx_check_errors(bpsx_sim* sim) {
 int bpsx_get_counters(bpsx_sim* sim, uint64_t* out) {
   if (!sim || !sim->finalized || !out) return fail(BPSX_E_STATE, "get_counters: simulator not finalized");
   { const int qrc = quiesce(sim); if (qrc) return qrc; }
-  HIP_TRY(hipMemcpy(out, sim->d_counters, BPSX_NUM_COUNTERS * 8, hipMemcpyDeviceToHost));
+  static_assert(BPSX_NUM_COUNTERS <= kCounterStride, "a copy holds every counter");
+  uint64_t shards[kCounterShards * kCounterStride];
+  HIP_TRY(hipMemcpy(shards, sim->d_counters, sizeof(shards), hipMemcpyDeviceToHost));
+  for (uint32_t k = 0; k < BPSX_NUM_COUNTERS; ++k) {
+    out[k] = 0;
+    for (uint32_t c = 0; c < kCounterShards; ++c) out[k] += shards[(size_t)c * kCounterStride + k];
+  }
   return BPSX_OK;
 }
 

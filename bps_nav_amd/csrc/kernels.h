@@ -49,12 +49,11 @@ constexpr uint32_t kNoSwap = 0xffffffffu;
 constexpr int kStepEvents = 5;  // timestamps recorded by launch_step when asked to
 
 // One step of a group.  Q holds the step's queries, among them the first queries of the episodes
-// that began in the previous step; the episodes that begin in this one are snapped on `side`
-// while the searches run on `st`, and their first queries go to Qnext, the next step's queues.
-// `moved` and `snapped` are events of the caller's for the fork and the join of the two streams.
+// that began in the previous step; the episodes that begin in this one are snapped in its last
+// launch, and their first queries go to Qnext, the next step's queues.  snap_blocks: most blocks for
+// the snaps.
 void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
-                 const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st,
-                 hipStream_t side, hipEvent_t moved, hipEvent_t snapped, hipEvent_t* ev);
+                 const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st, hipEvent_t* ev);
 // Reset of a whole group, all on st; Qother (the group's other set of queues) is emptied.
 void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
                   const GeoPool& G, uint32_t snap_blocks, hipStream_t st);

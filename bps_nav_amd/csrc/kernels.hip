@@ -1,27 +1,27 @@
 // HIP kernels of the batch environment step (gfx950) and their launch wrappers.
 //
-// One step of a group of n agents is four launches:
+// One step of a group of n agents is three launches:
 //   step_move      row of eight lanes per agent: action, turn / forward move with wall sliding, polar
 //                  observation, and a geodesic query (goal -> agent) when the agent moved or
 //                  the episode ended; an agent whose episode ended also picks its next episode
 //                  here and is queued for reset (simulator.cpp:620-632, 651-710, 601-610)
-//   reset_snap     two wavefronts per queued agent: snap start and goal of the new episode,
-//                  polar, and the new episode's first query (agent -> goal)
-//                                                        (simulator.cpp:611-614, 744-751)
 //   geodesic       wavefront per query, both kinds in one launch: A* + funnel; blocks of two
 //                  wavefronts so that the longest searches can take a block's whole LDS
 //                                                        (PathFinder.cpp:485-541)
 //   step_finish    lane per agent: info, reward, mask from the terminal transition, then the
-//                  new episode's distance bookkeeping    (simulator.cpp:634-641, 758-822, 749-755)
-// In a step, reset_snap runs on a second stream next to geodesic: the first query of an episode
-// that begins in step t is answered by step t + 1's geodesic launch, and its result enters the
-// bookkeeping at the start of step t + 1's step_finish.  No output of step t depends on it (the
-// reference computes it inside the reset and uses it from the next step on).  A reset of a
-// whole group (bpsx_reset) runs the four launches in order, first queries included.
-// The Flee and Exploration tasks (simulator.cpp:830-997) run through the same four launches:
+//                  new episode's distance bookkeeping    (simulator.cpp:634-641, 758-822, 749-755);
+//                  in blocks of their own a wavefront per snap: start and goal of the new episode,
+//                  polar, and the new episode's first query (agent -> goal)
+//                                                        (simulator.cpp:611-614, 744-751)
+// The first query of an episode that begins in step t is answered by step t + 1's geodesic launch, and
+// its result enters the bookkeeping at the start of step t + 1's step_finish.  No output of step t
+// depends on it (the reference computes it inside the reset and uses it from the next step on).  A reset
+// of a whole group (bpsx_reset) runs the snaps as a launch of their own before geodesic, first queries
+// included, and so does a step whose launches are timed.
+// The Flee and Exploration tasks (simulator.cpp:830-997) run through the same launches:
 // Flee keeps the episode's start point where PointNav keeps the snapped goal, so its
-// "distance from start" is the same start-point -> agent query; Exploration makes no queries
-// and keeps its visited cells per agent in HBM.
+// "distance from start" is the same start-point -> agent query; Exploration makes no queries,
+// needs no geodesic launch and keeps its visited cells per agent in HBM.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -103,6 +103,9 @@ BPSX_DEV void write_polar(const AgentArrays& A, uint32_t gi, const float* pos, c
   A.polars[(size_t)gi * 2 + 0] = sqrtf(x * x + y * y);
   A.polars[(size_t)gi * 2 + 1] = -atan2f(y, x);
 }
+
+// the copy of the counters that this block adds to
+BPSX_DEV uint64_t* counter_shard(uint64_t* counters) { return counters + (blockIdx.x % kCounterShards) * kCounterStride; }
 
 BPSX_DEV void load3(const float* p, size_t i, float* o) { o[0] = p[i * 3]; o[1] = p[i * 3 + 1]; o[2] = p[i * 3 + 2]; }
 BPSX_DEV void store3(float* p, size_t i, const float* v) { p[i * 3] = v[0]; p[i * 3 + 1] = v[1]; p[i * 3 + 2] = v[2]; }
@@ -338,26 +341,110 @@ __global__ __launch_bounds__(kMoveItems * 8) void k_step_move(NavData nav, Agent
   if (threadIdx.x <= (uint32_t)kGeoClasses && queue.count[threadIdx.x])
     queue.base[threadIdx.x] = atomicAdd(&Q.counts[threadIdx.x < (uint32_t)kGeoClasses ? kQGeo + threadIdx.x : (uint32_t)kQReset], queue.count[threadIdx.x]);
   if (threadIdx.x == 0 && queue.forward) {
-    atomicAdd((unsigned long long*)&P.counters[kCntForward], (unsigned long long)queue.forward);
-    atomicAdd((unsigned long long*)&P.counters[kCntMovePolys], (unsigned long long)queue.polys);
+    atomicAdd((unsigned long long*)&counter_shard(P.counters)[kCntForward], (unsigned long long)queue.forward);
+    atomicAdd((unsigned long long*)&counter_shard(P.counters)[kCntMovePolys], (unsigned long long)queue.polys);
   }
   __syncthreads();
   if (want) Q.queries[(size_t)cls * Q.stride + queue.base[cls] + place] = q;
   if (reset) Q.reset_list[queue.base[kGeoClasses] + rplace] = gi;
-  if (i == 0 && lead) atomicAdd((unsigned long long*)&P.counters[kCntSteps], (unsigned long long)P.n);
+  if (i == 0 && lead) atomicAdd((unsigned long long*)&counter_shard(P.counters)[kCntSteps], (unsigned long long)P.n);
 }
 
-// served: the counters of the lists of queries that this step's searches have just served;
-// before: those of the other set.  Both are left as the next step expects them, so that a step
-// needs no launch of its own for it: the served lists and their ticket counter empty, and the
-// reset list of the step before empty (its snaps, which read it, ended before this step began).
-__global__ __launch_bounds__(256) void k_step_finish(AgentArrays A, StepParams P, uint32_t* served, uint32_t* before) {
-  if (blockIdx.x == 0) {
-    static_assert(kQGeoHead == kQGeo + kGeoClasses && kGeoClasses + 1 < 256, "one thread per counter");
-    if (threadIdx.x <= (uint32_t)kGeoClasses) served[kQGeo + threadIdx.x] = 0;
-    else if (threadIdx.x == (uint32_t)kGeoClasses + 1u) before[kQReset] = 0;
+// The snaps of the episodes that begin, a wavefront for each start and, in PointNav, each goal (the
+// other tasks snap no goal, simulator.cpp:838-843, 906-916): wavefront w of nw takes every nw-th.  The
+// wavefront of the start writes the state that hangs on it and the polar observation; each writes its
+// half of the episode's first query (agent -> goal) to Qout, in the order of the reset list: the class
+// of unknown length is empty when this begins (the queues of the next step, or cleared ones) and
+// nothing else fills it meanwhile.
+BPSX_DEV void snap_new_episodes(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qout, const StepParams& P,
+                                uint32_t w, uint32_t nw, SnapLds& lds) {
+  const uint32_t n = Q.counts[kQReset];
+  const bool pointnav = P.task == BPSX_TASK_POINTNAV;
+  const bool first = (threadIdx.x & 63u) == 0;
+  uint32_t cands = 0;
+  for (uint32_t it = w; it < (pointnav ? 2u * n : n); it += nw) {
+    const uint32_t i = pointnav ? it >> 1 : it;
+    const bool ofGoal = pointnav && (it & 1u);
+    const uint32_t gi = Q.reset_list[i], scene = A.scene[gi];
+    float p[3];
+    load3(ofGoal ? A.goal : A.pos, gi, p);
+    const NavPt r = snap_point_wave(nav, nav.scenes[scene], p[0], p[1], p[2], lds, &cands);
+    if (!first) continue;
+    const float xyz[3] = {r.x, r.y, r.z};
+    GeoQuery* q = &Qout.queries[(size_t)kGeoClassUnknown * Qout.stride + i];   // a new episode: no history
+    if (ofGoal) {
+      store3(A.goal_xyz, gi, xyz);
+      A.goal_ref[gi] = r.ref;
+      q->b[0] = r.x; q->b[1] = r.y; q->b[2] = r.z; q->b_ref = r.ref;
+      continue;
+    }
+    store3(A.nav_xyz, gi, xyz);
+    A.nav_ref[gi] = r.ref;
+    float goal[3], rot[4];
+    load3(A.goal, gi, goal);
+    for (int k = 0; k < 4; ++k) rot[k] = A.rot[(size_t)gi * 4 + k];
+    write_polar(A, gi, p, rot, goal);
+    if (pointnav) {
+      q->a[0] = r.x; q->a[1] = r.y; q->a[2] = r.z; q->a_ref = r.ref;
+      q->scene = scene;
+      q->out = P.total + gi;
+      q->cost_slot = kNoCostSlot;   // searched agent -> goal: says little about the searches to come
+      q->pad = 0;
+      continue;
+    }
+    const float zero[3] = {0, 0, 0};
+    const bool flee = P.task == BPSX_TASK_FLEE;
+    store3(A.goal_xyz, gi, flee ? xyz : zero);   // Flee: navmeshStart_
+    A.goal_ref[gi] = flee ? r.ref : 0u;
+    if (!flee) {
+      // glm::inverse(q) = conjugate(q) / dot(q, q)
+      const float d = (rot[3] * rot[3] + rot[0] * rot[0]) + (rot[1] * rot[1] + rot[2] * rot[2]);
+      const float inv[4] = {-rot[0] / d, -rot[1] / d, -rot[2] / d, rot[3] / d};
+      for (int k = 0; k < 4; ++k) A.exp_inv[(size_t)gi * 4 + k] = inv[k];
+      store3(A.exp_init, gi, p);
+      cell_of(p, inv, p, A.exp_cells + (size_t)gi * A.cell_cap * 3);   // the set's first
+      A.exp_count[gi] = 1;
+    }
   }
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (w == 0 && first && n) {
+    atomicAdd((unsigned long long*)&counter_shard(P.counters)[kCntResets], (unsigned long long)n);
+    if (pointnav) Qout.counts[kQGeo + kGeoClassUnknown] = n;
+  }
+  if (first && cands) atomicAdd((unsigned long long*)&counter_shard(P.counters)[kCntSnapCands], (unsigned long long)cands);
+}
+constexpr uint32_t kSnapWaves = 4;   // per block
+__global__ __launch_bounds__(kSnapWaves * 64) void k_reset_snap(NavData nav, AgentArrays A, StepQueues Q, StepQueues Qout, StepParams P) {
+  __shared__ SnapLds lds[kSnapWaves];
+  const uint32_t half = threadIdx.x >> 6;
+  snap_new_episodes(nav, A, Q, Qout, P, blockIdx.x * kSnapWaves + half, gridDim.x * kSnapWaves, lds[half]);
+}
+
+// The bookkeeping of a step's agents, and in its first snap_blocks blocks the snaps of the episodes that
+// began in it, which touch nothing that the bookkeeping touches: no output of this step depends on an
+// episode's first distance (the reference computes it inside the reset and uses it from the next step
+// on), so its query goes to the next step's queues.
+// (On a second stream next to the searches they cost the step two waits between streams, 6 to 17 us before
+// the searches begin and 6 at its end, for the 9 us by which they outlast the bookkeeping of a small
+// group: a step of 64 agents 232 us, now 219, of 1017 exploring ones 62 and 41.  At 16384 agents, whose 655
+// new episodes take 22 us here, it makes no difference: 1193 us both ways without the copies of the counters.)
+// Q: the lists of queries that this step's searches have just served; Qnext: the other set.  The
+// counters of both are left as the next step expects them, so that a step needs no launch of its own
+// for it: the served lists and their ticket counter empty, and the reset list of the step before.
+__global__ __launch_bounds__(256) void k_step_finish(NavData nav, AgentArrays A, StepParams P, StepQueues Q, StepQueues Qnext, uint32_t snap_blocks) {
+  __shared__ SnapLds lds[kSnapWaves];
+  static_assert(kSnapWaves * 64 == 256, "a wavefront each");
+  if (blockIdx.x < snap_blocks) {
+    const uint32_t wave = threadIdx.x >> 6;
+    snap_new_episodes(nav, A, Q, Qnext, P, blockIdx.x * kSnapWaves + wave, snap_blocks * kSnapWaves, lds[wave]);
+    return;
+  }
+  const uint32_t block = blockIdx.x - snap_blocks;
+  if (block == 0) {
+    static_assert(kQGeoHead == kQGeo + kGeoClasses && kGeoClasses + 1 < 256, "one thread per counter");
+    if (threadIdx.x <= (uint32_t)kGeoClasses) Q.counts[kQGeo + threadIdx.x] = 0;
+    else if (threadIdx.x == (uint32_t)kGeoClasses + 1u) Qnext.counts[kQReset] = 0;
+  }
+  const uint32_t i = block * 256u + threadIdx.x;
   if (i >= P.n) return;
   const uint32_t gi = P.base + i;
   const uint32_t f = A.flags[gi];
@@ -462,74 +549,6 @@ __global__ __launch_bounds__(256) void k_reset_all(NavData nav, AgentArrays A, S
   if (i == 0) Q.counts[kQReset] = P.n;
 }
 
-// One block of two wavefronts per agent being reset: each takes one snap of the new episode (the
-// two are independent chains of dependent loads), then the first writes the state, the polar
-// observation and the episode's first geodesic query.
-__global__ __launch_bounds__(128) void k_reset_snap(NavData nav, AgentArrays A, StepQueues Q, StepQueues Qout, StepParams P) {
-  __shared__ SnapLds lds[2];
-  __shared__ NavPt goalPt;
-  const uint32_t n = Q.counts[kQReset];
-  const int lane = (int)(threadIdx.x & 63), half = (int)(threadIdx.x >> 6);
-  uint32_t cands = 0;
-  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-    const uint32_t gi = Q.reset_list[i];
-    const SceneDev& s = nav.scenes[A.scene[gi]];
-    float pos[3], goal[3], rot[4];
-    load3(A.pos, gi, pos);
-    load3(A.goal, gi, goal);
-    for (int k = 0; k < 4; ++k) rot[k] = A.rot[(size_t)gi * 4 + k];
-    const bool pointnav = P.task == BPSX_TASK_POINTNAV;   // the other tasks snap no goal (simulator.cpp:838-843, 906-916)
-    NavPt a{};
-    if (half == 0) a = snap_point_wave(nav, s, pos[0], pos[1], pos[2], lds[0], &cands);
-    else if (pointnav) {
-      const NavPt b = snap_point_wave(nav, s, goal[0], goal[1], goal[2], lds[1], &cands);
-      if (lane == 0) goalPt = b;
-    }
-    __syncthreads();
-    if (!pointnav) {
-      // no first query either
-      if (threadIdx.x == 0) {
-        const float axyz[3] = {a.x, a.y, a.z}, zero[3] = {0, 0, 0};
-        store3(A.nav_xyz, gi, axyz);
-        A.nav_ref[gi] = a.ref;
-        const bool flee = P.task == BPSX_TASK_FLEE;
-        store3(A.goal_xyz, gi, flee ? axyz : zero);   // Flee: navmeshStart_
-        A.goal_ref[gi] = flee ? a.ref : 0u;
-        write_polar(A, gi, pos, rot, goal);
-        if (!flee) {
-          // glm::inverse(q) = conjugate(q) / dot(q, q)
-          const float d = (rot[3] * rot[3] + rot[0] * rot[0]) + (rot[1] * rot[1] + rot[2] * rot[2]);
-          const float inv[4] = {-rot[0] / d, -rot[1] / d, -rot[2] / d, rot[3] / d};
-          for (int k = 0; k < 4; ++k) A.exp_inv[(size_t)gi * 4 + k] = inv[k];
-          store3(A.exp_init, gi, pos);
-          cell_of(pos, inv, pos, A.exp_cells + (size_t)gi * A.cell_cap * 3);   // the set's first
-          A.exp_count[gi] = 1;
-        }
-      }
-    } else if (threadIdx.x == 0) {
-      const NavPt b = goalPt;
-      const float axyz[3] = {a.x, a.y, a.z}, bxyz[3] = {b.x, b.y, b.z};
-      store3(A.nav_xyz, gi, axyz);
-      A.nav_ref[gi] = a.ref;
-      store3(A.goal_xyz, gi, bxyz);
-      A.goal_ref[gi] = b.ref;
-      write_polar(A, gi, pos, rot, goal);
-      GeoQuery q;
-      q.a[0] = a.x; q.a[1] = a.y; q.a[2] = a.z; q.a_ref = a.ref;
-      q.b[0] = b.x; q.b[1] = b.y; q.b[2] = b.z; q.b_ref = b.ref;
-      q.scene = A.scene[gi];
-      q.out = P.total + gi;
-      q.cost_slot = kNoCostSlot;   // searched agent -> goal: says little about the searches to come
-      q.pad = 0;
-      // a new episode: no history
-      Qout.queries[(size_t)kGeoClassUnknown * Qout.stride + atomicAdd(&Qout.counts[kQGeo + kGeoClassUnknown], 1u)] = q;
-    }
-    __syncthreads();   // goalPt is rewritten in the next round
-  }
-  if (threadIdx.x == 0 && blockIdx.x == 0 && n) atomicAdd((unsigned long long*)&P.counters[kCntResets], (unsigned long long)n);
-  if (lane == 0 && cands) atomicAdd((unsigned long long*)&P.counters[kCntSnapCands], (unsigned long long)cands);
-}
-
 #ifdef BPSX_QUERY_TRACE
 #include "diag_trace.h"   // diagnostic build only: per-query trace buffer
 #endif
@@ -628,6 +647,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
     return curCls;
   };
   GeoTotals T;
+  counters = counter_shard(counters);
   // The first query of every wavefront needs no ticket counter: the grid is what the device
   // holds at once, so block b takes long query b if there is one, and the wavefronts of the
   // other blocks take the queries after the long ones in the order of their index.  (Some
@@ -705,6 +725,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
   int cls = 0;
   uint32_t lo = 0, hi = (uint32_t)uniform_i((int)counts[0]);
   GeoTotals T;
+  counters = counter_shard(counters);
   // the first query by the block's index, further ones from the counter, the longest classes first
   for (uint32_t qi = blockIdx.x; qi < nq;) {
     while (qi >= hi) {
@@ -807,8 +828,7 @@ void launch_geodesic(const NavData& nav, const GeoQuery* queries, uint32_t strid
 }
 
 void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
-                 const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st,
-                 hipStream_t side, hipEvent_t moved, hipEvent_t snapped, hipEvent_t* ev) {
+                 const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st, hipEvent_t* ev) {
   int e = 0;
   auto mark = [&]() { if (ev) (void)hipEventRecord(ev[e++], st); };
   mark();
@@ -817,25 +837,17 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
   // lists of Qnext, were emptied by the previous step's last launch
   hipLaunchKernelGGL(k_step_move, grid_for(P.n, kMoveItems), dim3(kMoveItems * 8), 0, st, nav, A, Q, P, actions_dev);
   mark();
-  // the new episodes' snaps need nothing of this step's searches and the searches nothing of
-  // them: they run side by side
-  // (not when the launches are being timed one by one: then everything stays on st)
-  const bool fork = side && !ev;
-  if (fork) {
-    (void)hipEventRecord(moved, st);
-    (void)hipStreamWaitEvent(side, moved, 0);
-  }
-  // (a grid for one agent in sixteen ending its episode; more take further rounds.  Blocks
-  // without work would only wait for LDS that the searches hold and keep the join waiting.)
-  const uint32_t step_snap_blocks = std::min(snap_blocks, std::max(64u, P.n / 16u));
-  hipLaunchKernelGGL(k_reset_snap, dim3(step_snap_blocks), dim3(128), 0, fork ? side : st, nav, A, Q, Qnext, P);
-  if (fork) (void)hipEventRecord(snapped, side);
+  // a grid for one agent in sixteen ending its episode; more take further rounds
+  const uint32_t step_snap_blocks = std::min(snap_blocks, std::max(16u, P.n / 32u));
+  // (the snaps are a launch of their own when the launches are being timed one by one)
+  if (ev) hipLaunchKernelGGL(k_reset_snap, dim3(step_snap_blocks), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Qnext, P);
   mark();
-  launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                  A.last_cost, G, P.n - P.n / 4u, P.counters, st);   // three agents in five ask for a distance in a step
+  if (P.task != BPSX_TASK_EXPLORATION)   // which asks for no distance
+    launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
+                    A.last_cost, G, P.n - P.n / 4u, P.counters, st);   // three agents in five ask for a distance in a step
   mark();
-  hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, A, P, Q.counts, Qnext.counts);
-  if (fork) (void)hipStreamWaitEvent(st, snapped, 0);
+  const uint32_t with_snaps = ev ? 0u : step_snap_blocks;
+  hipLaunchKernelGGL(k_step_finish, dim3(with_snaps + grid_for(P.n, 256).x), dim3(256), 0, st, nav, A, P, Q, Qnext, with_snaps);
   mark();
 }
 
@@ -844,14 +856,14 @@ void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q,
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Qother);
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Qother, Qother);
   hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 32), dim3(256), 0, st, nav, A, Q, P);
-  hipLaunchKernelGGL(k_reset_snap, dim3(snap_blocks), dim3(128), 0, st, nav, A, Q, Q, P);
-  launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                  A.last_cost, G, P.n, P.counters, st);
-  hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, A, P, Q.counts, Qother.counts);
+  hipLaunchKernelGGL(k_reset_snap, dim3(std::min(snap_blocks, (P.n + 1u) / 2u)), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Q, P);
+  if (P.task != BPSX_TASK_EXPLORATION)
+    launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
+                    A.last_cost, G, P.n, P.counters, st);
+  hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, nav, A, P, Q, Qother, 0u);
   // the next step finds its lists of queries empty, not with this launch's queries still in them
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Q);
 }
-
 void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz, uint32_t* oref,
                        uint32_t snap_blocks, hipStream_t st) {
   hipLaunchKernelGGL(k_snap_batch, dim3(snap_blocks < n ? snap_blocks : n), dim3(64), 0, st, nav, scene, pts, n, oxyz, oref);
