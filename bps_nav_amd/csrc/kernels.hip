@@ -413,7 +413,9 @@ BPSX_DEV void snap_new_episodes(const NavData& nav, const AgentArrays& A, const 
   if (first && cands) atomicAdd((unsigned long long*)&counter_shard(P.counters)[kCntSnapCands], (unsigned long long)cands);
 }
 constexpr uint32_t kSnapWaves = 4;   // per block
-__global__ __launch_bounds__(kSnapWaves * 64) void k_reset_snap(NavData nav, AgentArrays A, StepQueues Q, StepQueues Qout, StepParams P) {
+// 128 of the 133 registers that the compiler would take, without scratch: a whole-group reset of 2048 agents
+// has 4096 snaps, which then all run at once.
+__global__ __launch_bounds__(kSnapWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_reset_snap(NavData nav, AgentArrays A, StepQueues Q, StepQueues Qout, StepParams P) {
   __shared__ SnapLds lds[kSnapWaves];
   const uint32_t half = threadIdx.x >> 6;
   snap_new_episodes(nav, A, Q, Qout, P, blockIdx.x * kSnapWaves + half, gridDim.x * kSnapWaves, lds[half]);

@@ -394,8 +394,11 @@ BPSX_DEV void closest_on_boundary(const NavData& nav, const PolyRegs& P, float p
 //
 // The walkable leaves lie in one array in that order, with the bounds of every 64 of them in another
 // (a run of the tree's in-order array is a compact part of the mesh): all groups' bounds are read at
-// once, then the leaves of the groups that overlap, 64 in one load, then one polygon per lane.  That
-// is four dependent loads where a descent of the binary tree has seventeen.
+// once, then the leaves of four groups that overlap, 64 in one load, then one polygon per lane.  That
+// is four dependent loads where a descent of the binary tree has seventeen.  (One load of groups and
+// one of leaves after the other, a batch evaluated as soon as it was full, and registers for three
+// instead of four wavefronts per SIMD: 277 us instead of 238 for 50000 points over a cluttered plan,
+// 31 instead of 20 for the 4096 of a reset over mazes.)
 //
 // Where the scene allows it (SceneDev::snap_prune) the box begins with a half extent of kSnapFirst and
 // grows: a polygon outside a box of half extent r is at least r - kSnapSlack away, so once the best
@@ -405,7 +408,7 @@ BPSX_DEV void closest_on_boundary(const NavData& nav, const PolyRegs& P, float p
 //
 // Bound by the latency of those loads and by the divide-heavy edge distances of the candidates: most
 // points are on the mesh, and of the 200 polygons of a cluttered plan in the full box five remain.
-// (50000 points over a cluttered plan of 20k polygons: 1730 -> 277 us; 4096 points there, a wavefront
+// (50000 points over a cluttered plan of 20k polygons: 1730 -> 277 us, now 238; 4096 points there, a wavefront
 // each, 64 -> 14 us; snaps of 165 new episodes there next to the searches 135 -> 24 us.  The descent
 // tested one level per load and evaluated the whole box, a field of a record at a time.)
 constexpr float kSnapFirst = 0.25f;
@@ -413,9 +416,12 @@ constexpr float kSnapFirst = 0.25f;
 // what height samples may lie outside of their polygon's bounds (kSnapOverhang, checked at load)
 constexpr float kSnapSlack = 1e-3f;
 static_assert(kSnapGroup == 64, "a lane per leaf of a group");
+constexpr int kSnapGroupLoads = 8, kSnapLeafLoads = 4;   // groups' bounds, 64 each, and groups' leaves that are asked for at once
 struct SnapLds {
-  uint16_t cand_rank[64];   // place among the leaves of the candidates of the current batch
-  uint16_t cand_poly[64];
+  uint16_t group[64 * kSnapGroupLoads];   // the groups that overlap the box
+  // candidates waiting: less than a batch is left when the leaves of further groups join
+  uint16_t cand_rank[64 * (kSnapLeafLoads + 1)];   // place among the leaves
+  uint16_t cand_poly[64 * (kSnapLeafLoads + 1)];
 };
 BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, float py, float pz, SnapLds& L,
                                uint32_t* ncand) {
@@ -434,11 +440,12 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
   uint32_t bestKey = 0xffffffffu;  // place of the lane's best candidate
   uint32_t bestIp = kInvalidPoly;
   float bp[3] = {0, 0, 0};
-  int ncands = 0;  // candidates waiting in the batch (uniform)
+  int ncands = 0;  // candidates waiting (uniform)
   auto flush = [&]() {
-    const bool have = lane < ncands;
-    *ncand += (uint32_t)ncands;
-    ncands = 0;
+    const int fit = ncands < 64 ? ncands : 64;
+    ncands -= fit;
+    const bool have = lane < fit;
+    *ncand += (uint32_t)fit;
     uint32_t ip = 0, key = 0;
     PolyRegs P;
     const PolyRec* rec = nullptr;
@@ -450,8 +457,8 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
       }
     };
     if (have) {
-      ip = L.cand_poly[lane];
-      key = L.cand_rank[lane];
+      ip = L.cand_poly[ncands + lane];
+      key = L.cand_rank[ncands + lane];
       rec = &nav.polys[s.poly_base + ip];
       P.load(rec);
       inside = poly_height(nav, P, *rec, px, py, pz, h);
@@ -486,35 +493,55 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
   SnapBox box = snap_box(s, px, py, pz, half), before = box;
   bool grown = false;   // what overlaps `before` has been looked at
   for (;;) {
-    for (uint32_t g0 = 0; g0 < ngroups; g0 += 64) {
-      const uint32_t g = g0 + (uint32_t)lane;
-      const BVNodeDev gr = groups[g < ngroups ? g : ngroups - 1u];
-      unsigned long long mg = __ballot(g < ngroups && box_overlaps(box, gr));
-      while (mg) {
-        const uint32_t at = (g0 + (uint32_t)__builtin_ctzll(mg)) * 64u + (uint32_t)lane;
-        mg &= mg - 1ull;
-        const BVNodeDev nd = leaves[at < nleaves ? at : nleaves - 1u];
-        bool isCand = at < nleaves && box_overlaps(box, nd) && !(grown && box_overlaps(before, nd));
-        // they join the candidate batch; a full batch is evaluated
-        unsigned long long mc = __ballot(isCand);
-        while (mc) {
-          const int room = 64 - ncands, found = (int)__popcll(mc);
-          const int fit = room < found ? room : found;
-          const int rank = __popcll(mc & ((1ull << lane) - 1ull));
-          if (isCand && rank < fit) {
-            L.cand_rank[ncands + rank] = (uint16_t)at;
-            L.cand_poly[ncands + rank] = nd.a;
-            isCand = false;
+    for (uint32_t g0 = 0; g0 < ngroups; g0 += 64 * kSnapGroupLoads) {
+      BVNodeDev gr[kSnapGroupLoads];
+#pragma unroll
+      for (int k = 0; k < kSnapGroupLoads; ++k) {
+        const uint32_t g = g0 + (uint32_t)(64 * k + lane);
+        gr[k] = groups[g < ngroups ? g : ngroups - 1u];
+      }
+      int ng = 0;
+#pragma unroll
+      for (int k = 0; k < kSnapGroupLoads; ++k) {
+        const uint32_t g = g0 + (uint32_t)(64 * k + lane);
+        const bool over = g < ngroups && box_overlaps(box, gr[k]);
+        const unsigned long long m = __ballot(over);
+        if (over) L.group[ng + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)g;
+        ng += (int)__popcll(m);
+      }
+      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      const bool last = g0 + 64 * kSnapGroupLoads >= ngroups;
+      for (int j = 0;; j += kSnapLeafLoads) {
+        if (j < ng) {
+          BVNodeDev nd[kSnapLeafLoads];
+          uint32_t at[kSnapLeafLoads];
+#pragma unroll
+          for (int k = 0; k < kSnapLeafLoads; ++k) {
+            const int gk = __builtin_amdgcn_readfirstlane((int)L.group[j + k < ng ? j + k : j]);
+            at[k] = (uint32_t)gk * kSnapGroup + (uint32_t)lane;
+            nd[k] = leaves[at[k] < nleaves ? at[k] : nleaves - 1u];
           }
-          ncands += fit;
+#pragma unroll
+          for (int k = 0; k < kSnapLeafLoads; ++k) {
+            // they join the candidates
+            const bool isCand = j + k < ng && at[k] < nleaves && box_overlaps(box, nd[k]) && !(grown && box_overlaps(before, nd[k]));
+            const unsigned long long m = __ballot(isCand);
+            if (isCand) {
+              const int c = ncands + (int)__popcll(m & ((1ull << lane) - 1ull));
+              L.cand_rank[c] = (uint16_t)at[k];
+              L.cand_poly[c] = nd[k].a;
+            }
+            ncands += (int)__popcll(m);
+          }
           __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
           __builtin_amdgcn_wave_barrier();
-          if (ncands == 64) flush();
-          mc = __ballot(isCand);
         }
+        const bool end = j + kSnapLeafLoads >= ng;
+        while (ncands >= (end && last ? 1 : 64)) flush();   // full batches, and what is left at the end
+        if (end) break;
       }
     }
-    if (ncands) flush();
     if (half >= kSnapHalf) break;
     const float reached = __uint_as_float(wave_umin(__float_as_uint(best)));
     const float clear = half - kSnapSlack;
