@@ -1048,10 +1048,9 @@ int bpsx_snap_points(bpsx_sim* sim, uint32_t scene, const float* pts, uint32_t n
   char* b = (char*)sim->d_batch;
   float* d_in = (float*)b; float* d_xyz = (float*)(b + f3); uint32_t* d_ref = (uint32_t*)(b + 2 * f3);
   HIP_TRY(hipMemcpy(d_in, pts, f3, hipMemcpyHostToDevice));
-  // a wavefront per point, as many as the device holds at once (32 per CU), not as a group has
-  // envs: 50000 samples, moves and snaps over a cluttered plan by a
-  // simulator of two envs took 316 ms, nearly all of it the snaps on 8 wavefronts, now 2.2 ms
-  launch_snap_batch(sim->nav, scene_entry(sim, scene), d_in, n, d_xyz, d_ref, sim->compute_units * 32u, nullptr);
+  // a wavefront per point for as many as the device holds at once (16 per CU); of more points each
+  // wavefront takes several
+  launch_snap_batch(sim->nav, scene_entry(sim, scene), d_in, n, d_xyz, d_ref, sim->compute_units * 16u, nullptr);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpy(out_xyz, d_xyz, f3, hipMemcpyDeviceToHost));
   HIP_TRY(hipMemcpy(out_ref, d_ref, (size_t)n * 4, hipMemcpyDeviceToHost));

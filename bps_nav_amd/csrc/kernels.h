@@ -58,7 +58,7 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
 void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
                   const GeoPool& G, uint32_t snap_blocks, hipStream_t st);
 void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz, uint32_t* oref,
-                       uint32_t snap_blocks, hipStream_t st);
+                       uint32_t waves, hipStream_t st);
 void launch_try_step_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                            uint32_t n, float* oxyz, uint32_t* oref, hipStream_t st);
 void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,

@@ -749,14 +749,27 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
 __global__ __launch_bounds__(64) void k_snap_batch(NavData nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz,
                                                    uint32_t* oref) {
   __shared__ SnapLds lds;
+  const uint32_t i = blockIdx.x;
+  if (i >= n) return;
   uint32_t c = 0;
-  for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-    const NavPt r = snap_point_wave(nav, nav.scenes[scene], pts[(size_t)i * 3], pts[(size_t)i * 3 + 1], pts[(size_t)i * 3 + 2], lds, &c);
-    if (threadIdx.x == 0) {
-      oxyz[(size_t)i * 3] = r.x; oxyz[(size_t)i * 3 + 1] = r.y; oxyz[(size_t)i * 3 + 2] = r.z;
-      oref[i] = r.ref;
-    }
+  const NavPt r = snap_point_wave(nav, nav.scenes[scene], pts[(size_t)i * 3], pts[(size_t)i * 3 + 1], pts[(size_t)i * 3 + 2], lds, &c);
+  if (threadIdx.x == 0) {
+    oxyz[(size_t)i * 3] = r.x; oxyz[(size_t)i * 3 + 1] = r.y; oxyz[(size_t)i * 3 + 2] = r.z;
+    oref[i] = r.ref;
   }
+}
+// per: points of a wavefront, up to kSnapBatch
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) void k_snap_points(NavData nav, uint32_t scene, const float* pts,
+                                                                                         uint32_t n, uint32_t per, float* oxyz, uint32_t* oref) {
+  __shared__ SnapBatchLds lds;
+  const uint32_t i = blockIdx.x * per + threadIdx.x;
+  const bool mine = threadIdx.x < per && i < n;
+  float p[3] = {0, 0, 0};
+  if (mine) load3(pts, i, p);
+  const NavPt r = snap_points_batch(nav, nav.scenes[scene], mine, p[0], p[1], p[2], lds);
+  if (!mine) return;
+  oxyz[(size_t)i * 3] = r.x; oxyz[(size_t)i * 3 + 1] = r.y; oxyz[(size_t)i * 3 + 2] = r.z;
+  oref[i] = r.ref;
 }
 __global__ __launch_bounds__(kMoveItems * 8) void k_try_step_batch(NavData nav, uint32_t scene, const float* sxyz, const uint32_t* sref,
                                                                    const float* exyz, uint32_t n, float* oxyz, uint32_t* oref) {
@@ -867,8 +880,17 @@ void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q,
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Q);
 }
 void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz, uint32_t* oref,
-                       uint32_t snap_blocks, hipStream_t st) {
-  hipLaunchKernelGGL(k_snap_batch, dim3(snap_blocks < n ? snap_blocks : n), dim3(64), 0, st, nav, scene, pts, n, oxyz, oref);
+                       uint32_t waves, hipStream_t st) {
+  // With more points than wavefronts the device holds at once, each wavefront takes several, so that all of them
+  // are under way from the start.  (4096 waves; 4200 points over a cluttered plan, a maze: 43, 36 us by a wavefront
+  // for each, 43, 38 by two points a wavefront; 6000: 52, 44 and 44, 39; 16384: 105, 87 and 72, 51.  Up to 4096,
+  // a wavefront for each is a shorter chain.)
+  if (n <= waves) {
+    hipLaunchKernelGGL(k_snap_batch, dim3(n), dim3(64), 0, st, nav, scene, pts, n, oxyz, oref);
+    return;
+  }
+  const uint32_t per = std::min((uint32_t)kSnapBatch, (n - 1u) / waves + 1u);
+  hipLaunchKernelGGL(k_snap_points, grid_for(n, per), dim3(64), 0, st, nav, scene, pts, n, per, oxyz, oref);
 }
 void launch_try_step_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                            uint32_t n, float* oxyz, uint32_t* oref, hipStream_t st) {

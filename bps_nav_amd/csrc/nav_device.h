@@ -408,7 +408,7 @@ BPSX_DEV void closest_on_boundary(const NavData& nav, const PolyRegs& P, float p
 //
 // Bound by the latency of those loads and by the divide-heavy edge distances of the candidates: most
 // points are on the mesh, and of the 200 polygons of a cluttered plan in the full box five remain.
-// (50000 points over a cluttered plan of 20k polygons: 1730 -> 277 us, now 238; 4096 points there, a wavefront
+// (50000 points over a cluttered plan of 20k polygons: 1730 -> 277 us, then 238; 4096 points there, a wavefront
 // each, 64 -> 14 us; snaps of 165 new episodes there next to the searches 135 -> 24 us.  The descent
 // tested one level per load and evaluated the whole box, a field of a record at a time.)
 constexpr float kSnapFirst = 0.25f;
@@ -423,6 +423,74 @@ struct SnapLds {
   uint16_t cand_rank[64 * (kSnapLeafLoads + 1)];   // place among the leaves
   uint16_t cand_poly[64 * (kSnapLeafLoads + 1)];
 };
+// the square of how far a point is at least from a polygon that it is not above or below
+BPSX_DEV float snap_bounds_dist2(const PolyRegs& P, float px, float pz) {
+  float x0 = P.x<0>(), x1 = x0, z0 = P.z<0>(), z1 = z0;
+  const int nv = P.nv();
+  static_for<1, kNvp>([&](auto I) BPSX_INLINE_LAMBDA {
+    constexpr int i = decltype(I)::value;
+    if (i < nv) {
+      x0 = fminf(x0, P.x<i>()); x1 = fmaxf(x1, P.x<i>());
+      z0 = fminf(z0, P.z<i>()); z1 = fmaxf(z1, P.z<i>());
+    }
+  });
+  const float bx = fmaxf(fmaxf(x0 - px, px - x1) - kSnapSlack, 0.0f), bz = fmaxf(fmaxf(z0 - pz, pz - z1) - kSnapSlack, 0.0f);
+  return bx * bx + bz * bz;
+}
+// The polygons of leaves that overlap `box`, without those that overlap `before` if that has been looked
+// at (grown), join the candidates: put(c, leaf, polygon) for the c-th.  flush() takes up to 64 of them out;
+// it is called while there are that many, and with `all` until none is left.
+template <class Put, class Flush>
+BPSX_DEV void snap_candidates(const BVNodeDev* leaves, uint32_t nleaves, uint16_t* list, const SnapBox& box, const SnapBox& before, bool grown,
+                              bool all, int lane, int& ncands, Put put, Flush flush) {
+  const uint32_t ngroups = (nleaves + 63u) / 64u;
+  const BVNodeDev* groups = leaves + nleaves;
+  for (uint32_t g0 = 0; g0 < ngroups; g0 += 64 * kSnapGroupLoads) {
+    BVNodeDev gr[kSnapGroupLoads];
+#pragma unroll
+    for (int k = 0; k < kSnapGroupLoads; ++k) {
+      const uint32_t g = g0 + (uint32_t)(64 * k + lane);
+      gr[k] = groups[g < ngroups ? g : ngroups - 1u];
+    }
+    int ng = 0;
+#pragma unroll
+    for (int k = 0; k < kSnapGroupLoads; ++k) {
+      const uint32_t g = g0 + (uint32_t)(64 * k + lane);
+      const bool over = g < ngroups && box_overlaps(box, gr[k]);
+      const unsigned long long m = __ballot(over);
+      if (over) list[ng + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)g;
+      ng += (int)__popcll(m);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    const bool last = all && g0 + 64 * kSnapGroupLoads >= ngroups;
+    for (int j = 0;; j += kSnapLeafLoads) {
+      if (j < ng) {
+        BVNodeDev nd[kSnapLeafLoads];
+        uint32_t at[kSnapLeafLoads];
+#pragma unroll
+        for (int k = 0; k < kSnapLeafLoads; ++k) {
+          const int gk = __builtin_amdgcn_readfirstlane((int)list[j + k < ng ? j + k : j]);
+          at[k] = (uint32_t)gk * kSnapGroup + (uint32_t)lane;
+          nd[k] = leaves[at[k] < nleaves ? at[k] : nleaves - 1u];
+        }
+#pragma unroll
+        for (int k = 0; k < kSnapLeafLoads; ++k) {
+          // they join the candidates
+          const bool isCand = j + k < ng && at[k] < nleaves && box_overlaps(box, nd[k]) && !(grown && box_overlaps(before, nd[k]));
+          const unsigned long long m = __ballot(isCand);
+          if (isCand) put(ncands + (int)__popcll(m & ((1ull << lane) - 1ull)), at[k], nd[k].a);
+          ncands += (int)__popcll(m);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      }
+      const bool end = j + kSnapLeafLoads >= ng;
+      while (ncands >= (end && last ? 1 : 64)) flush();   // full batches, and what is left at the end
+      if (end) break;
+    }
+  }
+}
 BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, float py, float pz, SnapLds& L,
                                uint32_t* ncand) {
   const int lane = (int)(threadIdx.x & 63);
@@ -432,9 +500,8 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
   if (!finite3(px, py, pz)) return out;
   if (!snap_box(s, px, py, pz, kSnapHalf).hit_tile || s.bv_count == 0) return out;
   if (!s.snap_leaves) return snap_point(nav, s, px, py, pz, ncand);  // every lane walks the same tree
-  const uint32_t nleaves = s.snap_leaves, ngroups = (nleaves + 63u) / 64u;
+  const uint32_t nleaves = s.snap_leaves;
   const BVNodeDev* leaves = nav.bv + s.bv_base + s.bv_count;
-  const BVNodeDev* groups = leaves + nleaves;
   const bool prune = s.snap_prune && fabsf(px) <= 2.0f * kSnapCoord && fabsf(pz) <= 2.0f * kSnapCoord;
   float best = kNone;              // per-lane running best
   uint32_t bestKey = 0xffffffffu;  // place of the lane's best candidate
@@ -469,17 +536,7 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
     }
     const float reached = __uint_as_float(wave_umin(__float_as_uint(best)));
     if (have && !inside) {
-      float x0 = P.x<0>(), x1 = x0, z0 = P.z<0>(), z1 = z0;
-      const int nv = P.nv();
-      static_for<1, kNvp>([&](auto I) BPSX_INLINE_LAMBDA {
-        constexpr int i = decltype(I)::value;
-        if (i < nv) {
-          x0 = fminf(x0, P.x<i>()); x1 = fmaxf(x1, P.x<i>());
-          z0 = fminf(z0, P.z<i>()); z1 = fmaxf(z1, P.z<i>());
-        }
-      });
-      const float bx = fmaxf(fmaxf(x0 - px, px - x1) - kSnapSlack, 0.0f), bz = fmaxf(fmaxf(z0 - pz, pz - z1) - kSnapSlack, 0.0f);
-      if (!(prune && bx * bx + bz * bz > reached)) {
+      if (!(prune && snap_bounds_dist2(P, px, pz) > reached)) {
         float cp[3];
         closest_on_boundary(nav, P, px, py, pz, cp);
         const float dx = px - cp[0], dy = py - cp[1], dz = pz - cp[2];
@@ -493,55 +550,10 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
   SnapBox box = snap_box(s, px, py, pz, half), before = box;
   bool grown = false;   // what overlaps `before` has been looked at
   for (;;) {
-    for (uint32_t g0 = 0; g0 < ngroups; g0 += 64 * kSnapGroupLoads) {
-      BVNodeDev gr[kSnapGroupLoads];
-#pragma unroll
-      for (int k = 0; k < kSnapGroupLoads; ++k) {
-        const uint32_t g = g0 + (uint32_t)(64 * k + lane);
-        gr[k] = groups[g < ngroups ? g : ngroups - 1u];
-      }
-      int ng = 0;
-#pragma unroll
-      for (int k = 0; k < kSnapGroupLoads; ++k) {
-        const uint32_t g = g0 + (uint32_t)(64 * k + lane);
-        const bool over = g < ngroups && box_overlaps(box, gr[k]);
-        const unsigned long long m = __ballot(over);
-        if (over) L.group[ng + __popcll(m & ((1ull << lane) - 1ull))] = (uint16_t)g;
-        ng += (int)__popcll(m);
-      }
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      const bool last = g0 + 64 * kSnapGroupLoads >= ngroups;
-      for (int j = 0;; j += kSnapLeafLoads) {
-        if (j < ng) {
-          BVNodeDev nd[kSnapLeafLoads];
-          uint32_t at[kSnapLeafLoads];
-#pragma unroll
-          for (int k = 0; k < kSnapLeafLoads; ++k) {
-            const int gk = __builtin_amdgcn_readfirstlane((int)L.group[j + k < ng ? j + k : j]);
-            at[k] = (uint32_t)gk * kSnapGroup + (uint32_t)lane;
-            nd[k] = leaves[at[k] < nleaves ? at[k] : nleaves - 1u];
-          }
-#pragma unroll
-          for (int k = 0; k < kSnapLeafLoads; ++k) {
-            // they join the candidates
-            const bool isCand = j + k < ng && at[k] < nleaves && box_overlaps(box, nd[k]) && !(grown && box_overlaps(before, nd[k]));
-            const unsigned long long m = __ballot(isCand);
-            if (isCand) {
-              const int c = ncands + (int)__popcll(m & ((1ull << lane) - 1ull));
-              L.cand_rank[c] = (uint16_t)at[k];
-              L.cand_poly[c] = nd[k].a;
-            }
-            ncands += (int)__popcll(m);
-          }
-          __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-        }
-        const bool end = j + kSnapLeafLoads >= ng;
-        while (ncands >= (end && last ? 1 : 64)) flush();   // full batches, and what is left at the end
-        if (end) break;
-      }
-    }
+    snap_candidates(leaves, nleaves, L.group, box, before, grown, true, lane, ncands, [&](int c, uint32_t at, uint16_t ip) BPSX_INLINE_LAMBDA {
+      L.cand_rank[c] = (uint16_t)at;
+      L.cand_poly[c] = ip;
+    }, flush);
     if (half >= kSnapHalf) break;
     const float reached = __uint_as_float(wave_umin(__float_as_uint(best)));
     const float clear = half - kSnapSlack;
@@ -565,6 +577,131 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
   out.y = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bp[1]), w));
   out.z = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(bp[2]), w));
   out.ref = s.ref_base | (uint32_t)__builtin_amdgcn_readlane((int)bestIp, w);
+  return out;
+}
+
+// The same for up to kSnapBatch points of one scene by one wavefront.  A point has about five candidates, so
+// evaluating each point's on their own leaves most lanes idle for the 2900 vector instructions of a
+// snap: here the points' boxes are scanned one after the other and their candidates are evaluated
+// together, 64 at a time, whichever points they belong to.  Point p's state is lane p's; the smallest
+// (distance, place in the array) of each point is found by atomics in LDS.  (50000 points over a cluttered
+// plan: 238 us by a wavefront for each, 159 here.)
+constexpr int kSnapBatch = 16;
+struct SnapBatchLds {
+  SnapLds snap;
+  uint8_t cand_point[64 * (kSnapLeafLoads + 1)];
+  unsigned long long best[kSnapBatch];   // bits of the smallest distance, place of its polygon
+  float pt[kSnapBatch][4];               // the point; whether its box grows
+  float at[kSnapBatch][4];               // the nearest point so far, its polygon
+};
+BPSX_DEV NavPt snap_points_batch(const NavData& nav, const SceneDev& s, bool mine, float px, float py, float pz, SnapBatchLds& B) {
+  const int lane = (int)(threadIdx.x & 63);
+  const float qnan = __int_as_float(0x7fc00000);
+  constexpr float kNone = 3.402823466e+38f;
+  NavPt out{qnan, qnan, qnan, 0};
+  uint32_t unused = 0;
+  if (!s.snap_leaves) return mine ? snap_point(nav, s, px, py, pz, &unused) : out;
+  auto sync = [&]() BPSX_INLINE_LAMBDA {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  mine = mine && finite3(px, py, pz);
+  mine = mine && snap_box(s, px, py, pz, kSnapHalf).hit_tile && s.bv_count != 0;
+  const bool prune = s.snap_prune && fabsf(px) <= 2.0f * kSnapCoord && fabsf(pz) <= 2.0f * kSnapCoord;
+  if (lane < kSnapBatch) {
+    B.best[lane] = ((unsigned long long)__float_as_uint(kNone) << 32) | 0xffffffffu;
+    B.pt[lane][0] = px; B.pt[lane][1] = py; B.pt[lane][2] = pz; B.pt[lane][3] = prune ? 1.0f : 0.0f;
+  }
+  sync();
+  const BVNodeDev* leaves = nav.bv + s.bv_base + s.bv_count;
+  int ncands = 0;
+  auto flush = [&]() {
+    const int fit = ncands < 64 ? ncands : 64;
+    ncands -= fit;
+    const bool have = lane < fit;
+    uint32_t ip = 0, key = 0, p = 0;
+    float qx = 0, qy = 0, qz = 0;
+    PolyRegs P;
+    bool inside = false, grows = false;
+    unsigned long long found = ~0ull;   // what the lane's polygon comes to
+    float cp[3] = {0, 0, 0};
+    if (have) {
+      ip = B.snap.cand_poly[ncands + lane];
+      key = B.snap.cand_rank[ncands + lane];
+      p = B.cand_point[ncands + lane];
+      qx = B.pt[p][0]; qy = B.pt[p][1]; qz = B.pt[p][2]; grows = B.pt[p][3] != 0;
+      const PolyRec* rec = &nav.polys[s.poly_base + ip];
+      P.load(rec);
+      float h = 0;
+      inside = poly_height(nav, P, *rec, qx, qy, qz, h);
+      if (inside) {
+        const float e = fabsf(qy - h) - s.climb, d = e > 0 ? e * e : 0;
+        cp[0] = qx; cp[1] = h; cp[2] = qz;
+        if (d < kNone) found = ((unsigned long long)__float_as_uint(d) << 32) | key;
+        atomicMin(&B.best[p], found);
+      }
+    }
+    sync();
+    if (have && !inside) {
+      const float reached = __uint_as_float((uint32_t)(B.best[p] >> 32));
+      if (!(grows && snap_bounds_dist2(P, qx, qz) > reached)) {
+        closest_on_boundary(nav, P, qx, qy, qz, cp);
+        const float dx = qx - cp[0], dy = qy - cp[1], dz = qz - cp[2];
+        const float d = dx * dx + dy * dy + dz * dz;
+        if (d < kNone) found = ((unsigned long long)__float_as_uint(d) << 32) | key;
+        atomicMin(&B.best[p], found);
+      }
+    }
+    sync();
+    if (have && found != ~0ull && B.best[p] == found) {   // one lane at most: a point meets each leaf once
+      B.at[p][0] = cp[0]; B.at[p][1] = cp[1]; B.at[p][2] = cp[2]; B.at[p][3] = __uint_as_float(ip);
+    }
+    sync();
+  };
+  float half = prune ? kSnapFirst : kSnapHalf;
+  SnapBox box = snap_box(s, px, py, pz, half), before = box;
+  bool grown = false;   // of all points that are still looked at alike: what overlaps `before` has been looked at
+  auto of_lane = [&](const SnapBox& b, int l) BPSX_INLINE_LAMBDA {
+    SnapBox r;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)((uint32_t)b.bmin[k] | ((uint32_t)b.bmax[k] << 16)), l);
+      r.bmin[k] = (uint16_t)v; r.bmax[k] = (uint16_t)(v >> 16);
+    }
+    r.hit_tile = true;
+    return r;
+  };
+  bool open = mine;
+  for (unsigned long long todo = __ballot(open); todo;) {
+    while (todo) {
+      const int p = __builtin_ctzll(todo);
+      todo &= todo - 1ull;
+      const SnapBox pb = of_lane(box, p), pbefore = of_lane(before, p);
+      snap_candidates(leaves, s.snap_leaves, B.snap.group, pb, pbefore, grown, todo == 0, lane, ncands, [&](int c, uint32_t at, uint16_t ip) BPSX_INLINE_LAMBDA {
+        B.snap.cand_rank[c] = (uint16_t)at;
+        B.snap.cand_poly[c] = ip;
+        B.cand_point[c] = (uint8_t)p;
+      }, flush);
+    }
+    if (open) {
+      const float reached = __uint_as_float((uint32_t)(B.best[lane] >> 32)), clear = half - kSnapSlack;
+      if (half >= kSnapHalf || reached < clear * clear) open = false;
+      else {
+        half = fminf(reached < kNone ? sqrtf(reached) * 1.0001f + 2.0f * kSnapSlack : 3.0f * half, kSnapHalf);
+        before = box;
+        box = snap_box(s, px, py, pz, half);
+      }
+    }
+    grown = true;
+    todo = __ballot(open);
+  }
+  if (!mine || (uint32_t)B.best[lane] == 0xffffffffu) return out;
+  const float x = B.at[lane][0];
+  if (isnan(x)) return out;
+  out.x = x;
+  out.y = B.at[lane][1];
+  out.z = B.at[lane][2];
+  out.ref = s.ref_base | __float_as_uint(B.at[lane][3]);
   return out;
 }
 

@@ -76,3 +76,29 @@ def test_snap_matches_the_walk_of_the_whole_box(oracle, name):
     assert len(bad) == 0, (len(bad), q[bad[:5]], xo[bad[:5]], xg[bad[:5]])
     cpu.close()
     gpu.close()
+
+
+@pytest.mark.parametrize("name", ["1", "4", "2 leaves"])
+def test_many_points_snap_like_few(name):
+    """A call of more points than wavefronts gives each several points and evaluates their candidates
+    together; every point's result is that of a call of few, bit for bit, whatever its neighbours are
+    and however the last wavefront is filled."""
+    import torch
+    from bps_nav_amd.bps_sim import nav_only
+    base, *how = name.split()
+    blob = scenes.config_scene(int(base), 1)
+    if how:
+        blob = changed(blob, how[0])
+    waves = 16 * torch.cuda.get_device_properties(0).multi_processor_count
+    q = points(blob, 6, 2000)
+    q = q[np.random.default_rng(7).permutation(len(q))]
+    gpu = nav_only([blob])
+    parts = [gpu.snap_points(0, q[i:i + 1000]) for i in range(0, len(q), 1000)]
+    x, r = (np.concatenate(v) for v in zip(*parts))
+    for n in (waves, waves + 1, 2 * waves + 5, 15 * waves + 1, 17 * waves + 3):
+        print(f"case: {n} snaps on {name}", flush=True)
+        at = np.arange(n) % len(q)
+        xn, rn = gpu.snap_points(0, q[at])
+        assert np.array_equal(rn, r[at])
+        assert np.array_equal(common.bits(xn), common.bits(x[at]))
+    gpu.close()
