@@ -8,7 +8,7 @@
 //   - the open list in registers: sorted by total, up to 256 entries (OpenList), which lets a
 //     pass expand up to kRows nodes at once (astar_fast); when totals tie, the reference's binary
 //     heap is rebuilt from a log of the list's operations (RefHeap, replay_log), and a search whose
-//     list outgrows the registers goes on with that heap,
+//     list outgrows the registers, or has a tie of more than 64, goes on with that heap,
 //   - the hash heads of the node pool,
 //   - for the first kLinksLds nodes one word with the polygon id and the hash chain link,
 //   - the position and cost of the kWindow most recently created nodes (slot = index
@@ -1026,18 +1026,20 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     if (ex == kAstarEmpty || ex == kAstarGoal) break;
     __builtin_amdgcn_s_setprio(3);   // a search that pays for a replay is late from here on
     replay_log(g, st);
-    if (ex == kAstarTie) {
-      // the reference pops what its heap has at the root: that entry goes first
+    // The reference pops what its heap has at the root: that entry goes first.  Equal totals have no
+    // defined order in the list, so where more than 64 share the smallest one (an end point so far away
+    // that a step's length is lost in the total's rounding) it may be none of the list's first 64.
+    const unsigned long long root = lanes_where(st.ol.n[0] == st.replayRoot && st.ol.t[0] == rlane(st.ol.t[0], 0));
+    if (ex == kAstarTie && root && st.replaySize == st.ol.size) {
       restore_window(g);
       g.tieReplays++;
-      const int p = first_lane(lanes_where(st.ol.n[0] == st.replayRoot));   // among the front's equal totals
       const uint32_t front = rlane(st.ol.n[0], 0);
       st.ol.n[0] = wlane(st.ol.n[0], st.replayRoot, 0);
-      st.ol.n[0] = wlane(st.ol.n[0], front, p);
+      st.ol.n[0] = wlane(st.ol.n[0], front, first_lane(root));
       resolved = true;
       continue;
     }
-    // a list beyond the registers or a full log: on with the reference's heap
+    // such a tie, a list beyond the registers or a full log: on with the reference's heap
     g.exactRuns++;
     if (ex == kAstarGrowHeap) g.heapSpills++;
     ex = astar_exact<true>(g, st, edges, endIp, endPos, pops);

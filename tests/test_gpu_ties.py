@@ -1,0 +1,40 @@
+"""Path searches in which many open nodes share the smallest total, against the oracle bit for bit.  The
+end point lies in a polygon of the mesh by its reference and far away by its coordinates, as far as the
+interface allows: a step's length is lost in the rounding of the totals, which then collapse to a few
+values or to one.  The order in which the reference's heap has equal totals decides the corridor."""
+import numpy as np
+import pytest
+
+from bps_nav_amd import scenes
+from tests import common
+
+pytestmark = pytest.mark.gpu
+
+
+# calls small enough for a wavefront with the whole pool in LDS each, for a block each, and beyond both
+@pytest.mark.parametrize("n,whole_block", [(400, True), (1600, True), (4000, False)])
+def test_equal_totals_match_oracle(oracle, n, whole_block):
+    from bps_nav_amd.bps_sim import nav_only
+    from oracle import bpo
+    print(f"case: {n} searches of equal totals", flush=True)
+    # 1936 polygons: a search of the whole room stays within the reference's pool of 2048 nodes
+    blob = scenes.gen_scene(scenes.BOX_ROOM, 7, cell=5, size_x=11.0, size_z=11.0, num_boxes=0)
+    cpu, gpu = bpo.Nav(oracle, blob), nav_only([blob])
+    pts = scenes.sample_points(blob, 9, 800)
+    x, r = cpu.snap(pts)
+    assert (r != 0).all()
+    a, ar, b, br = x[:400], r[:400], x[400:].copy(), r[400:]
+    # one distance in four as it is; up to 84 equal totals; over 700; all of them infinite
+    for k, far in enumerate((0.0, 1e6, 1e10, 1e25)):
+        b[k::4, 0] += np.float32(far)
+    want = cpu.geodesic(a, ar, b, br)
+    assert np.isfinite(want).all()
+    at = np.arange(n) % 400
+    got = gpu.geodesic(0, a[at], ar[at], b[at], br[at])
+    c = gpu.counters()   # of a new simulator: this call's
+    differ = np.nonzero(common.bits(want)[at] != common.bits(got))[0]
+    assert len(differ) == 0, (len(differ), differ[:8] % 4, want[at][differ[:5]], got[differ[:5]])
+    assert c["geo_tie_replays"] > n and c["geo_exact_runs"] >= n // 2
+    assert (c["geo_long_path"] == n) == whole_block
+    cpu.close()
+    gpu.close()
