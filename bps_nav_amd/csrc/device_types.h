@@ -45,12 +45,14 @@ static_assert(sizeof(PolyRec) == 128, "PolyRec must be one cache line");
 // with the same float operations) and which polygon lies behind it.  Six of them per polygon,
 // so lane j of a wavefront fetches edge j of the expanded polygon with one 16-byte load.
 struct AEdge {
-  float mid[3];
+  float mid[3];  // finite: a coordinate that is not (a vertex that is NaN or infinite) is kFarMid, whose
+                 // distances are infinite, where the reference's are NaN
   uint32_t nb;   // polygon index behind the edge if the search may enter it (internal link to
                  // a polygon that passes the query filter), else kNoNb
 };
 static_assert(sizeof(AEdge) == 16, "AEdge");
 constexpr int kEdgeStride = 8;   // records per polygon in HBM: six edges and two unused, one 128-byte line
+constexpr float kFarMid = 1e30f;   // its square overflows, its distance to itself is 0
 constexpr uint32_t kNoNb = 0xfffeu;   // (not all ones: that is what a lane past the end of its hash chain reads)
 
 // dtBVNode repacked at upload: same quantised bounds; a leaf carries its polygon index, an

@@ -109,6 +109,7 @@ template <int Ctrl, int RowMask> BPSX_DEV uint32_t umin_dpp(uint32_t v) {
 //   - the polygon that a node was reached from need not be left out of its neighbours: the way back
 //     costs no less than the parent's own cost (costs only ever fall, both ways have the same
 //     length, and rounding is monotonic), so its total is no better and it is left alone anyway.
+//     (With a NaN two nodes would update each other for ever: there is none, see AEdge.)
 // Without both a pass is some 25 of 630 instructions and three LDS accesses shorter: 1.286 -> 1.229 ms
 // of k_geodesic at 16384 agents over mazes, 5 % off the longest of 64 searches alone on the GPU.
 constexpr uint32_t kChainEnd = 0xffffu;
@@ -118,9 +119,9 @@ BPSX_DEV uint32_t link_next(uint32_t l) { return l >> 16; }
 BPSX_DEV uint32_t make_link(uint32_t id, uint32_t next) { return id | (next << 16); }
 
 // Open-list entries: the total as a bit pattern, compared as an unsigned integer (totals are sums of
-// distances, never negative and never NaN, and for such floats the integer order of the bits is the
-// float order), and the node's index (bits 0-10) with its polygon index above it, so that the entry
-// at the front names the edge records to fetch without a detour through LDS.
+// distances between finite points, never negative and never NaN, and for such floats the integer
+// order of the bits is the float order), and the node's index (bits 0-10) with its polygon index above
+// it, so that the entry at the front names the edge records to fetch without a detour through LDS.
 static_assert(kMaxNodes <= 2048, "open-list entries keep the node index in 11 bits");
 constexpr uint32_t kEmptyKey = 0x7fffffffu;   // above +inf; every key stays below 2^31
 
@@ -1124,8 +1125,15 @@ BPSX_DEV float funnel_length(int lane, FunnelLds* F, const NavData& nav, const S
   int npts = 1;
   float length = 0.0f;
   bool finished = false, overflow = false;
+  int merged = 0;
   auto append = [&](const float* p, bool isEnd) {
-    if (all(vequal(last, p))) return;  // merged with the previous point
+    if (all(vequal(last, p))) {
+      // Merged with the previous point.  Between finite portals the apex then moves on to a later one, but
+      // for once at the first.  At a side that is not finite all may stay as it was, and the reference walks
+      // for ever: no path.
+      if (++merged > 2 * kMaxPath) { overflow = true; finished = true; }
+      return;
+    }
     const float dx = last[0] - p[0], dy = last[1] - p[1], dz = last[2] - p[2];
     length += sqrtf(dx * dx + (dy * dy + dz * dz));
     last[0] = p[0]; last[1] = p[1]; last[2] = p[2];

@@ -251,7 +251,10 @@ int parse_navmesh(const uint8_t* b, size_t n, HostScene* out) {
       r.walk[k] = (ne && !(ne & kExtLink) && (s.polys[ne - 1].flags & kPolyFlagWalk)) ? ne : 0;
       const float* l = r.v[k];
       const float* rt = r.v[k + 1 < r.nv ? k + 1 : 0];
-      for (int c = 0; c < 3; ++c) e[k].mid[c] = (l[c] + rt[c]) * 0.5f;
+      for (int c = 0; c < 3; ++c) {
+        const float mid = (l[c] + rt[c]) * 0.5f;
+        e[k].mid[c] = std::isfinite(mid) ? mid : kFarMid;
+      }
       if (!r.walk[k]) continue;
       // a polygon behind two edges: expanding through the second never changes its node (same
       // position, not a lower cost), so only the first edge leads there
