@@ -379,7 +379,7 @@ struct GeoWave {
   GeoSlot* ws;
   int lane;
   int nodeCount;
-  uint32_t linkSpills, heapSpills;   // queries that left the LDS links / whose open list left the registers
+  uint32_t linkSpills, heapSpills;   // queries that left the LDS links / whose heap, once they went on with it, left LDS
 #ifdef BPSX_PHASE_TIMING
   unsigned long long phase[8], phase_t0;
 #endif
@@ -911,7 +911,6 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       // the reference carries on without the nodes that do not fit, but reports anything found
       // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): stop
       if (S && want > kMaxNodes) {
-        if (kLinksLds >= kMaxNodes) g.linkSpills++;   // where the LDS holds the links of a full pool: a search that needs more than those
         st.outOfNodes = true;
         return kAstarEmpty;
       }
@@ -1042,9 +1041,9 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     }
     // such a tie, a list beyond the registers or a full log: on with the reference's heap
     g.exactRuns++;
-    if (ex == kAstarGrowHeap) g.heapSpills++;
     ex = astar_exact<true>(g, st, edges, endIp, endPos, pops);
     if (ex == kAstarGrowHeap) {
+      g.heapSpills++;
       uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
       const uint2* h = g.L->heap();
       for (int i = lane + 1; i <= st.replaySize; i += 64) kept[i] = h[i];

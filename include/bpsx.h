@@ -207,8 +207,9 @@ BPSX_API int bpsx_check_errors(bpsx_sim *sim);
  * [4] corridor polygons string-pulled, [5] resets, [6] polygons visited by moves,
  * [7] snap candidates; [8..15] are zero unless the library was built with -DBPSX_PHASE_TIMING
  * (cycle counts of the A* loop's phases, a diagnostic build); [16] path searches that needed
- * more node links than the kernel keeps in LDS, [17] path searches whose open list outgrew
- * the kernel's registers (both continue in slower code; results are the same), [18] path
+ * more node links than the kernel keeps in LDS (none where it keeps those of a full pool), [17] path
+ * searches that went on with the reference's heap (see [19]) and whose heap outgrew LDS (both
+ * continue in slower code; results are the same), [18] path
  * searches that the kernel runs with larger LDS structures: those expected to be among the longest
  * of their step, or all where there is a block for each (same results).  The path search keeps its open list sorted by total instead of
  * in the reference's heap arrangement, which only matters when two open nodes share the

@@ -60,7 +60,13 @@ def test_batched_queries_match_oracle(oracle, torch_cuda, config):
     gg = gen.geodesic(0, a, ar, b, br)
     assert np.array_equal(common.bits(go), common.bits(gg)), \
         f"{(common.bits(go) != common.bits(gg)).sum()} of {m} geodesics differ"
-    if config == 4:  # maze-wide pairs: searches that outgrow the node links kept in LDS
+    if config == 4:
+        # maze-wide pairs: searches that outgrow the node links kept in LDS, in a call that has too many of
+        # them for a whole block's LDS each; in the one above there are links for a full pool
+        assert gen.counters()["geo_link_spills"] == 0
+        many = np.arange(3000) % m
+        gg = gen.geodesic(0, a[many], ar[many], b[many], br[many])
+        assert np.array_equal(common.bits(go)[many], common.bits(gg))
         assert gen.counters()["geo_link_spills"] > 20
     if config >= 3:  # equal totals at the front of the open list: taken as a pair, or settled from the operation log
         assert gen.counters()["geo_pair_ties"] > 5 and gen.counters()["geo_tie_replays"] > 0
@@ -167,8 +173,9 @@ def test_recast_built_meshes_match_reference_vectors(oracle, torch_cuda, name):
 
 def test_open_hall_queries_match_oracle(oracle, torch_cuda):
     """A hall without obstacles: A* spreads over a wide front, so the open list outgrows the
-    kernel's register heap, the node links outgrow LDS and long queries exhaust Detour's
-    2048-node pool.  Every continuation path of the kernel must still equal the oracle."""
+    registers, the node links outgrow LDS and long queries exhaust Detour's 2048-node pool; with end
+    points far away the heap that then takes the list's place outgrows LDS.  Every continuation path
+    of the kernel must still equal the oracle."""
     from bps_nav_amd import scenes
     from oracle import bpo
     print("case: open hall (spill paths of the A* kernel)", flush=True)
@@ -188,13 +195,21 @@ def test_open_hall_queries_match_oracle(oracle, torch_cuda):
     c0 = gen.counters()
     go = nav.geodesic(a, ar, b, br)
     gg = gen.geodesic(0, a, ar, b, br)
-    c1 = gen.counters()
     assert np.array_equal(common.bits(go), common.bits(gg)), \
         f"{(common.bits(go) != common.bits(gg)).sum()} of {m} geodesics differ"
     assert np.isinf(go).any() and np.isfinite(go).sum() > m // 3
-    # open lists beyond the sorted form's registers run again with the exact heap, which in turn
-    # leaves its registers; ties between equal totals occur on the way
-    assert c1["geo_exact_runs"] - c0["geo_exact_runs"] > 10, "exact re-run path not exercised"
+    # too many for a whole block's LDS each
+    many = np.arange(4 * m) % m
+    gm = gen.geodesic(0, a[many], ar[many], b[many], br[many])
+    assert np.array_equal(common.bits(go)[many], common.bits(gm))
+    assert gen.counters()["geo_link_spills"] - c0["geo_link_spills"] > 10, "link spill path not exercised"
+    far = b + np.array([1e10, 0, 0], np.float32)
+    gf = gen.geodesic(0, a, ar, far, br)
+    assert np.array_equal(common.bits(nav.geodesic(a, ar, far, br)), common.bits(gf))
+    c1 = gen.counters()
+    # open lists beyond the sorted form's registers go on with the reference's heap, which in turn
+    # leaves LDS; ties between equal totals occur on the way
+    assert c1["geo_exact_runs"] - c0["geo_exact_runs"] > 10, "exact path not exercised"
     assert c1["geo_heap_spills"] - c0["geo_heap_spills"] > 10, "heap spill path not exercised"
     assert c1["geo_pair_ties"] - c0["geo_pair_ties"] > 50 and c1["geo_tie_replays"] - c0["geo_tie_replays"] > 0, \
         "tie paths not exercised"
