@@ -875,7 +875,7 @@ static int batch_reserve(bpsx_sim* sim, size_t bytes) {
 // many blocks of k_geodesic as the device holds at once, or one per query where that is less.  The
 // steps' own pools serve if they are enough (a simulator has no more of them than envs in a group);
 // otherwise the batch has pools of its own, kept until a larger batch or bpsx_destroy replaces them
-// (at most 0.7 GB).
+// (at most 0.7 GB); where the device has no room for those, the steps' pools serve it all the same.
 // (1000 pairs over a maze, simulator of 4 envs, so far served by 4 blocks: 131 -> 2.3 ms a call.)
 static int batch_reserve_slots(bpsx_sim* sim, uint32_t n, GeoPool* out) {
   const bool few = n <= sim->max_few_blocks;
@@ -886,7 +886,11 @@ static int batch_reserve_slots(bpsx_sim* sim, uint32_t n, GeoPool* out) {
       if (sim->d_batch_slots) HIP_TRY(hipFree(sim->d_batch_slots));
       sim->d_batch_slots = nullptr;
       sim->batch_slots = 0;
-      HIP_TRY(hipMalloc((void**)&sim->d_batch_slots, (size_t)want * sizeof(GeoSlot)));
+      if (hipMalloc((void**)&sim->d_batch_slots, (size_t)want * sizeof(GeoSlot)) != hipSuccess) {
+        (void)hipGetLastError();   // answered here: not an error of the launches to come
+        sim->d_batch_slots = nullptr;
+        return BPSX_OK;
+      }
       sim->batch_slots = want;
     }
     out->slots = sim->d_batch_slots;
