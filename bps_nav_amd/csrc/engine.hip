@@ -711,6 +711,9 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   hipStream_t st = (hipStream_t)hip_stream;
   // steps that have completed leave the ring; a full ring makes the host wait for its oldest step
   if ((rc = retire_steps(sim, sim->ring_count == kStepRing ? 1 : 0))) return rc;
+  // Steps of all groups share the searches' node pools, so each waits for the one before, whichever
+  // stream that was given (on the same one it comes after it anyway).
+  if (sim->ring_count) HIP_TRY(hipStreamWaitEvent(st, sim->ring[(sim->ring_head + sim->ring_count - 1) % kStepRing].done, 0));
   const int64_t* d_act = actions;
   if (!actions_on_device) {
     // the staging buffer may still be waiting to be read by a step that has not run yet

@@ -187,13 +187,14 @@ BPSX_API int bpsx_step_end(bpsx_sim *sim, uint32_t group);
 /* Stream-ordered stepping ("step_end = no-op if the consumer is stream-ordered"): with
  * enabled != 0, step_end does not wait for the device.  The step's outputs are complete for
  * everything enqueued afterwards on the stream that step_start was given (device-to-device
- * copies into a rollout storage, the policy's kernels, the next step_start), and a consumer on
- * the host calls bpsx_synchronize (or synchronizes that stream) before it reads them.  The host
- * may run up to four steps ahead of the device; step_start waits for the oldest of them when it
- * would be more.  Host-side action arrays (actions_on_device == 0) make step_start wait for all
- * earlier steps; while per-kernel timing is on, step_end waits as in the default mode.  Entry
- * points that bring results to the host (reset, the batched queries, counters, errors, swap
- * status) wait for outstanding steps by themselves.  The one-outstanding-step rule
+ * copies into a rollout storage, the policy's kernels); the next step, of whichever group and on
+ * whichever stream, waits for this one on the device; a consumer on the host calls
+ * bpsx_synchronize (or synchronizes that stream) before it reads them.  The host may run up to four
+ * steps ahead of the device; step_start waits for the oldest of them when it would be more.
+ * Host-side action arrays (actions_on_device == 0) make step_start wait for all earlier steps;
+ * while per-kernel timing is on, step_end waits as in the default mode.  Entry points that bring
+ * results to the host (reset, the batched queries, counters, errors, swap status) wait for
+ * outstanding steps by themselves.  The one-outstanding-step rule
  * (simulator.cpp:1659-1662, 1679-1689) is unchanged: step_start, step_end, step_start, ... */
 BPSX_API int bpsx_set_stream_ordered(bpsx_sim *sim, int enabled);
 /* Waits until every step enqueued so far has completed on the device. */

@@ -127,14 +127,16 @@ def compare_recorded(cpu, rec, t, where, group=0):
     return co, cs
 
 
-@pytest.mark.parametrize("config,num_scenes,n,steps,groups", [(4, 4, 256, 260, 1), (2, 4, 256, 240, 2)])
-def test_stream_ordered_stepping_parity(oracle, torch_cuda, config, num_scenes, n, steps, groups):
+@pytest.mark.parametrize("config,num_scenes,n,steps,groups,own_streams", [
+    (4, 4, 256, 260, 1, False), (2, 4, 256, 240, 2, False), (4, 4, 512, 160, 2, True)])
+def test_stream_ordered_stepping_parity(oracle, torch_cuda, config, num_scenes, n, steps, groups, own_streams):
     """bpsx_set_stream_ordered: step_end does not wait, the host runs ahead of the device, and a
     consumer on the same stream (device-to-device copies after every step) sees every step
-    complete.  All recorded steps are compared with the oracle afterwards."""
+    complete, also where each group is stepped on a stream of its own.  All recorded steps are compared
+    with the oracle afterwards."""
     torch = torch_cuda
     from oracle import bpo
-    print(f"case: stream-ordered stepping, config {config}, {groups} group(s)", flush=True)
+    print(f"case: stream-ordered stepping, config {config}, {groups} group(s), streams of their own: {own_streams}", flush=True)
     sc = common.build_scenes(oracle, config, num_scenes, episodes_per_scene=32)
     gen = make_gen(sc, n, seed=37, double_buffered=groups == 2, stream_ordered=True)
     per = n // groups
@@ -143,13 +145,15 @@ def test_stream_ordered_stepping_parity(oracle, torch_cuda, config, num_scenes, 
     acts = common.action_stream(config, steps, per)
     dev_acts = torch.from_numpy(np.stack(acts)).cuda()
     recs = [Recorder(torch, gen, g, steps) for g in range(groups)]
+    streams = [torch.cuda.Stream() if own_streams else torch.cuda.current_stream() for _ in range(groups)]
     torch.cuda.synchronize()
     t0 = time.perf_counter()
     for t in range(steps):
         g = t % groups
-        gen.step_start(g, dev_acts[t])
-        gen.step_end(g)
-        recs[g].take(t)
+        with torch.cuda.stream(streams[g]):
+            gen.step_start(g, dev_acts[t])
+            gen.step_end(g)
+            recs[g].take(t)
     enqueued = time.perf_counter() - t0
     gen.synchronize()
     torch.cuda.synchronize()
