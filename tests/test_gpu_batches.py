@@ -10,6 +10,19 @@ from tests import common
 pytestmark = pytest.mark.gpu
 
 
+def compute_units():
+    import torch
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
+def limit(name):
+    """The largest batch that is served one way; one more item goes the next way.  Path queries: a wavefront
+    with the whole node pool in LDS each (three on a CU), a block of two wavefronts each (ten on a CU), more
+    share those.  Snaps: a wavefront each (sixteen on a CU), several to a wavefront.  Allocation-free path
+    queries: a wavefront with the whole pool in LDS for each of 768, more share as many."""
+    return {"pool": 3, "block": 10, "snap": 16, "static": 3}[name] * (256 if name == "static" else compute_units())
+
+
 def points(oracle, n):
     from oracle import bpo
     blob = scenes.config_scene(2, 3)
@@ -17,21 +30,46 @@ def points(oracle, n):
     return blob, bpo.Nav(oracle, blob), pts
 
 
-@pytest.mark.parametrize("n", [1, 2, 3, 513, 2304, 2305, 9001])
-def test_batch_sizes(oracle, n):
-    """Up to 2304 path queries get a block of two wavefronts each (nine blocks on each of 256 CUs),
-    more share them; up to 8192 snaps get a wavefront each."""
+SIZES = [1, 2, 3, 513, 2304, 2305, 9001] + [(name, k) for name in ("pool", "block", "snap") for k in (-1, 0, 1)]
+
+
+@pytest.mark.parametrize("size", SIZES, ids=lambda s: str(s) if isinstance(s, int) else f"{s[0]}{s[1]:+d}")
+def test_batch_sizes(oracle, size):
+    """Small and odd sizes, and each side of the limits above."""
     from bps_nav_amd.bps_sim import nav_only
-    from oracle import bpo
+    n = size if isinstance(size, int) else limit(size[0]) + size[1]
     print(f"case: batches of {n}", flush=True)
-    blob = scenes.config_scene(2, 3)
-    cpu, gpu = bpo.Nav(oracle, blob), nav_only([blob])
-    pts = scenes.sample_points(blob, 17, 2 * n) + np.random.default_rng(n).normal(0, 0.2, (2 * n, 3)).astype(np.float32)
-    xo, ro = cpu.snap(pts)
-    xg, rg = gpu.snap_points(0, pts)
+    blob, cpu, pts = points(oracle, n)
+    gpu = nav_only([blob])
+    xo, ro = cpu.snap(pts[:n])
+    xg, rg = gpu.snap_points(0, pts[:n])
     assert np.array_equal(ro, rg) and np.array_equal(common.bits(xo), common.bits(xg))
-    d = gpu.geodesic(0, xo[:n], ro[:n], xo[n:], ro[n:])
-    assert np.array_equal(common.bits(cpu.geodesic(xo[:n], ro[:n], xo[n:], ro[n:])), common.bits(d))
+    x2, r2 = cpu.snap(pts[n:])
+    d = gpu.geodesic(0, xo, ro, x2, r2)
+    assert np.array_equal(common.bits(cpu.geodesic(xo, ro, x2, r2)), common.bits(d))
+    # every search with larger LDS structures up to the second limit, none beyond
+    c = gpu.counters()
+    assert c["geo_long_path"] == (c["geodesic_queries"] if n <= limit("block") else 0)
+    cpu.close()
+    gpu.close()
+
+
+@pytest.mark.parametrize("size", [1, 383, 385, ("static", -1), ("static", 0), ("static", 1), 4096],
+                         ids=lambda s: str(s) if isinstance(s, int) else f"{s[0]}{s[1]:+d}")
+def test_allocation_free_sizes(oracle, size):
+    """The allocation-free entry point, which shares 384 blocks among more queries than it has pools for."""
+    import torch
+    from bps_nav_amd.bps_sim import nav_only
+    n = size if isinstance(size, int) else limit(size[0]) + size[1]
+    print(f"case: {n} allocation-free path queries", flush=True)
+    blob, cpu, pts = points(oracle, n)
+    gpu = nav_only([blob])
+    x, r = cpu.snap(pts)
+    dev = [torch.from_numpy(v).cuda() for v in (x[:n], r[:n].view(np.int32), x[n:], r[n:].view(np.int32))]
+    got = gpu.geodesic_static(0, *dev).cpu().numpy()
+    assert np.array_equal(common.bits(cpu.geodesic(x[:n], r[:n], x[n:], r[n:])), common.bits(got))
+    c = gpu.counters()
+    assert c["geodesic_queries"] == n and c["geo_long_path"] == (n if n <= limit("static") else 0)
     cpu.close()
     gpu.close()
 

@@ -1,4 +1,4 @@
-"""snapPoint by a wavefront: the box that grows with the best distance against the oracle's walk of the
+"""snapPoint by a wavefront, for one point and for several at once: the box that grows with the best distance against the oracle's walk of the
 whole 4 x 8 x 4 m box, bit for bit, on points where the two could part: on vertices, edges and
 midpoints shared by polygons, above and below the mesh, between rooms, at the mesh's corners (where the
 tree's spare zero leaf counts) and outside; and on navmeshes whose BV tree does not allow the growing
@@ -57,6 +57,7 @@ def points(blob, seed, n):
 
 @pytest.mark.parametrize("name", ["1", "2", "3", "4", "recast_room", "recast_two_floors", "2 leaves", "3 leaves", "2 inner", "recast_room leaves"])
 def test_snap_matches_the_walk_of_the_whole_box(oracle, name):
+    import torch
     from bps_nav_amd.bps_sim import nav_only
     from oracle import bpo
     print(f"case: snaps on {name}", flush=True)
@@ -71,9 +72,14 @@ def test_snap_matches_the_walk_of_the_whole_box(oracle, name):
     q = points(blob, 5, 1500)
     cpu, gpu = bpo.Nav(oracle, blob), nav_only([blob])
     xo, ro = cpu.snap(q)
-    xg, rg = gpu.snap_points(0, q)
-    bad = np.nonzero((ro != rg) | (common.bits(xo) != common.bits(xg)).any(axis=1))[0]
-    assert len(bad) == 0, (len(bad), q[bad[:5]], xo[bad[:5]], xg[bad[:5]])
+    # a wavefront for each point, as the resets snap them, and several points to a wavefront
+    waves = 16 * torch.cuda.get_device_properties(0).multi_processor_count
+    assert len(q) > waves
+    for per_call in (waves, len(q)):
+        parts = [gpu.snap_points(0, q[i:i + per_call]) for i in range(0, len(q), per_call)]
+        xg, rg = (np.concatenate(v) for v in zip(*parts))
+        bad = np.nonzero((ro != rg) | (common.bits(xo) != common.bits(xg)).any(axis=1))[0]
+        assert len(bad) == 0, (per_call, len(bad), q[bad[:5]], xo[bad[:5]], xg[bad[:5]])
     cpu.close()
     gpu.close()
 
