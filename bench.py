@@ -301,7 +301,7 @@ def main():
         f"{profiled_elapsed / P * 1e3:.3f} ms/step, per-kernel ms/step {json.dumps({k: round(v, 4) for k, v in kt.items()})}")
     log(f"per step: {d['geodesic_queries'] / P:.0f} geodesic queries, {d['astar_pops'] / max(1, d['geodesic_queries']):.0f} "
         f"A* pops/query, corridor {d['corridor_polys'] / max(1, d['geodesic_queries']):.1f} polys/query, "
-        f"{d['resets'] / P:.1f} resets, {d.get('geo_link_spills', 0) / P:.0f} link spills, {d.get('geo_heap_spills', 0) / P:.0f} heap spills, {d.get('geo_long_path', 0) / P:.0f} on the large-LDS path, {d.get('geo_exact_runs', 0) / P:.0f} run again with the exact heap, {d.get('geo_pair_ties', 0) / P:.0f} tied pairs taken in one pass, {d.get('geo_tie_replays', 0) / P:.0f} ties resolved from the log; non-finite distances now: {int((~np.isfinite(dist)).sum())} of {N}")
+        f"{d['resets'] / P:.1f} resets, {d.get('geo_link_spills', 0) / P:.0f} link spills, {d.get('geo_heap_spills', 0) / P:.0f} heap spills, {d.get('geo_long_path', 0) / P:.0f} on the large-LDS path, {d.get('geo_exact_runs', 0) / P:.0f} that went on with the reference's heap, {d.get('geo_pair_ties', 0) / P:.0f} tied pairs taken in one pass, {d.get('geo_tie_replays', 0) / P:.0f} ties resolved from the log; non-finite distances now: {int((~np.isfinite(dist)).sum())} of {N}")
     # roofline of the dominant kernel (geodesic over the step's queries), HIP-event timed; the
     # counters cover the profiled pass
     dominant = max(kt, key=kt.get)

@@ -319,7 +319,7 @@ namespace BPSX_GEO_NS {
 #define BPSX_WINDOW 128
 #endif
 constexpr int kLinksLds = BPSX_LINKS_LDS;   // nodes whose link word is kept in LDS
-constexpr int kWindow = BPSX_WINDOW;        // most recent nodes whose position/cost/total are kept in LDS
+constexpr int kWindow = BPSX_WINDOW;        // most recent nodes whose position and cost are kept in LDS
 #ifndef BPSX_HASH
 #define BPSX_HASH 512
 #endif
@@ -399,7 +399,7 @@ struct GeoWave {
     if (!S || kLinksLds >= kMaxNodes || i < kLinksLds) L->n_link[i] = v;
     else { BPSX_KEEP_APART(); ws->links[i] = v; BPSX_KEEP_APART(); }
   }
-  // node i still has its position/cost/total in LDS
+  // node i still has its position and cost in LDS
   BPSX_DEV bool in_window(int i) const { return kAllLds || i >= nodeCount - kWindow; }
   // node i, whose position and cost are not looked for in the window; and a node and its parent index stored outside of it
   BPSX_DEV float4 node(int i) const {
@@ -472,6 +472,7 @@ struct GeoWave {
 constexpr int kHeapLds = kAllLds ? 64 * OpenList::kPairs + 2 * kRows * kNvp + 1 : (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
 static_assert(kLinksLds % 4 == 0 && offsetof(GeoLds, w_node) == offsetof(GeoLds, n_link) + 4 * (kLinksLds + kTagSlots),
               "the marks are accessed as 16 bytes, and the heap lies over the marks and the window");
+// (383 entries, 639 of a whole block's LDS, 353 next to a whole node pool)
 static_assert(kHeapLds >= 64 * OpenList::kPairs + 2 * kRows * kNvp, "a heap with as many entries as the sorted list must fit");
 struct RefHeap {
   uint2* h;    // total bits, packed node

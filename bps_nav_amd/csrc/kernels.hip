@@ -857,9 +857,13 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
   // (the snaps are a launch of their own when the launches are being timed one by one)
   if (ev) hipLaunchKernelGGL(k_reset_snap, dim3(step_snap_blocks), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Qnext, P);
   mark();
+  // Three agents in five ask for a distance in a step; a group's queries are taken for three in four, with
+  // room for one that asks more, so k_geodesic_few serves groups of up to 1024 agents.  (The line could lie
+  // higher: a step over room plans, mazes takes 879, 728 us by k_geodesic and 836, 691 by k_geodesic_few at
+  // 1184 agents, 887, 782 and 837, 745 at 1600, where over rooms both take 320.)
   if (P.task != BPSX_TASK_EXPLORATION)   // which asks for no distance
     launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                    A.last_cost, G, P.n - P.n / 4u, P.counters, st);   // three agents in five ask for a distance in a step
+                    A.last_cost, G, P.n - P.n / 4u, P.counters, st);
   mark();
   const uint32_t with_snaps = ev ? 0u : step_snap_blocks;
   hipLaunchKernelGGL(k_step_finish, dim3(with_snaps + grid_for(P.n, 256).x), dim3(256), 0, st, nav, A, P, Q, Qnext, with_snaps);

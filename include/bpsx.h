@@ -171,12 +171,10 @@ BPSX_API int bpsx_num_groups(const bpsx_sim *sim, uint32_t *out);
 BPSX_API int bpsx_reset(bpsx_sim *sim, uint32_t group, void *hip_stream);
 /* step_start(group, actions): actions int64[n] in {0 stop, 1 forward, 2 left, 3 right};
  * actions_on_device != 0 => device pointer (read in stream order), else host pointer
- * (copied before returning).  Enqueues the step; returns without waiting.  Part of the step
- * (the snaps of the episodes that begin in it) runs on a stream of the library's own, forked
- * from and joined to hip_stream with events: work enqueued on hip_stream afterwards sees the
- * whole step.  The first distance of an episode that begins in a step is measured by the next
- * step (the reference measures it at once, simulator.cpp:744-751, and uses it from the next
- * step on): outputs and state arrays are the same after every step. */
+ * (copied before returning).  Enqueues the step on hip_stream; returns without waiting.  The
+ * first distance of an episode that begins in a step is measured by the next step (the reference
+ * measures it at once, simulator.cpp:744-751, and uses it from the next step on): outputs and
+ * state arrays are the same after every step. */
 BPSX_API int bpsx_step_start(bpsx_sim *sim, uint32_t group, const int64_t *actions,
                     int actions_on_device, void *hip_stream);
 /* step_end(group): waits until the step's outputs are complete (host-synchronous stepping, the
@@ -251,11 +249,11 @@ BPSX_API int bpsx_geodesic(bpsx_sim *sim, uint32_t scene, const float *start_xyz
  * loops, harnesses that forbid hipMalloc).  No counterpart in the reference.  Same distances as
  * bpsx_geodesic, but every pointer is a DEVICE pointer, the work is enqueued on hip_stream and
  * the call returns without waiting (out_dist is complete when the stream reaches that point),
- * and the call allocates nothing: its queue, A* node pools and operation logs live in an array of about 96 MB
- * that each GPU the library runs on holds from library load until the process ends.  At most
- * BPSX_STATIC_MAX_QUERIES queries per call (BPSX_E_INVAL beyond).  All calls on one GPU share
- * that array: calls that overlap on one GPU (other streams, other simulators) race; calls on
- * one stream are safe.  Must not be called between step_start and step_end. */
+ * and the call allocates nothing: its queue, A* node pools and operation logs live in an array of
+ * 97.7 MB that each GPU a process uses the library on holds from library load until the process
+ * ends.  At most BPSX_STATIC_MAX_QUERIES queries per call (BPSX_E_INVAL beyond).  All calls on one
+ * GPU share that array: calls that overlap on one GPU (other streams, other simulators) race;
+ * calls on one stream are safe.  Must not be called between step_start and step_end. */
 #define BPSX_STATIC_MAX_QUERIES 4096
 BPSX_API int bpsx_geodesic_static(bpsx_sim *sim, uint32_t scene, const float *start_xyz,
                          const uint32_t *start_ref, const float *end_xyz, const uint32_t *end_ref,

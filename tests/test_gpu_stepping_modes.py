@@ -239,7 +239,7 @@ def test_stream_ordered_stepping_with_automatic_rotation(oracle, torch_cuda, tmp
 
 def test_two_group_automatic_rotation(oracle, torch_cuda, tmp_path):
     """construct_envs' default, double_buffered=True, with automatic rotation: the two groups share
-    the loader thread, the scene choices and the side stream; a slot's swap is started by whichever
+    the loader thread and the scene choices; a slot's swap is started by whichever
     group steps next and completed by the steps of the slot's own group."""
     from bps_nav_amd import env_utils
     from oracle import bpo
