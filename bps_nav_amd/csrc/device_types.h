@@ -133,14 +133,13 @@ struct NavData {
   const float* episodes;   // [.][10]
 };
 
-// HBM slot of one A* wavefront: the node pool (LDS caches its hot part) and the open-list
-// entries beyond what LDS holds.
 // Record of the open-list operations of a search that keeps its open list sorted (see
 // geodesic_device.h): per pass one header (key = number of entries popped | number of records
 // that follow << 8, word = kOpHeader) followed by the pass's pushes and modifies in row and
-// edge order (key = total as bits, word = packed node | row of the pass << 26).  A header with kOpUnordered says that the pass's first two rows had the same
-// total: the reference expanded them in the order its heap had them in, which the replay finds
-// out; the header's low 26 bits then name row 0's node.
+// edge order (key = total as bits, word = packed node | row of the pass << 26).  A header with
+// kOpUnordered says that the pass's first two rows had the same total: the reference expanded them
+// in the order its heap had them in, which the replay finds out; the header's low 26 bits then name
+// row 0's node.
 struct OpRec {
   uint32_t key;
   uint32_t word;
@@ -149,10 +148,12 @@ constexpr uint32_t kOpHeader = 0x80000000u, kOpUnordered = 0x40000000u;
 constexpr int kOpLogCap = 8192;
 
 #ifdef __HIPCC__
+// HBM slot of one A* wavefront: the node pool (LDS caches its hot part), what LDS has no room for, and
+// the log.
 struct alignas(128) GeoSlot {
   float4 nodes[kMaxNodes];       // position and cost (dtNode, DetourNode.h:36-45; the total is their sum with the heuristic)
   uint32_t links[kMaxNodes];     // polygon index within the scene | next node of the hash chain << 16, of nodes beyond what LDS holds
-  uint2 heap_spill[kMaxNodes];   // the reference's heap between replays (total as bits, packed node)
+  uint2 heap_spill[kMaxNodes];   // the reference's heap between replays, and where it outgrows LDS (total as bits, packed node)
   OpRec oplog[kOpLogCap];
   uint16_t parents[kMaxNodes];   // per node, 1-based index of the node it was reached from, 0 for the start node: what the final walk up the path reads
 };

@@ -40,7 +40,7 @@ namespace bpsx {
 
 #ifdef BPSX_PHASE_TIMING
 // diagnostic build: cycles per phase of the sorted-list loop -> counters: 0 front of the list, 1 fetch, 2 lookup,
-// 3 costs, 4 rows that stand, 5 closing, new nodes and stores, 6 list and log; 7 counts the passes
+// 3 costs, 4 rows that stand, 5 new nodes and stores, 6 log and list; 7 counts the passes
 // (the comment that the asm statement leaves in the compiler's assembly output names the loop's
 // instantiation and the mark, for tests/measure_astar_loop_phases.py)
 #define FM(k) do { constexpr int slot_[11] = {7, 0, 1, 2, 3, 4, 5, 5, 5, 6, 6}; const unsigned long long now_ = __builtin_readcyclecounter(); \

@@ -3,8 +3,8 @@ sorted-list loop go, phase by phase.
 
 Both parts use the phase-timing diagnostic build (-DBPSX_PHASE_TIMING), whose loop carries eleven
 marks: 0 front of the list, 1 fetch of the edge records and the expanded nodes, 2 node lookup,
-3 costs, 4 rows that stand, 5 closing, 6 new nodes, 7 stores, 8 front entries leave and the log,
-9 list updates, 10 end of the pass.
+3 costs, 4 rows that stand, 5 what the pass commits, 6 new nodes, 7 stores, 8 the log and the chains
+of new nodes that share a bucket, 9 list updates, 10 end of the pass.
 
     python tests/measure_astar_loop_phases.py
         No GPU needed.  Compiles kernels.hip to assembly with the Makefile's own options and counts,
@@ -12,7 +12,7 @@ marks: 0 front of the list, 1 fetch of the edge records and the expanded nodes, 
         k_geodesic, the instructions between consecutive marks in the order the compiler laid them
         out, by class: vector ALU, scalar ALU, branch, LDS, memory, waits.  Blocks that the compiler
         moved out of line (rare cases) are counted where they lie, and a loop inside a phase (the
-        list updates, one per updated node) is counted once: the figures are those of the code,
+        list updates, a round per two updated nodes) is counted once: the figures are those of the code,
         not of its execution.
 
     make -C bps_nav_amd/csrc clean && make -C bps_nav_amd/csrc DIAG=-DBPSX_PHASE_TIMING OUT=../libbpsx_phase.so
@@ -29,8 +29,8 @@ import tempfile
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 CSRC = os.path.join(ROOT, "bps_nav_amd", "csrc")
-PHASES = ["front of the list", "fetch", "node lookup", "costs", "rows that stand", "closing", "new nodes", "stores",
-          "front leaves, log", "list updates (once)", "end of pass, loop top"]
+PHASES = ["front of the list", "fetch", "node lookup", "costs", "rows that stand", "what it commits", "new nodes", "stores",
+          "log, shared buckets", "list updates (once)", "end of pass, loop top"]
 
 
 def classify(line):
@@ -129,7 +129,7 @@ def cycles(steps):
     pops = float(c1["astar_pops"] - c0["astar_pops"])
     passes = d[7]
     names = ["front of the list (marks 0-1)", "fetch (1-2)", "node lookup (2-3)", "costs (3-4)", "rows that stand (4-5)",
-             "closing, new nodes, stores (5-8)", "front leaves, log, list updates (8-10)"]
+             "new nodes, stores (5-8)", "log, list updates (8-10)"]
     print(f"{steps} steps: {pops / steps:.0f} nodes expanded per step in {passes / steps:.0f} passes ({pops / passes:.2f} nodes per pass)")
     tot = sum(d[:7])
     for n, v in zip(names, d[:7]):
