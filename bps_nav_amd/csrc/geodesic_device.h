@@ -84,11 +84,25 @@ BPSX_DEV uint32_t wlane(uint32_t old, uint32_t v, int lane) {
   return old;
 }
 
+// lanes from .. from + n - 1 (n < 64)
+BPSX_DEV unsigned long long lane_range(int n, int from) {
+  unsigned long long r;
+  asm("s_bfm_b64 %0, %1, %2" : "=s"(r) : "s"(n), "s"(from));
+  return r;
+}
 // index of the lowest set bit, -1 for an empty mask (the instruction's own convention)
 BPSX_DEV int first_lane(unsigned long long mask) {
   int r;
   asm("s_ff1_i32_b64 %0, %1" : "=s"(r) : "s"(mask));
   return r;
+}
+// *p = (x, y) in the lanes of mask, p in LDS; called by whole wavefronts.  A store under a condition would get
+// a branch around it, which costs a wavefront more than the store.
+BPSX_DEV void lds_store_where(unsigned long long mask, uint2* p, uint32_t x, uint32_t y) {
+  typedef uint32_t Pair __attribute__((ext_vector_type(2)));
+  const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint2*)p;
+  const Pair v = {x, y};
+  asm volatile("s_mov_b64 exec, %0\n\tds_write_b64 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(at), "v"(v) : "memory");
 }
 BPSX_DEV unsigned long long without_lane(unsigned long long mask, int lane) {
   asm("s_bitset0_b64 %0, %1" : "+s"(mask) : "s"(lane));
@@ -464,7 +478,14 @@ struct GeoWave {
 // The reference's heap (dtNodeQueue, DetourNode.cpp:150-200), needed when the sorted list cannot say
 // what comes first (a tie) or cannot hold what is open: position q (root = 1) in entry q of an array
 // in LDS, over the conflict marks (but the first two) and the window, or in the wavefront's slot.  All lanes
-// work on one operation: a pop takes one round of accesses per five levels, a push one.
+// work on one operation: a push takes one round of accesses, a pop one up to 256 entries (searches
+// over mazes keep 23 on average, over cluttered plans 70), beyond that one per five levels.  Bound by
+// those rounds and the instructions of a lone wavefront, five cycles each; a replay is a chain of them.
+// (With each pop in rounds of six levels, which combined the siblings' comparisons on the scalar unit
+// and brought the deepest entry that moves back from there, with branches around the stores, a replay
+// took 0.4 us per node; now 0.2.  1000 pairs over a maze, whose longest search of 2002 nodes replays
+// them all, 1969 -> 1604 us; steps of 4096 agents over cluttered plans 2528 -> 2176, of 16384 over
+// mazes 1141 -> 1026.)
 // (A heap in registers, entry q in lane q mod 64, held 127 entries; one search in seven hundred over
 // a cluttered plan of 20k polygons ties with a longer list or outgrows the sorted list, and ran
 // again from its start with a heap walked level by level in HBM: 6.6 ms, against 1.5 ms for the
@@ -474,32 +495,55 @@ static_assert(kLinksLds % 4 == 0 && offsetof(GeoLds, w_node) == offsetof(GeoLds,
               "the marks are accessed as 16 bytes, and the heap lies over the marks and the window");
 // (383 entries, 639 of a whole block's LDS, 353 next to a whole node pool)
 static_assert(kHeapLds >= 64 * OpenList::kPairs + 2 * kRows * kNvp, "a heap with as many entries as the sorted list must fit");
-struct RefHeap {
+template <bool Lds> struct RefHeap {
   uint2* h;    // total bits, packed node
   int size, lane;
-  uint32_t anc0, anc1;   // as bits, the lane and its ancestors below the root of a subtree with node l in lane l
-  BPSX_DEV RefHeap(uint2* entries, int n, int lane_) : h(entries), size(n), lane(lane_) {
+  uint32_t anc0, anc1;   // as bits, the entries of 64 at and above entry `lane`, but for the root
+  uint32_t above_bit;    // the bit lane >> 1
+  BPSX_DEV RefHeap(uint2* entries, int n, int lane_) : h(entries), size(uniform_i(n)), lane(lane_) {
     unsigned long long a = 0;
 #pragma unroll
     for (int k = 0; k < 5; ++k)
       if ((lane >> k) >= 2) a |= 1ull << (lane >> k);
     anc0 = (uint32_t)a; anc1 = (uint32_t)(a >> 32);
+    above_bit = 1u << (lane >> 1);
   }
-  // the entry (t, n), on its way up from position q: lane k looks at the ancestor k levels up; those
-  // with a greater total, a run from q upwards, move down one level each
+  // h[at] = e in the lanes of mask (in LDS without a branch around it)
+  BPSX_DEV void put(unsigned long long mask, uint32_t at, uint32_t x, uint32_t y) const {
+    if constexpr (Lds) {
+      lds_store_where(mask, &h[at], x, y);
+    } else {
+      if (in_mask(mask)) h[at] = make_uint2(x, y);
+    }
+  }
+  // The entry (t, n), on its way up from position q: lane k has position q >> k and looks at the entry
+  // there and the one above.  Those with a greater total, a run from q upwards, move down one level each.
   BPSX_DEV void bubble_up(int q, uint32_t t, uint32_t n) {
-    const int up = q >> (lane & 31);
-    const bool on = lane >= 1 && lane < 31 && up >= 1;
-    const uint2 e = h[on ? up : 1];
+    const unsigned long long path = lane_range(32 - __builtin_clz((uint32_t)q), 0);   // as many as q has bits
+    const uint32_t at = (uint32_t)q >> (lane & 31);
+    const uint32_t own = h[at].x;
+    const uint2 above = h[at >> 1];
     wave_sync();
-    const unsigned long long greater = lanes_where(on && e.x > t) >> 1;
-    const int m = __builtin_ctzll(~greater);
-    if (on && lane <= m) h[q >> (lane - 1)] = e;
-    if (lane == 0) h[q >> m] = make_uint2(t, n);
+    const unsigned long long leaves = (lanes_where(own > t) | 1ull) & path;
+    const unsigned long long falls = lanes_where(above.x > t) & (path >> 1);
+    put(leaves, at, in_mask(falls) ? above.x : t, in_mask(falls) ? above.y : n);
     wave_sync();
   }
   // where node n's entry is, 0 if it has none
+  template <int K> BPSX_DEV int position(uint32_t n) const {
+    unsigned long long m[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) m[k] = lanes_where(h[64 * k + lane].y == n);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      m[k] &= upto(size - 64 * k) & (k ? ~0ull : ~1ull);
+      if (m[k]) return 64 * k + first_lane(m[k]);
+    }
+    return 0;
+  }
   BPSX_DEV int position(uint32_t n) const {
+    if (size < 64) return position<1>(n);
+    if (size < 256) return position<4>(n);
     for (int base = 1; base <= size; base += 64) {
       const int i = base + lane;
       const unsigned long long m = lanes_where(h[i <= size ? i : size].y == n);
@@ -507,6 +551,8 @@ struct RefHeap {
     }
     return 0;
   }
+  // lanes 0 .. i, none below 0
+  static BPSX_DEV unsigned long long upto(int i) { return i < 0 ? 0ull : i >= 63 ? ~0ull : (2ull << i) - 1ull; }
   // a node that has an entry takes a smaller total (dtNodeQueue::modify), one without gets one (push)
   BPSX_DEV void update(bool mayHaveEntry, uint32_t t, uint32_t n) {
     int q = mayHaveEntry ? position(n) : 0;
@@ -516,7 +562,65 @@ struct RefHeap {
   // The root leaves: the hole moves to a leaf along the smaller children (the left one of two
   // equal), then the former last entry rises from there.  Totals never decrease along that route,
   // so the entry lands above the first route element greater than it and nothing below moves.
+  //
+  // With up to 64 K entries, entry 64 k + l in lane l: an entry is on the route when neither it nor one above
+  // it is the greater of its pair of siblings, and whether it moves up, and whether the last entry
+  // comes to lie above it or in a leaf's place, each lane can tell from its own entry, the one
+  // above it and the last.  So a pop is one round of reads and two masked stores per 64 entries.
+  template <int K> BPSX_DEV void pop_at_once() {   // K = 1, 2, 4; more than 32 K entries if K > 1
+    const int s = size;
+    uint2 e[K], last = h[s];
+    uint32_t above[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) { e[k] = h[64 * k + lane]; above[k] = h[(64 * k + lane) >> 1].x; }
+#pragma unroll
+    for (int k = 0; k < K; ++k) asm("" : "+v"(e[k].x), "+v"(e[k].y), "+v"(above[k]), "+v"(last.x));   // all reads go out before the first is used
+    wave_sync();
+    // of the entries of each 64 lanes, those before the last, and those that have none below them
+    unsigned long long there[K], leaf[K];
+    const int leaves = (s + 1) >> 1;
+    if constexpr (K == 1) {
+      there[0] = lane_range(s - 1, 1);
+      leaf[0] = ~0ull << leaves;
+    } else if constexpr (K == 2) {
+      there[0] = ~1ull;
+      there[1] = ~0ull >> (128 - s);
+      leaf[0] = (~0ull << (leaves - 1)) << 1;
+      leaf[1] = ~0ull;
+    } else {
+      there[0] = ~1ull;
+      there[1] = ~0ull;
+      there[2] = s >= 192 ? ~0ull : ~0ull >> (192 - s);
+      there[3] = s > 192 ? ~0ull >> (256 - s) : 0ull;
+      leaf[0] = 0;
+      leaf[1] = (~0ull << (leaves - 65)) << 1;
+      leaf[2] = leaf[3] = ~0ull;
+    }
+    unsigned long long greater[K], on[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      // of two equal siblings the right one is the greater; a place without an entry is greater than all
+      const uint32_t key = in_mask(there[k]) ? (e[k].x << 1) | (uint32_t)(lane & 1) : 0xffffffffu;
+      const uint32_t sibling = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)key, 0xb1 /* quad_perm:[1,0,3,2] */, 0xf, 0xf, true);
+      greater[k] = lanes_where(key > sibling);
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k == 0) on[k] = lanes_where(((anc0 & (uint32_t)greater[0]) | (anc1 & (uint32_t)(greater[0] >> 32))) == 0) & there[k];
+      // the one above lies in the second half of the first 64 entries, and in the first and second of the next
+      else on[k] = lanes_where((above_bit & (uint32_t)(k == 2 ? on[k / 2] : on[k / 2] >> 32)) != 0) & there[k] & ~greater[k];
+      const unsigned long long rises = lanes_where(e[k].x <= last.x);
+      const uint32_t x = in_mask(rises) ? e[k].x : last.x, y = in_mask(rises) ? e[k].y : last.y;
+      put(on[k] & lanes_where(above[k] <= last.x) & (k ? ~0ull : ~3ull), (uint32_t)(64 * k + lane) >> 1, x, y);
+      if (K < 4 || k > 0) put(on[k] & rises & leaf[k], (uint32_t)(64 * k + lane), last.x, last.y);
+    }
+    size--;
+    wave_sync();
+  }
   BPSX_DEV void pop() {
+    if (size <= 64) return pop_at_once<1>();
+    if (size <= 128) return pop_at_once<2>();
+    if (size <= 256) return pop_at_once<4>();
     const int depth = 31 - __clz(lane | (lane == 0));
     uint32_t lt = 0, ln = 0;
     int root = 1, at = 1;
@@ -536,14 +640,14 @@ struct RefHeap {
       const bool take = there && e.x <= lt && ((anc0 & (uint32_t)greater) | (anc1 & (uint32_t)(greater >> 32))) == 0;
       const int q = 63 - __builtin_clzll(lanes_where(take && lane > 1) | 2ull);   // the deepest that moves up
       wave_sync();
-      if (take && lane > 1) h[pos >> 1] = e;
+      put(lanes_where(take && lane > 1), (uint32_t)pos >> 1, e.x, e.y);
       wave_sync();
       const int m = 31 - __builtin_clz((uint32_t)q);
       at = (root << m) | (q & ((1 << m) - 1));
       if (m < 5 || 2 * at >= size) break;
       root = at;
     }
-    if (lane == 0) h[at] = make_uint2(lt, ln);   // of a heap of one entry: that entry once more, beyond the end
+    put(1ull, (uint32_t)at, lt, ln);   // of a heap of one entry: that entry once more, beyond the end
     size--;
     wave_sync();
   }
@@ -557,7 +661,7 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
   const int lane = g.lane;
   const OpRec* log = g.ws->oplog;
   uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
-  RefHeap rh(g.L->heap(), st.replaySize, lane);
+  RefHeap<true> rh(g.L->heap(), st.replaySize, lane);
   // the pass that ended here has left its marks: the first of them, which ends the hash chains, lies
   // under the heap's unused entry 0 and has to stand while a search goes on with the heap
   g.clear_marks();
@@ -569,8 +673,8 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
   uint32_t rk = 0, rw = 0;
   auto fetch = [&](int from) {
     base = from;
-    rk = 0; rw = 0;
-    if (base + lane < st.logEnd) { const OpRec r = log[base + lane]; rk = r.key; rw = r.word; }
+    const OpRec r = log[base + lane < st.logEnd ? base + lane : base];   // what lies behind the end is not looked at
+    rk = r.key; rw = r.word;
   };
   for (int pos = st.synced; pos < st.logEnd;) {
     // a fetch is a round trip to HBM: one only when the pass at hand is not all there
@@ -581,14 +685,14 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
     const int c = (int)(hk & 0xffu), nrec = (int)(hk >> 8);
     // rows in the reference's order: the first two swap when the heap has row 1's node on top
     const bool swap = (hw & kOpUnordered) && (uint32_t)uniform_i((int)rh.h[1].y) != (hw & 0x3ffffffu);
-    const bool mine = lane > h && lane <= h + nrec;
-    const int myRow = (int)((rw >> 26) & 7u);
+    const unsigned long long mine = lane_range(nrec, h + 1);
+    const uint32_t myRow = (rw >> 26) & 7u;
     // the pass's new nodes are those whose index had not been given out before it
-    const unsigned long long fresh = lanes_where(mine && (int)(rw & 0x7ffu) >= seen);
+    const unsigned long long fresh = lanes_where((int)(rw & 0x7ffu) >= seen) & mine;
     for (int i = 0; i < c; ++i) {
       const int row = (swap && i < 2) ? 1 - i : i;
       rh.pop();
-      unsigned long long m = lanes_where(mine && myRow == row);
+      unsigned long long m = lanes_where(myRow == (uint32_t)row) & mine;
       while (m) {
         const int j = first_lane(m);
         m = without_lane(m, j);
@@ -630,7 +734,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
   const int lane = g.lane;
   GeoLds* L = g.L;
   const float H_SCALE = 0.999f;
-  RefHeap rh(Lds ? L->heap() : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
+  RefHeap<Lds> rh(Lds ? L->heap() : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
   for (;;) {
     st.replaySize = rh.size;
     if (rh.size <= 0) return kAstarEmpty;

@@ -39,3 +39,26 @@ def test_equal_totals_match_oracle(oracle, n, whole_block):
     assert (c["geo_long_path"] == n) == whole_block
     cpu.close()
     gpu.close()
+
+
+# rooms whose open lists come to up to 67, 140, 218 and 354 entries: the reference's heap grows and shrinks through
+# the sizes up to which a pop is one round of accesses to 64, 128 and 256 entries, and beyond
+@pytest.mark.parametrize("edge,far", [(6.0, 3e5), (8.0, 1e7), (11.0, 1e7), (8.0, 1e10)])
+def test_replayed_heaps_of_all_sizes_match_oracle(oracle, edge, far):
+    n = 64
+    from bps_nav_amd.bps_sim import nav_only
+    from oracle import bpo
+    print(f"case: a room of {edge} m, end points {far} m away", flush=True)
+    blob = scenes.gen_scene(scenes.BOX_ROOM, 5, cell=5, size_x=edge, size_z=edge, num_boxes=0)
+    cpu, gpu = bpo.Nav(oracle, blob), nav_only([blob])
+    pts = scenes.sample_points(blob, 3, 2 * n)
+    x, r = cpu.snap(pts)
+    a, ar, b, br = x[:n], r[:n], x[n:].copy(), r[n:]
+    b[::2, 0] += np.float32(far)
+    want = cpu.geodesic(a, ar, b, br)
+    got = gpu.geodesic(0, a, ar, b, br)
+    c = gpu.counters()
+    assert c["geo_tie_replays"] + c["geo_exact_runs"] > n // 2
+    assert np.array_equal(common.bits(want), common.bits(got))
+    cpu.close()
+    gpu.close()
