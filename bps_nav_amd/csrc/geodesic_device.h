@@ -96,13 +96,47 @@ BPSX_DEV int first_lane(unsigned long long mask) {
   asm("s_ff1_i32_b64 %0, %1" : "=s"(r) : "s"(mask));
   return r;
 }
-// *p = (x, y) in the lanes of mask, p in LDS; called by whole wavefronts.  A store under a condition would get
-// a branch around it, which costs a wavefront more than the store.
+// Stores in the lanes of a mask, called by whole wavefronts (all lanes active before and after).  A store under
+// a condition would get a branch around it, which costs a wavefront more than the store, and a loop
+// with such a branch in it is rebuilt by the compiler as if all its branches were the lanes' own: every
+// early way out then goes through copies of the loop's state and tests of flags.
+typedef float Float4 __attribute__((ext_vector_type(4)));
+BPSX_DEV uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
 BPSX_DEV void lds_store_where(unsigned long long mask, uint2* p, uint32_t x, uint32_t y) {
-  typedef uint32_t Pair __attribute__((ext_vector_type(2)));
-  const uint32_t at = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint2*)p;
-  const Pair v = {x, y};
-  asm volatile("s_mov_b64 exec, %0\n\tds_write_b64 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(at), "v"(v) : "memory");
+  const unsigned long long v = ((unsigned long long)y << 32) | x;
+  asm volatile("s_mov_b64 exec, %0\n\tds_write_b64 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(v) : "memory");
+}
+BPSX_DEV void lds_store_where(unsigned long long mask, float4* p, float4 f) {
+  const Float4 v = {f.x, f.y, f.z, f.w};
+  asm volatile("s_mov_b64 exec, %0\n\tds_write_b128 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(v) : "memory");
+}
+BPSX_DEV void lds_store_where(unsigned long long mask, uint32_t* p, uint32_t x) {
+  asm volatile("s_mov_b64 exec, %0\n\tds_write_b32 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x) : "memory");
+}
+BPSX_DEV void lds_store_where(unsigned long long mask, uint16_t* p, uint32_t x) {
+  asm volatile("s_mov_b64 exec, %0\n\tds_write_b16 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x) : "memory");
+}
+BPSX_DEV void lds_min_where(unsigned long long mask, uint32_t* p, uint32_t x) {
+  asm volatile("s_mov_b64 exec, %0\n\tds_min_u32 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x) : "memory");
+}
+// base[offset bytes] = v, base the same for all lanes
+BPSX_DEV void store_where(unsigned long long mask, void* base, uint32_t offset, uint32_t v) {
+  asm volatile("s_mov_b64 exec, %0\n\tglobal_store_dword %1, %2, %3\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(offset), "v"(v), "s"(base) : "memory");
+}
+BPSX_DEV void store_where(unsigned long long mask, void* base, uint32_t offset, uint32_t x, uint32_t y) {
+  const unsigned long long v = ((unsigned long long)y << 32) | x;
+  asm volatile("s_mov_b64 exec, %0\n\tglobal_store_dwordx2 %1, %2, %3\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(offset), "v"(v), "s"(base) : "memory");
+}
+// old with lane Lane replaced by v (uniform)
+template <int Lane> BPSX_DEV uint32_t wlane_at(uint32_t old, uint32_t v) {
+  asm("v_writelane_b32 %0, %1, %2" : "+v"(old) : "s"(__builtin_amdgcn_readfirstlane((int)v)), "n"(Lane));
+  return old;
+}
+// index of the lowest bit that is not set, -1 if all are
+BPSX_DEV int first_other_lane(unsigned long long mask) {
+  int r;
+  asm("s_ff0_i32_b64 %0, %1" : "=s"(r) : "s"(mask));
+  return r;
 }
 BPSX_DEV unsigned long long without_lane(unsigned long long mask, int lane) {
   asm("s_bitset0_b64 %0, %1" : "+s"(mask) : "s"(lane));
@@ -126,8 +160,9 @@ template <int Ctrl, int RowMask> BPSX_DEV uint32_t umin_dpp(uint32_t v) {
 //     (With a NaN two nodes would update each other for ever: there is none, see AEdge.)
 // Without both a pass is some 25 of 630 instructions and three LDS accesses shorter: 1.286 -> 1.229 ms
 // of k_geodesic at 16384 agents over mazes, 5 % off the longest of 64 searches alone on the GPU.
-constexpr uint32_t kChainEnd = 0xffffu;
-static_assert(kMaxNodes <= (int)kChainEnd, "node indices must stay below the chain end marker");
+// A chain is linked by the byte offsets of the nodes' words (GeoWave::offset_of), so that a step along it is
+// one access to LDS and three instructions.
+constexpr uint32_t kNoPoly = 0xffffu;   // what the word at a chain's end has for a polygon
 BPSX_DEV uint32_t link_id(uint32_t l) { return l & 0xffffu; }
 BPSX_DEV uint32_t link_next(uint32_t l) { return l >> 16; }
 BPSX_DEV uint32_t make_link(uint32_t id, uint32_t next) { return id | (next << 16); }
@@ -153,7 +188,7 @@ struct OpenList {
   uint32_t t[kPairs], n[kPairs];
   int size;
   static constexpr uint32_t kEmpty = kEmptyKey;
-  static constexpr uint32_t kNone = 0xffffffffu;    // no packed node looks like this (26 bits)
+  static constexpr uint32_t kNone = 0;   // the start node, which never enters the list again: what is read by it is there
   BPSX_DEV void init(int lane, uint32_t total, uint32_t node) { t[0] = lane ? kEmpty : total; n[0] = lane ? kNone : node; size = 1; }   // further pairs are cleared when the list grows into them
   BPSX_DEV void clear_pair(int k) { t[k] = kEmpty; n[k] = kNone; }
   // lane L takes v of lane L + 1, lane 63 keeps `last`
@@ -179,13 +214,14 @@ struct OpenList {
   // then took 1.229 ms instead of 1.207 at 16384 agents over mazes, 3.11 instead of 2.59 at 4096
   // over cluttered plans, whose lists fill two to four pairs, 1.16 instead of 0.99 at 1024 over room
   // plans, where a launch lasts as long as its longest search alone.)
-  // Returns entry `row` of the new list (anything where there is none).
-  template <int P> BPSX_DEV uint32_t merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
-                                           uint32_t packed, int lane, int row) {
+  // Returns the node of entry `row` of the new list and the total of the one behind it (of kNone and kEmpty
+  // where there is none).
+  template <int P> BPSX_DEV uint2 merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
+                                        uint32_t packed, int lane, int row) {
     unsigned long long dead[P];
 #pragma unroll
     for (int k = 0; k < P; ++k) dead[k] = 0;
-    dead[0] = (1ull << c) - 1ull;
+    dead[0] = lane_range(c, 0);
     while (known) {
       const int src = first_lane(known);
       known = without_lane(known, src);
@@ -203,8 +239,8 @@ struct OpenList {
     size += __popcll(upd) - (64 * P - live);
     uint32_t upTo = 0, before = 0;
     const unsigned long long key = ((unsigned long long)tb << 32) | (uint32_t)lane;   // equal totals in lane order
-    const bool enters = in_mask(upd);
-    uint32_t front;
+    const unsigned long long enters = upd;
+    uint2 front;
     // Two at a time, so that one's lane moves fill the other's waits.  With an odd number the last
     // round's second is lane 63 (first_lane of an empty mask, taken modulo 64): no edge's lane, its
     // total is above all keys and counts nowhere.
@@ -229,40 +265,41 @@ struct OpenList {
       upTo = wlane(upTo, (uint32_t)lb, sb);
     }
     const uint32_t place = upTo + before;
-    if (P == 1) {
+    if constexpr (P == 1) {
       // places up to 63 + 48 fit the buffer: no lane needs to be left out, those that leave go to its end
       buf[pick(dead[0], 127u, pos[0])] = make_uint2(t[0], n[0]);
-      if (enters) buf[place] = make_uint2(tb, packed);
+      lds_store_where(enters, &buf[place], tb, packed);
       wave_sync();
       const uint2 e = buf[lane];
-      front = buf[row].y;
+      front = make_uint2(buf[row].y, buf[row + 1].x);
       t[0] = lane < size ? e.x : kEmpty;
       n[0] = lane < size ? e.y : kNone;
     } else {
-      uint32_t a[P];
-#pragma unroll
-      for (int k = 0; k < P; ++k) a[k] = pick(dead[k], kEmpty, t[k]);
+      unsigned long long moves[P];
+      static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA { constexpr int k = decltype(K)::value; moves[k] = lanes_where(t[k] != kEmpty) & ~dead[k]; });
       uint32_t nt[P], nn[P];
-#pragma unroll
-      for (int half = 0; half < P / 2; ++half) {
-#pragma unroll
-        for (int k = 0; k < P; ++k)
-          if (a[k] != kEmpty && (pos[k] >> 7) == (uint32_t)half) buf[pos[k] & 127u] = make_uint2(t[k], n[k]);
-        if (enters && (place >> 7) == (uint32_t)half) buf[place & 127u] = make_uint2(tb, packed);
+      static_for<0, P / 2>([&](auto H) BPSX_INLINE_LAMBDA {
+        constexpr int half = decltype(H)::value;
+        static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA {
+          constexpr int k = decltype(K)::value;
+          lds_store_where(moves[k] & lanes_where((pos[k] >> 7) == (uint32_t)half), &buf[pos[k] & 127u], t[k], n[k]);
+        });
+        lds_store_where(enters & lanes_where((place >> 7) == (uint32_t)half), &buf[place & 127u], tb, packed);
         wave_sync();
-        if (half == 0) front = buf[row].y;
-#pragma unroll
-        for (int k = 2 * half; k < 2 * half + 2; ++k) {
+        if (half == 0) front = make_uint2(buf[row].y, buf[row + 1].x);
+        static_for<0, 2>([&](auto K) BPSX_INLINE_LAMBDA {
+          constexpr int k = 2 * half + decltype(K)::value;
           const uint2 e = buf[(k & 1) * 64 + lane];
           nt[k] = 64 * k + lane < size ? e.x : kEmpty;
           nn[k] = 64 * k + lane < size ? e.y : kNone;
-        }
+        });
         wave_sync();
-      }
-#pragma unroll
-      for (int k = 0; k < P; ++k) { t[k] = nt[k]; n[k] = nn[k]; }
+      });
+      static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA { constexpr int k = decltype(K)::value; t[k] = nt[k]; n[k] = nn[k]; });
     }
     wave_sync();
+    front.x = row < size ? front.x : kNone;
+    front.y = row + 1 < size ? front.y : kEmpty;
     return front;
   }
 };
@@ -278,28 +315,26 @@ struct AstarState {
   uint32_t replayRoot;   // packed node of the entry at its root after a replay
 };
 
-enum AstarExit { kAstarEmpty = 0, kAstarGoal = 1, kAstarGrowLinks = 2, kAstarGrowHeap = 3, kAstarTie = 4, kAstarLogFull = 5 };
+enum AstarExit { kAstarOn = -1, kAstarEmpty = 0, kAstarGoal = 1, kAstarGrowLinks = 2, kAstarGrowHeap = 3, kAstarTie = 4, kAstarLogFull = 5 };
 
-// Two correctly rounded square roots, the values sqrtf returns on the host: the hardware estimate is
-// within one unit in the last place, and the residuals of its two neighbours say which of the
-// three is the rounded root.  Same scheme as the compiler's own expansion of sqrtf, minus its
-// rescaling of arguments below 2^-96 (needed there for the residuals not to underflow): the
-// arguments here are squared distances, zero or far above that; a wavefront that meets one in
-// between takes the library routine.  One test of the arguments' range for both.
+// Two correctly rounded square roots, the values sqrtf returns on the host, of arguments that are zero or
+// at least 2^-96 and finite, as squared distances between points of a mesh are; a wavefront that meets
+// another (or zero, which this form would make NaN) takes the library routine.  One test of the
+// arguments' range for both.  One step from the reciprocal root's estimate, with the residual exact
+// through a fused multiply-add: compared with the root of the same number in 64 bits, rounded, it
+// is right for every float from 2^-96 up on this hardware.  (The estimate of the root and the residuals of its two
+// neighbours, which of the three it is, are nine instructions instead of five.)
 BPSX_DEV void sqrt_exact2(float x, float y, float* rx, float* ry) {
-  const uint32_t xb = __float_as_uint(x), yb = __float_as_uint(y);
-  if (__builtin_expect(lanes_where(xb - 1u < 0x0f800000u - 1u || yb - 1u < 0x0f800000u - 1u) != 0, 0)) {
-    *rx = sqrtf(x); *ry = sqrtf(y);   // 0 < argument < 2^-96 in some lane: never in practice
+  const uint32_t lo = 0x0f800000u, span = 0x7f800000u - lo;
+  const uint32_t xr = __float_as_uint(x) - lo, yr = __float_as_uint(y) - lo;
+  if (__builtin_expect(lanes_where((xr > yr ? xr : yr) >= span) != 0, 0)) {
+    *rx = sqrtf(x); *ry = sqrtf(y);
     return;
   }
-  const float s = __builtin_amdgcn_sqrtf(x), t = __builtin_amdgcn_sqrtf(y);
-  const float sd = __uint_as_float(__float_as_uint(s) - 1u), su = __uint_as_float(__float_as_uint(s) + 1u);
-  const float td = __uint_as_float(__float_as_uint(t) - 1u), tu = __uint_as_float(__float_as_uint(t) + 1u);
-  float r = fmaf(-sd, s, x) <= 0.0f ? sd : s;
-  r = fmaf(-su, s, x) > 0.0f ? su : r;
-  float q = fmaf(-td, t, y) <= 0.0f ? td : t;
-  q = fmaf(-tu, t, y) > 0.0f ? tu : q;
-  *rx = r; *ry = q;
+  const float px = __builtin_amdgcn_rsqf(x), py = __builtin_amdgcn_rsqf(y);
+  const float gx = x * px, gy = y * py;
+  *rx = fmaf(fmaf(-gx, gx, x), 0.5f * px, gx);
+  *ry = fmaf(fmaf(-gy, gy, y), 0.5f * py, gy);
 }
 
 BPSX_DEV float tri_area2d(const float* a, const float* b, const float* c) {
@@ -338,6 +373,10 @@ constexpr int kWindow = BPSX_WINDOW;        // most recent nodes whose position 
 #define BPSX_HASH 512
 #endif
 constexpr int kHashSize = BPSX_HASH;        // buckets of the node pool's hash table
+// Where all chains end: the word behind the links in LDS, which names no polygon and itself as the next.
+constexpr uint32_t kChainEnd = 4u * (uint32_t)kLinksLds;
+constexpr uint32_t kEndWord = kNoPoly | (kChainEnd << 16);
+static_assert(4 * (kMaxNodes + 1) <= 0xffff, "offsets of links have 16 bits");
 constexpr bool kAllLds = kWindow >= kMaxNodes;   // every node is kept in LDS, and none in HBM
 static_assert(!kAllLds || kLinksLds >= kMaxNodes, "a pool in LDS has its links there too");
 #ifndef BPSX_TAG_SLOTS
@@ -355,10 +394,10 @@ static_assert((kWindow & (kWindow - 1)) == 0 && kWindow >= 2 * kNvp, "window mus
 // LDS of one wavefront.
 struct GeoLds {
   uint16_t first[kHashSize];
-  // Node links: polygon index | next node of the hash chain << 16.  Behind them the marks of which row of
-  // a pass updates a polygon first (see astar_fast), all ones between passes and while chains are
-  // walked: the first of them is the word that ends every chain there.  A pass's open list moves
-  // to its new order over the marks.
+  // Node links: polygon index | offset of the next node's link in the hash chain << 16.  Behind them the
+  // marks of which row of a pass updates a polygon first (see astar_fast), all kEndWord between passes
+  // and while chains are walked: the first of them is the word that ends every chain.  A pass's
+  // open list moves to its new order over the marks.
   alignas(16) uint32_t n_link[kLinksLds + kTagSlots];
   alignas(16) float4 w_node[kWindow];   // position, cost
   BPSX_DEV uint32_t* marks() { return n_link + kLinksLds; }
@@ -402,6 +441,14 @@ struct GeoWave {
   uint32_t pairTies;                 // passes that took two nodes of equal total in one go
 
   // ---------------------------------------------------------------- node pool
+  // offset of node i's link: that of the links in LDS, beyond them that of the slot's shifted past kChainEnd
+  template <bool S> static BPSX_DEV uint32_t offset_of(uint32_t i) {
+    return !S || kLinksLds >= kMaxNodes ? 4u * i : 4u * (i + (i >= (uint32_t)kLinksLds ? 1u : 0u));
+  }
+  template <bool S> static BPSX_DEV int node_at(uint32_t offset) {
+    return (int)(!S || kLinksLds >= kMaxNodes ? offset >> 2 : (offset >> 2) - (offset > kChainEnd ? 1u : 0u));
+  }
+  // where node i's link lies
   template <bool S> BPSX_DEV uint32_t link(int i) const {
     if (!S || kLinksLds >= kMaxNodes || i < kLinksLds) return L->n_link[i];
     BPSX_KEEP_APART();
@@ -409,9 +456,14 @@ struct GeoWave {
     BPSX_KEEP_APART();
     return v;
   }
-  template <bool S> BPSX_DEV void set_link(int i, uint32_t v) const {
-    if (!S || kLinksLds >= kMaxNodes || i < kLinksLds) L->n_link[i] = v;
-    else { BPSX_KEEP_APART(); ws->links[i] = v; BPSX_KEEP_APART(); }
+  template <bool S> BPSX_DEV void set_links(unsigned long long mask, int i, uint32_t v) const {
+    if (!S || kLinksLds >= kMaxNodes) {
+      lds_store_where(mask, &L->n_link[i], v);
+    } else {
+      const unsigned long long near = lanes_where(i < kLinksLds);
+      lds_store_where(mask & near, &L->n_link[i], v);
+      store_where(mask & ~near, ws->links, (uint32_t)i * 4u, v);
+    }
   }
   // node i still has its position and cost in LDS
   BPSX_DEV bool in_window(int i) const { return kAllLds || i >= nodeCount - kWindow; }
@@ -423,13 +475,15 @@ struct GeoWave {
     return ws->nodes[i];
 #endif
   }
-  BPSX_DEV void keep_node(int i, float4 n, int parent) const {
+  // node i and its parent index, in the lanes of mask
+  BPSX_DEV void keep_node(unsigned long long mask, int i, float4 n, uint32_t parent) const {
+    const Float4 v = {n.x, n.y, n.z, n.w};
 #if BPSX_WINDOW >= 2048
-    L->w_node[i] = n;
-    L->parents[i] = (uint16_t)parent;
+    asm volatile("s_mov_b64 exec, %0\n\tds_write_b128 %1, %2\n\tds_write_b16 %3, %4\n\ts_mov_b64 exec, -1"
+                 :: "s"(mask), "v"(lds_address(&L->w_node[i])), "v"(v), "v"(lds_address(&L->parents[i])), "v"(parent) : "memory");
 #else
-    *reinterpret_cast<float4*>(reinterpret_cast<char*>(ws->nodes) + (uint32_t)i * (uint32_t)sizeof(float4)) = n;
-    *reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(ws->parents) + (uint32_t)i * 2u) = (uint16_t)parent;
+    asm volatile("s_mov_b64 exec, %0\n\tglobal_store_dwordx4 %1, %2, %3\n\tglobal_store_short %4, %5, %6\n\ts_mov_b64 exec, -1"
+                 :: "s"(mask), "v"((uint32_t)i * (uint32_t)sizeof(float4)), "v"(v), "s"(ws->nodes), "v"((uint32_t)i * 2u), "v"(parent), "s"(ws->parents) : "memory");
 #endif
   }
   // the multiply as the full-rate 24-bit instruction (polygon indices have 15 bits)
@@ -440,7 +494,7 @@ struct GeoWave {
   }
   BPSX_DEV void clear_marks() {
     static_assert(kTagSlots == 256, "one 16-byte store per lane");
-    reinterpret_cast<uint4*>(L->marks())[lane] = make_uint4(0xffffffffu, 0xffffffffu, 0xffffffffu, 0xffffffffu);
+    reinterpret_cast<uint4*>(L->marks())[lane] = make_uint4(kEndWord, kEndWord, kEndWord, kEndWord);
   }
   BPSX_DEV void clear() {
     for (int i = lane; i < kHashSize; i += 64) L->first[i] = (uint16_t)kChainEnd;
@@ -448,29 +502,34 @@ struct GeoWave {
     nodeCount = 0;
     wave_sync();
   }
-  // Node index of polygon ip, or -1; *head receives the bucket's first node (what a new node of
-  // this bucket links to).  Called by all lanes (idle ones with an ip that no polygon has): the
-  // chains are walked in step, one LDS access per lane and round, until every lane has hit or run
-  // out.  Where all links are in LDS a lane that is done goes on reading the word behind them.
-  template <bool S> BPSX_DEV int find(bool valid, uint32_t ip, uint32_t bucket, uint32_t* head) const {
+  // Offset of polygon ip's node (offset_of), kChainEnd if it has none; *head receives that of the bucket's first
+  // node (what a new node of this bucket links to).  Called by all lanes (those without a polygon with
+  // valid == false): the chains are walked in step, one LDS access per lane and round, until every lane
+  // has hit or run out, which reads the word at the chains' end again.
+  template <bool S> BPSX_DEV uint32_t find(unsigned long long valid, uint32_t ip, uint32_t bucket, uint32_t* head) const {
     uint32_t cur = L->first[bucket];
-    cur = valid ? cur : kChainEnd;
+    cur = in_mask(valid) ? cur : kChainEnd;
     *head = cur;
-    int found = -1;
-    while (lanes_where(cur != kChainEnd)) {
+    uint32_t found = kChainEnd;
+    const char* links = reinterpret_cast<const char*>(L->n_link);
+    do {
+      uint32_t l;
       if (!S || kLinksLds >= kMaxNodes) {
-        const uint32_t l = L->n_link[cur < (uint32_t)kLinksLds ? cur : (uint32_t)kLinksLds];
-        const bool hit = link_id(l) == ip;
-        found = hit ? (int)cur : found;
-        cur = hit ? kChainEnd : link_next(l);
+        l = *reinterpret_cast<const uint32_t*>(links + cur);
       } else {
-        const bool live = cur != kChainEnd;
-        const uint32_t l = link<S>(live ? (int)cur : 0);
-        const bool hit = live && link_id(l) == ip;
-        found = hit ? (int)cur : found;
-        cur = (live && !hit) ? link_next(l) : kChainEnd;
+        l = *reinterpret_cast<const uint32_t*>(links + (cur < kChainEnd ? cur : kChainEnd));
+        const unsigned long long far = lanes_where(cur > kChainEnd);
+        if (far) {
+          BPSX_KEEP_APART();
+          const uint32_t f = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(ws->links) + (in_mask(far) ? cur - 4u : 0u));
+          BPSX_KEEP_APART();
+          l = in_mask(far) ? f : l;
+        }
       }
-    }
+      const bool hit = link_id(l) == ip;
+      found = hit ? cur : found;
+      cur = hit ? kChainEnd : link_next(l);
+    } while (lanes_where(cur != kChainEnd));
     return found;
   }
 };
@@ -668,24 +727,28 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
   wave_sync();
   for (int i = lane + 1; i <= rh.size; i += 64) rh.h[i] = kept[i];
   wave_sync();
-  int base = -64;              // record held by lane 0
+  int base = st.synced;        // record held by lane 0
   int seen = st.replayNodes;   // nodes created so far
   uint32_t rk = 0, rw = 0;
+  unsigned long long headers = 0;
   auto fetch = [&](int from) {
     base = from;
     const OpRec r = log[base + lane < st.logEnd ? base + lane : base];   // what lies behind the end is not looked at
     rk = r.key; rw = r.word;
+    headers = lanes_where((rw & kOpHeader) != 0);
   };
+  if (base < st.logEnd) fetch(base);
   for (int pos = st.synced; pos < st.logEnd;) {
-    // a fetch is a round trip to HBM: one only when the pass at hand is not all there
-    if (pos >= base + 64) fetch(pos);
-    if (pos - base + 1 + (int)(rlane(rk, pos - base) >> 8) > 64) fetch(pos);
-    const int h = pos - base;
-    const uint32_t hk = rlane(rk, h), hw = rlane(rw, h);
+    // the pass ends with the next header; a fetch is a round trip to HBM: one only when the pass at hand is
+    // not all there
+    if (pos >= base + 64 || !(headers >> (pos - base))) fetch(pos);
+    const int h = pos - base;   // its first record, or the header if it has none
+    const int end = h + __builtin_ctzll(headers >> h);
+    const uint32_t hk = rlane(rk, end), hw = rlane(rw, end);
     const int c = (int)(hk & 0xffu), nrec = (int)(hk >> 8);
     // rows in the reference's order: the first two swap when the heap has row 1's node on top
     const bool swap = (hw & kOpUnordered) && (uint32_t)uniform_i((int)rh.h[1].y) != (hw & 0x3ffffffu);
-    const unsigned long long mine = lane_range(nrec, h + 1);
+    const unsigned long long mine = lane_range(nrec, h);
     const uint32_t myRow = (rw >> 26) & 7u;
     // the pass's new nodes are those whose index had not been given out before it
     const unsigned long long fresh = lanes_where((int)(rw & 0x7ffu) >= seen) & mine;
@@ -754,9 +817,10 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     const float4 b = g.node(bi);
     const uint32_t bucket = GeoWave::hash(nb);
     uint32_t chainHead;
-    int ni = g.find<true>(nb != kNoNb, nb, bucket, &chainHead);
     const bool valid = nb != kNoNb;
-    const bool known = valid && ni >= 0;
+    const uint32_t at = g.find<true>(lanes_where(valid), nb, bucket, &chainHead);
+    const bool known = at != kChainEnd;
+    int ni = GeoWave::node_at<true>(at);
     float oldCost = 0;
     if (known) {
       const float4 pc = g.node(ni);
@@ -780,15 +844,12 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     while (fresh) {
       const int src = first_lane(fresh);
       fresh = without_lane(fresh, src);
-      if (lane == src) {
-        g.set_link<true>(ni, make_link(nb, L->first[bucket]));
-        L->first[bucket] = (uint16_t)ni;
-      }
+      const uint32_t head = L->first[bucket];
+      g.set_links<true>(1ull << src, ni, make_link(nb, head));
+      lds_store_where(1ull << src, &L->first[bucket], GeoWave::offset_of<true>((uint32_t)ni));
       wave_sync();
     }
-    if (update) {
-      g.keep_node(ni, make_float4(m0, m1, m2, cost), bi + 1);
-    }
+    g.keep_node(lanes_where(update), ni, make_float4(m0, m1, m2, cost), (uint32_t)bi + 1u);
     wave_sync();
     const uint32_t packed = (uint32_t)ni | (nb << 11);
     const unsigned long long was = lanes_where(known);
@@ -832,94 +893,100 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
   endIp = (uint32_t)uniform_i((int)endIp);
   OpenList& ol = st.ol;
   const int row = lane >> kRowShift, el = lane & (kRowLanes - 1);
-  // of every row: the first lane, the edges' lanes, the lane that looks after the row's own node in the conflict test
-  constexpr unsigned long long kRowStart = 0x0101010101010101ull, kEdgeLanes = 0x3f3f3f3f3f3f3f3full, kOwnLanes = 0x4040404040404040ull;
+  // the lanes of every row that look after the row's own node in the conflict test
+  constexpr unsigned long long kOwnLanes = 0x4040404040404040ull;
   static_assert(kNvp == 6 && kRowLanes == 8, "the lane masks of a row");
   constexpr unsigned long long kRows1 = rows_below(1), kRows2 = rows_below(2);   // lanes of the first rows
-  unsigned long long resolved = frontResolved ? 1ull : 0ull;
-  uint32_t cand = (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4, (int)ol.n[0]);   // entry `row` of the list
+  constexpr int kHeaderLane = 63;   // no edge's lane, and all that a pass updates lies before it
+  const char* edges_of = reinterpret_cast<const char*>(edges);
+  bool resolved = frontResolved;
+  // of every row: its entry of the list, and the total of the entry behind that
+  uint32_t cand = (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4, (int)ol.n[0]);
+  uint32_t nextTotal = (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4 + 4, (int)ol.t[0]);
   // Written for few instructions and few waits on the common path: what is rare sits behind one branch
   // each; conditions are lane masks on the scalar unit; LDS reads whose results are needed later go out
   // early (the marks' before the scan over the rows, the chain heads' before the stores); the next
-  // pass's nodes come back with the merged list instead of through a lane permute; stores take 32-bit
-  // offsets from uniform bases.  Together: 1.207 -> 1.144 ms at 16384 agents over mazes, 0.99 -> 0.92
-  // at 1024 over room plans.
-  for (;;) {
-    if (ol.size <= 0) return kAstarEmpty;
-    if (!S && g.nodeCount > kLinksLds - kRows * kNvp) return kAstarGrowLinks;
+  // pass's nodes and totals come back with the merged list instead of through lane permutes; stores take
+  // 32-bit offsets from uniform bases.  No branch depends on the lanes: loads of lanes that have nothing
+  // to load go to an address that exists, stores go out under a mask.  A wavefront issues an
+  // instruction of any kind every five cycles at best, a branch costs it fifteen and a result that goes
+  // from the vector to the scalar unit and back twenty, so a search alone on a SIMD lasts as long as its
+  // instructions, and many of them are bound by the units' issue.  (With branches around loads and
+  // stores, and the loop rebuilt around them with some sixty instructions more per pass: steps of 64
+  // agents 216 us, now 184, of 1024 over room plans 836 and 697, of 16384 over mazes 1026 and 902, of
+  // 65536 over mixed scenes 3740 and 3233; a reset of 2048 over mazes 655 and 525.)
+  const auto pass = [&]() BPSX_INLINE_LAMBDA -> AstarExit {
     if (st.logEnd > kOpLogCap - (1 + kRows * kNvp)) return kAstarLogFull;
     FM(0);
-    // ---- how many entries at the front are each the only one with their total
+    // ---- how many entries at the front are each the only one with their total, and not the goal
     const unsigned long long uniq = lanes_where(ol.t[0] < OpenList::down1(OpenList::kEmpty, ol.t[0]));
-    int lim = __builtin_ctzll(~uniq | (1ull << kRows));
+    const unsigned long long goal = lanes_where((ol.n[0] >> 11) == endIp);
+    uint32_t lim = (uint32_t)first_other_lane(uniq & ~goal);
+    lim = lim < (uint32_t)kRows ? lim : (uint32_t)kRows;
     const int bi = (int)(cand & 0x7ffu);
     const uint32_t ip = cand >> 11;
-    const unsigned long long goal = lanes_where(ip == endIp) & kRowStart;
-    bool pairTie = false, goalInPair = false;
-    if (__builtin_expect((goal | ((uniq & 1ull) ^ 1ull) | resolved) != 0, 0)) {
-      if (resolved) { lim = 1; resolved = 0; }   // the caller has put the reference's next node first
-      else if (lim == 0) {
+    int pairTie = 0;   // 2: with the goal as one of the two
+    uint32_t headerWord = kOpHeader;
+    if (__builtin_expect(lim == 0, 0)) {
+      if (ol.size <= 0) return kAstarEmpty;
+      if (uniq & 1ull) lim = (uint32_t)kRows;   // the goal
+      else if (resolved) { lim = 1; resolved = false; }   // the caller has put the reference's next node first
+      else {
         // The first two entries share the smallest total.  When they are alone in that and their
         // expansions are independent of each other (neither updates what the other reads, and
         // whatever they put on the list lies above their total), the reference expands them one
         // after the other, in the order its heap has them in, and ends in the same state either
         // way: the pass takes both and notes in the log that their order is open.
         if (!(uniq & 2ull)) return kAstarTie;
-        pairTie = true;
+        pairTie = 1;
         g.pairTies++;   // counts the attempts: one that fails comes back through the log
-        lim = __builtin_ctzll(~(uniq | 3ull) | (1ull << kRows));
+        lim = (uint32_t)__builtin_ctzll(~(uniq | 3ull) | (1ull << kRows));
       }
       if ((goal & 1ull) && !pairTie) {
         st.lastBest = uniform_i(bi);
         return kAstarGoal;
       }
-      // the goal as one of a tied pair: both rows are looked at, the goal's row without its edges
-      if (pairTie && (goal & kRows2)) { goalInPair = true; lim = 2; }
-      else if (goal) { const int jg = __builtin_ctzll(goal) >> kRowShift; lim = jg < lim ? jg : lim; }
+      // the goal as one of a tied pair: both rows are looked at
+      if (pairTie && (goal & 3ull)) { pairTie = 2; lim = 2; }
+      else if (pairTie && goal) { const uint32_t jg = (uint32_t)__builtin_ctzll(goal); lim = jg < lim ? jg : lim; }
     }
     FM(1);
-    const unsigned long long rowOn = lanes_where(row < lim);
-    uint32_t nb = kNoNb;
-    float m0 = 0, m1 = 0, m2 = 0;
-    if (in_mask(rowOn & kEdgeLanes)) {
-      const AEdge e = edges[ip * kEdgeStride + (uint32_t)el];
-      nb = e.nb; m0 = e.mid[0]; m1 = e.mid[1]; m2 = e.mid[2];
-    }
-    if (__builtin_expect(goalInPair, 0)) nb = ip == endIp ? kNoNb : nb;
-    const int bw = bi & (kWindow - 1);
-    float4 b = L->w_node[bw];
+    const unsigned long long rowOn = lanes_where(row < (int)lim);
+    const uint32_t edgeAt = OpenList::pick(rowOn, (ip << 7) | (uint32_t)(el << 4), 0u);
+    static_assert(kEdgeStride * sizeof(AEdge) == 128, "a polygon's records");
+    const AEdge edge = *reinterpret_cast<const AEdge*>(edges_of + edgeAt);
+    float4 b = L->w_node[bi & (kWindow - 1)];
     if (!kAllLds) {
       const unsigned long long left = lanes_where(bi < g.nodeCount - kWindow) & rowOn;
       if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
-        if (in_mask(left)) {
-          BPSX_KEEP_APART();
-          b = g.ws->nodes[bi];
-          BPSX_KEEP_APART();
-        }
+        BPSX_KEEP_APART();
+        const float4 kept = g.ws->nodes[bi];
+        BPSX_KEEP_APART();
+        b.x = in_mask(left) ? kept.x : b.x; b.y = in_mask(left) ? kept.y : b.y; b.z = in_mask(left) ? kept.z : b.z; b.w = in_mask(left) ? kept.w : b.w;
       }
     }
     FM(2);
     // ---- node lookup; the row's own lane hashes its own polygon for the conflict test
+    const uint32_t nb = edge.nb;
+    const unsigned long long valid = lanes_where(nb != kNoNb) & rowOn;
     const uint32_t bucket = GeoWave::hash(in_mask(kOwnLanes) ? ip : nb);
     uint32_t chainHead;
-    const unsigned long long valid = lanes_where(nb != kNoNb);
-    int ni = g.find<S>(in_mask(valid), nb, bucket, &chainHead);
+    const uint32_t at = g.find<S>(valid, nb, bucket, &chainHead);
     FM(3);
-    // ---- costs.  A lane without a node to read (idle, or its node is new) reads the window's last slot.
-    const unsigned long long known = lanes_where(ni >= 0);
-    const int rw = ni & (kWindow - 1);
-    float4 p = L->w_node[rw];
+    // ---- costs.  A lane without a node to read (idle, or its node is new) reads one of the window's slots.
+    const unsigned long long known = lanes_where(at != kChainEnd);
+    int ni = GeoWave::node_at<S>(at);
+    float4 p = L->w_node[ni & (kWindow - 1)];
     if (!kAllLds) {
       const unsigned long long left = lanes_where(ni < g.nodeCount - kWindow) & known;
       if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
-        if (in_mask(left)) {
-          BPSX_KEEP_APART();
-          p = g.ws->nodes[ni];
-          BPSX_KEEP_APART();
-        }
+        BPSX_KEEP_APART();
+        const float4 kept = g.ws->nodes[in_mask(left) ? ni : 0];
+        BPSX_KEEP_APART();
+        p.x = in_mask(left) ? kept.x : p.x; p.y = in_mask(left) ? kept.y : p.y; p.z = in_mask(left) ? kept.z : p.z; p.w = in_mask(left) ? kept.w : p.w;
       }
     }
-    const float p0 = in_mask(known) ? p.x : m0, p1 = in_mask(known) ? p.y : m1, p2 = in_mask(known) ? p.z : m2;   // a new node lies on the portal's midpoint
+    const float p0 = in_mask(known) ? p.x : edge.mid[0], p1 = in_mask(known) ? p.y : edge.mid[1], p2 = in_mask(known) ? p.z : edge.mid[2];   // a new node lies on the portal's midpoint
     const float cx = p0 - b.x, cy = p1 - b.y, cz = p2 - b.z;
     const float ex = e0 - p0, ey = e1 - p1, ez = e2 - p2;
     const float cc = cx * cx + cy * cy + cz * cz, ee = ex * ex + ey * ey + ez * ez;
@@ -933,143 +1000,142 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     // the lanes that update their node, and the total as bits there, all ones elsewhere.  (A node's
     // total so far is the sum it was computed as, of its cost and the same heuristic.)
     unsigned long long upd = valid & ~(known & lanes_where(total >= p.w + heuristic));
-    uint32_t tb = in_mask(upd) ? __float_as_uint(total) : 0xffffffffu;
+    const uint32_t tb = in_mask(upd) ? __float_as_uint(total) : 0xffffffffu;
     FM(4);
-    if (__builtin_expect(goalInPair, 0)) {
-      // The goal shares the smallest total with one other node.  If the reference takes the goal
-      // first the search ends here; if it takes the other node first, it expands it and ends
-      // then.  The path is the goal's node and its ancestors: it is the same both ways when
-      // that expansion only creates nodes (none of them can be on the path) and the node pool
-      // holds them (an exhausted pool is reported as failure).  Otherwise the heap must say.
-      const int fresh = __popcll(upd);
-      if ((upd & known) || g.nodeCount + fresh > kMaxNodes) return kAstarTie;
-      st.lastBest = (int)rlane((uint32_t)bi, first_lane(goal & kRows2));
-      return kAstarGoal;
-    }
     // ---- how many rows stand
-    int c = lim;
-    bool pairFails = false;
-    if (lim > 1) {
-      // conflicts: the earliest row that updates a polygon leaves its mark at the
-      // polygon's hash, later rows look for it (no marks stand when a pass begins)
-      const uint32_t slot = bucket & (uint32_t)(kTagSlots - 1);
-      if (in_mask(upd)) atomicMin(&L->marks()[slot], (uint32_t)row);
-      wave_sync();
-      const uint32_t seen = L->marks()[slot];   // the marking row, or all ones
-      // the first entry j that an update of a row before it reaches or undercuts: the smallest
-      // updated total of every row, then of all rows up to it (a scan over the rows), and entry j's
-      // lane compares its total with that of the rows before j
-      uint32_t low = tb;   // all ones where the lane updates nothing
-      low = umin_dpp<0xb1, 0xf>(low);    // quad_perm [1,0,3,2]
-      low = umin_dpp<0x4e, 0xf>(low);    // quad_perm [2,3,0,1]
-      low = umin_dpp<0x141, 0xf>(low);   // row_half_mirror: every lane has its row's smallest
-      low = umin_dpp<0x118, 0xf>(low);   // row_shr:8: odd rows, with the row before
-      low = umin_dpp<0x142, 0xa>(low);   // row_bcast:15 into the second and fourth 16 lanes
-      low = umin_dpp<0x143, 0xc>(low);   // row_bcast:31 into the upper 32 lanes
-      uint32_t before = (uint32_t)__builtin_amdgcn_ds_bpermute((lane - 1) * (kRowLanes * 4), (int)low);
-      // a tied pair: both its rows must lie above entry 1's total
-      if (__builtin_expect(pairTie, 0)) before = lane == 1 ? rlane(low, kRowLanes) : before;
-      const unsigned long long reached = lanes_where(before <= ol.t[0]) & (rows_below(1) & ~1ull);
-      const int jv = reached ? __builtin_ctzll(reached) : kRows;
-      c = jv < c ? jv : c;
-      // an earlier row's update matters to a row only at its own node and at the polygons it
-      // updates itself: where it reads and leaves alone (a total no better than the node's), a
-      // total lowered further changes nothing
-      const unsigned long long cares = upd | (rowOn & kOwnLanes);
-      const uint32_t jc = (uint32_t)first_lane(lanes_where(seen < (uint32_t)row) & cares) >> kRowShift;   // none: far above kRows
-      c = jc < (uint32_t)c ? (int)jc : c;
-      // rows 0 and 1 of a tied pair in either order: row 0 must not read what row 1 updates either
-      if (__builtin_expect(pairTie, 0)) {
-        pairFails = c < 2 || (lanes_where(seen == 1u) & cares & kRows1) != 0;
-        if (pairFails && jv >= 2) {
-          // The marks are kept per polygon hash, and a pair that fails costs a replay of the log:
-          // the polygons that either row updates are compared with those the other row reads,
-          // and a clash that was two polygons with one hash lets the pair (and only it) stand.
-          const uint32_t readPoly = in_mask(cares & kOwnLanes) ? ip : (in_mask(upd) ? nb : 0xffffffffu);
-          unsigned long long w = upd & kRows2;
-          bool real = false;
-          while (w) {
-            const int src = first_lane(w);
-            w = without_lane(w, src);
-            const unsigned long long others = src < kRowLanes ? (kRows2 & ~kRows1) : kRows1;
-            if (lanes_where(readPoly == rlane(nb, src)) & others) real = true;
-          }
-          if (!real) { pairFails = false; c = 2; }
-        }
+    // conflicts: the earliest row that updates a polygon leaves its mark at the polygon's hash, later rows
+    // look for it (no marks stand when a pass begins)
+    uint32_t* mark = &L->marks()[bucket & (uint32_t)(kTagSlots - 1)];
+    lds_min_where(upd, mark, (uint32_t)row);
+    wave_sync();
+    const uint32_t seen = *mark;   // the marking row, or above all rows
+    // the first entry that an update of a row before it reaches or undercuts: the smallest updated total of
+    // every row, then of all rows up to it (a scan over the rows), and each row compares that with the
+    // total of the entry behind its own
+    uint32_t low = tb;   // all ones where the lane updates nothing
+    low = umin_dpp<0xb1, 0xf>(low);    // quad_perm [1,0,3,2]
+    low = umin_dpp<0x4e, 0xf>(low);    // quad_perm [2,3,0,1]
+    low = umin_dpp<0x141, 0xf>(low);   // row_half_mirror: every lane has its row's smallest
+    low = umin_dpp<0x118, 0xf>(low);   // row_shr:8: odd rows, with the row before
+    low = umin_dpp<0x142, 0xa>(low);   // row_bcast:15 into the second and fourth 16 lanes
+    low = umin_dpp<0x143, 0xc>(low);   // row_bcast:31 into the upper 32 lanes
+    const unsigned long long reached = lanes_where(low <= nextTotal) << kRowLanes;   // in the lanes of the row behind
+    // an earlier row's update matters to a row only at its own node and at the polygons it
+    // updates itself: where it reads and leaves alone (a total no better than the node's), a
+    // total lowered further changes nothing
+    const unsigned long long cares = upd | (rowOn & kOwnLanes);
+    const unsigned long long clash = lanes_where(seen < (uint32_t)row) & cares;
+    uint32_t c = (uint32_t)first_lane(clash | reached | ~rowOn);   // in the first row that does not stand
+    c = (c < 64u ? c : 64u) >> kRowShift;
+    if (__builtin_expect(pairTie != 0, 0)) {
+      asm("" : "+s"(pairTie));   // (or both tests of it come first)
+      if (pairTie == 2) {
+        // The goal shares the smallest total with one other node.  If the reference takes the goal
+        // first the search ends here; if it takes the other node first, it expands it and ends
+        // then.  The path is the goal's node and its ancestors: it is the same both ways when
+        // that expansion only creates nodes (none of them can be on the path) and the node pool
+        // holds them (an exhausted pool is reported as failure).  Otherwise the heap must say.
+        const unsigned long long other = upd & ~lanes_where(ip == endIp);
+        if ((other & known) || g.nodeCount + __popcll(other) > kMaxNodes) return kAstarTie;
+        st.lastBest = (int)rlane((uint32_t)bi, first_lane(goal & 3ull) << kRowShift);
+        return kAstarGoal;
       }
+      // a tied pair: both its rows must lie above entry 1's total, ...
+      const bool above = rlane(low, kRowLanes) > rlane(nextTotal, 0);
+      if (!above) c = 1;
+      // ... and in either order: row 0 must not read what row 1 updates either
+      bool fails = c < 2 || (lanes_where(seen == 1u) & cares & kRows1) != 0;
+      if (fails && above && !(reached & kRows2)) {
+        // The marks are kept per polygon hash, and a pair that fails costs a replay of the log:
+        // the polygons that either row updates are compared with those the other row reads,
+        // and a clash that was two polygons with one hash lets the pair (and only it) stand.
+        const uint32_t readPoly = OpenList::pick(cares & kOwnLanes, ip, OpenList::pick(upd, nb, 0xffffffffu));
+        unsigned long long w = upd & kRows2;
+        bool real = false;
+        while (w) {
+          const int src = first_lane(w);
+          w = without_lane(w, src);
+          const unsigned long long others = src < kRowLanes ? (kRows2 & ~kRows1) : kRows1;
+          if (lanes_where(readPoly == rlane(nb, src)) & others) real = true;
+        }
+        if (!real) { fails = false; c = 2; }
+      }
+      if (fails) return kAstarTie;
+      headerWord = kOpHeader | kOpUnordered | rlane(cand, 0);
     }
-    if (__builtin_expect(pairFails, 0)) return kAstarTie;
     FM(5);
-    upd &= lanes_where(row < c);
-    tb = in_mask(upd) ? tb : 0xffffffffu;
+    upd &= lanes_where(row < (int)c);
     const int nrec = __popcll(upd);
-    // nothing has changed yet: a list that would outgrow its registers goes on in the wider instantiation
-    if (__builtin_expect(ol.size - c + nrec > 64 * P, 0)) return kAstarGrowHeap;
-    (*pops) += (uint32_t)c;
+    const unsigned long long fresh = upd & ~known;
+    const int want = g.nodeCount + __popcll(fresh);
+    // Nothing has changed yet: a list that would outgrow its registers goes on in the wider instantiation,
+    // links that would outgrow LDS in the one that spills.
+    if (__builtin_expect(ol.size - (int)c + nrec > 64 * P, 0)) return kAstarGrowHeap;
+    if (!S && __builtin_expect(want > kLinksLds, 0)) return kAstarGrowLinks;
+    (*pops) += c;
+    // the reference carries on without the nodes that do not fit, but reports anything found
+    // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): stop
+    if (S && __builtin_expect(want > kMaxNodes, 0)) {
+      st.outOfNodes = true;
+      return kAstarEmpty;
+    }
     FM(6);
     // ---- new nodes (always taken) get consecutive indices in row and edge order
-    const unsigned long long fresh = upd & ~known;
-    uint32_t head = (uint32_t)ni;
-    if (fresh) {
-      const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(fresh >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)fresh, 0u));
-      const int want = g.nodeCount + __popcll(fresh);
-      // the reference carries on without the nodes that do not fit, but reports anything found
-      // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): stop
-      if (S && want > kMaxNodes) {
-        st.outOfNodes = true;
-        return kAstarEmpty;
-      }
-      // All insert at once in front of the chain head their lookup saw.  Of several that share a
-      // bucket one store wins; the others see that when the head that is read back here has come
-      // (looked at below, after the stores that need not wait for it).
-      if (in_mask(fresh)) {
-        ni = g.nodeCount + rank;
-        g.set_link<S>(ni, make_link(nb, chainHead));
-        L->first[bucket] = (uint16_t)ni;
-      }
-      g.nodeCount = want;
-      wave_sync();
-      head = L->first[bucket];
-    }
+    const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(fresh >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)fresh, 0u));
+    ni = (int)OpenList::pick(fresh, (uint32_t)(g.nodeCount + rank), (uint32_t)ni);
+    // All insert at once in front of the chain head their lookup saw.  Of several that share a
+    // bucket one store wins; the others see that when the head that is read back here has come
+    // (looked at below, after the stores that need not wait for it).
+    uint32_t own = GeoWave::offset_of<S>((uint32_t)ni);
+    asm("" : "+v"(own));   // (or offsets into the other arrays become multiplications of it)
+    uint16_t* const chain = &L->first[bucket];
+    g.set_links<S>(fresh, ni, make_link(nb, chainHead));
+    lds_store_where(fresh, chain, own);
+    g.nodeCount = want;
+    wave_sync();
+    uint32_t head = *chain;
     FM(7);
-    if (in_mask(upd)) {
+    {
       const float4 node = make_float4(p0, p1, p2, cost);
-      if (!kAllLds && g.in_window(ni)) L->w_node[ni & (kWindow - 1)] = node;
-      g.keep_node(ni, node, bi + 1);
+      if (!kAllLds) lds_store_where(upd & lanes_where(ni >= want - kWindow), &L->w_node[ni & (kWindow - 1)], node);
+      g.keep_node(upd, ni, node, (uint32_t)bi + 1u);
     }
     FM(8);
     const uint32_t packed = (uint32_t)ni | (nb << 11);
     {
-      // the pass in the operation log: the header from an idle lane, the updates in lane order
-      constexpr unsigned long long kHeader = 1ull << (kRowLanes - 1);   // neither an edge's lane nor the node's own
-      uint32_t headerWord = kOpHeader;
-      if (__builtin_expect(pairTie, 0)) headerWord = kOpHeader | kOpUnordered | rlane(cand, 0);
-      const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(upd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)upd, 1u));
-      if (in_mask(upd | kHeader)) {
-        OpRec r;
-        r.key = OpenList::pick(kHeader, (uint32_t)c | ((uint32_t)nrec << 8), tb);
-        r.word = OpenList::pick(kHeader, headerWord, packed | ((uint32_t)row << 26));
-        *reinterpret_cast<OpRec*>(reinterpret_cast<char*>(g.ws->oplog) + ((uint32_t)st.logEnd + OpenList::pick(kHeader, 0u, (uint32_t)rank)) * (uint32_t)sizeof(OpRec)) = r;
-      }
+      // the pass in the operation log: the updates in lane order, then the header
+      const int rec = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(upd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)upd, (uint32_t)st.logEnd));
+      const uint32_t key = wlane_at<kHeaderLane>(tb, c | ((uint32_t)nrec << 8));
+      const uint32_t word = wlane_at<kHeaderLane>(packed | ((uint32_t)row << 26), headerWord);
+      store_where(upd | (1ull << kHeaderLane), g.ws->oplog, (uint32_t)rec * (uint32_t)sizeof(OpRec), key, word);
       st.logEnd += 1 + nrec;
     }
     // new nodes that another of their bucket has overwritten at the chain's head go in behind it
-    for (unsigned long long lost = fresh & lanes_where(head != (uint32_t)ni); __builtin_expect(lost != 0, 0);) {
-      if (in_mask(lost)) {
-        g.set_link<S>(ni, make_link(nb, head));
-        L->first[bucket] = (uint16_t)ni;
-      }
+    for (unsigned long long lost = fresh & lanes_where(head != own); __builtin_expect(lost != 0, 0);) {
+      g.set_links<S>(lost, ni, make_link(nb, head));
+      lds_store_where(lost, chain, own);
       wave_sync();
-      head = L->first[bucket];
-      lost &= lanes_where(head != (uint32_t)ni);
+      head = *chain;
+      lost &= lanes_where(head != own);
       wave_sync();
     }
     FM(9);
     // ---- the open list: the committed entries leave, the updates enter
-    cand = ol.template merge<P>(L->entries(), c, upd, upd & known, tb, packed, lane, row);
+    const uint2 front = ol.template merge<P>(L->entries(), (int)c, upd, upd & known, tb, packed, lane, row);
+    cand = front.x;
+    nextTotal = front.y;
     g.clear_marks();
     FM(10);
-  }
+    return kAstarOn;
+  };
+  // All ways out of a pass meet here, and the loop has one end: with several the compiler keeps a flag for each,
+  // and copies of the loop's state.  (The empty statement keeps it from joining a way out to what follows it.)
+  int way;
+  do {
+    way = (int)pass();
+    asm volatile("" : "+s"(way));
+  } while (way == (int)kAstarOn);
+  return (AstarExit)way;
 }
 
 // Runs A* for one query. Returns the corridor length (corridor written to F->corridor), or 0
@@ -1091,11 +1157,11 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   if (lane == 0) {
     GeoLds* L = g.L;
     L->w_node[0] = make_float4(startPos[0], startPos[1], startPos[2], 0.0f);
-    g.keep_node(0, L->w_node[0], 0);
     L->n_link[0] = make_link(startIp, kChainEnd);
     L->first[GeoWave::hash(startIp)] = 0;
     reinterpret_cast<uint2*>(g.ws->heap_spill)[1] = make_uint2(__float_as_uint(total), startIp << 11);
   }
+  g.keep_node(1ull, 0, make_float4(startPos[0], startPos[1], startPos[2], 0.0f), 0u);
   wave_sync();
   st.lastBest = 0;
   st.outOfNodes = false;
@@ -1120,7 +1186,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     else ex = spill ? BPSX_FAST_RUN(true) : BPSX_FAST_RUN(false);
 #undef BPSX_FAST_RUN
     resolved = false;
-    if (ex == kAstarGrowLinks) { g.linkSpills++; spill = true; continue; }
+    if (ex == kAstarGrowLinks) { g.clear_marks(); g.linkSpills++; spill = true; continue; }   // as below
     if (ex == kAstarGrowHeap && pairs < OpenList::kPairs) {
       g.clear_marks();   // the pass that did not fit has left its own
       // the list grows into further registers, empty so far
