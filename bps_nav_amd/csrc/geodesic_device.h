@@ -106,12 +106,12 @@ BPSX_DEV void lds_store_where(unsigned long long mask, uint2* p, uint32_t x, uin
   const unsigned long long v = ((unsigned long long)y << 32) | x;
   asm volatile("s_mov_b64 exec, %0\n\tds_write_b64 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(v) : "memory");
 }
-BPSX_DEV void lds_store_where(unsigned long long mask, float4* p, float4 f) {
+BPSX_DEV void lds_store_where(unsigned long long mask, uint32_t address, float4 f) {
   const Float4 v = {f.x, f.y, f.z, f.w};
-  asm volatile("s_mov_b64 exec, %0\n\tds_write_b128 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(v) : "memory");
+  asm volatile("s_mov_b64 exec, %0\n\tds_write_b128 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(address), "v"(v) : "memory");
 }
-BPSX_DEV void lds_store_where(unsigned long long mask, uint32_t* p, uint32_t x) {
-  asm volatile("s_mov_b64 exec, %0\n\tds_write_b32 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x) : "memory");
+BPSX_DEV void lds_store_where(unsigned long long mask, uint32_t address, uint32_t x) {
+  asm volatile("s_mov_b64 exec, %0\n\tds_write_b32 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(address), "v"(x) : "memory");
 }
 BPSX_DEV void lds_store_where(unsigned long long mask, uint16_t* p, uint32_t x) {
   asm volatile("s_mov_b64 exec, %0\n\tds_write_b16 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x) : "memory");
@@ -214,10 +214,11 @@ struct OpenList {
   // then took 1.229 ms instead of 1.207 at 16384 agents over mazes, 3.11 instead of 2.59 at 4096
   // over cluttered plans, whose lists fill two to four pairs, 1.16 instead of 0.99 at 1024 over room
   // plans, where a launch lasts as long as its longest search alone.)
+  // meanwhile() is called while the entries come back from LDS.
   // Returns the node of entry `row` of the new list and the total of the one behind it (of kNone and kEmpty
   // where there is none).
-  template <int P> BPSX_DEV uint2 merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
-                                        uint32_t packed, int lane, int row) {
+  template <int P, class Meanwhile> BPSX_DEV uint2 merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
+                                                         uint32_t packed, int lane, int row, Meanwhile meanwhile) {
     unsigned long long dead[P];
 #pragma unroll
     for (int k = 0; k < P; ++k) dead[k] = 0;
@@ -272,6 +273,7 @@ struct OpenList {
       wave_sync();
       const uint2 e = buf[lane];
       front = make_uint2(buf[row].y, buf[row + 1].x);
+      meanwhile();
       t[0] = lane < size ? e.x : kEmpty;
       n[0] = lane < size ? e.y : kNone;
     } else {
@@ -287,12 +289,13 @@ struct OpenList {
         lds_store_where(enters & lanes_where((place >> 7) == (uint32_t)half), &buf[place & 127u], tb, packed);
         wave_sync();
         if (half == 0) front = make_uint2(buf[row].y, buf[row + 1].x);
-        static_for<0, 2>([&](auto K) BPSX_INLINE_LAMBDA {
-          constexpr int k = 2 * half + decltype(K)::value;
-          const uint2 e = buf[(k & 1) * 64 + lane];
-          nt[k] = 64 * k + lane < size ? e.x : kEmpty;
-          nn[k] = 64 * k + lane < size ? e.y : kNone;
-        });
+        const uint2 e0 = buf[lane], e1 = buf[64 + lane];
+        if (half == 0) meanwhile();
+        constexpr int k = 2 * half;
+        nt[k] = 64 * k + lane < size ? e0.x : kEmpty;
+        nn[k] = 64 * k + lane < size ? e0.y : kNone;
+        nt[k + 1] = 64 * k + 64 + lane < size ? e1.x : kEmpty;
+        nn[k + 1] = 64 * k + 64 + lane < size ? e1.y : kNone;
         wave_sync();
       });
       static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA { constexpr int k = decltype(K)::value; t[k] = nt[k]; n[k] = nn[k]; });
@@ -441,12 +444,13 @@ struct GeoWave {
   uint32_t pairTies;                 // passes that took two nodes of equal total in one go
 
   // ---------------------------------------------------------------- node pool
-  // offset of node i's link: that of the links in LDS, beyond them that of the slot's shifted past kChainEnd
-  template <bool S> static BPSX_DEV uint32_t offset_of(uint32_t i) {
-    return !S || kLinksLds >= kMaxNodes ? 4u * i : 4u * (i + (i >= (uint32_t)kLinksLds ? 1u : 0u));
+  // A node's index is handled as four times itself, the offset of its word among the links.  Offset of its link
+  // within the chains: that of the links in LDS, beyond them that of the slot's shifted past kChainEnd.
+  template <bool S> static BPSX_DEV uint32_t offset_of(uint32_t i4) {
+    return !S || kLinksLds >= kMaxNodes ? i4 : i4 + (i4 >= kChainEnd ? 4u : 0u);
   }
-  template <bool S> static BPSX_DEV int node_at(uint32_t offset) {
-    return (int)(!S || kLinksLds >= kMaxNodes ? offset >> 2 : (offset >> 2) - (offset > kChainEnd ? 1u : 0u));
+  template <bool S> static BPSX_DEV uint32_t node4_at(uint32_t offset) {
+    return !S || kLinksLds >= kMaxNodes ? offset : offset - (offset > kChainEnd ? 4u : 0u);
   }
   // where node i's link lies
   template <bool S> BPSX_DEV uint32_t link(int i) const {
@@ -456,17 +460,15 @@ struct GeoWave {
     BPSX_KEEP_APART();
     return v;
   }
-  template <bool S> BPSX_DEV void set_links(unsigned long long mask, int i, uint32_t v) const {
+  template <bool S> BPSX_DEV void set_links(unsigned long long mask, uint32_t i4, uint32_t v) const {
     if (!S || kLinksLds >= kMaxNodes) {
-      lds_store_where(mask, &L->n_link[i], v);
+      lds_store_where(mask, lds_address(L->n_link) + i4, v);
     } else {
-      const unsigned long long near = lanes_where(i < kLinksLds);
-      lds_store_where(mask & near, &L->n_link[i], v);
-      store_where(mask & ~near, ws->links, (uint32_t)i * 4u, v);
+      const unsigned long long near = lanes_where(i4 < kChainEnd);
+      lds_store_where(mask & near, lds_address(L->n_link) + i4, v);
+      store_where(mask & ~near, ws->links, i4, v);
     }
   }
-  // node i still has its position and cost in LDS
-  BPSX_DEV bool in_window(int i) const { return kAllLds || i >= nodeCount - kWindow; }
   // node i, whose position and cost are not looked for in the window; and a node and its parent index stored outside of it
   BPSX_DEV float4 node(int i) const {
 #if BPSX_WINDOW >= 2048
@@ -475,15 +477,17 @@ struct GeoWave {
     return ws->nodes[i];
 #endif
   }
-  // node i and its parent index, in the lanes of mask
-  BPSX_DEV void keep_node(unsigned long long mask, int i, float4 n, uint32_t parent) const {
-    const Float4 v = {n.x, n.y, n.z, n.w};
+  // the node and its parent index, in the lanes of mask; offsets of both by shifts of i4, which the caller keeps the
+  // compiler from knowing as a multiple of the index (it would multiply)
+  // (With all nodes in LDS: the parent index only.)
+  BPSX_DEV void keep_node(unsigned long long mask, uint32_t i4, float4 n, uint32_t parent) const {
 #if BPSX_WINDOW >= 2048
-    asm volatile("s_mov_b64 exec, %0\n\tds_write_b128 %1, %2\n\tds_write_b16 %3, %4\n\ts_mov_b64 exec, -1"
-                 :: "s"(mask), "v"(lds_address(&L->w_node[i])), "v"(v), "v"(lds_address(&L->parents[i])), "v"(parent) : "memory");
+    asm volatile("s_mov_b64 exec, %0\n\tds_write_b16 %1, %2\n\ts_mov_b64 exec, -1"
+                 :: "s"(mask), "v"(lds_address(L->parents) + (i4 >> 1)), "v"(parent) : "memory");
 #else
+    const Float4 v = {n.x, n.y, n.z, n.w};
     asm volatile("s_mov_b64 exec, %0\n\tglobal_store_dwordx4 %1, %2, %3\n\tglobal_store_short %4, %5, %6\n\ts_mov_b64 exec, -1"
-                 :: "s"(mask), "v"((uint32_t)i * (uint32_t)sizeof(float4)), "v"(v), "s"(ws->nodes), "v"((uint32_t)i * 2u), "v"(parent), "s"(ws->parents) : "memory");
+                 :: "s"(mask), "v"(i4 << 2), "v"(v), "s"(ws->nodes), "v"(i4 >> 1), "v"(parent), "s"(ws->parents) : "memory");
 #endif
   }
   // the multiply as the full-rate 24-bit instruction (polygon indices have 15 bits)
@@ -820,7 +824,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     const bool valid = nb != kNoNb;
     const uint32_t at = g.find<true>(lanes_where(valid), nb, bucket, &chainHead);
     const bool known = at != kChainEnd;
-    int ni = GeoWave::node_at<true>(at);
+    int ni = (int)(GeoWave::node4_at<true>(at) >> 2);
     float oldCost = 0;
     if (known) {
       const float4 pc = g.node(ni);
@@ -845,11 +849,14 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
       const int src = first_lane(fresh);
       fresh = without_lane(fresh, src);
       const uint32_t head = L->first[bucket];
-      g.set_links<true>(1ull << src, ni, make_link(nb, head));
-      lds_store_where(1ull << src, &L->first[bucket], GeoWave::offset_of<true>((uint32_t)ni));
+      g.set_links<true>(1ull << src, 4u * (uint32_t)ni, make_link(nb, head));
+      lds_store_where(1ull << src, &L->first[bucket], GeoWave::offset_of<true>(4u * (uint32_t)ni));
       wave_sync();
     }
-    g.keep_node(lanes_where(update), ni, make_float4(m0, m1, m2, cost), (uint32_t)bi + 1u);
+    uint32_t ni4 = 4u * (uint32_t)ni;
+    asm("" : "+v"(ni4));
+    g.keep_node(lanes_where(update), ni4, make_float4(m0, m1, m2, cost), (uint32_t)bi + 1u);
+    if (kAllLds) lds_store_where(lanes_where(update), lds_address(L->w_node) + (ni4 << 2), make_float4(m0, m1, m2, cost));
     wave_sync();
     const uint32_t packed = (uint32_t)ni | (nb << 11);
     const unsigned long long was = lanes_where(known);
@@ -915,16 +922,62 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
   // stores, and the loop rebuilt around them with some sixty instructions more per pass: steps of 64
   // agents 216 us, now 184, of 1024 over room plans 836 and 697, of 16384 over mazes 1026 and 902, of
   // 65536 over mixed scenes 3740 and 3233; a reset of 2048 over mazes 655 and 525.)
+  // The next pass's edge records are asked for as soon as its nodes are known, before it is known how many of them
+  // can be taken.  What a pass stores in HBM goes out while the list's entries come back from LDS: the wait
+  // for the records is one for all that was asked for before.  Where a wavefront has a search's whole
+  // links in LDS, and few others next to it, what a pass stores in LDS goes out behind that request, for
+  // whose time a lone search has it for nothing.  (Steps of 1024 agents over room plans 693 -> 656 us, of 510
+  // in two groups 1327 -> 1230, a reset of 2048 over mazes 525 -> 495; without that delay also of
+  // 16384 over mazes 902 -> 883, of 65536 over mixed scenes 3222 -> 3150, with it 910 and 3185.)
+  struct {
+    unsigned long long updated, fresh;   // lanes of updated nodes, of new ones among them
+    uint32_t node4, link;                // the node, its link
+    uint16_t* chain;
+    float4 node;
+  } late;
+  constexpr bool kLate = kLinksLds >= kMaxNodes;
+  late.updated = late.fresh = 0;
+  late.node4 = late.link = 0;
+  late.chain = L->first;
+  late.node = make_float4(0, 0, 0, 0);
+  const auto insert = [&]() BPSX_INLINE_LAMBDA {
+    // The new nodes insert all at once in front of the chain head their lookup saw.  Of several
+    // that share a bucket one store wins; the others see that when the head that is read back has come
+    // (looked at below, after the stores that need not wait for it).
+    if (kLate) g.clear_marks();
+    const uint32_t own = GeoWave::offset_of<S>(late.node4);
+    g.set_links<S>(late.fresh, late.node4, late.link);
+    lds_store_where(late.fresh, late.chain, own);
+    wave_sync();
+    uint32_t head = *late.chain;
+    if (kAllLds) lds_store_where(late.updated, lds_address(L->w_node) + (late.node4 << 2), late.node);
+    else lds_store_where(late.updated & lanes_where((int)late.node4 >= 4 * (g.nodeCount - kWindow)),
+                         lds_address(L->w_node) + ((late.node4 << 2) & (16u * (kWindow - 1))), late.node);
+    // new nodes that another of their bucket has overwritten at the chain's head go in behind it
+    for (unsigned long long lost = late.fresh & lanes_where(head != own); __builtin_expect(lost != 0, 0);) {
+      g.set_links<S>(lost, late.node4, make_link(link_id(late.link), head));
+      lds_store_where(lost, late.chain, own);
+      wave_sync();
+      head = *late.chain;
+      lost &= lanes_where(head != own);
+      wave_sync();
+    }
+  };
   const auto pass = [&]() BPSX_INLINE_LAMBDA -> AstarExit {
-    if (st.logEnd > kOpLogCap - (1 + kRows * kNvp)) return kAstarLogFull;
     FM(0);
+    // ---- the edge records of the first entries' polygons (of polygon 0 where there is no entry)
+    const uint32_t ip = cand >> 11;
+    static_assert(kEdgeStride * sizeof(AEdge) == 128, "a polygon's records");
+    const AEdge edge = *reinterpret_cast<const AEdge*>(edges_of + ((ip << 7) | (uint32_t)(el << 4)));
+    if (kLate) insert();
+    FM(1);
+    if (st.logEnd > kOpLogCap - (1 + kRows * kNvp)) return kAstarLogFull;
     // ---- how many entries at the front are each the only one with their total, and not the goal
     const unsigned long long uniq = lanes_where(ol.t[0] < OpenList::down1(OpenList::kEmpty, ol.t[0]));
     const unsigned long long goal = lanes_where((ol.n[0] >> 11) == endIp);
     uint32_t lim = (uint32_t)first_other_lane(uniq & ~goal);
     lim = lim < (uint32_t)kRows ? lim : (uint32_t)kRows;
     const int bi = (int)(cand & 0x7ffu);
-    const uint32_t ip = cand >> 11;
     int pairTie = 0;   // 2: with the goal as one of the two
     uint32_t headerWord = kOpHeader;
     if (__builtin_expect(lim == 0, 0)) {
@@ -950,11 +1003,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       if (pairTie && (goal & 3ull)) { pairTie = 2; lim = 2; }
       else if (pairTie && goal) { const uint32_t jg = (uint32_t)__builtin_ctzll(goal); lim = jg < lim ? jg : lim; }
     }
-    FM(1);
     const unsigned long long rowOn = lanes_where(row < (int)lim);
-    const uint32_t edgeAt = OpenList::pick(rowOn, (ip << 7) | (uint32_t)(el << 4), 0u);
-    static_assert(kEdgeStride * sizeof(AEdge) == 128, "a polygon's records");
-    const AEdge edge = *reinterpret_cast<const AEdge*>(edges_of + edgeAt);
     float4 b = L->w_node[bi & (kWindow - 1)];
     if (!kAllLds) {
       const unsigned long long left = lanes_where(bi < g.nodeCount - kWindow) & rowOn;
@@ -975,13 +1024,13 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     FM(3);
     // ---- costs.  A lane without a node to read (idle, or its node is new) reads one of the window's slots.
     const unsigned long long known = lanes_where(at != kChainEnd);
-    int ni = GeoWave::node_at<S>(at);
-    float4 p = L->w_node[ni & (kWindow - 1)];
+    uint32_t ni4 = GeoWave::node4_at<S>(at);
+    float4 p = L->w_node[(ni4 >> 2) & (kWindow - 1)];
     if (!kAllLds) {
-      const unsigned long long left = lanes_where(ni < g.nodeCount - kWindow) & known;
+      const unsigned long long left = lanes_where((int)ni4 < 4 * (g.nodeCount - kWindow)) & known;
       if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
         BPSX_KEEP_APART();
-        const float4 kept = g.ws->nodes[in_mask(left) ? ni : 0];
+        const float4 kept = g.ws->nodes[OpenList::pick(left, ni4 >> 2, 0u)];
         BPSX_KEEP_APART();
         p.x = in_mask(left) ? kept.x : p.x; p.y = in_mask(left) ? kept.y : p.y; p.z = in_mask(left) ? kept.z : p.z; p.w = in_mask(left) ? kept.w : p.w;
       }
@@ -1082,49 +1131,33 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     FM(6);
     // ---- new nodes (always taken) get consecutive indices in row and edge order
     const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(fresh >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)fresh, 0u));
-    ni = (int)OpenList::pick(fresh, (uint32_t)(g.nodeCount + rank), (uint32_t)ni);
-    // All insert at once in front of the chain head their lookup saw.  Of several that share a
-    // bucket one store wins; the others see that when the head that is read back here has come
-    // (looked at below, after the stores that need not wait for it).
-    uint32_t own = GeoWave::offset_of<S>((uint32_t)ni);
-    asm("" : "+v"(own));   // (or offsets into the other arrays become multiplications of it)
-    uint16_t* const chain = &L->first[bucket];
-    g.set_links<S>(fresh, ni, make_link(nb, chainHead));
-    lds_store_where(fresh, chain, own);
+    ni4 = OpenList::pick(fresh, 4u * (uint32_t)(g.nodeCount + rank), ni4);   // (opaque, as keep_node wants it)
+    late.fresh = fresh;
+    late.updated = upd;
+    late.node4 = ni4;
+    late.link = make_link(nb, chainHead);
+    late.chain = &L->first[bucket];
+    late.node = make_float4(p0, p1, p2, cost);
     g.nodeCount = want;
-    wave_sync();
-    uint32_t head = *chain;
     FM(7);
-    {
-      const float4 node = make_float4(p0, p1, p2, cost);
-      if (!kAllLds) lds_store_where(upd & lanes_where(ni >= want - kWindow), &L->w_node[ni & (kWindow - 1)], node);
-      g.keep_node(upd, ni, node, (uint32_t)bi + 1u);
-    }
-    FM(8);
-    const uint32_t packed = (uint32_t)ni | (nb << 11);
-    {
-      // the pass in the operation log: the updates in lane order, then the header
-      const int rec = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(upd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)upd, (uint32_t)st.logEnd));
-      const uint32_t key = wlane_at<kHeaderLane>(tb, c | ((uint32_t)nrec << 8));
-      const uint32_t word = wlane_at<kHeaderLane>(packed | ((uint32_t)row << 26), headerWord);
-      store_where(upd | (1ull << kHeaderLane), g.ws->oplog, (uint32_t)rec * (uint32_t)sizeof(OpRec), key, word);
+    // the pass in the operation log: the updates in lane order, then the header
+    const uint32_t packed = (ni4 >> 2) | (nb << 11);
+    const uint32_t key = wlane_at<kHeaderLane>(tb, c | ((uint32_t)nrec << 8));
+    const uint32_t word = wlane_at<kHeaderLane>(packed | ((uint32_t)row << 26), headerWord);
+    const auto store = [&]() BPSX_INLINE_LAMBDA {
+      const uint32_t rec = __builtin_amdgcn_mbcnt_hi((uint32_t)(upd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)upd, (uint32_t)st.logEnd));
+      store_where(upd | (1ull << kHeaderLane), g.ws->oplog, rec * (uint32_t)sizeof(OpRec), key, word);
+      g.keep_node(upd, ni4, late.node, (uint32_t)bi + 1u);
       st.logEnd += 1 + nrec;
-    }
-    // new nodes that another of their bucket has overwritten at the chain's head go in behind it
-    for (unsigned long long lost = fresh & lanes_where(head != own); __builtin_expect(lost != 0, 0);) {
-      g.set_links<S>(lost, ni, make_link(nb, head));
-      lds_store_where(lost, chain, own);
-      wave_sync();
-      head = *chain;
-      lost &= lanes_where(head != own);
-      wave_sync();
-    }
+    };
+    FM(8);
+    if (!kLate) insert();
     FM(9);
     // ---- the open list: the committed entries leave, the updates enter
-    const uint2 front = ol.template merge<P>(L->entries(), (int)c, upd, upd & known, tb, packed, lane, row);
+    const uint2 front = ol.template merge<P>(L->entries(), (int)c, upd, upd & known, tb, packed, lane, row, store);
     cand = front.x;
     nextTotal = front.y;
-    g.clear_marks();
+    if (!kLate) g.clear_marks();
     FM(10);
     return kAstarOn;
   };
