@@ -195,7 +195,55 @@ struct OpenList {
   static BPSX_DEV uint32_t down1(uint32_t last, uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp((int)last, (int)v, 0x130 /* wave_shl:1 */, 0xf, 0xf, false);
   }
-  // v as a select operand under a lane mask held in scalar registers
+  // lane L takes v of lane L - 1, lane 0 zero
+  static BPSX_DEV uint32_t up1(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138 /* wave_shr:1 */, 0xf, 0xf, true);
+  }
+  // The entries of lanes `rest` (totals tb, nodes `packed`) enter the first 64, which have room for them, one after the
+  // other, each behind those with totals up to its own: every lane keeps its entry, takes the new one or
+  // the one before it, and its total is the middle one of three.  As one piece: twelve instructions an entry, none
+  // of which waits for the scalar unit, in an order that keeps the distances that this hardware asks for and does
+  // not watch over, two instructions between a vector instruction that writes a scalar register (a
+  // comparison, a lane read) and the vector instruction that reads it, and between one that writes
+  // a register and the lane move that reads it.
+  BPSX_DEV void enter(unsigned long long rest, uint32_t tb, uint32_t packed) {
+    uint32_t tp, np, vn, st, sn;
+    int at;
+    unsigned long long above;
+    asm volatile("s_cmp_eq_u64 %[rest], 0\n\t"
+                 "s_cbranch_scc1 2f\n"
+                 "1:\n\t"
+                 "s_ff1_i32_b64 %[at], %[rest]\n\t"
+                 "s_bitset0_b64 %[rest], %[at]\n\t"
+                 "v_readlane_b32 %[st], %[tb], %[at]\n\t"
+                 "v_readlane_b32 %[sn], %[packed], %[at]\n\t"
+                 "v_mov_b32_dpp %[tp], %[t] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+                 "v_mov_b32_dpp %[np], %[n] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+                 "v_cmp_lt_u32_e64 %[above], %[st], %[t]\n\t"
+                 "v_mov_b32 %[vn], %[sn]\n\t"
+                 "v_cmp_lt_u32_e32 vcc, %[st], %[tp]\n\t"
+                 "v_med3_u32 %[t], %[tp], %[st], %[t]\n\t"
+                 "v_cndmask_b32_e64 %[n], %[n], %[vn], %[above]\n\t"
+                 "s_cmp_lg_u64 %[rest], 0\n\t"
+                 "v_cndmask_b32_e32 %[n], %[n], %[np], vcc\n\t"
+                 "s_cbranch_scc1 1b\n\t"
+                 "s_nop 1\n"
+                 "2:"
+                 : [rest] "+s"(rest), [t] "+v"(t[0]), [n] "+v"(n[0]), [tp] "=&v"(tp), [np] "=&v"(np), [vn] "=&v"(vn), [st] "=&s"(st), [sn] "=&s"(sn),
+                   [at] "=&s"(at), [above] "=&s"(above)
+                 : [tb] "v"(tb), [packed] "v"(packed)
+                 : "vcc", "scc");
+  }
+  // One entry, total and node the same for all lanes, in the lanes of `within`.
+  BPSX_DEV void enter_within(uint32_t total, uint32_t node, unsigned long long within) {
+    const uint32_t tp = up1(t[0]), np = up1(n[0]);
+    const unsigned long long above = lanes_where(t[0] > total) & within, shifted = lanes_where(tp > total) & within;
+    t[0] = pick(shifted, tp, pick(above, total, t[0]));
+    n[0] = pick(shifted, np, pick(above, node, n[0]));
+    asm volatile("s_nop 1" : "+v"(t[0]), "+v"(n[0]));   // as above, before the next lane move
+  }
+  // v as a select operand under a lane mask that a scalar instruction has written (the compiler does not know the
+  // select for a vector instruction, which has to keep two instructions' distance from a comparison)
   static BPSX_DEV uint32_t pick(unsigned long long mask, uint32_t yes, uint32_t no) {
     uint32_t r;
     asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(no), "v"(yes), "s"(mask));
@@ -219,6 +267,30 @@ struct OpenList {
   // where there is none).
   template <int P, class Meanwhile> BPSX_DEV uint2 merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
                                                          uint32_t packed, int lane, int row, Meanwhile meanwhile) {
+    if constexpr (P == 1) {
+      // Within 64 entries those that leave go by a lane permute, and the new ones enter one after the other.
+      // (Counted into place together and moved through LDS as the longer lists are: steps of 16384 agents
+      // over mazes 884 us, now 854, of 65536 over mixed scenes 3150 and 3078, of 64 179 and 170.)
+      uint32_t from = (uint32_t)(lane + c) * 4u;
+      from = from < 252u ? from : 252u;
+      t[0] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)from, (int)t[0]);
+      n[0] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)from, (int)n[0]);
+      meanwhile();
+      size += __popcll(upd) - c;
+      enter(upd & ~known, tb, packed);
+      // one whose node has an entry already (a modify; its total only falls) moves up from there to its place, one
+      // without is a push
+      while (known) {
+        const int src = first_lane(known);
+        known = without_lane(known, src);
+        const uint32_t node = rlane(packed, src);
+        const unsigned long long old = lanes_where(n[0] == node) & lanes_where(t[0] != kEmpty);
+        size -= __popcll(old);
+        enter_within(rlane(tb, src), node, old ^ (old - 1ull));   // up to its old place, or everywhere
+      }
+      wave_sync();
+      return make_uint2((uint32_t)__builtin_amdgcn_ds_bpermute(row * 4, (int)n[0]), (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4 + 4, (int)t[0]));
+    } else {
     unsigned long long dead[P];
 #pragma unroll
     for (int k = 0; k < P; ++k) dead[k] = 0;
@@ -266,17 +338,6 @@ struct OpenList {
       upTo = wlane(upTo, (uint32_t)lb, sb);
     }
     const uint32_t place = upTo + before;
-    if constexpr (P == 1) {
-      // places up to 63 + 48 fit the buffer: no lane needs to be left out, those that leave go to its end
-      buf[pick(dead[0], 127u, pos[0])] = make_uint2(t[0], n[0]);
-      lds_store_where(enters, &buf[place], tb, packed);
-      wave_sync();
-      const uint2 e = buf[lane];
-      front = make_uint2(buf[row].y, buf[row + 1].x);
-      meanwhile();
-      t[0] = lane < size ? e.x : kEmpty;
-      n[0] = lane < size ? e.y : kNone;
-    } else {
       unsigned long long moves[P];
       static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA { constexpr int k = decltype(K)::value; moves[k] = lanes_where(t[k] != kEmpty) & ~dead[k]; });
       uint32_t nt[P], nn[P];
@@ -299,11 +360,11 @@ struct OpenList {
         wave_sync();
       });
       static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA { constexpr int k = decltype(K)::value; t[k] = nt[k]; n[k] = nn[k]; });
-    }
     wave_sync();
     front.x = row < size ? front.x : kNone;
     front.y = row + 1 < size ? front.y : kEmpty;
     return front;
+    }
   }
 };
 
@@ -1119,7 +1180,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const int want = g.nodeCount + __popcll(fresh);
     // Nothing has changed yet: a list that would outgrow its registers goes on in the wider instantiation,
     // links that would outgrow LDS in the one that spills.
-    if (__builtin_expect(ol.size - (int)c + nrec > 64 * P, 0)) return kAstarGrowHeap;
+    if (__builtin_expect(ol.size - (int)c + nrec > (P == 1 ? 63 : 64 * P), 0)) return kAstarGrowHeap;
     if (!S && __builtin_expect(want > kLinksLds, 0)) return kAstarGrowLinks;
     (*pops) += c;
     // the reference carries on without the nodes that do not fit, but reports anything found
