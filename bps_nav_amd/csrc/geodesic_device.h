@@ -84,6 +84,12 @@ BPSX_DEV uint32_t wlane(uint32_t old, uint32_t v, int lane) {
   return old;
 }
 
+// The lane, for a part of the search that is entered once in a while: what is computed from it there is not worth
+// keeping in registers all the time, which the compiler would do.
+BPSX_DEV int lane_here(int lane) {
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
 // lanes from .. from + n - 1 (n < 64)
 BPSX_DEV unsigned long long lane_range(int n, int from) {
   unsigned long long r;
@@ -691,7 +697,7 @@ template <bool Lds> struct RefHeap {
   // it is the greater of its pair of siblings, and whether it moves up, and whether the last entry
   // comes to lie above it or in a leaf's place, each lane can tell from its own entry, the one
   // above it and the last.  So a pop is one round of reads and two masked stores per 64 entries.
-  template <int K> BPSX_DEV void pop_at_once() {   // K = 1, 2, 4; more than 32 K entries if K > 1
+  template <int K> BPSX_DEV void pop_at_once() {   // K = 1, 2, 4; more than 64, 128 entries if K > 1
     const int s = size;
     uint2 e[K], last = h[s];
     uint32_t above[K];
@@ -712,13 +718,14 @@ template <bool Lds> struct RefHeap {
       leaf[0] = (~0ull << (leaves - 1)) << 1;
       leaf[1] = ~0ull;
     } else {
-      there[0] = ~1ull;
-      there[1] = ~0ull;
-      there[2] = s >= 192 ? ~0ull : ~0ull >> (192 - s);
-      there[3] = s > 192 ? ~0ull >> (256 - s) : 0ull;
-      leaf[0] = 0;
-      leaf[1] = (~0ull << (leaves - 65)) << 1;
-      leaf[2] = leaf[3] = ~0ull;
+      constexpr int full = K - 2, half = K / 2 - 1;   // places that all have entries; the first 64 with one that has none below
+#pragma unroll
+      for (int k = 0; k < full; ++k) there[k] = k ? ~0ull : ~1ull;
+      there[full] = s >= 64 * (full + 1) ? ~0ull : ~0ull >> (64 * (full + 1) - s);
+      there[full + 1] = s > 64 * (full + 1) ? ~0ull >> (64 * K - s) : 0ull;
+#pragma unroll
+      for (int k = 0; k < K; ++k) leaf[k] = k < half ? 0ull : ~0ull;
+      leaf[half] = (~0ull << (leaves - 64 * half - 1)) << 1;
     }
     unsigned long long greater[K], on[K];
 #pragma unroll
@@ -731,12 +738,12 @@ template <bool Lds> struct RefHeap {
 #pragma unroll
     for (int k = 0; k < K; ++k) {
       if (k == 0) on[k] = lanes_where(((anc0 & (uint32_t)greater[0]) | (anc1 & (uint32_t)(greater[0] >> 32))) == 0) & there[k];
-      // the one above lies in the second half of the first 64 entries, and in the first and second of the next
-      else on[k] = lanes_where((above_bit & (uint32_t)(k == 2 ? on[k / 2] : on[k / 2] >> 32)) != 0) & there[k] & ~greater[k];
+      // the one above lies in the first or second half of 64 entries before these
+      else on[k] = lanes_where((above_bit & (uint32_t)(k & 1 ? on[k / 2] >> 32 : on[k / 2])) != 0) & there[k] & ~greater[k];
       const unsigned long long rises = lanes_where(e[k].x <= last.x);
       const uint32_t x = in_mask(rises) ? e[k].x : last.x, y = in_mask(rises) ? e[k].y : last.y;
       put(on[k] & lanes_where(above[k] <= last.x) & (k ? ~0ull : ~3ull), (uint32_t)(64 * k + lane) >> 1, x, y);
-      if (K < 4 || k > 0) put(on[k] & rises & leaf[k], (uint32_t)(64 * k + lane), last.x, last.y);
+      if (k >= K / 2 - 1) put(on[k] & rises & leaf[k], (uint32_t)(64 * k + lane), last.x, last.y);
     }
     size--;
     wave_sync();
@@ -782,7 +789,7 @@ template <bool Lds> struct RefHeap {
 // pass has at most 1 + 8 * 6 records).  Between replays the slot keeps the heap; during one it lies
 // over the window, which the caller has restored if it goes on with the sorted list.
 BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
-  const int lane = g.lane;
+  const int lane = lane_here(g.lane);
   const OpRec* log = g.ws->oplog;
   uint2* kept = reinterpret_cast<uint2*>(g.ws->heap_spill);
   RefHeap<true> rh(g.L->heap(), st.replaySize, lane);
@@ -859,7 +866,7 @@ BPSX_DEV void restore_window(GeoWave& g) {
 // kAstarGrowHeap before it outgrows it; otherwise it is in the slot, which holds any heap.
 template <bool Lds>
 BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops) {
-  const int lane = g.lane;
+  const int lane = lane_here(g.lane);
   GeoLds* L = g.L;
   const float H_SCALE = 0.999f;
   RefHeap<Lds> rh(Lds ? L->heap() : reinterpret_cast<uint2*>(g.ws->heap_spill), st.replaySize, lane);
@@ -870,27 +877,22 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     const uint32_t front = (uint32_t)uniform_i((int)rh.h[1].y);
     const int bi = (int)(front & 0x7ffu);
     const uint32_t bestIp = front >> 11;
-    rh.pop();
     if (bestIp == endIp) { st.lastBest = bi; return kAstarGoal; }
-    (*pops)++;
-    uint32_t nb = kNoNb;
-    float m0 = 0, m1 = 0, m2 = 0;
-    if (lane < kNvp) {
-      const AEdge e = edges[bestIp * kEdgeStride + (uint32_t)lane];
-      nb = e.nb; m0 = e.mid[0]; m1 = e.mid[1]; m2 = e.mid[2];
-    }
+    // what the expansion needs from HBM is asked for before the heap is set in order
+    const AEdge edge = edges[bestIp * kEdgeStride + (uint32_t)(lane & (kRowLanes - 1))];
     const float4 b = g.node(bi);
+    rh.pop();
+    (*pops)++;
+    const uint32_t nb = edge.nb;
+    float m0 = edge.mid[0], m1 = edge.mid[1], m2 = edge.mid[2];
     const uint32_t bucket = GeoWave::hash(nb);
     uint32_t chainHead;
-    const bool valid = nb != kNoNb;
-    const uint32_t at = g.find<true>(lanes_where(valid), nb, bucket, &chainHead);
-    const bool known = at != kChainEnd;
-    int ni = (int)(GeoWave::node4_at<true>(at) >> 2);
-    float oldCost = 0;
-    if (known) {
-      const float4 pc = g.node(ni);
-      m0 = pc.x; m1 = pc.y; m2 = pc.z; oldCost = pc.w;
-    }
+    const unsigned long long valid = lanes_where(nb != kNoNb) & ((1ull << kNvp) - 1ull);
+    const uint32_t at = g.find<true>(valid, nb, bucket, &chainHead);
+    const unsigned long long known = lanes_where(at != kChainEnd);
+    uint32_t ni4 = GeoWave::node4_at<true>(at);
+    const float4 pc = g.node((int)OpenList::pick(known, ni4 >> 2, 0u));
+    m0 = in_mask(known) ? pc.x : m0; m1 = in_mask(known) ? pc.y : m1; m2 = in_mask(known) ? pc.z : m2;
     const float cx = m0 - b.x, cy = m1 - b.y, cz = m2 - b.z;
     const float ex = endPos[0] - m0, ey = endPos[1] - m1, ez = endPos[2] - m2;
     float curCost, toEnd;
@@ -899,32 +901,30 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     const float cost = last ? b.w + curCost * 1.0f + toEnd * 1.0f : b.w + curCost * 1.0f;
     const float heuristic = last ? 0.0f : toEnd * H_SCALE;
     const float total = cost + heuristic;
-    const bool update = valid && !(known && total >= oldCost + heuristic);
+    const unsigned long long update = valid & ~(known & lanes_where(total >= pc.w + heuristic));
     // new nodes take consecutive indices in edge order; those that share a bucket are chained one after the other
-    unsigned long long fresh = lanes_where(update && !known);
+    const unsigned long long fresh = update & ~known;
     const int want = g.nodeCount + __popcll(fresh);
     if (want > kMaxNodes) { st.outOfNodes = true; return kAstarEmpty; }   // reported as failure whatever follows
-    if (update && !known) ni = g.nodeCount + (int)__builtin_amdgcn_mbcnt_lo((uint32_t)fresh, 0u);
+    ni4 = OpenList::pick(fresh, 4u * ((uint32_t)g.nodeCount + __builtin_amdgcn_mbcnt_lo((uint32_t)fresh, 0u)), ni4);
     g.nodeCount = want;
-    while (fresh) {
-      const int src = first_lane(fresh);
-      fresh = without_lane(fresh, src);
-      const uint32_t head = L->first[bucket];
-      g.set_links<true>(1ull << src, 4u * (uint32_t)ni, make_link(nb, head));
-      lds_store_where(1ull << src, &L->first[bucket], GeoWave::offset_of<true>(4u * (uint32_t)ni));
+    const uint32_t own = GeoWave::offset_of<true>(ni4);
+    for (unsigned long long rest = fresh; rest;) {
+      g.set_links<true>(rest, ni4, make_link(nb, chainHead));
+      lds_store_where(rest, &L->first[bucket], own);
+      wave_sync();
+      chainHead = L->first[bucket];
+      rest &= lanes_where(chainHead != own);   // another of the bucket has overwritten it at the chain's head: behind that
       wave_sync();
     }
-    uint32_t ni4 = 4u * (uint32_t)ni;
-    asm("" : "+v"(ni4));
-    g.keep_node(lanes_where(update), ni4, make_float4(m0, m1, m2, cost), (uint32_t)bi + 1u);
-    if (kAllLds) lds_store_where(lanes_where(update), lds_address(L->w_node) + (ni4 << 2), make_float4(m0, m1, m2, cost));
+    g.keep_node(update, ni4, make_float4(m0, m1, m2, cost), (uint32_t)bi + 1u);
+    if (kAllLds) lds_store_where(update, lds_address(L->w_node) + (ni4 << 2), make_float4(m0, m1, m2, cost));
     wave_sync();
-    const uint32_t packed = (uint32_t)ni | (nb << 11);
-    const unsigned long long was = lanes_where(known);
-    for (unsigned long long upd = lanes_where(update); upd;) {
+    const uint32_t packed = (ni4 >> 2) | (nb << 11);
+    for (unsigned long long upd = update; upd;) {
       const int src = first_lane(upd);
       upd = without_lane(upd, src);
-      rh.update(((was >> src) & 1ull) != 0, __float_as_uint(lane_f(total, src)), rlane(packed, src));
+      rh.update(((known >> src) & 1ull) != 0, __float_as_uint(lane_f(total, src)), rlane(packed, src));
     }
   }
 }
@@ -954,7 +954,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
 template <bool S, int P>
 BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops,
                              bool frontResolved) {
-  const int lane = g.lane;
+  const int lane = lane_here(g.lane);
   GeoLds* L = g.L;
   const float H_SCALE = 0.999f;
   const float e0 = endPos[0], e1 = endPos[1], e2 = endPos[2];
@@ -985,18 +985,16 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
   // 65536 over mixed scenes 3740 and 3233; a reset of 2048 over mazes 655 and 525.)
   // The next pass's edge records are asked for as soon as its nodes are known, before it is known how many of them
   // can be taken.  What a pass stores in HBM goes out while the list's entries come back from LDS: the wait
-  // for the records is one for all that was asked for before.  Where a wavefront has a search's whole
-  // links in LDS, and few others next to it, what a pass stores in LDS goes out behind that request, for
-  // whose time a lone search has it for nothing.  (Steps of 1024 agents over room plans 693 -> 656 us, of 510
-  // in two groups 1327 -> 1230, a reset of 2048 over mazes 525 -> 495; without that delay also of
-  // 16384 over mazes 902 -> 883, of 65536 over mixed scenes 3222 -> 3150, with it 910 and 3185.)
+  // for the records is one for all that was asked for before.  What a pass stores in LDS goes out behind that
+  // request, for whose time a lone search has it for nothing.  (Steps of 1024 agents over room plans 693 -> 656 us,
+  // of 510 in two groups 1327 -> 1230, of 16384 over mazes 902 -> 883 and, with the stores in LDS so late, 845 -> 829,
+  // of 65536 over mixed scenes 3222 -> 3150 and 2992 -> 2913, a reset of 2048 over mazes 525 -> 495.)
   struct {
     unsigned long long updated, fresh;   // lanes of updated nodes, of new ones among them
     uint32_t node4, link;                // the node, its link
     uint16_t* chain;
     float4 node;
   } late;
-  constexpr bool kLate = kLinksLds >= kMaxNodes;
   late.updated = late.fresh = 0;
   late.node4 = late.link = 0;
   late.chain = L->first;
@@ -1005,7 +1003,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     // The new nodes insert all at once in front of the chain head their lookup saw.  Of several
     // that share a bucket one store wins; the others see that when the head that is read back has come
     // (looked at below, after the stores that need not wait for it).
-    if (kLate) g.clear_marks();
+    g.clear_marks();
     const uint32_t own = GeoWave::offset_of<S>(late.node4);
     g.set_links<S>(late.fresh, late.node4, late.link);
     lds_store_where(late.fresh, late.chain, own);
@@ -1030,7 +1028,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const uint32_t ip = cand >> 11;
     static_assert(kEdgeStride * sizeof(AEdge) == 128, "a polygon's records");
     const AEdge edge = *reinterpret_cast<const AEdge*>(edges_of + ((ip << 7) | (uint32_t)(el << 4)));
-    if (kLate) insert();
+    insert();
     FM(1);
     if (st.logEnd > kOpLogCap - (1 + kRows * kNvp)) return kAstarLogFull;
     // ---- how many entries at the front are each the only one with their total, and not the goal
@@ -1212,13 +1210,11 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       st.logEnd += 1 + nrec;
     };
     FM(8);
-    if (!kLate) insert();
     FM(9);
     // ---- the open list: the committed entries leave, the updates enter
     const uint2 front = ol.template merge<P>(L->entries(), (int)c, upd, upd & known, tb, packed, lane, row, store);
     cand = front.x;
     nextTotal = front.y;
-    if (!kLate) g.clear_marks();
     FM(10);
     return kAstarOn;
   };
@@ -1236,7 +1232,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
 // when the reference would report anything but plain DT_SUCCESS.
 BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev& s, uint32_t startIp, uint32_t endIp,
                    const float* startPos, const float* endPos, uint32_t* pops) {
-  const int lane = g.lane;
+  const int lane = lane_here(g.lane);
   if (startIp == endIp) {
     if (lane == 0) F->corridor[0] = (uint16_t)startIp;
     wave_sync();
@@ -1359,28 +1355,71 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
 
 // String pulling over F->corridor[0..n) and the summed length; +inf for every outcome the
 // reference maps to "no path" (straight path of 256 points or more, missing portal).
+// A serial walk over the corridor's portals, bound by its instructions.  The tests of one portal are made at
+// once, by a lane each: five areas, of which one comparison of all lanes says what a portal
+// changes, where each test by all lanes alike and a branch behind it came to 600 cycles a portal.  The corridor's
+// edges are compared in registers, and its two end points projected next to each other, a lane
+// per edge.  (Of a search of 500 nodes over a maze, whose corridor has 72 polygons, 40 us of 390 went here.  Steps of
+// 64 agents 170 -> 161 us, of 1024 over room plans 651 -> 634, of 3007 fleeing ones 656 -> 566, a reset
+// of 2048 over mazes 483 -> 463.)
 BPSX_DEV float funnel_length(int lane, FunnelLds* F, const NavData& nav, const SceneDev& s, int n, const float* startPos,
                              const float* endPos) {
   const float INF = __int_as_float(0x7f800000);
+  lane = lane_here(lane);
   // gather the portals of the corridor, 64 at a time
   bool missing = false;
   for (int i = lane; i + 1 < n; i += 64) {
     const PolyRec& r = nav.polys[s.poly_base + F->corridor[i]];
-    const uint32_t to = F->corridor[i + 1];
+    const uint32_t* w = reinterpret_cast<const uint32_t*>(&r);
+    static_assert(offsetof(PolyRec, nei) == 72 && offsetof(PolyRec, nv) == 98, "words of a record");
+    const uint32_t codes[3] = {w[18], w[19], w[20]};
+    const int nv = (int)((w[24] >> 16) & 0xffu);
+    const uint32_t want = (uint32_t)F->corridor[i + 1] + 1u;   // below 0x8000: neither a wall nor a tile border
     int e = -1;
-    for (int k = 0; k < r.nv; ++k)
-      if (r.nei[k] && !(r.nei[k] & 0x8000) && (uint32_t)(r.nei[k] - 1) == to) { e = k; break; }
-    if (e < 0) { missing = true; continue; }
-    const float* l = r.v[e];
-    const float* rr = r.v[(e + 1) % r.nv];
+    static_for<0, kNvp>([&](auto K) BPSX_INLINE_LAMBDA {
+      constexpr int k = kNvp - 1 - decltype(K)::value;   // the first that fits
+      e = k < nv && ((codes[k >> 1] >> (16 * (k & 1))) & 0xffffu) == want ? k : e;
+    });
+    missing |= e < 0;
+    const float* l = r.v[e < 0 ? 0 : e];
+    const float* rr = r.v[e + 1 < nv ? e + 1 : 0];
     float* p = F->portals[i];
     p[0] = l[0]; p[1] = l[1]; p[2] = l[2]; p[3] = rr[0]; p[4] = rr[1]; p[5] = rr[2];
   }
+  // closestPointOnPolyBoundary of the start point in the first polygon (lanes 0 to 7 of sixteen) and of the end point
+  // in the last one (lanes 8 to 15): the point itself when inside (xz), else its projection onto the first of
+  // the nearest edges; lane j has the edge from vertex j.
+  float cs[3], ce[3];
+  {
+    const bool atEnd = (lane & 8) != 0;
+    const int j = lane & 7;
+    const float pos[3] = {atEnd ? endPos[0] : startPos[0], atEnd ? endPos[1] : startPos[1], atEnd ? endPos[2] : startPos[2]};
+    const PolyRec& r = nav.polys[s.poly_base + F->corridor[atEnd ? n - 1 : 0]];
+    const int nv = r.nv;
+    const float* va = r.v[j < nv ? j : 0];
+    const float* vb = r.v[j + 1 < nv ? j + 1 : 0];
+    const float a[3] = {va[0], va[1], va[2]}, b[3] = {vb[0], vb[1], vb[2]};
+    const bool crosses = j < nv && ((b[2] > pos[2]) != (a[2] > pos[2])) && (pos[0] < (a[0] - b[0]) * (pos[2] - b[2]) / (a[2] - b[2]) + b[0]);
+    float t;
+    const float d = dist_pt_seg_sqr2d(pos[0], pos[2], a, b, t);
+    // the smallest by their bits, which order distances; a NaN is never smaller than what came before, so it
+    // only counts as the first
+    uint32_t key = d == d ? __float_as_uint(d) : j == 0 ? 0u : 0xfffffffeu;
+    key = j < nv ? key : 0xffffffffu;
+    const uint32_t nearest = Row::umin(key);
+    const unsigned long long inside = lanes_where(crosses), first = lanes_where(key == nearest);
+    const float on[3] = {a[0] + (b[0] - a[0]) * t, a[1] + (b[1] - a[1]) * t, a[2] + (b[2] - a[2]) * t};
+    const int ls = first_lane(first & 0xffull), le = first_lane(first & 0xff00ull);
+    const bool sIn = __popcll(inside & 0xffull) & 1, eIn = __popcll(inside & 0xff00ull) & 1;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      cs[k] = sIn ? startPos[k] : lane_f(on[k], ls);
+      ce[k] = eIn ? endPos[k] : lane_f(on[k], le);
+    }
+  }
+  if (lane < 6) F->portals[n - 1][lane] = lane == 0 || lane == 3 ? ce[0] : lane == 1 || lane == 4 ? ce[1] : ce[2];   // where the walk ends
   wave_sync();
   if (lanes_where(missing)) return INF;
-  float cs[3], ce[3];
-  closest_on_poly_boundary(nav.polys[s.poly_base + F->corridor[0]], startPos, cs);
-  closest_on_poly_boundary(nav.polys[s.poly_base + F->corridor[n - 1]], endPos, ce);
   // straight-path points are only needed pairwise: keep the last one and the running length.
   // Every lane computes the same values; the conditions are taken through a ballot so that the
   // control flow is the scalar unit's (no lane masks, no copies at the joins).
@@ -1406,54 +1445,75 @@ BPSX_DEV float funnel_length(int lane, FunnelLds* F, const NavData& nav, const S
     if (isEnd) finished = true;
   };
   if (n > 1) {
-    float apex[3] = {cs[0], cs[1], cs[2]}, pl[3] = {cs[0], cs[1], cs[2]}, pr[3] = {cs[0], cs[1], cs[2]};
+    // The funnel's sides are kept relative to its apex, in the lanes that test them: lanes 0 to 3 have (side,
+    // point tested against it) = (right, portal's right), (left, right), (left, left), (right, left), lane 4 the
+    // portal's own right and left.  An area's sign is turned in lanes 0, 3 and 4, so that "not outside" (lanes 0,
+    // 2) reads >= 0 and "not across" (1, 3, 4) > 0.
+    const uint32_t turn = lane == 0 || lane == 3 || lane == 4 ? 0x80000000u : 0u;
+    const float* tested = &F->portals[0][lane < 2 ? 3 : 0];
+    float ax = cs[0], ay = cs[1], az = cs[2];
+    float sx = ax - ax, sy = ay - ay, sz = az - az;   // the side of lanes 0 to 3 (0, or NaN for an apex that is not finite, as the difference is)
+    const float thr = (1.0f / 16384.0f) * (1.0f / 16384.0f);
+    auto sides_at_apex = [&]() { return (uint32_t)lanes_where(sx * sx + sy * sy + sz * sz < thr); };   // vequal(apex, side)
+    uint32_t atApex = sides_at_apex();
     int apexIndex = 0, leftIndex = 0, rightIndex = 0;
-    bool leftIsEnd = false, rightIsEnd = false;  // "poly ref == 0" of the reference
-    for (int i = 0; i < n && !finished; ++i) {
-      float left[3], right[3];
-      if (i + 1 < n) {
-        const float* p = F->portals[i];
-        left[0] = p[0]; left[1] = p[1]; left[2] = p[2];
-        right[0] = p[3]; right[1] = p[4]; right[2] = p[5];
-        if (i == 0) {
-          float t;
-          if (all(dist_pt_seg_sqr2d(apex[0], apex[2], left, right, t) < 0.001f * 0.001f)) continue;
-        }
-      } else {
-        left[0] = right[0] = ce[0]; left[1] = right[1] = ce[1]; left[2] = right[2] = ce[2];
-      }
-      if (all(tri_area2d(apex, pr, right) <= 0.0f)) {
-        if (all(vequal(apex, pr)) || all(tri_area2d(apex, pl, right) > 0.0f)) {
-          pr[0] = right[0]; pr[1] = right[1]; pr[2] = right[2];
-          rightIsEnd = !(i + 1 < n);
-          rightIndex = i;
-        } else {
-          apex[0] = pl[0]; apex[1] = pl[1]; apex[2] = pl[2];
+    int leftMoved = 0, rightMoved = 0;       // since the apex last moved: the side is a portal's point
+    int leftLast = -1, rightLast = -1;       // the portal whose point the side was last: the last one is "poly ref == 0" of the reference
+    int i = 0;
+    {
+      const float* p = F->portals[0];
+      float t;
+      const float l[3] = {p[0], p[1], p[2]}, r[3] = {p[3], p[4], p[5]};
+      if (all(dist_pt_seg_sqr2d(ax, az, l, r, t) < 0.001f * 0.001f)) i = 1;
+    }
+    while (i < n) {
+      const float* c = tested + 6 * i;
+      const float px = c[0], py = c[1], pz = c[2];
+      const float cx = px - ax, cz = pz - az;
+      // lane 4 has the portal's right for its side: lane 0's point (into the second four lanes of sixteen)
+      const float bx = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(sx), __float_as_int(cx), 0x114 /* row_shr:4 */, 0xf, 0x2, false));
+      const float bz = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(sz), __float_as_int(cz), 0x114 /* row_shr:4 */, 0xf, 0x2, false));
+      const float area = __uint_as_float(__float_as_uint(cx * bz - bx * cz) ^ turn);
+      const uint32_t m = ((uint32_t)lanes_where(area >= 0.0f) & 0x05u) | ((uint32_t)lanes_where(area > 0.0f) & 0x1au);
+      const int at = i++;
+      if (!(m & 0x05u)) continue;   // both points outside: the funnel stays as it is
+      // the right point, then the left one with the right side as it then is
+      const uint32_t rightIn = m & 1u, leftIn = m & 4u;
+      const uint32_t across = rightIn ? m >> 4 : m >> 3;   // the left point against that right side
+      const uint32_t rightStops = rightIn & ~(atApex | (m >> 1)), leftStops = leftIn & ~(atApex | (across << 2));
+      if (__builtin_expect((rightStops | leftStops) != 0, 0)) {
+        if (rightStops) {
           apexIndex = leftIndex;
-          append(apex, leftIsEnd);
-          if (finished) break;
-          pl[0] = pr[0] = apex[0]; pl[1] = pr[1] = apex[1]; pl[2] = pr[2] = apex[2];
-          leftIndex = rightIndex = apexIndex;
-          i = apexIndex;
-          continue;
-        }
-      }
-      if (all(tri_area2d(apex, pl, left) >= 0.0f)) {
-        if (all(vequal(apex, pl)) || all(tri_area2d(apex, pr, left) < 0.0f)) {
-          pl[0] = left[0]; pl[1] = left[1]; pl[2] = left[2];
-          leftIsEnd = !(i + 1 < n);
-          leftIndex = i;
+          if (leftMoved) { const float* p = F->portals[leftIndex]; ax = p[0]; ay = p[1]; az = p[2]; }
         } else {
-          apex[0] = pr[0]; apex[1] = pr[1]; apex[2] = pr[2];
+          if (rightIn) { rightIndex = rightLast = at; rightMoved = 1; }
           apexIndex = rightIndex;
-          append(apex, rightIsEnd);
-          if (finished) break;
-          pl[0] = pr[0] = apex[0]; pl[1] = pr[1] = apex[1]; pl[2] = pr[2] = apex[2];
-          leftIndex = rightIndex = apexIndex;
-          i = apexIndex;
-          continue;
+          if (rightMoved) { const float* p = F->portals[rightIndex] + 3; ax = p[0]; ay = p[1]; az = p[2]; }
         }
+        const float apex[3] = {ax, ay, az};
+        append(apex, (rightStops ? leftLast : rightLast) + 1 == n);
+        if (finished) break;
+        sx = ax - ax; sy = ay - ay; sz = az - az;
+        atApex = sides_at_apex();
+        leftMoved = rightMoved = 0;
+        leftIndex = rightIndex = apexIndex;
+        i = apexIndex + 1;
+        continue;
       }
+      // the sides that move: of each lane, the point that its side moves to
+      const float cy = py - ay;
+      const float nx = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(cx), 0x28 /* quad_perm:[0,2,2,0] */, 0xf, 0xf, true));
+      const float ny = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(cy), 0x28 /* quad_perm:[0,2,2,0] */, 0xf, 0xf, true));
+      const float nz = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(cz), 0x28 /* quad_perm:[0,2,2,0] */, 0xf, 0xf, true));
+      const unsigned long long moves = 9u * rightIn + 6u * (leftIn >> 2);
+      sx = in_mask(moves) ? nx : sx;
+      sy = in_mask(moves) ? ny : sy;
+      sz = in_mask(moves) ? nz : sz;
+      atApex = sides_at_apex();
+      if (rightIn) rightIndex = rightLast = at;
+      if (leftIn) leftIndex = leftLast = at;
+      rightMoved |= (int)rightIn;
+      leftMoved |= (int)leftIn;
     }
   }
   if (!finished) {
