@@ -74,10 +74,9 @@ int dev_alloc(T** p, size_t count) {
 // GPU, held until the process ends: the queries built from the caller's arrays, the queue
 // counters, and the node pools of the kStaticBlocks * 2 wavefronts that serve the queue.
 namespace {
-// As many pools as k_geodesic_few keeps wavefronts on the device (three on each of 256 CUs): every
-// query of a call of that size has a wavefront of its own, larger calls share them in blocks of
-// k_geodesic.  (Those would be served sooner by as many wavefronts of k_geodesic_few: 1000, 4096 queries
-// over room plans 364, 947 us against 358, 925; over mazes 2576, 5706 against 2228, 4512.)
+// As many pools as k_geodesic_few keeps searches on the device (three on each of 256 CUs): every
+// query of a call of that size has a block of its own, larger calls share them in blocks of
+// k_geodesic.
 // The array is part of the library's device image: every process that loads the library holds it on
 // each GPU it uses, whether it makes such calls or not.
 constexpr uint32_t kStaticBlocks = 384;
@@ -220,7 +219,7 @@ struct bpsx_sim {
   std::vector<Group> groups;
   GeoPool geo{};                      // of the steps: what their envs can fill
   uint32_t snap_blocks = 0;
-  uint32_t max_geo_blocks = 0, max_few_blocks = 0, compute_units = 0;   // what the device holds at once, whatever the number of envs
+  uint32_t max_geo_blocks = 0, max_few_blocks = 0, max_mid_blocks = 0, compute_units = 0;   // what the device holds at once, whatever the number of envs
   uint32_t* d_error = nullptr;
   uint64_t* d_counters = nullptr;
   float turn_left[4], turn_right[4];
@@ -617,6 +616,10 @@ int bpsx_finalize(bpsx_sim* sim) {
   sim->geo.blocks = std::max(1u, blocks);
   sim->max_few_blocks = (uint32_t)prop.multiProcessorCount * geodesic_few_blocks_per_cu();
   sim->geo.few_blocks = std::min(sim->max_few_blocks, sim->geo.blocks * 2u);
+  sim->max_mid_blocks = (uint32_t)prop.multiProcessorCount * geodesic_mid_blocks_per_cu();
+  sim->geo.mid_blocks = std::min(sim->max_mid_blocks, sim->geo.blocks * 2u);
+  sim->geo.mid_steps = sim->max_mid_blocks * 9u / 4u;
+  sim->geo.mid_batch = sim->max_mid_blocks * 5u / 4u;
   sim->snap_blocks = (uint32_t)prop.multiProcessorCount * 8u;   // of four wavefronts: what the device holds at once
   if ((rc = sim->alloc(&sim->geo.slots, (size_t)sim->geo.blocks * 2))) return rc;   // one per wavefront
 
@@ -879,15 +882,16 @@ static int batch_reserve(bpsx_sim* sim, size_t bytes) {
   sim->batch_bytes = bytes;
   return BPSX_OK;
 }
-// Node pools for a batch of n path queries: one per query while k_geodesic_few serves it, else as
-// many blocks of k_geodesic as the device holds at once, or one per query where that is less.  The
+// Node pools for a batch of n path queries: one per query while k_geodesic_few serves it, else for as
+// many blocks of k_geodesic_mid or k_geodesic as the device holds at once, or one per query where that is less.  The
 // steps' own pools serve if they are enough (a simulator has no more of them than envs in a group);
 // otherwise the batch has pools of its own, kept until a larger batch or bpsx_destroy replaces them
 // (at most 0.7 GB); where the device has no room for those, the steps' pools serve it all the same.
 // (1000 pairs over a maze, simulator of 4 envs, so far served by 4 blocks: 131 -> 2.3 ms a call.)
 static int batch_reserve_slots(bpsx_sim* sim, uint32_t n, GeoPool* out) {
   const bool few = n <= sim->max_few_blocks;
-  const uint32_t want = few ? n : 2u * std::min(sim->max_geo_blocks, n);
+  const uint32_t mid = std::min(sim->max_mid_blocks, n);
+  const uint32_t want = few ? n : n <= sim->geo.mid_batch ? mid : 2u * std::min(sim->max_geo_blocks, n);
   *out = sim->geo;
   if (want > sim->geo.blocks * 2u) {
     if (want > sim->batch_slots) {
@@ -903,6 +907,7 @@ static int batch_reserve_slots(bpsx_sim* sim, uint32_t n, GeoPool* out) {
     }
     out->slots = sim->d_batch_slots;
     out->blocks = want / 2u;
+    out->mid_blocks = std::min(mid, want);
   }
   out->few_blocks = few ? n : 0u;
   return BPSX_OK;
@@ -1133,7 +1138,7 @@ int bpsx_geodesic_static(bpsx_sim* sim, uint32_t scene, const float* start_xyz, 
   // The counters are rewritten by a kernel at the start of every call; node pools and queries
   // are written before they are read.  Nothing else of the previous call's contents is used.
   launch_geodesic_batch(sim->nav, scene_entry(sim, scene), start_xyz, start_ref, end_xyz, end_ref, n, d_q, d_counts, out_dist,
-                        GeoPool{d_slots, std::min(kStaticBlocks, std::max(1u, (n + 1) / 2)), n <= kStaticBlocks * 2u ? n : 0u}, sim->d_counters,
+                        GeoPool{d_slots, std::min(kStaticBlocks, std::max(1u, (n + 1) / 2)), n <= kStaticBlocks * 2u ? n : 0u, 0u, 0u, 0u}, sim->d_counters,
                         (hipStream_t)hip_stream);
   HIP_TRY(hipGetLastError());
   return BPSX_OK;

@@ -7,7 +7,8 @@
 // frontier of A* is narrow), so LDS holds what is hot and small and HBM holds the rest:
 //   - the open list in registers: sorted by total, up to 256 entries (OpenList), which lets a
 //     pass expand up to kRows nodes at once (astar_fast); when totals tie, the reference's binary
-//     heap is rebuilt from a log of the list's operations (RefHeap, replay_log), and a search whose
+//     heap is rebuilt from a log of the list's operations (RefHeap, replay_log) or has been kept from it all
+//     along by a second wavefront (follow), and a search whose
 //     list outgrows the registers, or has a tie of more than 64, goes on with that heap,
 //   - the hash heads of the node pool,
 //   - for the first kLinksLds nodes one word with the polygon id and the hash chain link,
@@ -29,7 +30,8 @@
 // getEdgeMidPoint); DetourNode.cpp:50-200 (node pool, heap order); PathFinder.cpp:473-541.
 //
 // The sizes of the LDS structures are build parameters (BPSX_LINKS_LDS,
-// BPSX_WINDOW, BPSX_HASH, BPSX_TAG_SLOTS), and everything that depends on them lives in namespace
+// BPSX_WINDOW, BPSX_HASH, BPSX_TAG_SLOTS; BPSX_FOLLOWER: a second wavefront keeps the reference's heap),
+// and everything that depends on them lives in namespace
 // bpsx::BPSX_GEO_NS (default geo): the file can be included again with other values and
 // another namespace name to get a second instantiation of the same search.
 #include "nav_device.h"
@@ -108,6 +110,9 @@ BPSX_DEV int first_lane(unsigned long long mask) {
 // early way out then goes through copies of the loop's state and tests of flags.
 typedef float Float4 __attribute__((ext_vector_type(4)));
 BPSX_DEV uint32_t lds_address(const void* p) { return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p; }
+BPSX_DEV uint32_t lds_word(const uint32_t* p) {   // as another wavefront of the block may have written it
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
 BPSX_DEV void lds_store_where(unsigned long long mask, uint2* p, uint32_t x, uint32_t y) {
   const unsigned long long v = ((unsigned long long)y << 32) | x;
   asm volatile("s_mov_b64 exec, %0\n\tds_write_b64 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(v) : "memory");
@@ -385,6 +390,8 @@ struct AstarState {
   uint32_t replayRoot;   // packed node of the entry at its root after a replay
 };
 
+constexpr uint32_t kFollowEnd = 0xffffu, kFollowQuit = 0xffffffffu;   // see follow
+
 enum AstarExit { kAstarOn = -1, kAstarEmpty = 0, kAstarGoal = 1, kAstarGrowLinks = 2, kAstarGrowHeap = 3, kAstarTie = 4, kAstarLogFull = 5 };
 
 // Two correctly rounded square roots, the values sqrtf returns on the host, of arguments that are zero or
@@ -448,6 +455,10 @@ constexpr uint32_t kChainEnd = 4u * (uint32_t)kLinksLds;
 constexpr uint32_t kEndWord = kNoPoly | (kChainEnd << 16);
 static_assert(4 * (kMaxNodes + 1) <= 0xffff, "offsets of links have 16 bits");
 constexpr bool kAllLds = kWindow >= kMaxNodes;   // every node is kept in LDS, and none in HBM
+#ifndef BPSX_FOLLOWER
+#define BPSX_FOLLOWER 0
+#endif
+constexpr bool kFollower = BPSX_FOLLOWER;   // a second wavefront keeps the reference's heap up to date (follow)
 static_assert(!kAllLds || kLinksLds >= kMaxNodes, "a pool in LDS has its links there too");
 #ifndef BPSX_TAG_SLOTS
 #define BPSX_TAG_SLOTS 256
@@ -463,7 +474,7 @@ static_assert((kWindow & (kWindow - 1)) == 0 && kWindow >= 2 * kNvp, "window mus
 
 // LDS of one wavefront.
 struct GeoLds {
-  uint16_t first[kHashSize];
+  alignas(16) uint16_t first[kHashSize];
   // Node links: polygon index | offset of the next node's link in the hash chain << 16.  Behind them the
   // marks of which row of a pass updates a polygon first (see astar_fast), all kEndWord between passes
   // and while chains are walked: the first of them is the word that ends every chain.  A pass's
@@ -472,10 +483,20 @@ struct GeoLds {
   alignas(16) float4 w_node[kWindow];   // position, cost
   BPSX_DEV uint32_t* marks() { return n_link + kLinksLds; }
   BPSX_DEV uint2* entries() { return reinterpret_cast<uint2*>(n_link + kLinksLds); }   // 128 of them over the marks
+#if BPSX_FOLLOWER
+  // What the two wavefronts of a search share (see follow): how far the log has arrived, the heap and its size,
+  // the search's state, how far the log has been read, and the entry that a search begins with.
 #if BPSX_WINDOW >= 2048
-  // with every node in LDS: parent indices, and a place of its own for the reference's heap
-  uint2 ref_heap[64 * OpenList::kPairs + 2 * 8 * kNvp + 2];
+  // Next to every node, the parent indices; where a lane without a node would store its own, `arrived`.
   uint16_t parents[kMaxNodes];
+  uint16_t arrived, unused;
+#endif
+  uint2 ref_heap[64 * OpenList::kPairs + 2 * 8 * kNvp + 2];
+  uint2 start;
+  uint32_t published, applied, heap_size;
+#if BPSX_WINDOW < 2048
+  uint16_t arrived, unused;
+#endif
   BPSX_DEV uint2* heap() { return ref_heap; }
 #else
   BPSX_DEV uint2* heap() { return entries(); }
@@ -498,6 +519,8 @@ union GeoShared {
 // Accessors take the instantiation's spill switch S: with S false, or with room in LDS for the links
 // of all nodes, every node index is below kLinksLds and no address-space branch is generated.
 struct GeoWave {
+  using Shared = GeoShared;
+  static constexpr bool kFollowed = kFollower;
   GeoLds* L;
   GeoSlot* ws;
   int lane;
@@ -509,6 +532,15 @@ struct GeoWave {
   uint32_t exactRuns;                // queries that went on with the reference's heap
   uint32_t tieReplays;               // ties resolved by replaying the operation log through the exact heap
   uint32_t pairTies;                 // passes that took two nodes of equal total in one go
+#if BPSX_FOLLOWER
+  uint32_t epoch;                    // of the search, in the upper 16 bits (see follow)
+  BPSX_DEV void publish(uint32_t word) const { lds_store_where(1ull, lds_address(&L->published), word); }
+  // until the follower has done all that the word asks for
+  BPSX_DEV void settle(uint32_t word) const {
+    while ((uint32_t)uniform_i((int)lds_word(&L->applied)) != word) __builtin_amdgcn_s_sleep(1);
+    wave_sync();
+  }
+#endif
 
   // ---------------------------------------------------------------- node pool
   // A node's index is handled as four times itself, the offset of its word among the links.  Offset of its link
@@ -557,6 +589,29 @@ struct GeoWave {
                  :: "s"(mask), "v"(i4 << 2), "v"(v), "s"(ws->nodes), "v"(i4 >> 1), "v"(parent), "s"(ws->parents) : "memory");
 #endif
   }
+#if BPSX_FOLLOWER
+  // A pass's updated nodes and its records of the log, at `offset` bytes, and as `arrived` the number of records before
+  // the pass: those were stored before it asked for its edge records, for which it has waited, so they
+  // are in the L2.  All lanes that store a record store that number, or only the header's, which
+  // has no node, where its parent index would go.
+  BPSX_DEV void keep_pass(unsigned long long mask, unsigned long long header, uint32_t i4, float4 n, uint32_t parent, uint32_t before, uint32_t offset,
+                          uint32_t key, uint32_t word) const {
+    const unsigned long long r = ((unsigned long long)word << 32) | key;
+#if BPSX_WINDOW >= 2048
+    (void)n;
+    static_assert(kLinksLds == kMaxNodes && offsetof(GeoLds, arrived) == offsetof(GeoLds, parents) + kChainEnd / 2, "the header's lane has kChainEnd for a node");
+    const uint32_t p = wlane_at<63>(parent, before);
+    asm volatile("s_mov_b64 exec, %0\n\tglobal_store_dwordx2 %1, %2, %3\n\tds_write_b16 %4, %5\n\ts_mov_b64 exec, -1"
+                 :: "s"(mask | header), "v"(offset), "v"(r), "s"(ws->oplog), "v"(lds_address(L->parents) + (i4 >> 1)), "v"(p) : "memory");
+#else
+    const Float4 v = {n.x, n.y, n.z, n.w};
+    asm volatile("s_mov_b64 exec, %0\n\tglobal_store_dwordx4 %1, %2, %3\n\tglobal_store_short %4, %5, %6\n\t"
+                 "s_mov_b64 exec, %7\n\tglobal_store_dwordx2 %8, %9, %10\n\tds_write_b16 %11, %12\n\ts_mov_b64 exec, -1"
+                 :: "s"(mask), "v"(i4 << 2), "v"(v), "s"(ws->nodes), "v"(i4 >> 1), "v"(parent), "s"(ws->parents),
+                    "s"(mask | header), "v"(offset), "v"(r), "s"(ws->oplog), "v"(lds_address(&L->arrived)), "v"(before) : "memory");
+#endif
+  }
+#endif
   // the multiply as the full-rate 24-bit instruction (polygon indices have 15 bits)
   static BPSX_DEV uint32_t hash(uint32_t ip) {
     uint32_t m;
@@ -568,7 +623,11 @@ struct GeoWave {
     reinterpret_cast<uint4*>(L->marks())[lane] = make_uint4(kEndWord, kEndWord, kEndWord, kEndWord);
   }
   BPSX_DEV void clear() {
-    for (int i = lane; i < kHashSize; i += 64) L->first[i] = (uint16_t)kChainEnd;
+    constexpr uint32_t two = kChainEnd | (kChainEnd << 16);
+    static_assert(kHashSize % 512 == 0, "16 bytes a lane");
+    static_for<0, kHashSize / 512>([&](auto K) BPSX_INLINE_LAMBDA {
+      reinterpret_cast<uint4*>(L->first)[64 * decltype(K)::value + lane] = make_uint4(two, two, two, two);
+    });
     clear_marks();
     nodeCount = 0;
     wave_sync();
@@ -620,10 +679,10 @@ struct GeoWave {
 // a cluttered plan of 20k polygons ties with a longer list or outgrows the sorted list, and ran
 // again from its start with a heap walked level by level in HBM: 6.6 ms, against 1.5 ms for the
 // longest of the others.)
-constexpr int kHeapLds = kAllLds ? 64 * OpenList::kPairs + 2 * kRows * kNvp + 1 : (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
+constexpr int kHeapLds = kFollower ? 64 * OpenList::kPairs + 2 * kRows * kNvp + 1 : (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
 static_assert(kLinksLds % 4 == 0 && offsetof(GeoLds, w_node) == offsetof(GeoLds, n_link) + 4 * (kLinksLds + kTagSlots),
               "the marks are accessed as 16 bytes, and the heap lies over the marks and the window");
-// (383 entries, 639 of a whole block's LDS, 353 next to a whole node pool)
+// (383 entries, 353 where a second wavefront keeps it)
 static_assert(kHeapLds >= 64 * OpenList::kPairs + 2 * kRows * kNvp, "a heap with as many entries as the sorted list must fit");
 template <bool Lds> struct RefHeap {
   uint2* h;    // total bits, packed node
@@ -784,6 +843,103 @@ template <bool Lds> struct RefHeap {
   }
 };
 
+// Applies one pass of the log to the reference's heap.  The lanes hold records; the pass's begin in lane h and
+// end with the first of `headers` from there.  seen: nodes created by the passes before.  Returns the number of
+// records, header included.
+BPSX_DEV int apply_pass(RefHeap<true>& rh, uint32_t rk, uint32_t rw, unsigned long long headers, int h, int& seen) {
+  const int end = h + __builtin_ctzll(headers >> h);
+  const uint32_t hk = rlane(rk, end), hw = rlane(rw, end);
+  const int c = (int)(hk & 0xffu), nrec = (int)(hk >> 8);
+  // rows in the reference's order: the first two swap when the heap has row 1's node on top
+  const bool swap = (hw & kOpUnordered) && (uint32_t)uniform_i((int)rh.h[1].y) != (hw & 0x3ffffffu);
+  const unsigned long long mine = lane_range(nrec, h);
+  const uint32_t myRow = (rw >> 26) & 7u;
+  // the pass's new nodes are those whose index had not been given out before it
+  const unsigned long long fresh = lanes_where((int)(rw & 0x7ffu) >= seen) & mine;
+  for (int i = 0; i < c; ++i) {
+    const int row = (swap && i < 2) ? 1 - i : i;
+    rh.pop();
+    unsigned long long m = lanes_where(myRow == (uint32_t)row) & mine;
+    while (m) {
+      const int j = first_lane(m);
+      m = without_lane(m, j);
+      const uint32_t word = rlane(rw, j);
+      // a known node without an entry (closed, or its row came earlier in the pass) is pushed
+      rh.update(((fresh >> j) & 1ull) == 0, rlane(rk, j), word & 0x3ffffffu);
+    }
+  }
+  seen += __popcll(fresh);
+  return 1 + nrec;
+}
+
+#if BPSX_FOLLOWER
+// Where a search has a second wavefront to itself, that one applies the log to the reference's heap while the search
+// goes on, and a tie costs the search a question instead of a replay of all that came before.  Both are of
+// one block, so both are there until the block ends, and each wait of one is for something that the other does
+// in any case.
+//   published   written by the search: its epoch << 16 | 0 when it begins, the records of the log when it asks for the
+//               heap, kFollowEnd when it is over; kFollowQuit when there will be no more searches.
+//   arrived     written by every pass: the records of the log that may be read (GeoWave::keep_pass).
+//   applied     written by the follower: the last word of `published` that it has done all for.  The heap is the
+//               search's from then on, until it goes on with another pass.
+// A new search of the same slot writes over the log that the follower may still be fetching from: what has been
+// fetched is looked at only if the epoch is still the same afterwards.
+// Bound by the heap's operations, 0.2 us per node, which is less than the search takes per node alone.  For the
+// search it is one or two instructions a pass, and two fewer around its stores.  (With `arrived` stored apart, five
+// instructions a pass, it cost the searches without ties 2.5 %: steps of 64 agents 161 -> 165 us, a reset of 2048 over
+// mazes 471 -> 483.)
+static_assert(kOpLogCap < (int)kFollowEnd, "a count of records is told from the marks");
+BPSX_DEV void follow_init(GeoLds* L) { L->published = L->applied = kFollowEnd; }   // of a search before the first
+BPSX_DEV void follow(GeoLds* L, const GeoSlot* ws, int lane) {
+  lane = lane_here(lane);
+  RefHeap<true> rh(L->heap(), 0, lane);
+  const unsigned long long* log = reinterpret_cast<const unsigned long long*>(ws->oplog);
+  static_assert(sizeof(OpRec) == 8 && offsetof(GeoSlot, oplog) % 8 == 0, "a record is one access");
+  uint32_t done = kFollowEnd;
+  int pos = 0, seen = 1;   // of the search of done's epoch: records applied, nodes created by them
+  auto answer = [&](uint32_t word) {
+    lds_store_where(1ull, lds_address(&L->heap_size), (uint32_t)rh.size);
+    lds_store_where(1ull, lds_address(&L->applied), word);
+    done = word;
+  };
+  for (;;) {
+    const uint32_t word = (uint32_t)uniform_i((int)lds_word(&L->published));
+    if (word == kFollowQuit) return;
+    const int asked = (int)(word & 0xffffu);
+    if (asked == (int)kFollowEnd) {
+      if (word != done) answer(word);
+      __builtin_amdgcn_s_sleep(2);
+      continue;
+    }
+    if ((word ^ done) >> 16) {   // a search begins
+      wave_sync();
+      const uint2 e = L->start;
+      lds_store_where(1ull, &rh.h[1], e.x, e.y);
+      wave_sync();
+      rh.size = 1;
+      pos = 0; seen = 1;
+      done = word & 0xffff0000u;
+    }
+    wave_sync();
+    const int arrived = uniform_i((int)__hip_atomic_load(&L->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+    const int end = arrived > asked ? arrived : asked;
+    if (pos < end) {
+      const unsigned long long r = __hip_atomic_load(log + (pos + lane < end ? pos + lane : pos), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const uint32_t rk = (uint32_t)r, rw = (uint32_t)(r >> 32);
+      const unsigned long long headers = lanes_where((rw & kOpHeader) != 0) & lanes_where(pos + lane < end);
+      wave_sync();
+      if (((uint32_t)uniform_i((int)lds_word(&L->published)) ^ word) >> 16) continue;   // over, and perhaps written over
+      int h = 0;
+      while (h < 64 && (headers >> h)) h += apply_pass(rh, rk, rw, headers, h, seen);
+      pos += h;
+    }
+    if (pos != end) continue;
+    if (word != done) answer(word);
+    else __builtin_amdgcn_s_sleep(2);
+  }
+}
+#endif
+
 // Applies log records [st.synced, st.logEnd) to the reference's heap, pass by pass.  Records are
 // fetched 64 at a time, one per lane, and again when the next pass is not among them in full (a
 // pass has at most 1 + 8 * 6 records).  Between replays the slot keeps the heap; during one it lies
@@ -814,30 +970,7 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
     // the pass ends with the next header; a fetch is a round trip to HBM: one only when the pass at hand is
     // not all there
     if (pos >= base + 64 || !(headers >> (pos - base))) fetch(pos);
-    const int h = pos - base;   // its first record, or the header if it has none
-    const int end = h + __builtin_ctzll(headers >> h);
-    const uint32_t hk = rlane(rk, end), hw = rlane(rw, end);
-    const int c = (int)(hk & 0xffu), nrec = (int)(hk >> 8);
-    // rows in the reference's order: the first two swap when the heap has row 1's node on top
-    const bool swap = (hw & kOpUnordered) && (uint32_t)uniform_i((int)rh.h[1].y) != (hw & 0x3ffffffu);
-    const unsigned long long mine = lane_range(nrec, h);
-    const uint32_t myRow = (rw >> 26) & 7u;
-    // the pass's new nodes are those whose index had not been given out before it
-    const unsigned long long fresh = lanes_where((int)(rw & 0x7ffu) >= seen) & mine;
-    for (int i = 0; i < c; ++i) {
-      const int row = (swap && i < 2) ? 1 - i : i;
-      rh.pop();
-      unsigned long long m = lanes_where(myRow == (uint32_t)row) & mine;
-      while (m) {
-        const int j = first_lane(m);
-        m = without_lane(m, j);
-        const uint32_t word = rlane(rw, j);
-        // a known node without an entry (closed, or its row came earlier in the pass) is pushed
-        rh.update(((fresh >> j) & 1ull) == 0, rlane(rk, j), word & 0x3ffffffu);
-      }
-    }
-    pos += 1 + nrec;
-    seen += __popcll(fresh);
+    pos += apply_pass(rh, rk, rw, headers, pos - base, seen);
   }
   st.synced = st.logEnd;
   st.replayNodes = seen;
@@ -848,7 +981,7 @@ BPSX_DEV void replay_log(GeoWave& g, AstarState& st) {
 }
 // The window and the marks after something else has used their LDS.
 BPSX_DEV void restore_window(GeoWave& g) {
-  if (kAllLds) return;   // nothing else has
+  if (kFollower) return;   // nothing else has
   const int from = g.nodeCount > kWindow ? g.nodeCount - kWindow : 0;
   for (int i = from + g.lane; i < g.nodeCount; i += 64) {
     BPSX_KEEP_APART();
@@ -1205,8 +1338,13 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const uint32_t word = wlane_at<kHeaderLane>(packed | ((uint32_t)row << 26), headerWord);
     const auto store = [&]() BPSX_INLINE_LAMBDA {
       const uint32_t rec = __builtin_amdgcn_mbcnt_hi((uint32_t)(upd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)upd, (uint32_t)st.logEnd));
+#if BPSX_FOLLOWER
+      static_assert(kHeaderLane == 63);
+      g.keep_pass(upd, 1ull << kHeaderLane, ni4, late.node, (uint32_t)bi + 1u, (uint32_t)st.logEnd, rec * (uint32_t)sizeof(OpRec), key, word);
+#else
       store_where(upd | (1ull << kHeaderLane), g.ws->oplog, rec * (uint32_t)sizeof(OpRec), key, word);
       g.keep_node(upd, ni4, late.node, (uint32_t)bi + 1u);
+#endif
       st.logEnd += 1 + nrec;
     };
     FM(8);
@@ -1253,6 +1391,13 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   }
   g.keep_node(1ull, 0, make_float4(startPos[0], startPos[1], startPos[2], 0.0f), 0u);
   wave_sync();
+#if BPSX_FOLLOWER
+  g.settle(g.epoch | kFollowEnd);   // the search before is over for the follower too
+  g.epoch = (g.epoch + 0x10000u) & 0x7fff0000u;
+  if (lane == 0) { g.L->start = make_uint2(__float_as_uint(total), startIp << 11); g.L->arrived = 0; }
+  wave_sync();
+  g.publish(g.epoch);
+#endif
   st.lastBest = 0;
   st.outOfNodes = false;
   st.logEnd = st.synced = 0;
@@ -1286,7 +1431,16 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     }
     if (ex == kAstarEmpty || ex == kAstarGoal) break;
     __builtin_amdgcn_s_setprio(3);   // a search that pays for a replay is late from here on
+#if BPSX_FOLLOWER
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    g.publish(g.epoch | (uint32_t)st.logEnd);
+    g.clear_marks();   // the pass that ended here has left its own
+    g.settle(g.epoch | (uint32_t)st.logEnd);
+    st.replaySize = uniform_i((int)g.L->heap_size);
+    st.replayRoot = (uint32_t)uniform_i((int)g.L->heap()[1].y);
+#else
     replay_log(g, st);
+#endif
     // The reference pops what its heap has at the root: that entry goes first.  Equal totals have no
     // defined order in the list, so where more than 64 share the smallest one (an end point so far away
     // that a step's length is lost in the total's rounding) it may be none of the list's first 64.
@@ -1313,6 +1467,9 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
     }
     break;
   }
+#if BPSX_FOLLOWER
+  g.publish(g.epoch | kFollowEnd);
+#endif
   // an open list that ran empty, or a pool that ran out, is DT_PARTIAL_RESULT or
   // DT_OUT_OF_NODES in the reference: no path to build, the result is a failure
   if (ex != kAstarGoal || st.outOfNodes) return 0;
@@ -1325,11 +1482,19 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   static_assert(kTagSlots * sizeof(uint32_t) >= kMaxPath * sizeof(uint16_t), "the walk must fit the marks it reuses");
   uint16_t* walk = reinterpret_cast<uint16_t*>(g.L->marks());
   wave_sync();
+#if BPSX_FOLLOWER
+  // the follower's heap lies behind the window, and is free once it is done with the search
+  if (!kAllLds) g.settle(g.epoch | kFollowEnd);
+  [[maybe_unused]] constexpr size_t kBehind = sizeof(g.L->ref_heap);
+  static_assert(kAllLds || offsetof(GeoLds, ref_heap) == offsetof(GeoLds, w_node) + kWindow * sizeof(float4), "one place behind the other");
+#else
+  [[maybe_unused]] constexpr size_t kBehind = 0;
+#endif
 #if BPSX_WINDOW >= 2048
   const uint16_t* lparent = g.L->parents;
   constexpr int inLds = kMaxNodes;
 #else
-  constexpr int kParentsLds = kWindow * (int)(sizeof(float4) / sizeof(uint16_t));
+  constexpr int kParentsLds = (int)((kWindow * sizeof(float4) + kBehind) / sizeof(uint16_t));
   uint16_t* lparent = reinterpret_cast<uint16_t*>(g.L->w_node);
   const int inLds = g.nodeCount < kParentsLds ? g.nodeCount : kParentsLds;
   {
@@ -1343,7 +1508,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   for (int c = lastBest + 1; c && length <= kMaxNodes;) {
     if (lane == 0 && length < kMaxPath) walk[length] = (uint16_t)(c - 1);
     length++;
-    c = c - 1 < inLds ? uniform_i((int)lparent[c - 1]) : uniform_i((int)g.ws->parents[c - 1]);
+    c = inLds == kMaxNodes || c - 1 < inLds ? uniform_i((int)lparent[c - 1]) : uniform_i((int)g.ws->parents[c - 1]);
   }
   wave_sync();
   const bool ok = length <= kMaxPath && link_id(g.link<true>(lastBest)) == endIp && !st.outOfNodes;

@@ -10,7 +10,9 @@ namespace bpsx {
 struct GeoPool {
   GeoSlot* slots;
   uint32_t blocks;       // blocks of two wavefronts of k_geodesic
-  uint32_t few_blocks;   // blocks of one wavefront of k_geodesic_few; 0: never
+  uint32_t few_blocks;   // blocks of k_geodesic_few, one pool each; 0: never
+  uint32_t mid_blocks;   // blocks of k_geodesic_mid, one pool each
+  uint32_t mid_steps, mid_batch;   // most queries that it serves, in order of their expected cost and without such an order
 };
 
 enum QueueCounter { kQGeo = 0 /* one per cost class */, kQGeoHead = kGeoClasses, kQReset, kQCounters };
@@ -73,5 +75,6 @@ void launch_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint32_t s
 // Blocks of the A* kernels that one compute unit holds at once (bounded by their LDS).
 uint32_t geodesic_blocks_per_cu();
 uint32_t geodesic_few_blocks_per_cu();
+uint32_t geodesic_mid_blocks_per_cu();
 
 }  // namespace bpsx

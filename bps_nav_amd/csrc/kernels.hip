@@ -6,7 +6,8 @@
 //                  the episode ended; an agent whose episode ended also picks its next episode
 //                  here and is queued for reset (simulator.cpp:620-632, 651-710, 601-610)
 //   geodesic       wavefront per query, both kinds in one launch: A* + funnel; blocks of two
-//                  wavefronts so that the longest searches can take a block's whole LDS
+//                  wavefronts so that the longest searches can take a block's whole LDS, or in launches of
+//                  fewer queries a block per query
 //                                                        (PathFinder.cpp:485-541)
 //   step_finish    lane per agent: info, reward, mask from the terminal transition, then the
 //                  new episode's distance bookkeeping    (simulator.cpp:634-641, 758-822, 749-755);
@@ -40,14 +41,20 @@
 #define BPSX_WINDOW 256
 #define BPSX_HASH 1024
 #include "geodesic_device.h"
-// A third, for launches of few queries, where a launch lasts as long as its longest search: the
-// whole node pool and 2048 hash heads in LDS, 52 KB for each wavefront (see k_geodesic_few).
+// A third, for launches that have a block for each query or nearly so: 2048 hash heads, and a second
+// wavefront that keeps the reference's heap, 20 KB for both (see k_geodesic_mid).
+#undef BPSX_GEO_NS
+#undef BPSX_HASH
+#undef BPSX_FOLLOWER
+#define BPSX_GEO_NS geo_mid
+#define BPSX_HASH 2048
+#define BPSX_FOLLOWER 1
+#include "geodesic_device.h"
+// And a fourth, for launches of few queries: the whole node pool in LDS as well, 52 KB (see k_geodesic_few).
 #undef BPSX_GEO_NS
 #undef BPSX_WINDOW
-#undef BPSX_HASH
 #define BPSX_GEO_NS geo_few
 #define BPSX_WINDOW 2048
-#define BPSX_HASH 2048
 #include "geodesic_device.h"
 #include "kernels.h"
 
@@ -587,7 +594,8 @@ BPSX_DEV void serve_query(Wave& g, const NavData& nav, const GeoQuery& q, int cl
 #endif
   // the longer the expected search, the sooner its instructions issue; a search of unknown
   // length may be among the longest, but most are not: they run just below those known to be long
-  set_wave_priority(cls == (int)kGeoClassUnknown ? 2 : (int)(((uint32_t)(kGeoClasses - 1 - cls) * kGeoClassWidth) / 400u));
+  const int priority = cls == (int)kGeoClassUnknown ? 2 : (int)(((uint32_t)(kGeoClasses - 1 - cls) * kGeoClassWidth) / 400u);
+  set_wave_priority(Wave::kFollowed && priority < 1 ? 1 : priority);   // above the wavefronts that keep the heaps
   const float d = geodesic_query(g, nav, q, &T.pops, &T.corridor);
   if (g.lane == 0) {
 #ifdef BPSX_QUERY_TRACE
@@ -635,8 +643,7 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
     nq += (uint32_t)uniform_i((int)counts[c]);
     if (c + 1 == kLongClasses) nlong = nq;
   }
-  // With a block for every query all of them are run that way (1024 agents over room plans, 560
-  // queries: 0.90 -> 0.87 ms).
+  // With a block for every query all of them are run that way (560 queries over room plans: 0.90 -> 0.87 ms).
   if (nq <= gridDim.x) nlong = nq;
   int curCls = 0;
   uint32_t curLo = 0, curHi = (uint32_t)uniform_i((int)counts[0]);
@@ -703,27 +710,33 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
   T.count(lane, counters);
 }
 
-// The same for launches of few queries: one wavefront per block, three blocks per CU.  Such a launch
-// lasts as long as its longest search, a chain of dependent steps; with every node in LDS no step of it
-// waits for a node that has left a window, hash chains are short, and only the log is written.  (1024
-// agents over room plans, 560 queries: 0.87 ms with a block's 15 KB for each, 0.82 here; 510 agents in two
-// groups: 0.75 and 0.71 each.)
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_geodesic_few(NavData nav, const GeoQuery* __restrict__ queries, uint32_t stride,
-                                                  const uint32_t* __restrict__ counts, uint32_t* head,
-                                                  float* out, uint32_t* last_cost, GeoSlot* slots, uint64_t* counters) {
-  __shared__ __attribute__((aligned(16))) geo_few::GeoShared lds;
-  static_assert(sizeof(geo_few::GeoShared) <= 42 * 1280, "three blocks per CU");
-  geo_few::GeoWave g;
-  g.lane = (int)threadIdx.x;
-  g.L = &lds.a;
+// Launches with a block for each query, or nearly so, last as long as their longest searches, chains of dependent
+// steps.  A block has one search at a time, more LDS for it, and a second wavefront that keeps the
+// reference's heap next to it, so that a tie costs no replay (follow).  Replays were a fifth of such launches:
+// 1000 pairs over a maze 1368 -> 990 us, steps of 4096 agents over cluttered plans 1825 -> 1360.  The second
+// wavefronts take issue slots from the searches, 2 to 3 % where no search ties (a reset of 2048 over mazes 471 ->
+// 483).
+template <class Wave>
+BPSX_DEV void one_search_per_block(typename Wave::Shared* lds, const NavData& nav, const GeoQuery* __restrict__ queries, uint32_t stride,
+                                   const uint32_t* __restrict__ counts, uint32_t* head, float* out, uint32_t* last_cost, GeoSlot* slots,
+                                   uint64_t* counters) {
+  const int lane = (int)(threadIdx.x & 63), half = uniform_i((int)(threadIdx.x >> 6));
+  uint32_t nq = 0;
+  for (int c = 0; c < kGeoClasses; ++c) nq += (uint32_t)uniform_i((int)counts[c]);
+  if (blockIdx.x >= nq) return;
+  if (threadIdx.x == 0) follow_init(&lds->a);
+  __syncthreads();
+  if (half == 1) return follow(&lds->a, &slots[blockIdx.x], lane);
+  Wave g;
+  g.lane = lane;
+  g.L = &lds->a;
   g.ws = &slots[blockIdx.x];
   g.nodeCount = 0;
+  g.epoch = 0;
   g.linkSpills = g.heapSpills = g.exactRuns = g.tieReplays = g.pairTies = 0;
 #ifdef BPSX_PHASE_TIMING
   for (int k = 0; k < 8; ++k) g.phase[k] = 0;
 #endif
-  uint32_t nq = 0;
-  for (int c = 0; c < kGeoClasses; ++c) nq += (uint32_t)uniform_i((int)counts[c]);
   int cls = 0;
   uint32_t lo = 0, hi = (uint32_t)uniform_i((int)counts[0]);
   GeoTotals T;
@@ -737,12 +750,32 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 2))) void
     }
     const GeoQuery q = queries[(size_t)cls * stride + (qi - lo)];
     serve_query(g, nav, q, cls, out, last_cost, T);
-    if (g.lane == 0) qi = atomicAdd(head, 1u);
+    if (lane == 0) qi = atomicAdd(head, 1u);
     qi = gridDim.x + (uint32_t)uniform_i((int)qi);
   }
-  T.add(g, g.lane, counters);
-  T.count(g.lane, counters);
-  if (g.lane == 0 && T.done) atomicAdd((unsigned long long*)&counters[kCntLongPath], (unsigned long long)T.done);
+  g.publish(kFollowQuit);
+  T.add(g, lane, counters);
+  T.count(lane, counters);
+  if (lane == 0 && T.done) atomicAdd((unsigned long long*)&counters[kCntLongPath], (unsigned long long)T.done);
+}
+// Three blocks per CU.  With every node in LDS no step waits for a node that has left a window, and only the log
+// is written.  (1024 agents over room plans, 560 queries: 0.87 ms with a block's 15 KB for each, 0.82 here; 510
+// agents in two groups: 0.75 and 0.71 each.)
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_geodesic_few(NavData nav, const GeoQuery* __restrict__ queries, uint32_t stride,
+                                                  const uint32_t* __restrict__ counts, uint32_t* head,
+                                                  float* out, uint32_t* last_cost, GeoSlot* slots, uint64_t* counters) {
+  __shared__ __attribute__((aligned(16))) geo_few::GeoShared lds;
+  static_assert(sizeof(lds) <= 42 * 1280, "three blocks per CU");
+  one_search_per_block<geo_few::GeoWave>(&lds, nav, queries, stride, counts, head, out, last_cost, slots, counters);
+}
+// Eight blocks per CU.  (With 1024 hash heads and a window of 128, and the parent indices in their place: a reset of
+// 2048 over mazes 498 us instead of 483, 1000 pairs 987 instead of 925.)
+__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_geodesic_mid(NavData nav, const GeoQuery* __restrict__ queries, uint32_t stride,
+                                                  const uint32_t* __restrict__ counts, uint32_t* head,
+                                                  float* out, uint32_t* last_cost, GeoSlot* slots, uint64_t* counters) {
+  __shared__ __attribute__((aligned(16))) geo_mid::GeoShared lds;
+  static_assert(sizeof(lds) <= 16 * 1280, "eight blocks per CU");
+  one_search_per_block<geo_mid::GeoWave>(&lds, nav, queries, stride, counts, head, out, last_cost, slots, counters);
 }
 
 // ---- batched PathFinder-level kernels (one lane per item, or one group per item)
@@ -825,17 +858,32 @@ uint32_t geodesic_blocks_per_cu() {
 }
 uint32_t geodesic_few_blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic_few, 64, 0) != hipSuccess || n < 1) n = 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic_few, 128, 0) != hipSuccess || n < 1) n = 1;
   return (uint32_t)n;
 }
 
-// Where the number of queries to expect is no more than the wavefronts that k_geodesic_few keeps on
-// the device at once it serves them, otherwise k_geodesic.
+uint32_t geodesic_mid_blocks_per_cu() {
+  int n = 0;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic_mid, 128, 0) != hipSuccess || n < 1) n = 1;
+  return (uint32_t)n;
+}
+
+// Where the number of queries to expect is no more than the blocks that k_geodesic_few keeps on the device at once it
+// serves them.  Up to a multiple of its own blocks (2048) k_geodesic_mid does, which has fewer searches under way
+// than k_geodesic (5120), but each is shorter.  In a step the longest begin first, and it is ahead up to 9/4 of its
+// blocks, 6144 agents (us by k_geodesic, by k_geodesic_mid, over room plans, cluttered plans, mazes: 1536 agents
+// 665, 648; 1282, 1068; 519, 512; 6144: 812, 702; 1595, 1204; 643, 573; 12288: 850, 719; 1713, 1761; 706, 896).
+// Of a reset's or a batch's searches nothing is known, and a long one that begins late costs more: up to 5/4
+// (pairs over the same, 1000: 411, 420; 1848, 1311; 1308, 925; 2000: 552, 472; 2362, 1632; 1527, 1083; 6000: 575,
+// 630; 2756, 2655; 2402, 2203; resets over room plans, mazes, 2048: 634, 649; 470, 484; 4096: 855, 752; 624, 699).
 void launch_geodesic(const NavData& nav, const GeoQuery* queries, uint32_t stride, const uint32_t* counts, uint32_t* head,
-                     float* out, uint32_t* last_cost, const GeoPool& G, uint32_t expected,
+                     float* out, uint32_t* last_cost, const GeoPool& G, uint32_t expected, uint32_t mid_most,
                      uint64_t* counters, hipStream_t st) {
   if (expected <= G.few_blocks)
-    hipLaunchKernelGGL(k_geodesic_few, dim3(G.few_blocks), dim3(64), 0, st, nav, queries, stride, counts, head, out,
+    hipLaunchKernelGGL(k_geodesic_few, dim3(G.few_blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
+                       last_cost, G.slots, counters);
+  else if (expected <= mid_most)
+    hipLaunchKernelGGL(k_geodesic_mid, dim3(G.mid_blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
                        last_cost, G.slots, counters);
   else
     hipLaunchKernelGGL(k_geodesic, dim3(G.blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
@@ -863,7 +911,7 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
   // 1184 agents, 887, 782 and 837, 745 at 1600, where over rooms both take 320.)
   if (P.task != BPSX_TASK_EXPLORATION)   // which asks for no distance
     launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                    A.last_cost, G, P.n - P.n / 4u, P.counters, st);
+                    A.last_cost, G, P.n - P.n / 4u, G.mid_steps, P.counters, st);
   mark();
   const uint32_t with_snaps = ev ? 0u : step_snap_blocks;
   hipLaunchKernelGGL(k_step_finish, dim3(with_snaps + grid_for(P.n, 256).x), dim3(256), 0, st, nav, A, P, Q, Qnext, with_snaps);
@@ -878,7 +926,7 @@ void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q,
   hipLaunchKernelGGL(k_reset_snap, dim3(std::min(snap_blocks, (P.n + 1u) / 2u)), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Q, P);
   if (P.task != BPSX_TASK_EXPLORATION)
     launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                    A.last_cost, G, P.n, P.counters, st);
+                    A.last_cost, G, P.n, G.mid_batch, P.counters, st);
   hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, nav, A, P, Q, Qother, 0u);
   // the next step finds its lists of queries empty, not with this launch's queries still in them
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Q);
@@ -908,7 +956,7 @@ void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz
   hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n, (uint32_t)kGeoClasses - 1u);
   // stride 0 puts the class's queries at the start of the buffer
   launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, G, n,
-                  counters, st);
+                  G.mid_batch, counters, st);
 }
 void launch_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint32_t slot, uint32_t target, uint32_t envs,
                      hipStream_t st) {

@@ -62,3 +62,11 @@ def test_replayed_heaps_of_all_sizes_match_oracle(oracle, edge, far):
     assert np.array_equal(common.bits(want), common.bits(got))
     cpu.close()
     gpu.close()
+
+
+# more searches than blocks that have a second wavefront for the reference's heap (eight on a CU): some blocks have
+# several searches one after the other, and that wavefront begins anew for each
+@pytest.mark.parametrize("over", [1, 512])
+def test_equal_totals_one_search_after_the_other(oracle, over):
+    import torch
+    test_equal_totals_match_oracle(oracle, 8 * torch.cuda.get_device_properties(0).multi_processor_count + over, True)
