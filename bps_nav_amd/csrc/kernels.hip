@@ -10,10 +10,9 @@
 //                  fewer queries a block per query
 //                                                        (PathFinder.cpp:485-541)
 //   step_finish    lane per agent: info, reward, mask from the terminal transition, then the
-//                  new episode's distance bookkeeping    (simulator.cpp:634-641, 758-822, 749-755);
-//                  in blocks of their own a wavefront per snap: start and goal of the new episode,
-//                  polar, and the new episode's first query (agent -> goal)
-//                                                        (simulator.cpp:611-614, 744-751)
+//                  new episode's distance bookkeeping    (simulator.cpp:634-641, 758-822, 749-755)
+// In blocks of their own in one of the last two (geodesic where its searches leave room) a wavefront per snap: start
+// and goal of the new episode, polar, and the new episode's first query (agent -> goal) (simulator.cpp:611-614, 744-751).
 // The first query of an episode that begins in step t is answered by step t + 1's geodesic launch, and
 // its result enters the bookkeeping at the start of step t + 1's step_finish.  No output of step t
 // depends on it (the reference computes it inside the reset and uses it from the next step on).  A reset
@@ -26,6 +25,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "../../include/bpsx.h"
 #include "geodesic_device.h"
@@ -428,8 +428,8 @@ __global__ __launch_bounds__(kSnapWaves * 64) __attribute__((amdgpu_waves_per_eu
   snap_new_episodes(nav, A, Q, Qout, P, blockIdx.x * kSnapWaves + half, gridDim.x * kSnapWaves, lds[half]);
 }
 
-// The bookkeeping of a step's agents, and in its first snap_blocks blocks the snaps of the episodes that
-// began in it, which touch nothing that the bookkeeping touches: no output of this step depends on an
+// The bookkeeping of a step's agents, and in its first snap_blocks blocks, unless the searches' launch has taken
+// them, the snaps of the episodes that began in it, which touch nothing that the bookkeeping touches: no output of this step depends on an
 // episode's first distance (the reference computes it inside the reset and uses it from the next step
 // on), so its query goes to the next step's queues.
 // (On a second stream next to the searches they cost the step two waits between streams, 6 to 17 us before
@@ -716,11 +716,32 @@ __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(5, 5))) voi
 // 1000 pairs over a maze 1368 -> 990 us, steps of 4096 agents over cluttered plans 1825 -> 1360.  The second
 // wavefronts take issue slots from the searches, 2 to 3 % where no search ties (a reset of 2048 over mazes 471 ->
 // 483).
-template <class Wave>
+// The last blocks of a step's launch take the snaps of the episodes that begin in it, which touch nothing
+// that the searches touch: the step's last launch would last 9 us longer with them, here they end long before the
+// searches do.  (Steps of 64 agents 161 -> 154 us, of 510 in two groups 1199 -> 1186, of 1024 over room plans 625 ->
+// 618, of 4096 over cluttered plans 1350 -> 1320.  In k_geodesic, whose searches fill the device, they would cost
+// its loop registers.)
+struct SnapWork {
+  AgentArrays A;
+  StepQueues Q, Qnext;
+  StepParams P;
+  uint32_t blocks;
+};
+struct NoSnaps {};   // a launch without them, whose kernel is spared their code (it costs the searches 1.6 %)
+template <class Wave, class Snaps>
 BPSX_DEV void one_search_per_block(typename Wave::Shared* lds, const NavData& nav, const GeoQuery* __restrict__ queries, uint32_t stride,
                                    const uint32_t* __restrict__ counts, uint32_t* head, float* out, uint32_t* last_cost, GeoSlot* slots,
-                                   uint64_t* counters) {
+                                   uint64_t* counters, const Snaps& snaps) {
   const int lane = (int)(threadIdx.x & 63), half = uniform_i((int)(threadIdx.x >> 6));
+  uint32_t blocks = gridDim.x;   // for searches
+  if constexpr (std::is_same_v<Snaps, SnapWork>) {
+    blocks -= snaps.blocks;
+    if (blockIdx.x >= blocks) {
+      static_assert(2 * sizeof(SnapLds) <= sizeof(*lds) && sizeof(SnapLds) % 16 == 0, "one for each wavefront");
+      return snap_new_episodes(nav, snaps.A, snaps.Q, snaps.Qnext, snaps.P, (blockIdx.x - blocks) * 2u + (uint32_t)half, snaps.blocks * 2u,
+                               reinterpret_cast<SnapLds*>(lds)[half]);
+    }
+  }
   uint32_t nq = 0;
   for (int c = 0; c < kGeoClasses; ++c) nq += (uint32_t)uniform_i((int)counts[c]);
   if (blockIdx.x >= nq) return;
@@ -751,7 +772,7 @@ BPSX_DEV void one_search_per_block(typename Wave::Shared* lds, const NavData& na
     const GeoQuery q = queries[(size_t)cls * stride + (qi - lo)];
     serve_query(g, nav, q, cls, out, last_cost, T);
     if (lane == 0) qi = atomicAdd(head, 1u);
-    qi = gridDim.x + (uint32_t)uniform_i((int)qi);
+    qi = blocks + (uint32_t)uniform_i((int)qi);
   }
   g.publish(kFollowQuit);
   T.add(g, lane, counters);
@@ -761,21 +782,23 @@ BPSX_DEV void one_search_per_block(typename Wave::Shared* lds, const NavData& na
 // Three blocks per CU.  With every node in LDS no step waits for a node that has left a window, and only the log
 // is written.  (1024 agents over room plans, 560 queries: 0.87 ms with a block's 15 KB for each, 0.82 here; 510
 // agents in two groups: 0.75 and 0.71 each.)
+template <class Snaps>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1, 2))) void k_geodesic_few(NavData nav, const GeoQuery* __restrict__ queries, uint32_t stride,
                                                   const uint32_t* __restrict__ counts, uint32_t* head,
-                                                  float* out, uint32_t* last_cost, GeoSlot* slots, uint64_t* counters) {
+                                                  float* out, uint32_t* last_cost, GeoSlot* slots, uint64_t* counters, Snaps snaps) {
   __shared__ __attribute__((aligned(16))) geo_few::GeoShared lds;
   static_assert(sizeof(lds) <= 42 * 1280, "three blocks per CU");
-  one_search_per_block<geo_few::GeoWave>(&lds, nav, queries, stride, counts, head, out, last_cost, slots, counters);
+  one_search_per_block<geo_few::GeoWave>(&lds, nav, queries, stride, counts, head, out, last_cost, slots, counters, snaps);
 }
 // Eight blocks per CU.  (With 1024 hash heads and a window of 128, and the parent indices in their place: a reset of
 // 2048 over mazes 498 us instead of 483, 1000 pairs 987 instead of 925.)
+template <class Snaps>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_geodesic_mid(NavData nav, const GeoQuery* __restrict__ queries, uint32_t stride,
                                                   const uint32_t* __restrict__ counts, uint32_t* head,
-                                                  float* out, uint32_t* last_cost, GeoSlot* slots, uint64_t* counters) {
+                                                  float* out, uint32_t* last_cost, GeoSlot* slots, uint64_t* counters, Snaps snaps) {
   __shared__ __attribute__((aligned(16))) geo_mid::GeoShared lds;
   static_assert(sizeof(lds) <= 16 * 1280, "eight blocks per CU");
-  one_search_per_block<geo_mid::GeoWave>(&lds, nav, queries, stride, counts, head, out, last_cost, slots, counters);
+  one_search_per_block<geo_mid::GeoWave>(&lds, nav, queries, stride, counts, head, out, last_cost, slots, counters, snaps);
 }
 
 // ---- batched PathFinder-level kernels (one lane per item, or one group per item)
@@ -858,13 +881,13 @@ uint32_t geodesic_blocks_per_cu() {
 }
 uint32_t geodesic_few_blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic_few, 128, 0) != hipSuccess || n < 1) n = 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic_few<SnapWork>, 128, 0) != hipSuccess || n < 1) n = 1;
   return (uint32_t)n;
 }
 
 uint32_t geodesic_mid_blocks_per_cu() {
   int n = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic_mid, 128, 0) != hipSuccess || n < 1) n = 1;
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, k_geodesic_mid<SnapWork>, 128, 0) != hipSuccess || n < 1) n = 1;
   return (uint32_t)n;
 }
 
@@ -876,18 +899,24 @@ uint32_t geodesic_mid_blocks_per_cu() {
 // Of a reset's or a batch's searches nothing is known, and a long one that begins late costs more: up to 5/4
 // (pairs over the same, 1000: 411, 420; 1848, 1311; 1308, 925; 2000: 552, 472; 2362, 1632; 1527, 1083; 6000: 575,
 // 630; 2756, 2655; 2402, 2203; resets over room plans, mazes, 2048: 634, 649; 470, 484; 4096: 855, 752; 624, 699).
-void launch_geodesic(const NavData& nav, const GeoQuery* queries, uint32_t stride, const uint32_t* counts, uint32_t* head,
-                     float* out, uint32_t* last_cost, const GeoPool& G, uint32_t expected, uint32_t mid_most,
-                     uint64_t* counters, hipStream_t st) {
+// Returns whether the launch has taken the snaps.
+static uint32_t snap_blocks_of(const SnapWork& s) { return s.blocks; }
+static uint32_t snap_blocks_of(NoSnaps) { return 0; }
+template <class Snaps> static bool launch_geodesic(const NavData& nav, const GeoQuery* queries, uint32_t stride, const uint32_t* counts, uint32_t* head,
+                            float* out, uint32_t* last_cost, const GeoPool& G, uint32_t expected, uint32_t mid_most,
+                            uint64_t* counters, const Snaps& snaps, hipStream_t st) {
   if (expected <= G.few_blocks)
-    hipLaunchKernelGGL(k_geodesic_few, dim3(G.few_blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
-                       last_cost, G.slots, counters);
+    hipLaunchKernelGGL(k_geodesic_few<Snaps>, dim3(G.few_blocks + snap_blocks_of(snaps)), dim3(128), 0, st, nav, queries, stride, counts, head, out,
+                       last_cost, G.slots, counters, snaps);
   else if (expected <= mid_most)
-    hipLaunchKernelGGL(k_geodesic_mid, dim3(G.mid_blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
-                       last_cost, G.slots, counters);
-  else
+    hipLaunchKernelGGL(k_geodesic_mid<Snaps>, dim3(G.mid_blocks + snap_blocks_of(snaps)), dim3(128), 0, st, nav, queries, stride, counts, head, out,
+                       last_cost, G.slots, counters, snaps);
+  else {
     hipLaunchKernelGGL(k_geodesic, dim3(G.blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
                        last_cost, G.slots, counters);
+    return false;
+  }
+  return true;
 }
 
 void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
@@ -909,11 +938,13 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
   // room for one that asks more, so k_geodesic_few serves groups of up to 1024 agents.  (The line could lie
   // higher: a step over room plans, mazes takes 879, 728 us by k_geodesic and 836, 691 by k_geodesic_few at
   // 1184 agents, 887, 782 and 837, 745 at 1600, where over rooms both take 320.)
+  bool snapped = ev != nullptr;
   if (P.task != BPSX_TASK_EXPLORATION)   // which asks for no distance
-    launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                    A.last_cost, G, P.n - P.n / 4u, G.mid_steps, P.counters, st);
+    snapped |= launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
+                               A.last_cost, G, P.n - P.n / 4u, G.mid_steps, P.counters,
+                               SnapWork{A, Q, Qnext, P, ev ? 0u : step_snap_blocks * (kSnapWaves / 2u)}, st);
   mark();
-  const uint32_t with_snaps = ev ? 0u : step_snap_blocks;
+  const uint32_t with_snaps = snapped ? 0u : step_snap_blocks;
   hipLaunchKernelGGL(k_step_finish, dim3(with_snaps + grid_for(P.n, 256).x), dim3(256), 0, st, nav, A, P, Q, Qnext, with_snaps);
   mark();
 }
@@ -926,7 +957,7 @@ void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q,
   hipLaunchKernelGGL(k_reset_snap, dim3(std::min(snap_blocks, (P.n + 1u) / 2u)), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Q, P);
   if (P.task != BPSX_TASK_EXPLORATION)
     launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                    A.last_cost, G, P.n, G.mid_batch, P.counters, st);
+                    A.last_cost, G, P.n, G.mid_batch, P.counters, NoSnaps{}, st);
   hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, nav, A, P, Q, Qother, 0u);
   // the next step finds its lists of queries empty, not with this launch's queries still in them
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Q);
@@ -956,7 +987,7 @@ void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz
   hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n, (uint32_t)kGeoClasses - 1u);
   // stride 0 puts the class's queries at the start of the buffer
   launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, G, n,
-                  G.mid_batch, counters, st);
+                  G.mid_batch, counters, NoSnaps{}, st);
 }
 void launch_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint32_t slot, uint32_t target, uint32_t envs,
                      hipStream_t st) {
