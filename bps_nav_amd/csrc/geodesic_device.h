@@ -254,7 +254,8 @@ struct OpenList {
     asm volatile("s_nop 1" : "+v"(t[0]), "+v"(n[0]));   // as above, before the next lane move
   }
   // v as a select operand under a lane mask that a scalar instruction has written (the compiler does not know the
-  // select for a vector instruction, which has to keep two instructions' distance from a comparison)
+  // select for a vector instruction, which has to keep two instructions' distance from a comparison: a mask that a
+  // comparison alone has made takes a plain select on in_mask.  tests/test_inline_asm_distances.py reads the assembly.)
   static BPSX_DEV uint32_t pick(unsigned long long mask, uint32_t yes, uint32_t no) {
     uint32_t r;
     asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(no), "v"(yes), "s"(mask));
@@ -1024,7 +1025,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     const uint32_t at = g.find<true>(valid, nb, bucket, &chainHead);
     const unsigned long long known = lanes_where(at != kChainEnd);
     uint32_t ni4 = GeoWave::node4_at<true>(at);
-    const float4 pc = g.node((int)OpenList::pick(known, ni4 >> 2, 0u));
+    const float4 pc = g.node((int)(in_mask(known) ? ni4 >> 2 : 0u));   // (no pick: the mask is a comparison's)
     m0 = in_mask(known) ? pc.x : m0; m1 = in_mask(known) ? pc.y : m1; m2 = in_mask(known) ? pc.z : m2;
     const float cx = m0 - b.x, cy = m1 - b.y, cz = m2 - b.z;
     const float ex = endPos[0] - m0, ey = endPos[1] - m1, ez = endPos[2] - m2;
