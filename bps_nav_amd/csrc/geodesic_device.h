@@ -399,8 +399,9 @@ enum AstarExit { kAstarOn = -1, kAstarEmpty = 0, kAstarGoal = 1, kAstarGrowLinks
 // at least 2^-96 and finite, as squared distances between points of a mesh are; a wavefront that meets
 // another (or zero, which this form would make NaN) takes the library routine.  One test of the
 // arguments' range for both.  One step from the reciprocal root's estimate, with the residual exact
-// through a fused multiply-add: compared with the root of the same number in 64 bits, rounded, it
-// is right for every float from 2^-96 up on this hardware.  (The estimate of the root and the residuals of its two
+// through a fused multiply-add.  That by itself is not enough (an estimate a unit in the last place off can give the
+// neighbouring float); with this hardware's estimates it is right for every float from 2^-96 up, all of which
+// tests/test_gpu_roots.py compares.  (The estimate of the root and the residuals of its two
 // neighbours, which of the three it is, are nine instructions instead of five.)
 BPSX_DEV void sqrt_exact2(float x, float y, float* rx, float* ry) {
   const uint32_t lo = 0x0f800000u, span = 0x7f800000u - lo;
