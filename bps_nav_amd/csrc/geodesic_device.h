@@ -513,6 +513,8 @@ struct FunnelLds {
   float portals[kMaxPath][6];
 };
 static_assert(offsetof(FunnelLds, portals) == offsetof(GeoLds, n_link), "corridor must overlay the hash heads only");
+static_assert(!kFollower || sizeof(FunnelLds) <= offsetof(GeoLds, w_node) + kWindow * sizeof(float4),
+              "the portals must end before what the two wavefronts share: the follower may still be at work when they are written");
 union GeoShared {
   GeoLds a;
   FunnelLds f;
