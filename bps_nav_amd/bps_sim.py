@@ -285,6 +285,10 @@ class PointNavRolloutGenerator:
         k = max(1, steps.value)
         return {self._L.bpsx_kernel_name(i).decode(): ms[i] / k for i in range(4)}, steps.value
 
+    def search_kernel(self):
+        """The kernel that the newest step, reset or batch gave its path searches to ("" without any)."""
+        return self._L.bpsx_search_kernel(self._h).decode()
+
     # ---- batched PathFinder-level queries (host arrays)
     def snap_points(self, scene, pts):
         pts = np.ascontiguousarray(pts, np.float32).reshape(-1, 3)

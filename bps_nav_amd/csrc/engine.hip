@@ -34,6 +34,7 @@ using namespace bpsx;
 namespace {
 
 const char* const kKernelNames[BPSX_NUM_KERNELS] = {"step_move", "reset_snap", "geodesic", "step_finish"};
+const char* const kSearchKernelNames[] = {"k_geodesic_few", "k_geodesic_mid", "k_geodesic", ""};   // by SearchKernel
 
 struct Group {
   // Two sets of queues, used in turn: a step's launch serves Q[turn] and puts the first queries
@@ -218,6 +219,7 @@ struct bpsx_sim {
   std::vector<void*> owned;  // every device allocation, for destroy
   std::vector<Group> groups;
   GeoPool geo{};                      // of the steps: what their envs can fill
+  SearchKernel searches = kSearchNone;   // what the newest launch of path searches went to
   uint32_t snap_blocks = 0;
   uint32_t max_geo_blocks = 0, max_few_blocks = 0, max_mid_blocks = 0, compute_units = 0;   // what the device holds at once, whatever the number of envs
   uint32_t* d_error = nullptr;
@@ -701,7 +703,7 @@ int bpsx_reset(bpsx_sim* sim, uint32_t group, void* hip_stream) {
   HIP_TRY(hipSetDevice(sim->cfg.gpu_id));
   if ((rc = quiesce(sim))) return rc;
   hipStream_t st = (hipStream_t)hip_stream;
-  launch_reset(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], sim->params(group), sim->geo, sim->snap_blocks, st);
+  sim->searches = launch_reset(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], sim->params(group), sim->geo, sim->snap_blocks, st);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipStreamSynchronize(st));
   return BPSX_OK;
@@ -734,8 +736,8 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   g.profiled = sim->profiling;
   StepParams P = sim->params(group);
   P.defer_first_distance = 1;
-  launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->geo, sim->snap_blocks, st,
-              g.profiled ? g.ev : nullptr);
+  sim->searches = launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->geo, sim->snap_blocks, st,
+                              g.profiled ? g.ev : nullptr);
   g.turn ^= 1;
   HIP_TRY(hipGetLastError());
   g.record = (sim->ring_head + sim->ring_count) % kStepRing;
@@ -871,6 +873,7 @@ int bpsx_get_kernel_times(bpsx_sim* sim, double* out_ms_sum, uint64_t* out_steps
 }
 
 const char* bpsx_kernel_name(uint32_t idx) { return idx < BPSX_NUM_KERNELS ? kKernelNames[idx] : ""; }
+const char* bpsx_search_kernel(const bpsx_sim* sim) { return kSearchKernelNames[sim ? sim->searches : kSearchNone]; }
 
 // ---- batched PathFinder-level queries: host arrays in, host arrays out
 static int batch_reserve(bpsx_sim* sim, size_t bytes) {
@@ -1114,8 +1117,8 @@ int bpsx_geodesic(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const u
   HIP_TRY(hipMemcpy(d_e, end_xyz, f3, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_sr, start_ref, u1, hipMemcpyHostToDevice));
   HIP_TRY(hipMemcpy(d_er, end_ref, u1, hipMemcpyHostToDevice));
-  launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, d_q, sim->d_batch_counts, d_o, geo,
-                        sim->d_counters, nullptr);
+  sim->searches = launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, d_q, sim->d_batch_counts, d_o, geo,
+                                        sim->d_counters, nullptr);
   HIP_TRY(hipGetLastError());
   HIP_TRY(hipMemcpy(out_dist, d_o, u1, hipMemcpyDeviceToHost));
   return BPSX_OK;
@@ -1137,9 +1140,9 @@ int bpsx_geodesic_static(bpsx_sim* sim, uint32_t scene, const float* start_xyz, 
   GeoSlot* d_slots = (GeoSlot*)(base + kStaticQueriesBytes + kStaticCountsBytes);
   // The counters are rewritten by a kernel at the start of every call; node pools and queries
   // are written before they are read.  Nothing else of the previous call's contents is used.
-  launch_geodesic_batch(sim->nav, scene_entry(sim, scene), start_xyz, start_ref, end_xyz, end_ref, n, d_q, d_counts, out_dist,
-                        GeoPool{d_slots, std::min(kStaticBlocks, std::max(1u, (n + 1) / 2)), n <= kStaticBlocks * 2u ? n : 0u, 0u, 0u, 0u}, sim->d_counters,
-                        (hipStream_t)hip_stream);
+  sim->searches = launch_geodesic_batch(sim->nav, scene_entry(sim, scene), start_xyz, start_ref, end_xyz, end_ref, n, d_q, d_counts, out_dist,
+                                        GeoPool{d_slots, std::min(kStaticBlocks, std::max(1u, (n + 1) / 2)), n <= kStaticBlocks * 2u ? n : 0u, 0u, 0u, 0u},
+                                        sim->d_counters, (hipStream_t)hip_stream);
   HIP_TRY(hipGetLastError());
   return BPSX_OK;
 }

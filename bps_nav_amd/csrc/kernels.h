@@ -15,6 +15,9 @@ struct GeoPool {
   uint32_t mid_steps, mid_batch;   // most queries that it serves, in order of their expected cost and without such an order
 };
 
+// The kernels that serve path searches; kSearchNone: no launch of them.
+enum SearchKernel { kSearchFew, kSearchMid, kSearchMany, kSearchNone };
+
 enum QueueCounter { kQGeo = 0 /* one per cost class */, kQGeoHead = kGeoClasses, kQReset, kQCounters };
 
 // Work queues of one step, all in HBM, sized for every agent of a group.
@@ -53,19 +56,19 @@ constexpr int kStepEvents = 5;  // timestamps recorded by launch_step when asked
 // One step of a group.  Q holds the step's queries, among them the first queries of the episodes
 // that began in the previous step; the episodes that begin in this one are snapped in its last
 // launch, and their first queries go to Qnext, the next step's queues.  snap_blocks: most blocks for
-// the snaps.
-void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
+// the snaps.  These return what the searches went to.
+SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
                  const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st, hipEvent_t* ev);
 // Reset of a whole group, all on st; Qother (the group's other set of queues) is emptied.
-void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
+SearchKernel launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
                   const GeoPool& G, uint32_t snap_blocks, hipStream_t st);
 void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz, uint32_t* oref,
                        uint32_t waves, hipStream_t st);
 void launch_try_step_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                            uint32_t n, float* oxyz, uint32_t* oref, hipStream_t st);
-void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
-                           const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */,
-                           float* out, const GeoPool& G, uint64_t* counters, hipStream_t st);
+SearchKernel launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
+                                   const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */,
+                                   float* out, const GeoPool& G, uint64_t* counters, hipStream_t st);
 void launch_random_points(const NavData& nav, uint32_t scene, const float* u, uint32_t n, float* oxyz, uint32_t* oref,
                           hipStream_t st);
 

@@ -899,27 +899,28 @@ uint32_t geodesic_mid_blocks_per_cu() {
 // Of a reset's or a batch's searches nothing is known, and a long one that begins late costs more: up to 5/4
 // (pairs over the same, 1000: 411, 420; 1848, 1311; 1308, 925; 2000: 552, 472; 2362, 1632; 1527, 1083; 6000: 575,
 // 630; 2756, 2655; 2402, 2203; resets over room plans, mazes, 2048: 634, 649; 470, 484; 4096: 855, 752; 624, 699).
-// Returns whether the launch has taken the snaps.
+// k_geodesic takes no snaps.
 static uint32_t snap_blocks_of(const SnapWork& s) { return s.blocks; }
 static uint32_t snap_blocks_of(NoSnaps) { return 0; }
-template <class Snaps> static bool launch_geodesic(const NavData& nav, const GeoQuery* queries, uint32_t stride, const uint32_t* counts, uint32_t* head,
+template <class Snaps> static SearchKernel launch_geodesic(const NavData& nav, const GeoQuery* queries, uint32_t stride, const uint32_t* counts, uint32_t* head,
                             float* out, uint32_t* last_cost, const GeoPool& G, uint32_t expected, uint32_t mid_most,
                             uint64_t* counters, const Snaps& snaps, hipStream_t st) {
-  if (expected <= G.few_blocks)
+  if (expected <= G.few_blocks) {
     hipLaunchKernelGGL(k_geodesic_few<Snaps>, dim3(G.few_blocks + snap_blocks_of(snaps)), dim3(128), 0, st, nav, queries, stride, counts, head, out,
                        last_cost, G.slots, counters, snaps);
-  else if (expected <= mid_most)
+    return kSearchFew;
+  }
+  if (expected <= mid_most) {
     hipLaunchKernelGGL(k_geodesic_mid<Snaps>, dim3(G.mid_blocks + snap_blocks_of(snaps)), dim3(128), 0, st, nav, queries, stride, counts, head, out,
                        last_cost, G.slots, counters, snaps);
-  else {
-    hipLaunchKernelGGL(k_geodesic, dim3(G.blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
-                       last_cost, G.slots, counters);
-    return false;
+    return kSearchMid;
   }
-  return true;
+  hipLaunchKernelGGL(k_geodesic, dim3(G.blocks), dim3(128), 0, st, nav, queries, stride, counts, head, out,
+                     last_cost, G.slots, counters);
+  return kSearchMany;
 }
 
-void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
+SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
                  const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st, hipEvent_t* ev) {
   int e = 0;
   auto mark = [&]() { if (ev) (void)hipEventRecord(ev[e++], st); };
@@ -938,29 +939,33 @@ void launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, 
   // room for one that asks more, so k_geodesic_few serves groups of up to 1024 agents.  (The line could lie
   // higher: a step over room plans, mazes takes 879, 728 us by k_geodesic and 836, 691 by k_geodesic_few at
   // 1184 agents, 887, 782 and 837, 745 at 1600, where over rooms both take 320.)
-  bool snapped = ev != nullptr;
+  SearchKernel searches = kSearchNone;
   if (P.task != BPSX_TASK_EXPLORATION)   // which asks for no distance
-    snapped |= launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
+    searches = launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
                                A.last_cost, G, P.n - P.n / 4u, G.mid_steps, P.counters,
                                SnapWork{A, Q, Qnext, P, ev ? 0u : step_snap_blocks * (kSnapWaves / 2u)}, st);
   mark();
+  const bool snapped = ev || searches == kSearchFew || searches == kSearchMid;
   const uint32_t with_snaps = snapped ? 0u : step_snap_blocks;
   hipLaunchKernelGGL(k_step_finish, dim3(with_snaps + grid_for(P.n, 256).x), dim3(256), 0, st, nav, A, P, Q, Qnext, with_snaps);
   mark();
+  return searches;
 }
 
-void launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
+SearchKernel launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
                   const GeoPool& G, uint32_t snap_blocks, hipStream_t st) {
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Qother);
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Qother, Qother);
   hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 32), dim3(256), 0, st, nav, A, Q, P);
   hipLaunchKernelGGL(k_reset_snap, dim3(std::min(snap_blocks, (P.n + 1u) / 2u)), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Q, P);
+  SearchKernel searches = kSearchNone;
   if (P.task != BPSX_TASK_EXPLORATION)
-    launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
-                    A.last_cost, G, P.n, G.mid_batch, P.counters, NoSnaps{}, st);
+    searches = launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
+                               A.last_cost, G, P.n, G.mid_batch, P.counters, NoSnaps{}, st);
   hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, nav, A, P, Q, Qother, 0u);
   // the next step finds its lists of queries empty, not with this launch's queries still in them
   hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Q);
+  return searches;
 }
 void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz, uint32_t* oref,
                        uint32_t waves, hipStream_t st) {
@@ -979,15 +984,15 @@ void launch_try_step_batch(const NavData& nav, uint32_t scene, const float* sxyz
                            uint32_t n, float* oxyz, uint32_t* oref, hipStream_t st) {
   hipLaunchKernelGGL(k_try_step_batch, grid_for(n, kMoveItems), dim3(kMoveItems * 8), 0, st, nav, scene, sxyz, sref, exyz, n, oxyz, oref);
 }
-void launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
-                           const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */, float* out,
-                           const GeoPool& G, uint64_t* counters, hipStream_t st) {
+SearchKernel launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
+                                   const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */, float* out,
+                                   const GeoPool& G, uint64_t* counters, hipStream_t st) {
   hipLaunchKernelGGL(k_make_queries, grid_for(n, 256), dim3(256), 0, st, scene, sxyz, sref, exyz, eref, n, qbuf);
   // one class only, that of the shortest
   hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n, (uint32_t)kGeoClasses - 1u);
   // stride 0 puts the class's queries at the start of the buffer
-  launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, G, n,
-                  G.mid_batch, counters, NoSnaps{}, st);
+  return launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, G, n,
+                         G.mid_batch, counters, NoSnaps{}, st);
 }
 void launch_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint32_t slot, uint32_t target, uint32_t envs,
                      hipStream_t st) {

@@ -209,8 +209,8 @@ BPSX_API int bpsx_check_errors(bpsx_sim *sim);
  * more node links than the kernel keeps in LDS (none where it keeps those of a full pool), [17] path
  * searches that went on with the reference's heap (see [19]) and whose heap outgrew LDS (both
  * continue in slower code; results are the same), [18] path
- * searches that the kernel runs with larger LDS structures: those expected to be among the longest
- * of their step, or all where there is a block for each (same results).  The path search keeps its open list sorted by total instead of
+ * searches that run with larger LDS structures: those expected to be among the longest of their
+ * step, or, in launches of fewer searches, all (same results).  The path search keeps its open list sorted by total instead of
  * in the reference's heap arrangement, which only matters when two open nodes share the
  * smallest total: [21] counts the passes that found such a pair and tried to expand both at once
  * (possible when neither affects the other), [20] the times the reference's arrangement had to be
@@ -229,6 +229,10 @@ BPSX_API int bpsx_set_profiling(bpsx_sim *sim, int enabled);
 BPSX_API int bpsx_get_kernel_times(bpsx_sim *sim, double *out_ms_sum /* [BPSX_NUM_KERNELS] */,
                           uint64_t *out_steps);
 BPSX_API const char *bpsx_kernel_name(uint32_t idx);
+/* Which kernel the newest step, reset or batch of the simulator gave its path searches to, for tests
+ * of the sizes at which that changes: "k_geodesic_few", "k_geodesic_mid", "k_geodesic", or "" where
+ * there were none. */
+BPSX_API const char *bpsx_search_kernel(const bpsx_sim *sim);
 
 /* ---- batched PathFinder queries on one uploaded scene (PathFinder.h:99-227) ----
  * All pointers are host pointers; n items; results copied back before returning. */

@@ -16,10 +16,11 @@ def compute_units():
 
 
 def limit(name):
-    """The largest batch that is served one way; one more item goes the next way.  Path queries: a wavefront
-    with the whole node pool in LDS each (three on a CU), a block of two wavefronts each (ten on a CU), more
-    share those.  Snaps: a wavefront each (sixteen on a CU), several to a wavefront.  Allocation-free path
-    queries: a wavefront with the whole pool in LDS for each of 768, more share as many."""
+    """The largest batch that is served one way; one more item goes the next way.  Path queries: a block with
+    the whole node pool in LDS each (three on a CU), blocks of a search each with a window (eight on a CU, which
+    serve up to ten), blocks of two searches.  Snaps: a wavefront each (sixteen on a CU), several to a
+    wavefront.  Allocation-free path queries: a block with the whole pool in LDS for each of 768, more in blocks
+    of two searches."""
     return {"pool": 3, "block": 10, "snap": 16, "static": 3}[name] * (256 if name == "static" else compute_units())
 
 
@@ -47,6 +48,7 @@ def test_batch_sizes(oracle, size):
     x2, r2 = cpu.snap(pts[n:])
     d = gpu.geodesic(0, xo, ro, x2, r2)
     assert np.array_equal(common.bits(cpu.geodesic(xo, ro, x2, r2)), common.bits(d))
+    assert gpu.search_kernel() == ("k_geodesic_few" if n <= limit("pool") else "k_geodesic_mid" if n <= limit("block") else "k_geodesic")
     # every search with larger LDS structures up to the second limit, none beyond
     c = gpu.counters()
     assert c["geo_long_path"] == (c["geodesic_queries"] if n <= limit("block") else 0)
@@ -69,6 +71,7 @@ def test_allocation_free_sizes(oracle, size):
     got = gpu.geodesic_static(0, *dev).cpu().numpy()
     assert np.array_equal(common.bits(cpu.geodesic(x[:n], r[:n], x[n:], r[n:])), common.bits(got))
     c = gpu.counters()
+    assert gpu.search_kernel() == ("k_geodesic_few" if n <= limit("static") else "k_geodesic")
     assert c["geodesic_queries"] == n and c["geo_long_path"] == (n if n <= limit("static") else 0)
     cpu.close()
     gpu.close()
