@@ -886,8 +886,8 @@ BPSX_DEV int apply_pass(RefHeap<true>& rh, uint32_t rk, uint32_t rw, unsigned lo
 //   arrived     written by every pass: the records of the log that may be read (GeoWave::keep_pass).
 //   applied     written by the follower: the last word of `published` that it has done all for.  The heap is the
 //               search's from then on, until it goes on with another pass.
-// A new search of the same slot writes over the log that the follower may still be fetching from: what has been
-// fetched is looked at only if the epoch is still the same afterwards.
+// A new search begins, and writes over the log and the heap, only when the follower has answered the end of the one
+// before (astar waits for that).  The end of all searches it does not answer: what it has fetched by then is not applied.
 // Bound by the heap's operations, 0.2 us per node, which is less than the search takes per node alone.  For the
 // search it is one or two instructions a pass, and two fewer around its stores.  (With `arrived` stored apart, five
 // instructions a pass, it cost the searches without ties 2.5 %: steps of 64 agents 161 -> 165 us, a reset of 2048 over
@@ -932,7 +932,7 @@ BPSX_DEV void follow(GeoLds* L, const GeoSlot* ws, int lane) {
       const uint32_t rk = (uint32_t)r, rw = (uint32_t)(r >> 32);
       const unsigned long long headers = lanes_where((rw & kOpHeader) != 0) & lanes_where(pos + lane < end);
       wave_sync();
-      if (((uint32_t)uniform_i((int)lds_word(&L->published)) ^ word) >> 16) continue;   // over, and perhaps written over
+      if (((uint32_t)uniform_i((int)lds_word(&L->published)) ^ word) >> 16) continue;   // there are no more searches
       int h = 0;
       while (h < 64 && (headers >> h)) h += apply_pass(rh, rk, rw, headers, h, seen);
       pos += h;
@@ -1487,7 +1487,8 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   uint16_t* walk = reinterpret_cast<uint16_t*>(g.L->marks());
   wave_sync();
 #if BPSX_FOLLOWER
-  // the follower's heap lies behind the window, and is free once it is done with the search
+  // the follower's heap lies behind the window, and is free once it is done with the search: parents that the window
+  // does not hold go there (one of 256 nodes holds them all)
   if (!kAllLds) g.settle(g.epoch | kFollowEnd);
   [[maybe_unused]] constexpr size_t kBehind = sizeof(g.L->ref_heap);
   static_assert(kAllLds || offsetof(GeoLds, ref_heap) == offsetof(GeoLds, w_node) + kWindow * sizeof(float4), "one place behind the other");

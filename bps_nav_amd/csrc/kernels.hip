@@ -891,14 +891,22 @@ uint32_t geodesic_mid_blocks_per_cu() {
   return (uint32_t)n;
 }
 
-// Where the number of queries to expect is no more than the blocks that k_geodesic_few keeps on the device at once it
-// serves them.  Up to a multiple of its own blocks (2048) k_geodesic_mid does, which has fewer searches under way
-// than k_geodesic (5120), but each is shorter.  In a step the longest begin first, and it is ahead up to 9/4 of its
-// blocks, 6144 agents (us by k_geodesic, by k_geodesic_mid, over room plans, cluttered plans, mazes: 1536 agents
-// 665, 648; 1282, 1068; 519, 512; 6144: 812, 702; 1595, 1204; 643, 573; 12288: 850, 719; 1713, 1761; 706, 896).
-// Of a reset's or a batch's searches nothing is known, and a long one that begins late costs more: up to 5/4
-// (pairs over the same, 1000: 411, 420; 1848, 1311; 1308, 925; 2000: 552, 472; 2362, 1632; 1527, 1083; 6000: 575,
-// 630; 2756, 2655; 2402, 2203; resets over room plans, mazes, 2048: 634, 649; 470, 484; 4096: 855, 752; 624, 699).
+// Where the number of queries to expect is no more than the blocks that k_geodesic_few keeps on the device at once
+// (768) it serves them.  Up to a multiple of its own blocks (2048) k_geodesic_mid does, which has fewer searches under
+// way than k_geodesic (5120), but each is shorter.  In a step the longest begin first, and it is ahead up to 9/4
+// of its blocks, 6144 agents.  Of a reset's or a batch's searches nothing is known, and a long one that begins late
+// costs more: up to 5/4 of them.  All in us over room plans, cluttered plans, mazes:
+//   k_geodesic_few, _mid    resets of 768: 582, 622; 926, 997; 436, 454; 1024: 586, 630; 946, 1011; 499, 458
+//                           pairs, 768: 312, 335; 1154, 1301; 817, 825; 1000: 326, 323; 1272, 1209; 1149, 814
+//   k_geodesic_mid, k_geodesic
+//                           steps of 3072: 648, 694; 1044, 1372; 527, 576; 6144: 665, 822; 1117, 1541; 555, 638;
+//                           12288: 717, 877; 1687, 1730; 883, 692
+//                           resets of 2048: 641, 633; 1039, 1049; 480, 468; 3072: 664, 785; 1136, 1283; 601, 572;
+//                           4096: 693, 812; 1326, 1369; 686, 622
+//                           pairs, 2000: 326, 312; 1362, 1874; 947, 1341; 2560: 382, 366; 1527, 1704; 1239, 1373;
+//                           4000: 444, 489; 2000, 2183; 1538, 1850; 6000: 493, 465; 2525, 2678; 2067, 2107
+// The line at 5/4 is not the best one everywhere: k_geodesic_mid is ahead for pairs up to 4000 at least, behind for resets
+// over mazes at 2048 already (2 %) and ahead for resets over plans beyond the line.
 // k_geodesic takes no snaps.
 static uint32_t snap_blocks_of(const SnapWork& s) { return s.blocks; }
 static uint32_t snap_blocks_of(NoSnaps) { return 0; }
@@ -937,8 +945,8 @@ SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQue
   mark();
   // Three agents in five ask for a distance in a step; a group's queries are taken for three in four, with
   // room for one that asks more, so k_geodesic_few serves groups of up to 1024 agents.  (The line could lie
-  // higher: a step over room plans, mazes takes 879, 728 us by k_geodesic and 836, 691 by k_geodesic_few at
-  // 1184 agents, 887, 782 and 837, 745 at 1600, where over rooms both take 320.)
+  // higher: a step over room plans, cluttered plans, mazes takes 574, 944, 470 us by k_geodesic_few and 620, 975, 479 by
+  // k_geodesic_mid at 1024 agents, 591, 962, 501 and 647, 1002, 528 at 1600.)
   SearchKernel searches = kSearchNone;
   if (P.task != BPSX_TASK_EXPLORATION)   // which asks for no distance
     searches = launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
