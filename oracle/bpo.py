@@ -149,9 +149,9 @@ class Nav:
     def pass_check(self, rows):
         """Switches the check of the GPU kernel's multi-node pass rules (orc::Query::PassCheck) to
         `rows` nodes per pass (0: off) and returns the counts gathered since the last call."""
-        out = np.zeros(6, np.uint64)
+        out = np.zeros(7, np.uint64)
         self.lib.L.bpo_nav_pass_check(self.h, int(rows), out)
-        return dict(zip(("passes", "nodes", "wrong_node", "wrong_update", "pairs", "ties"), (int(v) for v in out)))
+        return dict(zip(("passes", "nodes", "wrong_node", "wrong_update", "pairs", "ties", "fallen"), (int(v) for v in out)))
 
     def last_corridor(self):
         buf = np.zeros(256, np.uint32)

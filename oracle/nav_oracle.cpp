@@ -837,7 +837,7 @@ float Query::geodesic(const NavPoint& start, const NavPoint& end) {
     float lastBestCost = startNode->total;
     bool outOfNodes = false;
     // ---- check of the multi-node pass rules (see Query::PassCheck); no effect on the search
-    struct PlanUpd { uint32_t ref; float total; float pos[3]; };
+    struct PlanUpd { uint32_t ref; float total; float pos[3]; float cost; };
     struct Plan {
       int count = 0, done = 0, first = 0;
       bool pair = false, blind = false;
@@ -880,13 +880,13 @@ float Query::geodesic(const NavPoint& start, const NavPoint& end) {
         else { cost = best->cost + vdist(best->pos, npos) * 1.0f; heuristic = vdist(npos, end.xyz) * H_SCALE; }
         const float total = cost + heuristic;
         if (flags && total >= ntotal) continue;
-        upds.push_back({nref, total, {npos[0], npos[1], npos[2]}});
+        upds.push_back({nref, total, {npos[0], npos[1], npos[2]}, cost});
       }
     };
     auto make_plan = [&]() {
       plan = Plan();
       const int rows = (passCheck.rows & 0xff) < 8 ? (passCheck.rows & 0xff) : 8;
-      const bool keyRule = !(passCheck.rows & 0x100), readRule = !(passCheck.rows & 0x200);   // switches for the tests that drop a rule
+      const bool keyRule = !(passCheck.rows & 0x100), readRule = !(passCheck.rows & 0x200), anyFalls = passCheck.rows & 0x400;   // switches for the tests that drop a rule
       // the open list sorted by total: the first rows + 1 entries
       std::vector<int> order(q.heapSize);
       for (int i = 0; i < q.heapSize; ++i) order[i] = q.heap[i];
@@ -921,12 +921,30 @@ float Query::geodesic(const NavPoint& start, const NavPoint& end) {
         for (const PlanUpd& u : plan.upd[j]) reads[j].push_back(u.ref);
       }
       int c = lim;
+      // a row's update of a node that an earlier row updates falls away when its way there, to where the earlier
+      // one has put the node, is surely no better (with room for the rounding, as in the kernel)
+      auto falls_away = [&](int j, const PlanUpd& earlier) {
+        if (anyFalls) return true;
+        const Node& b = q.nodes[order[j]];
+        float d[3];
+        for (int k = 0; k < 3; ++k) d[k] = earlier.pos[k] - b.pos[k];
+        const float less = earlier.cost - b.cost;
+        return (d[0] * d[0] + d[1] * d[1] + d[2] * d[2] >= less * less * 1.00001f) || less <= 0.0f;
+      };
+      std::vector<PlanUpd> raw[8];
+      for (int j = 0; j < lim; ++j) raw[j] = plan.upd[j];
       for (int j = 1; j < c; ++j) {
         bool stands = true;
         for (int i = 0; i < j && stands; ++i)
-          for (const PlanUpd& u : plan.upd[i]) {
+          for (const PlanUpd& u : raw[i]) {
             if (keyRule && u.total <= key(j)) { stands = false; break; }
-            if (readRule) for (uint32_t r : reads[j]) if (r == u.ref) { stands = false; break; }
+            if (!readRule) continue;
+            if (u.ref == reads[j][0]) { stands = false; break; }
+            for (size_t k = 0; k < plan.upd[j].size() && stands; ++k) {
+              if (plan.upd[j][k].ref != u.ref) continue;
+              if (plan.pair || !falls_away(j, u)) stands = false;
+              else { plan.upd[j].erase(plan.upd[j].begin() + (long)k); passCheck.fallen++; break; }
+            }
             if (!stands) break;
           }
         if (!stands) { c = j; break; }
@@ -1006,7 +1024,7 @@ float Query::geodesic(const NavPoint& start, const NavPoint& end) {
         nn->flags = (uint8_t)(nn->flags & ~NODE_CLOSED);
         nn->cost = cost;
         nn->total = total;
-        if (checking >= 0) actual.push_back({nref, total, {0, 0, 0}});
+        if (checking >= 0) actual.push_back({nref, total, {0, 0, 0}, 0});
         if (nn->flags & NODE_OPEN) {
           q.modify(nn);
         } else {

@@ -89,7 +89,8 @@ class Query {
   // pop, from the open list sorted by total and the state as it is, which nodes the next pops
   // will be and what their expansions will write, by the kernel's rules: entry j stands while its
   // total is below entry j + 1's, no earlier entry's update reaches its total or touches a
-  // polygon it reads, and it is not the goal; two entries that share the smallest total stand
+  // polygon it reads and would update (or that update falls away: the earlier one has put the node where the way
+  // through the later one is no better), and it is not the goal; two entries that share the smallest total stand
   // together, in either order, when neither touches what the other reads.  The search itself is
   // the reference's, unchanged; every prediction is compared with what it then does.
   struct PassCheck {
@@ -97,6 +98,7 @@ class Query {
     uint64_t passes = 0, nodes = 0;        // predictions made, pops they covered
     uint64_t wrongNode = 0, wrongUpdate = 0;   // pops of another node / expansions that wrote something else
     uint64_t pairs = 0, ties = 0;          // tied pairs predicted as a pair / ties left to the heap
+    uint64_t fallen = 0;                   // updates that fall away behind an earlier row's
   } passCheck;
 
  private:

@@ -102,7 +102,7 @@ BPO_API void bpo_nav_geodesic_field(void* h, const float* sxyz, const uint32_t* 
 BPO_API void bpo_nav_pass_check(void* h, int rows, uint64_t* out) {
   orc::Query& q = *((ApiImpl<OracleBackend>::Nav*)h)->ctx->q[0];
   const orc::Query::PassCheck& p = q.passCheck;
-  out[0] = p.passes; out[1] = p.nodes; out[2] = p.wrongNode; out[3] = p.wrongUpdate; out[4] = p.pairs; out[5] = p.ties;
+  out[0] = p.passes; out[1] = p.nodes; out[2] = p.wrongNode; out[3] = p.wrongUpdate; out[4] = p.pairs; out[5] = p.ties; out[6] = p.fallen;
   q.passCheck = orc::Query::PassCheck();
   q.passCheck.rows = rows;
 }

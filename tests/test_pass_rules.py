@@ -63,3 +63,23 @@ def test_each_rule_is_needed(oracle, dropped, what):
     st = nav.pass_check(0)
     nav.close()
     assert st[what] > 0, st
+
+
+@pytest.mark.parametrize("config,queries", [(1, 400), (2, 200), (3, 80), (4, 100)])
+def test_updates_that_fall_away(oracle, config, queries):
+    """Of two rows that update one node the later one's update falls away when its way to where the earlier one has put
+    the node is no shorter: predictions stay right, and more nodes go through.  Taking every later update
+    for one that falls away gives wrong predictions."""
+    blob = scenes.config_scene(config, 0)
+    nav = bpo.Nav(oracle, blob)
+    x, r = nav.snap(scenes.sample_points(blob, 13, 2 * queries))
+    q = queries
+    nav.pass_check(8)
+    nav.geodesic(x[:q], r[:q], x[q:], r[q:])
+    st = nav.pass_check(8 | 0x400)
+    nav.geodesic(x[:q], r[:q], x[q:], r[q:])
+    all_fall = nav.pass_check(0)
+    nav.close()
+    assert st["wrong_node"] == 0 and st["wrong_update"] == 0, st
+    assert st["fallen"] > 0.1 * st["passes"], st
+    assert all_fall["wrong_update"] > 0, all_fall
