@@ -151,7 +151,8 @@ constexpr int kOpLogCap = 8192;
 // the log.
 struct alignas(128) GeoSlot {
   float4 nodes[kMaxNodes];       // position and cost (dtNode, DetourNode.h:36-45; the total is their sum with the heuristic)
-  uint32_t links[kMaxNodes];     // polygon index within the scene | next node of the hash chain << 16, of nodes beyond what LDS holds
+  uint32_t links[kMaxNodes];     // polygon index within the scene | next node of the hash chain << 16, of nodes beyond what LDS holds;
+                                 // before them, entries that the open list keeps apart
   uint2 heap_spill[kMaxNodes];   // the reference's heap between replays, and where it outgrows LDS (total as bits, packed node)
   OpRec oplog[kOpLogCap];
   uint16_t parents[kMaxNodes];   // per node, 1-based index of the node it was reached from, 0 for the start node: what the final walk up the path reads

@@ -5,7 +5,7 @@
 // Execution model: one wavefront (64 lanes) owns one query at a time and pulls the next from
 // a shared queue when done.  The search touches almost only nodes it created recently (the
 // frontier of A* is narrow), so LDS holds what is hot and small and HBM holds the rest:
-//   - the open list in registers: sorted by total, up to 256 entries (OpenList), which lets a
+//   - the open list in registers: its smallest entries sorted by total (OpenList), which lets a
 //     pass expand up to kRows nodes at once (astar_fast); when totals tie, the reference's binary
 //     heap is rebuilt from a log of the list's operations (RefHeap, replay_log) or has been kept from it all
 //     along by a second wavefront (follow), and a search whose
@@ -46,7 +46,7 @@ namespace bpsx {
 // (the comment that the asm statement leaves in the compiler's assembly output names the loop's
 // instantiation and the mark, for tests/measure_astar_loop_phases.py)
 #define FM(k) do { constexpr int slot_[11] = {7, 0, 1, 2, 3, 4, 5, 5, 5, 6, 6}; const unsigned long long now_ = __builtin_readcyclecounter(); \
-    asm volatile("; astar_fast spill=%0 pairs=%1 mark=%2" :: "i"((int)S), "i"(P), "i"(k)); \
+    asm volatile("; astar_fast spill=%0 mark=%1" :: "i"((int)S), "i"(k)); \
     if ((k) == 0) g.phase[7]++; else g.phase[slot_[k]] += now_ - g.phase_t0; g.phase_t0 = now_; } while (0)
 #else
 #define FM(k) do { } while (0)
@@ -183,25 +183,63 @@ BPSX_DEV uint32_t make_link(uint32_t id, uint32_t next) { return id | (next << 1
 // order of the bits is the float order), and the node's index (bits 0-10) with its polygon index above
 // it, so that the entry at the front names the edge records to fetch without a detour through LDS.
 static_assert(kMaxNodes <= 2048, "open-list entries keep the node index in 11 bits");
-constexpr uint32_t kEmptyKey = 0x7fffffffu;   // above +inf; every key stays below 2^31
+constexpr uint32_t kEmptyKey = 0x7fefffffu;   // above +inf, and below the totals' bits that would make an entry of the list a NaN (OpenList)
 
 // The open list as a sorted array in registers.  dtNodeQueue::pop returns the entry with the
 // smallest total; while that smallest total is held by one entry only, which entry that is
 // does not depend on how the reference's binary heap happens to be arranged.  So a search can
 // keep its open list in any form that yields the minimum, as long as it notices when two
 // entries share the smallest total (a tie, about one pop in ten thousand) and then asks the
-// exact heap.  Sorted by total, entry i in lane i & 63 of pair i >> 6: the next nodes to expand
-// are the first lanes, a pop is a shift of all lanes by one, and an insertion is one comparison
-// of all lanes with the new total and a shift of those above it.  Unused places hold kEmpty
-// keys and kNone nodes.  Entries with equal totals sit next to each other in no defined order.
+// exact heap.
+// An entry is 64 bits, the total over the packed node: as bits of a double, which for such numbers are in the
+// order of the integers (denormal ones among them, which this target's double arithmetic keeps), so that one
+// minimum and one maximum put an entry in its place.  Sorted, one per lane, the smallest in lane `base`, the greatest
+// in the last but one; zeros below (node kNone), which are smaller than every entry, and a total above all in the last lane.  The
+// list grows downwards: an entry that enters moves those below it down a lane, and what a pass
+// expands leaves by a move of the base.
+// Entries with totals from `bound` on are kept apart, in no order, in the wavefront's slot (GeoSlot::far): they cost one store
+// now, and a search comes back to half of them at most.  Where fewer than kRefill are left in registers, those up to a new
+// bound come from there (refill); where more than kSplit are, the greater ones go there (split).  An entry whose node is
+// updated meanwhile stays there, and is known by its total when it is looked at.
+// (With up to 256 sorted entries in four register pairs, counted into place together and moved through LDS from the second
+// pair on, and with totals and nodes selected apart and a lane permute that closed the gap of those that left: 600 to 860
+// cycles of a pass instead of 500 to 600, 1500 instead of 600 over cluttered plans, whose lists have 73 entries on average and up to
+// 260.  Steps of 64 agents 148 -> 136 us, of 1024 over room plans 589 -> 500, of 510 in two groups 1112 -> 968, of 4096 over
+// cluttered plans 1280 -> 1190, of 16384 over mazes 805 -> 796, of 65536 over mixed scenes 2810 -> 2676, a reset of 2048 over mazes
+// 476 -> 447, 300 queries over room plans 265 -> 242, 1000 pairs over a maze 949 -> 931.)
 struct OpenList {
-  static constexpr int kPairs = 4;
-  uint32_t t[kPairs], n[kPairs];
-  int size;
+  static constexpr int kEnd = 63;       // the lane behind the last entry
+  static constexpr int kMost = 62;      // entries in registers at most: there is always a zero below them
+  static constexpr int kSplit = 48, kRefill = 9;   // a pass looks at nine entries
+  static constexpr int kFarMost = 244;  // entries apart before a pass at most ...
+  static constexpr int kFarKeep = 236;  // ... and, once those of updated nodes are gone, for the search to go on in this form
+  static constexpr int kFarCap = 315;
+  static_assert(kFarMost + kMost <= kFarCap, "a pass adds up to 48, and what a split adds was in registers");
+  static constexpr int kMostOfAll = kSplit + kFarMost + 48;   // entries, behind a pass
   static constexpr uint32_t kEmpty = kEmptyKey;
   static constexpr uint32_t kNone = 0;   // the start node, which never enters the list again: what is read by it is there
-  BPSX_DEV void init(int lane, uint32_t total, uint32_t node) { t[0] = lane ? kEmpty : total; n[0] = lane ? kNone : node; size = 1; }   // further pairs are cleared when the list grows into them
-  BPSX_DEV void clear_pair(int k) { t[k] = kEmpty; n[k] = kNone; }
+  unsigned long long e;
+  int base;
+  uint32_t bound;
+  int far;
+  int low;         // a pass may go on while base - low, without a sign, is no more than
+  uint32_t span;
+  BPSX_DEV uint32_t total() const { return (uint32_t)(e >> 32); }
+  BPSX_DEV uint32_t node() const { return (uint32_t)e; }
+  static BPSX_DEV unsigned long long entry(uint32_t total, uint32_t node) { return ((unsigned long long)total << 32) | node; }
+  BPSX_DEV int size() const { return kEnd - base; }
+  BPSX_DEV void init(int lane, uint32_t first, uint32_t node) {
+    e = lane == kEnd ? entry(kEmpty, kNone) : lane == kEnd - 1 ? entry(first, node) : 0ull;
+    base = kEnd - 1;
+    bound = kEmpty;
+    far = 0;
+    set_limits();
+  }
+  BPSX_DEV void set_limits() {
+    low = far > kFarMost ? 2 * kEnd : kEnd - kSplit;
+    span = (uint32_t)((far ? kEnd - kRefill : kEnd) - (kEnd - kSplit));
+  }
+  BPSX_DEV bool needs_care() const { return (uint32_t)(base - low) > span; }
   // lane L takes v of lane L + 1, lane 63 keeps `last`
   static BPSX_DEV uint32_t down1(uint32_t last, uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp((int)last, (int)v, 0x130 /* wave_shl:1 */, 0xf, 0xf, false);
@@ -210,48 +248,43 @@ struct OpenList {
   static BPSX_DEV uint32_t up1(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x138 /* wave_shr:1 */, 0xf, 0xf, true);
   }
-  // The entries of lanes `rest` (totals tb, nodes `packed`) enter the first 64, which have room for them, one after the
-  // other, each behind those with totals up to its own: every lane keeps its entry, takes the new one or
-  // the one before it, and its total is the middle one of three.  As one piece: twelve instructions an entry, none
-  // of which waits for the scalar unit, in an order that keeps the distances that this hardware asks for and does
+  // The entries of lanes `rest` (totals tb, nodes `packed`) enter, one after the other: every lane takes the smaller of the
+  // entry above its own and the greater of its own and the new one.  As one piece, two entries a round, nine instructions each, of
+  // which none waits for the scalar unit, in an order that keeps the distances that this hardware asks for and does
   // not watch over, two instructions between a vector instruction that writes a scalar register (a
-  // comparison, a lane read) and the vector instruction that reads it, and between one that writes
-  // a register and the lane move that reads it.
+  // lane read) and the vector instruction that reads it, and between one that writes
+  // a register and the lane move that reads it.  With an odd number the last round's second is lane 63 (the first of an
+  // empty mask, taken modulo 64), where tb is all ones: a NaN, which minima and maxima leave out.
   BPSX_DEV void enter(unsigned long long rest, uint32_t tb, uint32_t packed) {
-    uint32_t tp, np, vn, st, sn;
+    unsigned long long above, greater;
     int at;
-    unsigned long long above;
+    const unsigned long long end = entry(kEmpty, kNone);   // what lane 63, which has no lane above it, has there
     asm volatile("s_cmp_eq_u64 %[rest], 0\n\t"
                  "s_cbranch_scc1 2f\n"
                  "1:\n\t"
                  "s_ff1_i32_b64 %[at], %[rest]\n\t"
                  "s_bitset0_b64 %[rest], %[at]\n\t"
-                 "v_readlane_b32 %[st], %[tb], %[at]\n\t"
-                 "v_readlane_b32 %[sn], %[packed], %[at]\n\t"
-                 "v_mov_b32_dpp %[tp], %[t] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
-                 "v_mov_b32_dpp %[np], %[n] wave_shr:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
-                 "v_cmp_lt_u32_e64 %[above], %[st], %[t]\n\t"
-                 "v_mov_b32 %[vn], %[sn]\n\t"
-                 "v_cmp_lt_u32_e32 vcc, %[st], %[tp]\n\t"
-                 "v_med3_u32 %[t], %[tp], %[st], %[t]\n\t"
-                 "v_cndmask_b32_e64 %[n], %[n], %[vn], %[above]\n\t"
+                 "v_readlane_b32 vcc_lo, %[packed], %[at]\n\t"
+                 "v_readlane_b32 vcc_hi, %[tb], %[at]\n\t"
+                 "v_mov_b32_dpp v42, v40 wave_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mov_b32_dpp v43, v41 wave_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_max_f64 v[44:45], vcc, v[40:41]\n\t"
+                 "s_ff1_i32_b64 %[at], %[rest]\n\t"
+                 "s_bitset0_b64 %[rest], %[at]\n\t"
+                 "v_min_f64 v[40:41], v[42:43], v[44:45]\n\t"
+                 "v_readlane_b32 vcc_lo, %[packed], %[at]\n\t"
+                 "v_readlane_b32 vcc_hi, %[tb], %[at]\n\t"
+                 "v_mov_b32_dpp v42, v40 wave_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mov_b32_dpp v43, v41 wave_shl:1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_max_f64 v[44:45], vcc, v[40:41]\n\t"
                  "s_cmp_lg_u64 %[rest], 0\n\t"
-                 "v_cndmask_b32_e32 %[n], %[n], %[np], vcc\n\t"
+                 "v_min_f64 v[40:41], v[42:43], v[44:45]\n\t"
                  "s_cbranch_scc1 1b\n\t"
                  "s_nop 1\n"
                  "2:"
-                 : [rest] "+s"(rest), [t] "+v"(t[0]), [n] "+v"(n[0]), [tp] "=&v"(tp), [np] "=&v"(np), [vn] "=&v"(vn), [st] "=&s"(st), [sn] "=&s"(sn),
-                   [at] "=&s"(at), [above] "=&s"(above)
-                 : [tb] "v"(tb), [packed] "v"(packed)
+                 : [rest] "+s"(rest), "+{v[40:41]}"(e), "={v[42:43]}"(above), "=&{v[44:45]}"(greater), [at] "=&s"(at)
+                 : [tb] "v"(tb), [packed] "v"(packed), "2"(end)
                  : "vcc", "scc");
-  }
-  // One entry, total and node the same for all lanes, in the lanes of `within`.
-  BPSX_DEV void enter_within(uint32_t total, uint32_t node, unsigned long long within) {
-    const uint32_t tp = up1(t[0]), np = up1(n[0]);
-    const unsigned long long above = lanes_where(t[0] > total) & within, shifted = lanes_where(tp > total) & within;
-    t[0] = pick(shifted, tp, pick(above, total, t[0]));
-    n[0] = pick(shifted, np, pick(above, node, n[0]));
-    asm volatile("s_nop 1" : "+v"(t[0]), "+v"(n[0]));   // as above, before the next lane move
   }
   // v as a select operand under a lane mask that a scalar instruction has written (the compiler does not know the
   // select for a vector instruction, which has to keep two instructions' distance from a comparison: a mask that a
@@ -261,122 +294,34 @@ struct OpenList {
     asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(no), "v"(yes), "s"(mask));
     return r;
   }
-  // A pass's changes at once: the first c entries leave, and so does the entry of every node in lanes
-  // `known` that has one (a modify; a node without an entry is pushed); the nodes in lanes `upd`,
-  // packed and with total bits tb, enter behind the entries with totals up to theirs.  P: register
-  // pairs in use (64 entries each).  buf: 128 entries in LDS.
-  // Every entry's new place is counted, then all of them move through LDS: an old entry's place is
-  // the number of entries before it that stay plus that of new totals below its own, a new one's
-  // the number of old entries up to it plus that of new ones before it.  Per new entry that is one
-  // comparison with the old ones and one with the other new ones, and no comparison waits for the one
-  // before.  (One insertion after the other, each a shift of the list behind the place that a
-  // comparison found, is a chain of some ten dependent steps per entry and register pair: k_geodesic
-  // then took 1.229 ms instead of 1.207 at 16384 agents over mazes, 3.11 instead of 2.59 at 4096
-  // over cluttered plans, whose lists fill two to four pairs, 1.16 instead of 0.99 at 1024 over room
-  // plans, where a launch lasts as long as its longest search alone.)
-  // meanwhile() is called while the entries come back from LDS.
+  // A pass's changes: the first c entries leave, and so does the entry of every node in lanes
+  // `known` that has one here (a modify; a node without an entry is pushed); the nodes in lanes `upd`,
+  // packed and with total bits tb, enter.
   // Returns the node of entry `row` of the new list and the total of the one behind it (of kNone and kEmpty
   // where there is none).
-  template <int P, class Meanwhile> BPSX_DEV uint2 merge(uint2* buf, int c, unsigned long long upd, unsigned long long known, uint32_t tb,
-                                                         uint32_t packed, int lane, int row, Meanwhile meanwhile) {
-    if constexpr (P == 1) {
-      // Within 64 entries those that leave go by a lane permute, and the new ones enter one after the other.
-      // (Counted into place together and moved through LDS as the longer lists are: steps of 16384 agents
-      // over mazes 884 us, now 854, of 65536 over mixed scenes 3150 and 3078, of 64 179 and 170.)
-      uint32_t from = (uint32_t)(lane + c) * 4u;
-      from = from < 252u ? from : 252u;
-      t[0] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)from, (int)t[0]);
-      n[0] = (uint32_t)__builtin_amdgcn_ds_bpermute((int)from, (int)n[0]);
-      meanwhile();
-      size += __popcll(upd) - c;
-      enter(upd & ~known, tb, packed);
-      // one whose node has an entry already (a modify; its total only falls) moves up from there to its place, one
-      // without is a push
-      while (known) {
-        const int src = first_lane(known);
-        known = without_lane(known, src);
-        const uint32_t node = rlane(packed, src);
-        const unsigned long long old = lanes_where(n[0] == node) & lanes_where(t[0] != kEmpty);
-        size -= __popcll(old);
-        enter_within(rlane(tb, src), node, old ^ (old - 1ull));   // up to its old place, or everywhere
-      }
-      wave_sync();
-      return make_uint2((uint32_t)__builtin_amdgcn_ds_bpermute(row * 4, (int)n[0]), (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4 + 4, (int)t[0]));
-    } else {
-    unsigned long long dead[P];
-#pragma unroll
-    for (int k = 0; k < P; ++k) dead[k] = 0;
-    dead[0] = lane_range(c, 0);
+  BPSX_DEV uint2 merge(int c, unsigned long long upd, unsigned long long known, uint32_t tb, uint32_t packed, int row) {
+    base += c;
+    const unsigned long long left = lane_range(base, 0);
+    e = in_mask(left) ? 0ull : e;
+    const int n = __popcll(upd);
     while (known) {
       const int src = first_lane(known);
       known = without_lane(known, src);
-      const uint32_t node = rlane(packed, src);
-#pragma unroll
-      for (int k = 0; k < P; ++k) dead[k] |= lanes_where(n[k] == node);
+      const unsigned long long old = lanes_where(node() == rlane(packed, src));   // (kNone is no node that is updated)
+      if (!old) continue;
+      // those below it move up a lane
+      const unsigned long long upTo = old ^ (old - 1ull);
+      const uint32_t t = up1(total()), nd = up1(node());
+      e = in_mask(upTo) ? entry(t, nd) : e;
+      base++;
     }
-    uint32_t pos[P];
-    int live = 0;
-#pragma unroll
-    for (int k = 0; k < P; ++k) {
-      pos[k] = (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(~dead[k] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)~dead[k], (uint32_t)live));
-      live += __popcll(~dead[k]);
-    }
-    size += __popcll(upd) - (64 * P - live);
-    uint32_t upTo = 0, before = 0;
-    const unsigned long long key = ((unsigned long long)tb << 32) | (uint32_t)lane;   // equal totals in lane order
-    const unsigned long long enters = upd;
-    uint2 front;
-    // Two at a time, so that one's lane moves fill the other's waits.  With an odd number the last
-    // round's second is lane 63 (first_lane of an empty mask, taken modulo 64): no edge's lane, its
-    // total is above all keys and counts nowhere.
-    while (upd) {
-      const int sa = first_lane(upd);
-      upd = without_lane(upd, sa);
-      const int sb = first_lane(upd);
-      upd = without_lane(upd, sb);
-      const uint32_t ta = rlane(tb, sa), tc = rlane(tb, sb);
-      int la = 0, lb = 0;
-#pragma unroll
-      for (int k = 0; k < P; ++k) {
-        const bool above = t[k] > ta, above2 = t[k] > tc;
-        la += __popcll(~(lanes_where(above) | dead[k]));
-        lb += __popcll(~(lanes_where(above2) | dead[k]));
-        pos[k] += above;
-        pos[k] += above2;
-      }
-      before += key > (((unsigned long long)ta << 32) | (uint32_t)sa);
-      before += key > (((unsigned long long)tc << 32) | (uint32_t)sb);
-      upTo = wlane(upTo, (uint32_t)la, sa);
-      upTo = wlane(upTo, (uint32_t)lb, sb);
-    }
-    const uint32_t place = upTo + before;
-      unsigned long long moves[P];
-      static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA { constexpr int k = decltype(K)::value; moves[k] = lanes_where(t[k] != kEmpty) & ~dead[k]; });
-      uint32_t nt[P], nn[P];
-      static_for<0, P / 2>([&](auto H) BPSX_INLINE_LAMBDA {
-        constexpr int half = decltype(H)::value;
-        static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA {
-          constexpr int k = decltype(K)::value;
-          lds_store_where(moves[k] & lanes_where((pos[k] >> 7) == (uint32_t)half), &buf[pos[k] & 127u], t[k], n[k]);
-        });
-        lds_store_where(enters & lanes_where((place >> 7) == (uint32_t)half), &buf[place & 127u], tb, packed);
-        wave_sync();
-        if (half == 0) front = make_uint2(buf[row].y, buf[row + 1].x);
-        const uint2 e0 = buf[lane], e1 = buf[64 + lane];
-        if (half == 0) meanwhile();
-        constexpr int k = 2 * half;
-        nt[k] = 64 * k + lane < size ? e0.x : kEmpty;
-        nn[k] = 64 * k + lane < size ? e0.y : kNone;
-        nt[k + 1] = 64 * k + 64 + lane < size ? e1.x : kEmpty;
-        nn[k + 1] = 64 * k + 64 + lane < size ? e1.y : kNone;
-        wave_sync();
-      });
-      static_for<0, P>([&](auto K) BPSX_INLINE_LAMBDA { constexpr int k = decltype(K)::value; t[k] = nt[k]; n[k] = nn[k]; });
-    wave_sync();
-    front.x = row < size ? front.x : kNone;
-    front.y = row + 1 < size ? front.y : kEmpty;
-    return front;
-    }
+    enter(upd, tb, packed);
+    base -= n;
+    return front(row);
+  }
+  BPSX_DEV uint2 front(int row) const {
+    const int from = (base + row) * 4;
+    return make_uint2((uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)node()), (uint32_t)__builtin_amdgcn_ds_bpermute(from + 4, (int)total()));
   }
 };
 
@@ -393,7 +338,7 @@ struct AstarState {
 
 constexpr uint32_t kFollowEnd = 0xffffu, kFollowQuit = 0xffffffffu;   // see follow
 
-enum AstarExit { kAstarOn = -1, kAstarEmpty = 0, kAstarGoal = 1, kAstarGrowLinks = 2, kAstarGrowHeap = 3, kAstarTie = 4, kAstarLogFull = 5 };
+enum AstarExit { kAstarOn = -1, kAstarEmpty = 0, kAstarGoal = 1, kAstarGrowLinks = 2, kAstarGrowHeap = 3, kAstarTie = 4, kAstarLogFull = 5, kAstarCare = 6 };
 
 // Two correctly rounded square roots, the values sqrtf returns on the host, of arguments that are zero or
 // at least 2^-96 and finite, as squared distances between points of a mesh are; a wavefront that meets
@@ -478,13 +423,11 @@ static_assert((kWindow & (kWindow - 1)) == 0 && kWindow >= 2 * kNvp, "window mus
 struct GeoLds {
   alignas(16) uint16_t first[kHashSize];
   // Node links: polygon index | offset of the next node's link in the hash chain << 16.  Behind them the
-  // marks of which row of a pass updates a polygon first (see astar_fast), all kEndWord between passes
-  // and while chains are walked: the first of them is the word that ends every chain.  A pass's
-  // open list moves to its new order over the marks.
+  // marks of which lane of a pass updates a polygon first (see astar_fast), all kEndWord between passes
+  // and while chains are walked: the first of them is the word that ends every chain.
   alignas(16) uint32_t n_link[kLinksLds + kTagSlots];
   alignas(16) float4 w_node[kWindow];   // position, cost
   BPSX_DEV uint32_t* marks() { return n_link + kLinksLds; }
-  BPSX_DEV uint2* entries() { return reinterpret_cast<uint2*>(n_link + kLinksLds); }   // 128 of them over the marks
 #if BPSX_FOLLOWER
   // What the two wavefronts of a search share (see follow): how far the log has arrived, the heap and its size,
   // the search's state, how far the log has been read, and the entry that a search begins with.
@@ -493,7 +436,7 @@ struct GeoLds {
   uint16_t parents[kMaxNodes];
   uint16_t arrived, unused;
 #endif
-  uint2 ref_heap[64 * OpenList::kPairs + 2 * 8 * kNvp + 2];
+  uint2 ref_heap[354];
   uint2 start;
   uint32_t published, applied, heap_size;
 #if BPSX_WINDOW < 2048
@@ -501,7 +444,7 @@ struct GeoLds {
 #endif
   BPSX_DEV uint2* heap() { return ref_heap; }
 #else
-  BPSX_DEV uint2* heap() { return entries(); }
+  BPSX_DEV uint2* heap() { return reinterpret_cast<uint2*>(n_link + kLinksLds); }
 #endif
 };
 // After A* its LDS is dead; the funnel reuses it for the corridor and its portals.  The
@@ -571,6 +514,11 @@ struct GeoWave {
       lds_store_where(mask & near, lds_address(L->n_link) + i4, v);
       store_where(mask & ~near, ws->links, i4, v);
     }
+  }
+  // The entries that the open list keeps apart, over the links that LDS has places for
+  BPSX_DEV void* far_list() const {
+    static_assert(OpenList::kFarCap * sizeof(uint2) <= kLinksLds * sizeof(uint32_t) && offsetof(GeoSlot, links) % 8 == 0, "the slot's links begin behind them");
+    return ws->links;
   }
   // node i, whose position and cost are not looked for in the window; and a node and its parent index stored outside of it
   BPSX_DEV float4 node(int i) const {
@@ -683,11 +631,11 @@ struct GeoWave {
 // a cluttered plan of 20k polygons ties with a longer list or outgrows the sorted list, and ran
 // again from its start with a heap walked level by level in HBM: 6.6 ms, against 1.5 ms for the
 // longest of the others.)
-constexpr int kHeapLds = kFollower ? 64 * OpenList::kPairs + 2 * kRows * kNvp + 1 : (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
+constexpr int kHeapLds = kFollower ? 353 : (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
 static_assert(kLinksLds % 4 == 0 && offsetof(GeoLds, w_node) == offsetof(GeoLds, n_link) + 4 * (kLinksLds + kTagSlots),
               "the marks are accessed as 16 bytes, and the heap lies over the marks and the window");
 // (383 entries, 353 where a second wavefront keeps it)
-static_assert(kHeapLds >= 64 * OpenList::kPairs + 2 * kRows * kNvp, "a heap with as many entries as the sorted list must fit");
+static_assert(2 * kRows * kNvp <= 2 * 48 && kHeapLds >= OpenList::kMostOfAll + kRows, "a heap with as many entries as the sorted list must fit");
 template <bool Lds> struct RefHeap {
   uint2* h;    // total bits, packed node
   int size, lane;
@@ -927,6 +875,7 @@ BPSX_DEV void follow(GeoLds* L, const GeoSlot* ws, int lane) {
     wave_sync();
     const int arrived = uniform_i((int)__hip_atomic_load(&L->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
     const int end = arrived > asked ? arrived : asked;
+    if (asked) __builtin_amdgcn_s_setprio(3);   // the search waits
     if (pos < end) {
       const unsigned long long r = __hip_atomic_load(log + (pos + lane < end ? pos + lane : pos), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const uint32_t rk = (uint32_t)r, rw = (uint32_t)(r >> 32);
@@ -938,7 +887,7 @@ BPSX_DEV void follow(GeoLds* L, const GeoSlot* ws, int lane) {
       pos += h;
     }
     if (pos != end) continue;
-    if (word != done) answer(word);
+    if (word != done) { answer(word); __builtin_amdgcn_s_setprio(0); }
     else __builtin_amdgcn_s_sleep(2);
   }
 }
@@ -1066,6 +1015,110 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
   }
 }
 
+// The entries that the list keeps apart, looked through: those of nodes that have been updated since are dropped, and the
+// smallest, if the list has room for them, enter it: kPull of them at most if there is a bound that parts so few from
+// the others.  False if the search cannot go on in this form.
+// Bound by two round trips to HBM, for the entries and their nodes, and nine instructions for each that enters; once in ten
+// to fifty passes.
+BPSX_DEV bool refill(const GeoWave& g, OpenList& ol, uint32_t endIp, const float* endPos) {
+  // 63 entries at a time: none in lane 63 (enter)
+  constexpr int kAtOnce = 63, K = OpenList::kFarCap / kAtOnce, kPull = 40, kPullLeast = 16;
+  static_assert(OpenList::kFarCap % kAtOnce == 0, "whole rounds");
+  const int lane = lane_here(g.lane);
+  uint2* apart = reinterpret_cast<uint2*>(g.far_list());
+  uint32_t t[K], n[K];
+  unsigned long long live[K];
+  static_for<0, K>([&](auto J) BPSX_INLINE_LAMBDA {
+    constexpr int k = decltype(J)::value;
+    t[k] = n[k] = 0;
+    if (ol.far > kAtOnce * k) {
+      const uint2 v = apart[kAtOnce * k + lane < ol.far ? kAtOnce * k + lane : 0];
+      t[k] = v.x; n[k] = v.y;
+    }
+  });
+  int count = 0;
+  uint32_t most = 0;
+  static_for<0, K>([&](auto J) BPSX_INLINE_LAMBDA {
+    constexpr int k = decltype(J)::value;
+    live[k] = 0;
+    if (ol.far > kAtOnce * k) {
+      // an entry is its node's if its total is what the node's would be now
+      const float4 p = g.node((int)(n[k] & 0x7ffu));
+      const float ex = endPos[0] - p.x, ey = endPos[1] - p.y, ez = endPos[2] - p.z;
+      const float ee = ex * ex + ey * ey + ez * ez;
+      float toEnd, same;
+      sqrt_exact2(ee, ee, &toEnd, &same);
+      const float heuristic = (n[k] >> 11) == endIp ? 0.0f : toEnd * 0.999f;
+      live[k] = lanes_where(__float_as_uint(p.w + heuristic) == t[k]) & lanes_where(kAtOnce * k + lane < ol.far) & ~(1ull << kAtOnce);
+      count += __popcll(live[k]);
+      const uint32_t mine = in_mask(live[k]) ? t[k] : 0u;
+      most = mine > most ? mine : most;
+    }
+  });
+  const auto below = [&](uint32_t bound) BPSX_INLINE_LAMBDA {
+    int c = 0;
+    static_for<0, K>([&](auto J) BPSX_INLINE_LAMBDA { constexpr int k = decltype(J)::value; c += __popcll(lanes_where(t[k] < bound) & live[k]); });
+    return c;
+  };
+  uint32_t bound = ol.bound;   // below it there is none
+  if (ol.size() < OpenList::kRefill) {
+    bound = OpenList::kEmpty;
+    if (count > kPull) {
+      // the greatest of all lanes, in the last one
+      most = umin_dpp<0x118, 0xf>(umin_dpp<0x114, 0xf>(umin_dpp<0x112, 0xf>(umin_dpp<0x111, 0xf>(~most))));
+      most = ~umin_dpp<0x143, 0xc>(umin_dpp<0x142, 0xa>(most));
+      uint32_t lo = ol.bound, hi = rlane(most, 63) + 1u;   // too few below the one, too many below the other
+      int at_lo = 0, at_hi = count;
+      while (hi - lo > 1u) {
+        const uint32_t mid = lo + (hi - lo) / 2u;
+        const int c = below(mid);
+        if (c > kPull) { hi = mid; at_hi = c; }
+        else { lo = mid; at_lo = c; if (c >= kPullLeast) break; }
+      }
+      // (entries of one total stay together)
+      bound = at_lo >= kPullLeast || at_hi + ol.size() > OpenList::kSplit ? lo : hi;
+    }
+  }
+  int kept = 0;
+  static_for<0, K>([&](auto J) BPSX_INLINE_LAMBDA {
+    constexpr int k = decltype(J)::value;
+    if (live[k]) {
+      const unsigned long long in = lanes_where(t[k] < bound) & live[k], out = live[k] & ~in;
+      ol.enter(in, in_mask(in) ? t[k] : 0xffffffffu, n[k]);
+      ol.base -= __popcll(in);
+      store_where(out, apart, 8u * (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(out >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)out, (uint32_t)kept)), t[k], n[k]);
+      kept += __popcll(out);
+    }
+  });
+  ol.far = kept;
+  ol.bound = kept ? bound : OpenList::kEmpty;
+  return kept <= OpenList::kFarKeep && (!kept || ol.size() >= OpenList::kRefill);
+}
+// The list put in order between two passes, as its limits ask for; full: the next pass has no room for what it adds.
+// (Equal totals that a replay has put in another order leave the list before anything enters it: one that is full is
+// only split.)
+BPSX_DEV bool care_for_list(const GeoWave& g, OpenList& ol, uint32_t endIp, const float* endPos, bool full) {
+  const int lane = lane_here(g.lane);
+  if (!full && (ol.far > OpenList::kFarMost || ol.size() < OpenList::kRefill) && !refill(g, ol, endIp, endPos)) return false;
+  if (full || ol.size() > OpenList::kSplit) {
+    // the greater ones, from the first of their total on
+    const int keep = ol.size() > OpenList::kSplit ? 32 : ol.size() >> 1;
+    const uint32_t bound = rlane(ol.total(), ol.base + keep);
+    if (bound == rlane(ol.total(), ol.base)) return false;
+    const unsigned long long away = lanes_where(ol.total() >= bound) & ~(1ull << OpenList::kEnd);
+    const int n = __popcll(away);
+    store_where(away, g.far_list(), 8u * (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(away >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)away, (uint32_t)ol.far)), ol.total(), ol.node());
+    const int from = (lane - n) * 4;   // of the lanes from n on; zeros come before
+    const uint32_t t = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)ol.total()), nd = (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)ol.node());
+    ol.e = lane == OpenList::kEnd ? ol.e : lane < n ? 0ull : OpenList::entry(t, nd);
+    ol.far += n;
+    ol.base += n;
+    ol.bound = bound;
+  }
+  ol.set_limits();
+  return true;
+}
+
 // The expansion loop with the open list as a sorted array (OpenList), up to kRows nodes per
 // pass.  Row r of kRowLanes lanes works on entry r of the list (lane kRowLanes r + j on edge j
 // of its polygon, the lane after the last edge on the node itself): the edge records of all of them arrive in one load, and node lookup, costs, node
@@ -1089,7 +1142,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
 // node of an earlier one (it sees it as open, the reference as closed): both views lead to
 // the same node state and the same list, because a modify that finds no entry is a push.
 // Returns kAstarTie when the first two entries share the smallest total.
-template <bool S, int P>
+template <bool S>
 BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops,
                              bool frontResolved) {
   const int lane = lane_here(g.lane);
@@ -1107,8 +1160,8 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
   const char* edges_of = reinterpret_cast<const char*>(edges);
   bool resolved = frontResolved;
   // of every row: its entry of the list, and the total of the entry behind that
-  uint32_t cand = (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4, (int)ol.n[0]);
-  uint32_t nextTotal = (uint32_t)__builtin_amdgcn_ds_bpermute(row * 4 + 4, (int)ol.t[0]);
+  const uint2 first = ol.front(row);
+  uint32_t cand = first.x, nextTotal = first.y;
   // Written for few instructions and few waits on the common path: what is rare sits behind one branch
   // each; conditions are lane masks on the scalar unit; LDS reads whose results are needed later go out
   // early (the marks' before the scan over the rows, the chain heads' before the stores); the next
@@ -1169,16 +1222,17 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     insert();
     FM(1);
     if (st.logEnd > kOpLogCap - (1 + kRows * kNvp)) return kAstarLogFull;
+    if (ol.needs_care()) return kAstarCare;
     // ---- how many entries at the front are each the only one with their total, and not the goal
-    const unsigned long long uniq = lanes_where(ol.t[0] < OpenList::down1(OpenList::kEmpty, ol.t[0]));
-    const unsigned long long goal = lanes_where((ol.n[0] >> 11) == endIp);
+    const unsigned long long uniq = lanes_where(ol.total() < OpenList::down1(OpenList::kEmpty, ol.total())) >> ol.base;
+    const unsigned long long goal = lanes_where((ol.node() >> 11) == endIp) >> ol.base;
     uint32_t lim = (uint32_t)first_other_lane(uniq & ~goal);
     lim = lim < (uint32_t)kRows ? lim : (uint32_t)kRows;
     const int bi = (int)(cand & 0x7ffu);
     int pairTie = 0;   // 2: with the goal as one of the two
     uint32_t headerWord = kOpHeader;
     if (__builtin_expect(lim == 0, 0)) {
-      if (ol.size <= 0) return kAstarEmpty;
+      if (ol.base >= OpenList::kEnd) return kAstarEmpty;
       if (uniq & 1ull) lim = (uint32_t)kRows;   // the goal
       else if (resolved) { lim = 1; resolved = false; }   // the caller has put the reference's next node first
       else {
@@ -1339,9 +1393,10 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const int nrec = __popcll(upd);
     const unsigned long long fresh = upd & ~known;
     const int want = g.nodeCount + __popcll(fresh);
-    // Nothing has changed yet: a list that would outgrow its registers goes on in the wider instantiation,
-    // links that would outgrow LDS in the one that spills.
-    if (__builtin_expect(ol.size - (int)c + nrec > (P == 1 ? 63 : 64 * P), 0)) return kAstarGrowHeap;
+    const unsigned long long nearby = upd & lanes_where(tb < ol.bound);
+    // Nothing has changed yet: a list that would outgrow its registers is split first,
+    // links that would outgrow LDS go on in the instantiation that spills.
+    if (__builtin_expect(ol.base + (int)c - __popcll(nearby) < OpenList::kEnd - OpenList::kMost, 0)) return kAstarGrowHeap;
     if (!S && __builtin_expect(want > kLinksLds, 0)) return kAstarGrowLinks;
     (*pops) += c;
     // the reference carries on without the nodes that do not fit, but reports anything found
@@ -1378,9 +1433,16 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       st.logEnd += 1 + nrec;
     };
     FM(8);
+    store();
+    if (upd & ~nearby) {
+      const unsigned long long away = upd & ~nearby;
+      store_where(away, g.far_list(), 8u * (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(away >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)away, (uint32_t)ol.far)), tb, packed);
+      ol.far += __popcll(away);
+      ol.set_limits();
+    }
     FM(9);
     // ---- the open list: the committed entries leave, the updates enter
-    const uint2 front = ol.template merge<P>(L->entries(), (int)c, upd, upd & known, tb, packed, lane, row, store);
+    const uint2 front = ol.merge((int)c, nearby, nearby & known, tb, packed, row);
     cand = front.x;
     nextTotal = front.y;
     FM(10);
@@ -1437,27 +1499,22 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
 #endif
   st.ol.init(lane, __float_as_uint(total), startIp << 11);
   // the loop is instantiated for links in LDS only or spilling (one instantiation where the LDS
-  // holds all links), and for a list within one register pair, two or four; a search moves on when
-  // one more pass could outgrow what it runs in
+  // holds all links); a search moves on when one more pass could outgrow what it runs in
   AstarExit ex;
   bool resolved = false;
   bool spill = kLinksLds >= kMaxNodes;
-  int pairs = 1;   // register pairs of the list in use
+  int cared = -1, times = 0;   // where the log was when the list was last put in order, and how often it was there
   for (;;) {
-#define BPSX_FAST_RUN(SP) (pairs == 1 ? astar_fast<SP, 1>(g, st, edges, endIp, endPos, pops, resolved) : \
-                           pairs == 2 ? astar_fast<SP, 2>(g, st, edges, endIp, endPos, pops, resolved) : \
-                                        astar_fast<SP, 4>(g, st, edges, endIp, endPos, pops, resolved))
-    if constexpr (kLinksLds >= kMaxNodes) ex = BPSX_FAST_RUN(true);
-    else ex = spill ? BPSX_FAST_RUN(true) : BPSX_FAST_RUN(false);
-#undef BPSX_FAST_RUN
+    if constexpr (kLinksLds >= kMaxNodes) ex = astar_fast<true>(g, st, edges, endIp, endPos, pops, resolved);
+    else ex = spill ? astar_fast<true>(g, st, edges, endIp, endPos, pops, resolved) : astar_fast<false>(g, st, edges, endIp, endPos, pops, resolved);
     resolved = false;
-    if (ex == kAstarGrowLinks) { g.clear_marks(); g.linkSpills++; spill = true; continue; }   // as below
-    if (ex == kAstarGrowHeap && pairs < OpenList::kPairs) {
-      g.clear_marks();   // the pass that did not fit has left its own
-      // the list grows into further registers, empty so far
-      if (pairs == 1) { st.ol.clear_pair(1); pairs = 2; }
-      else { st.ol.clear_pair(2); st.ol.clear_pair(3); pairs = 4; }
-      continue;
+    if (ex == kAstarGrowLinks) { g.clear_marks(); g.linkSpills++; spill = true; continue; }   // the pass that did not fit has left its marks
+    if (ex == kAstarCare || ex == kAstarGrowHeap) {
+      g.clear_marks();
+      // (a list that is not in order after a few rounds, of equal totals, does not come to be)
+      times = cared == st.logEnd ? times + 1 : 0;
+      cared = st.logEnd;
+      if (times < 4 && care_for_list(g, st.ol, endIp, endPos, ex == kAstarGrowHeap)) continue;
     }
     if (ex == kAstarEmpty || ex == kAstarGoal) break;
     __builtin_amdgcn_s_setprio(3);   // a search that pays for a replay is late from here on
@@ -1471,16 +1528,15 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
 #else
     replay_log(g, st);
 #endif
-    // The reference pops what its heap has at the root: that entry goes first.  Equal totals have no
-    // defined order in the list, so where more than 64 share the smallest one (an end point so far away
-    // that a step's length is lost in the total's rounding) it may be none of the list's first 64.
-    const unsigned long long root = lanes_where(st.ol.n[0] == st.replayRoot && st.ol.t[0] == rlane(st.ol.t[0], 0));
-    if (ex == kAstarTie && root && st.replaySize == st.ol.size) {
+    // The reference pops what its heap has at the root: that entry goes first, and what was before it moves up a lane,
+    // in the order that it has.
+    const unsigned long long root = lanes_where(st.ol.node() == st.replayRoot && st.ol.total() == rlane(st.ol.total(), st.ol.base));
+    if (ex == kAstarTie && root) {
       restore_window(g);
       g.tieReplays++;
-      const uint32_t front = rlane(st.ol.n[0], 0);
-      st.ol.n[0] = wlane(st.ol.n[0], st.replayRoot, 0);
-      st.ol.n[0] = wlane(st.ol.n[0], front, first_lane(root));
+      const uint32_t before = OpenList::up1(st.ol.node());
+      const uint32_t node = in_mask(root | (root - 1ull)) ? (lane == st.ol.base ? st.replayRoot : before) : st.ol.node();
+      st.ol.e = lane < st.ol.base ? 0ull : OpenList::entry(st.ol.total(), node);
       resolved = true;
       continue;
     }

@@ -8,7 +8,7 @@ of new nodes that share a bucket, 9 list updates, 10 end of the pass.
 
     python tests/measure_astar_loop_phases.py
         No GPU needed.  Compiles kernels.hip to assembly with the Makefile's own options and counts,
-        for the loop's most used instantiation (links in LDS, list in one register pair) inside
+        for the loop's most used instantiation (links in LDS) inside
         k_geodesic, the instructions between consecutive marks in the order the compiler laid them
         out, by class: vector ALU, scalar ALU, branch, LDS, memory, waits.  Blocks that the compiler
         moved out of line (rare cases) are counted where they lie, and a loop inside a phase (the
@@ -70,7 +70,7 @@ def static_counts():
     body = text[start:end]
     marks = {}
     for i, l in enumerate(body):
-        m = re.search(r"; astar_fast spill=0 pairs=1 mark=(\d+)", l)
+        m = re.search(r"; astar_fast spill=0 mark=(\d+)", l)
         if m:
             marks[int(m.group(1))] = i
     assert sorted(marks) == list(range(11)), "marks of the loop not found in the assembly"
@@ -87,7 +87,7 @@ def static_counts():
             break
     rows.append((PHASES[10], body[marks[10]:tail_end + 1] + body[header:marks[0]]))
     classes = ["valu", "salu", "branch", "lds", "mem", "smem", "wait"]
-    print("instructions between the marks of astar_fast<links in LDS, one register pair> in k_geodesic, as laid out by the compiler")
+    print("instructions between the marks of astar_fast<links in LDS> in k_geodesic, as laid out by the compiler")
     print("%-26s" % "phase" + "".join("%8s" % c for c in classes))
     total = dict.fromkeys(classes, 0)
     for name, lines in rows:
