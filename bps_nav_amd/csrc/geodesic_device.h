@@ -1568,20 +1568,12 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   static_assert(kTagSlots * sizeof(uint32_t) >= kMaxPath * sizeof(uint16_t), "the walk must fit the marks it reuses");
   uint16_t* walk = reinterpret_cast<uint16_t*>(g.L->marks());
   wave_sync();
-#if BPSX_FOLLOWER
-  // the follower's heap lies behind the window, and is free once it is done with the search: parents that the window
-  // does not hold go there (one of 256 nodes holds them all)
-  if (!kAllLds) g.settle(g.epoch | kFollowEnd);
-  [[maybe_unused]] constexpr size_t kBehind = sizeof(g.L->ref_heap);
-  static_assert(kAllLds || offsetof(GeoLds, ref_heap) == offsetof(GeoLds, w_node) + kWindow * sizeof(float4), "one place behind the other");
-#else
-  [[maybe_unused]] constexpr size_t kBehind = 0;
-#endif
 #if BPSX_WINDOW >= 2048
   const uint16_t* lparent = g.L->parents;
   constexpr int inLds = kMaxNodes;
 #else
-  constexpr int kParentsLds = (int)((kWindow * sizeof(float4) + kBehind) / sizeof(uint16_t));
+  // (of 256 nodes it holds them all.  The follower may still be at work on its heap: waiting for it cost a search 8 us)
+  constexpr int kParentsLds = (int)(kWindow * sizeof(float4) / sizeof(uint16_t));
   uint16_t* lparent = reinterpret_cast<uint16_t*>(g.L->w_node);
   const int inLds = g.nodeCount < kParentsLds ? g.nodeCount : kParentsLds;
   {
