@@ -1599,13 +1599,12 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
 
 // String pulling over F->corridor[0..n) and the summed length; +inf for every outcome the
 // reference maps to "no path" (straight path of 256 points or more, missing portal).
-// A serial walk over the corridor's portals, bound by its instructions.  The tests of one portal are made at
-// once, by a lane each: five areas, of which one comparison of all lanes says what a portal
-// changes, where each test by all lanes alike and a branch behind it came to 600 cycles a portal.  The corridor's
-// edges are compared in registers, and its two end points projected next to each other, a lane
-// per edge.  (Of a search of 500 nodes over a maze, whose corridor has 72 polygons, 40 us of 390 went here.  Steps of
-// 64 agents 170 -> 161 us, of 1024 over room plans 651 -> 634, of 3007 fleeing ones 656 -> 566, a reset
-// of 2048 over mazes 483 -> 463.)
+// Bound by its instructions: a round of sixteen portals is some 130 of them and ends with a move of the apex as a rule, after
+// five or six portals on average.  The corridor's edges are compared in registers, and its two end points projected next to each
+// other, a lane per edge.  (One portal after the other, its five areas a lane each, took 600 to 750 cycles a portal: 23 us of
+// the 176 of a search over mazes when each has a wavefront to itself, 29 of 241 among 20 wavefronts per CU.  Steps of 64
+// agents 141 -> 135 us, of 1024 over room plans 492 -> 484, of 16384 over mazes 779 -> 757, of 65536 over mixed scenes 2655 ->
+// 2541, a reset of 2048 over mazes 433 -> 421, 300 queries over room plans 264 -> 254.)
 BPSX_DEV float funnel_length(int lane, FunnelLds* F, const NavData& nav, const SceneDev& s, int n, const float* startPos,
                              const float* endPos) {
   const float INF = __int_as_float(0x7f800000);
@@ -1689,19 +1688,27 @@ BPSX_DEV float funnel_length(int lane, FunnelLds* F, const NavData& nav, const S
     if (isEnd) finished = true;
   };
   if (n > 1) {
-    // The funnel's sides are kept relative to its apex, in the lanes that test them: lanes 0 to 3 have (side,
-    // point tested against it) = (right, portal's right), (left, right), (left, left), (right, left), lane 4 the
-    // portal's own right and left.  An area's sign is turned in lanes 0, 3 and 4, so that "not outside" (lanes 0,
-    // 2) reads >= 0 and "not across" (1, 3, 4) > 0.
-    const uint32_t turn = lane == 0 || lane == 3 || lane == 4 ? 0x80000000u : 0u;
-    const float* tested = &F->portals[0][lane < 2 ? 3 : 0];
-    float ax = cs[0], ay = cs[1], az = cs[2];
-    float sx = ax - ax, sy = ay - ay, sz = az - az;   // the side of lanes 0 to 3 (0, or NaN for an apex that is not finite, as the difference is)
+    // Sixteen portals at a time: the first sixteen lanes have their right points, the next their left ones, relative to the
+    // apex and, the left ones, mirrored, so that one rule serves both: a point that does not lie outside its side becomes
+    // the side.  What the sides are behind each portal is a scan, of the narrower of two points; the comparisons of rounded
+    // areas need not be transitive, so every portal's own test, against the side that the scan has put before it,
+    // is made too, and where one of them says otherwise than the scan the round ends before that portal.  The first portal at
+    // which a point crosses to the other side moves the apex.  A point's third word: its portal's index + 1 (0: the apex), and
+    // whether it lies at the apex (vequal).
+    const bool isLeft = (lane & 16) != 0;
+    const uint32_t mirror = isLeft ? 0x80000000u : 0u, kAtApex = 0x10000u;
+    const int j = lane & 15;
+    const float* mine = &F->portals[0][isLeft ? 0 : 3];
     const float thr = (1.0f / 16384.0f) * (1.0f / 16384.0f);
-    auto sides_at_apex = [&]() { return (uint32_t)lanes_where(sx * sx + sy * sy + sz * sz < thr); };   // vequal(apex, side)
-    uint32_t atApex = sides_at_apex();
-    int apexIndex = 0, leftIndex = 0, rightIndex = 0;
-    int leftMoved = 0, rightMoved = 0;       // since the apex last moved: the side is a portal's point
+    float ax = cs[0], ay = cs[1], az = cs[2];
+    struct Side { float x, z; uint32_t at; } side;
+    auto narrow = [&]() BPSX_INLINE_LAMBDA {   // both sides at the apex (0, or NaN for an apex that is not finite, as the difference is)
+      const float x = ax - ax, y = ay - ay, z = az - az;
+      side = {x, z, x * x + y * y + z * z < thr ? kAtApex : 0u};
+    };
+    narrow();
+    auto area = [](float sx, float sz, float px, float pz) BPSX_INLINE_LAMBDA { return px * sz - sx * pz; };   // tri_area2d(apex, side, point)
+    int apexIndex = 0;
     int leftLast = -1, rightLast = -1;       // the portal whose point the side was last: the last one is "poly ref == 0" of the reference
     int i = 0;
     {
@@ -1711,53 +1718,70 @@ BPSX_DEV float funnel_length(int lane, FunnelLds* F, const NavData& nav, const S
       if (all(dist_pt_seg_sqr2d(ax, az, l, r, t) < 0.001f * 0.001f)) i = 1;
     }
     while (i < n) {
-      const float* c = tested + 6 * i;
-      const float px = c[0], py = c[1], pz = c[2];
-      const float cx = px - ax, cz = pz - az;
-      // lane 4 has the portal's right for its side: lane 0's point (into the second four lanes of sixteen)
-      const float bx = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(sx), __float_as_int(cx), 0x114 /* row_shr:4 */, 0xf, 0x2, false));
-      const float bz = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(sz), __float_as_int(cz), 0x114 /* row_shr:4 */, 0xf, 0x2, false));
-      const float area = __uint_as_float(__float_as_uint(cx * bz - bx * cz) ^ turn);
-      const uint32_t m = ((uint32_t)lanes_where(area >= 0.0f) & 0x05u) | ((uint32_t)lanes_where(area > 0.0f) & 0x1au);
-      const int at = i++;
-      if (!(m & 0x05u)) continue;   // both points outside: the funnel stays as it is
-      // the right point, then the left one with the right side as it then is
-      const uint32_t rightIn = m & 1u, leftIn = m & 4u;
-      const uint32_t across = rightIn ? m >> 4 : m >> 3;   // the left point against that right side
-      const uint32_t rightStops = rightIn & ~(atApex | (m >> 1)), leftStops = leftIn & ~(atApex | (across << 2));
-      if (__builtin_expect((rightStops | leftStops) != 0, 0)) {
-        if (rightStops) {
-          apexIndex = leftIndex;
-          if (leftMoved) { const float* p = F->portals[leftIndex]; ax = p[0]; ay = p[1]; az = p[2]; }
-        } else {
-          if (rightIn) { rightIndex = rightLast = at; rightMoved = 1; }
-          apexIndex = rightIndex;
-          if (rightMoved) { const float* p = F->portals[rightIndex] + 3; ax = p[0]; ay = p[1]; az = p[2]; }
-        }
-        const float apex[3] = {ax, ay, az};
-        append(apex, (rightStops ? leftLast : rightLast) + 1 == n);
-        if (finished) break;
-        sx = ax - ax; sy = ay - ay; sz = az - az;
-        atApex = sides_at_apex();
-        leftMoved = rightMoved = 0;
-        leftIndex = rightIndex = apexIndex;
-        i = apexIndex + 1;
+      const int k = i + j;
+      const float* p = mine + 6 * (k < n ? k : n - 1);
+      Side own, in, ex;
+      const float px = p[0] - ax, py = p[1] - ay;
+      own.z = p[2] - az;
+      own.at = (uint32_t)(k + 1) | (px * px + py * py + own.z * own.z < thr ? kAtApex : 0u);
+      own.x = __uint_as_float(__float_as_uint(px) ^ mirror);
+      in = own;
+      if (j == 0 && !(area(side.x, side.z, own.x, own.z) <= 0.0f)) in = side;
+      static_for<0, 4>([&](auto K) BPSX_INLINE_LAMBDA {
+        constexpr int up = 0x110 + (1 << decltype(K)::value);   // row_shr: that many lanes up
+        const float ox = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(in.x), __float_as_int(in.x), up, 0xf, 0xf, false));
+        const float oz = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(in.z), __float_as_int(in.z), up, 0xf, 0xf, false));
+        const uint32_t oat = (uint32_t)__builtin_amdgcn_update_dpp((int)in.at, (int)in.at, up, 0xf, 0xf, false);
+        const bool narrower = area(ox, oz, in.x, in.z) <= 0.0f;
+        in.x = narrower ? in.x : ox;
+        in.z = narrower ? in.z : oz;
+        in.at = narrower ? in.at : oat;
+      });
+      // the sides before each portal
+      ex.x = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(side.x), __float_as_int(in.x), 0x111, 0xf, 0xf, false));
+      ex.z = __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(side.z), __float_as_int(in.z), 0x111, 0xf, 0xf, false));
+      ex.at = (uint32_t)__builtin_amdgcn_update_dpp((int)side.at, (int)in.at, 0x111, 0xf, 0xf, false);
+      const bool moves = area(ex.x, ex.z, own.x, own.z) <= 0.0f;
+      const bool differs = in.at != (moves ? own.at : ex.at);
+      // the other side: for a right point the left one before the portal, for a left point the right one behind it
+      const uint32_t sx = __float_as_uint(isLeft ? ex.x : in.x), sz = __float_as_uint(isLeft ? ex.z : in.z);
+      const auto tx = __builtin_amdgcn_permlane16_swap(sx, sx, false, false), tz = __builtin_amdgcn_permlane16_swap(sz, sz, false, false);
+      const float ox = -__uint_as_float(isLeft ? tx[0] : tx[1]), oz = __uint_as_float(isLeft ? tz[0] : tz[1]);   // mirrored as this lane's points
+      const bool within = area(ox, oz, own.x, own.z) > 0.0f;
+      const uint32_t valid = (n - i >= 16 ? 0xffffu : (1u << (n - i)) - 1u) * 0x10001u;
+      const uint32_t bad = (uint32_t)lanes_where(differs) & valid;
+      const uint32_t stops = (uint32_t)(lanes_where(moves) & ~(lanes_where((ex.at & kAtApex) != 0) | lanes_where(within))) & valid;
+      // the first portals of either kind, 16 or more for none
+      const int badAt = __builtin_ctz(((bad | (bad >> 16)) & 0xffffu) | 0x10000u);
+      const int rightStop = __builtin_ctz((stops & 0xffffu) | 0x10000u), leftStop = __builtin_ctz((stops >> 16) | 0x10000u);
+      const int stop = rightStop < leftStop ? rightStop : leftStop;
+      if (stop >= badAt || stop == 16) {
+        int m = n - i < 16 ? n - i : 16;
+        m = badAt < m ? badAt : m;
+        const uint32_t ra = rlane(in.at, m - 1), la = rlane(in.at, m + 15);
+        side.x = isLeft ? lane_f(in.x, m + 15) : lane_f(in.x, m - 1);
+        side.z = isLeft ? lane_f(in.z, m + 15) : lane_f(in.z, m - 1);
+        side.at = isLeft ? la : ra;
+        if (ra & 0xffffu) rightLast = (int)(ra & 0xffffu) - 1;
+        if (la & 0xffffu) leftLast = (int)(la & 0xffffu) - 1;
+        i += m;
         continue;
       }
-      // the sides that move: of each lane, the point that its side moves to
-      const float cy = py - ay;
-      const float nx = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(cx), 0x28 /* quad_perm:[0,2,2,0] */, 0xf, 0xf, true));
-      const float ny = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(cy), 0x28 /* quad_perm:[0,2,2,0] */, 0xf, 0xf, true));
-      const float nz = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(cz), 0x28 /* quad_perm:[0,2,2,0] */, 0xf, 0xf, true));
-      const unsigned long long moves = 9u * rightIn + 6u * (leftIn >> 2);
-      sx = in_mask(moves) ? nx : sx;
-      sy = in_mask(moves) ? ny : sy;
-      sz = in_mask(moves) ? nz : sz;
-      atApex = sides_at_apex();
-      if (rightIn) rightIndex = rightLast = at;
-      if (leftIn) leftIndex = leftLast = at;
-      rightMoved |= (int)rightIn;
-      leftMoved |= (int)leftIn;
+      const bool atRight = rightStop <= leftStop;   // of one portal the right point comes first
+      const int ra = (int)(rlane(atRight ? ex.at : in.at, stop) & 0xffffu), la = (int)(rlane(ex.at, stop + 16) & 0xffffu);
+      if (ra) rightLast = ra - 1;
+      if (la) leftLast = la - 1;
+      const int to = atRight ? la : ra;
+      if (to) {
+        apexIndex = to - 1;
+        const float* q = F->portals[apexIndex] + (atRight ? 0 : 3);
+        ax = q[0]; ay = q[1]; az = q[2];
+      }
+      const float apex[3] = {ax, ay, az};
+      append(apex, (atRight ? leftLast : rightLast) + 1 == n);
+      if (finished) break;
+      narrow();
+      i = apexIndex + 1;
     }
   }
   if (!finished) {
