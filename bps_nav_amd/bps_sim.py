@@ -293,7 +293,7 @@ class PointNavRolloutGenerator:
     def snap_points(self, scene, pts):
         pts = np.ascontiguousarray(pts, np.float32).reshape(-1, 3)
         n = len(pts)
-        xyz, ref = np.zeros((n, 3), np.float32), np.zeros(n, np.uint32)
+        xyz, ref = np.empty((n, 3), np.float32), np.empty(n, np.uint32)
         _lib.check(self._L.bpsx_snap_points(self._h, scene, pts.ctypes.data, n, xyz.ctypes.data, ref.ctypes.data))
         return xyz, ref
 
@@ -302,7 +302,7 @@ class PointNavRolloutGenerator:
         exyz = np.ascontiguousarray(exyz, np.float32).reshape(-1, 3)
         sref = np.ascontiguousarray(sref, np.uint32)
         n = len(sxyz)
-        xyz, ref = np.zeros((n, 3), np.float32), np.zeros(n, np.uint32)
+        xyz, ref = np.empty((n, 3), np.float32), np.empty(n, np.uint32)
         _lib.check(self._L.bpsx_try_steps(self._h, scene, sxyz.ctypes.data, sref.ctypes.data, exyz.ctypes.data, n,
                                           xyz.ctypes.data, ref.ctypes.data))
         return xyz, ref
@@ -313,7 +313,7 @@ class PointNavRolloutGenerator:
         sref = np.ascontiguousarray(sref, np.uint32)
         eref = np.ascontiguousarray(eref, np.uint32)
         n = len(sxyz)
-        out = np.zeros(n, np.float32)
+        out = np.empty(n, np.float32)
         _lib.check(self._L.bpsx_geodesic(self._h, scene, sxyz.ctypes.data, sref.ctypes.data, exyz.ctypes.data,
                                          eref.ctypes.data, n, out.ctypes.data))
         return out
@@ -337,7 +337,7 @@ class PointNavRolloutGenerator:
     def random_points(self, scene, u):
         u = np.ascontiguousarray(u, np.float32).reshape(-1, 3)
         n = len(u)
-        xyz, ref = np.zeros((n, 3), np.float32), np.zeros(n, np.uint32)
+        xyz, ref = np.empty((n, 3), np.float32), np.empty(n, np.uint32)
         _lib.check(self._L.bpsx_random_points(self._h, scene, u.ctypes.data, n, xyz.ctypes.data, ref.ctypes.data))
         return xyz, ref
 

@@ -234,6 +234,8 @@ struct bpsx_sim {
   uint64_t profiled_steps = 0;
   // scratch for the batched query entry points
   void* d_batch = nullptr;
+  char* h_stage = nullptr;   // pinned: the host arrays of batched calls pass through it (BatchArrays)
+  size_t stage_bytes = 0;
   size_t batch_bytes = 0;
   GeoSlot* d_batch_slots = nullptr;   // node pools of a batch of path queries that needs more wavefronts than the steps have
   uint32_t batch_slots = 0;
@@ -681,6 +683,7 @@ void bpsx_destroy(bpsx_sim* sim) {
   }
   for (void* p : sim->owned) (void)hipFree(p);
   if (sim->d_batch) (void)hipFree(sim->d_batch);
+  if (sim->h_stage) (void)hipHostFree(sim->h_stage);
   if (sim->d_batch_slots) (void)hipFree(sim->d_batch_slots);
   delete sim;
 }
@@ -888,6 +891,73 @@ static int batch_reserve(bpsx_sim* sim, size_t bytes) {
   sim->batch_bytes = bytes;
   return BPSX_OK;
 }
+// The host arrays of a batched call.  Up to kStageMost bytes of them pass through pinned memory that the simulator keeps, and
+// that the kernels read and write where it lies: copies between pageable memory and the device take 10 us each however
+// small, and 33 us for 600 KB, where a copy within host memory takes 7.  Larger calls, and calls that find no pinned memory, copy.
+extern "C++" {
+class BatchArrays {
+ public:
+  // bytes: of all arrays; scratch: device memory besides, returned in *d_scratch
+  int reserve(bpsx_sim* sim, size_t bytes, size_t scratch = 0, void** d_scratch = nullptr) {
+    sim_ = sim;
+    bytes += kArrays * kAlign;
+    staged_ = bytes <= kStageMost;
+    if (staged_ && bytes > sim->stage_bytes) {
+      if (sim->h_stage) HIP_TRY(hipHostFree(sim->h_stage));
+      sim->h_stage = nullptr;
+      sim->stage_bytes = 0;
+      const size_t want = std::min(kStageMost, bytes + bytes / 2);   // calls that grow slowly do not allocate each time
+      if (hipHostMalloc((void**)&sim->h_stage, want, hipHostMallocDefault) == hipSuccess) {
+        sim->stage_bytes = want;
+      } else {
+        (void)hipGetLastError();   // answered here: not an error of the launches to come
+        sim->h_stage = nullptr;
+        staged_ = false;
+      }
+    }
+    const int rc = batch_reserve(sim, scratch + (staged_ ? 0 : bytes));
+    if (rc) return rc;
+    at_ = staged_ ? sim->h_stage : (char*)sim->d_batch + scratch;
+    if (d_scratch) *d_scratch = sim->d_batch;
+    return BPSX_OK;
+  }
+  template <class T> int in(const T* host, size_t count, const T** dev) {
+    T* p = take<T>(count);
+    if (staged_) memcpy(p, host, count * sizeof(T));
+    else HIP_TRY(hipMemcpy(p, host, count * sizeof(T), hipMemcpyHostToDevice));
+    *dev = p;
+    return BPSX_OK;
+  }
+  template <class T> T* out(T* host, size_t count) {
+    T* p = take<T>(count);
+    outs_[n_outs_++] = {host, p, count * sizeof(T)};
+    return p;
+  }
+  // after the launches: the outputs, complete, where the caller wants them
+  int finish() {
+    if (staged_) HIP_TRY(hipStreamSynchronize(nullptr));
+    for (int i = 0; i < n_outs_; ++i) {
+      if (staged_) memcpy(outs_[i].host, outs_[i].from, outs_[i].bytes);
+      else HIP_TRY(hipMemcpy(outs_[i].host, outs_[i].from, outs_[i].bytes, hipMemcpyDeviceToHost));
+    }
+    return BPSX_OK;
+  }
+
+ private:
+  static constexpr size_t kStageMost = 16u << 20, kAlign = 256;
+  static constexpr int kArrays = 6;
+  template <class T> T* take(size_t count) {
+    T* p = (T*)at_;
+    at_ += (count * sizeof(T) + kAlign - 1) / kAlign * kAlign;
+    return p;
+  }
+  bpsx_sim* sim_ = nullptr;
+  bool staged_ = false;
+  char* at_ = nullptr;
+  struct Out { void* host; const void* from; size_t bytes; } outs_[2];
+  int n_outs_ = 0;
+};
+}  // extern "C++"
 // Node pools for a batch of n path queries: one per query while k_geodesic_few serves it, else for as
 // many blocks of k_geodesic_mid or k_geodesic as the device holds at once, or one per query where that is less.  The
 // steps' own pools serve if they are enough (a simulator has no more of them than envs in a group);
@@ -1066,18 +1136,15 @@ int bpsx_snap_points(bpsx_sim* sim, uint32_t scene, const float* pts, uint32_t n
   if (rc) return rc;
   if (!n) return BPSX_OK;
   if (!pts || !out_xyz || !out_ref) return fail(BPSX_E_INVAL, "snap_points: null argument");
-  const size_t f3 = (size_t)n * 12;
-  if ((rc = batch_reserve(sim, 2 * f3 + (size_t)n * 4))) return rc;
-  char* b = (char*)sim->d_batch;
-  float* d_in = (float*)b; float* d_xyz = (float*)(b + f3); uint32_t* d_ref = (uint32_t*)(b + 2 * f3);
-  HIP_TRY(hipMemcpy(d_in, pts, f3, hipMemcpyHostToDevice));
+  const size_t n3 = (size_t)n * 3;
+  BatchArrays io;
+  const float* d_in;
+  if ((rc = io.reserve(sim, (2 * n3 + n) * 4)) || (rc = io.in(pts, n3, &d_in))) return rc;
   // a wavefront per point for as many as the device holds at once (16 per CU); of more points each
   // wavefront takes several
-  launch_snap_batch(sim->nav, scene_entry(sim, scene), d_in, n, d_xyz, d_ref, sim->compute_units * 16u, nullptr);
+  launch_snap_batch(sim->nav, scene_entry(sim, scene), d_in, n, io.out(out_xyz, n3), io.out(out_ref, n), sim->compute_units * 16u, nullptr);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpy(out_xyz, d_xyz, f3, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(out_ref, d_ref, (size_t)n * 4, hipMemcpyDeviceToHost));
-  return BPSX_OK;
+  return io.finish();
 }
 
 int bpsx_try_steps(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const uint32_t* start_ref, const float* end_xyz,
@@ -1086,19 +1153,16 @@ int bpsx_try_steps(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const 
   if (rc) return rc;
   if (!n) return BPSX_OK;
   if (!start_xyz || !start_ref || !end_xyz || !out_xyz || !out_ref) return fail(BPSX_E_INVAL, "try_steps: null argument");
-  const size_t f3 = (size_t)n * 12, u1 = (size_t)n * 4;
-  if ((rc = batch_reserve(sim, 3 * f3 + 2 * u1))) return rc;
-  char* b = (char*)sim->d_batch;
-  float* d_s = (float*)b; float* d_e = (float*)(b + f3); float* d_o = (float*)(b + 2 * f3);
-  uint32_t* d_sr = (uint32_t*)(b + 3 * f3); uint32_t* d_or = (uint32_t*)(b + 3 * f3 + u1);
-  HIP_TRY(hipMemcpy(d_s, start_xyz, f3, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(d_e, end_xyz, f3, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(d_sr, start_ref, u1, hipMemcpyHostToDevice));
-  launch_try_step_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, n, d_o, d_or, nullptr);
+  const size_t n3 = (size_t)n * 3;
+  BatchArrays io;
+  const float *d_s, *d_e;
+  const uint32_t* d_sr;
+  if ((rc = io.reserve(sim, (3 * n3 + 2 * (size_t)n) * 4)) || (rc = io.in(start_xyz, n3, &d_s)) || (rc = io.in(end_xyz, n3, &d_e)) ||
+      (rc = io.in(start_ref, n, &d_sr)))
+    return rc;
+  launch_try_step_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, n, io.out(out_xyz, n3), io.out(out_ref, n), nullptr);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpy(out_xyz, d_o, f3, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(out_ref, d_or, u1, hipMemcpyDeviceToHost));
-  return BPSX_OK;
+  return io.finish();
 }
 
 int bpsx_geodesic(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const uint32_t* start_ref, const float* end_xyz,
@@ -1107,24 +1171,19 @@ int bpsx_geodesic(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const u
   if (rc) return rc;
   if (!n) return BPSX_OK;
   if (!start_xyz || !start_ref || !end_xyz || !end_ref || !out_dist) return fail(BPSX_E_INVAL, "geodesic: null argument");
-  const size_t f3 = (size_t)n * 12, u1 = (size_t)n * 4, qb = (size_t)n * sizeof(GeoQuery);
-  if ((rc = batch_reserve(sim, 2 * f3 + 3 * u1 + qb + 64))) return rc;
-  char* b = (char*)sim->d_batch;
-  GeoQuery* d_q = (GeoQuery*)b;  // first: keeps the 4-byte members aligned trivially
-  float* d_s = (float*)(b + qb); float* d_e = (float*)(b + qb + f3);
-  uint32_t* d_sr = (uint32_t*)(b + qb + 2 * f3); uint32_t* d_er = (uint32_t*)(b + qb + 2 * f3 + u1);
-  float* d_o = (float*)(b + qb + 2 * f3 + 2 * u1);
+  const size_t n3 = (size_t)n * 3;
+  BatchArrays io;
+  const float *d_s, *d_e;
+  const uint32_t *d_sr, *d_er;
+  void* d_q;
   GeoPool geo{};
-  if ((rc = batch_reserve_slots(sim, n, &geo))) return rc;
-  HIP_TRY(hipMemcpy(d_s, start_xyz, f3, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(d_e, end_xyz, f3, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(d_sr, start_ref, u1, hipMemcpyHostToDevice));
-  HIP_TRY(hipMemcpy(d_er, end_ref, u1, hipMemcpyHostToDevice));
-  sim->searches = launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, d_q, sim->d_batch_counts, d_o, geo,
-                                        sim->d_counters, nullptr);
+  if ((rc = io.reserve(sim, (2 * n3 + 3 * (size_t)n) * 4, (size_t)n * sizeof(GeoQuery), &d_q)) || (rc = batch_reserve_slots(sim, n, &geo)) ||
+      (rc = io.in(start_xyz, n3, &d_s)) || (rc = io.in(end_xyz, n3, &d_e)) || (rc = io.in(start_ref, n, &d_sr)) || (rc = io.in(end_ref, n, &d_er)))
+    return rc;
+  sim->searches = launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, (GeoQuery*)d_q, sim->d_batch_counts,
+                                        io.out(out_dist, n), geo, sim->d_counters, nullptr);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpy(out_dist, d_o, u1, hipMemcpyDeviceToHost));
-  return BPSX_OK;
+  return io.finish();
 }
 
 int bpsx_geodesic_static(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const uint32_t* start_ref,
@@ -1155,16 +1214,13 @@ int bpsx_random_points(bpsx_sim* sim, uint32_t scene, const float* u, uint32_t n
   if (rc) return rc;
   if (!n) return BPSX_OK;
   if (!u || !out_xyz || !out_ref) return fail(BPSX_E_INVAL, "random_points: null argument");
-  const size_t f3 = (size_t)n * 12;
-  if ((rc = batch_reserve(sim, 2 * f3 + (size_t)n * 4))) return rc;
-  char* b = (char*)sim->d_batch;
-  float* d_in = (float*)b; float* d_xyz = (float*)(b + f3); uint32_t* d_ref = (uint32_t*)(b + 2 * f3);
-  HIP_TRY(hipMemcpy(d_in, u, f3, hipMemcpyHostToDevice));
-  launch_random_points(sim->nav, scene_entry(sim, scene), d_in, n, d_xyz, d_ref, nullptr);
+  const size_t n3 = (size_t)n * 3;
+  BatchArrays io;
+  const float* d_in;
+  if ((rc = io.reserve(sim, (2 * n3 + n) * 4)) || (rc = io.in(u, n3, &d_in))) return rc;
+  launch_random_points(sim->nav, scene_entry(sim, scene), d_in, n, io.out(out_xyz, n3), io.out(out_ref, n), nullptr);
   HIP_TRY(hipGetLastError());
-  HIP_TRY(hipMemcpy(out_xyz, d_xyz, f3, hipMemcpyDeviceToHost));
-  HIP_TRY(hipMemcpy(out_ref, d_ref, (size_t)n * 4, hipMemcpyDeviceToHost));
-  return BPSX_OK;
+  return io.finish();
 }
 
 }  // extern "C"

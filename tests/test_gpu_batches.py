@@ -104,3 +104,30 @@ def test_batch_without_room_for_pools_of_its_own(oracle):
     assert np.array_equal(common.bits(got), common.bits(again))
     cpu.close()
     gpu.close()
+
+
+# calls whose arrays pass through pinned memory of at most 16 MiB, and calls beyond, which copy: 28 bytes a snap or sample, 44 a
+# move, 36 a distance
+@pytest.mark.parametrize("call,each", [("snap", 28), ("sample", 28), ("move", 44), ("distance", 36)])
+def test_calls_beyond_the_pinned_memory(oracle, call, each):
+    from bps_nav_amd.bps_sim import nav_only
+    few = 1000
+    blob, cpu, pts = points(oracle, few)
+    cpu.close()
+    pts = pts[:few]
+    u = np.random.default_rng(5).random((few, 3), dtype=np.float32)
+    gpu = nav_only([blob])
+    x, r = gpu.snap_points(0, pts)
+    to = x + np.float32(0.2)
+    gx, gr = gpu.snap_points(0, x + np.float32(0.4))
+    rep = lambda v, at: np.ascontiguousarray(v[at])  # noqa: E731
+    ask = {"snap": lambda at: gpu.snap_points(0, rep(pts, at)), "sample": lambda at: gpu.random_points(0, rep(u, at)),
+           "move": lambda at: gpu.try_steps(0, rep(x, at), rep(r, at), rep(to, at)),
+           "distance": lambda at: (gpu.geodesic(0, rep(x, at), rep(r, at), rep(gx, at), rep(gr, at)),)}[call]
+    want = ask(np.arange(few))
+    for n in (16 * 2 ** 20 // each - 100, 16 * 2 ** 20 // each + 1, 7):
+        print(f"case: {call} of {n}", flush=True)
+        at = np.arange(n) % few
+        for w, g in zip(want, ask(at)):
+            assert np.array_equal(common.bits(w)[at] if w.dtype == np.float32 else w[at], common.bits(g) if g.dtype == np.float32 else g)
+    gpu.close()
