@@ -157,14 +157,9 @@ __global__ void k_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint
   }
 }
 
-// Empties all of Q, and the reset list and the ticket counters of R (which may be Q again): R's
-// lists of queries may already hold what an earlier launch has put there for the coming one.
-__global__ void k_clear_queues(StepQueues Q, StepQueues R) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
-    for (int c = 0; c < kGeoClasses; ++c) Q.counts[kQGeo + c] = 0;
-    Q.counts[kQGeoHead] = 0; Q.counts[kQReset] = 0;
-    R.counts[kQGeoHead] = 0; R.counts[kQReset] = 0;
-  }
+// Empties all lists of Q.
+__global__ void k_clear_queues(StepQueues Q) {
+  if (blockIdx.x == 0 && threadIdx.x < kQCounters) Q.counts[threadIdx.x] = 0;
 }
 
 // Picks the next episode of agent gi in scene-table entry sc and writes its pose; the snaps follow in
@@ -546,7 +541,12 @@ __global__ __launch_bounds__(256) void k_step_finish(NavData nav, AgentArrays A,
   }
 }
 
-__global__ __launch_bounds__(256) void k_reset_all(NavData nav, AgentArrays A, StepQueues Q, StepParams P) {
+__global__ __launch_bounds__(256) void k_reset_all(NavData nav, AgentArrays A, StepQueues Q, StepQueues Qother, StepParams P) {
+  // both sets of queues are empty but for the list of resets
+  if (blockIdx.x == 0 && threadIdx.x < kQCounters) {
+    Q.counts[threadIdx.x] = threadIdx.x == kQReset ? P.n : 0u;
+    Qother.counts[threadIdx.x] = 0u;
+  }
   const uint32_t i = blockIdx.x * 32u + (threadIdx.x >> 3);   // a row of eight lanes per agent
   if (i >= P.n) return;
   const Row row;
@@ -555,7 +555,6 @@ __global__ __launch_bounds__(256) void k_reset_all(NavData nav, AgentArrays A, S
   if (row.el != 0) return;
   A.flags[gi] = kAgentResetOnly;
   Q.reset_list[i] = gi;
-  if (i == 0) Q.counts[kQReset] = P.n;
 }
 
 #ifdef BPSX_QUERY_TRACE
@@ -842,9 +841,11 @@ __global__ __launch_bounds__(kMoveItems * 8) void k_try_step_batch(NavData nav, 
   oxyz[(size_t)i * 3] = r.x; oxyz[(size_t)i * 3 + 1] = r.y; oxyz[(size_t)i * 3 + 2] = r.z;
   oref[i] = r.ref;
 }
-__global__ void k_make_queries(uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
-                               const uint32_t* eref, uint32_t n, GeoQuery* q) {
+// and the counts and the ticket counter of a batch of n queries, all in class cls
+__global__ __launch_bounds__(256) void k_make_queries(uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
+                               const uint32_t* eref, uint32_t n, GeoQuery* q, uint32_t* counts, uint32_t cls) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i <= (uint32_t)kGeoClasses) counts[i] = i == cls ? n : 0u;
   if (i >= n) return;
   GeoQuery o;
   for (int k = 0; k < 3; ++k) { o.a[k] = sxyz[(size_t)i * 3 + k]; o.b[k] = exyz[(size_t)i * 3 + k]; }
@@ -863,10 +864,6 @@ __global__ __launch_bounds__(256) void k_random_points(NavData nav, uint32_t sce
   if (row.el != 0) return;
   oxyz[(size_t)i * 3] = p[0]; oxyz[(size_t)i * 3 + 1] = p[1]; oxyz[(size_t)i * 3 + 2] = p[2];
   oref[i] = ok ? (s.ref_base | ip) : 0;
-}
-// counts and ticket counter of a batch of n queries, all in class cls
-__global__ void k_set_counts(uint32_t* p, uint32_t n, uint32_t cls) {
-  if (threadIdx.x <= (uint32_t)kGeoClasses) p[threadIdx.x] = threadIdx.x == cls ? n : 0u;
 }
 
 }  // namespace
@@ -962,9 +959,7 @@ SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQue
 
 SearchKernel launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
                   const GeoPool& G, uint32_t snap_blocks, hipStream_t st) {
-  hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Qother);
-  hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Qother, Qother);
-  hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 32), dim3(256), 0, st, nav, A, Q, P);
+  hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 32), dim3(256), 0, st, nav, A, Q, Qother, P);
   hipLaunchKernelGGL(k_reset_snap, dim3(std::min(snap_blocks, (P.n + 1u) / 2u)), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Q, P);
   SearchKernel searches = kSearchNone;
   if (P.task != BPSX_TASK_EXPLORATION)
@@ -972,7 +967,8 @@ SearchKernel launch_reset(const NavData& nav, const AgentArrays& A, const StepQu
                                A.last_cost, G, P.n, G.mid_batch, P.counters, NoSnaps{}, st);
   hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, nav, A, P, Q, Qother, 0u);
   // the next step finds its lists of queries empty, not with this launch's queries still in them
-  hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q, Q);
+  static_assert(kQCounters <= 64);
+  hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q);
   return searches;
 }
 void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz, uint32_t* oref,
@@ -995,9 +991,9 @@ void launch_try_step_batch(const NavData& nav, uint32_t scene, const float* sxyz
 SearchKernel launch_geodesic_batch(const NavData& nav, uint32_t scene, const float* sxyz, const uint32_t* sref, const float* exyz,
                                    const uint32_t* eref, uint32_t n, GeoQuery* qbuf, uint32_t* count_head /* [kGeoClasses + 1] */, float* out,
                                    const GeoPool& G, uint64_t* counters, hipStream_t st) {
-  hipLaunchKernelGGL(k_make_queries, grid_for(n, 256), dim3(256), 0, st, scene, sxyz, sref, exyz, eref, n, qbuf);
   // one class only, that of the shortest
-  hipLaunchKernelGGL(k_set_counts, dim3(1), dim3(128), 0, st, count_head, n, (uint32_t)kGeoClasses - 1u);
+  static_assert(kGeoClasses < 256, "the first block writes the counts");
+  hipLaunchKernelGGL(k_make_queries, grid_for(n, 256), dim3(256), 0, st, scene, sxyz, sref, exyz, eref, n, qbuf, count_head, (uint32_t)kGeoClasses - 1u);
   // stride 0 puts the class's queries at the start of the buffer
   return launch_geodesic(nav, qbuf, 0, &count_head[0], &count_head[kGeoClasses], out, nullptr, G, n,
                          G.mid_batch, counters, NoSnaps{}, st);
