@@ -1564,9 +1564,10 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   // which overlays the hash heads; the links stay readable while it is written.  The walk is a
   // chain of dependent reads, 70 of them on average: the parent indices, which HBM also holds
   // side by side, are first copied into the window's arrays (no longer needed), so that the
-  // chain runs in LDS; a node beyond what fits there is read from HBM.
-  static_assert(kTagSlots * sizeof(uint32_t) >= kMaxPath * sizeof(uint16_t), "the walk must fit the marks it reuses");
-  uint16_t* walk = reinterpret_cast<uint16_t*>(g.L->marks());
+  // chain runs in LDS; a node beyond what fits there is read from HBM.  The i-th node is noted in lane i mod 64 of a
+  // register: a step is the read and six instructions.  (Through a scalar
+  // register, with the nodes noted in LDS and copies of two parents a lane: steps of 64 agents 134 us, now 130, of 1024 over room
+  // plans 483 and 473, of 16384 over mazes 757 and 750, a reset of 2048 over mazes 417 and 407.)
   wave_sync();
 #if BPSX_WINDOW >= 2048
   const uint16_t* lparent = g.L->parents;
@@ -1575,24 +1576,46 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   // (of 256 nodes it holds them all.  The follower may still be at work on its heap: waiting for it cost a search 8 us)
   constexpr int kParentsLds = (int)(kWindow * sizeof(float4) / sizeof(uint16_t));
   uint16_t* lparent = reinterpret_cast<uint16_t*>(g.L->w_node);
-  const int inLds = g.nodeCount < kParentsLds ? g.nodeCount : kParentsLds;
+  const int inLds = kParentsLds >= kMaxNodes ? kMaxNodes : kParentsLds;
   {
-    const uint32_t* src = reinterpret_cast<const uint32_t*>(g.ws->parents);
-    uint32_t* dst = reinterpret_cast<uint32_t*>(lparent);
-    for (int i = lane; i < (inLds + 1) / 2; i += 64) dst[i] = src[i];
+    static_assert(offsetof(GeoSlot, parents) % 16 == 0 && kParentsLds % 512 == 0, "eight parents a lane");
+    const uint4* src = reinterpret_cast<const uint4*>(g.ws->parents);
+    uint4* dst = reinterpret_cast<uint4*>(lparent);
+    static_for<0, kParentsLds / 512>([&](auto K) BPSX_INLINE_LAMBDA {
+      constexpr int k = decltype(K)::value;
+      if (g.nodeCount > 512 * k) dst[64 * k + lane] = src[64 * k + lane];
+    });
   }
   wave_sync();
 #endif
+  constexpr int kWalk = kMaxPath / 64;
+  static_assert(kMaxPath % 64 == 0);
+  uint32_t walk[kWalk];
   int length = 0;
-  for (int c = lastBest + 1; c && length <= kMaxNodes;) {
-    if (lane == 0 && length < kMaxPath) walk[length] = (uint16_t)(c - 1);
-    length++;
-    c = inLds == kMaxNodes || c - 1 < inLds ? uniform_i((int)lparent[c - 1]) : uniform_i((int)g.ws->parents[c - 1]);
-  }
+  uint32_t up = (uint32_t)lastBest + 1u;   // the same in all lanes
+  static_for<0, kWalk>([&](auto K) BPSX_INLINE_LAMBDA {
+    constexpr int k = decltype(K)::value;
+    walk[k] = 1u;
+    for (int m = 0; m < 64 && lanes_where(up != 0); ++m) {
+      walk[k] = lane == m ? up : walk[k];
+      length++;
+      if (inLds == kMaxNodes || !lanes_where(up > (uint32_t)inLds)) {
+        up = lparent[up - 1u];
+      } else {
+        BPSX_KEEP_APART();
+        up = g.ws->parents[up - 1u];
+        BPSX_KEEP_APART();
+      }
+    }
+  });
   wave_sync();
-  const bool ok = length <= kMaxPath && link_id(g.link<true>(lastBest)) == endIp && !st.outOfNodes;
+  const bool ok = !lanes_where(up != 0) && link_id(g.link<true>(lastBest)) == endIp && !st.outOfNodes;
   if (!ok) return 0;
-  for (int i = lane; i < length; i += 64) F->corridor[length - 1 - i] = (uint16_t)link_id(g.link<true>((int)walk[i]));
+  static_for<0, kWalk>([&](auto K) BPSX_INLINE_LAMBDA {
+    constexpr int k = decltype(K)::value;
+    const int i = 64 * k + lane;
+    if (i < length) F->corridor[length - 1 - i] = (uint16_t)link_id(g.link<true>((int)walk[k] - 1));
+  });
   wave_sync();
   return length;
 }
