@@ -210,10 +210,13 @@ constexpr uint32_t kEmptyKey = 0x7fefffffu;   // above +inf, and below the total
 struct OpenList {
   static constexpr int kEnd = 63;       // the lane behind the last entry
   static constexpr int kMost = 62;      // entries in registers at most: there is always a zero below them
-  static constexpr int kSplit = 48, kRefill = 9;   // a pass looks at nine entries
-  static constexpr int kFarMost = 244;  // entries apart before a pass at most ...
-  static constexpr int kFarKeep = 236;  // ... and, once those of updated nodes are gone, for the search to go on in this form
-  static constexpr int kFarCap = 315;
+  static constexpr int kSplit = 54, kRefill = 9;   // a pass looks at nine entries
+  // As much as the reference's heap has LDS for where a second wavefront keeps it.  (With 48 and 244, and 40 entries brought back at
+  // most instead of 46, one search over cluttered plans in a few thousand outgrew the list, and a step of 4096 agents, as long as its
+  // longest search, took 1154 us instead of 1060; 1024 agents over room plans 474 and 467, 65536 over mixed scenes 2518 and 2480.)
+  static constexpr int kFarMost = 268;  // entries apart before a pass at most ...
+  static constexpr int kFarKeep = 260;  // ... and, once those of updated nodes are gone, for the search to go on in this form
+  static constexpr int kFarCap = 378;
   static_assert(kFarMost + kMost <= kFarCap, "a pass adds up to 48, and what a split adds was in registers");
   static constexpr int kMostOfAll = kSplit + kFarMost + 48;   // entries, behind a pass
   static constexpr uint32_t kEmpty = kEmptyKey;
@@ -436,7 +439,7 @@ struct GeoLds {
   uint16_t parents[kMaxNodes];
   uint16_t arrived, unused;
 #endif
-  uint2 ref_heap[354];
+  uint2 ref_heap[380];
   uint2 start;
   uint32_t published, applied, heap_size;
 #if BPSX_WINDOW < 2048
@@ -631,10 +634,10 @@ struct GeoWave {
 // a cluttered plan of 20k polygons ties with a longer list or outgrows the sorted list, and ran
 // again from its start with a heap walked level by level in HBM: 6.6 ms, against 1.5 ms for the
 // longest of the others.)
-constexpr int kHeapLds = kFollower ? 353 : (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
+constexpr int kHeapLds = kFollower ? 379 : (kTagSlots * 4 + kWindow * 16) / (int)sizeof(uint2) - 1;
 static_assert(kLinksLds % 4 == 0 && offsetof(GeoLds, w_node) == offsetof(GeoLds, n_link) + 4 * (kLinksLds + kTagSlots),
               "the marks are accessed as 16 bytes, and the heap lies over the marks and the window");
-// (383 entries, 353 where a second wavefront keeps it)
+// (383 entries, 379 where a second wavefront keeps it)
 static_assert(2 * kRows * kNvp <= 2 * 48 && kHeapLds >= OpenList::kMostOfAll + kRows, "a heap with as many entries as the sorted list must fit");
 template <bool Lds> struct RefHeap {
   uint2* h;    // total bits, packed node
@@ -1022,7 +1025,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
 // to fifty passes.
 BPSX_DEV bool refill(const GeoWave& g, OpenList& ol, uint32_t endIp, const float* endPos) {
   // 63 entries at a time: none in lane 63 (enter)
-  constexpr int kAtOnce = 63, K = OpenList::kFarCap / kAtOnce, kPull = 40, kPullLeast = 16;
+  constexpr int kAtOnce = 63, K = OpenList::kFarCap / kAtOnce, kPull = 46, kPullLeast = 30;
   static_assert(OpenList::kFarCap % kAtOnce == 0, "whole rounds");
   const int lane = lane_here(g.lane);
   uint2* apart = reinterpret_cast<uint2*>(g.far_list());
@@ -1102,7 +1105,7 @@ BPSX_DEV bool care_for_list(const GeoWave& g, OpenList& ol, uint32_t endIp, cons
   if (!full && (ol.far > OpenList::kFarMost || ol.size() < OpenList::kRefill) && !refill(g, ol, endIp, endPos)) return false;
   if (full || ol.size() > OpenList::kSplit) {
     // the greater ones, from the first of their total on
-    const int keep = ol.size() > OpenList::kSplit ? 32 : ol.size() >> 1;
+    const int keep = ol.size() > OpenList::kSplit ? 42 : ol.size() >> 1;
     const uint32_t bound = rlane(ol.total(), ol.base + keep);
     if (bound == rlane(ol.total(), ol.base)) return false;
     const unsigned long long away = lanes_where(ol.total() >= bound) & ~(1ull << OpenList::kEnd);
