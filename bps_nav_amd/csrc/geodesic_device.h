@@ -104,6 +104,13 @@ BPSX_DEV int first_lane(unsigned long long mask) {
   asm("s_ff1_i32_b64 %0, %1" : "=s"(r) : "s"(mask));
   return r;
 }
+// `Bits` bits of v from bit From on, as an instruction that the compiler cannot join to the scaling of an index: an LDS
+// address is then two instructions instead of three
+template <int From, int Bits> BPSX_DEV uint32_t field(uint32_t v) {
+  uint32_t r;
+  asm("v_bfe_u32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "n"(From), "n"(Bits));
+  return r;
+}
 // Stores in the lanes of a mask, called by whole wavefronts (all lanes active before and after).  A store under
 // a condition would get a branch around it, which costs a wavefront more than the store, and a loop
 // with such a branch in it is rebuilt by the compiler as if all its branches were the lanes' own: every
@@ -127,8 +134,9 @@ BPSX_DEV void lds_store_where(unsigned long long mask, uint32_t address, uint32_
 BPSX_DEV void lds_store_where(unsigned long long mask, uint16_t* p, uint32_t x) {
   asm volatile("s_mov_b64 exec, %0\n\tds_write_b16 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x) : "memory");
 }
-BPSX_DEV void lds_min_where(unsigned long long mask, uint32_t* p, uint32_t x) {
-  asm volatile("s_mov_b64 exec, %0\n\tds_min_u32 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x) : "memory");
+// (Offset: bytes behind p)
+template <int Offset> BPSX_DEV void lds_min_where(unsigned long long mask, const uint32_t* p, uint32_t x) {
+  asm volatile("s_mov_b64 exec, %0\n\tds_min_u32 %1, %2 offset:%3\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x), "n"(Offset) : "memory");
 }
 // base[offset bytes] = v, base the same for all lanes
 BPSX_DEV void store_where(unsigned long long mask, void* base, uint32_t offset, uint32_t v) {
@@ -568,11 +576,19 @@ struct GeoWave {
   }
 #endif
   // the multiply as the full-rate 24-bit instruction (polygon indices have 15 bits)
-  static BPSX_DEV uint32_t hash(uint32_t ip) {
+  static BPSX_DEV uint32_t hash_product(uint32_t ip) {
     uint32_t m;
     asm("v_mul_u32_u24 %0, %1, %2" : "=v"(m) : "v"(ip), "s"(0x9e3779u));
-    return (m >> 9) & (kHashSize - 1);
+    return m;
   }
+  // the bucket, of `size` ones
+  template <int size> static BPSX_DEV uint32_t bucket_of(uint32_t product) {
+    static_assert((size & (size - 1)) == 0);
+    return field<9, __builtin_ctz(size)>(product);
+  }
+  static BPSX_DEV uint32_t hash(uint32_t ip) { return bucket_of<kHashSize>(hash_product(ip)); }
+  // where in the window node i4 lies (any place for one that has left it)
+  static BPSX_DEV uint32_t window_slot(uint32_t i4) { return kAllLds ? (i4 >> 2) & (kWindow - 1) : field<2, __builtin_ctz(kWindow)>(i4); }
   BPSX_DEV void clear_marks() {
     static_assert(kTagSlots == 256, "one 16-byte store per lane");
     reinterpret_cast<uint4*>(L->marks())[lane] = make_uint4(kEndWord, kEndWord, kEndWord, kEndWord);
@@ -1205,7 +1221,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     uint32_t head = *late.chain;
     if (kAllLds) lds_store_where(late.updated, lds_address(L->w_node) + (late.node4 << 2), late.node);
     else lds_store_where(late.updated & lanes_where((int)late.node4 >= 4 * (g.nodeCount - kWindow)),
-                         lds_address(L->w_node) + ((late.node4 << 2) & (16u * (kWindow - 1))), late.node);
+                         lds_address(L->w_node) + 16u * GeoWave::window_slot(late.node4), late.node);
     // new nodes that another of their bucket has overwritten at the chain's head go in behind it
     for (unsigned long long lost = late.fresh & lanes_where(head != own); __builtin_expect(lost != 0, 0);) {
       g.set_links<S>(lost, late.node4, make_link(link_id(late.link), head));
@@ -1272,14 +1288,14 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     // ---- node lookup; the row's own lane hashes its own polygon for the conflict test
     const uint32_t nb = edge.nb;
     const unsigned long long valid = lanes_where(nb != kNoNb) & rowOn;
-    const uint32_t bucket = GeoWave::hash(in_mask(kOwnLanes) ? ip : nb);
+    const uint32_t hashed = GeoWave::hash_product(in_mask(kOwnLanes) ? ip : nb), bucket = GeoWave::bucket_of<kHashSize>(hashed);
     uint32_t chainHead;
     const uint32_t at = g.find<S>(valid, nb, bucket, &chainHead);
     FM(3);
     // ---- costs.  A lane without a node to read (idle, or its node is new) reads one of the window's slots.
     const unsigned long long known = lanes_where(at != kChainEnd);
     uint32_t ni4 = GeoWave::node4_at<S>(at);
-    float4 p = L->w_node[(ni4 >> 2) & (kWindow - 1)];
+    float4 p = L->w_node[GeoWave::window_slot(ni4)];
     if (!kAllLds) {
       const unsigned long long left = lanes_where((int)ni4 < 4 * (g.nodeCount - kWindow)) & known;
       if (__builtin_expect(left != 0, 0)) {   // a node has left the window: rare
@@ -1308,10 +1324,11 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     // ---- how many rows stand
     // conflicts: the first lane that updates a polygon leaves its mark at the polygon's hash, lanes of later rows
     // look for it (no marks stand when a pass begins)
-    uint32_t* mark = &L->marks()[bucket & (uint32_t)(kTagSlots - 1)];
-    lds_min_where(upd, mark, (uint32_t)lane);
+    const uint32_t* mark = reinterpret_cast<const uint32_t*>(L) + GeoWave::bucket_of<kTagSlots>(hashed);
+    constexpr int marksAt = (int)offsetof(GeoLds, n_link) + 4 * kLinksLds;
+    lds_min_where<marksAt>(upd, mark, (uint32_t)lane);
     wave_sync();
-    const uint32_t seen = *mark;   // the marking lane, or above all lanes
+    const uint32_t seen = mark[marksAt / 4];   // the marking lane, or above all lanes
     // the first entry that an update of a row before it reaches or undercuts: the smallest updated total of
     // every row, then of all rows up to it (a scan over the rows), and each row compares that with the
     // total of the entry behind its own
@@ -1454,6 +1471,9 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
   // All ways out of a pass meet here, and the loop has one end: with several the compiler keeps a flag for each,
   // and copies of the loop's state.  (The empty statement keeps it from joining a way out to what follows it.)
   int way;
+  // Else the compiler has every pass wait for loads that came before the loop.  (Not where a search has a SIMD nearly to itself, where
+  // the wait is none and the other order of instructions costs 0.7 %.)
+  if constexpr (!kFollower) __builtin_amdgcn_s_waitcnt(0x0f70);   // vmcnt(0)
   do {
     way = (int)pass();
     asm volatile("" : "+s"(way));
