@@ -235,7 +235,7 @@ struct bpsx_sim {
   // scratch for the batched query entry points
   void* d_batch = nullptr;
   char* h_stage = nullptr;   // pinned: the host arrays of batched calls pass through it (BatchArrays)
-  size_t stage_bytes = 0;
+  size_t stage_bytes = 0, stage_missed = 0;   // its size; bytes of the calls that were too large for it and have copied
   size_t batch_bytes = 0;
   GeoSlot* d_batch_slots = nullptr;   // node pools of a batch of path queries that needs more wavefronts than the steps have
   uint32_t batch_slots = 0;
@@ -893,7 +893,12 @@ static int batch_reserve(bpsx_sim* sim, size_t bytes) {
 }
 // The host arrays of a batched call.  Up to kStageMost bytes of them pass through pinned memory that the simulator keeps, and
 // that the kernels read and write where it lies: copies between pageable memory and the device take 10 us each however
-// small, and 33 us for 600 KB, where a copy within host memory takes 7.  Larger calls, and calls that find no pinned memory, copy.
+// small, and 33 us for 600 KB, where a copy within host memory takes 7.  (1000 pairs, two snaps and a distance each: 959 -> 843
+// us; 50000 samples, moves and snaps: 544 -> 420.)  Larger calls, and calls that find no pinned memory, copy.
+// A new page of pinned memory costs the host 1.5 us when it is first written or read, 0.4 ms a megabyte, and an allocation 0.1 to
+// 0.4 ms.  So calls of more than kStageAtOnce copy, until they have copied kStagePays times as much as the largest: about what
+// the memory then costs is what copying has cost so far.  (With it at once, the first 50000 samples, moves and snaps of a
+// simulator took 2.7 ms instead of 0.7.)
 extern "C++" {
 class BatchArrays {
  public:
@@ -903,16 +908,20 @@ class BatchArrays {
     bytes += kArrays * kAlign;
     staged_ = bytes <= kStageMost;
     if (staged_ && bytes > sim->stage_bytes) {
-      if (sim->h_stage) HIP_TRY(hipHostFree(sim->h_stage));
-      sim->h_stage = nullptr;
-      sim->stage_bytes = 0;
-      const size_t want = std::min(kStageMost, bytes + bytes / 2);   // calls that grow slowly do not allocate each time
-      if (hipHostMalloc((void**)&sim->h_stage, want, hipHostMallocDefault) == hipSuccess) {
-        sim->stage_bytes = want;
-      } else {
-        (void)hipGetLastError();   // answered here: not an error of the launches to come
+      sim->stage_missed += bytes;
+      staged_ = bytes <= kStageAtOnce || sim->stage_missed > kStagePays * bytes;
+      if (staged_) {
+        if (sim->h_stage) HIP_TRY(hipHostFree(sim->h_stage));
         sim->h_stage = nullptr;
-        staged_ = false;
+        sim->stage_bytes = sim->stage_missed = 0;
+        const size_t want = std::min(kStageMost, std::max(kStageAtOnce, bytes + bytes / 2));   // calls that grow slowly do not allocate each time
+        if (hipHostMalloc((void**)&sim->h_stage, want, hipHostMallocDefault) == hipSuccess) {
+          sim->stage_bytes = want;
+        } else {
+          (void)hipGetLastError();   // answered here: not an error of the launches to come
+          sim->h_stage = nullptr;
+          staged_ = false;
+        }
       }
     }
     const int rc = batch_reserve(sim, scratch + (staged_ ? 0 : bytes));
@@ -944,7 +953,7 @@ class BatchArrays {
   }
 
  private:
-  static constexpr size_t kStageMost = 16u << 20, kAlign = 256;
+  static constexpr size_t kStageMost = 16u << 20, kStageAtOnce = 256u << 10, kStagePays = 8, kAlign = 256;
   static constexpr int kArrays = 6;
   template <class T> T* take(size_t count) {
     T* p = (T*)at_;

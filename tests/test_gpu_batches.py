@@ -106,8 +106,8 @@ def test_batch_without_room_for_pools_of_its_own(oracle):
     gpu.close()
 
 
-# calls whose arrays pass through pinned memory of at most 16 MiB, and calls beyond, which copy: 28 bytes a snap or sample, 44 a
-# move, 36 a distance
+# calls whose arrays pass through pinned memory of at most 16 MiB, and calls beyond, which copy, as do the first few of more than
+# 256 KiB: 28 bytes a snap or sample, 44 a move, 36 a distance
 @pytest.mark.parametrize("call,each", [("snap", 28), ("sample", 28), ("move", 44), ("distance", 36)])
 def test_calls_beyond_the_pinned_memory(oracle, call, each):
     from bps_nav_amd.bps_sim import nav_only
@@ -125,7 +125,8 @@ def test_calls_beyond_the_pinned_memory(oracle, call, each):
            "move": lambda at: gpu.try_steps(0, rep(x, at), rep(r, at), rep(to, at)),
            "distance": lambda at: (gpu.geodesic(0, rep(x, at), rep(r, at), rep(gx, at), rep(gr, at)),)}[call]
     want = ask(np.arange(few))
-    for n in (16 * 2 ** 20 // each - 100, 16 * 2 ** 20 // each + 1, 7):
+    some = 256 * 2 ** 10 // each
+    for n in (some - 60, some, *[some + 1000] * 12, 4 * some, 16 * 2 ** 20 // each - 100, 16 * 2 ** 20 // each + 1, 7):
         print(f"case: {call} of {n}", flush=True)
         at = np.arange(n) % few
         for w, g in zip(want, ask(at)):
