@@ -9,7 +9,7 @@
 //     pass expand up to kRows nodes at once (astar_fast); when totals tie, the reference's binary
 //     heap is rebuilt from a log of the list's operations (RefHeap, replay_log) or has been kept from it all
 //     along by a second wavefront (follow), and a search whose
-//     list outgrows the registers, or has a tie of more than 64, goes on with that heap,
+//     list outgrows what this form holds, or has more equal totals in front than registers, goes on with that heap,
 //   - the hash heads of the node pool,
 //   - for the first kLinksLds nodes one word with the polygon id and the hash chain link,
 //   - the position and cost of the kWindow most recently created nodes (slot = index
@@ -205,7 +205,7 @@ constexpr uint32_t kEmptyKey = 0x7fefffffu;   // above +inf, and below the total
 // in the last but one; zeros below (node kNone), which are smaller than every entry, and a total above all in the last lane.  The
 // list grows downwards: an entry that enters moves those below it down a lane, and what a pass
 // expands leaves by a move of the base.
-// Entries with totals from `bound` on are kept apart, in no order, in the wavefront's slot (GeoSlot::far): they cost one store
+// Entries with totals from `bound` on are kept apart, in no order, in the wavefront's slot (GeoWave::far_list): they cost one store
 // now, and a search comes back to half of them at most.  Where fewer than kRefill are left in registers, those up to a new
 // bound come from there (refill); where more than kSplit are, the greater ones go there (split).  An entry whose node is
 // updated meanwhile stays there, and is known by its total when it is looked at.
@@ -654,7 +654,7 @@ constexpr int kHeapLds = kFollower ? 379 : (kTagSlots * 4 + kWindow * 16) / (int
 static_assert(kLinksLds % 4 == 0 && offsetof(GeoLds, w_node) == offsetof(GeoLds, n_link) + 4 * (kLinksLds + kTagSlots),
               "the marks are accessed as 16 bytes, and the heap lies over the marks and the window");
 // (383 entries, 379 where a second wavefront keeps it)
-static_assert(2 * kRows * kNvp <= 2 * 48 && kHeapLds >= OpenList::kMostOfAll + kRows, "a heap with as many entries as the sorted list must fit");
+static_assert(kRows * kNvp <= 48 && kHeapLds >= OpenList::kMostOfAll + kRows, "a heap with as many entries as the sorted list must fit");
 template <bool Lds> struct RefHeap {
   uint2* h;    // total bits, packed node
   int size, lane;
@@ -966,7 +966,7 @@ BPSX_DEV void restore_window(GeoWave& g) {
 }
 
 // One node per round with the reference's heap as it is: what a search goes on with when its open
-// list outgrows the sorted form's registers or its log is full.  The nodes' bodies are read from
+// list outgrows the sorted form or its log is full.  The nodes' bodies are read from
 // the slot (the heap lies over the window).  Lds: the heap is in LDS, and the loop ends with
 // kAstarGrowHeap before it outgrows it; otherwise it is in the slot, which holds any heap.
 template <bool Lds>

@@ -942,8 +942,8 @@ SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQue
   mark();
   // Three agents in five ask for a distance in a step; a group's queries are taken for three in four, with
   // room for one that asks more, so k_geodesic_few serves groups of up to 1024 agents.  (The line could lie
-  // higher: a step over room plans, cluttered plans, mazes takes 574, 944, 470 us by k_geodesic_few and 620, 975, 479 by
-  // k_geodesic_mid at 1024 agents, 591, 962, 501 and 647, 1002, 528 at 1600.)
+  // higher: a step over room plans, cluttered plans, mazes takes 450, 718, 414 us by k_geodesic_few and 493, 775, 433 by
+  // k_geodesic_mid at 1200 agents, 472, 747, 482 and 516, 788, 507 at 2048, 479, 839, 499 and 518, 835, 471 at 3072.)
   SearchKernel searches = kSearchNone;
   if (P.task != BPSX_TASK_EXPLORATION)   // which asks for no distance
     searches = launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
