@@ -1362,9 +1362,10 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
       const float q2 = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(p2)));
       const float theirCost = __int_as_float(__builtin_amdgcn_ds_bpermute(from, __float_as_int(cost)));
       // its way costs no less if its step is as long as the costs' difference, with room for the rounding of both
-      // (cost = b.w + the step's length never falls when the length grows)
-      const float mx = q0 - b.x, my = q1 - b.y, mz = q2 - b.z, less = theirCost - b.w;
-      const unsigned long long far = lanes_where(mx * mx + my * my + mz * mz >= less * less * 1.00001f) | lanes_where(less <= 0.0f);
+      // (cost = b.w + the step's length never falls when the length grows).  The square of a difference below 2^-63 has fewer
+      // bits than that room needs, or none, and where there is no difference any step is long enough: there one of 2^-63 has to be.
+      const float mx = q0 - b.x, my = q1 - b.y, mz = q2 - b.z, less = fmaxf(theirCost - b.w, 0x1p-63f);
+      const unsigned long long far = lanes_where(mx * mx + my * my + mz * mz >= less * less * 1.00001f);
       const unsigned long long falls = pairTie ? 0ull : far & lanes_where(theirs == nb) & clash & upd;
       upd &= ~falls;
       clash &= ~falls;

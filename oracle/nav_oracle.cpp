@@ -928,8 +928,8 @@ float Query::geodesic(const NavPoint& start, const NavPoint& end) {
         const Node& b = q.nodes[order[j]];
         float d[3];
         for (int k = 0; k < 3; ++k) d[k] = earlier.pos[k] - b.pos[k];
-        const float less = earlier.cost - b.cost;
-        return (d[0] * d[0] + d[1] * d[1] + d[2] * d[2] >= less * less * 1.00001f) || less <= 0.0f;
+        const float less = fmaxf(earlier.cost - b.cost, 0x1p-63f);
+        return d[0] * d[0] + d[1] * d[1] + d[2] * d[2] >= less * less * 1.00001f;
       };
       std::vector<PlanUpd> raw[8];
       for (int j = 0; j < lim; ++j) raw[j] = plan.upd[j];

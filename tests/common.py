@@ -38,3 +38,29 @@ def action_stream(config, steps, n):
 def bits(a):
     a = np.ascontiguousarray(a)
     return a.view(np.uint32) if a.dtype == np.float32 else a
+
+
+def crossing_portals(seed, n, unit):
+    """Navmesh of n polygons, each joined to three others at random, whose portals' middles all have x = z = 0 and heights of up
+    to 1000 units: the distances of a search within it are of any size that floats have.  And the middle's neighbourhood
+    in it: f(count) -> points and polygons."""
+    rng = np.random.default_rng(seed)
+    while True:
+        ends = rng.permutation(np.repeat(np.arange(n), 3)).reshape(-1, 2)
+        if (ends[:, 0] != ends[:, 1]).all() and len(np.unique(np.sort(ends, 1), axis=0)) == len(ends):
+            break
+    verts, joined = [], [[] for _ in range(n)]
+    for k, (p, q) in enumerate(ends.tolist()):
+        x, z = (int(v) for v in rng.integers(1, 60, 2) * rng.choice([-1, 1], 2))
+        verts += [(64 + x, int(rng.integers(0, 1000)), 64 + z), (64 - x, int(rng.integers(0, 1000)), 64 - z)]
+        joined[p].append((q, 2 * k, 2 * k + 1))
+        joined[q].append((p, 2 * k + 1, 2 * k))
+    polys = [[v for _, a, b in j for v in (a, b)] for j in joined]
+    neis = [[v for q, _, _ in j for v in (q, -1)] for j in joined]
+    blob = scenes.navmesh_from_polys(verts, polys, neis, bmin=(-4.0, 0.0, -4.0), cs=0.0625, ch=unit)
+
+    def near(refs, count):
+        at = rng.integers(-1000, 1001, (count, 3))
+        at[:, 1] = np.abs(at[:, 1])
+        return (at * np.float64(unit)).astype(np.float32), refs[rng.integers(0, n, count)]
+    return blob, near

@@ -83,3 +83,22 @@ def test_updates_that_fall_away(oracle, config, queries):
     assert st["wrong_node"] == 0 and st["wrong_update"] == 0, st
     assert st["fallen"] > 0.1 * st["passes"], st
     assert all_fall["wrong_update"] > 0, all_fall
+
+
+@pytest.mark.parametrize("unit", [1e16, 1e-3, 1e-18, 1e-21, 1e-22, 1e-23, 3e-24, 1e-24, 1e-25])
+def test_updates_that_fall_away_at_all_distances(oracle, unit):
+    """Squares of distances below 2^-63 have fewer than 24 bits, or none: there they do not tell the longer way."""
+    st = dict.fromkeys(("passes", "fallen", "wrong_node", "wrong_update"), 0)
+    for seed in range(4):
+        blob, near = common.crossing_portals(seed, 100, unit)
+        nav = bpo.Nav(oracle, blob)
+        refs = nav.poly_info()[0]
+        nav.pass_check(8)
+        nav.geodesic(*near(refs, 300), *near(refs, 300))
+        for k, v in nav.pass_check(0).items():
+            st[k] = st.get(k, 0) + v
+        nav.close()
+    assert st["wrong_node"] == 0 and st["wrong_update"] == 0, st
+    assert st["passes"] > 1000, st
+    if unit >= 1e-18:
+        assert st["fallen"] > 0.02 * st["passes"], st
