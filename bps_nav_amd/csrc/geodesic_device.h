@@ -894,7 +894,7 @@ BPSX_DEV void follow(GeoLds* L, const GeoSlot* ws, int lane) {
     wave_sync();
     const int arrived = uniform_i((int)__hip_atomic_load(&L->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
     const int end = arrived > asked ? arrived : asked;
-    if (asked) __builtin_amdgcn_s_setprio(3);   // the search waits
+    if (word != done) __builtin_amdgcn_s_setprio(3);   // the search waits (done is the word of one that has not asked)
     if (pos < end) {
       const unsigned long long r = __hip_atomic_load(log + (pos + lane < end ? pos + lane : pos), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const uint32_t rk = (uint32_t)r, rw = (uint32_t)(r >> 32);
