@@ -22,6 +22,7 @@
 #include "errors.h"
 #include "kernels.h"
 #include "navmesh_host.h"
+#include "stage_rule.h"
 
 using namespace bpsx;
 
@@ -235,7 +236,7 @@ struct bpsx_sim {
   // scratch for the batched query entry points
   void* d_batch = nullptr;
   char* h_stage = nullptr;   // pinned: the host arrays of batched calls pass through it (BatchArrays)
-  size_t stage_bytes = 0, stage_missed = 0;   // its size; bytes of the calls that were too large for it and have copied
+  StageRule stage;           // its size
   size_t batch_bytes = 0;
   GeoSlot* d_batch_slots = nullptr;   // node pools of a batch of path queries that needs more wavefronts than the steps have
   uint32_t batch_slots = 0;
@@ -891,39 +892,30 @@ static int batch_reserve(bpsx_sim* sim, size_t bytes) {
   sim->batch_bytes = bytes;
   return BPSX_OK;
 }
-// The host arrays of a batched call.  Up to kStageMost bytes of them pass through pinned memory that the simulator keeps, and
+// The host arrays of a batched call.  Up to 16 MiB of them pass through pinned memory that the simulator keeps, and
 // that the kernels read and write where it lies: copies between pageable memory and the device take 10 us each however
 // small, and 33 us for 600 KB, where a copy within host memory takes 7.  (1000 pairs, two snaps and a distance each: 959 -> 843
 // us; 50000 samples, moves and snaps: 544 -> 420.)  Larger calls, and calls that find no pinned memory, copy.
-// A new page of pinned memory costs the host 1.5 us when it is first written or read, 0.4 ms a megabyte, and an allocation 0.1 to
-// 0.4 ms.  So calls of more than kStageAtOnce copy, until they have copied kStagePays times as much as the largest: about what
-// the memory then costs is what copying has cost so far.  (With it at once, the first 50000 samples, moves and snaps of a
-// simulator took 2.7 ms instead of 0.7.)
+// What is kept, and from when on: StageRule.
 extern "C++" {
 class BatchArrays {
  public:
   // bytes: of all arrays; scratch: device memory besides, returned in *d_scratch
   int reserve(bpsx_sim* sim, size_t bytes, size_t scratch = 0, void** d_scratch = nullptr) {
-    sim_ = sim;
     bytes += kArrays * kAlign;
-    staged_ = bytes <= kStageMost;
-    if (staged_ && bytes > sim->stage_bytes) {
-      sim->stage_missed += bytes;
-      staged_ = bytes <= kStageAtOnce || sim->stage_missed > kStagePays * bytes;
-      if (staged_) {
-        if (sim->h_stage) HIP_TRY(hipHostFree(sim->h_stage));
-        sim->h_stage = nullptr;
-        sim->stage_bytes = sim->stage_missed = 0;
-        const size_t want = std::min(kStageMost, std::max(kStageAtOnce, bytes + bytes / 2));   // calls that grow slowly do not allocate each time
-        if (hipHostMalloc((void**)&sim->h_stage, want, hipHostMallocDefault) == hipSuccess) {
-          sim->stage_bytes = want;
-        } else {
-          (void)hipGetLastError();   // answered here: not an error of the launches to come
-          sim->h_stage = nullptr;
-          staged_ = false;
-        }
+    const size_t want = sim->stage.wanted(bytes);
+    if (want != sim->stage.held) {
+      void* p = nullptr;
+      if (hipHostMalloc(&p, want, hipHostMallocDefault) == hipSuccess) {
+        if (sim->h_stage) (void)hipHostFree(sim->h_stage);
+        sim->h_stage = (char*)p;
+        sim->stage.holds(want);
+      } else {
+        (void)hipGetLastError();   // answered here: not an error of the launches to come
+        sim->stage.refused();
       }
     }
+    staged_ = bytes <= sim->stage.held;
     const int rc = batch_reserve(sim, scratch + (staged_ ? 0 : bytes));
     if (rc) return rc;
     at_ = staged_ ? sim->h_stage : (char*)sim->d_batch + scratch;
@@ -953,14 +945,13 @@ class BatchArrays {
   }
 
  private:
-  static constexpr size_t kStageMost = 16u << 20, kStageAtOnce = 256u << 10, kStagePays = 8, kAlign = 256;
+  static constexpr size_t kAlign = 256;
   static constexpr int kArrays = 6;
   template <class T> T* take(size_t count) {
     T* p = (T*)at_;
     at_ += (count * sizeof(T) + kAlign - 1) / kAlign * kAlign;
     return p;
   }
-  bpsx_sim* sim_ = nullptr;
   bool staged_ = false;
   char* at_ = nullptr;
   struct Out { void* host; const void* from; size_t bytes; } outs_[2];
