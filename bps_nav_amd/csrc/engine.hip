@@ -934,9 +934,12 @@ class BatchArrays {
     outs_[n_outs_++] = {host, p, count * sizeof(T)};
     return p;
   }
-  // after the launches: the outputs, complete, where the caller wants them
+  // After the launches: their error, or the outputs, complete, where the caller wants them.  Either way nothing is at work on the
+  // pinned memory any more, into which the next call writes without waiting for the stream.
   int finish() {
+    const hipError_t launched = hipGetLastError();
     if (staged_) HIP_TRY(hipStreamSynchronize(nullptr));
+    HIP_TRY(launched);
     for (int i = 0; i < n_outs_; ++i) {
       if (staged_) memcpy(outs_[i].host, outs_[i].from, outs_[i].bytes);
       else HIP_TRY(hipMemcpy(outs_[i].host, outs_[i].from, outs_[i].bytes, hipMemcpyDeviceToHost));
@@ -1143,7 +1146,6 @@ int bpsx_snap_points(bpsx_sim* sim, uint32_t scene, const float* pts, uint32_t n
   // a wavefront per point for as many as the device holds at once (16 per CU); of more points each
   // wavefront takes several
   launch_snap_batch(sim->nav, scene_entry(sim, scene), d_in, n, io.out(out_xyz, n3), io.out(out_ref, n), sim->compute_units * 16u, nullptr);
-  HIP_TRY(hipGetLastError());
   return io.finish();
 }
 
@@ -1161,7 +1163,6 @@ int bpsx_try_steps(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const 
       (rc = io.in(start_ref, n, &d_sr)))
     return rc;
   launch_try_step_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, n, io.out(out_xyz, n3), io.out(out_ref, n), nullptr);
-  HIP_TRY(hipGetLastError());
   return io.finish();
 }
 
@@ -1182,7 +1183,6 @@ int bpsx_geodesic(bpsx_sim* sim, uint32_t scene, const float* start_xyz, const u
     return rc;
   sim->searches = launch_geodesic_batch(sim->nav, scene_entry(sim, scene), d_s, d_sr, d_e, d_er, n, (GeoQuery*)d_q, sim->d_batch_counts,
                                         io.out(out_dist, n), geo, sim->d_counters, nullptr);
-  HIP_TRY(hipGetLastError());
   return io.finish();
 }
 
@@ -1219,7 +1219,6 @@ int bpsx_random_points(bpsx_sim* sim, uint32_t scene, const float* u, uint32_t n
   const float* d_in;
   if ((rc = io.reserve(sim, (2 * n3 + n) * 4)) || (rc = io.in(u, n3, &d_in))) return rc;
   launch_random_points(sim->nav, scene_entry(sim, scene), d_in, n, io.out(out_xyz, n3), io.out(out_ref, n), nullptr);
-  HIP_TRY(hipGetLastError());
   return io.finish();
 }
 

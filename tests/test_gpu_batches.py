@@ -132,3 +132,25 @@ def test_calls_beyond_the_pinned_memory(oracle, call, each):
         for w, g in zip(want, ask(at)):
             assert np.array_equal(common.bits(w)[at] if w.dtype == np.float32 else w[at], common.bits(g) if g.dtype == np.float32 else g)
     gpu.close()
+
+
+def test_a_call_after_one_that_failed(oracle):
+    """A call that finds an error of an earlier one behind its launches fails, but not before these are done: the next one's
+    arrays take the place of its own in the pinned memory."""
+    from bps_nav_amd import _lib
+    from bps_nav_amd.bps_sim import nav_only
+    n = 5000
+    blob, cpu, pts = points(oracle, n)
+    pts = np.resize(pts, (n, 3))
+    few = pts[:50]
+    want = cpu.snap(few)
+    cpu.close()
+    gpu = nav_only([blob])
+    print("case: a call after one that failed", flush=True)
+    for _ in range(5):
+        assert _lib.lib().hipSetDevice(1 << 20) != 0   # (of the runtime that the library is bound to)
+        with pytest.raises(RuntimeError):
+            gpu.snap_points(0, pts)
+        x, r = gpu.snap_points(0, few)
+        assert np.array_equal(common.bits(x), common.bits(want[0])) and np.array_equal(r, want[1])
+    gpu.close()
