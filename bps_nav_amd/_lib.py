@@ -95,6 +95,8 @@ def lib():
             L.bpsx_kernel_name.restype = C.c_char_p
             L.bpsx_search_kernel.argtypes = [C.c_void_p]
             L.bpsx_search_kernel.restype = C.c_char_p
+            L.bpsx_batch_route.argtypes = [C.c_void_p]
+            L.bpsx_batch_route.restype = C.c_char_p
             L.bpsx_snap_points.argtypes = [C.c_void_p, C.c_uint32, C.c_void_p, C.c_uint32, C.c_void_p, C.c_void_p]
             L.bpsx_try_steps.argtypes = [C.c_void_p, C.c_uint32, C.c_void_p, C.c_void_p, C.c_void_p,
                                          C.c_uint32, C.c_void_p, C.c_void_p]

@@ -289,6 +289,10 @@ class PointNavRolloutGenerator:
         """The kernel that the newest step, reset or batch gave its path searches to ("" without any)."""
         return self._L.bpsx_search_kernel(self._h).decode()
 
+    def batch_route(self):
+        """How the newest batched query's host arrays reached the kernels: "pinned" or "copied" ("" before the first)."""
+        return self._L.bpsx_batch_route(self._h).decode()
+
     # ---- batched PathFinder-level queries (host arrays)
     def snap_points(self, scene, pts):
         pts = np.ascontiguousarray(pts, np.float32).reshape(-1, 3)

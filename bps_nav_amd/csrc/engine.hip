@@ -237,6 +237,7 @@ struct bpsx_sim {
   void* d_batch = nullptr;
   char* h_stage = nullptr;   // pinned: the host arrays of batched calls pass through it (BatchArrays)
   StageRule stage;           // its size
+  const char* batch_route = "";   // of the newest batched call
   size_t batch_bytes = 0;
   GeoSlot* d_batch_slots = nullptr;   // node pools of a batch of path queries that needs more wavefronts than the steps have
   uint32_t batch_slots = 0;
@@ -881,6 +882,7 @@ int bpsx_get_kernel_times(bpsx_sim* sim, double* out_ms_sum, uint64_t* out_steps
 
 const char* bpsx_kernel_name(uint32_t idx) { return idx < BPSX_NUM_KERNELS ? kKernelNames[idx] : ""; }
 const char* bpsx_search_kernel(const bpsx_sim* sim) { return kSearchKernelNames[sim ? sim->searches : kSearchNone]; }
+const char* bpsx_batch_route(const bpsx_sim* sim) { return sim ? sim->batch_route : ""; }
 
 // ---- batched PathFinder-level queries: host arrays in, host arrays out
 static int batch_reserve(bpsx_sim* sim, size_t bytes) {
@@ -916,6 +918,7 @@ class BatchArrays {
       }
     }
     staged_ = bytes <= sim->stage.held;
+    sim->batch_route = staged_ ? "pinned" : "copied";
     const int rc = batch_reserve(sim, scratch + (staged_ ? 0 : bytes));
     if (rc) return rc;
     at_ = staged_ ? sim->h_stage : (char*)sim->d_batch + scratch;

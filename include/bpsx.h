@@ -233,6 +233,9 @@ BPSX_API const char *bpsx_kernel_name(uint32_t idx);
  * of the sizes at which that changes: "k_geodesic_few", "k_geodesic_mid", "k_geodesic", or "" where
  * there were none. */
 BPSX_API const char *bpsx_search_kernel(const bpsx_sim *sim);
+/* How the host arrays of the newest batched query below reached the kernels, likewise for tests:
+ * "pinned" (through memory that the simulator keeps for them) or "copied"; "" before the first. */
+BPSX_API const char *bpsx_batch_route(const bpsx_sim *sim);
 
 /* ---- batched PathFinder queries on one uploaded scene (PathFinder.h:99-227) ----
  * All pointers are host pointers; n items; results copied back before returning. */

@@ -106,8 +106,8 @@ def test_batch_without_room_for_pools_of_its_own(oracle):
     gpu.close()
 
 
-# calls whose arrays pass through pinned memory of at most 16 MiB, and calls beyond, which copy, as do the first few of more than
-# 256 KiB: 28 bytes a snap or sample, 44 a move, 36 a distance
+# calls whose arrays pass through pinned memory of at most 16 MiB, and calls beyond, which copy, as do calls of more than 256
+# KiB until eight times as much has been copied as the largest needs: 28 bytes a snap or sample, 44 a move, 36 a distance
 @pytest.mark.parametrize("call,each", [("snap", 28), ("sample", 28), ("move", 44), ("distance", 36)])
 def test_calls_beyond_the_pinned_memory(oracle, call, each):
     from bps_nav_amd.bps_sim import nav_only
@@ -125,12 +125,17 @@ def test_calls_beyond_the_pinned_memory(oracle, call, each):
            "move": lambda at: gpu.try_steps(0, rep(x, at), rep(r, at), rep(to, at)),
            "distance": lambda at: (gpu.geodesic(0, rep(x, at), rep(r, at), rep(gx, at), rep(gr, at)),)}[call]
     want = ask(np.arange(few))
-    some = 256 * 2 ** 10 // each
-    for n in (some - 60, some, *[some + 1000] * 12, 4 * some, 16 * 2 ** 20 // each - 100, 16 * 2 ** 20 // each + 1, 7):
+    most, at_once, middle = (size // each for size in (16 * 2 ** 20, 256 * 2 ** 10, 2 ** 21))
+    assert gpu.batch_route() == "pinned"   # of the 1000
+    routes = [(at_once - 60, "pinned"), (at_once, "copied")]   # the arrays take up to 1536 bytes more than their own
+    for n in (at_once + 1000, middle, most - 100):
+        routes += [(n, "copied")] * 8 + [(n, "pinned")] * 2
+    for n, route in routes + [(most + 1, "copied"), (7, "pinned")]:
         print(f"case: {call} of {n}", flush=True)
         at = np.arange(n) % few
         for w, g in zip(want, ask(at)):
-            assert np.array_equal(common.bits(w)[at] if w.dtype == np.float32 else w[at], common.bits(g) if g.dtype == np.float32 else g)
+            assert np.array_equal(common.bits(w)[at], common.bits(g))
+        assert gpu.batch_route() == route
     gpu.close()
 
 
