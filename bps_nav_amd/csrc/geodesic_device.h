@@ -74,17 +74,8 @@ BPSX_DEV unsigned long long lanes_where(bool b) { return __builtin_amdgcn_ballot
 // instead of conditions that are widened to integers and compared again for the next mask
 BPSX_DEV bool in_mask(unsigned long long m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
 BPSX_DEV int uniform_i(int v) { return __builtin_amdgcn_readfirstlane(v); }
-BPSX_DEV float uniform_f(float v) { return __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(v))); }
 BPSX_DEV float lane_f(float v, int lane) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane)); }
-BPSX_DEV int lane_i(int v, int lane) { return __builtin_amdgcn_readlane(v, lane); }
 BPSX_DEV uint32_t rlane(uint32_t v, int lane) { return (uint32_t)__builtin_amdgcn_readlane((int)v, lane); }
-// old with lane `lane` replaced by v (v and lane uniform).  The lane select travels in M0:
-// gfx9 encodings take at most one general scalar register per vector instruction.
-BPSX_DEV uint32_t wlane(uint32_t old, uint32_t v, int lane) {
-  const int sv = __builtin_amdgcn_readfirstlane((int)v), sl = __builtin_amdgcn_readfirstlane(lane);
-  asm("s_mov_b32 m0, %2\n\tv_writelane_b32 %0, %1, m0" : "+v"(old) : "s"(sv), "s"(sl) : "m0");
-  return old;
-}
 
 // The lane, for a part of the search that is entered once in a while: what is computed from it there is not worth
 // keeping in registers all the time, which the compiler would do.
