@@ -203,7 +203,7 @@ constexpr uint32_t kEmptyKey = 0x7fefffffu;   // above +inf, and below the total
 // (With up to 256 sorted entries in four register pairs, counted into place together and moved through LDS from the second
 // pair on, and with totals and nodes selected apart and a lane permute that closed the gap of those that left: 600 to 860
 // cycles of a pass instead of 500 to 600, 1500 instead of 600 over cluttered plans, whose lists have 73 entries on average and up to
-// 260.  Steps of 64 agents 148 -> 136 us, of 1024 over room plans 589 -> 500, of 510 in two groups 1112 -> 968, of 4096 over
+// 300.  Steps of 64 agents 148 -> 136 us, of 1024 over room plans 589 -> 500, of 510 in two groups 1112 -> 968, of 4096 over
 // cluttered plans 1280 -> 1190, of 16384 over mazes 805 -> 796, of 65536 over mixed scenes 2810 -> 2676, a reset of 2048 over mazes
 // 476 -> 447, 300 queries over room plans 265 -> 242, 1000 pairs over a maze 949 -> 931.)
 struct OpenList {
@@ -630,7 +630,7 @@ struct GeoWave {
 // what comes first (a tie) or cannot hold what is open: position q (root = 1) in entry q of an array
 // in LDS, over the conflict marks (but the first two) and the window, or in the wavefront's slot.  All lanes
 // work on one operation: a push takes one round of accesses, a pop one up to 256 entries (searches
-// over mazes keep 23 on average, over cluttered plans 70), beyond that one per five levels.  Bound by
+// over mazes keep 23 on average, over cluttered plans 73), beyond that one per five levels.  Bound by
 // those rounds and the instructions of a lone wavefront, five cycles each; a replay is a chain of them.
 // (With each pop in rounds of six levels, which combined the siblings' comparisons on the scalar unit
 // and brought the deepest entry that moves back from there, with branches around the stores, a replay
@@ -885,7 +885,9 @@ BPSX_DEV void follow(GeoLds* L, const GeoSlot* ws, int lane) {
     wave_sync();
     const int arrived = uniform_i((int)__hip_atomic_load(&L->arrived, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
     const int end = arrived > asked ? arrived : asked;
-    if (word != done) __builtin_amdgcn_s_setprio(3);   // the search waits (done is the word of one that has not asked)
+    // The search waits for a word that is not done: at the highest priority until the answer, and not for the passes behind it, which
+    // would issue before other blocks' searches.
+    if (word != done) __builtin_amdgcn_s_setprio(3);
     if (pos < end) {
       const unsigned long long r = __hip_atomic_load(log + (pos + lane < end ? pos + lane : pos), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       const uint32_t rk = (uint32_t)r, rw = (uint32_t)(r >> 32);

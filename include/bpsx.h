@@ -216,7 +216,8 @@ BPSX_API int bpsx_check_errors(bpsx_sim *sim);
  * (possible when neither affects the other), [20] the times the reference's arrangement had to be
  * rebuilt from the search's operation log to tell which of the two comes first, [19] the searches
  * that went on with the reference's heap, rebuilt from the log, because the open list outgrew the
- * sorted form's 256 entries, the log was full or more than 64 open nodes shared the smallest total.
+ * sorted form (more than 260 entries besides those in registers), the log was full or more open nodes
+ * shared the smallest total than there are registers for.
  * Same results in all cases. */
 #define BPSX_NUM_COUNTERS 22
 BPSX_API int bpsx_get_counters(bpsx_sim *sim, uint64_t *out /* [BPSX_NUM_COUNTERS] */);
