@@ -12,7 +12,44 @@ __global__ __launch_bounds__(256) void k_roots(uint32_t first, uint32_t n, float
   if (i >= n) return;
   bpsx::sqrt_exact2(__uint_as_float(first + i), __uint_as_float(first + n - 1u - i), &a[i], &b[n - 1u - i]);
 }
+// the records of `slot`'s log, `n` of them, applied to the heap that it keeps, of size[0] entries and size[1] - 1 nodes so far
+__global__ __launch_bounds__(64) void k_replay(bpsx::GeoSlot* slot, int n, int* size) {
+  using namespace bpsx::geo;
+  __shared__ GeoShared lds;
+  GeoWave g;
+  g.lane = (int)threadIdx.x;
+  g.L = &lds.a;
+  g.ws = slot;
+  g.nodeCount = 0;
+  bpsx::AstarState st;
+  st.synced = 0;
+  st.logEnd = n;
+  st.replaySize = size[0];
+  st.replayNodes = size[1];
+  replay_log(g, st);
+  if (threadIdx.x == 0) { size[0] = st.replaySize; size[1] = st.replayNodes; }
+}
 }  // namespace
+
+// The reference's heap of `size` entries (total's bits, packed node; entry 1 the root, entry 0 unused, room for 384) after a log of
+// n records, `nodes` nodes having been created before it.  Host pointers; returns the entries, or -1 for what no search keeps.
+extern "C" __attribute__((visibility("default"))) int bpsx_check_replay(uint32_t* entries, int size, int nodes, const uint32_t* log, int n) {
+  constexpr size_t kEntries = 384 * sizeof(uint2);
+  if (size < 1 || size > bpsx::geo::kHeapLds || nodes < 1 || nodes > bpsx::kMaxNodes || n < 1 || n > bpsx::kOpLogCap) return -1;
+  bpsx::GeoSlot* slot = nullptr;
+  int* dsize = nullptr;
+  int sizes[2] = {size, nodes};
+  const bool ok = hipMalloc(&slot, sizeof(*slot)) == hipSuccess && hipMalloc(&dsize, sizeof(sizes)) == hipSuccess &&
+                  hipMemcpy(slot->heap_spill, entries, kEntries, hipMemcpyHostToDevice) == hipSuccess &&
+                  hipMemcpy(slot->oplog, log, (size_t)n * sizeof(bpsx::OpRec), hipMemcpyHostToDevice) == hipSuccess &&
+                  hipMemcpy(dsize, sizes, sizeof(sizes), hipMemcpyHostToDevice) == hipSuccess;
+  if (ok) hipLaunchKernelGGL(k_replay, dim3(1), dim3(64), 0, nullptr, slot, n, dsize);
+  const bool done = ok && hipGetLastError() == hipSuccess && hipMemcpy(sizes, dsize, sizeof(sizes), hipMemcpyDeviceToHost) == hipSuccess &&
+                    hipMemcpy(entries, slot->heap_spill, kEntries, hipMemcpyDeviceToHost) == hipSuccess;
+  (void)hipFree(slot);
+  (void)hipFree(dsize);
+  return done ? sizes[0] : -1;
+}
 
 // a[i] = b[i] = the root of the float with bits first + i, each by another of sqrt_exact2's arguments, i < n.
 // Device pointers to n floats; returns hipSuccess or the launch's error.
