@@ -122,9 +122,10 @@ BPSX_DEV void lds_store_where(unsigned long long mask, uint32_t address, float4 
 BPSX_DEV void lds_store_where(unsigned long long mask, uint32_t address, uint32_t x) {
   asm volatile("s_mov_b64 exec, %0\n\tds_write_b32 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(address), "v"(x) : "memory");
 }
-BPSX_DEV void lds_store_where(unsigned long long mask, uint16_t* p, uint32_t x) {
-  asm volatile("s_mov_b64 exec, %0\n\tds_write_b16 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x) : "memory");
+BPSX_DEV void lds_store_half_where(unsigned long long mask, uint32_t address, uint32_t x) {
+  asm volatile("s_mov_b64 exec, %0\n\tds_write_b16 %1, %2\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(address), "v"(x) : "memory");
 }
+BPSX_DEV uint32_t lds_half(uint32_t address) { return *(__attribute__((address_space(3))) const uint16_t*)(uintptr_t)address; }
 // (Offset: bytes behind p)
 template <int Offset> BPSX_DEV void lds_min_where(unsigned long long mask, const uint32_t* p, uint32_t x) {
   asm volatile("s_mov_b64 exec, %0\n\tds_min_u32 %1, %2 offset:%3\n\ts_mov_b64 exec, -1" :: "s"(mask), "v"(lds_address(p)), "v"(x), "n"(Offset) : "memory");
@@ -246,9 +247,9 @@ struct OpenList {
     span = (uint32_t)((far ? kEnd - kRefill : kEnd) - (kEnd - kSplit));
   }
   BPSX_DEV bool needs_care() const { return (uint32_t)(base - low) > span; }
-  // lane L takes v of lane L + 1, lane 63 keeps `last`
-  static BPSX_DEV uint32_t down1(uint32_t last, uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp((int)last, (int)v, 0x130 /* wave_shl:1 */, 0xf, 0xf, false);
+  // lane L takes v of lane L + 1, lane 63 zero
+  static BPSX_DEV uint32_t down1(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x130 /* wave_shl:1 */, 0xf, 0xf, true);
   }
   // lane L takes v of lane L - 1, lane 0 zero
   static BPSX_DEV uint32_t up1(uint32_t v) {
@@ -359,14 +360,13 @@ enum AstarExit { kAstarOn = -1, kAstarEmpty = 0, kAstarGoal = 1, kAstarGrowLinks
 BPSX_DEV void sqrt_exact2(float x, float y, float* rx, float* ry) {
   const uint32_t lo = 0x0f800000u, span = 0x7f800000u - lo;
   const uint32_t xr = __float_as_uint(x) - lo, yr = __float_as_uint(y) - lo;
-  if (__builtin_expect(lanes_where((xr > yr ? xr : yr) >= span) != 0, 0)) {
-    *rx = sqrtf(x); *ry = sqrtf(y);
-    return;
-  }
+  const unsigned long long others = lanes_where((xr > yr ? xr : yr) >= span);
   const float px = __builtin_amdgcn_rsqf(x), py = __builtin_amdgcn_rsqf(y);
   const float gx = x * px, gy = y * py;
-  *rx = fmaf(fmaf(-gx, gx, x), 0.5f * px, gx);
-  *ry = fmaf(fmaf(-gy, gy, y), 0.5f * py, gy);
+  float sx = fmaf(fmaf(-gx, gx, x), 0.5f * px, gx), sy = fmaf(fmaf(-gy, gy, y), 0.5f * py, gy);
+  asm volatile("" : "+v"(sx), "+v"(sy));   // the branch comes behind them, when the test has long been made
+  if (__builtin_expect(others != 0, 0)) { sx = sqrtf(x); sy = sqrtf(y); }
+  *rx = sx; *ry = sy;
 }
 
 BPSX_DEV float tri_area2d(const float* a, const float* b, const float* c) {
@@ -514,13 +514,16 @@ struct GeoWave {
     BPSX_KEEP_APART();
     return v;
   }
-  template <bool S> BPSX_DEV void set_links(unsigned long long mask, uint32_t i4, uint32_t v) const {
+  // and that of the node as its chain's first
+  template <bool S> BPSX_DEV void set_links(unsigned long long mask, uint32_t i4, uint32_t v, uint32_t first, uint32_t own) const {
     if (!S || kLinksLds >= kMaxNodes) {
-      lds_store_where(mask, lds_address(L->n_link) + i4, v);
+      asm volatile("s_mov_b64 exec, %0\n\tds_write_b32 %1, %2\n\tds_write_b16 %3, %4\n\ts_mov_b64 exec, -1"
+                   :: "s"(mask), "v"(lds_address(L->n_link) + i4), "v"(v), "v"(first), "v"(own) : "memory");
     } else {
       const unsigned long long near = lanes_where(i4 < kChainEnd);
       lds_store_where(mask & near, lds_address(L->n_link) + i4, v);
       store_where(mask & ~near, ws->links, i4, v);
+      lds_store_half_where(mask, first, own);
     }
   }
   // The entries that the open list keeps apart, over the links that LDS has places for
@@ -560,7 +563,7 @@ struct GeoWave {
 #if BPSX_WINDOW >= 2048
     (void)n;
     static_assert(kLinksLds == kMaxNodes && offsetof(GeoLds, arrived) == offsetof(GeoLds, parents) + kChainEnd / 2, "the header's lane has kChainEnd for a node");
-    const uint32_t p = wlane_at<63>(parent, before);
+    const uint32_t p = wlane_at<62>(parent, before);
     asm volatile("s_mov_b64 exec, %0\n\tglobal_store_dwordx2 %1, %2, %3\n\tds_write_b16 %4, %5\n\ts_mov_b64 exec, -1"
                  :: "s"(mask | header), "v"(offset), "v"(r), "s"(ws->oplog), "v"(lds_address(L->parents) + (i4 >> 1)), "v"(p) : "memory");
 #else
@@ -600,12 +603,12 @@ struct GeoWave {
     nodeCount = 0;
     wave_sync();
   }
-  // Offset of polygon ip's node (offset_of), kChainEnd if it has none; *head receives that of the bucket's first
+  // Offset of polygon ip's node (offset_of), whose chain's first has address `chain`, kChainEnd if it has none; *head receives that of the bucket's first
   // node (what a new node of this bucket links to).  Called by all lanes (those without a polygon with
   // valid == false): the chains are walked in step, one LDS access per lane and round, until every lane
   // has hit or run out, which reads the word at the chains' end again.
-  template <bool S> BPSX_DEV uint32_t find(unsigned long long valid, uint32_t ip, uint32_t bucket, uint32_t* head) const {
-    uint32_t cur = L->first[bucket];
+  template <bool S> BPSX_DEV uint32_t find(unsigned long long valid, uint32_t ip, uint32_t chain, uint32_t* head) const {
+    uint32_t cur = lds_half(chain);
     cur = in_mask(valid) ? cur : kChainEnd;
     *head = cur;
     uint32_t found = kChainEnd;
@@ -1003,7 +1006,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     const uint32_t bucket = GeoWave::hash(nb);
     uint32_t chainHead;
     const unsigned long long valid = lanes_where(nb != kNoNb) & ((1ull << kNvp) - 1ull);
-    const uint32_t at = g.find<true>(valid, nb, bucket, &chainHead);
+    const uint32_t at = g.find<true>(valid, nb, lds_address(&L->first[bucket]), &chainHead);
     const unsigned long long known = lanes_where(at != kChainEnd);
     uint32_t ni4 = GeoWave::node4_at<true>(at);
     const float4 pc = g.node((int)(in_mask(known) ? ni4 >> 2 : 0u));   // (no pick: the mask is a comparison's)
@@ -1025,8 +1028,7 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
     g.nodeCount = want;
     const uint32_t own = GeoWave::offset_of<true>(ni4);
     for (unsigned long long rest = fresh; rest;) {
-      g.set_links<true>(rest, ni4, make_link(nb, chainHead));
-      lds_store_where(rest, &L->first[bucket], own);
+      g.set_links<true>(rest, ni4, make_link(nb, chainHead), lds_address(&L->first[bucket]), own);
       wave_sync();
       chainHead = L->first[bucket];
       rest &= lanes_where(chainHead != own);   // another of the bucket has overwritten it at the chain's head: behind that
@@ -1173,7 +1175,7 @@ BPSX_DEV bool care_for_list(const GeoWave& g, OpenList& ol, uint32_t endIp, cons
 // Returns kAstarTie when the first two entries share the smallest total.
 template <bool S>
 BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, uint32_t endIp, const float* endPos, uint32_t* pops,
-                             bool frontResolved) {
+                             int frontResolved) {
   const int lane = lane_here(g.lane);
   GeoLds* L = g.L;
   const float H_SCALE = 0.999f;
@@ -1185,9 +1187,9 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
   constexpr unsigned long long kOwnLanes = 0x4040404040404040ull;
   static_assert(kNvp == 6 && kRowLanes == 8, "the lane masks of a row");
   constexpr unsigned long long kRows1 = rows_below(1), kRows2 = rows_below(2);   // lanes of the first rows
-  constexpr int kHeaderLane = 63;   // no edge's lane, and all that a pass updates lies before it
+  constexpr int kHeaderLane = 62;   // no edge's lane, and all that a pass updates lies before it
   const char* edges_of = reinterpret_cast<const char*>(edges);
-  bool resolved = frontResolved;
+  int resolved = uniform_i(frontResolved);   // (a truth value would be a mask of lanes, and the branches around it the lanes' own)
   // of every row: its entry of the list, and the total of the entry behind that
   const uint2 first = ol.front(row);
   uint32_t cand = first.x, nextTotal = first.y;
@@ -1212,12 +1214,12 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
   struct {
     unsigned long long updated, fresh;   // lanes of updated nodes, of new ones among them
     uint32_t node4, link;                // the node, its link
-    uint16_t* chain;
+    uint32_t chain;                      // address of its chain's first among L->first
     float4 node;
   } late;
   late.updated = late.fresh = 0;
   late.node4 = late.link = 0;
-  late.chain = L->first;
+  late.chain = lds_address(L->first);
   late.node = make_float4(0, 0, 0, 0);
   const auto insert = [&]() BPSX_INLINE_LAMBDA {
     // The new nodes insert all at once in front of the chain head their lookup saw.  Of several
@@ -1225,22 +1227,33 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     // (looked at below, after the stores that need not wait for it).
     g.clear_marks();
     const uint32_t own = GeoWave::offset_of<S>(late.node4);
-    g.set_links<S>(late.fresh, late.node4, late.link);
-    lds_store_where(late.fresh, late.chain, own);
+    g.set_links<S>(late.fresh, late.node4, late.link, late.chain, own);
     wave_sync();
-    uint32_t head = *late.chain;
+    uint32_t head = lds_half(late.chain);
     if (kAllLds) lds_store_where(late.updated, lds_address(L->w_node) + (late.node4 << 2), late.node);
     else lds_store_where(late.updated & lanes_where((int)late.node4 >= 4 * (g.nodeCount - kWindow)),
                          lds_address(L->w_node) + 16u * GeoWave::window_slot(late.node4), late.node);
     // new nodes that another of their bucket has overwritten at the chain's head go in behind it
     for (unsigned long long lost = late.fresh & lanes_where(head != own); __builtin_expect(lost != 0, 0);) {
-      g.set_links<S>(lost, late.node4, make_link(link_id(late.link), head));
-      lds_store_where(lost, late.chain, own);
+      g.set_links<S>(lost, late.node4, make_link(link_id(late.link), head), late.chain, own);
       wave_sync();
-      head = *late.chain;
+      head = lds_half(late.chain);
       lost &= lanes_where(head != own);
       wave_sync();
     }
+  };
+  // What is late on a way out of the loop is no more than a name: else the compiler keeps it for that way, and copies it at every
+  // pass's end.  (Not where links may spill, whose two instantiations it then gives loops of several ends: 65536 agents over
+  // mixed scenes 2465 -> 2604 us.)  With it, the branch of the roots behind them, and the stores that share a mask in one
+  // statement, a pass is 332 -> 322 instructions in k_geodesic_few: steps of 64 agents 124.7 -> 122.6 us, of 1024 over room plans
+  // 478 -> 468, 3007 fleeing ones 487 -> 463, of 65536 over mixed scenes 2469 -> 2430, of 16384 over mazes 722 -> 710, 300 queries
+  // over room plans 246 -> 240.
+  const auto leave = [&](AstarExit way) BPSX_INLINE_LAMBDA -> AstarExit {
+    if constexpr (kLinksLds >= kMaxNodes) {
+      asm("" : "=s"(late.updated), "=s"(late.fresh), "=v"(late.node4), "=v"(late.link), "=v"(late.chain));
+      asm("" : "=v"(late.node.x), "=v"(late.node.y), "=v"(late.node.z), "=v"(late.node.w));
+    }
+    return way;
   };
   const auto pass = [&]() BPSX_INLINE_LAMBDA -> AstarExit {
     FM(0);
@@ -1250,10 +1263,10 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const AEdge edge = *reinterpret_cast<const AEdge*>(edges_of + ((ip << 7) | (uint32_t)(el << 4)));
     insert();
     FM(1);
-    if (st.logEnd > kOpLogCap - (1 + kRows * kNvp)) return kAstarLogFull;
-    if (ol.needs_care()) return kAstarCare;
+    if (st.logEnd > kOpLogCap - (1 + kRows * kNvp)) return leave(kAstarLogFull);
+    if (ol.needs_care()) return leave(kAstarCare);
     // ---- how many entries at the front are each the only one with their total, and not the goal
-    const unsigned long long uniq = lanes_where(ol.total() < OpenList::down1(OpenList::kEmpty, ol.total())) >> ol.base;
+    const unsigned long long uniq = lanes_where(ol.total() < OpenList::down1(ol.total())) >> ol.base;
     const unsigned long long goal = lanes_where((ol.node() >> 11) == endIp) >> ol.base;
     uint32_t lim = (uint32_t)first_other_lane(uniq & ~goal);
     lim = lim < (uint32_t)kRows ? lim : (uint32_t)kRows;
@@ -1261,23 +1274,23 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     int pairTie = 0;   // 2: with the goal as one of the two
     uint32_t headerWord = kOpHeader;
     if (__builtin_expect(lim == 0, 0)) {
-      if (ol.base >= OpenList::kEnd) return kAstarEmpty;
+      if (ol.base >= OpenList::kEnd) return leave(kAstarEmpty);
       if (uniq & 1ull) lim = (uint32_t)kRows;   // the goal
-      else if (resolved) { lim = 1; resolved = false; }   // the caller has put the reference's next node first
+      else if (resolved) { lim = 1; resolved = 0; }   // the caller has put the reference's next node first
       else {
         // The first two entries share the smallest total.  When they are alone in that and their
         // expansions are independent of each other (neither updates what the other reads, and
         // whatever they put on the list lies above their total), the reference expands them one
         // after the other, in the order its heap has them in, and ends in the same state either
         // way: the pass takes both and notes in the log that their order is open.
-        if (!(uniq & 2ull)) return kAstarTie;
+        if (!(uniq & 2ull)) return leave(kAstarTie);
         pairTie = 1;
         g.pairTies++;   // counts the attempts: one that fails comes back through the log
         lim = (uint32_t)__builtin_ctzll(~(uniq | 3ull) | (1ull << kRows));
       }
       if ((goal & 1ull) && !pairTie) {
         st.lastBest = uniform_i(bi);
-        return kAstarGoal;
+        return leave(kAstarGoal);
       }
       // the goal as one of a tied pair: both rows are looked at
       if (pairTie && (goal & 3ull)) { pairTie = 2; lim = 2; }
@@ -1299,8 +1312,9 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const uint32_t nb = edge.nb;
     const unsigned long long valid = lanes_where(nb != kNoNb) & rowOn;
     const uint32_t hashed = GeoWave::hash_product(in_mask(kOwnLanes) ? ip : nb), bucket = GeoWave::bucket_of<kHashSize>(hashed);
+    const uint32_t chain = lds_address(&L->first[bucket]);
     uint32_t chainHead;
-    const uint32_t at = g.find<S>(valid, nb, bucket, &chainHead);
+    const uint32_t at = g.find<S>(valid, nb, chain, &chainHead);
     FM(3);
     // ---- costs.  A lane without a node to read (idle, or its node is new) reads one of the window's slots.
     const unsigned long long known = lanes_where(at != kChainEnd);
@@ -1329,7 +1343,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     // the lanes that update their node, and the total as bits there, all ones elsewhere.  (A node's
     // total so far is the sum it was computed as, of its cost and the same heuristic.)
     unsigned long long upd = valid & ~(known & lanes_where(total >= p.w + heuristic));
-    const uint32_t tb = in_mask(upd) ? __float_as_uint(total) : 0xffffffffu;
+    uint32_t tb = in_mask(upd) ? __float_as_uint(total) : 0xffffffffu;
     FM(4);
     // ---- how many rows stand
     // conflicts: the first lane that updates a polygon leaves its mark at the polygon's hash, lanes of later rows
@@ -1392,9 +1406,9 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
         // that expansion only creates nodes (none of them can be on the path) and the node pool
         // holds them (an exhausted pool is reported as failure).  Otherwise the heap must say.
         const unsigned long long other = upd & ~lanes_where(ip == endIp);
-        if ((other & known) || g.nodeCount + __popcll(other) > kMaxNodes) return kAstarTie;
+        if ((other & known) || g.nodeCount + __popcll(other) > kMaxNodes) return leave(kAstarTie);
         st.lastBest = (int)rlane((uint32_t)bi, first_lane(goal & 3ull) << kRowShift);
-        return kAstarGoal;
+        return leave(kAstarGoal);
       }
       // a tied pair: both its rows must lie above entry 1's total, ...
       const bool above = rlane(low, kRowLanes) > rlane(nextTotal, 0);
@@ -1416,7 +1430,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
         }
         if (!real) { fails = false; c = 2; }
       }
-      if (fails) return kAstarTie;
+      if (fails) return leave(kAstarTie);
       headerWord = kOpHeader | kOpUnordered | rlane(cand, 0);
     }
     FM(5);
@@ -1427,14 +1441,14 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     const unsigned long long nearby = upd & lanes_where(tb < ol.bound);
     // Nothing has changed yet: a list that would outgrow its registers is split first,
     // links that would outgrow LDS go on in the instantiation that spills.
-    if (__builtin_expect(ol.base + (int)c - __popcll(nearby) < OpenList::kEnd - OpenList::kMost, 0)) return kAstarGrowHeap;
-    if (!S && __builtin_expect(want > kLinksLds, 0)) return kAstarGrowLinks;
+    if (__builtin_expect(ol.base + (int)c - __popcll(nearby) < OpenList::kEnd - OpenList::kMost, 0)) return leave(kAstarGrowHeap);
+    if (!S && __builtin_expect(want > kLinksLds, 0)) return leave(kAstarGrowLinks);
     (*pops) += c;
     // the reference carries on without the nodes that do not fit, but reports anything found
     // after that as failure (only plain DT_SUCCESS counts, PathFinder.cpp:506): stop
     if (S && __builtin_expect(want > kMaxNodes, 0)) {
       st.outOfNodes = true;
-      return kAstarEmpty;
+      return leave(kAstarEmpty);
     }
     FM(6);
     // ---- new nodes (always taken) get consecutive indices in row and edge order
@@ -1444,21 +1458,21 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     late.updated = upd;
     late.node4 = ni4;
     late.link = make_link(nb, chainHead);
-    late.chain = &L->first[bucket];
+    late.chain = chain;
     late.node = make_float4(p0, p1, p2, cost);
     g.nodeCount = want;
     FM(7);
     // the pass in the operation log: the updates in lane order, then the header
     const uint32_t packed = (ni4 >> 2) | (nb << 11);
-    const uint32_t key = wlane_at<kHeaderLane>(tb, c | ((uint32_t)nrec << 8));
+    tb = wlane_at<kHeaderLane>(tb, c | ((uint32_t)nrec << 8));
     const uint32_t word = wlane_at<kHeaderLane>(packed | ((uint32_t)row << 26), headerWord);
     const auto store = [&]() BPSX_INLINE_LAMBDA {
       const uint32_t rec = __builtin_amdgcn_mbcnt_hi((uint32_t)(upd >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)upd, (uint32_t)st.logEnd));
 #if BPSX_FOLLOWER
-      static_assert(kHeaderLane == 63);
-      g.keep_pass(upd, 1ull << kHeaderLane, ni4, late.node, (uint32_t)bi + 1u, (uint32_t)st.logEnd, rec * (uint32_t)sizeof(OpRec), key, word);
+      static_assert(kHeaderLane == 62);
+      g.keep_pass(upd, 1ull << kHeaderLane, ni4, late.node, (uint32_t)bi + 1u, (uint32_t)st.logEnd, rec * (uint32_t)sizeof(OpRec), tb, word);
 #else
-      store_where(upd | (1ull << kHeaderLane), g.ws->oplog, rec * (uint32_t)sizeof(OpRec), key, word);
+      store_where(upd | (1ull << kHeaderLane), g.ws->oplog, rec * (uint32_t)sizeof(OpRec), tb, word);
       g.keep_node(upd, ni4, late.node, (uint32_t)bi + 1u);
 #endif
       st.logEnd += 1 + nrec;
@@ -1489,6 +1503,7 @@ BPSX_DEV AstarExit astar_fast(GeoWave& g, AstarState& st, const AEdge* edges, ui
     way = (int)pass();
     asm volatile("" : "+s"(way));
   } while (way == (int)kAstarOn);
+  asm volatile("" : "+s"(way));   // (what is asked about it behind the loop is not joined to what the loop asks)
   return (AstarExit)way;
 }
 
@@ -1535,14 +1550,14 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
   // the loop is instantiated for links in LDS only or spilling (one instantiation where the LDS
   // holds all links); a search moves on when one more pass could outgrow what it runs in
   AstarExit ex;
-  bool resolved = false;
-  bool spill = kLinksLds >= kMaxNodes;
+  int resolved = 0;
+  int spill = kLinksLds >= kMaxNodes;
   int cared = -1, times = 0;   // where the log was when the list was last put in order, and how often it was there
   for (;;) {
     if constexpr (kLinksLds >= kMaxNodes) ex = astar_fast<true>(g, st, edges, endIp, endPos, pops, resolved);
-    else ex = spill ? astar_fast<true>(g, st, edges, endIp, endPos, pops, resolved) : astar_fast<false>(g, st, edges, endIp, endPos, pops, resolved);
-    resolved = false;
-    if (ex == kAstarGrowLinks) { g.clear_marks(); g.linkSpills++; spill = true; continue; }   // the pass that did not fit has left its marks
+    else ex = uniform_i(spill) ? astar_fast<true>(g, st, edges, endIp, endPos, pops, resolved) : astar_fast<false>(g, st, edges, endIp, endPos, pops, resolved);
+    resolved = 0;
+    if (ex == kAstarGrowLinks) { g.clear_marks(); g.linkSpills++; spill = 1; continue; }   // the pass that did not fit has left its marks
     if (ex == kAstarCare || ex == kAstarGrowHeap) {
       g.clear_marks();
       // (a list that is not in order after a few rounds, of equal totals, does not come to be)
@@ -1571,7 +1586,7 @@ BPSX_DEV int astar(GeoWave& g, FunnelLds* F, const NavData& nav, const SceneDev&
       const uint32_t before = OpenList::up1(st.ol.node());
       const uint32_t node = in_mask(root | (root - 1ull)) ? (lane == st.ol.base ? st.replayRoot : before) : st.ol.node();
       st.ol.e = lane < st.ol.base ? 0ull : OpenList::entry(st.ol.total(), node);
-      resolved = true;
+      resolved = 1;
       continue;
     }
     // such a tie, a list beyond the registers or a full log: on with the reference's heap
