@@ -158,8 +158,11 @@ BPSX_DEV float snap_candidate(const NavData& nav, const SceneDev& s, const PolyR
 }
 
 constexpr float kSnapHalf = 2.0f;
+// A box in the tree's units as it is compared with a node's bounds, two 16-bit numbers a word: no number of the first two may be
+// below that of the node's first two words, nor one of the third above that of the node's third, where what stands for
+// the greater end of an interval in a word of smaller ends (bmin x in w1) is there as its complement.
 struct SnapBox {
-  uint16_t bmin[3], bmax[3];
+  uint32_t w0, w1, w2;   // bmax x, y; bmax z, ~bmin x; bmin y, z
   bool hit_tile;
 };
 BPSX_DEV float clampf(float v, float lo, float hi) { return v < lo ? lo : (v > hi ? hi : v); }
@@ -171,20 +174,34 @@ BPSX_DEV SnapBox snap_box(const SceneDev& s, float px, float py, float pz, float
   const int minx = (int)floorf((qmin[0] - s.orig[0]) / s.tile_w), miny = (int)floorf((qmin[2] - s.orig[2]) / s.tile_h);
   const int maxx = (int)floorf((qmax[0] - s.orig[0]) / s.tile_w), maxy = (int)floorf((qmax[2] - s.orig[2]) / s.tile_h);
   b.hit_tile = !(s.tx < minx || s.tx > maxx || s.ty < miny || s.ty > maxy);
+  uint32_t lo16[3], hi16[3];
   for (int k = 0; k < 3; ++k) {
     const float lo = clampf(qmin[k], s.bmin[k], s.bmax[k]) - s.bmin[k];
     const float hi = clampf(qmax[k], s.bmin[k], s.bmax[k]) - s.bmin[k];
-    b.bmin[k] = (uint16_t)((uint16_t)(int)(s.qfac * lo) & 0xfffe);
-    b.bmax[k] = (uint16_t)((uint16_t)(int)(s.qfac * hi + 1) | 1);
+    lo16[k] = (uint16_t)((uint16_t)(int)(s.qfac * lo) & 0xfffe);
+    hi16[k] = (uint16_t)((uint16_t)(int)(s.qfac * hi + 1) | 1);
   }
+  b.w0 = hi16[0] | (hi16[1] << 16);
+  b.w1 = hi16[2] | ((lo16[0] ^ 0xffffu) << 16);
+  b.w2 = lo16[1] | (lo16[2] << 16);
   return b;
 }
-BPSX_DEV bool box_overlaps(const SnapBox& box, const BVNodeDev& nd) {
-  bool overlap = true;
-#pragma unroll
-  for (int k = 0; k < 3; ++k)
-    if (box.bmin[k] > nd.bmax[k] || box.bmax[k] < nd.bmin[k]) overlap = false;
-  return overlap;
+// by how much the 16-bit halves of a are above those of b, each 0 if it is not
+BPSX_DEV uint32_t above16(uint32_t a, uint32_t b) {
+  uint32_t d;
+  asm("v_pk_sub_u16 %0, %1, %2 clamp" : "=v"(d) : "v"(a), "v"(b));
+  return d;
+}
+// (Number by number the test is some twenty instructions, this way six.)
+struct BVBounds { uint32_t w0, w1, w2, ab; };   // a node's words
+static_assert(sizeof(BVBounds) == sizeof(BVNodeDev) && offsetof(BVNodeDev, bmax) == 6 && offsetof(BVNodeDev, a) == 12, "bmin x, y; bmin z, bmax x; bmax y, z");
+BPSX_DEV bool box_overlaps(const SnapBox& box, uint32_t w0, uint32_t w1, uint32_t w2) {
+  return (above16(w0, box.w0) | above16(w1 ^ 0xffff0000u, box.w1) | above16(box.w2, w2)) == 0;
+}
+BPSX_DEV bool box_overlaps(const SnapBox& box, const BVBounds& nd) { return box_overlaps(box, nd.w0, nd.w1, nd.w2); }
+BPSX_DEV BVBounds bv_node(const BVNodeDev* nodes, uint32_t i) {
+  const uint4 v = reinterpret_cast<const uint4*>(nodes)[i];
+  return {v.x, v.y, v.z, v.w};
 }
 
 // snapPoint, one lane per point: BV-tree walk with escape indices, candidates taken in tree
@@ -201,20 +218,21 @@ BPSX_DEV NavPt snap_point(const NavData& nav, const SceneDev& s, float px, float
   uint32_t bestIp = kInvalidPoly;
   uint32_t i = 0;
   while (i < s.bv_count) {
-    const BVNodeDev nd = nav.bv[s.bv_base + i];
+    const BVBounds nd = bv_node(nav.bv, s.bv_base + i);
     const bool overlap = box_overlaps(box, nd);
-    const bool leaf = nd.b == kBVLeaf;
+    const uint32_t a = nd.ab & 0xffffu;
+    const bool leaf = nd.ab >> 16 == kBVLeaf;
     if (leaf && overlap) {
-      const PolyRec& r = nav.polys[s.poly_base + (uint32_t)nd.a];
+      const PolyRec& r = nav.polys[s.poly_base + a];
       if (r.flags & 1) {
         float cp[3];
         const float d = snap_candidate(nav, s, r, px, py, pz, cp);
         (*ncand)++;
-        if (d < best) { best = d; bestIp = (uint32_t)nd.a; bp[0] = cp[0]; bp[1] = cp[1]; bp[2] = cp[2]; }
+        if (d < best) { best = d; bestIp = a; bp[0] = cp[0]; bp[1] = cp[1]; bp[2] = cp[2]; }
       }
     }
     if (overlap || leaf) i++;
-    else i += (uint32_t)nd.a;
+    else i += a;
   }
   if (bestIp == kInvalidPoly || isnan(bp[0])) return out;
   out.x = bp[0]; out.y = bp[1]; out.z = bp[2];
@@ -446,11 +464,11 @@ BPSX_DEV void snap_candidates(const BVNodeDev* leaves, uint32_t nleaves, uint16_
   const uint32_t ngroups = (nleaves + 63u) / 64u;
   const BVNodeDev* groups = leaves + nleaves;
   for (uint32_t g0 = 0; g0 < ngroups; g0 += 64 * kSnapGroupLoads) {
-    BVNodeDev gr[kSnapGroupLoads];
+    BVBounds gr[kSnapGroupLoads];
 #pragma unroll
     for (int k = 0; k < kSnapGroupLoads; ++k) {
       const uint32_t g = g0 + (uint32_t)(64 * k + lane);
-      gr[k] = groups[g < ngroups ? g : ngroups - 1u];
+      gr[k] = bv_node(groups, g < ngroups ? g : ngroups - 1u);
     }
     int ng = 0;
 #pragma unroll
@@ -466,20 +484,20 @@ BPSX_DEV void snap_candidates(const BVNodeDev* leaves, uint32_t nleaves, uint16_
     const bool last = all && g0 + 64 * kSnapGroupLoads >= ngroups;
     for (int j = 0;; j += kSnapLeafLoads) {
       if (j < ng) {
-        BVNodeDev nd[kSnapLeafLoads];
+        BVBounds nd[kSnapLeafLoads];
         uint32_t at[kSnapLeafLoads];
 #pragma unroll
         for (int k = 0; k < kSnapLeafLoads; ++k) {
           const int gk = __builtin_amdgcn_readfirstlane((int)list[j + k < ng ? j + k : j]);
           at[k] = (uint32_t)gk * kSnapGroup + (uint32_t)lane;
-          nd[k] = leaves[at[k] < nleaves ? at[k] : nleaves - 1u];
+          nd[k] = bv_node(leaves, at[k] < nleaves ? at[k] : nleaves - 1u);
         }
 #pragma unroll
         for (int k = 0; k < kSnapLeafLoads; ++k) {
           // they join the candidates
           const bool isCand = j + k < ng && at[k] < nleaves && box_overlaps(box, nd[k]) && !(grown && box_overlaps(before, nd[k]));
           const unsigned long long m = __ballot(isCand);
-          if (isCand) put(ncands + (int)__popcll(m & ((1ull << lane) - 1ull)), at[k], nd[k].a);
+          if (isCand) put(ncands + (int)__popcll(m & ((1ull << lane) - 1ull)), at[k], (uint16_t)nd[k].ab);
           ncands += (int)__popcll(m);
         }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -584,12 +602,19 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
 // evaluating each point's on their own leaves most lanes idle for the 2900 vector instructions of a
 // snap: here the points' boxes are scanned one after the other and their candidates are evaluated
 // together, 64 at a time, whichever points they belong to.  Point p's state is lane p's; the smallest
-// (distance, place in the array) of each point is found by atomics in LDS.  (50000 points over a cluttered
-// plan: 238 us by a wavefront for each, 159 here.)
+// (distance, place in the array) of each point is found by atomics in LDS.  The groups' bounds are read once for all points,
+// and the leaves of four groups at a time, whichever points' boxes those overlap.  Bound by the evaluation, five batches of 64
+// candidates for 13 points, 60 % of a wavefront's time, and by the wavefronts whose points have most of them.
+// (50000 points over a cluttered plan, read and written in pinned memory: 168 us with the groups scanned anew for every
+// point, their list read back from LDS before their leaves were asked for, and boxes compared number by number; 155 now.  In
+// device memory 238 us by a wavefront for each, 150, 136.)
 constexpr int kSnapBatch = 16;
+constexpr int kSnapPairs = 1024, kSnapPairShift = 12;   // all groups of a round for one point more fit
+static_assert(kSnapPairs > 64 * kSnapGroupLoads && kSnapBatch <= (1 << (16 - kSnapPairShift)) && 0x8000u / kSnapGroup <= (1u << kSnapPairShift), "a pair has 16 bits, and a tile up to 32767 polygons");
 struct SnapBatchLds {
   SnapLds snap;
   uint8_t cand_point[64 * (kSnapLeafLoads + 1)];
+  uint16_t pair[kSnapPairs];             // a group that overlaps a point's box, the point
   unsigned long long best[kSnapBatch];   // bits of the smallest distance, place of its polygon
   float pt[kSnapBatch][4];               // the point; whether its box grows
   float at[kSnapBatch][4];               // the nearest point so far, its polygon
@@ -663,25 +688,82 @@ BPSX_DEV NavPt snap_points_batch(const NavData& nav, const SceneDev& s, bool min
   bool grown = false;   // of all points that are still looked at alike: what overlaps `before` has been looked at
   auto of_lane = [&](const SnapBox& b, int l) BPSX_INLINE_LAMBDA {
     SnapBox r;
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      const uint32_t v = (uint32_t)__builtin_amdgcn_readlane((int)((uint32_t)b.bmin[k] | ((uint32_t)b.bmax[k] << 16)), l);
-      r.bmin[k] = (uint16_t)v; r.bmax[k] = (uint16_t)(v >> 16);
-    }
+    r.w0 = (uint32_t)__builtin_amdgcn_readlane((int)b.w0, l);
+    r.w1 = (uint32_t)__builtin_amdgcn_readlane((int)b.w1, l);
+    r.w2 = (uint32_t)__builtin_amdgcn_readlane((int)b.w2, l);
     r.hit_tile = true;
     return r;
   };
+  const uint32_t nleaves = s.snap_leaves, ngroups = (nleaves + 63u) / 64u;
+  const BVNodeDev* groups = leaves + nleaves;
+  int npairs = 0;
+  // the leaves of the pairs' groups that overlap their points' boxes join the candidates; with `last` all of those are evaluated
+  auto look = [&](bool last) {
+    sync();
+    uint32_t pairs = 0;
+    for (int j = 0;; j += kSnapLeafLoads) {
+      if (j < npairs) {
+        if ((j & 63) == 0) pairs = B.pair[j + lane < npairs ? j + lane : npairs - 1];
+        BVBounds nd[kSnapLeafLoads];
+        uint32_t at[kSnapLeafLoads];
+        int pt[kSnapLeafLoads];
+#pragma unroll
+        for (int k = 0; k < kSnapLeafLoads; ++k) {
+          const uint32_t pair = (uint32_t)__builtin_amdgcn_readlane((int)pairs, (j + k < npairs ? j + k : j) & 63);
+          pt[k] = (int)(pair >> kSnapPairShift);
+          at[k] = (pair & ((1u << kSnapPairShift) - 1u)) * kSnapGroup + (uint32_t)lane;
+          nd[k] = bv_node(leaves, at[k] < nleaves ? at[k] : nleaves - 1u);
+        }
+#pragma unroll
+        for (int k = 0; k < kSnapLeafLoads; ++k) {
+          const bool isCand = j + k < npairs && at[k] < nleaves && box_overlaps(of_lane(box, pt[k]), nd[k]) && !(grown && box_overlaps(of_lane(before, pt[k]), nd[k]));
+          const unsigned long long m = __ballot(isCand);
+          if (isCand) {
+            const int c = ncands + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            B.snap.cand_rank[c] = (uint16_t)at[k];
+            B.snap.cand_poly[c] = (uint16_t)nd[k].ab;
+            B.cand_point[c] = (uint8_t)pt[k];
+          }
+          ncands += (int)__popcll(m);
+        }
+        sync();
+      }
+      const bool end = j + kSnapLeafLoads >= npairs;
+      while (ncands >= (end && last ? 1 : 64)) flush();
+      if (end) break;
+    }
+    npairs = 0;
+  };
+  static_assert(64 % kSnapLeafLoads == 0);
   bool open = mine;
   for (unsigned long long todo = __ballot(open); todo;) {
-    while (todo) {
-      const int p = __builtin_ctzll(todo);
-      todo &= todo - 1ull;
-      const SnapBox pb = of_lane(box, p), pbefore = of_lane(before, p);
-      snap_candidates(leaves, s.snap_leaves, B.snap.group, pb, pbefore, grown, todo == 0, lane, ncands, [&](int c, uint32_t at, uint16_t ip) BPSX_INLINE_LAMBDA {
-        B.snap.cand_rank[c] = (uint16_t)at;
-        B.snap.cand_poly[c] = ip;
-        B.cand_point[c] = (uint8_t)p;
-      }, flush);
+    for (uint32_t g0 = 0; g0 < ngroups; g0 += 64 * kSnapGroupLoads) {
+      for (unsigned long long rest = todo; rest;) {
+        // the groups' bounds are read once for all points, if the pairs have room
+        uint32_t g_w0[kSnapGroupLoads], g_w1[kSnapGroupLoads], g_w2[kSnapGroupLoads];
+#pragma unroll
+        for (int k = 0; k < kSnapGroupLoads; ++k) {
+          const uint32_t g = g0 + (uint32_t)(64 * k + lane);
+          const BVBounds v = bv_node(groups, g < ngroups ? g : ngroups - 1u);
+          g_w0[k] = v.w0; g_w1[k] = v.w1; g_w2[k] = v.w2;
+        }
+        do {
+          const int p = __builtin_ctzll(rest);
+          rest &= rest - 1ull;
+          const SnapBox pb = of_lane(box, p);
+#pragma unroll
+          for (int k = 0; k < kSnapGroupLoads; ++k) {
+            if (g0 + 64u * (uint32_t)k >= ngroups) break;
+            const uint32_t g = g0 + (uint32_t)(64 * k + lane);
+            const bool over = g < ngroups && box_overlaps(pb, g_w0[k], g_w1[k], g_w2[k]);
+            const unsigned long long m = __ballot(over);
+            if (over)
+              B.pair[npairs + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = (uint16_t)(g | ((uint32_t)p << kSnapPairShift));
+            npairs += (int)__popcll(m);
+          }
+        } while (rest && npairs <= kSnapPairs - 64 * kSnapGroupLoads);
+        look(!rest && g0 + 64 * kSnapGroupLoads >= ngroups);
+      }
     }
     if (open) {
       const float reached = __uint_as_float((uint32_t)(B.best[lane] >> 32)), clear = half - kSnapSlack;
