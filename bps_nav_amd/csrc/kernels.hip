@@ -18,10 +18,10 @@
 // depends on it (the reference computes it inside the reset and uses it from the next step on).  A reset
 // of a whole group (bpsx_reset) runs the snaps as a launch of their own before geodesic, first queries
 // included, and so does a step whose launches are timed.
-// The Flee and Exploration tasks (simulator.cpp:830-997) run through the same launches:
+// The Flee task (simulator.cpp:830-869) runs through the same launches:
 // Flee keeps the episode's start point where PointNav keeps the snapped goal, so its
-// "distance from start" is the same start-point -> agent query; Exploration makes no queries,
-// needs no geodesic launch and keeps its visited cells per agent in HBM.
+// "distance from start" is the same start-point -> agent query.  Exploration makes no queries and
+// keeps its visited cells per agent in HBM; a step is one launch of its own (k_step_explore).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -162,13 +162,11 @@ __global__ void k_clear_queues(StepQueues Q) {
   if (blockIdx.x == 0 && threadIdx.x < kQCounters) Q.counts[threadIdx.x] = 0;
 }
 
-// Picks the next episode of agent gi in scene-table entry sc and writes its pose; the snaps follow in
-// reset_snap.  By a row of eight lanes; count: the agent's resets so far.
-BPSX_DEV void begin_reset(const Row& row, const NavData& nav, const AgentArrays& A, const StepParams& P, uint32_t gi, uint32_t sc,
-                          uint32_t count) {
+// The next episode of agent gi in scene-table entry sc, its pose (position, rotation) and goal; returns its index.  By a
+// row of eight lanes; count: the agent's resets so far.
+BPSX_DEV uint32_t draw_episode(const Row& row, const NavData& nav, const StepParams& P, uint32_t gi, uint32_t sc, uint32_t count, float* ep) {
   const SceneDev& s = nav.scenes[sc];
   const uint64_t key = reset_key(P.seed, gi, count);
-  float ep[10];
   uint32_t e = 0;
   if (P.reset_mode == 0) {
     e = draw_index(reset_draw(key, 0), s.ep_count);
@@ -185,7 +183,10 @@ BPSX_DEV void begin_reset(const Row& row, const NavData& nav, const AgentArrays&
     ep[3] = q[0]; ep[4] = q[1]; ep[5] = q[2]; ep[6] = q[3];
     ep[7] = b[0]; ep[8] = b[1]; ep[9] = b[2];
   }
-  if (row.el != 0) return;
+  return e;
+}
+// and by one lane, the episode as the agent's
+BPSX_DEV void store_episode(const AgentArrays& A, uint32_t gi, uint32_t count, uint32_t e, const float* ep) {
   A.nresets[gi] = count + 1;
   A.step[gi] = 1;
   A.last_cost[gi] = kCostUnknown;
@@ -193,6 +194,22 @@ BPSX_DEV void begin_reset(const Row& row, const NavData& nav, const AgentArrays&
   store3(A.pos, gi, ep);
   for (int k = 0; k < 4; ++k) A.rot[(size_t)gi * 4 + k] = ep[3 + k];
   store3(A.goal, gi, ep + 7);
+}
+// Picks the next episode of agent gi and writes its pose; the snaps follow in reset_snap.
+BPSX_DEV void begin_reset(const Row& row, const NavData& nav, const AgentArrays& A, const StepParams& P, uint32_t gi, uint32_t sc,
+                          uint32_t count) {
+  float ep[10];
+  const uint32_t e = draw_episode(row, nav, P, gi, sc, count, ep);
+  if (row.el == 0) store_episode(A, gi, count, e, ep);
+}
+// Where the agent's next episode takes place: if a new scene waits for this env's slot, there (simulator.cpp:1636-1642).
+// By one lane.
+BPSX_DEV uint32_t next_scene(const AgentArrays& A, const StepParams& P, uint32_t gi, uint32_t scene) {
+  const uint32_t tgt = P.swap_target[scene % P.num_slots];
+  if (tgt == kNoSwap || tgt == scene) return scene;
+  A.scene[gi] = tgt;
+  atomicSub(&P.swap_remaining[scene % P.num_slots], 1u);
+  return tgt;
 }
 
 // A row of eight lanes per agent, kMoveItems agents per block: all lanes of a row read the agent's state
@@ -246,14 +263,6 @@ __global__ __launch_bounds__(kMoveItems * 8) void k_step_move(NavData nav, Agent
       const bool distOk = A.dist_ok[gi] == 1;
       const uint32_t expected = A.last_cost[gi];
       const uint32_t resets = A.nresets[gi];
-      const bool explore = P.task == BPSX_TASK_EXPLORATION;
-      uint32_t cnt = 0;
-      float ip[3] = {0, 0, 0}, iq[4] = {0, 0, 0, 0};
-      if (explore) {
-        cnt = A.exp_count[gi];
-        load3(A.exp_init, gi, ip);
-        for (int k = 0; k < 4; ++k) iq[k] = A.exp_inv[(size_t)gi * 4 + k];
-      }
       if (lead) A.step[gi] = step;
       bool done = (float)step >= P.max_steps;
       bool moved = false;
@@ -290,15 +299,10 @@ __global__ __launch_bounds__(kMoveItems * 8) void k_step_move(NavData nav, Agent
         if (lead) write_polar(A, gi, pos, rot, goal);
       }
       // PointNav measures the distance on every move and at the end of the episode, Flee on
-      // moves only, Exploration never (simulator.cpp:758-790, 845-856, 918-927)
-      const bool measure = P.task == BPSX_TASK_POINTNAV ? (done || moved) : (P.task == BPSX_TASK_FLEE && moved);
+      // moves only (simulator.cpp:758-790, 845-856)
+      const bool measure = moved || (done && P.task == BPSX_TASK_POINTNAV);
       const bool reuse = measure && samePoint && distOk;
       if (lead) A.flags[gi] = (done ? kAgentDone : 0u) | (moved ? kAgentMoved : 0u) | (reuse ? kAgentReuse : 0u);
-      if (explore) {
-        // the count is taken before the pose arrays move on to the next episode
-        if (moved) cnt = visit_cell(row, A, gi, cnt, ip, iq, pos);
-        if (lead) A.geo[gi] = (float)(cnt - 1);
-      }
       if (measure && !reuse) {
         want = true;
         for (int k = 0; k < 3; ++k) { q.a[k] = goalNav[k]; q.b[k] = navNow[k]; }
@@ -312,17 +316,10 @@ __global__ __launch_bounds__(kMoveItems * 8) void k_step_move(NavData nav, Agent
       }
       if (done) {
         // the terminal query above holds copies of the old episode's points: the pose arrays can
-        // take the next episode now; distance bookkeeping waits for step_finish.  If a new scene
-        // waits for this env's slot, the next episode is drawn there (simulator.cpp:1636-1642).
+        // take the next episode now; distance bookkeeping waits for step_finish.
         uint32_t scene = scene0;
-        const uint32_t tgt = P.swap_target[scene0 % P.num_slots];
-        if (tgt != kNoSwap && tgt != scene0) {
-          scene = tgt;
-          if (lead) {
-            A.scene[gi] = tgt;
-            atomicSub(&P.swap_remaining[scene0 % P.num_slots], 1u);
-          }
-        }
+        if (lead) scene = next_scene(A, P, gi, scene0);
+        scene = row.get(scene, 0);
         begin_reset(row, nav, A, P, gi, scene, resets);
         reset = true;
       }
@@ -350,6 +347,28 @@ __global__ __launch_bounds__(kMoveItems * 8) void k_step_move(NavData nav, Agent
   if (want) Q.queries[(size_t)cls * Q.stride + queue.base[cls] + place] = q;
   if (reset) Q.reset_list[queue.base[kGeoClasses] + rplace] = gi;
   if (i == 0 && lead) atomicAdd((unsigned long long*)&counter_shard(P.counters)[kCntSteps], (unsigned long long)P.n);
+}
+
+// The state that hangs on an episode's start point, p snapped to r, and the polar observation.  By one lane.
+BPSX_DEV void start_state(const AgentArrays& A, uint32_t task, uint32_t gi, const float* p, const float* rot, const float* goal, const NavPt& r) {
+  const float xyz[3] = {r.x, r.y, r.z};
+  store3(A.nav_xyz, gi, xyz);
+  A.nav_ref[gi] = r.ref;
+  write_polar(A, gi, p, rot, goal);
+  if (task == BPSX_TASK_POINTNAV) return;
+  const float zero[3] = {0, 0, 0};
+  const bool flee = task == BPSX_TASK_FLEE;
+  store3(A.goal_xyz, gi, flee ? xyz : zero);   // Flee: navmeshStart_
+  A.goal_ref[gi] = flee ? r.ref : 0u;
+  if (!flee) {
+    // glm::inverse(q) = conjugate(q) / dot(q, q)
+    const float d = (rot[3] * rot[3] + rot[0] * rot[0]) + (rot[1] * rot[1] + rot[2] * rot[2]);
+    const float inv[4] = {-rot[0] / d, -rot[1] / d, -rot[2] / d, rot[3] / d};
+    for (int k = 0; k < 4; ++k) A.exp_inv[(size_t)gi * 4 + k] = inv[k];
+    store3(A.exp_init, gi, p);
+    cell_of(p, inv, p, A.exp_cells + (size_t)gi * A.cell_cap * 3);   // the set's first
+    A.exp_count[gi] = 1;
+  }
 }
 
 // The snaps of the episodes that begin, a wavefront for each start and, in PointNav, each goal (the
@@ -380,32 +399,16 @@ BPSX_DEV void snap_new_episodes(const NavData& nav, const AgentArrays& A, const 
       q->b[0] = r.x; q->b[1] = r.y; q->b[2] = r.z; q->b_ref = r.ref;
       continue;
     }
-    store3(A.nav_xyz, gi, xyz);
-    A.nav_ref[gi] = r.ref;
     float goal[3], rot[4];
     load3(A.goal, gi, goal);
     for (int k = 0; k < 4; ++k) rot[k] = A.rot[(size_t)gi * 4 + k];
-    write_polar(A, gi, p, rot, goal);
+    start_state(A, P.task, gi, p, rot, goal, r);
     if (pointnav) {
       q->a[0] = r.x; q->a[1] = r.y; q->a[2] = r.z; q->a_ref = r.ref;
       q->scene = scene;
       q->out = P.total + gi;
       q->cost_slot = kNoCostSlot;   // searched agent -> goal: says little about the searches to come
       q->pad = 0;
-      continue;
-    }
-    const float zero[3] = {0, 0, 0};
-    const bool flee = P.task == BPSX_TASK_FLEE;
-    store3(A.goal_xyz, gi, flee ? xyz : zero);   // Flee: navmeshStart_
-    A.goal_ref[gi] = flee ? r.ref : 0u;
-    if (!flee) {
-      // glm::inverse(q) = conjugate(q) / dot(q, q)
-      const float d = (rot[3] * rot[3] + rot[0] * rot[0]) + (rot[1] * rot[1] + rot[2] * rot[2]);
-      const float inv[4] = {-rot[0] / d, -rot[1] / d, -rot[2] / d, rot[3] / d};
-      for (int k = 0; k < 4; ++k) A.exp_inv[(size_t)gi * 4 + k] = inv[k];
-      store3(A.exp_init, gi, p);
-      cell_of(p, inv, p, A.exp_cells + (size_t)gi * A.cell_cap * 3);   // the set's first
-      A.exp_count[gi] = 1;
     }
   }
   if (w == 0 && first && n) {
@@ -456,21 +459,15 @@ __global__ __launch_bounds__(256) void k_step_finish(NavData nav, AgentArrays A,
   const bool done = f & kAgentDone, moved = f & kAgentMoved;
   if (P.task != BPSX_TASK_POINTNAV) {
     if (!(f & kAgentResetOnly)) {
-      float v, reward;
-      if (P.task == BPSX_TASK_FLEE) {
-        v = A.info_prev[gi];
-        if (moved) {
-          if (!(f & kAgentReuse)) v = A.geo[gi];
-          A.info_prev[gi] = v;
-          A.dist_ok[gi] = 1;
-        }
-        reward = v - A.rew_prev[gi];
-      } else {
-        v = A.geo[gi];
-        reward = (float)(0.25 * (double)(v - A.rew_prev[gi]));
+      // Flee (an exploring agent comes here for its reset only)
+      float v = A.info_prev[gi];
+      if (moved) {
+        if (!(f & kAgentReuse)) v = A.geo[gi];
+        A.info_prev[gi] = v;
+        A.dist_ok[gi] = 1;
       }
+      A.rewards[gi] = v - A.rew_prev[gi];
       A.rew_prev[gi] = v;
-      A.rewards[gi] = reward;
       A.masks[gi] = done ? 0 : 1;
       A.infos[gi] = v;
     }
@@ -538,6 +535,144 @@ __global__ __launch_bounds__(256) void k_step_finish(NavData nav, AgentArrays A,
     float pos[3];
     load3(A.pos, gi, pos);
     store3(A.prev_pos, gi, pos);
+  }
+}
+
+// A step of exploring agents, which ask for no distance: one launch, the rows of eight lanes as in k_step_move, the bookkeeping by
+// the row itself, and kExploreSnaps wavefronts of the block that snap the starts of the episodes that begin in it while the
+// rows move: whether an episode ends hangs on the action and on the step's number alone.  What they write is in the rows'
+// place only when those are done; if more episodes end in a block than it has such wavefronts, all of the block's take the rest.
+// Bound by latency, as moves and snaps are, 12 us each.  No list of queries or resets is filled, so the counters of both sets of queues
+// stay as they are, empty.
+// (As k_step_move and k_step_finish, with the snaps in the second, one after the other: 1017 agents over room plans 41.0 us a
+// step, now 30.4; without the host's wait 64 in a room, of whom a quarter end their episode in every step, 29.4 and 28.8, 256 over
+// plans with sampled resets 37.6 and 26.5, 4096 over plans 31.8 and 22.8, 16384 34.5 and 27.8, 32768 48.4 and 43.0, 8192 and 32768 over
+// cluttered plans with sampled resets 48.4 and 45, 74.9 and 73.1.)
+constexpr uint32_t kExploreSnaps = 4;
+__global__ __launch_bounds__(kMoveItems * 8 + kExploreSnaps * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_step_explore(
+    NavData nav, AgentArrays A, StepParams P, const int64_t* __restrict__ actions) {
+  constexpr uint32_t kRowWaves = kMoveItems / 8, kWaves = kRowWaves + kExploreSnaps;
+  __shared__ MoveLds move_lds;
+  __shared__ __attribute__((aligned(16))) uint16_t entered[kMoveItems][kTinyNodes];
+  __shared__ SnapLds snap_lds[kWaves];
+  __shared__ struct {
+    uint32_t count, forward, polys, cands;
+    uint32_t gi[kMoveItems], scene[kMoveItems], resets[kMoveItems];
+    float pose[kWaves][10];   // of the episode that a wavefront begins, and its index
+    uint32_t episode[kWaves];
+  } ends;   // the episodes that end in the block
+  if (threadIdx.x == 0) ends.count = ends.forward = ends.polys = ends.cands = 0;
+  __syncthreads();
+  const Row row;
+  const uint32_t wave = (uint32_t)uniform_i((int)(threadIdx.x >> 6));
+  const bool lead = row.el == 0, of_rows = wave < kRowWaves;
+  const uint32_t item = threadIdx.x >> 3, i = blockIdx.x * kMoveItems + item;
+  uint32_t gi = 0, scene0 = 0, navRef = 0, cnt = 0;
+  int64_t action = -1;
+  bool done = false;
+  float pos[3], rot[4], goal[3], navNow[3], ip[3], iq[4], rewPrev = 0;
+  if (of_rows && i < P.n) {
+    gi = P.base + i;
+    action = actions[i];
+    if (action < 0 || action > 3) {
+      // the reference aborts here (simulator.cpp:704-708); flag it and leave the agent alone
+      if (lead) atomicOr(P.error_flag, 1u);
+      action = -1;
+    } else {
+      // all that the step needs of the agent, asked for together
+      const uint32_t step = A.step[gi] + 1, resets = A.nresets[gi];
+      scene0 = A.scene[gi];
+      load3(A.pos, gi, pos);
+      load3(A.goal, gi, goal);
+      for (int k = 0; k < 4; ++k) rot[k] = A.rot[(size_t)gi * 4 + k];
+      load3(A.nav_xyz, gi, navNow);
+      navRef = A.nav_ref[gi];
+      cnt = A.exp_count[gi];
+      load3(A.exp_init, gi, ip);
+      for (int k = 0; k < 4; ++k) iq[k] = A.exp_inv[(size_t)gi * 4 + k];
+      rewPrev = A.rew_prev[gi];
+      done = action == 0 || (float)step >= P.max_steps;
+      if (lead) {
+        A.step[gi] = step;
+        if (done) {
+          const uint32_t k = atomicAdd(&ends.count, 1u);
+          ends.gi[k] = gi; ends.scene[k] = next_scene(A, P, gi, scene0); ends.resets[k] = resets;
+        }
+      }
+    }
+  }
+  __syncthreads();
+  const uint32_t nends = (uint32_t)uniform_i((int)ends.count);
+  uint32_t cands = 0;
+  NavPt start{};
+  auto begin = [&](uint32_t k) {
+    float ep[10];
+    const uint32_t e = draw_episode(row, nav, P, ends.gi[k], ends.scene[k], ends.resets[k], ep);
+    if ((threadIdx.x & 63u) == 0) {
+      for (int j = 0; j < 10; ++j) ends.pose[wave][j] = ep[j];
+      ends.episode[wave] = e;
+    }
+    start = snap_point_wave(nav, nav.scenes[ends.scene[k]], ep[0], ep[1], ep[2], snap_lds[wave], &cands);
+  };
+  auto store = [&](uint32_t k) {
+    if ((threadIdx.x & 63u) != 0) return;
+    const float* ep = ends.pose[wave];
+    store_episode(A, ends.gi[k], ends.resets[k], ends.episode[wave], ep);
+    start_state(A, BPSX_TASK_EXPLORATION, ends.gi[k], ep, ep + 3, ep + 7, start);
+  };
+  const bool snaps = !of_rows && wave - kRowWaves < nends;
+  if (!of_rows) {
+    if (snaps) begin(wave - kRowWaves);
+  } else if (action >= 0) {
+    bool moved = false;
+    if (action == 1) {
+      const float fwd[3] = {0.f * 0.25f, 0.f * 0.25f, -1.f * 0.25f};
+      float delta[3];
+      quat_rotate(rot, fwd, delta);
+      const NavPt st{navNow[0], navNow[1], navNow[2], navRef};
+      uint32_t polys = 0;
+      const NavPt r = try_step_row(row, nav, nav.scenes[scene0], st, pos[0] + delta[0], pos[1] + delta[1], pos[2] + delta[2], &polys,
+                                   entered[item], move_lds, (int)item);
+      pos[0] = r.x; pos[1] = r.y; pos[2] = r.z;
+      if (lead) {
+        store3(A.nav_xyz, gi, pos);
+        A.nav_ref[gi] = r.ref;
+        store3(A.pos, gi, pos);
+        if (polys) { atomicAdd(&ends.forward, 1u); atomicAdd(&ends.polys, polys); }
+      }
+      moved = true;
+    } else if (action > 1) {
+      quat_mul(rot, action == 2 ? P.turn_left : P.turn_right, rot);
+      if (lead) for (int k = 0; k < 4; ++k) A.rot[(size_t)gi * 4 + k] = rot[k];
+    }
+    if (moved) cnt = visit_cell(row, A, gi, cnt, ip, iq, pos);
+    if (lead) {
+      if (action != 0) write_polar(A, gi, pos, rot, goal);
+      // (simulator.cpp:918-940)
+      const float v = (float)(cnt - 1);
+      A.rewards[gi] = (float)(0.25 * (double)(v - rewPrev));
+      A.masks[gi] = done ? 0 : 1;
+      A.infos[gi] = v;
+      A.rew_prev[gi] = done ? 0.0f : v;
+      if (done) { A.info_prev[gi] = 0.0f; A.dist_ok[gi] = 0; }
+    }
+  }
+  __syncthreads();
+  if (snaps) store(wave - kRowWaves);
+  for (uint32_t k = kExploreSnaps + wave; k < nends; k += kWaves) {
+    begin(k);
+    store(k);
+  }
+  if ((threadIdx.x & 63u) == 0 && cands) atomicAdd(&ends.cands, cands);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    uint64_t* counters = counter_shard(P.counters);
+    auto count = [&](int c, uint32_t n) { if (n) atomicAdd((unsigned long long*)&counters[c], (unsigned long long)n); };
+    count(kCntForward, ends.forward);
+    count(kCntMovePolys, ends.polys);
+    count(kCntResets, nends);
+    count(kCntSnapCands, ends.cands);
+    if (blockIdx.x == 0) count(kCntSteps, P.n);
   }
 }
 
@@ -930,6 +1065,11 @@ SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQue
   int e = 0;
   auto mark = [&]() { if (ev) (void)hipEventRecord(ev[e++], st); };
   mark();
+  if (P.task == BPSX_TASK_EXPLORATION) {
+    hipLaunchKernelGGL(k_step_explore, grid_for(P.n, kMoveItems), dim3(kMoveItems * 8 + kExploreSnaps * 64), 0, st, nav, A, P, actions_dev);
+    for (int k = 1; k < kStepEvents; ++k) mark();
+    return kSearchNone;
+  }
   // Q's lists of queries were emptied two steps ago and have since taken the first queries of
   // the episodes that began in the previous step; its reset list and ticket counter, and the
   // lists of Qnext, were emptied by the previous step's last launch
@@ -944,9 +1084,7 @@ SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQue
   // room for one that asks more, so k_geodesic_few serves groups of up to 1024 agents.  (The line could lie
   // higher: a step over room plans, cluttered plans, mazes takes 450, 718, 414 us by k_geodesic_few and 493, 775, 433 by
   // k_geodesic_mid at 1200 agents, 472, 747, 482 and 516, 788, 507 at 2048, 479, 839, 499 and 518, 835, 471 at 3072.)
-  SearchKernel searches = kSearchNone;
-  if (P.task != BPSX_TASK_EXPLORATION)   // which asks for no distance
-    searches = launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
+  const SearchKernel searches = launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
                                A.last_cost, G, P.n - P.n / 4u, G.mid_steps, P.counters,
                                SnapWork{A, Q, Qnext, P, ev ? 0u : step_snap_blocks * (kSnapWaves / 2u)}, st);
   mark();
