@@ -157,11 +157,6 @@ __global__ void k_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint
   }
 }
 
-// Empties all lists of Q.
-__global__ void k_clear_queues(StepQueues Q) {
-  if (blockIdx.x == 0 && threadIdx.x < kQCounters) Q.counts[threadIdx.x] = 0;
-}
-
 // The next episode of agent gi in scene-table entry sc, its pose (position, rotation) and goal; returns its index.  By a
 // row of eight lanes; count: the agent's resets so far.
 BPSX_DEV uint32_t draw_episode(const Row& row, const NavData& nav, const StepParams& P, uint32_t gi, uint32_t sc, uint32_t count, float* ep) {
@@ -1103,10 +1098,9 @@ SearchKernel launch_reset(const NavData& nav, const AgentArrays& A, const StepQu
   if (P.task != BPSX_TASK_EXPLORATION)
     searches = launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
                                A.last_cost, G, P.n, G.mid_batch, P.counters, NoSnaps{}, st);
-  hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, nav, A, P, Q, Qother, 0u);
-  // the next step finds its lists of queries empty, not with this launch's queries still in them
-  static_assert(kQCounters <= 64);
-  hipLaunchKernelGGL(k_clear_queues, dim3(1), dim3(64), 0, st, Q);
+  // and, as the next step expects them, all lists of Q empty, the reset list among them; Qother's have been since k_reset_all
+  // (by a launch of its own a reset of 2048 agents over mazes took 393.1 us, now 391.4)
+  hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, nav, A, P, Q, Q, 0u);
   return searches;
 }
 void launch_snap_batch(const NavData& nav, uint32_t scene, const float* pts, uint32_t n, float* oxyz, uint32_t* oref,
