@@ -48,6 +48,8 @@ struct Group {
   bool in_flight = false;
   bool profiled = false;
   int record = -1;               // ring entry of the step in flight
+  bool tells = false;            // its last launch tells the host of its end
+  hipStream_t stream = nullptr;  // the one that it was given
 };
 
 // A step that has been enqueued and whose completion the host has not yet seen.  The host may
@@ -58,6 +60,7 @@ struct Group {
 constexpr int kStepRing = 4;
 struct StepRecord {
   hipEvent_t done = nullptr;
+  bool seen = false;             // its last launch has told the host that it is complete: there is no event of it
   uint32_t* remaining = nullptr;   // pinned, one word per scene slot
   uint64_t ordinal = 0;            // sim->steps_started when the step was enqueued
   bool has_remaining = false;
@@ -235,6 +238,9 @@ struct bpsx_sim {
   uint64_t profiled_steps = 0;
   // scratch for the batched query entry points
   void* d_batch = nullptr;
+  uint32_t* h_done = nullptr;        // pinned: number of the newest launch that has told of its end (tell_host)
+  uint32_t* d_done_blocks = nullptr;
+  uint32_t told = 0;                 // launches that have been asked to
   char* h_stage = nullptr;   // pinned: the host arrays of batched calls pass through it (BatchArrays)
   StageRule stage;           // its size
   const char* batch_route = "";   // of the newest batched call
@@ -483,7 +489,8 @@ static void rotation_post_step(bpsx_sim* sim, const StepRecord& rec) {
 static int retire_steps(bpsx_sim* sim, int wait_for) {
   while (sim->ring_count > 0) {
     StepRecord& rec = sim->ring[sim->ring_head];
-    if (wait_for > 0) {
+    if (rec.seen) {
+    } else if (wait_for > 0) {
       HIP_TRY(hipEventSynchronize(rec.done));
     } else {
       const hipError_t q = hipEventQuery(rec.done);
@@ -494,6 +501,35 @@ static int retire_steps(bpsx_sim* sim, int wait_for) {
     sim->ring_head = (sim->ring_head + 1) % kStepRing;
     sim->ring_count--;
     wait_for--;
+  }
+  return BPSX_OK;
+}
+// Groups of at most so many agents have their launches tell the host of their end.  The last launch of larger ones has the caches
+// written back by so many blocks that it takes longer than an event (exploring agents, event and flag: 2048 36.4 and 31.9 us,
+// 8192 41.2 and 38.7, 16384 43.6 and 44.4, 32768 64 and 69; point-goal agents: 8192 682 and 680, 65536 1141 and 1169).
+constexpr uint32_t kTellAgents = 8192;
+static void ask_to_be_told(bpsx_sim* sim, StepParams* P) {
+  P->done_flag = sim->h_done;
+  P->done_blocks = sim->d_done_blocks;
+  P->done_value = ++sim->told;
+}
+// Waits for that, and after two milliseconds asks the stream as well, which says if a launch has failed.  (The stream may have been
+// given work behind the launch: that is not waited for.  It may be gone, too: then only the device can say.)
+static int wait_to_be_told(bpsx_sim* sim, hipStream_t st) {
+  const auto heard = [sim] { return __atomic_load_n(sim->h_done, __ATOMIC_ACQUIRE) == sim->told; };
+  const auto begun = std::chrono::steady_clock::now();
+  for (uint32_t n = 1; !heard(); ++n) {
+    __builtin_ia32_pause();
+    if (n % 256u || std::chrono::steady_clock::now() - begun < std::chrono::milliseconds(2)) continue;
+    const hipError_t q = hipStreamQuery(st);
+    if (q != hipSuccess) (void)hipGetLastError();
+    if (q == hipErrorNotReady) {
+      std::this_thread::yield();
+      continue;
+    }
+    if (q != hipSuccess && q != hipErrorInvalidHandle && q != hipErrorContextIsDestroyed) HIP_TRY(q);
+    if (!heard()) HIP_TRY(hipDeviceSynchronize());
+    break;
   }
   return BPSX_OK;
 }
@@ -556,7 +592,7 @@ int bpsx_finalize(bpsx_sim* sim) {
   if ((rc = sim->alloc(&sim->d_dverts, cdv * 3))) return rc;
   if ((rc = sim->alloc(&sim->d_scenes, 2 * (size_t)S))) return rc;
   if ((rc = sim->alloc(&sim->d_episodes, cep * 10))) return rc;
-  if ((rc = sim->alloc(&sim->d_swap_target, S)) || (rc = sim->alloc(&sim->d_swap_remaining, S))) return rc;
+  if ((rc = sim->alloc(&sim->d_swap_target, S)) || (rc = sim->alloc(&sim->d_swap_remaining, S)) || (rc = sim->alloc(&sim->d_done_blocks, 1))) return rc;
   sim->ar_poly.init(cpoly); sim->ar_bv.init(cbv); sim->ar_tri.init(ctri); sim->ar_dv.init(cdv); sim->ar_ep.init(cep);
   sim->ranges.assign(2 * (size_t)S, SceneRanges{});
   sim->nav = NavData{sim->d_polys, sim->d_aedges, sim->d_bv, sim->d_dtris, sim->d_dverts, sim->d_scenes, sim->d_episodes};
@@ -567,6 +603,8 @@ int bpsx_finalize(bpsx_sim* sim) {
   HIP_TRY(hipStreamCreateWithFlags(&sim->upload_stream, hipStreamNonBlocking));
   HIP_TRY(hipHostMalloc((void**)&sim->h_swap_remaining, (size_t)S * 4, hipHostMallocDefault));
   memset(sim->h_swap_remaining, 0, (size_t)S * 4);
+  HIP_TRY(hipHostMalloc((void**)&sim->h_done, sizeof(uint32_t), hipHostMallocCoherent));
+  *sim->h_done = 0;
   for (StepRecord& rec : sim->ring) {
     HIP_TRY(hipEventCreateWithFlags(&rec.done, hipEventDisableTiming));
     HIP_TRY(hipHostMalloc((void**)&rec.remaining, (size_t)S * 4, hipHostMallocDefault));
@@ -674,6 +712,7 @@ void bpsx_destroy(bpsx_sim* sim) {
   }
   if (sim->upload_stream) (void)hipStreamDestroy(sim->upload_stream);
   if (sim->h_swap_remaining) (void)hipHostFree(sim->h_swap_remaining);
+  if (sim->h_done) (void)hipHostFree(sim->h_done);
   for (StepRecord& rec : sim->ring) {
     if (rec.done) (void)hipEventDestroy(rec.done);
     if (rec.remaining) (void)hipHostFree(rec.remaining);
@@ -711,8 +750,12 @@ int bpsx_reset(bpsx_sim* sim, uint32_t group, void* hip_stream) {
   HIP_TRY(hipSetDevice(sim->cfg.gpu_id));
   if ((rc = quiesce(sim))) return rc;
   hipStream_t st = (hipStream_t)hip_stream;
-  sim->searches = launch_reset(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], sim->params(group), sim->geo, sim->snap_blocks, st);
+  StepParams P = sim->params(group);
+  const bool tells = P.n <= kTellAgents;
+  if (tells) ask_to_be_told(sim, &P);
+  sim->searches = launch_reset(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, sim->geo, sim->snap_blocks, st);
   HIP_TRY(hipGetLastError());
+  if (tells) return wait_to_be_told(sim, st);
   HIP_TRY(hipStreamSynchronize(st));
   return BPSX_OK;
 }
@@ -744,10 +787,6 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   g.profiled = sim->profiling;
   StepParams P = sim->params(group);
   P.defer_first_distance = 1;
-  sim->searches = launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->geo, sim->snap_blocks, st,
-                              g.profiled ? g.ev : nullptr);
-  g.turn ^= 1;
-  HIP_TRY(hipGetLastError());
   g.record = (sim->ring_head + sim->ring_count) % kStepRing;
   StepRecord& rec = sim->ring[g.record];
   rec.ordinal = sim->steps_started;
@@ -755,9 +794,18 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   rec.has_remaining = false;
   for (uint32_t slot = 0; slot < sim->cfg.num_active_scenes && !rec.has_remaining; ++slot)
     rec.has_remaining = sim->slots[slot].target != kNoSwap && sim->slots[slot].target != sim->slots[slot].current;
+  // Where step_end will wait for nothing but the step's own launches the last of them may tell the host; else there is an event.
+  rec.seen = false;
+  g.tells = P.n <= kTellAgents && !sim->stream_ordered && !g.profiled && !rec.has_remaining;
+  g.stream = st;
+  if (g.tells) ask_to_be_told(sim, &P);
+  sim->searches = launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->geo, sim->snap_blocks, st,
+                              g.profiled ? g.ev : nullptr);
+  g.turn ^= 1;
+  HIP_TRY(hipGetLastError());
   if (rec.has_remaining)
     HIP_TRY(hipMemcpyAsync(rec.remaining, sim->d_swap_remaining, (size_t)sim->cfg.num_active_scenes * 4, hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipEventRecord(rec.done, st));
+  if (!g.tells) HIP_TRY(hipEventRecord(rec.done, st));
   sim->ring_count++;
   g.in_flight = true;
   sim->steps_started++;
@@ -774,6 +822,10 @@ int bpsx_step_end(bpsx_sim* sim, uint32_t group) {
   // Host-synchronous stepping waits for the step here.  Stream-ordered stepping does not: the
   // step's outputs are complete for whatever is enqueued next on the stream step_start was
   // given, and the host only looks at what earlier steps have brought back.
+  if (g.tells) {
+    if ((rc = wait_to_be_told(sim, g.stream))) return rc;
+    sim->ring[g.record].seen = true;
+  }
   if ((rc = retire_steps(sim, (sim->stream_ordered && !g.profiled) ? 0 : sim->ring_count))) return rc;
   g.in_flight = false;
   if (g.profiled) {

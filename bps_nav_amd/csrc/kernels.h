@@ -48,6 +48,11 @@ struct StepParams {
   // 1: the first distance of an episode that begins in this step is measured in the next step's
   // launch (see launch_step); 0: in this one
   uint32_t defer_first_distance;
+  // what the launch's last block tells a waiting host (tell_host): done_value at done_flag, in pinned memory, null if nobody waits;
+  // done_blocks counts the blocks that have ended, and is 0 between launches
+  uint32_t* done_flag;
+  uint32_t* done_blocks;
+  uint32_t done_value;
 };
 constexpr uint32_t kNoSwap = 0xffffffffu;
 

@@ -149,6 +149,20 @@ BPSX_DEV uint32_t visit_cell(const Row& row, const AgentArrays& A, uint32_t gi, 
   return n + 1;
 }
 
+// The end of a block of a step's last launch, for all its threads.  Its last block of `blocks` tells a host that waits that all
+// that the launch has written can be seen: a host that waits for an event behind the launch hears of it later (a step of 64
+// agents in a room 121.4 -> 117.1 us, of 1017 that explore 30.4 -> 26.5).  One write-back for a block, once its
+// wavefronts' stores have arrived: one for each wavefront costs the half of the gain.
+BPSX_DEV void tell_host(const StepParams& P, uint32_t blocks) {
+  if (!P.done_flag) return;
+  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+  const uint32_t before = atomicInc(P.done_blocks, blocks - 1u);   // 0 again after the last
+  if (before == blocks - 1u) __hip_atomic_store(P.done_flag, P.done_value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // makes scene-table entry `target` what the envs of `slot` move to when their episodes end
 __global__ void k_set_swap(uint32_t* swap_target, uint32_t* swap_remaining, uint32_t slot, uint32_t target, uint32_t envs) {
   if (threadIdx.x == 0 && blockIdx.x == 0) {
@@ -421,34 +435,8 @@ __global__ __launch_bounds__(kSnapWaves * 64) __attribute__((amdgpu_waves_per_eu
   snap_new_episodes(nav, A, Q, Qout, P, blockIdx.x * kSnapWaves + half, gridDim.x * kSnapWaves, lds[half]);
 }
 
-// The bookkeeping of a step's agents, and in its first snap_blocks blocks, unless the searches' launch has taken
-// them, the snaps of the episodes that began in it, which touch nothing that the bookkeeping touches: no output of this step depends on an
-// episode's first distance (the reference computes it inside the reset and uses it from the next step
-// on), so its query goes to the next step's queues.
-// (On a second stream next to the searches they cost the step two waits between streams, 6 to 17 us before
-// the searches begin and 6 at its end, for the 9 us by which they outlast the bookkeeping of a small
-// group: a step of 64 agents 232 us, now 219, of 1017 exploring ones 62 and 41.  At 16384 agents, whose 655
-// new episodes take 22 us here, it makes no difference: 1193 us both ways without the copies of the counters.)
-// Q: the lists of queries that this step's searches have just served; Qnext: the other set.  The
-// counters of both are left as the next step expects them, so that a step needs no launch of its own
-// for it: the served lists and their ticket counter empty, and the reset list of the step before.
-__global__ __launch_bounds__(256) void k_step_finish(NavData nav, AgentArrays A, StepParams P, StepQueues Q, StepQueues Qnext, uint32_t snap_blocks) {
-  __shared__ SnapLds lds[kSnapWaves];
-  static_assert(kSnapWaves * 64 == 256, "a wavefront each");
-  if (blockIdx.x < snap_blocks) {
-    const uint32_t wave = threadIdx.x >> 6;
-    snap_new_episodes(nav, A, Q, Qnext, P, blockIdx.x * kSnapWaves + wave, snap_blocks * kSnapWaves, lds[wave]);
-    return;
-  }
-  const uint32_t block = blockIdx.x - snap_blocks;
-  if (block == 0) {
-    static_assert(kQGeoHead == kQGeo + kGeoClasses && kGeoClasses + 1 < 256, "one thread per counter");
-    if (threadIdx.x <= (uint32_t)kGeoClasses) Q.counts[kQGeo + threadIdx.x] = 0;
-    else if (threadIdx.x == (uint32_t)kGeoClasses + 1u) Qnext.counts[kQReset] = 0;
-  }
-  const uint32_t i = block * 256u + threadIdx.x;
-  if (i >= P.n) return;
-  const uint32_t gi = P.base + i;
+// The bookkeeping of a step's agent.
+BPSX_DEV void finish_agent(const AgentArrays& A, const StepParams& P, uint32_t gi) {
   const uint32_t f = A.flags[gi];
   if (f & kAgentSkip) return;
   const bool done = f & kAgentDone, moved = f & kAgentMoved;
@@ -669,6 +657,37 @@ __global__ __launch_bounds__(kMoveItems * 8 + kExploreSnaps * 64) __attribute__(
     count(kCntSnapCands, ends.cands);
     if (blockIdx.x == 0) count(kCntSteps, P.n);
   }
+  tell_host(P, gridDim.x);
+}
+
+// The bookkeeping of a step's agents, and in its first snap_blocks blocks, unless the searches' launch has taken
+// them, the snaps of the episodes that began in it, which touch nothing that the bookkeeping touches: no output of this step depends on an
+// episode's first distance (the reference computes it inside the reset and uses it from the next step
+// on), so its query goes to the next step's queues.
+// (On a second stream next to the searches they cost the step two waits between streams, 6 to 17 us before
+// the searches begin and 6 at its end, for the 9 us by which they outlast the bookkeeping of a small
+// group: a step of 64 agents 232 us, now 219, of 1017 exploring ones 62 and 41.  At 16384 agents, whose 655
+// new episodes take 22 us here, it makes no difference: 1193 us both ways without the copies of the counters.)
+// Q: the lists of queries that this step's searches have just served; Qnext: the other set.  The
+// counters of both are left as the next step expects them, so that a step needs no launch of its own
+// for it: the served lists and their ticket counter empty, and the reset list of the step before.
+__global__ __launch_bounds__(256) void k_step_finish(NavData nav, AgentArrays A, StepParams P, StepQueues Q, StepQueues Qnext, uint32_t snap_blocks) {
+  __shared__ SnapLds lds[kSnapWaves];
+  static_assert(kSnapWaves * 64 == 256, "a wavefront each");
+  if (blockIdx.x < snap_blocks) {
+    const uint32_t wave = threadIdx.x >> 6;
+    snap_new_episodes(nav, A, Q, Qnext, P, blockIdx.x * kSnapWaves + wave, snap_blocks * kSnapWaves, lds[wave]);
+  } else {
+    const uint32_t block = blockIdx.x - snap_blocks;
+    if (block == 0) {
+      static_assert(kQGeoHead == kQGeo + kGeoClasses && kGeoClasses + 1 < 256, "one thread per counter");
+      if (threadIdx.x <= (uint32_t)kGeoClasses) Q.counts[kQGeo + threadIdx.x] = 0;
+      else if (threadIdx.x == (uint32_t)kGeoClasses + 1u) Qnext.counts[kQReset] = 0;
+    }
+    const uint32_t i = block * 256u + threadIdx.x;
+    if (i < P.n) finish_agent(A, P, P.base + i);
+  }
+  tell_host(P, gridDim.x);
 }
 
 __global__ __launch_bounds__(256) void k_reset_all(NavData nav, AgentArrays A, StepQueues Q, StepQueues Qother, StepParams P) {
