@@ -323,9 +323,9 @@ BPSX_DEV bool point_in_poly(float px, float pz, const PolyRegs& P) {
 // dtNavMesh::getPolyHeight on a record in registers (`mem`: the same record in memory, for the
 // rare fall-back to the detail edges).  The index words of the first four detail triangles go
 // out together.
-BPSX_DEV bool poly_height(const NavData& nav, const PolyRegs& P, const PolyRec& mem, float px, float py, float pz, float& h) {
-  if (P.type() != 0) return false;
-  if (!point_in_poly(px, pz, P)) return false;
+BPSX_DEV bool poly_over(const PolyRegs& P, float px, float pz) { return P.type() == 0 && point_in_poly(px, pz, P); }
+BPSX_DEV float height_over(const NavData& nav, const PolyRegs& P, const PolyRec& mem, float px, float py, float pz) {   // of a polygon that it is over
+  float h;
   const int tc = P.tri_count(), nv = P.nv();
   const uint32_t* tris = reinterpret_cast<const uint32_t*>(nav.dtris) + P.tri_base();   // four bytes per triangle
   const uint32_t t0 = 0 < tc ? tris[0] : 0u, t1 = 1 < tc ? tris[1] : 0u, t2 = 2 < tc ? tris[2] : 0u, t3 = 3 < tc ? tris[3] : 0u;
@@ -341,15 +341,19 @@ BPSX_DEV bool poly_height(const NavData& nav, const PolyRegs& P, const PolyRec& 
     corner(t & 0xffu, a); corner((t >> 8) & 0xffu, b); corner((t >> 16) & 0xffu, c);
     return height_on_triangle(px, pz, a, b, c, h);
   };
-  if (0 < tc && inside(t0)) return true;
-  if (1 < tc && inside(t1)) return true;
-  if (2 < tc && inside(t2)) return true;
-  if (3 < tc && inside(t3)) return true;
+  if (0 < tc && inside(t0)) return h;
+  if (1 < tc && inside(t1)) return h;
+  if (2 < tc && inside(t2)) return h;
+  if (3 < tc && inside(t3)) return h;
   for (int j = 4; j < tc; ++j)
-    if (inside(tris[j])) return true;
+    if (inside(tris[j])) return h;
   float c[3];
   closest_on_detail_edges<false>(nav, mem, px, py, pz, c);
-  h = c[1];
+  return c[1];
+}
+BPSX_DEV bool poly_height(const NavData& nav, const PolyRegs& P, const PolyRec& mem, float px, float py, float pz, float& h) {
+  if (!poly_over(P, px, pz)) return false;
+  h = height_over(nav, P, mem, px, py, pz);
   return true;
 }
 
@@ -598,17 +602,21 @@ BPSX_DEV NavPt snap_point_wave(const NavData& nav, const SceneDev& s, float px, 
   return out;
 }
 
-// The same for up to kSnapBatch points of one scene by one wavefront.  A point has about five candidates, so
-// evaluating each point's on their own leaves most lanes idle for the 2900 vector instructions of a
-// snap: here the points' boxes are scanned one after the other and their candidates are evaluated
-// together, 64 at a time, whichever points they belong to.  Point p's state is lane p's; the smallest
-// (distance, place in the array) of each point is found by atomics in LDS.  The groups' bounds are read once for all points,
-// and the leaves of four groups at a time, whichever points' boxes those overlap.  Bound by the evaluation, five batches of 64
-// candidates for 13 points, 60 % of a wavefront's time, and by the wavefronts whose points have most of them.
+// The same for up to kSnapBatch points of one scene by one wavefront.  A point has about five candidates in the first box and some
+// twenty in all, so evaluating each point's on their own leaves most lanes idle: here the points' boxes are scanned one after the
+// other and their candidates are looked at together, 64 at a time, whichever points they belong to.  Point p's state is lane p's;
+// the smallest (distance, place in the array) of each point is found by atomics in LDS.  The groups' bounds are read once for all
+// points, and the leaves of four groups at a time, whichever points' boxes those overlap.
+//
+// The candidates are first only sorted: whether their points are over them takes a tenth of the instructions that a distance
+// does.  The few that are (one or two of a point's) are evaluated together, and then, with what those have reached, the others
+// that may still be nearer.  So full wavefronts evaluate heights and edges, each once or twice in a round of boxes, where 64
+// candidates as they came had some of either kind.  Bound by the sorting's and the scan's instructions.
 // (50000 points over a cluttered plan, read and written in pinned memory: 168 us with the groups scanned anew for every
-// point, their list read back from LDS before their leaves were asked for, and boxes compared number by number; 155 now.  In
-// device memory 238 us by a wavefront for each, 150, 136.)
+// point, their list read back from LDS before their leaves were asked for, and boxes compared number by number; 155 with five
+// batches of 64 candidates evaluated as they came; 127 now.  In device memory 238 us by a wavefront for each, 150, 136, 106.)
 constexpr int kSnapBatch = 16;
+constexpr int kSnapBeside = 256;   // 13 points' candidates of a round
 constexpr int kSnapPairs = 1024, kSnapPairShift = 12;   // all groups of a round for one point more fit
 static_assert(kSnapPairs > 64 * kSnapGroupLoads && kSnapBatch <= (1 << (16 - kSnapPairShift)) && 0x8000u / kSnapGroup <= (1u << kSnapPairShift), "a pair has 16 bits, and a tile up to 32767 polygons");
 struct SnapBatchLds {
@@ -618,6 +626,10 @@ struct SnapBatchLds {
   unsigned long long best[kSnapBatch];   // bits of the smallest distance, place of its polygon
   float pt[kSnapBatch][4];               // the point; whether its box grows
   float at[kSnapBatch][4];               // the nearest point so far, its polygon
+  // candidates, place and polygon, whose points are over them, and the others with a bound of their squared distances
+  uint32_t over[128], beside[kSnapBeside];
+  float beside_dist2[kSnapBeside];
+  uint8_t over_point[128], beside_point[kSnapBeside];
 };
 BPSX_DEV NavPt snap_points_batch(const NavData& nav, const SceneDev& s, bool mine, float px, float py, float pz, SnapBatchLds& B) {
   const int lane = (int)(threadIdx.x & 63);
@@ -640,48 +652,107 @@ BPSX_DEV NavPt snap_points_batch(const NavData& nav, const SceneDev& s, bool min
   sync();
   const BVNodeDev* leaves = nav.bv + s.bv_base + s.bv_count;
   int ncands = 0;
-  auto flush = [&]() {
+  int nover = 0, nbeside = 0;
+  const auto before_me = [](unsigned long long m) BPSX_INLINE_LAMBDA {
+    return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+  };
+  const auto reached_by = [&](uint32_t p) BPSX_INLINE_LAMBDA { return __uint_as_float((uint32_t)(B.best[p] >> 32)); };
+  // a candidate (place << 16 | polygon) of point p lies at cp, the square root of d away
+  auto offer = [&](bool have, uint32_t cand, uint32_t p, float d, float x, float y, float z) BPSX_INLINE_LAMBDA {
+    const bool counts = have && d < kNone;
+    const unsigned long long found = ((unsigned long long)__float_as_uint(d) << 32) | (cand >> 16);
+    if (counts) atomicMin(&B.best[p], found);
+    sync();
+    if (counts && B.best[p] == found) {   // one lane at most: a point meets each leaf once
+      B.at[p][0] = x; B.at[p][1] = y; B.at[p][2] = z; B.at[p][3] = __uint_as_float(cand & 0xffffu);
+    }
+    sync();
+  };
+  // 64 candidates become ones over which their points are and ones beside them
+  auto sort_out = [&]() BPSX_INLINE_LAMBDA {
     const int fit = ncands < 64 ? ncands : 64;
     ncands -= fit;
-    const bool have = lane < fit;
-    uint32_t ip = 0, key = 0, p = 0;
-    float qx = 0, qy = 0, qz = 0;
-    PolyRegs P;
-    bool inside = false, grows = false;
-    unsigned long long found = ~0ull;   // what the lane's polygon comes to
-    float cp[3] = {0, 0, 0};
-    if (have) {
-      ip = B.snap.cand_poly[ncands + lane];
-      key = B.snap.cand_rank[ncands + lane];
+    uint32_t cand = 0, p = 0;
+    bool over = false, beside = false;
+    float dist2 = 0;
+    if (lane < fit) {
+      cand = ((uint32_t)B.snap.cand_rank[ncands + lane] << 16) | B.snap.cand_poly[ncands + lane];
       p = B.cand_point[ncands + lane];
-      qx = B.pt[p][0]; qy = B.pt[p][1]; qz = B.pt[p][2]; grows = B.pt[p][3] != 0;
-      const PolyRec* rec = &nav.polys[s.poly_base + ip];
+      const float qx = B.pt[p][0], qz = B.pt[p][2];
+      PolyRegs P;
+      P.load(&nav.polys[s.poly_base + (cand & 0xffffu)]);
+      over = poly_over(P, qx, qz);
+      if (B.pt[p][3] != 0) dist2 = snap_bounds_dist2(P, qx, qz);
+      beside = !over && !(dist2 > reached_by(p));
+    }
+    const unsigned long long o = __ballot(over), b = __ballot(beside);
+    if (over) { const int at = nover + before_me(o); B.over[at] = cand; B.over_point[at] = (uint8_t)p; }
+    if (beside) { const int at = nbeside + before_me(b); B.beside[at] = cand; B.beside_point[at] = (uint8_t)p; B.beside_dist2[at] = dist2; }
+    nover += (int)__popcll(o); nbeside += (int)__popcll(b);
+    sync();
+  };
+  auto heights = [&]() BPSX_INLINE_LAMBDA {
+    const int fit = nover < 64 ? nover : 64;
+    nover -= fit;
+    const bool have = lane < fit;
+    uint32_t cand = 0, p = 0;
+    float d = 0, qx = 0, qz = 0, h = 0;
+    if (have) {
+      cand = B.over[nover + lane]; p = B.over_point[nover + lane];
+      const PolyRec* rec = &nav.polys[s.poly_base + (cand & 0xffffu)];
+      PolyRegs P;
       P.load(rec);
-      float h = 0;
-      inside = poly_height(nav, P, *rec, qx, qy, qz, h);
-      if (inside) {
-        const float e = fabsf(qy - h) - s.climb, d = e > 0 ? e * e : 0;
-        cp[0] = qx; cp[1] = h; cp[2] = qz;
-        if (d < kNone) found = ((unsigned long long)__float_as_uint(d) << 32) | key;
-        atomicMin(&B.best[p], found);
+      const float qy = B.pt[p][1];
+      qx = B.pt[p][0]; qz = B.pt[p][2];
+      h = height_over(nav, P, *rec, qx, qy, qz);
+      const float e = fabsf(qy - h) - s.climb;
+      d = e > 0 ? e * e : 0;
+    }
+    offer(have, cand, p, d, qx, h, qz);
+  };
+  auto boundaries = [&]() BPSX_INLINE_LAMBDA {
+    const int fit = nbeside < 64 ? nbeside : 64;
+    nbeside -= fit;
+    bool have = lane < fit;
+    uint32_t cand = 0, p = 0;
+    float d = 0, cp[3] = {0, 0, 0};
+    if (have) {
+      cand = B.beside[nbeside + lane]; p = B.beside_point[nbeside + lane];
+      have = !(B.beside_dist2[nbeside + lane] > reached_by(p));
+    }
+    if (have) {
+      PolyRegs P;
+      P.load(&nav.polys[s.poly_base + (cand & 0xffffu)]);
+      const float qx = B.pt[p][0], qy = B.pt[p][1], qz = B.pt[p][2];
+      closest_on_boundary(nav, P, qx, qy, qz, cp);
+      const float dx = qx - cp[0], dy = qy - cp[1], dz = qz - cp[2];
+      d = dx * dx + dy * dy + dz * dz;
+    }
+    offer(have, cand, p, d, cp[0], cp[1], cp[2]);
+  };
+  // Makes room for another sort_out, or evaluates all: the heights first, then of the candidates beside their points those
+  // that may still be nearer.
+  auto evaluate = [&](bool all) BPSX_INLINE_LAMBDA {
+    const bool full = all || nbeside > kSnapBeside - 64;
+    while (nover >= (full ? 1 : 64)) heights();
+    if (!full) return;
+    int left = 0;
+    for (int j = 0; j < nbeside; j += 64) {
+      uint32_t cand = 0, p = 0;
+      float dist2 = 0;
+      bool stays = false;
+      if (j + lane < nbeside) {
+        cand = B.beside[j + lane]; p = B.beside_point[j + lane]; dist2 = B.beside_dist2[j + lane];
+        stays = !(dist2 > reached_by(p));
       }
+      const unsigned long long m = __ballot(stays);
+      sync();
+      if (stays) { const int at = left + before_me(m); B.beside[at] = cand; B.beside_point[at] = (uint8_t)p; B.beside_dist2[at] = dist2; }
+      left += (int)__popcll(m);
+      sync();
     }
-    sync();
-    if (have && !inside) {
-      const float reached = __uint_as_float((uint32_t)(B.best[p] >> 32));
-      if (!(grows && snap_bounds_dist2(P, qx, qz) > reached)) {
-        closest_on_boundary(nav, P, qx, qy, qz, cp);
-        const float dx = qx - cp[0], dy = qy - cp[1], dz = qz - cp[2];
-        const float d = dx * dx + dy * dy + dz * dz;
-        if (d < kNone) found = ((unsigned long long)__float_as_uint(d) << 32) | key;
-        atomicMin(&B.best[p], found);
-      }
-    }
-    sync();
-    if (have && found != ~0ull && B.best[p] == found) {   // one lane at most: a point meets each leaf once
-      B.at[p][0] = cp[0]; B.at[p][1] = cp[1]; B.at[p][2] = cp[2]; B.at[p][3] = __uint_as_float(ip);
-    }
-    sync();
+    nbeside = left;
+    while (nbeside > (all ? 0 : kSnapBeside - 64)) boundaries();
   };
   float half = prune ? kSnapFirst : kSnapHalf;
   SnapBox box = snap_box(s, px, py, pz, half), before = box;
@@ -719,7 +790,7 @@ BPSX_DEV NavPt snap_points_batch(const NavData& nav, const SceneDev& s, bool min
           const bool isCand = j + k < npairs && at[k] < nleaves && box_overlaps(of_lane(box, pt[k]), nd[k]) && !(grown && box_overlaps(of_lane(before, pt[k]), nd[k]));
           const unsigned long long m = __ballot(isCand);
           if (isCand) {
-            const int c = ncands + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+            const int c = ncands + before_me(m);
             B.snap.cand_rank[c] = (uint16_t)at[k];
             B.snap.cand_poly[c] = (uint16_t)nd[k].ab;
             B.cand_point[c] = (uint8_t)pt[k];
@@ -729,7 +800,12 @@ BPSX_DEV NavPt snap_points_batch(const NavData& nav, const SceneDev& s, bool min
         sync();
       }
       const bool end = j + kSnapLeafLoads >= npairs;
-      while (ncands >= (end && last ? 1 : 64)) flush();
+      for (const int least = end && last ? 1 : 64;;) {
+        if (ncands >= least) sort_out();
+        const bool more = ncands >= least;
+        evaluate(end && last && !more);
+        if (!more) break;
+      }
       if (end) break;
     }
     npairs = 0;
@@ -758,7 +834,7 @@ BPSX_DEV NavPt snap_points_batch(const NavData& nav, const SceneDev& s, bool min
             const bool over = g < ngroups && box_overlaps(pb, g_w0[k], g_w1[k], g_w2[k]);
             const unsigned long long m = __ballot(over);
             if (over)
-              B.pair[npairs + (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] = (uint16_t)(g | ((uint32_t)p << kSnapPairShift));
+              B.pair[npairs + before_me(m)] = (uint16_t)(g | ((uint32_t)p << kSnapPairShift));
             npairs += (int)__popcll(m);
           }
         } while (rest && npairs <= kSnapPairs - 64 * kSnapGroupLoads);
