@@ -293,6 +293,54 @@ struct OpenList {
                  : [tb] "v"(tb), [packed] "v"(packed), "2"(end)
                  : "vcc", "scc");
   }
+  // The list with as many entries in the lanes from 0 on, in any order, as it has zeros at least: all of them in order, five
+  // instructions for each of the 21 steps of a bitonic sort, where `enter` has nine for each entry.  A step leaves the smaller
+  // of two entries in the lower one of two lanes and the greater one in the other.  For that the upper one of them has its
+  // negative, and takes the smaller of that and the negative of what the other has.  Distances as in `enter`; the sign of
+  // the next step is made between the last one's and the lane moves.
+#define BPSX_SORT_STEP(get, next) "v_bfi_b32 v41, %[keep], v41, v44\n\tv_lshlrev_b32 v44, " next ", %[lane]\n\t" get "v_min_f64 v[40:41], v[40:41], -v[42:43]\n\t"
+#define BPSX_SORT_DPP(ctrl) "v_mov_b32_dpp v42, v40 " ctrl " row_mask:0xf bank_mask:0xf\n\tv_mov_b32_dpp v43, v41 " ctrl " row_mask:0xf bank_mask:0xf\n\t"
+#define BPSX_SORT_SHIFT4 "v_mov_b32_dpp v42, v40 row_shl:4 row_mask:0xf bank_mask:0x5\n\tv_mov_b32_dpp v43, v41 row_shl:4 row_mask:0xf bank_mask:0x5\n\t" \
+                         "v_mov_b32_dpp v42, v40 row_shr:4 row_mask:0xf bank_mask:0xa\n\tv_mov_b32_dpp v43, v41 row_shr:4 row_mask:0xf bank_mask:0xa\n\t"
+#define BPSX_SORT_LDS(op, which) op " v42, v40 " which "\n\t" op " v43, v41 " which "\n\ts_waitcnt lgkmcnt(0)\n\t"
+#define BPSX_SORT_FAR "ds_bpermute_b32 v42, %[far], v40\n\tds_bpermute_b32 v43, %[far], v41\n\ts_waitcnt lgkmcnt(0)\n\t"
+  BPSX_DEV void sort(int lane) {
+    unsigned long long other, sign;
+    const int far_lane = (63 - lane) * 4;
+    asm volatile("v_lshlrev_b32 v44, 31, %[lane]\n\t"
+                 // blocks of 2, 4, 8 lanes and so on: with the mirror image in the block, then with what is half a block away, a quarter ...
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[1,0,3,2]"), "30")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[3,2,1,0]"), "31")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[1,0,3,2]"), "29")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("row_half_mirror"), "30")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[2,3,0,1]"), "31")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[1,0,3,2]"), "28")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("row_mirror"), "29")
+                 BPSX_SORT_STEP(BPSX_SORT_SHIFT4, "30")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[2,3,0,1]"), "31")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[1,0,3,2]"), "27")
+                 BPSX_SORT_STEP(BPSX_SORT_LDS("ds_swizzle_b32", "offset:0x7c1f"), "28")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("row_ror:8"), "29")
+                 BPSX_SORT_STEP(BPSX_SORT_SHIFT4, "30")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[2,3,0,1]"), "31")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[1,0,3,2]"), "26")
+                 BPSX_SORT_STEP(BPSX_SORT_FAR, "27")
+                 BPSX_SORT_STEP(BPSX_SORT_LDS("ds_swizzle_b32", "offset:0x401f"), "28")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("row_ror:8"), "29")
+                 BPSX_SORT_STEP(BPSX_SORT_SHIFT4, "30")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[2,3,0,1]"), "31")
+                 BPSX_SORT_STEP(BPSX_SORT_DPP("quad_perm:[1,0,3,2]"), "31")
+                 "v_and_b32 v41, %[keep], v41\n\t"
+                 "s_nop 1"
+                 : "+{v[40:41]}"(e), "=&{v[42:43]}"(other), "=&{v[44:45]}"(sign)
+                 : [lane] "v"(lane), [far] "v"(far_lane), [keep] "s"(0x7fffffff)
+                 : "memory");
+  }
+#undef BPSX_SORT_STEP
+#undef BPSX_SORT_DPP
+#undef BPSX_SORT_SHIFT4
+#undef BPSX_SORT_LDS
+#undef BPSX_SORT_FAR
   // v as a select operand under a lane mask that a scalar instruction has written (the compiler does not know the
   // select for a vector instruction, which has to keep two instructions' distance from a comparison: a mask that a
   // comparison alone has made takes a plain select on in_mask.  tests/test_inline_asm_distances.py reads the assembly.)
@@ -1049,8 +1097,10 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
 // The entries that the list keeps apart, looked through: those of nodes that have been updated since are dropped, and the
 // smallest, if the list has room for them, enter it: kPull of them at most if there is a bound that parts so few from
 // the others.  False if the search cannot go on in this form.
-// Bound by two round trips to HBM, for the entries and their nodes, and nine instructions for each that enters; once in ten
-// to fifty passes.
+// Bound by two round trips to HBM, for the entries and their nodes, the search for the bound and the sort; once in ten
+// to fifty passes.  (With those that enter taken one after the other, nine instructions each for some forty: steps of 510 agents
+// in two groups 898 -> 881 us, of 1024 over room plans 462 -> 449, of 4096 over cluttered plans 953 -> 936, of 65536 over mixed
+// scenes 2441 -> 2414, 300 queries over room plans 267 -> 265.5.)
 BPSX_DEV bool refill(const GeoWave& g, OpenList& ol, uint32_t endIp, const float* endPos) {
   // 63 entries at a time: none in lane 63 (enter)
   constexpr int kAtOnce = 63, K = OpenList::kFarCap / kAtOnce, kPull = 46, kPullLeast = 30;
@@ -1110,17 +1160,24 @@ BPSX_DEV bool refill(const GeoWave& g, OpenList& ol, uint32_t endIp, const float
       bound = at_lo >= kPullLeast || at_hi + ol.size() > OpenList::kSplit ? lo : hi;
     }
   }
-  int kept = 0;
+  int kept = 0, entered = 0;
   static_for<0, K>([&](auto J) BPSX_INLINE_LAMBDA {
     constexpr int k = decltype(J)::value;
     if (live[k]) {
       const unsigned long long in = lanes_where(t[k] < bound) & live[k], out = live[k] & ~in;
-      ol.enter(in, in_mask(in) ? t[k] : 0xffffffffu, n[k]);
-      ol.base -= __popcll(in);
+      // those that enter go to the lanes from `entered` on; the others to the last one, where nobody looks
+      const int c = __popcll(in);
+      const uint32_t place = __builtin_amdgcn_mbcnt_hi((uint32_t)(in >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)in, (uint32_t)entered));
+      const int to = (int)(in_mask(in) ? place : 63u) * 4;
+      const uint32_t pt = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)t[k]), pn = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)n[k]);
+      ol.e = in_mask(lane_range(c, entered)) ? OpenList::entry(pt, pn) : ol.e;
+      entered += c;
       store_where(out, apart, 8u * (uint32_t)__builtin_amdgcn_mbcnt_hi((uint32_t)(out >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)out, (uint32_t)kept)), t[k], n[k]);
       kept += __popcll(out);
     }
   });
+  ol.base -= entered;
+  if (entered) ol.sort(lane);
   ol.far = kept;
   ol.bound = kept ? bound : OpenList::kEmpty;
   return kept <= OpenList::kFarKeep && (!kept || ol.size() >= OpenList::kRefill);
