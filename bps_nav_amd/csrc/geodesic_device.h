@@ -1095,15 +1095,17 @@ BPSX_DEV AstarExit astar_exact(GeoWave& g, AstarState& st, const AEdge* edges, u
 }
 
 // The entries that the list keeps apart, looked through: those of nodes that have been updated since are dropped, and the
-// smallest, if the list has room for them, enter it: kPull of them at most if there is a bound that parts so few from
-// the others.  False if the search cannot go on in this form.
+// smallest, if the list has room for them, enter it: kPull of them at most, and kPullLeast at least, if there is a bound that
+// parts so few from the others.  False if the search cannot go on in this form.  (A bound is found in five or six guesses.  With
+// 30 at least there was one guess less, but the entries lasted for fewer passes: 4096 agents over cluttered plans 902 and 892 us,
+// 65536 over mixed scenes 2408 and 2399.  With 38 at most and 26 at least 918 and 2430.)
 // Bound by two round trips to HBM, for the entries and their nodes, the search for the bound and the sort; once in ten
 // to fifty passes.  (With those that enter taken one after the other, nine instructions each for some forty: steps of 510 agents
 // in two groups 898 -> 881 us, of 1024 over room plans 462 -> 449, of 4096 over cluttered plans 953 -> 936, of 65536 over mixed
 // scenes 2441 -> 2414, 300 queries over room plans 267 -> 265.5.)
 BPSX_DEV bool refill(const GeoWave& g, OpenList& ol, uint32_t endIp, const float* endPos) {
   // 63 entries at a time: none in lane 63 (enter)
-  constexpr int kAtOnce = 63, K = OpenList::kFarCap / kAtOnce, kPull = 46, kPullLeast = 30;
+  constexpr int kAtOnce = 63, K = OpenList::kFarCap / kAtOnce, kPull = 46, kPullLeast = 42;
   static_assert(OpenList::kFarCap % kAtOnce == 0, "whole rounds");
   const int lane = lane_here(g.lane);
   uint2* apart = reinterpret_cast<uint2*>(g.far_list());
