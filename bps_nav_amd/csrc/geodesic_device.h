@@ -913,8 +913,7 @@ BPSX_DEV int apply_pass(RefHeap<true>& rh, uint32_t rk, uint32_t rw, unsigned lo
 //               search's from then on, until it goes on with another pass.
 // A new search begins, and writes over the log and the heap, only when the follower has answered the end of the one
 // before (astar waits for that).  The end of all searches it does not answer: what it has fetched by then is not applied.
-// Bound by the heap's operations, 0.3 us per node over mazes and 0.4 over cluttered plans among the wavefronts of eight blocks, where a
-// search takes 0.24 and 0.26.  For the
+// Bound by the heap's operations (RefHeap), which take a little longer than the search's passes where lists are long.  For the
 // search it is one or two instructions a pass, and two fewer around its stores.  (With `arrived` stored apart, five
 // instructions a pass, it cost the searches without ties 2.5 %: steps of 64 agents 161 -> 165 us, a reset of 2048 over
 // mazes 471 -> 483.)
