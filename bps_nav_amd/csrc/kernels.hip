@@ -380,6 +380,20 @@ BPSX_DEV void start_state(const AgentArrays& A, uint32_t task, uint32_t gi, cons
   }
 }
 
+// by one lane: the snapped goal, and it and the snapped start in the episode's first query
+BPSX_DEV void goal_state(const AgentArrays& A, uint32_t gi, const NavPt& r, GeoQuery* q) {
+  const float xyz[3] = {r.x, r.y, r.z};
+  store3(A.goal_xyz, gi, xyz);
+  A.goal_ref[gi] = r.ref;
+  q->b[0] = r.x; q->b[1] = r.y; q->b[2] = r.z; q->b_ref = r.ref;
+}
+BPSX_DEV void start_of_query(const StepParams& P, uint32_t gi, uint32_t scene, const NavPt& r, GeoQuery* q) {
+  q->a[0] = r.x; q->a[1] = r.y; q->a[2] = r.z; q->a_ref = r.ref;
+  q->scene = scene;
+  q->out = P.total + gi;
+  q->cost_slot = kNoCostSlot;   // searched agent -> goal: says little about the searches to come
+  q->pad = 0;
+}
 // The snaps of the episodes that begin, a wavefront for each start and, in PointNav, each goal (the
 // other tasks snap no goal, simulator.cpp:838-843, 906-916): wavefront w of nw takes every nw-th.  The
 // wavefront of the start writes the state that hangs on it and the polar observation; each writes its
@@ -400,25 +414,16 @@ BPSX_DEV void snap_new_episodes(const NavData& nav, const AgentArrays& A, const 
     load3(ofGoal ? A.goal : A.pos, gi, p);
     const NavPt r = snap_point_wave(nav, nav.scenes[scene], p[0], p[1], p[2], lds, &cands);
     if (!first) continue;
-    const float xyz[3] = {r.x, r.y, r.z};
     GeoQuery* q = &Qout.queries[(size_t)kGeoClassUnknown * Qout.stride + i];   // a new episode: no history
     if (ofGoal) {
-      store3(A.goal_xyz, gi, xyz);
-      A.goal_ref[gi] = r.ref;
-      q->b[0] = r.x; q->b[1] = r.y; q->b[2] = r.z; q->b_ref = r.ref;
+      goal_state(A, gi, r, q);
       continue;
     }
     float goal[3], rot[4];
     load3(A.goal, gi, goal);
     for (int k = 0; k < 4; ++k) rot[k] = A.rot[(size_t)gi * 4 + k];
     start_state(A, P.task, gi, p, rot, goal, r);
-    if (pointnav) {
-      q->a[0] = r.x; q->a[1] = r.y; q->a[2] = r.z; q->a_ref = r.ref;
-      q->scene = scene;
-      q->out = P.total + gi;
-      q->cost_slot = kNoCostSlot;   // searched agent -> goal: says little about the searches to come
-      q->pad = 0;
-    }
+    if (pointnav) start_of_query(P, gi, scene, r, q);
   }
   if (w == 0 && first && n) {
     atomicAdd((unsigned long long*)&counter_shard(P.counters)[kCntResets], (unsigned long long)n);
@@ -690,6 +695,7 @@ __global__ __launch_bounds__(256) void k_step_finish(NavData nav, AgentArrays A,
   tell_host(P, gridDim.x);
 }
 
+// A reset of all agents of a group: their episodes drawn, for k_reset_snap.
 __global__ __launch_bounds__(256) void k_reset_all(NavData nav, AgentArrays A, StepQueues Q, StepQueues Qother, StepParams P) {
   // both sets of queues are empty but for the list of resets
   if (blockIdx.x == 0 && threadIdx.x < kQCounters) {
@@ -704,6 +710,56 @@ __global__ __launch_bounds__(256) void k_reset_all(NavData nav, AgentArrays A, S
   if (row.el != 0) return;
   A.flags[gi] = kAgentResetOnly;
   Q.reset_list[i] = gi;
+}
+
+// Both by one launch: the wavefront of a start draws its agent's episode, for that of the goal too.  Both sets of queues are empty but
+// for the episodes' first queries.  Bound by latency, the chain of the draw and of the snap.  (As two launches, and as one: 64
+// point-goal agents 127 and 123 us, 2048 over mazes 383 and 380, 1024 fleeing ones 33.7 and 29.5, 4096 exploring ones 52.3 and 49.8.)
+__global__ __launch_bounds__(kSnapWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_reset_begin(NavData nav, AgentArrays A, StepQueues Q, StepQueues Qother, StepParams P) {
+  __shared__ SnapLds lds[kSnapWaves];
+  __shared__ float pose[kSnapWaves][10];   // of the episode that a wavefront has drawn
+  const bool pointnav = P.task == BPSX_TASK_POINTNAV;
+  const uint32_t wave = (uint32_t)uniform_i((int)(threadIdx.x >> 6)), items = pointnav ? 2u * P.n : P.n;
+  const bool first = (threadIdx.x & 63u) == 0;
+  static_assert(kQCounters <= kSnapWaves * 64, "one thread per counter");
+  if (blockIdx.x == 0 && threadIdx.x < kQCounters) {
+    Q.counts[threadIdx.x] = pointnav && threadIdx.x == kQGeo + kGeoClassUnknown ? P.n : 0u;
+    Qother.counts[threadIdx.x] = 0u;
+  }
+  const Row row;
+  const uint32_t it = blockIdx.x * kSnapWaves + wave, i = pointnav ? it >> 1 : it, gi = P.base + i;
+  const bool ofGoal = pointnav && (wave & 1u);
+  uint32_t scene = 0;
+  if (it < items) {
+    scene = (uint32_t)uniform_i((int)A.scene[gi]);
+    if (!ofGoal) {
+      const uint32_t count = (uint32_t)uniform_i((int)A.nresets[gi]);
+      float ep[10];
+      const uint32_t e = draw_episode(row, nav, P, gi, scene, count, ep);
+      if (first) {
+        store_episode(A, gi, count, e, ep);
+        for (int k = 0; k < 10; ++k) pose[wave][k] = ep[k];
+      }
+    }
+  }
+  __syncthreads();
+  if (it >= items) return;
+  uint32_t cands = 0;
+  const float* ep = pose[ofGoal ? wave - 1u : wave];
+  const float* p = ofGoal ? ep + 7 : ep;
+  const NavPt r = snap_point_wave(nav, nav.scenes[scene], lane_f(p[0], 0), lane_f(p[1], 0), lane_f(p[2], 0), lds[wave], &cands);
+  if (!first) return;
+  uint64_t* shard = counter_shard(P.counters);
+  if (it == 0) atomicAdd((unsigned long long*)&shard[kCntResets], (unsigned long long)P.n);
+  if (cands) atomicAdd((unsigned long long*)&shard[kCntSnapCands], (unsigned long long)cands);
+  GeoQuery* q = &Q.queries[(size_t)kGeoClassUnknown * Q.stride + i];   // a new episode: no history
+  if (ofGoal) {
+    goal_state(A, gi, r, q);
+    return;
+  }
+  start_state(A, P.task, gi, ep, ep + 3, ep + 7, r);
+  if (pointnav) start_of_query(P, gi, scene, r, q);
+  A.flags[gi] = kAgentResetOnly;
 }
 
 #ifdef BPSX_QUERY_TRACE
@@ -1111,13 +1167,21 @@ SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQue
 
 SearchKernel launch_reset(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qother, const StepParams& P,
                   const GeoPool& G, uint32_t snap_blocks, hipStream_t st) {
-  hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 32), dim3(256), 0, st, nav, A, Q, Qother, P);
-  hipLaunchKernelGGL(k_reset_snap, dim3(std::min(snap_blocks, (P.n + 1u) / 2u)), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Q, P);
+  const uint32_t snaps = P.task == BPSX_TASK_POINTNAV ? 2u * P.n : P.n, blocks = (snaps + kSnapWaves - 1u) / kSnapWaves;
+  // In one launch as long as the device holds all blocks at once, four on each compute unit (half of snap_blocks): a draw by a
+  // wavefront of its own takes the place of a snap.  (Two launches, and one: 8192 exploring agents of sampled episodes 68.5 and 78 us,
+  // 4096 point-goal agents of sampled episodes 789 and 793, over mazes 527 and 525.)
+  if (2u * blocks <= snap_blocks) {
+    hipLaunchKernelGGL(k_reset_begin, dim3(blocks), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Qother, P);
+  } else {
+    hipLaunchKernelGGL(k_reset_all, grid_for(P.n, 32), dim3(256), 0, st, nav, A, Q, Qother, P);
+    hipLaunchKernelGGL(k_reset_snap, dim3(snap_blocks), dim3(kSnapWaves * 64), 0, st, nav, A, Q, Q, P);
+  }
   SearchKernel searches = kSearchNone;
   if (P.task != BPSX_TASK_EXPLORATION)
     searches = launch_geodesic(nav, Q.queries, Q.stride, &Q.counts[kQGeo], &Q.counts[kQGeoHead], A.geo,
                                A.last_cost, G, P.n, G.mid_batch, P.counters, NoSnaps{}, st);
-  // and, as the next step expects them, all lists of Q empty, the reset list among them; Qother's have been since k_reset_all
+  // and, as the next step expects them, all lists of Q empty; Qother's have been from the start
   // (by a launch of its own a reset of 2048 agents over mazes took 393.1 us, now 391.4)
   hipLaunchKernelGGL(k_step_finish, grid_for(P.n, 256), dim3(256), 0, st, nav, A, P, Q, Q, 0u);
   return searches;
