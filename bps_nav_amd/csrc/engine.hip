@@ -46,9 +46,6 @@ struct Group {
   hipEvent_t ev[kStepEvents] = {};
   bool in_flight = false;
   bool profiled = false;
-  int record = -1;               // ring entry of the step in flight
-  bool tells = false;            // its last launch tells the host of its end
-  hipStream_t stream = nullptr;  // the one that it was given
 };
 
 // A step that has been enqueued and whose completion the host has not yet seen.  The host may
@@ -59,7 +56,9 @@ struct Group {
 constexpr int kStepRing = 4;
 struct StepRecord {
   hipEvent_t done = nullptr;
-  bool seen = false;             // its last launch has told the host that it is complete: there is no event of it
+  bool tells = false;            // its last launch tells the host of its end, by the number `told`: there is no event of it
+  uint32_t told = 0;
+  hipStream_t stream = nullptr;  // the one that it was given
   uint32_t* remaining = nullptr;   // pinned, one word per scene slot
   uint64_t ordinal = 0;            // sim->steps_started when the step was enqueued
   bool has_remaining = false;
@@ -483,12 +482,46 @@ static void rotation_post_step(bpsx_sim* sim, const StepRecord& rec) {
   }
 }
 
+// Groups of at most so many agents have their launches tell the host of their end.  The last launch of larger ones has the caches
+// written back by so many blocks that it takes longer than an event (exploring agents, event and flag: 2048 36.4 and 31.9 us,
+// 8192 41.2 and 38.7, 16384 43.6 and 44.4, 32768 64 and 69; point-goal agents: 8192 682 and 680, 65536 1141 and 1169).
+constexpr uint32_t kTellAgents = 8192;
+// Returns the number that the launch will tell.  Launches that tell run one after the other (a reset waits for the step in flight
+// before it, and for itself), so the newest number that has been told speaks for all before it.
+static uint32_t ask_to_be_told(bpsx_sim* sim, StepParams* P) {
+  P->done_flag = sim->h_done;
+  P->done_blocks = sim->d_done_blocks;
+  return P->done_value = ++sim->told;
+}
+static bool heard_of(const bpsx_sim* sim, uint32_t told) { return (int32_t)(__atomic_load_n(sim->h_done, __ATOMIC_ACQUIRE) - told) >= 0; }
+// Waits for that, and after two milliseconds asks the stream as well, which says if a launch has failed.  (The stream may have been
+// given work behind the launch: that is not waited for.  It may be gone, too: then only the device can say.)
+static int wait_to_be_told(bpsx_sim* sim, uint32_t told, hipStream_t st) {
+  const auto begun = std::chrono::steady_clock::now();
+  for (uint32_t n = 1; !heard_of(sim, told); ++n) {
+    __builtin_ia32_pause();
+    if (n % 256u || std::chrono::steady_clock::now() - begun < std::chrono::milliseconds(2)) continue;
+    const hipError_t q = hipStreamQuery(st);
+    if (q != hipSuccess) (void)hipGetLastError();
+    if (q == hipErrorNotReady) {
+      std::this_thread::yield();
+      continue;
+    }
+    if (q != hipSuccess && q != hipErrorInvalidHandle && q != hipErrorContextIsDestroyed) HIP_TRY(q);
+    if (!heard_of(sim, told)) HIP_TRY(hipDeviceSynchronize());
+    break;
+  }
+  return BPSX_OK;
+}
 // Takes the records whose steps have completed off the ring, oldest first.  wait_for: number of
-// records that must leave, waiting for their events if need be (ring_count: all of them).
+// records that must leave, waiting for what tells of their end if need be (ring_count: all of them).
 static int retire_steps(bpsx_sim* sim, int wait_for) {
   while (sim->ring_count > 0) {
     StepRecord& rec = sim->ring[sim->ring_head];
-    if (rec.seen) {
+    if (rec.tells) {
+      if (wait_for <= 0 && !heard_of(sim, rec.told)) break;
+      const int rc = wait_to_be_told(sim, rec.told, rec.stream);
+      if (rc) return rc;
     } else if (wait_for > 0) {
       HIP_TRY(hipEventSynchronize(rec.done));
     } else {
@@ -500,35 +533,6 @@ static int retire_steps(bpsx_sim* sim, int wait_for) {
     sim->ring_head = (sim->ring_head + 1) % kStepRing;
     sim->ring_count--;
     wait_for--;
-  }
-  return BPSX_OK;
-}
-// Groups of at most so many agents have their launches tell the host of their end.  The last launch of larger ones has the caches
-// written back by so many blocks that it takes longer than an event (exploring agents, event and flag: 2048 36.4 and 31.9 us,
-// 8192 41.2 and 38.7, 16384 43.6 and 44.4, 32768 64 and 69; point-goal agents: 8192 682 and 680, 65536 1141 and 1169).
-constexpr uint32_t kTellAgents = 8192;
-static void ask_to_be_told(bpsx_sim* sim, StepParams* P) {
-  P->done_flag = sim->h_done;
-  P->done_blocks = sim->d_done_blocks;
-  P->done_value = ++sim->told;
-}
-// Waits for that, and after two milliseconds asks the stream as well, which says if a launch has failed.  (The stream may have been
-// given work behind the launch: that is not waited for.  It may be gone, too: then only the device can say.)
-static int wait_to_be_told(bpsx_sim* sim, hipStream_t st) {
-  const auto heard = [sim] { return __atomic_load_n(sim->h_done, __ATOMIC_ACQUIRE) == sim->told; };
-  const auto begun = std::chrono::steady_clock::now();
-  for (uint32_t n = 1; !heard(); ++n) {
-    __builtin_ia32_pause();
-    if (n % 256u || std::chrono::steady_clock::now() - begun < std::chrono::milliseconds(2)) continue;
-    const hipError_t q = hipStreamQuery(st);
-    if (q != hipSuccess) (void)hipGetLastError();
-    if (q == hipErrorNotReady) {
-      std::this_thread::yield();
-      continue;
-    }
-    if (q != hipSuccess && q != hipErrorInvalidHandle && q != hipErrorContextIsDestroyed) HIP_TRY(q);
-    if (!heard()) HIP_TRY(hipDeviceSynchronize());
-    break;
   }
   return BPSX_OK;
 }
@@ -750,10 +754,10 @@ int bpsx_reset(bpsx_sim* sim, uint32_t group, void* hip_stream) {
   hipStream_t st = (hipStream_t)hip_stream;
   StepParams P = sim->params(group);
   const bool tells = P.n <= kTellAgents;
-  if (tells) ask_to_be_told(sim, &P);
+  const uint32_t told = tells ? ask_to_be_told(sim, &P) : 0;
   sim->searches = launch_reset(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, sim->geo, sim->snap_blocks, st);
   HIP_TRY(hipGetLastError());
-  if (tells) return wait_to_be_told(sim, st);
+  if (tells) return wait_to_be_told(sim, told, st);
   HIP_TRY(hipStreamSynchronize(st));
   return BPSX_OK;
 }
@@ -771,7 +775,8 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   // steps that have completed leave the ring; a full ring makes the host wait for its oldest step
   if ((rc = retire_steps(sim, sim->ring_count == kStepRing ? 1 : 0))) return rc;
   // Steps of all groups share the searches' node pools, so each waits for the one before, whichever
-  // stream that was given (on the same one it comes after it anyway).
+  // stream that was given (on the same one it comes after it anyway).  A step that tells the host of its end is not among them: its
+  // step_end has waited for it.
   if (sim->ring_count) HIP_TRY(hipStreamWaitEvent(st, sim->ring[(sim->ring_head + sim->ring_count - 1) % kStepRing].done, 0));
   const int64_t* d_act = actions;
   if (!actions_on_device) {
@@ -787,25 +792,23 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   g.profiled = sim->profiling;
   StepParams P = sim->params(group);
   P.defer_first_distance = 1;
-  g.record = (sim->ring_head + sim->ring_count) % kStepRing;
-  StepRecord& rec = sim->ring[g.record];
+  StepRecord& rec = sim->ring[(sim->ring_head + sim->ring_count) % kStepRing];
   rec.ordinal = sim->steps_started;
   // how many envs of each slot are still on a scene that is leaving: read back with the step
   rec.has_remaining = false;
   for (uint32_t slot = 0; slot < sim->cfg.num_active_scenes && !rec.has_remaining; ++slot)
     rec.has_remaining = sim->slots[slot].target != kNoSwap && sim->slots[slot].target != sim->slots[slot].current;
   // Where step_end will wait for nothing but the step's own launches the last of them may tell the host; else there is an event.
-  rec.seen = false;
-  g.tells = P.n <= kTellAgents && !sim->stream_ordered && !g.profiled && !rec.has_remaining;
-  g.stream = st;
-  if (g.tells) ask_to_be_told(sim, &P);
+  rec.tells = P.n <= kTellAgents && !sim->stream_ordered && !g.profiled && !rec.has_remaining;
+  rec.stream = st;
+  if (rec.tells) rec.told = ask_to_be_told(sim, &P);
   sim->searches = launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->geo, sim->snap_blocks, st,
                               g.profiled ? g.ev : nullptr);
   g.turn ^= 1;
   HIP_TRY(hipGetLastError());
   if (rec.has_remaining)
     HIP_TRY(hipMemcpyAsync(rec.remaining, sim->d_swap_remaining, (size_t)sim->cfg.num_active_scenes * 4, hipMemcpyDeviceToHost, st));
-  if (!g.tells) HIP_TRY(hipEventRecord(rec.done, st));
+  if (!rec.tells) HIP_TRY(hipEventRecord(rec.done, st));
   sim->ring_count++;
   g.in_flight = true;
   sim->steps_started++;
@@ -822,10 +825,6 @@ int bpsx_step_end(bpsx_sim* sim, uint32_t group) {
   // Host-synchronous stepping waits for the step here.  Stream-ordered stepping does not: the
   // step's outputs are complete for whatever is enqueued next on the stream step_start was
   // given, and the host only looks at what earlier steps have brought back.
-  if (g.tells) {
-    if ((rc = wait_to_be_told(sim, g.stream))) return rc;
-    sim->ring[g.record].seen = true;
-  }
   if ((rc = retire_steps(sim, (sim->stream_ordered && !g.profiled) ? 0 : sim->ring_count))) return rc;
   g.in_flight = false;
   if (g.profiled) {
