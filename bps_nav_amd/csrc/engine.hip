@@ -493,6 +493,13 @@ static uint32_t ask_to_be_told(bpsx_sim* sim, StepParams* P) {
   P->done_blocks = sim->d_done_blocks;
   return P->done_value = ++sim->told;
 }
+// Work that is being captured tells nothing: it does not run now, and its replays would write a number of long ago.
+static bool may_tell(const StepParams& P, hipStream_t st) {
+  if (P.n > kTellAgents) return false;
+  hipStreamCaptureStatus status = hipStreamCaptureStatusActive;
+  if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();   // the launches will say why
+  return status == hipStreamCaptureStatusNone;
+}
 static bool heard_of(const bpsx_sim* sim, uint32_t told) { return (int32_t)(__atomic_load_n(sim->h_done, __ATOMIC_ACQUIRE) - told) >= 0; }
 // Waits for that, and after two milliseconds asks the stream as well, which says if a launch has failed.  (The stream may have been
 // given work behind the launch: that is not waited for.  It may be gone, too: then only the device can say.)
@@ -753,7 +760,7 @@ int bpsx_reset(bpsx_sim* sim, uint32_t group, void* hip_stream) {
   if ((rc = quiesce(sim))) return rc;
   hipStream_t st = (hipStream_t)hip_stream;
   StepParams P = sim->params(group);
-  const bool tells = P.n <= kTellAgents;
+  const bool tells = may_tell(P, st);
   const uint32_t told = tells ? ask_to_be_told(sim, &P) : 0;
   sim->searches = launch_reset(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, sim->geo, sim->snap_blocks, st);
   HIP_TRY(hipGetLastError());
@@ -799,7 +806,7 @@ int bpsx_step_start(bpsx_sim* sim, uint32_t group, const int64_t* actions, int a
   for (uint32_t slot = 0; slot < sim->cfg.num_active_scenes && !rec.has_remaining; ++slot)
     rec.has_remaining = sim->slots[slot].target != kNoSwap && sim->slots[slot].target != sim->slots[slot].current;
   // Where step_end will wait for nothing but the step's own launches the last of them may tell the host; else there is an event.
-  rec.tells = P.n <= kTellAgents && !sim->stream_ordered && !g.profiled && !rec.has_remaining;
+  rec.tells = !sim->stream_ordered && !g.profiled && !rec.has_remaining && may_tell(P, st);
   rec.stream = st;
   if (rec.tells) rec.told = ask_to_be_told(sim, &P);
   sim->searches = launch_step(sim->nav, sim->A, g.Q[g.turn], g.Q[g.turn ^ 1], P, d_act, sim->geo, sim->snap_blocks, st,
