@@ -4,6 +4,7 @@
 
 #include "geodesic_device.h"
 #include "stage_rule.h"
+#include "wait_rule.h"
 
 namespace {
 // the two roots of bits first + i and first + n - 1 - i, a lane per i
@@ -73,4 +74,24 @@ extern "C" __attribute__((visibility("default"))) uint32_t bpsx_check_stage(cons
     held[i] = rule.held;
   }
   return made;
+}
+
+// A wait for a word that comes at look `comes` (0: never), and with `drained` when the device has nothing left to do; the stream answers
+// the i-th question, from the look `patience` on, with answers[i], the last of them again and again (StreamIs).  Returns what the wait
+// comes to (Wait), and in out the looks, the questions, and how often the device was waited for.
+extern "C" __attribute__((visibility("default"))) int bpsx_check_wait(uint32_t comes, int drained, uint32_t patience, const int* answers, uint32_t n, uint32_t* out) {
+  struct {
+    uint32_t comes, patience, n, looks, asked, drains;
+    int drained;
+    const int* answers;
+    bool heard() { ++looks; return (comes && looks >= comes) || (drains && drained > 0); }
+    bool patient() const { return looks < patience; }
+    bpsx::StreamIs stream() { return (bpsx::StreamIs)answers[asked++ < n ? asked - 1u : n - 1u]; }
+    bool drain() { ++drains; return drained >= 0; }
+    void pause() const {}
+    void yield() const {}
+  } rt{comes, patience, n, 0, 0, 0, drained, answers};
+  const int r = (int)bpsx::wait_for_word(rt);
+  out[0] = rt.looks; out[1] = rt.asked; out[2] = rt.drains;
+  return r;
 }

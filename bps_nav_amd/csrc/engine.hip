@@ -23,6 +23,7 @@
 #include "kernels.h"
 #include "navmesh_host.h"
 #include "stage_rule.h"
+#include "wait_rule.h"
 
 using namespace bpsx;
 
@@ -501,24 +502,32 @@ static bool may_tell(const StepParams& P, hipStream_t st) {
   return status == hipStreamCaptureStatusNone;
 }
 static bool heard_of(const bpsx_sim* sim, uint32_t told) { return (int32_t)(__atomic_load_n(sim->h_done, __ATOMIC_ACQUIRE) - told) >= 0; }
-// Waits for that, and after two milliseconds asks the stream as well, which says if a launch has failed.  (The stream may have been
-// given work behind the launch: that is not waited for.  It may be gone, too: then only the device can say.)
+// Waits for that (wait_for_word).
 static int wait_to_be_told(bpsx_sim* sim, uint32_t told, hipStream_t st) {
-  const auto begun = std::chrono::steady_clock::now();
-  for (uint32_t n = 1; !heard_of(sim, told); ++n) {
-    __builtin_ia32_pause();
-    if (n % 256u || std::chrono::steady_clock::now() - begun < std::chrono::milliseconds(2)) continue;
-    const hipError_t q = hipStreamQuery(st);
-    if (q != hipSuccess) (void)hipGetLastError();
-    if (q == hipErrorNotReady) {
-      std::this_thread::yield();
-      continue;
+  struct {
+    const bpsx_sim* sim;
+    uint32_t told;
+    hipStream_t st;
+    std::chrono::steady_clock::time_point begun;
+    hipError_t error;
+    bool heard() const { return heard_of(sim, told); }
+    bool patient() const { return std::chrono::steady_clock::now() - begun < std::chrono::milliseconds(2); }
+    StreamIs stream() {
+      error = hipStreamQuery(st);
+      if (error == hipSuccess) return StreamIs::kIdle;
+      (void)hipGetLastError();
+      if (error == hipErrorNotReady) return StreamIs::kBusy;
+      return error == hipErrorInvalidHandle || error == hipErrorContextIsDestroyed ? StreamIs::kGone : StreamIs::kFailed;
     }
-    if (q != hipSuccess && q != hipErrorInvalidHandle && q != hipErrorContextIsDestroyed) HIP_TRY(q);
-    if (!heard_of(sim, told)) HIP_TRY(hipDeviceSynchronize());
-    break;
+    bool drain() { return (error = hipDeviceSynchronize()) == hipSuccess; }
+    void pause() const { __builtin_ia32_pause(); }
+    void yield() const { std::this_thread::yield(); }
+  } rt{sim, told, st, std::chrono::steady_clock::now(), hipSuccess};
+  switch (wait_for_word(rt)) {
+    case Wait::kTold: return BPSX_OK;
+    case Wait::kNeverTold: return fail(BPSX_E_HIP, "a launch that was to tell of its end has not run");
+    default: return fail(BPSX_E_HIP, std::string("waiting for a launch: ") + hipGetErrorString(rt.error));
   }
-  return BPSX_OK;
 }
 // Takes the records whose steps have completed off the ring, oldest first.  wait_for: number of
 // records that must leave, waiting for what tells of their end if need be (ring_count: all of them).
