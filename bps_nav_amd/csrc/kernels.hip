@@ -526,35 +526,36 @@ BPSX_DEV void finish_agent(const AgentArrays& A, const StepParams& P, uint32_t g
   }
 }
 
-// A step of exploring agents, which ask for no distance: one launch, the rows of eight lanes as in k_step_move, the bookkeeping by
-// the row itself, and kExploreSnaps wavefronts of the block that snap the starts of the episodes that begin in it while the
-// rows move: whether an episode ends hangs on the action and on the step's number alone.  What they write is in the rows'
-// place only when those are done; if more episodes end in a block than it has such wavefronts, all of the block's take the rest.
+// A step of exploring agents, which ask for no distance: one launch.  A block has kRowWaves wavefronts of eight agents each, a row
+// of eight lanes for an agent as in k_step_move, with the bookkeeping by the row itself, and kSnaps wavefronts that begin the episodes
+// of those that end while the rows move: whether an episode ends hangs on the action and on the step's number alone.  Their
+// rows draw all of the block's episodes, one each, and each wavefront snaps the start of one.  What that writes is in the rows'
+// place only when those are done; if more episodes end than there are such wavefronts, all of the block's take the rest.  With no
+// such wavefront the others draw when they have moved.
 // Bound by latency, as moves and snaps are, 12 us each.  No list of queries or resets is filled, so the counters of both sets of queues
 // stay as they are, empty.
 // (As k_step_move and k_step_finish, with the snaps in the second, one after the other: 1017 agents over room plans 41.0 us a
-// step, now 30.4; without the host's wait 64 in a room, of whom a quarter end their episode in every step, 29.4 and 28.8, 256 over
-// plans with sampled resets 37.6 and 26.5, 4096 over plans 31.8 and 22.8, 16384 34.5 and 27.8, 32768 48.4 and 43.0, 8192 and 32768 over
-// cluttered plans with sampled resets 48.4 and 45, 74.9 and 73.1.)
-constexpr uint32_t kExploreSnaps = 4;
-__global__ __launch_bounds__(kMoveItems * 8 + kExploreSnaps * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_step_explore(
+// step, now 26.)
+template <uint32_t kRowWaves, uint32_t kSnaps>
+__global__ __launch_bounds__((kRowWaves + kSnaps) * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_step_explore(
     NavData nav, AgentArrays A, StepParams P, const int64_t* __restrict__ actions) {
-  constexpr uint32_t kRowWaves = kMoveItems / 8, kWaves = kRowWaves + kExploreSnaps;
+  constexpr uint32_t kWaves = kRowWaves + kSnaps, kItems = kRowWaves * 8;
+  static_assert(kItems <= kMoveItems);
   __shared__ MoveLds move_lds;
-  __shared__ __attribute__((aligned(16))) uint16_t entered[kMoveItems][kTinyNodes];
+  __shared__ __attribute__((aligned(16))) uint16_t entered[kItems][kTinyNodes];
   __shared__ SnapLds snap_lds[kWaves];
   __shared__ struct {
     uint32_t count, forward, polys, cands;
-    uint32_t gi[kMoveItems], scene[kMoveItems], resets[kMoveItems];
-    float pose[kWaves][10];   // of the episode that a wavefront begins, and its index
-    uint32_t episode[kWaves];
+    uint32_t gi[kItems], scene[kItems], resets[kItems];
+    float pose[kItems][10];   // of the episodes that begin, and their indices
+    uint32_t episode[kItems];
   } ends;   // the episodes that end in the block
   if (threadIdx.x == 0) ends.count = ends.forward = ends.polys = ends.cands = 0;
   __syncthreads();
   const Row row;
   const uint32_t wave = (uint32_t)uniform_i((int)(threadIdx.x >> 6));
   const bool lead = row.el == 0, of_rows = wave < kRowWaves;
-  const uint32_t item = threadIdx.x >> 3, i = blockIdx.x * kMoveItems + item;
+  const uint32_t item = threadIdx.x >> 3, i = blockIdx.x * kItems + item;
   uint32_t gi = 0, scene0 = 0, navRef = 0, cnt = 0;
   int64_t action = -1;
   bool done = false;
@@ -593,24 +594,38 @@ __global__ __launch_bounds__(kMoveItems * 8 + kExploreSnaps * 64) __attribute__(
   const uint32_t nends = (uint32_t)uniform_i((int)ends.count);
   uint32_t cands = 0;
   NavPt start{};
-  auto begin = [&](uint32_t k) {
-    float ep[10];
-    const uint32_t e = draw_episode(row, nav, P, ends.gi[k], ends.scene[k], ends.resets[k], ep);
-    if ((threadIdx.x & 63u) == 0) {
-      for (int j = 0; j < 10; ++j) ends.pose[wave][j] = ep[j];
-      ends.episode[wave] = e;
-    }
-    start = snap_point_wave(nav, nav.scenes[ends.scene[k]], ep[0], ep[1], ep[2], snap_lds[wave], &cands);
+  auto snap = [&](uint32_t k) {
+    const float* ep = ends.pose[k];
+    const uint32_t scene = (uint32_t)uniform_i((int)ends.scene[k]);
+    start = snap_point_wave(nav, nav.scenes[scene], lane_f(ep[0], 0), lane_f(ep[1], 0), lane_f(ep[2], 0), snap_lds[wave], &cands);
   };
   auto store = [&](uint32_t k) {
     if ((threadIdx.x & 63u) != 0) return;
-    const float* ep = ends.pose[wave];
-    store_episode(A, ends.gi[k], ends.resets[k], ends.episode[wave], ep);
+    const float* ep = ends.pose[k];
+    store_episode(A, ends.gi[k], ends.resets[k], ends.episode[k], ep);
     start_state(A, BPSX_TASK_EXPLORATION, ends.gi[k], ep, ep + 3, ep + 7, start);
   };
-  const bool snaps = !of_rows && wave - kRowWaves < nends;
+  // a wavefront's share of all that end, eight at a time
+  constexpr uint32_t kDrawers = kSnaps ? kSnaps : kWaves;
+  const uint32_t mine = kSnaps ? wave - kRowWaves : wave;
+  auto draw = [&]() {
+    for (uint32_t k0 = mine; k0 < nends; k0 += kDrawers * 8u) {
+      const uint32_t k = k0 + kDrawers * ((threadIdx.x & 63u) >> 3);
+      if (k < nends) {
+        float ep[10];
+        const uint32_t e = draw_episode(row, nav, P, ends.gi[k], ends.scene[k], ends.resets[k], ep);
+        if (lead) {
+          for (int j = 0; j < 10; ++j) ends.pose[k][j] = ep[j];
+          ends.episode[k] = e;
+        }
+      }
+    }
+    wave_sync();
+  };
+  const bool snaps = !of_rows && mine < nends;
   if (!of_rows) {
-    if (snaps) begin(wave - kRowWaves);
+    draw();
+    if (snaps) snap(mine);
   } else if (action >= 0) {
     bool moved = false;
     if (action == 1) {
@@ -645,10 +660,11 @@ __global__ __launch_bounds__(kMoveItems * 8 + kExploreSnaps * 64) __attribute__(
       if (done) { A.info_prev[gi] = 0.0f; A.dist_ok[gi] = 0; }
     }
   }
+  if constexpr (kSnaps == 0) draw();
   __syncthreads();
-  if (snaps) store(wave - kRowWaves);
-  for (uint32_t k = kExploreSnaps + wave; k < nends; k += kWaves) {
-    begin(k);
+  if (snaps) store(mine);
+  for (uint32_t k = kSnaps + wave; k < nends; k += kWaves) {
+    snap(k);
     store(k);
   }
   if ((threadIdx.x & 63u) == 0 && cands) atomicAdd(&ends.cands, cands);
@@ -1130,13 +1146,37 @@ template <class Snaps> static SearchKernel launch_geodesic(const NavData& nav, c
   return kSearchMany;
 }
 
+// Blocks of as few agents as leave one block for each compute unit, and as many wavefronts to begin episodes as have one for each of
+// eight agents, or half as many; of 32 agents and four such wavefronts while two blocks on each compute unit hold all agents; and
+// beyond that without them, since blocks that wait for a place cost more than a draw and a snap behind the moves.  Us a step
+// if none of the agents ends its episode, one in 25, one in four, all; over cluttered plans with sampled episodes:
+//   agents   as two launches      <1, 8>               <2, 4>               <4, 4>               <4, 0>
+//       64   28  49  54   44      22  32  36   39      22  33  44   55      23  33  46   71      23  42   63   98
+//     2048   30  54  73  113      24  34  37   40      24  34  46   61      24  36  52   75      24  47   70  103
+//     4096   30  54  70  114      36  53  60   67      25  35  47   61      24  39  53   76      24  48   71  103
+//     8192   30  55  70  117      57  82 105  122      28  38  52   71      25  40  54   79      25  49   72  106
+//    16384   31  59  76  132      88 132 183  211      45  65  99  154      29  47  63   93      29  56   82  120
+//    32768   42  80 122  230     160 241 339  391      67 103 157  247      47  72 110  163      32  62   91  145
+// (In one form, <4, 4> with a wavefront for each draw, 64 agents 23 33 57 105, 32768 48 80 134 248.)
+template <uint32_t kRowWaves, uint32_t kSnaps>
+static void launch_explore_as(const NavData& nav, const AgentArrays& A, const StepParams& P, const int64_t* actions_dev, hipStream_t st) {
+  hipLaunchKernelGGL((k_step_explore<kRowWaves, kSnaps>), grid_for(P.n, kRowWaves * 8), dim3((kRowWaves + kSnaps) * 64), 0, st, nav, A, P, actions_dev);
+}
+static void launch_explore(const NavData& nav, const AgentArrays& A, const StepParams& P, const int64_t* actions_dev, uint32_t compute_units,
+                           hipStream_t st) {
+  if (P.n <= 8u * compute_units) launch_explore_as<1, 8>(nav, A, P, actions_dev, st);
+  else if (P.n <= 16u * compute_units) launch_explore_as<2, 4>(nav, A, P, actions_dev, st);
+  else if (P.n <= 64u * compute_units) launch_explore_as<4, 4>(nav, A, P, actions_dev, st);
+  else launch_explore_as<4, 0>(nav, A, P, actions_dev, st);
+}
+
 SearchKernel launch_step(const NavData& nav, const AgentArrays& A, const StepQueues& Q, const StepQueues& Qnext, const StepParams& P,
                  const int64_t* actions_dev, const GeoPool& G, uint32_t snap_blocks, hipStream_t st, hipEvent_t* ev) {
   int e = 0;
   auto mark = [&]() { if (ev) (void)hipEventRecord(ev[e++], st); };
   mark();
   if (P.task == BPSX_TASK_EXPLORATION) {
-    hipLaunchKernelGGL(k_step_explore, grid_for(P.n, kMoveItems), dim3(kMoveItems * 8 + kExploreSnaps * 64), 0, st, nav, A, P, actions_dev);
+    launch_explore(nav, A, P, actions_dev, snap_blocks / 8u, st);
     for (int k = 1; k < kStepEvents; ++k) mark();
     return kSearchNone;
   }
