@@ -278,7 +278,8 @@ class PointNavRolloutGenerator:
         _lib.check(self._L.bpsx_set_profiling(self._h, int(enabled)))
 
     def kernel_times(self):
-        """{kernel name: average ms per step} over the steps profiled so far, and the step count."""
+        """{kernel name: average ms per step} over the steps profiled so far, and the step count.  (Exploring agents: all under the
+        first name, their step is one launch.)"""
         ms = (C.c_double * 4)()
         steps = C.c_uint64()
         _lib.check(self._L.bpsx_get_kernel_times(self._h, ms, C.byref(steps)))

@@ -484,8 +484,8 @@ static void rotation_post_step(bpsx_sim* sim, const StepRecord& rec) {
 }
 
 // Groups of at most so many agents have their launches tell the host of their end.  The last launch of larger ones has the caches
-// written back by so many blocks that it takes longer than an event (exploring agents, event and flag: 2048 36.4 and 31.9 us,
-// 8192 41.2 and 38.7, 16384 43.6 and 44.4, 32768 64 and 69; point-goal agents: 8192 682 and 680, 65536 1141 and 1169).
+// written back by so many blocks that it takes longer than an event (exploring agents, event and flag: 2048 27.3 and 23.4 us,
+// 8192 33.1 and 30.1, 16384 35.4 and 34.8, 32768 44.8 and 49.7; point-goal agents: 8192 649 and 645, 16384 774 and 776, 65536 1141 and 1169).
 constexpr uint32_t kTellAgents = 8192;
 // Returns the number that the launch will tell.  Launches that tell run one after the other (a reset waits for the step in flight
 // before it, and for itself), so the newest number that has been told speaks for all before it.

@@ -696,6 +696,9 @@ struct GeoWave {
 // looking for its records among the lanes, a pass 500 besides.  Steps of 4096 agents over cluttered plans, of which the longest
 // search waits for this at a tie, 1069 -> 965 us, of 16384 over mazes 769 -> 734, of 65536 over mixed scenes 2505 -> 2469,
 // 1000 pairs over a maze 813 -> 732.)
+// (In the slot, heaps of up to 256 entries had a form of their own with one round, and geo_long's stayed in LDS up to 639 entries.
+// Searches of equal totals over a room, all of whose heaps come to leave LDS, and some back to a few entries: 400 of them 2.67 ms with
+// those and the pops above, now 2.58; 4000 4.86 and 4.60.)
 // (In registers, entry q in lane q mod 64, with the entries that move exchanged between lanes instead of through
 // LDS, the levels from the seventh on one after the other on the scalar unit: 300, 465, 800, 1025 cycles a pop, 250 to 670
 // a push, 804 us for 1000 pairs.)

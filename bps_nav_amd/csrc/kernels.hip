@@ -1,6 +1,6 @@
 // HIP kernels of the batch environment step (gfx950) and their launch wrappers.
 //
-// One step of a group of n agents is three launches:
+// One step of a group of n point-goal or fleeing agents is three launches:
 //   step_move      row of eight lanes per agent: action, turn / forward move with wall sliding, polar
 //                  observation, and a geodesic query (goal -> agent) when the agent moved or
 //                  the episode ended; an agent whose episode ended also picks its next episode
@@ -16,8 +16,9 @@
 // The first query of an episode that begins in step t is answered by step t + 1's geodesic launch, and
 // its result enters the bookkeeping at the start of step t + 1's step_finish.  No output of step t
 // depends on it (the reference computes it inside the reset and uses it from the next step on).  A reset
-// of a whole group (bpsx_reset) runs the snaps as a launch of their own before geodesic, first queries
-// included, and so does a step whose launches are timed.
+// of a whole group (bpsx_reset) draws the episodes and snaps their points before geodesic, first queries
+// included: by one launch (k_reset_begin) while the device holds a wavefront for each point, by two beyond
+// (k_reset_all, k_reset_snap).  A step whose launches are timed has k_reset_snap for the snaps, too.
 // The Flee task (simulator.cpp:830-869) runs through the same launches:
 // Flee keeps the episode's start point where PointNav keeps the snapped goal, so its
 // "distance from start" is the same start-point -> agent query.  Exploration makes no queries and
@@ -687,7 +688,7 @@ __global__ __launch_bounds__((kRowWaves + kSnaps) * 64) __attribute__((amdgpu_wa
 // on), so its query goes to the next step's queues.
 // (On a second stream next to the searches they cost the step two waits between streams, 6 to 17 us before
 // the searches begin and 6 at its end, for the 9 us by which they outlast the bookkeeping of a small
-// group: a step of 64 agents 232 us, now 219, of 1017 exploring ones 62 and 41.  At 16384 agents, whose 655
+// group: a step of 64 agents 232 us, now 219.  At 16384 agents, whose 655
 // new episodes take 22 us here, it makes no difference: 1193 us both ways without the copies of the counters.)
 // Q: the lists of queries that this step's searches have just served; Qnext: the other set.  The
 // counters of both are left as the next step expects them, so that a step needs no launch of its own

@@ -222,8 +222,9 @@ BPSX_API int bpsx_check_errors(bpsx_sim *sim);
 #define BPSX_NUM_COUNTERS 22
 BPSX_API int bpsx_get_counters(bpsx_sim *sim, uint64_t *out /* [BPSX_NUM_COUNTERS] */);
 /* Per-kernel timing with HIP events on the step's own stream. While enabled, every
- * step records a timestamp before each of its BPSX_NUM_KERNELS launches; step_end adds the
- * elapsed times up.  get_kernel_times returns the sums in milliseconds and the number of
+ * step records a timestamp before each of its BPSX_NUM_KERNELS launches and one behind the last; step_end
+ * adds the elapsed times up.  A step of exploring agents is one launch: all of its time counts for the first
+ * kernel, "step_move", and next to nothing for the others.  get_kernel_times returns the sums in milliseconds and the number of
  * steps they cover; enabling clears the sums. */
 #define BPSX_NUM_KERNELS 4
 BPSX_API int bpsx_set_profiling(bpsx_sim *sim, int enabled);

@@ -49,7 +49,10 @@ def test_outputs_are_there_when_the_call_returns(oracle, n, task):
             gen.step_start(g, torch.from_numpy(a).cuda() if t % 4 < 2 else a)
             if t == 20:
                 torch.cuda._sleep(20_000_000)   # some ten milliseconds
+                behind = streams[t % 3 % 2].record_event()
             gen.step_end(g)
+            if t == 20:
+                assert not behind.query(), "step_end has waited for what the stream does behind the step"
         if ordered:
             streams[t % 3 % 2].synchronize()
         with torch.cuda.stream(streams[2]):
