@@ -152,7 +152,7 @@ BPSX_DEV uint32_t visit_cell(const Row& row, const AgentArrays& A, uint32_t gi, 
 
 // The end of a block of a step's last launch, for all its threads.  Its last block of `blocks` tells a host that waits that all
 // that the launch has written can be seen: a host that waits for an event behind the launch hears of it later (a step of 64
-// agents in a room 121.4 -> 117.1 us, of 1017 that explore 30.4 -> 26.5).  One write-back for a block, once its
+// agents in a room 121.4 -> 117.1 us, of 1024 that explore 27.4 -> 23.4).  One write-back for a block, once its
 // wavefronts' stores have arrived: one for each wavefront costs the half of the gain.
 BPSX_DEV void tell_host(const StepParams& P, uint32_t blocks) {
   if (!P.done_flag) return;
@@ -535,8 +535,8 @@ BPSX_DEV void finish_agent(const AgentArrays& A, const StepParams& P, uint32_t g
 // such wavefront the others draw when they have moved.
 // Bound by latency, as moves and snaps are, 12 us each.  No list of queries or resets is filled, so the counters of both sets of queues
 // stay as they are, empty.
-// (As k_step_move and k_step_finish, with the snaps in the second, one after the other: 1017 agents over room plans 41.0 us a
-// step, now 26.)
+// (As k_step_move and k_step_finish, with the snaps in the second, one after the other: 1017 agents over room plans 41.4 us a
+// step, now 24.)
 template <uint32_t kRowWaves, uint32_t kSnaps>
 __global__ __launch_bounds__((kRowWaves + kSnaps) * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_step_explore(
     NavData nav, AgentArrays A, StepParams P, const int64_t* __restrict__ actions) {
