@@ -497,6 +497,7 @@ static uint32_t ask_to_be_told(bpsx_sim* sim, StepParams* P) {
 // Work that is being captured tells nothing: it does not run now, and its replays would write a number of long ago.
 static bool may_tell(const StepParams& P, hipStream_t st) {
   if (P.n > kTellAgents) return false;
+  if (!st) return true;   // the null stream cannot be captured
   hipStreamCaptureStatus status = hipStreamCaptureStatusActive;
   if (hipStreamIsCapturing(st, &status) != hipSuccess) (void)hipGetLastError();   // the launches will say why
   return status == hipStreamCaptureStatusNone;
